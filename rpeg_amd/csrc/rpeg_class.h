@@ -75,10 +75,26 @@ RPEG_HD unsigned blocked_mask(const NodeRec& r, uint64_t dpne) {
 
 struct GroupRec { uint16_t begin, count; };  // sub-node chains that share the chain's top rank
 
+// The same graph for the kernel that gives a plan a whole wavefront (rpeg_kernel_plan.h), in two further orders.
+// By level: nodes without successors first, then those whose successors are all in earlier levels, and so on, so that
+// the ranks of a level can be computed side by side; records and successors are named by their place in this order.
+struct LevelRec {
+  uint16_t succ[4];     // places of the first four successors, n_nodes (the neutral element) where there are fewer
+  uint16_t node;        // the node, by its number in the reference's order
+  uint8_t slot, blocked, cond, indeg, n_succ, pad;
+};
+// By tie-break class (ptkey): within a class the ranks decide the order.
+struct OrderRec {
+  uint16_t at;          // place in the level order
+  uint16_t b0, b1;      // the stretch of this order that the node's class takes
+  uint8_t chain_n, chain_i;   // nodes in its chain group (1: none) and its index there, which share the chain's top rank
+};
+
 struct ClassHdr {
   uint32_t n_nodes, n_slots, n_succ, n_init, n_groups, n_gmembers;
   uint32_t off_node, off_succ, off_init, off_topo, off_slot, off_group, off_gmember;  // byte offsets in the blob
   uint32_t off_pbeg, off_pred;       // predecessor lists in edge order: pred[pbeg[v] .. pbeg[v+1])
+  uint32_t n_levels, off_lrec, off_lbeg, off_orec, off_glvl, off_place;   // LevelRec, first place of every level (and n_nodes), OrderRec; gmember by place; node -> place
   uint32_t off_umap;                 // per slot: its index in the structure's slot universe (slot_universe)
   uint32_t bytes;
   uint32_t structure, split, error;  // error != 0: the reference would raise for this class
@@ -98,6 +114,11 @@ struct ClassView {
   const uint16_t* pbeg;
   const uint16_t* pred;
   const uint8_t* umap;
+  const LevelRec* lrec;
+  const uint16_t* lbeg;
+  const OrderRec* orec;
+  const uint16_t* glvl;
+  const uint16_t* place;
 };
 
 RPEG_HD ClassView class_view(const uint8_t* blob) {
@@ -113,6 +134,11 @@ RPEG_HD ClassView class_view(const uint8_t* blob) {
   v.pbeg = (const uint16_t*)(blob + v.h->off_pbeg);
   v.pred = (const uint16_t*)(blob + v.h->off_pred);
   v.umap = blob + v.h->off_umap;
+  v.lrec = (const LevelRec*)(blob + v.h->off_lrec);
+  v.lbeg = (const uint16_t*)(blob + v.h->off_lbeg);
+  v.orec = (const OrderRec*)(blob + v.h->off_orec);
+  v.glvl = (const uint16_t*)(blob + v.h->off_glvl);
+  v.place = (const uint16_t*)(blob + v.h->off_place);
   return v;
 }
 

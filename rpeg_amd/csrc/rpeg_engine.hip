@@ -412,17 +412,25 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) vo
   for (uint64_t w = blockIdx.x; w < L.n_waves; w += gridDim.x) kq_eval_wave(L, w, kq_lds);
 }
 
-// One plan per wavefront (rpeg_kernel_plan.h); perm[w] is the plan of wavefront task w.
+// One plan per wavefront (rpeg_kernel_plan.h); perm[w] is the plan of wavefront task w.  TR: KpTrace.
+template <int TR>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_plan(const EvalLaunch L) {
   extern __shared__ uint8_t kp_lds[];
   for (uint64_t w = blockIdx.x; w < L.n_waves; w += gridDim.x) {
     const uint64_t pi = L.perm ? L.perm[w] : w;
     const uint32_t off = L.wave_cls[w];
     if (off == KP_SKIP) continue;   // uniform: a task without a plan to evaluate
-    kp_eval_plan(L, w, pi, class_view(L.pool + off), kp_lds);
+    kp_eval_plan<TR>(L, w, pi, class_view(L.pool + off), kp_lds);
     // (lane 0 wrote the outputs of the task: its release store orders them before the flag)
     if (L.done && threadIdx.x == 0) __hip_atomic_store(&L.done[w], L.done_tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
+}
+
+// The launch of k_plan that keeps as much of the schedule as its outputs need.
+static void launch_plan(unsigned grid, size_t lds, hipStream_t s, const EvalLaunch& L) {
+  if (L.util) hipLaunchKernelGGL(k_plan<KP_TIMES_ORDER>, dim3(grid), dim3(WAVE), lds, s, L);
+  else if (L.mass) hipLaunchKernelGGL(k_plan<KP_TIMES>, dim3(grid), dim3(WAVE), lds, s, L);
+  else hipLaunchKernelGGL(k_plan<KP_NO_TRACE>, dim3(grid), dim3(WAVE), lds, s, L);
 }
 
 // Generic single-wavefront kernel over the host/device-shared scheduler template; used for the
@@ -612,7 +620,9 @@ static uint8_t* static_scratch_ptr(int dev, hipError_t* st) {
 // (python -m rpeg_amd.engine.profile) and then to the step time of configuration 2 over a sweep of each figure;
 // rpeg_engine_set_split_model replaces them (a measurement aid).  A wrong figure
 // costs time, never a result: every kernel computes the same bits.
-//   plan_a + plan_b x nodes                    what a plan costs k_plan (one plan per wavefront), beside the main kernel
+//   plan_a + plan_b x nodes                    what a plan costs k_plan (one plan per wavefront), beside the main kernel;
+//                                              plan_list times as much beyond KP_LANE_NODES nodes, where its scheduler
+//                                              keeps the nodes in LDS and fewer of its wavefronts fit on a compute unit
 //   quad_a + nodes x (quad_b + quad_c x pops)  a wavefront of k_quad (sixteen plans); pops = heap pops per dispatch,
 //                                              as the main kernel measured them for the class
 //   eff_beside_quad                            the part of the modelled room beside the main kernel that k_plan really
@@ -620,7 +630,7 @@ static uint8_t* static_scratch_ptr(int dev, hipError_t* st) {
 //   quad_margin                                a class moves to k_quad only if it ends this much later in the main kernel
 //   gain_threshold, gain_classes               a split by class size / by measured time must model this much earlier
 struct SplitModel {
-  double plan_a = 40.0, plan_b = 2.2;
+  double plan_a = 12.0, plan_b = 0.9, plan_list = 1.2;
   double quad_a = 40.0, quad_b = 1.6, quad_c = 0.45;
   double eff_beside_quad = 0.65;
   double quad_margin = 1.15;
@@ -1238,12 +1248,14 @@ struct DeepModel {
   double eff = 1.0;   // the part of the modelled room beside the main kernel that k_plan really gets
   uint64_t r_max;
   SplitModel sm;
-  double plan_cost(uint32_t plans, uint32_t nodes) const { return (double)plans * (sm.plan_a + sm.plan_b * (double)nodes); }
+  double plan_cost(uint32_t plans, uint32_t nodes) const {
+    return (double)plans * (sm.plan_a + sm.plan_b * (double)nodes) * (nodes > (uint32_t)KP_LANE_NODES ? sm.plan_list : 1.0);
+  }
   double total(double w_main, double w_plan, double max_t, uint64_t r) const {
     const double t_main = std::max(max_t, w_main / (n_cu * (double)r));
     const double room = eff * std::max(0.0, std::min(16.0 - 2.0 * (double)r, std::floor((160.0 * 1024 - (double)r * lds_main) / lds_plan)));
     const double left = std::max(0.0, w_plan - t_main * n_cu * room);
-    return t_main + left / (n_cu * 16.0);
+    return t_main + left / (n_cu * std::min(16.0, std::floor(160.0 * 1024 / lds_plan)));
   }
   double best(double w_main, double w_plan, double max_t, uint64_t* r_best) const {
     double b = 0.0;
@@ -1352,7 +1364,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     L.mass = mass; L.prof = nullptr;
     const size_t lds = kp_lds_bytes(e->max_nodes, e->max_slots);
     if (e->timing) HIP_TRY(e, hipEventRecord(e->ev0, s));
-    hipLaunchKernelGGL(k_plan, dim3((unsigned)std::min<uint64_t>(n, (uint64_t)e->n_cu * 32)), dim3(WAVE), lds, s, L);
+    launch_plan((unsigned)std::min<uint64_t>(n, (uint64_t)e->n_cu * 32), lds, s, L);
     HIP_TRY(e, hipGetLastError());
     if (e->timing) HIP_TRY(e, hipEventRecord(e->ev1, s));
     HIP_TRY(e, hipMemcpyAsync(e->h_ccount, d_unknown, 4, hipMemcpyDeviceToHost, s));
@@ -2008,7 +2020,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   };
   auto launch_main = [&]() {
     if (n_waves == 0) {
-    } else if (one) hipLaunchKernelGGL(k_plan, dim3(grid), dim3(WAVE), lds, sm, L);
+    } else if (one) launch_plan(grid, lds, sm, L);
     else switch (ls) {
       case 0: hipLaunchKernelGGL(k_eval<0>, dim3(grid), dim3(WAVE), lds, sm, L); break;
       case 8: hipLaunchKernelGGL(k_eval<8>, dim3(grid), dim3(WAVE), lds, sm, L); break;
@@ -2040,8 +2052,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     S.wave_cls = e->d_cls + n_host_tasks;
     S.n_waves = n_solo;
     if (L.prof) S.prof = L.prof + (n_waves + n_quad_waves) * 8;
-    hipLaunchKernelGGL(k_plan, dim3((unsigned)std::min<uint64_t>(n_solo, (uint64_t)e->n_cu * 32)), dim3(WAVE),
-                       kp_lds_bytes(e->max_nodes, e->max_slots), e->s2, S);
+    launch_plan((unsigned)std::min<uint64_t>(n_solo, (uint64_t)e->n_cu * 32), kp_lds_bytes(e->max_nodes, e->max_slots), e->s2, S);
     HIP_TRY(e, hipGetLastError());
   }
   if (peaks_deferred) {
@@ -2154,7 +2165,7 @@ int rpeg_eval_batch_static(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   L.flags = flags & RPEG_GATE_STALE; L.makespan = makespan; L.peak = peak; L.score = score; L.mask = mask;
   L.mass = nullptr; L.prof = nullptr;
   const size_t lds = kp_lds_bytes(e->max_nodes, e->max_slots);
-  hipLaunchKernelGGL(k_plan, dim3((unsigned)std::min<uint64_t>(n, (uint64_t)e->n_cu * 32)), dim3(WAVE), lds, s, L);
+  launch_plan((unsigned)std::min<uint64_t>(n, (uint64_t)e->n_cu * 32), lds, s, L);
   HIP_TRY(e, hipGetLastError());
   e->stats[0] = 0; e->stats[1] = 0; e->stats[2] = n; e->stats[3] = lds; e->stats[4] = 0; e->stats[5] = 1; e->stats[6] = 0;
   e->stats[7] = 0;
@@ -2551,7 +2562,7 @@ int host_small_submit(rpeg_engine_t* e, HostLane& ln, uint64_t n, GET get, uint3
   const unsigned grid = (unsigned)std::min<uint64_t>(m, (uint64_t)e->n_cu * 32);
   e->stats[3] = lds;
   if (e->timing) HIP_TRY(e, hipEventRecord(e->ev0, s));
-  hipLaunchKernelGGL(k_plan, dim3(grid), dim3(WAVE), lds, s, L);
+  launch_plan(grid, lds, s, L);
   HIP_TRY(e, hipGetLastError());
   if (e->timing) HIP_TRY(e, hipEventRecord(e->ev1, s));
   ln.launched = true;

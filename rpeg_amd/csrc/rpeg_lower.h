@@ -10,6 +10,7 @@
 #ifndef RPEG_LOWER_H
 #define RPEG_LOWER_H
 
+#include <algorithm>
 #include <cstring>
 #include <stdexcept>
 #include <string>
@@ -388,6 +389,45 @@ inline LoweredClass lower_class(const rpeg_problem_t& P, uint64_t sig_bits) {
     groups.push_back(GroupRec{(uint16_t)gmember.size(), (uint16_t)(chain_beg[k + 1] - chain_beg[k])});
     for (int j = chain_beg[k]; j < chain_beg[k + 1]; ++j) gmember.push_back((uint16_t)chain_of[j]);
   }
+  // the orders of the one-plan-per-wavefront kernel: by level (from the nodes without successors up), and by
+  // tie-break class
+  std::vector<LevelRec> lrec(n);
+  std::vector<OrderRec> orec(n);
+  std::vector<uint16_t> lbeg, glvl(gmember.size()), place16(n);
+  {
+    std::vector<int> level(n, 0), place(n, 0);
+    int n_levels = n ? 1 : 0;
+    for (int h = (int)topo.size() - 1; h >= 0; --h) {
+      const int v = topo[h];
+      for (int j = adj_beg[v]; j < adj_beg[v + 1]; ++j) level[v] = std::max(level[v], level[adj_to[j]] + 1);
+      n_levels = std::max(n_levels, level[v] + 1);
+    }
+    lbeg.assign(n_levels + 1, 0);
+    for (int v = 0; v < n; ++v) ++lbeg[level[v] + 1];
+    for (int l = 0; l < n_levels; ++l) lbeg[l + 1] = (uint16_t)(lbeg[l + 1] + lbeg[l]);
+    std::vector<uint16_t> cur(lbeg.begin(), lbeg.end() - 1);
+    for (int v = 0; v < n; ++v) { place[v] = cur[level[v]]++; place16[v] = (uint16_t)place[v]; }
+    for (int v = 0; v < n; ++v) {
+      LevelRec& r = lrec[place[v]];
+      for (int j = 0; j < 4; ++j) r.succ[j] = (uint16_t)(j < recs[v].n_succ ? place[adj_to[adj_beg[v] + j]] : n);
+      r.node = (uint16_t)v;
+      r.slot = recs[v].slot; r.blocked = recs[v].blocked; r.cond = recs[v].cond; r.indeg = recs[v].indeg;
+      r.n_succ = recs[v].n_succ; r.pad = 0;
+    }
+    for (size_t k = 0; k < gmember.size(); ++k) glvl[k] = (uint16_t)place[gmember[k]];
+    std::vector<int> first(257, 0), chain_n(n, 1), chain_i(n, 0);
+    for (int v = 0; v < n; ++v) ++first[recs[v].ptkey + 1];
+    for (int k = 0; k < 256; ++k) first[k + 1] += first[k];
+    std::vector<int> at(first.begin(), first.end() - 1);
+    for (const GroupRec& g : groups) {
+      if (g.count > 255) throw std::runtime_error("chain group too long");
+      for (int j = 0; j < g.count; ++j) { chain_n[gmember[g.begin + j]] = g.count; chain_i[gmember[g.begin + j]] = j; }
+    }
+    for (int v = 0; v < n; ++v) {
+      const int k = recs[v].ptkey;
+      orec[at[k]++] = OrderRec{(uint16_t)place[v], (uint16_t)first[k], (uint16_t)first[k + 1], (uint8_t)chain_n[v], (uint8_t)chain_i[v]};
+    }
+  }
   // every slot's place in the structure's slot universe
   std::vector<uint8_t> umap(slots.size(), 0);
   {
@@ -426,6 +466,12 @@ inline LoweredClass lower_class(const rpeg_problem_t& P, uint64_t sig_bits) {
   h.off_pbeg = (uint32_t)off; off = align8(off + pbeg.size() * 2);
   h.off_pred = (uint32_t)off; off = align8(off + pred.size() * 2);
   h.off_umap = (uint32_t)off; off = align8(off + umap.size());
+  h.n_levels = (uint32_t)lbeg.size() - 1;
+  h.off_lrec = (uint32_t)(off = (off + 15) & ~size_t(15)); off = align8(off + lrec.size() * sizeof(LevelRec));
+  h.off_orec = (uint32_t)off; off = align8(off + orec.size() * sizeof(OrderRec));
+  h.off_lbeg = (uint32_t)off; off = align8(off + lbeg.size() * 2);
+  h.off_place = (uint32_t)off; off = align8(off + place16.size() * 2);
+  h.off_glvl = (uint32_t)off; off = (off + glvl.size() * 2 + 15) & ~size_t(15);   // (blobs start on sixteen-byte boundaries of the pool)
   h.bytes = (uint32_t)off;
   out.blob.assign(off, 0);
   std::memcpy(out.blob.data(), &h, sizeof h);
@@ -439,6 +485,11 @@ inline LoweredClass lower_class(const rpeg_problem_t& P, uint64_t sig_bits) {
   std::memcpy(out.blob.data() + h.off_pbeg, pbeg.data(), pbeg.size() * 2);
   if (!pred.empty()) std::memcpy(out.blob.data() + h.off_pred, pred.data(), pred.size() * 2);
   if (!umap.empty()) std::memcpy(out.blob.data() + h.off_umap, umap.data(), umap.size());
+  if (!lrec.empty()) std::memcpy(out.blob.data() + h.off_lrec, lrec.data(), lrec.size() * sizeof(LevelRec));
+  if (!orec.empty()) std::memcpy(out.blob.data() + h.off_orec, orec.data(), orec.size() * sizeof(OrderRec));
+  std::memcpy(out.blob.data() + h.off_lbeg, lbeg.data(), lbeg.size() * 2);
+  if (!place16.empty()) std::memcpy(out.blob.data() + h.off_place, place16.data(), place16.size() * 2);
+  if (!glvl.empty()) std::memcpy(out.blob.data() + h.off_glvl, glvl.data(), glvl.size() * 2);
   return out;
 }
 

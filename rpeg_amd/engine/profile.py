@@ -86,7 +86,7 @@ def main() -> None:
             ph = np.diff(b[sl][ok][:, :7], axis=1) / 100.0
             names = ("plan fields", "durations", "memory model", "ranks", "scheduling", "outputs") if name == "k_eval" else \
                     ("plan fields", "durations", "memory model", "ranks and positions", "scheduling", "outputs") if name == "k_quad" else \
-                    ("plan fields", "durations", "memory model and ranks", "positions in the order", "scheduling", "outputs")
+                    ("plan fields and durations", "memory model", "ranks", "positions", "scheduling", "outputs")
             print("   phases, mean us per task: " + ", ".join(f"{nm} {x:.1f}" for nm, x in zip(names, ph.mean(0))))
             slow = np.argsort(-d)[:40]
             print("   phases of the 40 longest: " + ", ".join(f"{nm} {x:.1f}" for nm, x in zip(names, ph[slow].mean(0))))
