@@ -213,8 +213,8 @@ int rpeg_eval_batch_mass(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* pl
    configurations held by the host (RPEG/search/optimizer.py:793-798, the `map` over `_eval_worker`; and
    every single call of evaluate / evaluate_cached, RPEG/search/evaluate.py:235-403).  For a batch of at most
    32 plans per compute unit the host computes the lowering class of each plan itself and the call is one
-   copy to the device, one launch (one plan per wavefront) whose results land in pinned host memory, and one
-   wait; larger batches are staged through device memory and take the path of rpeg_eval_batch.  Returns when
+   launch (one plan per wavefront) that reads the plans from pinned host memory, leaves the results there and
+   flags them; larger batches are staged through device memory and take the path of rpeg_eval_batch.  Returns when
    the results are in place. */
 int rpeg_eval_host(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, uint32_t flags, double* makespan,
                    double* peak, double* score, uint8_t* mask, double* mass, void* stream);
@@ -230,6 +230,19 @@ int rpeg_eval_host(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, u
    rpeg_eval_trace_metrics (the same numbers, one launch per plan). */
 int rpeg_eval_host_util(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, uint32_t flags, double* makespan,
                         double* peak, double* score, uint8_t* mask, double* utilization, void* stream);
+
+/* What evaluate_cached() returns of ONE plan (RPEG/search/evaluate.py:329-403), from one launch: result[0..2] =
+   makespan, peak, score and the mask as by rpeg_eval_host for a single plan; start and finish of every lowered node
+   in node order as by rpeg_eval_trace, dispatched[k] = the node dispatched k-th; and, described on the host while the
+   launch runs, the node_* arrays of rpeg_lower_plan and rpeg_eval_trace (each may be NULL).  `cap` nodes of capacity.
+   Returns the node count (the times hold where the mask has RPEG_MASK_VALID and not RPEG_MASK_ERROR; 0 nodes for a
+   plan that is not valid); -8 where the engine would not run this plan on the plan-per-wavefront kernel (a class above
+   384 nodes, or another layout asked for): the caller then uses rpeg_eval_host and rpeg_eval_trace. */
+int rpeg_eval_host_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t* head4, uint32_t flags,
+                         double* result, uint8_t* mask, double* start, double* finish, int32_t* dispatched,
+                         int32_t* node_kind, int32_t* node_vertex, int32_t* node_step, int32_t* node_sub,
+                         int32_t* node_src, int64_t* node_payload, int32_t* node_ref, uint8_t* node_reserved,
+                         int32_t cap, void* stream);
 
 /* Single-node durations and isolated peaks: the batched form of the candidate-directory loop
    (RPEG/search/moves.py:532-549): for strategy i, time = NodeCostModel.time(mock node) and

@@ -418,9 +418,15 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) vo
   extern __shared__ uint8_t kp_lds[];
   for (uint64_t w = blockIdx.x; w < L.n_waves; w += gridDim.x) {
     const uint64_t pi = L.perm ? L.perm[w] : w;
-    const uint32_t off = L.wave_cls[w];
+    uint32_t rec = 0u, off;
+    if (L.rec) {
+      rec = L.rec[w * (KE_REC_BYTES / 4) + (threadIdx.x & (KE_REC_BYTES / 4 - 1))];
+      off = (uint32_t)__builtin_amdgcn_readlane((int)rec, KE_REC_BYTES / 4 - 1);
+    } else {
+      off = L.wave_cls[w];
+    }
     if (off == KP_SKIP) continue;   // uniform: a task without a plan to evaluate
-    kp_eval_plan<TR>(L, w, pi, class_view(L.pool + off), kp_lds);
+    kp_eval_plan<TR>(L, w, pi, rec, class_view(L.pool + off), kp_lds);
     // (lane 0 wrote the outputs of the task: its release store orders them before the flag)
     if (L.done && threadIdx.x == 0) __hip_atomic_store(&L.done[w], L.done_tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
@@ -428,7 +434,7 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) vo
 
 // The launch of k_plan that keeps as much of the schedule as its outputs need.
 static void launch_plan(unsigned grid, size_t lds, hipStream_t s, const EvalLaunch& L) {
-  if (L.util) hipLaunchKernelGGL(k_plan<KP_TIMES_ORDER>, dim3(grid), dim3(WAVE), lds, s, L);
+  if (L.util || L.trace) hipLaunchKernelGGL(k_plan<KP_TIMES_ORDER>, dim3(grid), dim3(WAVE), lds, s, L);
   else if (L.mass) hipLaunchKernelGGL(k_plan<KP_TIMES>, dim3(grid), dim3(WAVE), lds, s, L);
   else hipLaunchKernelGGL(k_plan<KP_NO_TRACE>, dim3(grid), dim3(WAVE), lds, s, L);
 }
@@ -638,23 +644,22 @@ struct SplitModel {
 };
 constexpr int SPLIT_MODEL_FIELDS = 9;
 
-// Staging of one small host-pointer evaluation: plans and class offsets in (pinned, then device), results out (pinned,
-// written by the kernel itself), and which of the caller's plans went to the device.
+// Staging of one small host-pointer evaluation: plan records in (EvalLaunch::rec), results out, both pinned, and which
+// of the caller's plans went to the device.  The kernel reads the records where they lie (no copy ahead of the launch)
+// and flags every finished plan in the result block, where the host polls for it instead of waiting for the launch to
+// end: what counts in these calls is latency.
 struct HostLane {
-  uint8_t *in = nullptr, *dev = nullptr, *out = nullptr;
-  // `direct`: the kernel reads the plans from the pinned block itself (no copy ahead of the launch) and flags every
-  // finished plan in the pinned result block, where the host polls for it instead of waiting for the launch to end:
-  // for the steps of an annealing run, whose latency is what counts
-  bool direct = false;
+  uint8_t *in = nullptr, *out = nullptr;
   uint8_t *in_dev = nullptr, *out_dev = nullptr;   // the pinned blocks as the device addresses them
   uint32_t tag = 0;
-  size_t cap = 0;
+  size_t cap = 0;          // a multiple of 64
+  size_t flag_bytes() const { return 4 * cap; }   // `out` begins with the flags: nothing but tags is ever written there
   std::vector<uint32_t> idx;
   size_t n = 0, stride = 0;
   bool launched = false;
   void release() {
-    if (in) { hipHostFree(in); hipFree(dev); hipHostFree(out); }
-    in = dev = out = in_dev = out_dev = nullptr;
+    if (in) { hipHostFree(in); hipHostFree(out); }
+    in = out = in_dev = out_dev = nullptr;
     cap = 0;
   }
 };
@@ -704,6 +709,8 @@ struct rpeg_engine_s {
   size_t d_stage_cap = 0;
   uint8_t* h_stage = nullptr;   // pinned mirror of the result region of d_stage
   size_t h_stage_cap = 0;
+  uint8_t *h_times = nullptr, *h_times_dev = nullptr;   // pinned: EvalLaunch::trace
+  size_t h_times_nodes = 0;
   uint8_t* d_trace = nullptr;   // rpeg_eval_trace: one plan's fields and header, then start / finish / dispatch index
   uint8_t* d_detail = nullptr;  // rpeg_plan_detail: one plan's fields and header, then slot durations and vertex-set peaks
   size_t d_trace_nodes = 0;
@@ -1109,6 +1116,7 @@ void rpeg_engine_destroy(rpeg_engine_t* e) {
   e->lane0.release();
   if (e->d_stage) hipFree(e->d_stage);
   if (e->h_stage) hipHostFree(e->h_stage);
+  if (e->h_times) hipHostFree(e->h_times);
   if (e->d_trace) hipFree(e->d_trace);
   if (e->d_detail) hipFree(e->d_detail);
   if (e->d_ws) hipFree(e->d_ws);
@@ -2117,6 +2125,42 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   return 0;
 }
 
+// What the records of lower() hold of every node of a plan's class (arrays may be null).
+static void describe_nodes(const rpeg_problem_t& problem, const rpeg_struct_t& st, const PlanHead& h, const VPlan (&a)[RPEG_MAX_V],
+                           const LoweredClass& lc, int32_t* node_kind, int32_t* node_vertex, int32_t* node_step, int32_t* node_sub,
+                           int32_t* node_src, int64_t* node_payload, int32_t* node_ref) {
+  const ClassView cv = class_view(lc.blob.data());
+  for (size_t i = 0; i < lc.nodes.size(); ++i) {
+    const LoweredNode& nd = lc.nodes[i];
+    const SlotDesc sd = cv.slot[nd.slot];
+    if (node_kind) node_kind[i] = nd.kind;
+    if (node_vertex) node_vertex[i] = nd.kind == 0 ? nd.vertex : nd.a1;
+    if (node_step) node_step[i] = nd.step;
+    if (node_sub) node_sub[i] = nd.sub;
+    if (node_src) node_src[i] = nd.kind == 0 ? nd.vertex : nd.a0;
+    int64_t payload = 0;
+    int32_t ref = -1;
+    if (sd.type == SLOT_COMM_DATA) {
+      payload = sd.q == 0xFF ? st.edge[sd.a].full_bytes : st.edge[sd.a].sub_bytes[h.split][sd.q];
+      ref = sd.a;
+    } else if (sd.type == SLOT_COMM_PUB) {
+      const rpeg_pub_t& pb = st.pub[sd.a];
+      payload = pub_payload(problem, a[pb.src], a[pb.dst], pb.model);
+      ref = 16 + pb.model;
+    } else if (sd.type == SLOT_RESHARD) {
+      payload = problem.model[sd.b].n_params * problem.model[sd.b].sb;
+      ref = 16 + sd.b;
+    }
+    if (node_payload) node_payload[i] = payload;
+    if (node_ref) node_ref[i] = ref;
+  }
+}
+
+static int host_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t* head4, uint32_t flags, double* result,
+                      uint8_t* mask, double* start, double* finish, int32_t* dispatched, int32_t* node_kind, int32_t* node_vertex,
+                      int32_t* node_step, int32_t* node_sub, int32_t* node_src, int64_t* node_payload, int32_t* node_ref,
+                      uint8_t* node_reserved, int32_t cap, hipStream_t s, LoweredClass& lc);
+
 extern "C" {
 
 int rpeg_engine_host_us(const rpeg_engine_t* e, double* out, int32_t n) {
@@ -2211,6 +2255,23 @@ int rpeg_eval_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t*
   if (!plan_valid(e->P, h, a)) { e->err = "plan violates the integer validity rules"; return -6; }
   const uint64_t sg = plan_signature(e->P, h.structure, h.split, h.tau0, h.tau1, a);
   LoweredClass lc;
+  {   // a graph that k_plan takes: one launch, whose times land in pinned memory
+    double result[3];
+    uint8_t mask = 0;
+    std::vector<int32_t> dispatched((size_t)std::max(cap, 1));
+    const int m = host_trace(e, vert_fields, head4, 0u, result, &mask, start, finish, dispatched.data(), node_kind, node_vertex,
+                             node_step, node_sub, node_src, nullptr, nullptr, node_reserved, cap, nullptr, lc);
+    if (m < 0 && m != -8) return m;
+    if (m >= 0 && (mask & RPEG_MASK_VALID) && !(mask & RPEG_MASK_ERROR)) {
+      if (edges && (int)lc.edges.size() > cap) { e->err = "trace arrays too small"; return -7; }
+      if (dispatch_index)
+        for (int k = 0; k < m; ++k) dispatch_index[dispatched[k]] = k;
+      if (edges)
+        for (size_t j = 0; j < lc.edges.size(); ++j) { edges[2 * j] = lc.edges[j].first; edges[2 * j + 1] = lc.edges[j].second; }
+      if (n_edges) *n_edges = (int32_t)lc.edges.size();
+      return m;
+    }
+  }
   try { lc = lower_class(e->P, sg); } catch (const std::exception& ex) { e->err = ex.what(); return -5; }
   const int n = (int)lc.nodes.size();
   if (n > cap || (edges && (int)lc.edges.size() > cap)) { e->err = "trace arrays too small"; return -7; }
@@ -2249,13 +2310,7 @@ int rpeg_eval_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t*
   HIP_TRY(e, hipMemcpy(start, d_tr, (size_t)n * 8, hipMemcpyDeviceToHost));
   HIP_TRY(e, hipMemcpy(finish, d_tr + n, (size_t)n * 8, hipMemcpyDeviceToHost));
   if (dispatch_index) HIP_TRY(e, hipMemcpy(dispatch_index, d_tr + 2 * (size_t)n, (size_t)n * 4, hipMemcpyDeviceToHost));
-  for (int i = 0; i < n; ++i) {
-    if (node_kind) node_kind[i] = lc.nodes[i].kind;
-    if (node_vertex) node_vertex[i] = lc.nodes[i].kind == 0 ? lc.nodes[i].vertex : lc.nodes[i].a1;
-    if (node_step) node_step[i] = lc.nodes[i].step;
-    if (node_sub) node_sub[i] = lc.nodes[i].sub;
-    if (node_src) node_src[i] = lc.nodes[i].kind == 0 ? lc.nodes[i].vertex : lc.nodes[i].a0;
-  }
+  describe_nodes(e->P, e->P.st[h.structure], h, a, lc, node_kind, node_vertex, node_step, node_sub, node_src, nullptr, nullptr);
   if (node_reserved) {   // the vertices whose allocations the scheduler reserves for the node
     const ClassView cv = class_view(e->pool.data() + off);
     const uint64_t dpne = plan_masks(a, e->P.st[h.structure].n_vertex).dpne;
@@ -2286,31 +2341,7 @@ int rpeg_lower_plan(const rpeg_problem_t* problem, const int16_t* vert_fields, c
   try { lc = lower_class(*problem, sg); } catch (const std::exception&) { return -5; }
   const int n = (int)lc.nodes.size();
   if (n > cap || (edges && (int)lc.edges.size() > cap)) return -7;
-  const ClassView cv = class_view(lc.blob.data());
-  for (int i = 0; i < n; ++i) {
-    const LoweredNode& nd = lc.nodes[i];
-    const SlotDesc sd = cv.slot[nd.slot];
-    if (node_kind) node_kind[i] = nd.kind;
-    if (node_vertex) node_vertex[i] = nd.kind == 0 ? nd.vertex : nd.a1;
-    if (node_step) node_step[i] = nd.step;
-    if (node_sub) node_sub[i] = nd.sub;
-    if (node_src) node_src[i] = nd.kind == 0 ? nd.vertex : nd.a0;
-    int64_t payload = 0;
-    int32_t ref = -1;
-    if (sd.type == SLOT_COMM_DATA) {
-      payload = sd.q == 0xFF ? st.edge[sd.a].full_bytes : st.edge[sd.a].sub_bytes[h.split][sd.q];
-      ref = sd.a;
-    } else if (sd.type == SLOT_COMM_PUB) {
-      const rpeg_pub_t& pb = st.pub[sd.a];
-      payload = pub_payload(*problem, a[pb.src], a[pb.dst], pb.model);
-      ref = 16 + pb.model;
-    } else if (sd.type == SLOT_RESHARD) {
-      payload = problem->model[sd.b].n_params * problem->model[sd.b].sb;
-      ref = 16 + sd.b;
-    }
-    if (node_payload) node_payload[i] = payload;
-    if (node_ref) node_ref[i] = ref;
-  }
+  describe_nodes(*problem, st, h, a, lc, node_kind, node_vertex, node_step, node_sub, node_src, node_payload, node_ref);
   if (edges)
     for (size_t j = 0; j < lc.edges.size(); ++j) { edges[2 * j] = lc.edges[j].first; edges[2 * j + 1] = lc.edges[j].second; }
   if (n_edges) *n_edges = (int32_t)lc.edges.size();
@@ -2456,16 +2487,15 @@ int rpeg_eval_trace_metrics(rpeg_engine_t* e, const int16_t* vert_fields, const 
 // masses) and read back in one synchronisation.
 namespace {
 
-constexpr size_t HS_IN_BYTES = (size_t)RPEG_MAX_V * RPEG_FIELDS * 2 + 4 + 4;   // per plan: fields, header, class offset
-constexpr size_t HS_OUT_BYTES = 3 * 8 + (size_t)RPEG_MAX_V * 8 + 8 + 8 + 8;    // makespan, peak, score, mass, utilisation, mask (padded), done flag (padded)
+static_assert((size_t)RPEG_MAX_V * RPEG_FIELDS * 2 + 4 + 4 == KE_REC_BYTES, "a plan record: fields, header, class offset");
+constexpr size_t HS_OUT_BYTES = 4 + 3 * 8 + (size_t)RPEG_MAX_V * 8 + 8 + 8;   // per plan: flag; makespan, peak, score, mass, utilisation, mask (padded)
 
 int ensure_host_stage(rpeg_engine_t* e, HostLane& ln, size_t n, hipStream_t s) {
   if (n <= ln.cap) return 0;
   HIP_TRY(e, hipStreamSynchronize(s));
   ln.release();
   const size_t cap = (std::max<size_t>(n + n / 2, 1024) + 63) & ~size_t(63);
-  HIP_TRY(e, hipHostMalloc(&ln.in, HS_IN_BYTES * cap));
-  HIP_TRY(e, hipMalloc(&ln.dev, HS_IN_BYTES * cap));
+  HIP_TRY(e, hipHostMalloc(&ln.in, KE_REC_BYTES * cap));
   HIP_TRY(e, hipHostMalloc(&ln.out, HS_OUT_BYTES * cap, hipHostMallocCoherent));   // (the host reads it while a launch runs)
   std::memset(ln.out, 0, HS_OUT_BYTES * cap);
   HIP_TRY(e, hipHostGetDevicePointer((void**)&ln.in_dev, ln.in, 0));
@@ -2476,22 +2506,20 @@ int ensure_host_stage(rpeg_engine_t* e, HostLane& ln, size_t n, hipStream_t s) {
 
 // Plans in host memory, results to host memory, for a batch small enough for one plan per wavefront: the
 // host computes the class of every plan itself (validity gate, signature, table lookup: ~100 ns per plan),
-// so the call is one copy to the device, one launch of k_plan, whose first lanes write the results straight
-// into pinned host memory, and one wait.  get(i, head, a) yields plan i.  The work comes in two halves so that a
-// caller with several lanes (staging buffers and a stream each) can keep one evaluation running while it prepares
-// the next: host_small_submit stages and launches, host_small_collect waits and hands the results out.  Submit
+// so the call is one launch of k_plan, which reads the plans from pinned memory, writes the results straight
+// into pinned memory and flags every plan it has finished.  get(i, head, a) yields plan i.  The work comes in two halves
+// so that a caller with several lanes (staging buffers and a stream each) can keep one evaluation running while it
+// prepares the next: host_small_submit stages and launches, host_small_collect waits and hands the results out.  Submit
 // returns 1 when the batch is not eligible (a class too large for k_plan); the caller then takes the device path.
+// trace: EvalLaunch::trace, for a batch of one plan.
 template <class GET>
 int host_small_submit(rpeg_engine_t* e, HostLane& ln, uint64_t n, GET get, uint32_t flags, bool want_mass, bool want_util,
-                      hipStream_t s) {
+                      hipStream_t s, double* trace = nullptr) {
   ln.n = n; ln.launched = false; ln.idx.clear();
   if (n == 0) return 0;
   const size_t stride = ((size_t)n + 63) & ~size_t(63);
   ln.stride = stride;
   if (int rc = ensure_host_stage(e, ln, stride, s)) return rc;
-  int16_t* in_vert = (int16_t*)ln.in;
-  uint8_t* in_head = ln.in + (size_t)RPEG_MAX_V * RPEG_FIELDS * 2 * stride;
-  uint32_t* in_cls = (uint32_t*)(in_head + 4 * stride);
   uint64_t n_new = 0;
   for (uint64_t i = 0; i < n; ++i) {
     PlanHead h;
@@ -2505,24 +2533,26 @@ int host_small_submit(rpeg_engine_t* e, HostLane& ln, uint64_t n, GET get, uint3
     n_new += is_new ? 1 : 0;
     const size_t j = ln.idx.size();
     ln.idx.push_back((uint32_t)i);
+    int16_t rec[KE_REC_BYTES / 2];
     for (int v = 0; v < nv; ++v) {
-      int16_t* p = in_vert + (size_t)v * RPEG_FIELDS * stride + j;
-      p[0 * stride] = (int16_t)a[v].dp; p[1 * stride] = (int16_t)a[v].pp; p[2 * stride] = (int16_t)a[v].tp; p[3 * stride] = (int16_t)a[v].mb;
-      p[4 * stride] = (int16_t)a[v].o[0]; p[5 * stride] = (int16_t)a[v].o[1]; p[6 * stride] = (int16_t)a[v].o[2];
-      p[7 * stride] = (int16_t)a[v].e[0]; p[8 * stride] = (int16_t)a[v].e[1]; p[9 * stride] = (int16_t)a[v].e[2];
+      int16_t* p = rec + v * RPEG_FIELDS;
+      p[0] = (int16_t)a[v].dp; p[1] = (int16_t)a[v].pp; p[2] = (int16_t)a[v].tp; p[3] = (int16_t)a[v].mb;
+      p[4] = (int16_t)a[v].o[0]; p[5] = (int16_t)a[v].o[1]; p[6] = (int16_t)a[v].o[2];
+      p[7] = (int16_t)a[v].e[0]; p[8] = (int16_t)a[v].e[1]; p[9] = (int16_t)a[v].e[2];
     }
-    in_head[0 * stride + j] = (uint8_t)h.structure; in_head[1 * stride + j] = (uint8_t)h.split;
-    in_head[2 * stride + j] = (uint8_t)h.tau0; in_head[3 * stride + j] = (uint8_t)h.tau1;
-    in_cls[j] = (uint32_t)off;
+    for (int x = nv * RPEG_FIELDS; x < RPEG_MAX_V * RPEG_FIELDS; ++x) rec[x] = 1;
+    const uint8_t head[4] = {(uint8_t)h.structure, (uint8_t)h.split, (uint8_t)h.tau0, (uint8_t)h.tau1};
+    const uint32_t cls = (uint32_t)off;
+    std::memcpy(rec + RPEG_MAX_V * RPEG_FIELDS, head, 4);
+    std::memcpy(rec + RPEG_MAX_V * RPEG_FIELDS + 2, &cls, 4);
+    std::memcpy(ln.in + KE_REC_BYTES * j, rec, KE_REC_BYTES);
   }
   const size_t m = ln.idx.size();
   e->stats[0] = 0; e->stats[1] = n_new; e->stats[2] = m; e->stats[3] = 0; e->stats[4] = 0; e->stats[5] = 1; e->stats[6] = 0;
   if (m == 0) return 0;
   if (e->max_nodes > (uint32_t)(WAVE * KP_MAX_NS) || kp_lds_bytes(e->max_nodes, e->max_slots) > 64 * 1024) return 1;
   if (int rc = ensure_pool(e, s)) return rc;
-  if (!ln.direct) HIP_TRY(e, hipMemcpyAsync(ln.dev, ln.in, HS_IN_BYTES * stride, hipMemcpyHostToDevice, s));
-  const uint8_t* d_in = ln.direct ? ln.in_dev : ln.dev;
-  double* o_makespan = (double*)ln.out_dev;
+  double* o_makespan = (double*)(ln.out_dev + ln.flag_bytes());
   double* o_peak = o_makespan + stride;
   double* o_score = o_peak + stride;
   double* o_mass = o_score + stride;
@@ -2530,11 +2560,11 @@ int host_small_submit(rpeg_engine_t* e, HostLane& ln, uint64_t n, GET get, uint3
   uint8_t* o_mask = (uint8_t*)(o_util + stride);
   EvalLaunch L;
   L.P = e->dP;
-  L.vert = (const int16_t*)d_in;
-  L.head = d_in + (size_t)RPEG_MAX_V * RPEG_FIELDS * 2 * stride;
-  L.stride = stride;
+  L.vert = nullptr; L.head = nullptr; L.stride = 0;
   L.perm = nullptr;
-  L.wave_cls = (const uint32_t*)(L.head + 4 * stride);
+  L.wave_cls = nullptr;
+  L.rec = (const uint32_t*)ln.in_dev;
+  L.trace = trace;
   L.pool = e->d_pool; L.ws = nullptr;
   L.n_waves = m; L.ws_nodes = e->max_nodes; L.ws_slots = e->max_slots;
   L.cls_bytes = 0; L.rcap = 0; L.max_v = e->max_v; L.ovf = nullptr; L.need = nullptr;
@@ -2553,11 +2583,9 @@ int host_small_submit(rpeg_engine_t* e, HostLane& ln, uint64_t n, GET get, uint3
     e->prof_waves = m;
     L.prof = e->d_prof;
   }
-  if (ln.direct) {
-    if (++ln.tag == 0) ++ln.tag;
-    L.done = (uint32_t*)(o_mask + stride);
-    L.done_tag = ln.tag;
-  }
+  if (++ln.tag == 0) ++ln.tag;
+  L.done = (uint32_t*)ln.out_dev;
+  L.done_tag = ln.tag;
   const size_t lds = kp_lds_bytes(e->max_nodes, e->max_slots);
   const unsigned grid = (unsigned)std::min<uint64_t>(m, (uint64_t)e->n_cu * 32);
   e->stats[3] = lds;
@@ -2578,9 +2606,9 @@ int host_small_collect(rpeg_engine_t* e, HostLane& ln, double* makespan, double*
     ln.launched = false;
     --e->lanes_busy;
     bool seen = false;
-    if (ln.direct) {
+    if (!e->timing && !e->prof_on) {
       // the flags of all plans, in pinned memory: a plan's results are there once its flag is
-      const uint32_t* done = (const uint32_t*)(ln.out + (3 * 8 + (size_t)RPEG_MAX_V * 8 + 8) * stride + stride);
+      const uint32_t* done = (const uint32_t*)ln.out;
       const auto t0 = std::chrono::steady_clock::now();
       size_t j = 0;
       for (uint64_t spins = 0;; ++spins) {
@@ -2613,7 +2641,7 @@ int host_small_collect(rpeg_engine_t* e, HostLane& ln, double* makespan, double*
     }
   }
   if (m == 0) return 0;
-  const double* o_makespan = (const double*)ln.out;
+  const double* o_makespan = (const double*)(ln.out + ln.flag_bytes());
   const double* o_peak = o_makespan + stride;
   const double* o_score = o_peak + stride;
   const double* o_mass = o_score + stride;
@@ -2642,6 +2670,62 @@ int eval_host_small(rpeg_engine_t* e, uint64_t n, GET get, uint32_t flags, doubl
 }
 
 }  // namespace
+
+// One plan with the times of its nodes from one launch (rpeg_eval_host_trace); lc: its lowered class.
+static int host_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t* head4, uint32_t flags, double* result,
+                      uint8_t* mask, double* start, double* finish, int32_t* dispatched, int32_t* node_kind, int32_t* node_vertex,
+                      int32_t* node_step, int32_t* node_sub, int32_t* node_src, int64_t* node_payload, int32_t* node_ref,
+                      uint8_t* node_reserved, int32_t cap, hipStream_t s, LoweredClass& lc) {
+  e->err.clear();
+  if (e->state_lanes != -1 && e->state_lanes != 1) return -8;   // (a layout was asked for: the caller goes the long way)
+  PlanHead h = load_head(head4, 1, 0);
+  VPlan a[RPEG_MAX_V];
+  std::memset(a, 0, sizeof a);
+  *mask = 0;
+  if (h.structure >= e->P.n_struct) return 0;
+  const rpeg_struct_t& st = e->P.st[h.structure];
+  for (int v = 0; v < st.n_vertex; ++v) load_vertex(vert_fields, 1, 0, v, &a[v]);
+  if (!plan_valid(e->P, h, a)) return 0;
+  const uint64_t sg = plan_signature(e->P, h.structure, h.split, h.tau0, h.tau1, a);
+  const int64_t off = class_offset(e, sg, nullptr);
+  if (off < 0) return -5;
+  const size_t rows = e->max_nodes;
+  if (rows > (size_t)(WAVE * KP_MAX_NS)) return -8;
+  if (rows > e->h_times_nodes) {   // (no launch that writes the old block is under way: the call that made one has waited for it)
+    if (e->h_times) hipHostFree(e->h_times);
+    e->h_times = nullptr;
+    e->h_times_nodes = 0;
+    HIP_TRY(e, hipHostMalloc(&e->h_times, rows * 18, hipHostMallocCoherent));
+    HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_times_dev, e->h_times, 0));
+    e->h_times_nodes = rows;
+  }
+  auto get = [&](uint64_t, PlanHead& ph, VPlan (&pa)[RPEG_MAX_V]) { ph = h; std::memcpy(pa, a, sizeof pa); };
+  e->last_ms = -1.0;
+  const int rc = host_small_submit(e, e->lane0, 1, get, flags, false, false, s, (double*)e->h_times_dev);
+  if (rc) return rc == 1 ? -8 : rc;
+  // while the launch runs: what the records of the nodes hold
+  bool lowered = true;
+  try { lc = lower_class(e->P, sg); } catch (const std::exception& ex) { lowered = false; e->err = ex.what(); }
+  const int n = (int)lc.nodes.size();
+  if (lowered && n <= cap) {
+    describe_nodes(e->P, st, h, a, lc, node_kind, node_vertex, node_step, node_sub, node_src, node_payload, node_ref);
+    if (node_reserved) {
+      const ClassView cv = class_view(lc.blob.data());
+      const uint64_t dpne = plan_masks(a, st.n_vertex).dpne;
+      for (int i = 0; i < n; ++i) node_reserved[i] = (uint8_t)blocked_mask(cv.node[i], dpne);
+    }
+  }
+  if (const int rc2 = host_small_collect(e, e->lane0, result, result + 1, result + 2, mask, nullptr, nullptr, s)) return rc2;
+  if (!lowered) return -5;
+  if (n > cap) { e->err = "trace arrays too small"; return -7; }
+  if (*mask & RPEG_MASK_ERROR) return n;
+  const double* t = (const double*)e->h_times;
+  std::memcpy(start, t, (size_t)n * 8);
+  std::memcpy(finish, t + rows, (size_t)n * 8);
+  const uint16_t* d = (const uint16_t*)(t + 2 * rows);
+  for (int k = 0; k < n; ++k) dispatched[k] = d[k];
+  return n;
+}
 
 // rpeg_eval_host: plans and results in host memory.  Small batches go through eval_host_small; larger ones
 // (or problems whose classes are too large for it) are copied to the device and take the batch path.
@@ -2748,7 +2832,6 @@ struct GpuSaBackend : SaBackend {
   GpuSaBackend(rpeg_engine_t* eng, hipStream_t st, int capacity, int n_lanes = 1) : e(eng), s(st), cap(capacity) {
     lane.resize((size_t)std::max(1, n_lanes));
     for (Lane& l : lane) {
-      l.st.direct = true;
       if (hipStreamCreateWithFlags(&l.s, hipStreamNonBlocking) != hipSuccess) { rc_alloc = -2; e->err = "hipStreamCreate failed"; l.s = nullptr; }
     }
     const size_t V = RPEG_MAX_V * RPEG_FIELDS;
@@ -2827,7 +2910,7 @@ struct GpuSaBackend : SaBackend {
         for (int x = 0; x < RPEG_MAX_V; ++x) out[i].mass[x] = nan;
       }
     }
-    const double* o_score = (const double*)l.st.out + 2 * stride;
+    const double* o_score = (const double*)(l.st.out + l.st.flag_bytes()) + 2 * stride;
     const double* o_mass = o_score + stride;
     const uint8_t* o_mask = (const uint8_t*)(o_mass + (size_t)RPEG_MAX_V * stride + stride);
     for (size_t j = 0; j < m; ++j) {
@@ -2846,7 +2929,7 @@ struct GpuSaBackend : SaBackend {
   // take that path (the caller then asks per plan)
   int evaluate(int n, const SaPlan* plans, const uint8_t* variant, SaEval* out, bool with_util) override {
     if (n > cap) { e->err = "annealing batch exceeds its buffers"; return -1; }
-    {  // a step's proposals are a small batch: one copy, one launch (eval_host_small)
+    {  // a step's proposals are a small batch: one launch (eval_host_small)
       const auto t0 = std::chrono::steady_clock::now();
       auto get = [&](uint64_t i, PlanHead& h, VPlan (&a)[RPEG_MAX_V]) {
         const uint8_t* hd = head_of[variant[i]];
@@ -2950,6 +3033,16 @@ int rpeg_eval_host_util(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* pla
     if (int rc = rpeg_eval_trace_metrics(e, f, h4, &utilization[i], nullptr)) return rc;
   }
   return 0;
+}
+
+int rpeg_eval_host_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t* head4, uint32_t flags, double* result,
+                         uint8_t* mask, double* start, double* finish, int32_t* dispatched, int32_t* node_kind, int32_t* node_vertex,
+                         int32_t* node_step, int32_t* node_sub, int32_t* node_src, int64_t* node_payload, int32_t* node_ref,
+                         uint8_t* node_reserved, int32_t cap, void* stream) {
+  if (!e || !vert_fields || !head4 || !result || !mask || !start || !finish || !dispatched) return -1;
+  LoweredClass lc;
+  return host_trace(e, vert_fields, head4, flags, result, mask, start, finish, dispatched, node_kind, node_vertex, node_step, node_sub,
+                    node_src, node_payload, node_ref, node_reserved, cap, (hipStream_t)stream, lc);
 }
 
 int rpeg_sa_run(rpeg_engine_t* e, const rpeg_sa_params_t* prm, const int16_t* base_plan, rpeg_sa_result_t* res,

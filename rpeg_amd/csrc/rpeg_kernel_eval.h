@@ -30,6 +30,8 @@ constexpr uint32_t KE_IDLE = 0xFFFFFFFFu;
 constexpr uint32_t KE_CLS_LDS = 0x80000000u;   // flag in EvalLaunch::wave_cls
 constexpr int KE_FEW = 8;                      // plans of a wavefront so flagged
 
+constexpr size_t KE_REC_BYTES = 128;            // EvalLaunch::rec
+
 struct EvalLaunch {              // uniform launch parameters
   const rpeg_problem_t* P;
   const int16_t* vert;
@@ -73,6 +75,12 @@ struct EvalLaunch {              // uniform launch parameters
   uint32_t* done = nullptr;      // k_plan only: done[w] = done_tag once the outputs of wave task w are written (a release
   uint32_t done_tag = 0;         // store at system scope, for a host that polls pinned memory instead of waiting for the
                                  // end of the launch); or null
+  // k_plan only: the plans as records of KE_REC_BYTES in memory the host wrote -- fields (vertex by vertex, ones behind
+  // the last vertex), four header bytes, class blob offset -- in place of vert, head and wave_cls.  A record is two cache
+  // lines, which a wavefront fetches across the bus in one load; or null.
+  const uint32_t* rec = nullptr;
+  double* trace = nullptr;       // k_plan only: start[node], then finish[node], then dispatched[k] (uint16) of the one plan
+                                 // of the launch, each `ws_nodes` long; or null
   uint32_t* limit = nullptr;     // plans whose ready set outgrew what this kernel holds for good (no launch with a
                                  // longer list follows): limit[0] counts them, then (plan, class blob offset) pairs.
                                  // The launch that ends the call redoes them with a ready list as long as the

@@ -293,11 +293,12 @@ __device__ inline double kp_utilization(const ClassView& cv, const int n, const 
   return count ? total / (double)count : 0.0;
 }
 
-// One plan, evaluated by the whole wavefront.  pi: plan index (uniform).  TR (KpTrace): what the outputs of the launch
+// One plan, evaluated by the whole wavefront.  pi: plan index (uniform).  rec: lane l < 32 holds word l of the plan's
+// record where the launch has records.  TR (KpTrace): what the outputs of the launch
 // need of the schedule -- nothing, the times for L.mass, the dispatch order too for L.util.
 template <int TR>
-__device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const uint64_t pi, const ClassView cv,
-                                    uint8_t* lds) {
+__device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const uint64_t pi, const uint32_t rec,
+                                    const ClassView cv, uint8_t* lds) {
   const int lane = threadIdx.x;
   const rpeg_problem_t& P = *L.P;
   const int n = (int)cv.h->n_nodes, n_slots = (int)cv.h->n_slots;
@@ -348,8 +349,16 @@ __device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const
     KE_STAMP(1);
     KE_STAMP(2);
   } else {
-    const PlanHead h = load_head(L.head, L.stride, pi);
-    if (lane < KP_PLAN_I16) l_plan[lane] = lane < nv * RPEG_FIELDS ? L.vert[(uint64_t)lane * L.stride + pi] : (int16_t)1;
+    PlanHead h;
+    if (L.rec) {
+      const uint32_t hw = (uint32_t)__builtin_amdgcn_readlane((int)rec, RPEG_MAX_V * RPEG_FIELDS / 2);
+      h.structure = (int)(hw & 0xFFu); h.split = (int)((hw >> 8) & 0xFFu);
+      h.tau0 = (int)((hw >> 16) & 0xFFu); h.tau1 = (int)(hw >> 24);
+      if (lane < KP_PLAN_I16 / 2) ((uint32_t*)l_plan)[lane] = lane < RPEG_MAX_V * RPEG_FIELDS / 2 ? rec : 0x00010001u;
+    } else {
+      h = load_head(L.head, L.stride, pi);
+      if (lane < KP_PLAN_I16) l_plan[lane] = lane < nv * RPEG_FIELDS ? L.vert[(uint64_t)lane * L.stride + pi] : (int16_t)1;
+    }
     __syncthreads();
 
     // ---- pair relations: lane 8u+v tests vertices u and v, the ballots are the masks
@@ -447,6 +456,16 @@ __device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const
     if ((L.flags & RPEG_GATE_STALE) && !stale_ok) score = 0.0;
     out_makespan = makespan;
     out_score = score;
+  }
+  if (TR == KP_TIMES_ORDER && L.trace && !err) {
+    __syncthreads();
+    double* const t = L.trace;
+    uint16_t* const d = (uint16_t*)(t + 2 * (size_t)L.ws_nodes);
+    for (int i = lane; i < n; i += KE_WAVE) {
+      t[i] = l_start[i];
+      t[(size_t)L.ws_nodes + i] = l_rank[i];
+      d[i] = l_ord[i];
+    }
   }
   double m = __builtin_nan("");   // lane x < RPEG_MAX_V: mass of vertex x
   if (TR != KP_NO_TRACE && L.mass) {

@@ -25,7 +25,7 @@ EXPORTS = ("rpeg_engine_create", "rpeg_engine_destroy", "rpeg_last_error", "rpeg
            "rpeg_engine_last_kernel_ms", "rpeg_device_exp", "rpeg_engine_reset_classes", "rpeg_eval_batch_mass",
            "rpeg_sa_run", "rpeg_sa_propose", "rpeg_eval_host_util", "rpeg_engine_set_state_lanes", "rpeg_engine_set_sa_groups", "rpeg_engine_set_side_layout", "rpeg_engine_host_us", "rpeg_engine_set_split_model", "rpeg_engine_set_quad_share", "rpeg_engine_set_ready_cap", "rpeg_engine_profile", "rpeg_sa_optimize", "rpeg_eval_host",
            "rpeg_sa_optimize_families", "rpeg_eval_trace_metrics", "rpeg_eval_batch_static", "rpeg_plan_detail",
-           "rpeg_lower_plan")
+           "rpeg_lower_plan", "rpeg_eval_host_trace")
 
 
 class EngineError(RuntimeError):
@@ -69,6 +69,8 @@ def load_library(path: Optional[str] = None):
     lib.rpeg_op_time_batch.argtypes = [vp, u64, i32, i32, vp, u64, vp, vp, vp]
     lib.rpeg_eval_trace.restype = C.c_int
     lib.rpeg_eval_trace.argtypes = [vp] * 13 + [i32, vp]
+    lib.rpeg_eval_host_trace.restype = C.c_int
+    lib.rpeg_eval_host_trace.argtypes = [vp, vp, vp, u32] + [vp] * 13 + [i32, vp]
     lib.rpeg_eval_trace_metrics.restype = C.c_int
     lib.rpeg_eval_trace_metrics.argtypes = [vp] * 5
     lib.rpeg_lower_plan.restype = C.c_int
@@ -481,6 +483,34 @@ class Engine:
         self._check(n, "rpeg_eval_trace")
         return dict(start=start[:n], finish=finish[:n], order=order[:n], kind=kind[:n], vertex=vertex[:n], step=step[:n],
                     sub=sub[:n], src=src[:n], edges=edges[:2 * ne.value].reshape(-1, 2), reserved=reserved[:n])
+
+    def eval_trace(self, batch: PlanBatch, gate_stale: bool = True, cap: int = 512):
+        """`eval` of the one plan of `batch` with the times and the description of its nodes from the same launch
+        (rpeg_eval_host_trace), as lists by node; `dispatched[k]` is the node dispatched k-th.  None where the plan
+        does not go to the plan-per-wavefront kernel (whose graphs have at most 384 nodes)."""
+        torch = _torch()
+        vert = np.ascontiguousarray(batch.vert[:, 0], dtype=np.int16)
+        head = np.ascontiguousarray(batch.head[:, 0], dtype=np.uint8)
+        times = np.empty((2, cap))
+        result = np.empty(3)
+        ints = np.empty((7, cap), np.int32)    # dispatched, kind, vertex, step, sub, src, ref
+        payload = np.empty(cap, np.int64)
+        bytes_ = np.empty(cap + 1, np.uint8)   # reserved; then the mask
+        at, row = ints.ctypes.data, cap * 4
+        with torch.cuda.device(self.device):
+            n = self.lib.rpeg_eval_host_trace(self._h, vert.ctypes.data, head.ctypes.data, abi.GATE_STALE if gate_stale else 0,
+                                              result.ctypes.data, bytes_.ctypes.data + cap, times.ctypes.data,
+                                              times.ctypes.data + cap * 8, *(at + k * row for k in range(6)),
+                                              payload.ctypes.data, at + 6 * row, bytes_.ctypes.data, cap,
+                                              torch.cuda.current_stream(self.device).cuda_stream)
+        if n == -8:
+            return None
+        self._check(n, "rpeg_eval_host_trace")
+        start, finish = times[:, :n].tolist()
+        dispatched, kind, vertex, step, sub, src, ref = ints[:, :n].tolist()
+        return dict(makespan=float(result[0]), peak=float(result[1]), score=float(result[2]), mask=int(bytes_[cap]),
+                    start=start, finish=finish, dispatched=dispatched, kind=kind, vertex=vertex, step=step, sub=sub,
+                    src=src, ref=ref, payload=payload[:n].tolist(), reserved=bytes_[:n].tolist())
 
     def plan_detail(self, batch: PlanBatch, i: int, cap: int = 4096):
         """NodeCostModel.time, payload bytes and label reference of every lowered node of plan i (the reference's
