@@ -143,6 +143,11 @@ class TemplateVertex:
     id: str
     kind: OperatorKind
 
+    # (every table of a plan is keyed by vertices: hashing the kind's containers took 3 us a lookup, the id's hash is
+    # the string's own and kept by it)
+    def __hash__(self):
+        return hash(self.id)
+
 
 @dataclass(frozen=True)
 class TemplateEdge:

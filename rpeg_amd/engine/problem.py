@@ -117,10 +117,14 @@ class PlanBatch:
         self.head[0, i], self.head[1, i] = structure, split
         for t, tau in enumerate(taus):
             self.head[2 + t, i] = tau
-        for s, v in enumerate(rpeg.vertices):
+        rows = []
+        for v in rpeg.vertices:
             a = plan.sigma[v]
-            row = list(plan.pi[v]) + [plan.mb[v]] + list(a.origin) + list(a.extent)
-            self.vert[s * FIELDS_PER_VERTEX:(s + 1) * FIELDS_PER_VERTEX, i] = row
+            row = (*plan.pi[v], plan.mb[v], *a.origin, *a.extent)
+            if len(row) != FIELDS_PER_VERTEX:
+                raise ValueError(f"vertex {v.id}: a strategy has three degrees, an allocation three coordinates")
+            rows += row
+        self.vert[:len(rows), i] = rows
 
     def configuration(self, problem: EvalProblem, i: int):
         """(rpeg, ExecutionPlan, Workload) of candidate i in the reference's representation."""

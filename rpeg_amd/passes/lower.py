@@ -154,46 +154,84 @@ def lower(rpeg, unrolled: UnrolledRPEG, plan, suite, K_eval: int, workload: Opti
         cap *= 8
     if n < 0:
         raise ValueError(f"rpeg_lower_plan failed with status {n}")
-    phases = gen_phases(workload) if workload is not None and workload.gen_quantiles else []
-    verts = rpeg.vertices
-    copies: Dict[tuple, UnrolledNode] = {} if unrolled is None else {(x.template_vertex, x.k): x for x in unrolled.nodes}
+    kind, vertex, step, sub, src, ref, payload = (x[:n].tolist() for x in (kind, vertex, step, sub, src, ref, payload))
     graph = ExecutableRPEG.__new__(ExecutableRPEG)
     home = weakref.ref(graph)      # (weak: a graph and its nodes must not keep each other alive in a cycle)
-    nodes = []
-    n_comm = n_reshard = 0
-    for i in range(n):
-        v = verts[vertex[i]]
-        if kind[i] == 0:
-            op = copies.get((v, int(step[i]))) or UnrolledNode(v, int(step[i]))
-            more = {}
-            tag = ""
-            if sub[i] >= 0:
-                n_act, n_seq, steps, t0, pf = phases[sub[i]]
-                if v.kind.role.value == "GEN":
-                    tag = f":g{sub[i]}"
-                    more = dict(n_seqs=n_seq, n_active=n_act, phase_steps=steps, phase_t_start=t0, is_prefill_phase=pf)
-                else:
-                    tag = f":i{sub[i]}"
-                    more = dict(n_seqs=n_seq)
-            nodes.append(ExecNode(id=f"{v.id}@{step[i]}{tag}", kind=ExecNodeType.OP, allocs=(plan.sigma[v],), op=op,
-                                  model=v.kind.model, pi=plan.pi[v], mb=plan.mb.get(v, None), _home=(home, i), **more))
-            continue
-        allocs = (plan.sigma[verts[src[i]]], plan.sigma[v])
-        label = rpeg.data_edges[ref[i]].container.name if ref[i] < 16 else f"W_{_MODEL_BY_CODE[ref[i] - 16].value}"
-        if kind[i] == 1:
-            n_comm += 1
-            nodes.append(ExecNode(id=f"comm{n_comm}", kind=ExecNodeType.COMM, allocs=allocs,
-                                  payload_in_bytes=int(payload[i]), label=label, _home=(home, i)))
-        else:
-            n_reshard += 1
-            nodes.append(ExecNode(id=f"reshard{n_reshard}", kind=ExecNodeType.RESHARD, allocs=allocs,
-                                  model=_MODEL_BY_CODE[ref[i] - 16], payload_in_bytes=int(payload[i]), label=label,
-                                  _home=(home, i)))
-    pairs = edges[:2 * ne.value].reshape(-1, 2)
+    nodes = graph_nodes(rpeg, unrolled, plan, workload, home, kind, vertex, step, sub, src, ref, payload)
+    links = []
+    for a, b in edges[:2 * ne.value].reshape(-1, 2).tolist():
+        link = ExecEdge.__new__(ExecEdge)
+        link.__dict__.update(src=nodes[a], dst=nodes[b])
+        links.append(link)
     object.__setattr__(graph, "nodes", tuple(nodes))
-    object.__setattr__(graph, "edges", tuple(ExecEdge(nodes[a], nodes[b]) for a, b in pairs))
+    object.__setattr__(graph, "edges", tuple(links))
     object.__setattr__(graph, "composite_operators", ())
     object.__setattr__(graph, "source", LoweringSource(rpeg, plan, suite, K_eval, workload))
     if verbose:
         print(f"RPEG lowered successfully: {len(nodes)} nodes, {len(graph.edges)} edges.")
     return graph
+
+
+def graph_nodes(rpeg, unrolled, plan, workload, home, kind, vertex, step, sub, src, ref, payload):
+    """The ExecNodes of a lowered graph from the library's description of them (lists by node).  A graph has a hundred
+    and more: what the nodes of one vertex share is put together once, and the records are filled without their
+    constructor, which sets every one of fifteen frozen fields by a call."""
+    phases = gen_phases(workload) if workload is not None and workload.gen_quantiles else []
+    verts = rpeg.vertices
+    copies: Dict[tuple, UnrolledNode] = {} if unrolled is None else {(x.template_vertex, x.k): x for x in unrolled.nodes}
+    blank = dict(id=None, kind=None, allocs=None, op=None, model=None, pi=None, mb=None, n_seqs=None, n_active=None,
+                 phase_steps=None, phase_t_start=None, is_prefill_phase=False, fusion_group=None, payload_in_bytes=0,
+                 label=None, _home=None)
+    shared = {}     # of the operator nodes of a vertex
+    tags = {}       # (vertex, phase) -> ending of the id, the phase's fields
+    ops = {}        # (vertex, step) -> UnrolledNode
+    nodes = []
+    n_comm = n_reshard = 0
+    sigma = [plan.sigma.get(v) for v in verts]
+    new = ExecNode.__new__
+    for i, (what, x) in enumerate(zip(kind, vertex)):
+        node = new(ExecNode)
+        f = node.__dict__
+        if what == 0:
+            if x not in shared:
+                v = verts[x]
+                shared[x] = dict(blank, kind=ExecNodeType.OP, allocs=(sigma[x],), model=v.kind.model, pi=plan.pi[v],
+                                 mb=plan.mb.get(v, None))
+            f.update(shared[x])
+            k = step[i]
+            op = ops.get((x, k))
+            if op is None:
+                op = ops[x, k] = copies.get((verts[x], k)) or UnrolledNode(verts[x], k)
+            q = sub[i]
+            if q < 0:
+                f["id"] = f"{verts[x].id}@{k}"
+            else:
+                hit = tags.get((x, q))
+                if hit is None:
+                    n_act, n_seq, steps, t0, pf = phases[q]
+                    if verts[x].kind.role.value == "GEN":
+                        hit = (f":g{q}", dict(n_seqs=n_seq, n_active=n_act, phase_steps=steps, phase_t_start=t0, is_prefill_phase=pf))
+                    else:
+                        hit = (f":i{q}", dict(n_seqs=n_seq))
+                    tags[x, q] = hit
+                f["id"] = f"{verts[x].id}@{k}{hit[0]}"
+                f.update(hit[1])
+            f["op"] = op
+        else:
+            f.update(blank)
+            r = ref[i]
+            f["allocs"] = (sigma[src[i]], sigma[x])
+            f["payload_in_bytes"] = payload[i]
+            f["label"] = rpeg.data_edges[r].container.name if r < 16 else f"W_{_MODEL_BY_CODE[r - 16].value}"
+            if what == 1:
+                n_comm += 1
+                f["id"] = f"comm{n_comm}"
+                f["kind"] = ExecNodeType.COMM
+            else:
+                n_reshard += 1
+                f["id"] = f"reshard{n_reshard}"
+                f["kind"] = ExecNodeType.RESHARD
+                f["model"] = _MODEL_BY_CODE[r - 16]
+        f["_home"] = (home, i)
+        nodes.append(node)
+    return nodes

@@ -8,6 +8,8 @@ the graph's own nodes, in dispatch order as the reference fills its dictionaries
 
 from __future__ import annotations
 
+import numpy as np
+
 from ..core.types import DeviceSpace, RPEG_TRANSFER_RESOURCE_POLICY, TransferResourcePolicy
 from ..engine.problem import PlanBatch
 from .trace import Trace
@@ -30,19 +32,28 @@ def trace_on(eng, executable, batch) -> Trace:
     nodes = executable.nodes
     if len(tr["start"]) != len(nodes):
         raise ValueError("the lowered graph does not belong to this plan")
-    by_dispatch = sorted(range(len(nodes)), key=lambda i: int(tr["order"][i]))   # scheduler.py:517-518
-    start = {nodes[i]: float(tr["start"][i]) for i in by_dispatch}
-    finish = {nodes[i]: float(tr["finish"][i]) for i in by_dispatch}
-    # the allocations the scheduler reserved: of a node's allocations (source first) those whose vertex the engine
-    # reserved, identical allocations once (transfer_resources.py:138-148)
-    sigma = executable.source.plan.sigma
-    verts = executable.source.rpeg.vertices
-    reserved = {}
-    for i, node in enumerate(nodes):
-        mask = int(tr["reserved"][i])
-        owners = (int(tr["vertex"][i]),) if tr["kind"][i] == 0 else (int(tr["src"][i]), int(tr["vertex"][i]))
-        reserved[node] = tuple(dict.fromkeys(sigma[verts[x]] for x in owners if (mask >> x) & 1))
-    return Trace(start=start, finish=finish, reserved_allocations=reserved)
+    src = executable.source
+    dispatched = np.argsort(tr["order"], kind="stable").tolist()
+    return trace_from(nodes, src.rpeg.vertices, src.plan.sigma, dispatched,
+                      *(tr[k].tolist() for k in ("start", "finish", "kind", "vertex", "src", "reserved")))
+
+
+def trace_from(nodes, verts, sigma, dispatched, start, finish, kind, vertex, src, reserved) -> Trace:
+    """Trace of `nodes` from the engine's lists by node: times keyed in dispatch order (scheduler.py:517-518), and the
+    allocations the scheduler reserved: of a node's allocations (source first) those whose vertex the engine reserved,
+    identical allocations once (transfer_resources.py:138-148), put together once per pair of vertices."""
+    order = [nodes[i] for i in dispatched]
+    sets = {}
+    kept = []
+    for owners in zip(kind, vertex, src, reserved):
+        hit = sets.get(owners)
+        if hit is None:
+            what, x, y, mask = owners
+            hit = sets[owners] = tuple(dict.fromkeys(sigma[verts[z]] for z in ((x,) if what == 0 else (y, x)) if (mask >> z) & 1))
+        kept.append(hit)
+    return Trace(start=dict(zip(order, [start[i] for i in dispatched])),
+                 finish=dict(zip(order, [finish[i] for i in dispatched])),
+                 reserved_allocations=dict(zip(nodes, kept)))
 
 
 def schedule(executable, cost_model, device_space: DeviceSpace, *,

@@ -14,6 +14,7 @@ integer part of `is_valid`) are host code as in the reference.
 
 from __future__ import annotations
 
+import weakref
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -29,7 +30,8 @@ from ..model.hardware import Hardware
 from ..model.memory import MemoryPolicy, NodeMemoryModel
 from ..model.models import ModelSuite
 from ..model.workload import Workload
-from ..passes.lower import ExecEdge, ExecNode, ExecNodeType, ExecutableRPEG, lower   # noqa: F401  (re-exported)
+from ..passes.lower import ExecEdge, ExecNode, ExecNodeType, ExecutableRPEG, graph_nodes, lower   # noqa: F401  (re-exported)
+from ..schedule.scheduler import trace_from
 from ..schedule.trace import Trace   # noqa: F401  (re-exported: the reference's evaluate module names it)
 from .cache import EvalCache, config_hash
 
@@ -197,6 +199,16 @@ def _pack(configs: Sequence[Configuration], st, workload: Workload) -> PlanBatch
     return batch
 
 
+def _raise_for(mask: int):
+    """The error of a configuration whose mask this is (of a batch: all bits of any, MASK_VALID of all)."""
+    if not mask & abi.MASK_VALID:
+        raise ValueError("a configuration violates the integer validity rules of is_valid")
+    if mask & abi.MASK_LIMIT:
+        raise EngineLimitError("a configuration exceeds a limit of the evaluation engine: it was not evaluated")
+    if mask & abi.MASK_ERROR:
+        raise ZeroDivisionError("a configuration has a degenerate node duration or makespan")
+
+
 @dataclass
 class BatchResult:
     score: np.ndarray      # evaluate_cached semantics (0 where the stale-layout rule fails)
@@ -228,12 +240,7 @@ def evaluate_batch(configs: Sequence[Configuration], suite: ModelSuite, workload
     else:
         out = eng.eval(batch, gate_stale=gate_stale)
     mask = out["mask"]
-    if np.any((mask & abi.MASK_VALID) == 0):
-        raise ValueError("a configuration violates the integer validity rules of is_valid")
-    if np.any(mask & abi.MASK_LIMIT):
-        raise EngineLimitError("a configuration exceeds a limit of the evaluation engine: it was not evaluated")
-    if np.any(mask & abi.MASK_ERROR):
-        raise ZeroDivisionError("a configuration has a degenerate node duration or makespan")
+    _raise_for(int(np.bitwise_or.reduce(mask)) & ~abi.MASK_VALID | int(np.bitwise_and.reduce(mask)) & abi.MASK_VALID)
     feasible = ((mask & abi.MASK_MEM_OK) != 0) & ((mask & abi.MASK_STALE_OK) != 0)
     score = out["score"].copy()
     if ABLATION_HARD_OOM:
@@ -297,14 +304,27 @@ def evaluation_cache_key(config: Configuration, memory_policy: MemoryPolicy = Me
             f"groups={memory_policy.max_worker_groups_per_gpu}")
 
 
+_no_graph = weakref.ref(Trace({}, {}))     # (of an object that is gone)
+
+
 def _score_one(config, suite, workload, hw, K_eval, memory_policy, gate_stale):
     _check_supported(config)
     eng, st = _engine_for(config.rpeg, suite, workload, hw, config.device_space, K_eval, memory_policy,
                           transfer_policy=config.transfer_resource_policy)
     batch = _pack([config], st, workload)
-    res = evaluate_batch([config], suite, workload, hw, K_eval, memory_policy, gate_stale=gate_stale)
-    trace, _ = _trace_of(eng, st, config, batch, workload, suite)
-    return float(res.score[0]), trace, res
+    t = eng.eval_trace(batch, gate_stale=gate_stale)
+    if t is None:     # a graph beyond the plan-per-wavefront kernel
+        res = evaluate_batch([config], suite, workload, hw, K_eval, memory_policy, gate_stale=gate_stale)
+        trace, _ = _trace_of(eng, st, config, batch, workload, suite)
+        return float(res.score[0]), trace, int(res.mask[0])
+    mask = t["mask"]
+    _raise_for(mask)
+    # (the graph the nodes belong to is not part of the result: nothing refers to it)
+    nodes = graph_nodes(config.rpeg, None, config.plan, workload, _no_graph, t["kind"], t["vertex"], t["step"], t["sub"],
+                        t["src"], t["ref"], t["payload"])
+    trace = trace_from(nodes, config.rpeg.vertices, config.plan.sigma, t["dispatched"], t["start"], t["finish"],
+                       t["kind"], t["vertex"], t["src"], t["reserved"])
+    return 0.0 if ABLATION_HARD_OOM and not mask & abi.MASK_MEM_OK else t["score"], trace, mask
 
 
 def evaluate_cached(config: Configuration, cache: EvalCache, suite: ModelSuite, workload: Workload, hw: Hardware,
@@ -316,8 +336,8 @@ def evaluate_cached(config: Configuration, cache: EvalCache, suite: ModelSuite, 
     if h in cache:
         score, trace, feasible = cache.get(h)
         return score, trace, feasible, False
-    score, trace, res = _score_one(config, suite, workload, hw, K_eval, memory_policy, gate_stale=True)
-    feasible = bool(res.feasible[0])
+    score, trace, mask = _score_one(config, suite, workload, hw, K_eval, memory_policy, gate_stale=True)
+    feasible = bool(mask & abi.MASK_MEM_OK) and bool(mask & abi.MASK_STALE_OK)
     cache.put(h, score, trace, feasible)
     return score, trace, feasible, True
 
@@ -329,5 +349,5 @@ def _eval_worker(args):
         memory_policy = MemoryPolicy()
     else:
         config, suite, workload, hw, K_eval, memory_policy = args
-    score, trace, res = _score_one(config, suite, workload, hw, K_eval, memory_policy, gate_stale=False)
-    return score, trace, bool(res.mask[0] & abi.MASK_MEM_OK)
+    score, trace, mask = _score_one(config, suite, workload, hw, K_eval, memory_policy, gate_stale=False)
+    return score, trace, bool(mask & abi.MASK_MEM_OK)

@@ -40,3 +40,22 @@ def test_every_form_of_the_scheduler_equals_the_host_build(c, K):
             assert float(util["util"][i]).hex() == float(eng.trace_metrics(batch, int(i))[0]).hex(), i
     finally:
         eng.close()
+
+
+@pytest.mark.parametrize("c,K", [(1, 4), (3, 10), (1, 16)])
+def test_one_plan_at_a_time_equals_the_oracle_on_either_side_of_the_largest_graph(c, K):
+    """evaluate_cached and its trace: from one launch up to 384 nodes, over the staged path and the single-plan trace
+    beyond (config 1 at 16 unrolled steps has graphs on either side)."""
+    from oracle import rpeg_oracle as oracle
+    from rpeg_amd.search.cache import EvalCache
+    from rpeg_amd.search.evaluate import Configuration, evaluate_cached
+    cfg, batch = seeded_batch(c, 3)
+    p = cfg.problem
+    for i in range(3):
+        rpeg, plan, wl = batch.configuration(p, i)
+        want = oracle.evaluate_plan(rpeg, plan, p.device_space, p.suite, wl, p.hw, K, p.memory_policy, check_stale=True,
+                                    want_trace=True)
+        score, trace, feasible, miss = evaluate_cached(Configuration(rpeg, plan, p.device_space), EvalCache(), p.suite, wl, p.hw, K)
+        assert miss and score == want["score"] and feasible == want["feasible"]
+        assert {n.id: t for n, t in trace.finish.items()} == want["finish"]
+        assert list(trace.start) == list(trace.finish) and len(trace.start) == len(want["nodes"])
