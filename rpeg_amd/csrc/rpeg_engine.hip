@@ -416,8 +416,31 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) vo
 template <int TR>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_plan(const EvalLaunch L) {
   extern __shared__ uint8_t kp_lds[];
+  __shared__ KpShared shared;
   for (uint64_t w = blockIdx.x; w < L.n_waves; w += gridDim.x) {
     const uint64_t pi = L.perm ? L.perm[w] : w;
+    const uint32_t off = L.wave_cls[w];
+    if (off == KP_SKIP) continue;   // uniform: a task without a plan to evaluate
+    const ClassView cv = class_view(L.pool + off);
+    kp_sync();   // the previous plan of this wavefront is done with LDS
+    uint32_t head = 0u;
+    if (!L.dur) {
+      head = kp_load_plan(L, pi, 0u, L.P->st[cv.h->structure].n_vertex, threadIdx.x, (int16_t*)kp_lds);
+      kp_sync();
+    }
+    kp_eval_plan<TR, 1>(L, w, pi, 0, head, cv, kp_lds, shared);
+  }
+}
+
+// One plan per block of four wavefronts, block by block in order (no perm): launches of at most four blocks per compute
+// unit, and the only kernel that reads plan records and sets done flags.
+template <int TR>
+__global__ __launch_bounds__(4 * WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_plan_block(const EvalLaunch L) {
+  extern __shared__ uint8_t kp_lds[];
+  __shared__ KpShared shared;
+  const uint64_t w = blockIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+  if (wave == 0) {
     uint32_t rec = 0u, off;
     if (L.rec) {
       rec = L.rec[w * (KE_REC_BYTES / 4) + (threadIdx.x & (KE_REC_BYTES / 4 - 1))];
@@ -425,18 +448,35 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) vo
     } else {
       off = L.wave_cls[w];
     }
-    if (off == KP_SKIP) continue;   // uniform: a task without a plan to evaluate
-    kp_eval_plan<TR>(L, w, pi, rec, class_view(L.pool + off), kp_lds);
-    // (lane 0 wrote the outputs of the task: its release store orders them before the flag)
-    if (L.done && threadIdx.x == 0) __hip_atomic_store(&L.done[w], L.done_tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    const int nv = !L.rec && off != KP_SKIP ? L.P->st[class_view(L.pool + off).h->structure].n_vertex : 0;
+    const uint32_t head = kp_load_plan(L, w, rec, nv, threadIdx.x, (int16_t*)kp_lds);
+    if (threadIdx.x == 0) {
+      shared.err = 0u;
+      shared.head = head;
+      shared.off = off;
+    }
   }
+  __syncthreads();
+  const uint32_t off = kp_scalar(shared.off), head = kp_scalar(shared.head);
+  if (off == KP_SKIP) return;   // uniform: a task without a plan to evaluate
+  kp_eval_plan<TR, 4>(L, w, w, wave, head, class_view(L.pool + off), kp_lds, shared);
+  // (wavefront 0 wrote the outputs of the task: its release store orders them before the flag)
+  if (L.done && threadIdx.x == 0) __hip_atomic_store(&L.done[w], L.done_tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// The launch of k_plan that keeps as much of the schedule as its outputs need.
-static void launch_plan(unsigned grid, size_t lds, hipStream_t s, const EvalLaunch& L) {
-  if (L.util || L.trace) hipLaunchKernelGGL(k_plan<KP_TIMES_ORDER>, dim3(grid), dim3(WAVE), lds, s, L);
-  else if (L.mass) hipLaunchKernelGGL(k_plan<KP_TIMES>, dim3(grid), dim3(WAVE), lds, s, L);
-  else hipLaunchKernelGGL(k_plan<KP_NO_TRACE>, dim3(grid), dim3(WAVE), lds, s, L);
+// The launch of k_plan that keeps as much of the schedule as its outputs need.  Up to four plans per compute unit get four
+// wavefronts each: at 128 registers a compute unit holds sixteen.
+template <int TR>
+static void launch_plan_tr(size_t lds, hipStream_t s, const EvalLaunch& L, int n_cu) {
+  if (L.rec || (!L.dur && !L.perm && L.n_waves <= 4ull * (uint64_t)n_cu))
+    hipLaunchKernelGGL(k_plan_block<TR>, dim3((unsigned)L.n_waves), dim3(4 * WAVE), lds, s, L);
+  else
+    hipLaunchKernelGGL(k_plan<TR>, dim3((unsigned)std::min<uint64_t>(L.n_waves, (uint64_t)n_cu * 32)), dim3(WAVE), lds, s, L);
+}
+static void launch_plan(size_t lds, hipStream_t s, const EvalLaunch& L, int n_cu) {
+  if (L.util || L.trace) launch_plan_tr<KP_TIMES_ORDER>(lds, s, L, n_cu);
+  else if (L.mass) launch_plan_tr<KP_TIMES>(lds, s, L, n_cu);
+  else launch_plan_tr<KP_NO_TRACE>(lds, s, L, n_cu);
 }
 
 // Generic single-wavefront kernel over the host/device-shared scheduler template; used for the
@@ -1372,7 +1412,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     L.mass = mass; L.prof = nullptr;
     const size_t lds = kp_lds_bytes(e->max_nodes, e->max_slots);
     if (e->timing) HIP_TRY(e, hipEventRecord(e->ev0, s));
-    launch_plan((unsigned)std::min<uint64_t>(n, (uint64_t)e->n_cu * 32), lds, s, L);
+    launch_plan(lds, s, L, e->n_cu);
     HIP_TRY(e, hipGetLastError());
     if (e->timing) HIP_TRY(e, hipEventRecord(e->ev1, s));
     HIP_TRY(e, hipMemcpyAsync(e->h_ccount, d_unknown, 4, hipMemcpyDeviceToHost, s));
@@ -2028,7 +2068,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   };
   auto launch_main = [&]() {
     if (n_waves == 0) {
-    } else if (one) launch_plan(grid, lds, sm, L);
+    } else if (one) launch_plan(lds, sm, L, e->n_cu);
     else switch (ls) {
       case 0: hipLaunchKernelGGL(k_eval<0>, dim3(grid), dim3(WAVE), lds, sm, L); break;
       case 8: hipLaunchKernelGGL(k_eval<8>, dim3(grid), dim3(WAVE), lds, sm, L); break;
@@ -2060,7 +2100,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     S.wave_cls = e->d_cls + n_host_tasks;
     S.n_waves = n_solo;
     if (L.prof) S.prof = L.prof + (n_waves + n_quad_waves) * 8;
-    launch_plan((unsigned)std::min<uint64_t>(n_solo, (uint64_t)e->n_cu * 32), kp_lds_bytes(e->max_nodes, e->max_slots), e->s2, S);
+    launch_plan(kp_lds_bytes(e->max_nodes, e->max_slots), e->s2, S, e->n_cu);
     HIP_TRY(e, hipGetLastError());
   }
   if (peaks_deferred) {
@@ -2209,7 +2249,7 @@ int rpeg_eval_batch_static(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   L.flags = flags & RPEG_GATE_STALE; L.makespan = makespan; L.peak = peak; L.score = score; L.mask = mask;
   L.mass = nullptr; L.prof = nullptr;
   const size_t lds = kp_lds_bytes(e->max_nodes, e->max_slots);
-  launch_plan((unsigned)std::min<uint64_t>(n, (uint64_t)e->n_cu * 32), lds, s, L);
+  launch_plan(lds, s, L, e->n_cu);
   HIP_TRY(e, hipGetLastError());
   e->stats[0] = 0; e->stats[1] = 0; e->stats[2] = n; e->stats[3] = lds; e->stats[4] = 0; e->stats[5] = 1; e->stats[6] = 0;
   e->stats[7] = 0;
@@ -2587,10 +2627,9 @@ int host_small_submit(rpeg_engine_t* e, HostLane& ln, uint64_t n, GET get, uint3
   L.done = (uint32_t*)ln.out_dev;
   L.done_tag = ln.tag;
   const size_t lds = kp_lds_bytes(e->max_nodes, e->max_slots);
-  const unsigned grid = (unsigned)std::min<uint64_t>(m, (uint64_t)e->n_cu * 32);
   e->stats[3] = lds;
   if (e->timing) HIP_TRY(e, hipEventRecord(e->ev0, s));
-  launch_plan(grid, lds, s, L);
+  launch_plan(lds, s, L, e->n_cu);
   HIP_TRY(e, hipGetLastError());
   if (e->timing) HIP_TRY(e, hipEventRecord(e->ev1, s));
   ln.launched = true;

@@ -41,34 +41,45 @@ __host__ __device__ inline size_t kp_lds_bytes(uint32_t nodes, uint32_t slots) {
 
 #if defined(__HIPCC__)
 
-// Critical-chain mass per template vertex (critical_mass of rpeg_class.h; moves.py:590-642) for one plan per
-// wavefront.  What the walk needs at a node -- the predecessor it goes on to (the first one, in edge order, of largest
-// finish time) and the vertex the node counts for -- is found for all nodes at once, a node per lane, and left in
-// LDS; the walk itself, one hop after the other from the first node of largest finish time, then reads LDS only.
+// Critical-chain mass per template vertex (critical_mass of rpeg_class.h; moves.py:590-642) for one plan.  What the walk
+// needs at a node -- the predecessor it goes on to (the first one, in edge order, of largest finish time) and the vertex
+// the node counts for -- is found for all nodes at once, a node per lane, and left in LDS; the walk itself, one hop after
+// the other from the first node of largest finish time, then reads LDS only.  KpHop: what the class says of a node,
+// which a wavefront that has nothing else to do fetches while the plan is scheduled.
+struct KpHop {
+  uint32_t begin = 0, end = 0, first = 0, vx = 0xFF;   // predecessors, the first of them; vertex
+};
+__device__ inline KpHop kp_hop_of(const ClassView& cv, int v) {
+  KpHop p;
+  p.begin = cv.pbeg[v]; p.end = cv.pbeg[v + 1];
+  p.first = cv.pred[p.begin < p.end ? p.begin : 0];
+  const SlotDesc sd = cv.slot[cv.node[v].slot];
+  p.vx = sd.type <= SLOT_OP_SUB ? sd.a : 0xFFu;
+  return p;
+}
+__device__ inline void kp_hop(const ClassView& cv, int v, const KpHop& p, const double* l_fin, uint16_t* l_next, uint8_t* l_vx) {
+  uint32_t nx = 0xFFFFu;
+  if (p.begin != p.end) {
+    nx = p.first;
+    double b = l_fin[nx];
+    for (uint32_t j = p.begin + 1; j < p.end; ++j) {
+      const uint32_t q = cv.pred[j];
+      const double fq = l_fin[q];
+      if (fq > b) { b = fq; nx = q; }
+    }
+  }
+  l_next[v] = (uint16_t)nx;
+  l_vx[v] = (uint8_t)p.vx;
+}
 // Lane x < RPEG_MAX_V returns the mass of vertex x, summed in the order of the walk.
-__device__ inline double kp_critical_mass(const ClassView& cv, const int n, const int lane, const double* l_fin,
-                                          const double* l_start, uint16_t* l_next, uint8_t* l_vx) {
+__device__ inline double kp_critical_mass(const int n, const int lane, const double* l_fin, const double* l_start,
+                                          const uint16_t* l_next, const uint8_t* l_vx) {
   double bf = -1.0;
   uint32_t bi = 0xFFFFFFFFu;
   for (int v = lane; v < n; v += KE_WAVE) {
     const double f = l_fin[v];
     if (f > bf) { bf = f; bi = (uint32_t)v; }
-    const int pb = cv.pbeg[v], pe = cv.pbeg[v + 1];
-    uint32_t nx = 0xFFFFu;
-    if (pb != pe) {
-      nx = cv.pred[pb];
-      double b = l_fin[nx];
-      for (int j = pb + 1; j < pe; ++j) {
-        const uint32_t q = cv.pred[j];
-        const double fq = l_fin[q];
-        if (fq > b) { b = fq; nx = q; }
-      }
-    }
-    l_next[v] = (uint16_t)nx;
-    const SlotDesc sd = cv.slot[cv.node[v].slot];
-    l_vx[v] = sd.type <= SLOT_OP_SUB ? sd.a : (uint8_t)0xFF;
   }
-  __syncthreads();
   const double top = kp_wave_reduce(bf, KpMax());
   int cur = (int)kp_wave_umin(bf == top ? bi : 0xFFFFFFFFu);
   double m = 0.0;
@@ -227,7 +238,7 @@ __device__ inline double kp_utilization(const ClassView& cv, const int n, const 
     if (open) merged += ce - cs;
     l_tab[lane] = merged / ms;
   }
-  __syncthreads();
+  kp_sync();
   // vertices by first reservation, four bits each
   uint32_t order = 0u;
   int n_ev = 0;
@@ -293,17 +304,99 @@ __device__ inline double kp_utilization(const ClassView& cv, const int n, const 
   return count ? total / (double)count : 0.0;
 }
 
-// One plan, evaluated by the whole wavefront.  pi: plan index (uniform).  rec: lane l < 32 holds word l of the plan's
-// record where the launch has records.  TR (KpTrace): what the outputs of the launch
-// need of the schedule -- nothing, the times for L.mass, the dispatch order too for L.util.
-template <int TR>
-__device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const uint64_t pi, const uint32_t rec,
-                                    const ClassView cv, uint8_t* lds) {
-  const int lane = threadIdx.x;
+// What wavefront 3 of a block finds out while the others go on, and flags of the durations.
+struct KpShared {
+  double peak, pen;
+  uint32_t gates;      // RPEG_MASK_STALE_OK | RPEG_MASK_MEM_OK
+  uint32_t err;        // bit w: wavefront w met a node the reference raises for
+  uint32_t head, off;  // of the plan's record
+};
+
+// The fields of plan pi into LDS, by one wavefront: header bytes (structure, split, tau0, tau1).  rec: lane l < 32 holds
+// word l of the plan's record where the launch has records.
+__device__ inline uint32_t kp_load_plan(const EvalLaunch& L, const uint64_t pi, const uint32_t rec, const int nv, const int lane,
+                                        int16_t* l_plan) {
+  if (L.rec) {
+    if (lane < KP_PLAN_I16 / 2) ((uint32_t*)l_plan)[lane] = lane < RPEG_MAX_V * RPEG_FIELDS / 2 ? rec : 0x00010001u;
+    return (uint32_t)__builtin_amdgcn_readlane((int)rec, RPEG_MAX_V * RPEG_FIELDS / 2);
+  }
+  for (int x = lane; x < KP_PLAN_I16; x += KE_WAVE) l_plan[x] = x < nv * RPEG_FIELDS ? L.vert[(uint64_t)x * L.stride + pi] : (int16_t)1;
+  const uint32_t b = L.head[(uint64_t)(lane & 3) * L.stride + pi];
+  return (uint32_t)__builtin_amdgcn_readlane((int)b, 0) | (uint32_t)__builtin_amdgcn_readlane((int)b, 1) << 8 |
+         (uint32_t)__builtin_amdgcn_readlane((int)b, 2) << 16 | (uint32_t)__builtin_amdgcn_readlane((int)b, 3) << 24;
+}
+
+// Memory model (memory.py:608-841) of the plan, by one wavefront, in the order of first appearance of the vertices among
+// the lowered operator nodes (position i = vertex vorder[i]): that order fixes the order of the float sums.
+// One vertex per lane (kp_memory_vertices), then one vertex subset per lane tests whether it is a device class (a maximal
+// clique of the overlap graph); the few that are get evaluated one after the other with uniform control flow.
+__device__ inline KpOrdered kp_memory_vertices(const rpeg_problem_t& P, const rpeg_struct_t& st, const ClassView& cv, const int lane,
+                                               const int16_t* l_plan, double* l_vm) {
+  const int nv = st.n_vertex;
+  const uint8_t* order = cv.h->vorder;
+  const bool coresident = struct_coresident(st);
+  if (lane < nv) {
+    const int v = order[lane];
+    const VMem m = vertex_memory(P, st.vertex[v], ke_vplan<1>(l_plan, v), coresident);
+    l_vm[lane * 4 + 0] = (double)m.w_shard;
+    l_vm[lane * 4 + 1] = m.mem_w;
+    l_vm[lane * 4 + 2] = m.opt;
+    l_vm[lane * 4 + 3] = m.extra;
+  }
+  KpOrdered om;
+  const int i = lane >> 3, j = lane & 7;
+  const bool valid = i < nv && j < nv;
+  const int vi = order[valid ? i : 0], vj = order[valid ? j : 0];
+  const VPlan ai = ke_vplan<1>(l_plan, vi), aj = ke_vplan<1>(l_plan, vj);
+  const rpeg_vertex_t &xi = st.vertex[vi], &xj = st.vertex[vj];
+  om.ovl = __ballot(valid && !alloc_disjoint(ai, aj));
+  om.eq = __ballot(valid && alloc_equal(ai, aj));
+  om.same_model = __ballot(valid && xi.model == xj.model);
+  om.train_same = __ballot(valid && xi.model == xj.model && xj.role == RPEG_ROLE_TRAIN);
+  const unsigned long long t = __ballot(valid && j == 0 && xi.role == RPEG_ROLE_TRAIN),
+                           tr = __ballot(valid && j == 0 && st.mem_trainable[xi.model] != 0);   // bit 8i: position i
+  om.train = om.trainable = 0u;
+  om.coresident = coresident;
+#pragma unroll
+  for (int q = 0; q < RPEG_MAX_V; ++q) {
+    om.train |= (unsigned)((t >> (8 * q)) & 1ull) << q;
+    om.trainable |= (unsigned)((tr >> (8 * q)) & 1ull) << q;
+  }
+  return om;
+}
+__device__ inline double kp_memory_peak(const rpeg_problem_t& P, const rpeg_struct_t& st, const ClassView& cv, const int lane,
+                                        const KpOrdered& om, const double* l_vm) {
+  const int nv = st.n_vertex;
+  kp_sync();
+  double peak = -1.0;
+  const unsigned M = (unsigned)lane + 1u;
+  unsigned long long classes = __ballot(M < (1u << nv) && kp_maximal_clique(nv, om.ovl, M));
+  while (classes) {
+    const unsigned Mu = (unsigned)__builtin_ctzll(classes) + 1u;
+    classes &= classes - 1ull;
+    const double p = kp_class_peak(P, st, cv.h->vorder, nv, om, l_vm, Mu);
+    peak = p > peak ? p : peak;
+  }
+  return peak;
+}
+
+// One plan, evaluated by NW wavefronts (this is number `wave`).  pi: plan index (uniform).  head: its header bytes, with
+// its fields in LDS.  TR (KpTrace): what the outputs of the launch need of the schedule -- nothing, the times for
+// L.mass, the dispatch order too for L.util and L.trace.
+//
+// NW = 4, for launches whose plans all find a place at once: what one wavefront does one after the other for 13 us before
+// its first rank is known is shared out by kind -- generation, other operators, transfers, the memory model -- because
+// the kinds are branches of divergent code that a single wavefront walks through in turn; all four count positions; and
+// three fetch what the critical chain needs of the class while the first one schedules.
+// Measured, 150 PPO plans (K = 4) in one launch: to the first rank 14.7 -> 4.7 us, positions 5.6 -> 4.9 (300 nodes: 34 ->
+// 14.5), a plan 73 -> 61 us on average, the launch 128 -> 110 us.
+template <int TR, int NW>
+__device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const uint64_t pi, const int wave, const uint32_t head,
+                                    const ClassView cv, uint8_t* lds, KpShared& shared) {
+  const int lane = (int)__lane_id();
   const rpeg_problem_t& P = *L.P;
   const int n = (int)cv.h->n_nodes, n_slots = (int)cv.h->n_slots;
-  int first_lane = 0;
-  (void)first_lane;
+  const int first_lane = NW == 1 || wave == 0 ? 0 : -1;
 
   int16_t* l_plan = (int16_t*)lds;
   double* l_vm = (double*)(lds + KP_PLAN_I16 * 2);
@@ -319,8 +412,9 @@ __device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const
   uint16_t* l_ord = (uint16_t*)l_at;
   uint16_t* l_next = l_ord + L.ws_nodes;
   uint8_t* l_pt = (uint8_t*)l_q;
+  const KpLds M{(const KP_LDS double*)l_dur, (KP_LDS LevelRec*)l_rec, (KP_LDS double*)l_rank, (KP_LDS double*)l_start,
+                (KP_LDS uint32_t*)l_at, (KP_LDS uint16_t*)l_q, (KP_LDS uint16_t*)l_ord, (KP_LDS uint16_t*)l_next, (KP_LDS uint8_t*)l_pt};
 
-  __syncthreads();   // the previous plan of this wavefront is done with LDS
   KE_STAMP(0);
   const rpeg_struct_t& st = P.st[cv.h->structure];
   const int nv = st.n_vertex;
@@ -328,7 +422,7 @@ __device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const
   pm.ovl = pm.eq = pm.dpne = 0;
   bool err = cv.h->error != 0, stale_ok = false, mem_ok = false;
   double peak = -1.0, pen = 1.0;
-  if (L.dur) {
+  if (NW == 1 && L.dur) {
     // a task of a laid-out batch: the prologue launches have left the durations of the slot universe, the pair
     // relations, the penalty factor and the gate bits by plan index (and written the peak themselves)
     const uint64_t sp = pi;
@@ -345,21 +439,14 @@ __device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const
     const uint8_t gates = L.aux_mask ? L.aux_mask[sp] : (uint8_t)(RPEG_MASK_VALID | RPEG_MASK_STALE_OK | RPEG_MASK_MEM_OK);
     stale_ok = (gates & RPEG_MASK_STALE_OK) != 0;
     mem_ok = (gates & RPEG_MASK_MEM_OK) != 0;
-    __syncthreads();
+    kp_stage((const uint8_t*)cv.h, M);
+    kp_sync();
     KE_STAMP(1);
     KE_STAMP(2);
   } else {
     PlanHead h;
-    if (L.rec) {
-      const uint32_t hw = (uint32_t)__builtin_amdgcn_readlane((int)rec, RPEG_MAX_V * RPEG_FIELDS / 2);
-      h.structure = (int)(hw & 0xFFu); h.split = (int)((hw >> 8) & 0xFFu);
-      h.tau0 = (int)((hw >> 16) & 0xFFu); h.tau1 = (int)(hw >> 24);
-      if (lane < KP_PLAN_I16 / 2) ((uint32_t*)l_plan)[lane] = lane < RPEG_MAX_V * RPEG_FIELDS / 2 ? rec : 0x00010001u;
-    } else {
-      h = load_head(L.head, L.stride, pi);
-      if (lane < KP_PLAN_I16) l_plan[lane] = lane < nv * RPEG_FIELDS ? L.vert[(uint64_t)lane * L.stride + pi] : (int16_t)1;
-    }
-    __syncthreads();
+    h.structure = (int)(head & 0xFFu); h.split = (int)((head >> 8) & 0xFFu);
+    h.tau0 = (int)((head >> 16) & 0xFFu); h.tau1 = (int)(head >> 24);
 
     // ---- pair relations: lane 8u+v tests vertices u and v, the ballots are the masks
     {
@@ -367,75 +454,72 @@ __device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const
       const bool valid = u < nv && v < nv;
       const VPlan au = ke_vplan<1>(l_plan, valid ? u : 0), av = ke_vplan<1>(l_plan, valid ? v : 0);
       pm.ovl = __ballot(valid && !alloc_disjoint(au, av));
-      pm.eq = 0;   // the memory model below works on position-indexed masks of its own
+      pm.eq = 0;   // the memory model works on position-indexed masks of its own
       pm.dpne = __ballot(valid && au.dp != av.dp);
     }
 
     // ---- durations of the class's slots, one slot per lane
-    bool zero_div = false;
-    const int split = (int)cv.h->split;
-    for (int s = lane; s < n_slots; s += KE_WAVE) l_dur[s] = ke_slot_duration<1>(P, st, split, cv.slot[s], l_plan, &zero_div);
-    err = err || __ballot(zero_div) != 0ull;
-    KE_STAMP(1);
-
-    // ---- memory model (memory.py:608-841), in the order of first appearance of the vertices among the
-    // lowered operator nodes (position i = vertex vorder[i]): that order fixes the order of the float sums.
-    // One vertex per lane, then one vertex subset per lane tests whether it is a device class (a maximal clique
-    // of the overlap graph); the few that are get evaluated one after the other with uniform control flow.
-    const uint8_t* order = cv.h->vorder;
-    const bool coresident = struct_coresident(st);
-    if (lane < nv) {
-      const int v = order[lane];
-      const VMem m = vertex_memory(P, st.vertex[v], ke_vplan<1>(l_plan, v), coresident);
-      l_vm[lane * 4 + 0] = (double)m.w_shard;
-      l_vm[lane * 4 + 1] = m.mem_w;
-      l_vm[lane * 4 + 2] = m.opt;
-      l_vm[lane * 4 + 3] = m.extra;
+    if (NW == 1 || wave < 3) {
+      bool zero_div = false;
+      const int split = (int)cv.h->split;
+      for (int s = lane; s < n_slots; s += KE_WAVE) {
+        const SlotDesc sd = cv.slot[s];
+        if (NW > 1) {
+          const int mine = sd.type > SLOT_OP_SUB ? 2 : st.vertex[sd.a].role == RPEG_ROLE_GEN ? 0 : 1;
+          if (mine != wave) continue;
+        }
+        l_dur[s] = ke_slot_duration<1>(P, st, split, sd, l_plan, &zero_div);
+      }
+      const bool bad = __ballot(zero_div) != 0ull;
+      if (NW == 1) err = err || bad;
+      else if (bad && lane == 0) atomicOr(&shared.err, 1u);
     }
+    if (NW == 1 || wave == 2) kp_stage((const uint8_t*)cv.h, M);
     KpOrdered om;
-    {
-      const int i = lane >> 3, j = lane & 7;
-      const bool valid = i < nv && j < nv;
-      const int vi = order[valid ? i : 0], vj = order[valid ? j : 0];
-      const VPlan ai = ke_vplan<1>(l_plan, vi), aj = ke_vplan<1>(l_plan, vj);
-      const rpeg_vertex_t &xi = st.vertex[vi], &xj = st.vertex[vj];
-      om.ovl = __ballot(valid && !alloc_disjoint(ai, aj));
-      om.eq = __ballot(valid && alloc_equal(ai, aj));
-      om.same_model = __ballot(valid && xi.model == xj.model);
-      om.train_same = __ballot(valid && xi.model == xj.model && xj.role == RPEG_ROLE_TRAIN);
-      const unsigned long long t = __ballot(valid && j == 0 && xi.role == RPEG_ROLE_TRAIN),
-                               tr = __ballot(valid && j == 0 && st.mem_trainable[xi.model] != 0);   // bit 8i: position i
-      om.train = om.trainable = 0u;
-      om.coresident = coresident;
-#pragma unroll
-      for (int q = 0; q < RPEG_MAX_V; ++q) {
-        om.train |= (unsigned)((t >> (8 * q)) & 1ull) << q;
-        om.trainable |= (unsigned)((tr >> (8 * q)) & 1ull) << q;
+    if (NW == 1 || wave == 3) om = kp_memory_vertices(P, st, cv, lane, l_plan, l_vm);
+    kp_barrier<NW>();
+    KE_STAMP(1);
+    if (NW > 1) err = err || shared.err != 0u;
+    if (NW == 1 || wave == 3) {
+      peak = kp_memory_peak(P, st, cv, lane, om, l_vm);
+      stale_ok = stale_layout_ok(st, h, pm.ovl);
+      mem_ok = !(peak > P.cap);
+      if (!mem_ok) pen = oom_penalty(peak, P.cap);
+      if (NW > 1 && lane == 0) {
+        shared.peak = peak;
+        shared.pen = pen;
+        shared.gates = (stale_ok ? RPEG_MASK_STALE_OK : 0u) | (mem_ok ? RPEG_MASK_MEM_OK : 0u);
       }
     }
-    __syncthreads();
-    {
-      const unsigned M = (unsigned)lane + 1u;
-      unsigned long long classes = __ballot(M < (1u << nv) && kp_maximal_clique(nv, om.ovl, M));
-      while (classes) {
-        const unsigned Mu = (unsigned)__builtin_ctzll(classes) + 1u;
-        classes &= classes - 1ull;
-        const double p = kp_class_peak(P, st, order, nv, om, l_vm, Mu);
-        peak = p > peak ? p : peak;
-      }
-    }
-    stale_ok = stale_layout_ok(st, h, pm.ovl);
-    mem_ok = !(peak > P.cap);
-    if (!mem_ok) pen = oom_penalty(peak, P.cap);
     KE_STAMP(2);
   }
-  unsigned long long* stamp = L.prof && lane == 0 ? L.prof + w * 8 : nullptr;
+  unsigned long long* stamp = L.prof && lane == first_lane ? L.prof + w * 8 : nullptr;
 
-  // ---- ranks and list scheduling
+  // ---- ranks, positions and list scheduling
   double makespan = 0.0;
+  if (!err && (NW == 1 || wave == 0)) kp_ranks((uint64_t)cv.h, M);
+  kp_barrier<NW>();
+  if (stamp) stamp[3] = wall_clock64();
+  if (!err) kp_positions<NW>((uint64_t)cv.h, wave, M);
+  if (NW > 1 && wave == 0) {
+    peak = shared.peak;
+    pen = shared.pen;
+    stale_ok = (shared.gates & RPEG_MASK_STALE_OK) != 0u;
+    mem_ok = (shared.gates & RPEG_MASK_MEM_OK) != 0u;
+  }
+  const bool chain = TR != KP_NO_TRACE && L.mass && !err;   // (uniform over the wavefronts, also where there is no schedule)
+  if (NW > 1 && wave != 0) {
+    if (!chain) return;
+    const int v0 = (wave - 1) * KE_WAVE + lane;
+    KpHop hop;
+    if (v0 < n) hop = kp_hop_of(cv, v0);
+    __syncthreads();   // the plan is scheduled
+    if (v0 < n) kp_hop(cv, v0, hop, l_rank, l_next, l_pt);
+    for (int v = v0 + (NW - 1) * KE_WAVE; v < n; v += (NW - 1) * KE_WAVE) kp_hop(cv, v, kp_hop_of(cv, v), l_rank, l_next, l_pt);
+    __syncthreads();
+    return;
+  }
   if (!err) {
-    const KpLds M{(const KP_LDS double*)l_dur, (KP_LDS LevelRec*)l_rec, (KP_LDS double*)l_rank, (KP_LDS double*)l_start,
-                  (KP_LDS uint32_t*)l_at, (KP_LDS uint16_t*)l_q, (KP_LDS uint16_t*)l_ord, (KP_LDS uint16_t*)l_next, (KP_LDS uint8_t*)l_pt};
     makespan = kp_schedule<TR>((const uint8_t*)cv.h, n, pm.ovl, pm.dpne, M, stamp);
     err = makespan < 0.0;
   }
@@ -457,8 +541,8 @@ __device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const
     out_makespan = makespan;
     out_score = score;
   }
+  kp_sync();
   if (TR == KP_TIMES_ORDER && L.trace && !err) {
-    __syncthreads();
     double* const t = L.trace;
     uint16_t* const d = (uint16_t*)(t + 2 * (size_t)L.ws_nodes);
     for (int i = lane; i < n; i += KE_WAVE) {
@@ -467,15 +551,20 @@ __device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const
       d[i] = l_ord[i];
     }
   }
-  double m = __builtin_nan("");   // lane x < RPEG_MAX_V: mass of vertex x
-  if (TR != KP_NO_TRACE && L.mass) {
-    __syncthreads();
-    if (!err) m = kp_critical_mass(cv, n, lane, l_rank, l_start, l_next, l_pt);
-  }
   double util = 0.0;
-  if (TR == KP_TIMES_ORDER && L.util) {
-    __syncthreads();
+  if (TR == KP_TIMES_ORDER && L.util)
     util = err ? __builtin_nan("") : kp_utilization(cv, n, lane, nv, l_plan, pm.dpne, l_start, l_rank, l_ord, l_tab, makespan);
+  double m = __builtin_nan("");   // lane x < RPEG_MAX_V: mass of vertex x
+  if (chain) {
+    if (NW > 1) {
+      __syncthreads();
+      __syncthreads();   // (the others leave what the walk needs at every node)
+    } else {
+      kp_sync();
+      for (int v = lane; v < n; v += KE_WAVE) kp_hop(cv, v, kp_hop_of(cv, v), l_rank, l_next, l_pt);
+      kp_sync();
+    }
+    if (!err) m = kp_critical_mass(n, lane, l_rank, l_start, l_next, l_pt);
   }
   if (lane == 0) {
     if (TR == KP_TIMES_ORDER && L.util) L.util[pi] = util;

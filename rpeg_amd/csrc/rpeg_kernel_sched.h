@@ -1,8 +1,9 @@
 // rpeg_kernel_sched.h - the list scheduler of the one-plan-per-wavefront kernel (device only).
 //
-// A wavefront schedules one plan.  Three parts, functions of their own (inside the kernel the register allocator would
+// A wavefront schedules one plan.  Its parts, functions of their own (inside the kernel the register allocator would
 // have to find room for them among the launch record and the cost model, and spill in their loops):
-//   kp_order        ranks of the lowered nodes, and from them every node's position in the order that breaks ties
+//   kp_ranks        ranks of the lowered nodes
+//   kp_positions    from them every node's position in the order that breaks ties
 //   kp_lanes        the scheduler for graphs of at most 128 nodes: every node has a lane of its own
 //   kp_list         the scheduler for larger graphs: every waiting node has a lane, the others live in LDS
 //   kp_plain        the textbook form, for a graph whose waiting nodes outgrow a wavefront in kp_list
@@ -149,8 +150,18 @@ struct KpClass {
   __device__ const KP_CONST T* at(uint32_t off) const { return (const KP_CONST T*)(base + off); }
   __device__ const KP_CONST ClassHdr* hdr() const { return at<ClassHdr>(0); }
 };
-// wavefronts of one per block: what one lane wrote to LDS another may read
-__device__ inline void kp_sync() { __syncthreads(); }
+// within a wavefront: what one lane wrote to LDS another may read (a wavefront's LDS instructions execute in order)
+__device__ inline void kp_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// NW wavefronts work on a plan: with one the barrier is kp_sync
+template <int NW>
+__device__ inline void kp_barrier() {
+  if (NW == 1) kp_sync();
+  else __syncthreads();
+}
 
 // Places of the fifth successor on of the node at level place `at`.
 template <class VISIT>
@@ -177,18 +188,22 @@ __device__ inline uint32_t kp_reserved(uint32_t blocked, uint32_t cond, uint64_t
   return b | (touch << 8);
 }
 
-// Ranks and positions.  The class's level records go to LDS first.
-__device__ __attribute__((noinline)) void kp_order(uint64_t blob, const KpLds M, unsigned long long* stamp) {
+// The class's level records go to LDS.
+__device__ inline void kp_stage(const uint8_t* blob, const KpLds& M) {
+  const int lane = (int)__lane_id();
+  const KpClass T{kp_scalar64((uint64_t)blob)};
+  const KP_CONST ClassHdr* h = T.hdr();
+  const int n = (int)h->n_nodes;
+  const KP_CONST uint4* src = T.at<uint4>(h->off_lrec);
+  for (int v = lane; v < n; v += KE_WAVE) ((KP_LDS uint4*)M.rec)[v] = src[v];
+}
+
+// Ranks.
+__device__ __attribute__((noinline)) void kp_ranks(uint64_t blob, const KpLds M) {
   const int lane = (int)__lane_id();
   const KpClass T{kp_scalar64(blob)};
   const KP_CONST ClassHdr* h = T.hdr();
   const int n = (int)h->n_nodes, n_levels = (int)h->n_levels;
-  const KP_CONST uint64_t* orec = T.at<uint64_t>(h->off_orec);
-  uint64_t oword = orec[lane < n ? lane : 0];   // the records by tie-break class: the first ones on their way from here on
-  {
-    const KP_CONST uint4* src = T.at<uint4>(h->off_lrec);
-    for (int v = lane; v < n; v += KE_WAVE) ((KP_LDS uint4*)M.rec)[v] = src[v];
-  }
   if (lane == 0) M.rank[n] = 0.0;
   kp_sync();
 
@@ -241,21 +256,32 @@ __device__ __attribute__((noinline)) void kp_order(uint64_t blob, const KpLds M,
     }
   }
   kp_sync();
-  if (stamp) stamp[3] = wall_clock64();
+}
 
-  // ---- positions: within its tie-break class a node comes behind those of larger rank.  Nodes that agree are told apart
-  // by their place in the order; `shared` where they are more than the node's own chain.
+// Positions: within its tie-break class a node comes behind those of larger rank.  Nodes that agree are told apart by
+// their place in the order; `shared` where they are more than the node's own chain.  NW wavefronts share the nodes (the
+// counting is a pass over the class for each: 34 us of one wavefront's time on a graph of 300 nodes).
+template <int NW>
+__device__ __attribute__((noinline)) void kp_positions(uint64_t blob, int wave, const KpLds M) {
+  const int first = wave * KE_WAVE + (int)__lane_id();
+  constexpr int STEP = NW * KE_WAVE;
+  const KpClass T{kp_scalar64(blob)};
+  const KP_CONST ClassHdr* h = T.hdr();
+  const int n = (int)h->n_nodes;
+  const KP_CONST uint64_t* orec = T.at<uint64_t>(h->off_orec);
+  const uint64_t w0 = orec[first < n ? first : 0];   // the records by tie-break class
   {
-    uint64_t w = oword;
-    for (int p = lane; p - lane < n; p += KE_WAVE) {
-      const uint64_t next = orec[p + KE_WAVE < n ? p + KE_WAVE : 0];
-      if (p < n) M.rk[p] = M.rank[w & 0xFFFFu];
+    uint64_t w = w0;
+    for (int p = first; p < n; p += STEP) {
+      const uint64_t next = orec[p + STEP < n ? p + STEP : 0];
+      M.rk[p] = M.rank[w & 0xFFFFu];
       w = next;
     }
   }
-  kp_sync();
-  for (int p = lane; p - lane < n; p += KE_WAVE) {
-    const uint64_t next = orec[p + KE_WAVE < n ? p + KE_WAVE : 0];
+  kp_barrier<NW>();
+  uint64_t oword = w0;
+  for (int p = first; p - (int)__lane_id() < n; p += STEP) {
+    const uint64_t next = orec[p + STEP < n ? p + STEP : 0];
     const bool ok = p < n;
     const double rk = M.rk[ok ? p : 0];
     const int b0 = (int)((oword >> 16) & 0xFFFFu), b1 = ok ? (int)((oword >> 32) & 0xFFFFu) : b0;
@@ -287,8 +313,8 @@ __device__ __attribute__((noinline)) void kp_order(uint64_t blob, const KpLds M,
     }
     oword = next;
   }
-  if (lane == 0) M.q[n] = 0xFFFFu;
-  kp_sync();
+  if (first == 0) M.q[n] = 0xFFFFu;
+  kp_barrier<NW>();
 }
 
 // A graph of at most 64 * NS nodes: the nodes are dealt to the lanes by position (q: register slot q >> 6, lane q & 63),
@@ -926,11 +952,11 @@ __device__ __attribute__((noinline)) double kp_plain(uint64_t blob, uint64_t ovl
   return error ? -1.0 : ms;
 }
 
-// The schedule of a plan on this wavefront: makespan, or a negative number where there is none.
+// The schedule of a plan whose nodes have their positions, on this wavefront: makespan, or a negative number where there
+// is none.
 template <int TR>
 __device__ inline double kp_schedule(const uint8_t* blob, int n, uint64_t ovl, uint64_t dpne, const KpLds& M, unsigned long long* stamp) {
   const uint64_t b = (uint64_t)blob;
-  kp_order(b, M, stamp);
   if (n <= 64) return kp_lanes<1, TR>(b, ovl, dpne, M, stamp);
   if (n <= KP_LANE_NODES) return kp_lanes<2, TR>(b, ovl, dpne, M, stamp);
   const double ms = kp_list<TR>(b, ovl, dpne, M, stamp);
