@@ -467,18 +467,18 @@ int rpeg_engine_host_us(const rpeg_engine_t* e, double* out, int32_t n);
    layout: a batch too small to fill the chip finishes sooner); fails at the next call when the state
    of the problem's largest class does not fit.  lanes = 1: one plan per wavefront, its nodes spread
    over the lanes (the layout of lowest latency, for batches of a few thousand plans at most; classes of
-   up to 384 nodes).  lanes = 4: four lanes per plan, sixteen plans per wavefront, the ready entries (at most 32
-   at once; a plan with more is redone by the launch that ends the call) in the registers of the four lanes (the
-   layout for dense graphs, whose plan-per-lane wavefronts end last).
+   up to 384 nodes).  lanes = 4: two or four lanes per plan, 32 or 16 plans per wavefront, the ready
+   entries (at most 24 at once; a plan with more is redone by the launch that ends the call) in the registers of the
+   plan's lanes.
    lanes = -1 (default): chosen per batch from its size.
    Results do not depend on the setting. */
 int rpeg_engine_set_state_lanes(rpeg_engine_t* e, int32_t lanes);
 
 /* The nine fitted figures by which a full batch is split between the three scheduling kernels (microseconds of a
-   wavefront on an MI355X): cost of a plan in the one-plan-per-wavefront kernel a + b x nodes (40, 2.2); of a wavefront
-   of the four-lanes-per-plan kernel a + nodes x (b + c x heap pops per dispatch) (40, 1.6, 0.45); the share of the
-   modelled room that the former really gets beside the latter (0.65); how much later a class must end in the main
-   kernel to move to the four-lanes-per-plan kernel (1.15); the modelled gain that a split by class size (0.97) and by
+   wavefront on an MI355X): cost of a plan in the one-plan-per-wavefront kernel a + b x nodes (12, 0.9); of a wavefront
+   of the kernel of two or four lanes per plan a + nodes x (b + c x heap pops per dispatch) (10, 1.3, 0.2); the share of
+   a compute unit that the former really gets beside the latter (0.65); how much later the main kernel must end for a
+   batch to move to the kernel of two or four lanes per plan (1.15); the modelled gain that a split by class size (0.97) and by
    measured time (0.98) must reach.  A measurement aid: the figures decide where a plan is evaluated, never what
    the result is.  No counterpart in the reference. */
 int rpeg_engine_set_split_model(rpeg_engine_t* e, const double* values, int32_t n);
@@ -498,11 +498,12 @@ int rpeg_engine_set_sa_groups(rpeg_engine_t* e, int32_t groups);
    it.  No counterpart in the reference. */
 int rpeg_engine_set_side_layout(rpeg_engine_t* e, int32_t on);
 
-/* With lanes = -1 and a batch that fills the chip in one round of wavefronts: the largest share of the batch's
-   plans, in percent, that the four-lanes-per-plan kernel may take on a stream of its own (default 25; 0: none).
-   Which classes it takes is learned: the main kernel records, per class, how long its slowest wavefront ran and how
-   many heap pops per dispatch it needed, and from the second call on the classes that would end last there (dense
-   graphs) are moved.  Results do not depend on the setting.  No reference counterpart (a tuning knob). */
+/* With lanes = -1: whether full batches may run in the kernel of two or four lanes per plan (percent > 0, default 25;
+   0: no, and nothing that was measured decides where a class runs).  What it takes is learned: the main kernel records, per class,
+   how long its slowest wavefront ran, how many heap pops per dispatch it needed and the longest ready set, and from
+   the second call on a batch that would end earlier there moves, its smallest classes and largest graphs to the
+   one-plan-per-wavefront kernel beside it.  Results do not depend on the setting.  No reference counterpart (a tuning
+   knob). */
 int rpeg_engine_set_quad_share(rpeg_engine_t* e, int32_t percent);
 
 /* Ready-list entries per plan in the main kernel: 8, 16, 24 or 32 (default).  A plan with that many nodes

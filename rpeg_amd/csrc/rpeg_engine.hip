@@ -405,11 +405,15 @@ __global__ __launch_bounds__(WAVE) void k_eval(const EvalLaunch L) {
 }
 
 // Four lanes per plan, sixteen plans per wavefront (rpeg_kernel_quad.h); tasks and permutation as for k_eval.
-// At most 128 vector registers, so that a wavefront of it fits beside one of the main kernel and one of k_plan on a
-// SIMD (the cost model spills a little; the scheduling loop does not).
+// QL: lanes per plan; SL: ready entries per lane.
+struct QuadKind { uint32_t plans, entries; };
+constexpr QuadKind QUAD_KIND[3] = {{32, 8}, {16, 16}, {16, 24}};   // k_quad<2, 4>, <4, 4>, <4, 6>
+template <int QL, int SL>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_quad(const EvalLaunch L) {
   extern __shared__ uint8_t kq_lds[];
-  for (uint64_t w = blockIdx.x; w < L.n_waves; w += gridDim.x) kq_eval_wave(L, w, kq_lds);
+  const uint64_t w = blockIdx.x;
+  if (SL == 4 && QL == 4 && (L.wave_cls[w] & KE_CLS_LDS)) kq_eval_wave<QL, 2>(L, w, kq_lds);   // uniform branch
+  else kq_eval_wave<QL, SL>(L, w, kq_lds);
 }
 
 // One plan per wavefront (rpeg_kernel_plan.h); perm[w] is the plan of wavefront task w.  TR: KpTrace.
@@ -429,6 +433,18 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) vo
       kp_sync();
     }
     kp_eval_plan<TR, 1>(L, w, pi, 0, head, cv, kp_lds, shared);
+  }
+}
+
+// The plans on the list of those whose ready set outgrew their kernel (EvalLaunch::limit), one per wavefront.
+template <int TR>
+__global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_plan_limit(const EvalLaunch L) {
+  extern __shared__ uint8_t kp_lds[];
+  __shared__ KpShared shared;
+  const uint32_t n = kp_scalar(L.limit[0]);
+  for (uint32_t w = blockIdx.x; w < n; w += gridDim.x) {
+    kp_sync();   // the previous plan of this wavefront is done with LDS
+    kp_eval_plan<TR, 1>(L, w, kp_scalar(L.limit[1 + 2 * (size_t)w]), 0, 0u, class_view(L.pool + kp_scalar(L.limit[2 + 2 * (size_t)w])), kp_lds, shared);
   }
 }
 
@@ -669,15 +685,15 @@ static uint8_t* static_scratch_ptr(int dev, hipError_t* st) {
 //   plan_a + plan_b x nodes                    what a plan costs k_plan (one plan per wavefront), beside the main kernel;
 //                                              plan_list times as much beyond KP_LANE_NODES nodes, where its scheduler
 //                                              keeps the nodes in LDS and fewer of its wavefronts fit on a compute unit
-//   quad_a + nodes x (quad_b + quad_c x pops)  a wavefront of k_quad (sixteen plans); pops = heap pops per dispatch,
-//                                              as the main kernel measured them for the class
-//   eff_beside_quad                            the part of the modelled room beside the main kernel that k_plan really
-//                                              gets where k_quad takes its share of a compute unit too
-//   quad_margin                                a class moves to k_quad only if it ends this much later in the main kernel
+//   quad_a + nodes x (quad_b + quad_c x pops)  a wavefront of k_quad; pops = heap pops per dispatch, as the main kernel
+//                                              measured them for the class
+//   eff_beside_quad                            the part of a compute unit's sixteen wavefronts of k_plan that get
+//                                              through where k_quad runs beside them
+//   quad_margin                                a batch moves to k_quad only if the main kernel would end this much later
 //   gain_threshold, gain_classes               a split by class size / by measured time must model this much earlier
 struct SplitModel {
   double plan_a = 12.0, plan_b = 0.9, plan_list = 1.2;
-  double quad_a = 40.0, quad_b = 1.6, quad_c = 0.45;
+  double quad_a = 10.0, quad_b = 1.3, quad_c = 0.2;
   double eff_beside_quad = 0.65;
   double quad_margin = 1.15;
   double gain_threshold = 0.97, gain_classes = 0.98;
@@ -715,11 +731,13 @@ struct rpeg_engine_s {
   std::vector<uint32_t> cls_off, cls_nodes, cls_slots;
   std::vector<uint32_t> cls_pops16;                  // learned, of the slowest full wavefront of the class in the main kernel:
                                                      // microseconds << 12 | heap pops per dispatch in sixteenths
-  uint32_t* d_cstat = nullptr;                       // the device's copy, written by the main kernel
+  std::vector<uint32_t> cls_need;                    // learned: the longest ready set of the class's plans in k_quad (0: none yet)
+  uint32_t* d_cstat = nullptr;                       // the device's copies, one behind the other (cstat_cap words each)
   uint32_t cstat_cap = 0;
   std::vector<uint8_t> cls_split;                    // where every class ran when that was last decided: 0 main kernel, 1 k_plan,
   uint64_t split_for_n = 0, split_at = 0;            // 2 k_quad, 255 not in that batch; the batch size and the call of that decision
   bool split_mass = false;
+  bool split_quad = false;                           // k_quad took the batch
   uint32_t learn_calls = 0;                          // calls left after which the statistic is read back
   uint64_t batch_calls = 0;
   uint64_t* d_hkey = nullptr;                        // device table signature -> class id
@@ -777,6 +795,8 @@ struct rpeg_engine_s {
   hipStream_t s2 = nullptr;                     // second stream: single-plan wavefronts of a large batch run beside the others
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   hipEvent_t ev_counts = nullptr;               // the statistic of a call has reached the host (the calls that read it)
+  hipStream_t s4 = nullptr;                     // fourth stream and its join: k_quad's second launches
+  hipEvent_t ev_join4 = nullptr;
   hipStream_t s3 = nullptr;                     // third stream: the four-lanes-per-plan wavefronts (k_quad)
   hipEvent_t ev_join3 = nullptr;
   hipEvent_t ev_sig = nullptr;                  // the signature kernel of a call is done (its class ids are there)
@@ -911,9 +931,10 @@ static int ensure_class_tables(rpeg_engine_t* e, hipStream_t s) {
     const uint32_t cap = std::max<uint32_t>(2 * ncls, 4096);
     if (e->d_cstat) hipFree(e->d_cstat);
     e->d_cstat = nullptr; e->cstat_cap = 0;
-    HIP_TRY(e, hipMalloc(&e->d_cstat, (size_t)cap * 4));
-    HIP_TRY(e, hipMemset(e->d_cstat, 0, (size_t)cap * 4));
+    HIP_TRY(e, hipMalloc(&e->d_cstat, 2 * (size_t)cap * 4));
+    HIP_TRY(e, hipMemset(e->d_cstat, 0, 2 * (size_t)cap * 4));
     HIP_TRY(e, hipMemcpy(e->d_cstat, e->cls_pops16.data(), (size_t)ncls * 4, hipMemcpyHostToDevice));
+    HIP_TRY(e, hipMemcpy(e->d_cstat + cap, e->cls_need.data(), (size_t)ncls * 4, hipMemcpyHostToDevice));
     e->cstat_cap = cap;
   }
   e->tables_for = ncls;
@@ -980,6 +1001,7 @@ static int64_t class_append(rpeg_engine_t* e, uint64_t sig, const LoweredClass& 
   e->cls_nodes.push_back(h->n_nodes);
   e->cls_slots.push_back(h->n_slots);
   e->cls_pops16.push_back(0);
+  e->cls_need.push_back(0);
   e->learn_calls = 3;
   return off;
 }
@@ -1150,7 +1172,7 @@ void rpeg_engine_destroy(rpeg_engine_t* e) {
   if (e->d_cls) { hipFree(e->d_cls); hipHostFree(e->h_cls); }
   // (the side streams belong to the device, not to the engine: side_streams)
   if (e->s2) { hipStreamSynchronize(e->s2); hipEventDestroy(e->ev_fork); hipEventDestroy(e->ev_join); }
-  if (e->s3) { hipStreamSynchronize(e->s3); hipEventDestroy(e->ev_join3); }
+  if (e->s3) { hipStreamSynchronize(e->s3); hipEventDestroy(e->ev_join3); hipStreamSynchronize(e->s4); hipEventDestroy(e->ev_join4); }
   if (e->ev_sig) hipEventDestroy(e->ev_sig);
   if (e->ev_counts) hipEventDestroy(e->ev_counts);
   e->lane0.release();
@@ -1251,6 +1273,7 @@ int rpeg_engine_reset_classes(rpeg_engine_t* e) {
   e->cls_nodes.clear();
   e->cls_slots.clear();
   e->cls_pops16.clear();
+  e->cls_need.clear();
   e->cls_split.clear();
   e->split_for_n = 0;
   if (e->d_cstat) { hipFree(e->d_cstat); e->d_cstat = nullptr; e->cstat_cap = 0; }
@@ -1328,29 +1351,31 @@ static DeepModel deep_model(const rpeg_engine_t* e, uint32_t rcap) {
 // process (never destroyed).  A process has few hardware queues (four by default): with a pair of side streams per
 // engine, two engines that evaluate at the same time on two caller streams are six streams, several of which share
 // a queue and then wait for each other's kernels; with one pair they are four.
-static int side_streams(rpeg_engine_t* e, hipStream_t* plan_stream, hipStream_t* quad_stream) {
+static int side_streams(rpeg_engine_t* e, hipStream_t* plan_stream, hipStream_t* quad_stream, hipStream_t* second_quad_stream) {
   static std::mutex mu;
-  static hipStream_t pair[64][2] = {};
+  static hipStream_t pair[64][3] = {};
   int dev = 0;
   HIP_TRY(e, hipGetDevice(&dev));
   if (dev < 0 || dev >= 64) { e->err = "device index out of range"; return -2; }
   std::lock_guard<std::mutex> lock(mu);
-  for (int k = 0; k < 2; ++k)
+  for (int k = 0; k < 3; ++k)
     if (!pair[dev][k]) HIP_TRY(e, hipStreamCreateWithFlags(&pair[dev][k], hipStreamNonBlocking));
   if (plan_stream) *plan_stream = pair[dev][0];
   if (quad_stream) *quad_stream = pair[dev][1];
+  if (second_quad_stream) *second_quad_stream = pair[dev][2];
   return 0;
 }
 
 // The engine's handles on the two side streams and the events of its forks and joins.
 static int ensure_side(rpeg_engine_t* e) {
   if (!e->s2) {
-    if (int rc = side_streams(e, &e->s2, nullptr)) return rc;
+    if (int rc = side_streams(e, &e->s2, nullptr, nullptr)) return rc;
     HIP_TRY(e, hipEventCreateWithFlags(&e->ev_fork, hipEventDisableTiming));
     HIP_TRY(e, hipEventCreateWithFlags(&e->ev_join, hipEventDisableTiming));
   }
   if (!e->s3) {
-    if (int rc = side_streams(e, nullptr, &e->s3)) return rc;
+    if (int rc = side_streams(e, nullptr, &e->s3, &e->s4)) return rc;
+    HIP_TRY(e, hipEventCreateWithFlags(&e->ev_join4, hipEventDisableTiming));
     HIP_TRY(e, hipEventCreateWithFlags(&e->ev_join3, hipEventDisableTiming));
     HIP_TRY(e, hipEventCreateWithFlags(&e->ev_sig, hipEventDisableTiming));
     HIP_TRY(e, hipGetDevice(&e->side_dev));
@@ -1368,7 +1393,7 @@ static bool side_claim(rpeg_engine_t* e) {
   const void* last = owner[e->side_dev];
   owner[e->side_dev] = e;
   if (last == e || last == nullptr) return true;
-  return hipStreamQuery(e->s2) == hipSuccess && hipStreamQuery(e->s3) == hipSuccess;
+  return hipStreamQuery(e->s2) == hipSuccess && hipStreamQuery(e->s3) == hipSuccess && hipStreamQuery(e->s4) == hipSuccess;
 }
 
 static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, uint32_t flags, double* makespan,
@@ -1514,7 +1539,10 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     }
     hipLaunchKernelGGL(k_hand_counts, dim3(1), dim3(HAND_BLOCK), 0, s, e->d_ccount, e->d_need, ncls, shards, e->h_tot_dev, e->h_sigflag_dev, tag);
     HIP_TRY(e, hipGetLastError());
-    if (read_stat) HIP_TRY(e, hipMemcpyAsync(e->cls_pops16.data(), e->d_cstat, (size_t)ncls * 4, hipMemcpyDeviceToHost, s));
+    if (read_stat) {
+      HIP_TRY(e, hipMemcpyAsync(e->cls_pops16.data(), e->d_cstat, (size_t)ncls * 4, hipMemcpyDeviceToHost, s));
+      HIP_TRY(e, hipMemcpyAsync(e->cls_need.data(), e->d_cstat + e->cstat_cap, (size_t)ncls * 4, hipMemcpyDeviceToHost, s));
+    }
     if (round == 0) {
       if (!handed) {   // (the copy of the statistic has to be waited for: an event, so that the wait leaves the launch below alone)
         if (!e->ev_counts) HIP_TRY(e, hipEventCreateWithFlags(&e->ev_counts, hipEventDisableTiming));
@@ -1569,10 +1597,10 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // wavefronts of fewer plans whose state fits in LDS, which shortens every scheduler step.
   int ls = e->state_lanes;
   bool one = false;   // one plan per wavefront (k_plan)
-  const bool quad_all = ls == 4;   // every class in the four-lanes-per-plan kernel (k_quad)
+  const bool quad_all = ls == 4;   // every class in the kernel of two or four lanes per plan (k_quad)
   if (quad_all) {
     ls = 0;
-    if (kq_lds_bytes((e->max_cls_bytes + 15u) & ~15u, e->max_nodes, e->max_slots, e->max_v, (uint32_t)KQ_PLANS, mass != nullptr) > 160 * 1024) {
+    if (kq_lds_bytes(16, e->max_nodes, e->max_slots, mass != nullptr) > 160 * 1024 || e->max_nodes > KQ_MAX_NODES) {
       e->err = "per-plan state of this problem does not fit in LDS with sixteen plans per wavefront";
       return -8;
     }
@@ -1624,26 +1652,102 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   std::vector<uint32_t> first(counts.size(), 0), clpw(counts.size(), lpw);
   // ready-list capacity of the main kernel: the full list until the longest list of earlier launches is known
   const uint32_t rcap_main = e->need > 0 ? std::min(e->ready_cap, std::max(8u, (e->need + 2 + 7) & ~7u)) : e->ready_cap;
+  // k_quad: the form with the fewest entries that the longest ready set of the class's earlier plans fits.  Two lanes per
+  // plan only up to QUAD_TWO_NODES nodes: thirty-two plans of larger graphs leave too few wavefronts room in LDS.  (No
+  // class / 35 / 60 nodes / all of them, us per step: GRPO 65,536 381 / 386 / 366 / 382; PPO 60,000 787 / 796 / 786 / 1,022.)
+  constexpr uint32_t QUAD_TWO_NODES = 60;
+  auto quad_kind = [&](size_t c) {
+    const uint32_t need = e->cls_need[cids[c]];
+    return need == 0 ? 2 : need <= QUAD_KIND[0].entries && e->cls_nodes[cids[c]] <= QUAD_TWO_NODES ? 0 : need <= QUAD_KIND[1].entries ? 1 : 2;
+  };
   std::vector<uint8_t> solo(counts.size(), 0), quad(counts.size(), quad_all ? 1 : 0);
-  uint32_t quad_nodes = quad_all ? e->max_nodes : 0, quad_slots = quad_all ? e->max_slots : 0;
+  const bool plan_fits = e->max_nodes <= (uint32_t)(WAVE * KP_MAX_NS) && kp_lds_bytes(e->max_nodes, e->max_slots) <= 64 * 1024;
+  constexpr uint32_t QUAD_TINY = 8, QUAD_MEAN_NODES = 128;
+  // k_quad takes the batch, with k_plan beside it, where the model below has them done before the main kernel would be.
+  // Into k_plan go the classes of fewer than QUAD_TINY plans (a wavefront of k_quad lasts as long with one plan as with
+  // all; 4, 8 and 16 measured: 8 is best or within 2 % on five batches), those whose ready sets outgrow sixteen entries,
+  // and as many of the largest graphs as make the end earliest: a wavefront of k_quad lasts two to three times as long
+  // as a plan in k_plan.  The time of k_quad: its wavefronts' (SplitModel) over those a compute unit holds by LDS, all
+  // classes' and k_plan's together, and no less than its longest wavefront.  Only once half of the plans it
+  // would take are in classes whose ready sets the main kernel has measured; the others' unknown ready sets take the form with
+  // the most entries.
+  // Measured, us per step, main kernel / k_quad: GRPO (51 nodes on average) 17,000 plans 402 / 270, 65,536 460 / 365,
+  // 131,072 716 / 580; PPO (98) 20,011 548 / 410, 131,072 1,616 / 1,505; DPO (28) 65,536 277 / 140, 1,048,576 1,686 /
+  // 1,225.  AC-share (152): 20,011 1,216 / 930, but 65,536 2,353 / 2,300-2,500 and 262,144 5,549 / 8,426: of large graphs
+  // few plans have room in LDS, and the main kernel keeps its state in HBM: a batch of more than sixteen of its wavefronts
+  // per compute unit stays there where the plans have more than QUAD_MEAN_NODES nodes on average.
+  auto plan_quad = [&]() -> bool {
+    if (e->state_lanes != -1 || !e->quad_share_pct || !e->split_heavy || !plan_fits) return false;
+    const DeepModel dm = deep_model(e, rcap_main);
+    double t_sum = 0.0, nodes_sum = 0.0, pops_sum = 0.0;
+    uint64_t takes = 0, measured = 0, known = 0, nodes = 0, main_tasks = 0;
+    for (size_t c = 0; c < counts.size(); ++c) {
+      const uint32_t w = e->cls_pops16[cids[c]];
+      nodes += (uint64_t)counts[c] * e->cls_nodes[cids[c]];
+      main_tasks += (counts[c] + WAVE - 1) / WAVE;
+      if (counts[c] >= QUAD_TINY) { takes += counts[c]; measured += e->cls_need[cids[c]] ? counts[c] : 0; }
+      if (w) { t_sum += (double)(w >> 12); nodes_sum += (double)e->cls_nodes[cids[c]]; pops_sum += (w & 0xFFFu) / 16.0; ++known; }
+    }
+    if (nodes > QUAD_MEAN_NODES * n && main_tasks > (uint64_t)e->n_cu * 16) return false;
+    if (!measured || measured * 2 < takes || !known || t_sum <= 0.0) return false;
+    const double per_node = t_sum / nodes_sum, pops = pops_sum / (double)known;
+    double w_main = 0.0, max_main = 0.0, w_quad = 0.0, w_plan = 0.0;
+    auto t_quad = [&](uint32_t c) {   // one wavefront
+      const uint32_t w = e->cls_pops16[cids[c]];
+      return dm.sm.quad_a + (double)e->cls_nodes[cids[c]] * (dm.sm.quad_b + dm.sm.quad_c * (w ? (w & 0xFFFu) / 16.0 : pops));
+    };
+    auto cost_quad = [&](uint32_t c) {   // all of the class's, in time of a compute unit
+      const QuadKind& k = QUAD_KIND[quad_kind(c)];
+      const double held = std::min(16.0, std::floor(160.0 * 1024 / (double)kq_lds_bytes(k.plans, e->cls_nodes[cids[c]], e->cls_slots[cids[c]], mass != nullptr)));
+      return (double)((counts[c] + k.plans - 1) / k.plans) * t_quad(c) / std::max(1.0, held);
+    };
+    auto cost_plan = [&](uint32_t c) { return dm.plan_cost(counts[c], e->cls_nodes[cids[c]]) / (16.0 * dm.sm.eff_beside_quad); };
+    std::vector<uint8_t> to_plan(counts.size(), 0);
+    double base_plan = 0.0;
+    for (uint32_t c : order) {
+      const double t0 = (double)(e->cls_pops16[cids[c]] >> 12), t = t0 > 0.0 ? t0 : per_node * (double)e->cls_nodes[cids[c]];
+      if (counts[c] >= TINY_CLASS) { w_main += (double)((counts[c] + WAVE - 1) / WAVE) * t; max_main = std::max(max_main, t); }
+      else base_plan += dm.plan_cost(counts[c], e->cls_nodes[cids[c]]);
+      to_plan[c] = counts[c] < QUAD_TINY || e->cls_need[cids[c]] > QUAD_KIND[1].entries || e->cls_nodes[cids[c]] > KQ_MAX_NODES;
+      if (to_plan[c]) w_plan += cost_plan(c);
+      else w_quad += cost_quad(c);
+    }
+    double best = 0.0;
+    size_t best_k = 0;
+    for (size_t k = 0; k <= order.size(); ++k) {   // the k largest graphs to k_plan
+      while (k < order.size() && to_plan[order[k]]) ++k;
+      const double t = std::max((w_quad + w_plan) / dm.n_cu, k < order.size() ? t_quad(order[k]) : 0.0);
+      if (best == 0.0 || t < dm.sm.gain_classes * best) { best = t; best_k = k; }
+      if (k < order.size()) { w_quad -= cost_quad(order[k]); w_plan += cost_plan(order[k]); }
+    }
+    if (!(dm.sm.quad_margin * best < dm.best(w_main, base_plan, max_main, nullptr))) return false;
+    for (size_t k = 0; k < order.size(); ++k) {
+      const uint32_t c = order[k];
+      if (to_plan[c] || k < best_k) solo[c] = 1;
+      else quad[c] = 1;
+    }
+    return true;
+  };
   // Where every class runs is decided from the class counts and what has been measured (below): on a batch of
   // thousands of classes that is 0.2 ms of host work.  The decision is kept per class for the next fifteen calls on
   // batches of about the same size (a class not seen then goes by the plain size rule), unless new measurements
   // are about to be read.
+  bool by_quad = false;
   const bool keep_split = !ls && !one && !quad_all && e->quad_share_pct && e->split_for_n && e->learn_calls == 0 &&
                           n * 4 >= e->split_for_n * 3 && n * 3 <= e->split_for_n * 4 && e->batch_calls - e->split_at < 16 &&
                           e->split_mass == (mass != nullptr);
   if (keep_split) {
     for (size_t c = 0; c < counts.size(); ++c) {
       const uint8_t a = cids[c] < e->cls_split.size() ? e->cls_split[cids[c]] : (uint8_t)255;
-      if (a == 255) solo[c] = counts[c] < TINY_CLASS ? 1 : 0;
+      if (a == 255 && e->split_quad) (counts[c] < QUAD_TINY || e->cls_nodes[cids[c]] > KQ_MAX_NODES ? solo[c] : quad[c]) = 1;
+      else if (a == 255) solo[c] = counts[c] < TINY_CLASS ? 1 : 0;
       else if (a == 1) solo[c] = 1;
       else if (a == 2) {
         quad[c] = 1;
-        quad_nodes = std::max(quad_nodes, e->cls_nodes[cids[c]]);
-        quad_slots = std::max(quad_slots, e->cls_slots[cids[c]]);
       }
     }
+  } else if (!ls && !one && !quad_all && !order.empty() && (by_quad = plan_quad())) {
+    // (decided: every class in k_quad or, tiny classes and the largest graphs, in k_plan)
   } else if (!ls && !one && !quad_all && !order.empty()) {
     // The kernel ends with its slowest wavefront, and a wavefront is as slow as its slowest plan.  The
     // classes with the largest graphs (up to 15 % of the batch: beyond that the single-plan kernel would be
@@ -1657,7 +1761,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     const bool split = e->split_heavy && one_fits;
     // node count from which a class counts as large: the smallest one, not under `floor` percent of the
     // largest, such that the large classes hold at most `share` percent of the batch
-    // (eight percent when k_quad takes the dense classes: a plan costs k_plan four times the instructions)
+    // (eight percent while the batch is at most twelve wavefronts per compute unit deep)
     const uint64_t floor_pct = split ? 60ull : 70ull;
     uint64_t share_pct = split ? 15ull : 25ull;
     {
@@ -1753,8 +1857,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     // longest classes are taken out, as many of them as make the modelled end of the step (deep_model) earliest.
     if (split && e->quad_share_pct) {
       DeepModel dm = deep_model(e, rcap_main);
-      // (where k_quad is going to take its share of a compute unit's wavefront slots and LDS, k_plan gets through
-      // about two thirds of what the model gives it beside the main kernel: measured on configs 2 and 5)
+      // (in a batch that shallow k_plan gets through about two thirds of what the model gives it beside the main kernel)
       if (waves64 <= (uint64_t)e->n_cu * 12) dm.eff = dm.sm.eff_beside_quad;
       double w_main = 0.0, w_plan = 0.0, t_sum = 0.0, nodes_sum = 0.0;
       std::vector<uint32_t> cand;
@@ -1789,62 +1892,17 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
         for (size_t k = 0; k < best_k; ++k) solo[cand[k]] = 1;
       }
     }
-    // Of what stays, the wavefronts that end last are those of dense graphs (long ready lists, keys that go stale
-    // often).  The main kernel measures itself: per class, the time of its slowest wavefront on earlier launches and
-    // the heap pops per dispatch it needed (cls_pops16).  What a wavefront of k_quad takes: SplitModel.  The classes
-    // are taken in the order of their measured time while one still ends later by SplitModel::quad_margin
-    // in the main kernel than the slowest chosen class ends in k_quad, up to `quad_share_pct`
-    // percent of the batch.  Nothing is known before the first launch of a class: it stays in the main kernel then.
-    if (split && e->quad_share_pct && waves64 <= (uint64_t)e->n_cu * 12) {
-      auto t_main = [&](uint32_t c) { return (double)(e->cls_pops16[cids[c]] >> 12); };
-      auto t_quad = [&](uint32_t c) {
-        const double nd = e->cls_nodes[cids[c]], p = (e->cls_pops16[cids[c]] & 0xFFFu) / 16.0;
-        return e->split_model.quad_a + nd * (e->split_model.quad_b + e->split_model.quad_c * p);
-      };
-      std::vector<uint32_t> cand;
-      for (uint32_t c = 0; c < counts.size(); ++c)
-        if (!solo[c] && e->cls_pops16[cids[c]]) cand.push_back(c);
-      std::sort(cand.begin(), cand.end(), [&](uint32_t x, uint32_t y) { return t_main(x) > t_main(y); });
-      // (k_quad's wavefronts have the LDS that the main kernel's wavefronts and a few of k_plan's leave on a compute
-      // unit: beyond one round of them the time of a wavefront counts as many times as there are rounds)
-      const size_t lds_main = ke_lds_bytes((e->max_cls_bytes + 15u) & ~15u, rcap_main, 0, e->max_nodes, e->max_slots, e->max_v);
-      uint64_t main_tasks = 0;
-      for (uint32_t c = 0; c < counts.size(); ++c)
-        if (!solo[c]) main_tasks += (counts[c] + WAVE - 1) / WAVE;
-      double slowest_quad = 0.0;
-      uint64_t taken = 0, tasks = 0;
-      for (uint32_t c : cand) {
-        const uint32_t nodes = e->cls_nodes[cids[c]], slots = e->cls_slots[cids[c]];
-        const size_t qlds = kq_lds_bytes((e->max_cls_bytes + 15u) & ~15u, std::max(quad_nodes, nodes), std::max(quad_slots, slots), e->max_v,
-                                         (uint32_t)KQ_PLANS, mass != nullptr);
-        if (qlds > 64 * 1024) continue;
-        const uint64_t c_tasks = (counts[c] + KQ_PLANS - 1) / KQ_PLANS;
-        const uint64_t main_left = main_tasks - std::min<uint64_t>(main_tasks, (counts[c] + WAVE - 1) / WAVE);
-        const double lds_left = 144.0 * 1024 - (double)((main_left + e->n_cu - 1) / e->n_cu) * (double)lds_main;
-        const double room = (double)e->n_cu * std::max(1.0, std::floor(lds_left / (double)qlds));
-        const double tq = std::max(slowest_quad, t_quad(c));
-        const double rounds = std::max(1.0, (double)(tasks + c_tasks) / room);
-        if (t_main(c) <= e->split_model.quad_margin * tq * rounds) break;   // (a margin: beyond the classes that clearly end later, more wavefronts of k_quad cost more than they save)
-        if ((taken + counts[c]) * 100 > (uint64_t)n * e->quad_share_pct) break;
-        quad[c] = 1;
-        taken += counts[c];
-        tasks += c_tasks;
-        main_tasks = main_left;
-        slowest_quad = tq;
-        quad_nodes = std::max(quad_nodes, nodes);
-        quad_slots = std::max(quad_slots, slots);
-      }
-    }
-    if (split && e->quad_share_pct) {   // kept for the next calls
-      e->cls_split.assign(ncls, (uint8_t)255);
-      for (size_t c = 0; c < counts.size(); ++c) e->cls_split[cids[c]] = solo[c] ? 1 : quad[c] ? 2 : 0;
-      e->split_for_n = n; e->split_at = e->batch_calls; e->split_mass = mass != nullptr;
-      // a class that runs in the main kernel for the first time is measured by this launch: read it in the next call
-      // (at most once in eight calls, so that a class whose measurement never arrives cannot keep the read-back on)
-      bool unmeasured = false;
-      for (size_t c = 0; c < counts.size() && !unmeasured; ++c) unmeasured = !solo[c] && !quad[c] && (e->cls_pops16[cids[c]] >> 12) == 0;
-      if (unmeasured && e->learn_calls == 0 && e->batch_calls - e->relearn_at >= 8) { e->learn_calls = 1; e->relearn_at = e->batch_calls; }
-    }
+  }
+  if (!keep_split && !ls && !one && !quad_all && !order.empty() && e->split_heavy && plan_fits && e->quad_share_pct) {   // kept for the next calls
+    e->cls_split.assign(ncls, (uint8_t)255);
+    for (size_t c = 0; c < counts.size(); ++c) e->cls_split[cids[c]] = solo[c] ? 1 : quad[c] ? 2 : 0;
+    e->split_for_n = n; e->split_at = e->batch_calls; e->split_mass = mass != nullptr;
+    e->split_quad = by_quad;
+    // a class that runs in the main kernel or in k_quad for the first time is measured by this launch: read it in the next call
+    // (at most once in eight calls, so that a class whose measurement never arrives cannot keep the read-back on)
+    bool unmeasured = false;
+    for (size_t c = 0; c < counts.size() && !unmeasured; ++c) unmeasured = quad[c] ? e->cls_need[cids[c]] == 0 : !solo[c] && (e->cls_pops16[cids[c]] >> 12) == 0;
+    if (unmeasured && e->learn_calls == 0 && e->batch_calls - e->relearn_at >= 8) { e->learn_calls = 1; e->relearn_at = e->batch_calls; }
   }
   uint32_t n_eval_waves = 0, n_quad_waves = 0, n_solo = 0;
   for (size_t k = 0; k < order.size(); ++k) {
@@ -1853,12 +1911,45 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     first[c] = n_eval_waves;
     n_eval_waves += (counts[c] + clpw[c] - 1) / clpw[c];
   }
-  for (size_t k = 0; k < order.size(); ++k) {   // the tasks of k_quad follow those of the main kernel
-    const uint32_t c = order[k];
-    if (!quad[c]) continue;
-    clpw[c] = (uint32_t)(uint32_t)KQ_PLANS;
-    first[c] = n_eval_waves + n_quad_waves;
-    n_quad_waves += (counts[c] + clpw[c] - 1) / clpw[c];
+  // The tasks of k_quad follow those of the main kernel: a launch for every form, each on a stream of its
+  // own, and where a stream is left, one for the larger and one for the smaller graphs of a form -- the LDS of a launch is
+  // that of its largest graph, and LDS bounds the wavefronts in flight.  The line lies where the sum over the tasks of
+  // time (nodes) times LDS is smallest.
+  struct QuadLaunch { uint32_t first = 0, waves = 0, nodes = 0, slots = 0; int kind = 0; } quad_launch[4];
+  {
+    auto waves_of = [&](uint32_t c, int kind) { return (counts[c] + QUAD_KIND[kind].plans - 1) / QUAD_KIND[kind].plans; };
+    for (int kind : {2, 0, 1}) {
+      std::vector<uint32_t> qc;
+      double all = 0.0;
+      for (uint32_t c : order)   // (largest graphs first)
+        if (quad[c] && quad_kind(c) == kind) {
+          qc.push_back(c);
+          all += (double)waves_of(c, kind) * (double)e->cls_nodes[cids[c]];
+        }
+      size_t cut = qc.size();
+      if (kind != 2 && !quad_launch[2].waves && !quad_launch[3].waves && !qc.empty()) {
+        auto lds_of = [&](uint32_t c) { return (double)kq_lds_bytes(QUAD_KIND[kind].plans, e->cls_nodes[cids[c]], e->max_slots, mass != nullptr); };
+        double upto = 0.0, best = all * lds_of(qc[0]);
+        for (size_t k = 0; k + 1 < qc.size(); ++k) {
+          upto += (double)waves_of(qc[k], kind) * (double)e->cls_nodes[cids[qc[k]]];
+          if (e->cls_nodes[cids[qc[k]]] == e->cls_nodes[cids[qc[k + 1]]]) continue;
+          const double cost = upto * lds_of(qc[0]) + (all - upto) * lds_of(qc[k + 1]);
+          if (cost < 0.95 * best) { best = cost; cut = k + 1; }
+        }
+      }
+      for (size_t k = 0; k < qc.size(); ++k) {
+        const uint32_t c = qc[k];
+        QuadLaunch& q = quad_launch[k < cut ? kind : 3];
+        clpw[c] = QUAD_KIND[kind].plans;
+        first[c] = n_eval_waves + n_quad_waves;
+        const uint32_t nw = waves_of(c, kind);
+        if (!q.waves) { q.first = n_quad_waves; q.kind = kind; }
+        q.waves += nw;
+        q.nodes = std::max(q.nodes, e->cls_nodes[cids[c]]);
+        q.slots = std::max(q.slots, e->cls_slots[cids[c]]);
+        n_quad_waves += nw;
+      }
+    }
   }
   const uint32_t n_lane_waves = n_eval_waves + n_quad_waves;
   const uint32_t pstride = one ? 1u : (uint32_t)WAVE;
@@ -1911,7 +2002,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       continue;
     } else {
       // (never for a task of k_quad, whose eight plans of eight lanes each are not that layout)
-      const uint32_t flag = !quad[c] && few_in_lds && clpw[c] == (uint32_t)KE_FEW ? KE_CLS_LDS : 0u;
+      const uint32_t flag = (quad[c] ? quad_kind(c) == 1 && e->cls_need[cids[c]] <= QUAD_KIND[0].entries : few_in_lds && clpw[c] == (uint32_t)KE_FEW) ? KE_CLS_LDS : 0u;
       const uint32_t nw = (counts[c] + clpw[c] - 1) / clpw[c];
       for (uint32_t t = 0; t < nw; ++t) h_tasks[first[c] + t] = offs[c] | flag;
     }
@@ -1988,6 +2079,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   L.ovf = short_list ? e->d_ovf : nullptr;
   L.need = !ls && !one ? e->d_need : nullptr;
   L.cstat = !ls && !one && e->quad_share_pct ? e->d_cstat : nullptr;
+  L.cneed = L.cstat ? L.cstat + e->cstat_cap : nullptr;
   L.queue = queued ? e->d_queues : nullptr;
   L.flags = flags; L.makespan = makespan; L.peak = peak; L.score = score; L.mask = mask;
   L.mass = mass;
@@ -2048,21 +2140,25 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   } else if (e->timing) {
     HIP_TRY(e, hipEventRecord(e->ev0, s));
   }
-  auto launch_quad = [&]() -> int {   // the four-lanes-per-plan wavefronts, beside the main kernel
-    if (!n_quad_waves) return 0;
+  auto launch_quad = [&](const QuadLaunch& q, hipStream_t on) -> int {
+    if (!q.waves) return 0;
     EvalLaunch Q = L;
-    Q.perm = e->d_perm + (uint64_t)n_eval_waves * WAVE;
-    Q.wave_cls = L.wave_cls + n_eval_waves;
-    Q.n_waves = n_quad_waves;
-    Q.ws_nodes = quad_nodes; Q.ws_slots = quad_slots;
-    Q.ovf = nullptr; Q.need = nullptr; Q.cstat = nullptr; Q.queue = nullptr;   // (a plan that outgrows the 32 entries is flagged in Q.limit)
-    if (L.prof) Q.prof = L.prof + n_waves * 8;
-    const size_t qlds = kq_lds_bytes(L.cls_bytes, quad_nodes, quad_slots, e->max_v, (uint32_t)KQ_PLANS, mass != nullptr);
+    Q.perm = e->d_perm + ((uint64_t)n_eval_waves + q.first) * WAVE;
+    Q.wave_cls = L.wave_cls + n_eval_waves + q.first;
+    Q.n_waves = q.waves;
+    Q.ws_nodes = q.nodes; Q.ws_slots = q.slots;
+    Q.ovf = nullptr; Q.cstat = nullptr; Q.queue = nullptr;   // (a plan that outgrows the entries is flagged in Q.limit)
+    if (L.prof) Q.prof = L.prof + (n_waves + q.first) * 8;
+    const size_t qlds = kq_lds_bytes(QUAD_KIND[q.kind].plans, q.nodes, q.slots, mass != nullptr);
     if (qlds > 64 * 1024 && !e->quad_attr_set) {
-      HIP_TRY(e, hipFuncSetAttribute((const void*)k_quad, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+      HIP_TRY(e, hipFuncSetAttribute((const void*)k_quad<2, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+      HIP_TRY(e, hipFuncSetAttribute((const void*)k_quad<4, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+      HIP_TRY(e, hipFuncSetAttribute((const void*)k_quad<4, 6>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
       e->quad_attr_set = true;
     }
-    hipLaunchKernelGGL(k_quad, dim3((unsigned)std::min<uint64_t>(n_quad_waves, (uint64_t)e->n_cu * 16)), dim3(WAVE), qlds, sq, Q);
+    if (q.kind == 0) hipLaunchKernelGGL((k_quad<2, 4>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q);
+    else if (q.kind == 1) hipLaunchKernelGGL((k_quad<4, 4>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q);
+    else hipLaunchKernelGGL((k_quad<4, 6>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q);
     HIP_TRY(e, hipGetLastError());
     return 0;
   };
@@ -2091,7 +2187,11 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   }
   // (k_quad second: measured against k_quad first, 0.50 against 0.52-0.53 ms on config 2, and against k_quad last,
   // 0.59 ms; its wavefronts need the most LDS after the main kernel's)
-  if (int rc = launch_quad()) return rc;
+  if (quad_launch[2].waves || quad_launch[3].waves) HIP_TRY(e, hipStreamWaitEvent(e->s4, e->ev_fork, 0));
+  if (int rc = launch_quad(quad_launch[2], e->s4)) return rc;
+  if (int rc = launch_quad(quad_launch[0], sm)) return rc;
+  if (int rc = launch_quad(quad_launch[1], sq)) return rc;
+  if (int rc = launch_quad(quad_launch[3], e->s4)) return rc;
   if (n_solo) {   // the single-plan wavefronts, beside the main kernel
     HIP_TRY(e, hipStreamWaitEvent(e->s2, e->ev_fork, 0));
     EvalLaunch S = L;
@@ -2105,7 +2205,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   }
   if (peaks_deferred) {
     const unsigned pblk = (unsigned)((n + WAVE - 1) / WAVE);
-    hipLaunchKernelGGL(k_peaks, dim3(pblk), dim3(WAVE), kpeaks_lds_bytes(e->max_v), peaks_aside ? sq : sm, G);
+    hipLaunchKernelGGL(k_peaks, dim3(pblk), dim3(WAVE), kpeaks_lds_bytes(e->max_v), peaks_aside ? sq : n_solo && !n_waves ? e->s2 : sm, G);
     HIP_TRY(e, hipGetLastError());
   }
   if (n_solo) HIP_TRY(e, hipEventRecord(e->ev_join, e->s2));
@@ -2131,6 +2231,10 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     ahead_join.joined = true;
   }
   if (n_solo) HIP_TRY(e, hipStreamWaitEvent(s, e->ev_join, 0));
+  if (quad_launch[2].waves || quad_launch[3].waves) {
+    HIP_TRY(e, hipEventRecord(e->ev_join4, e->s4));
+    HIP_TRY(e, hipStreamWaitEvent(s, e->ev_join4, 0));
+  }
   if (peaks_deferred) {   // (before k_eval_limit, whose plans get their final outputs from that kernel itself)
     // (the layout tables in the counters' buffer have been read by now: the counters of the next call are cleared here)
     const uint32_t zero_n = (uint32_t)std::min<size_t>(std::max<size_t>((size_t)COUNT_SLOTS, ncls) + 1, 4 * (size_t)e->ccap + COUNT_SLOTS);
@@ -2142,7 +2246,15 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   if (bounded) {   // the plans flagged by the kernels above, without a bound on the ready set (ends at once when there is none)
     EvalLaunch U = L;
     U.queue = nullptr;
-    hipLaunchKernelGGL(k_eval_limit, dim3(e->limit_grid), dim3(WAVE), 0, s, U, e->d_limit_ws);
+    const size_t plan_lds = kp_lds_bytes(e->max_nodes, e->max_slots);
+    if (L.dur && e->max_nodes <= (uint32_t)(WAVE * KP_MAX_NS) && plan_lds <= 64 * 1024) {
+      U.aux_pen = e->d_aux_pen; U.aux_mask = e->d_aux_mask;   // (the memory-model launch is done: final outputs from here)
+      U.prof = nullptr;
+      if (mass) hipLaunchKernelGGL(k_plan_limit<KP_TIMES>, dim3((unsigned)e->n_cu * 8u), dim3(WAVE), plan_lds, s, U);
+      else hipLaunchKernelGGL(k_plan_limit<KP_NO_TRACE>, dim3((unsigned)e->n_cu * 8u), dim3(WAVE), plan_lds, s, U);
+    } else {
+      hipLaunchKernelGGL(k_eval_limit, dim3(e->limit_grid), dim3(WAVE), 0, s, U, e->d_limit_ws);
+    }
     HIP_TRY(e, hipGetLastError());
   }
   {

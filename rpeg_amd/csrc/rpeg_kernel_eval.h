@@ -62,6 +62,7 @@ struct EvalLaunch {              // uniform launch parameters
                                  // they become free; null: block b takes tasks b, b + grid, ...
   uint32_t* cstat = nullptr;     // per class (ClassHdr::id), of its slowest 64-plan wavefront so far: microseconds
                                  // << 12 | heap pops per dispatch in sixteenths; or null
+  uint32_t* cneed = nullptr;     // per class: the longest ready set of its plans so far; or null
   // What the prologue launches (rpeg_kernel_prologue.h) computed for every plan of the call, indexed by plan.  All null
   // where a kernel computes these itself (the single-plan kernel without a layout).
   const double* dur = nullptr;         // [universe slot][plan], rows dur_stride apart; NaN where the reference would raise
@@ -645,6 +646,7 @@ __device__ inline void ke_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
     }
     uint32_t* slot = L.need + (blockIdx.x & (KE_NEED_SHARDS - 1));
     if (lane == first_lane && (uint32_t)m > *slot) atomicMax(slot, (uint32_t)m);
+    if (L.cneed && lane == first_lane && (uint32_t)m > L.cneed[cv.h->id]) atomicMax(&L.cneed[cv.h->id], (uint32_t)m);
   }
   KE_STAMP(5);
   if (L.prof) atomicMax(&L.prof[w * 8 + 7], ((unsigned long long)n << 32) | (unsigned long long)guard_total);

@@ -1,50 +1,61 @@
-// rpeg_kernel_quad.h - four lanes per plan, sixteen plans per wavefront (device only).
+// rpeg_kernel_quad.h - two or four lanes per plan, 32 or 16 plans of one class per wavefront (device only).
 //
-// For the classes whose wavefronts would end last in the plan-per-lane kernel (rpeg_kernel_eval.h): dense graphs
-// whose ready lists are long and whose keys go stale often.  There a scheduling step is a chain of dependent LDS
-// round trips; here the ready set of a plan lives in the REGISTERS of its four lanes, eight entries each, unordered:
+// The kernel of large batches.  The ready set of a plan lives in the REGISTERS of its QL lanes, SL entries each
+// (two, four or six, by what the classes of the launch need), unordered.  An entry:
 //
-//   entry = key (est, 8 bytes) | order word: position << 20 | tie | meta: node | reserved vertices << 12
+//   e     true start time: the larger of the node's key and the availability of the devices it reserves, raised at every
+//         dispatch that reserves one of them
+//   key   the key the reference's heap holds for it, where its position is shared (below); infinity elsewhere
+//   word  position << 20 | tie
+//   meta  node id | duration slot | reserved vertices | vertices whose allocations overlap those | register slot
 //
-// `position` is the place of the node in the order (comm_prio*8+topo_idx ascending, rank descending) of the plan's
-// nodes, equal for nodes that agree in both; `tie` counts pushes.  (est, position, tie) is the reference's heap key
-// (est, comm_prio, topo_idx, -rank, tie) of scheduler.py:427, so the heap is taken literally: a pop is the minimum
-// over the 32 entries (minima in each lane, two quad-permute steps across the lanes, no memory access), a stale
-// entry is re-keyed in place with a fresh tie (scheduler.py:437-443), a dispatched entry is cleared in place.  The
-// four lanes look at four successors at once; those that became ready are handed, in successor order, to the lanes
-// that have a free slot (one each per round, the rounds repeated until all are filed).  A plan with more than 32
-// entries ready at once, or more than 2^20 pushes, is not evaluated here: it is flagged (EvalLaunch::limit) and redone
-// by the launch that ends the call, whose ready list is as long as the graph.
+// Order.  The heap's key is (est, comm_prio, topo_idx, -rank, tie) (scheduler.py:427); (comm_prio, topo_idx, -rank) is
+// replaced by the node's position, equal for nodes that agree in all three.  The heap pops stale entries (key < e) in key
+// order and pushes each back with e and a fresh tie (scheduler.py:437-443) until the minimum is current: what it then
+// dispatches is the minimum of (e, position, tie).  Where no other node has a node's position, neither key nor tie of its
+// push-backs is ever looked at: they are not carried out.  For shared positions they are: first the entries with a key
+// below the smallest e (all of them stale) -- those that meet no other of their position side by side, the others one
+// after the other in the heap's order --, then, at that key, the stale ones whose (position, tie) is below the dispatched
+// one's.
 //
-// Per-plan state (ready time, rank, position, in-degree per node, duration per slot) is in LDS, interleaved by plan.
-// Before the scheduling loop the four lanes of a plan share the cost model (slots by lane), the per-vertex memory
-// terms, the positions and the initialisation; the rank sweep runs in all four alike.
+// So every plan of a wavefront dispatches one node per round, and all of them end together: a class has one node count.
+// (With every push-back carried out a round lasted as long as that of the plan with the most of them.)
+//
+// Per-plan state in LDS, interleaved by plan: ready time (the rank before that), in-degree and a word of everything
+// else a new entry needs, per node; durations by slot; availability by vertex.  A round is three LDS trips:
+// the successors' places and the duration of the dispatched node; the state of up to four successors, each looked at by
+// a lane that has room for it; the availability of their vertices.
+//
+// A plan with more entries ready at once than its lanes hold is not evaluated here: it is flagged (EvalLaunch::limit)
+// and redone by the launch that ends the call, a plan per wavefront.  Ranks go level by level with a node per lane of the plan.  A node's id is its place by
+// tie-break class, so that counting the larger ranks of its class walks through consecutive rows.
+//
+// Bound: LDS, which holds the wavefronts in flight to 1-2 per SIMD (13 bytes per node and 8 per slot for a plan), and
+// with them the latency of a round: measured on 65,536 GRPO plans with four lanes of four entries, a round is 394 vector,
+// 75 scalar and 24 LDS instructions, 40 % of its time vector issue and 38 % waiting.  DPO graphs (28 nodes) fill the SIMDs
+// and are bound by issue.
+// Scheduling a wavefront: 42-node GRPO class 60 us, 92 nodes 130-190, 28-node DPO class 35.  The step, main kernel and
+// the earlier form of this one (every push-back carried out) against now: 65,536 GRPO plans 460 -> 365 us, 1,048,576 DPO
+// plans 1,686 -> 1,225, 20,011 PPO plans 548 -> 410.
 #ifndef RPEG_KERNEL_QUAD_H
 #define RPEG_KERNEL_QUAD_H
 
 #include "rpeg_kernel_eval.h"
+#include "rpeg_kernel_sched.h"
 
 namespace rpeg {
 
-constexpr int KQ_LANES = 4;       // lanes per plan
-constexpr int KQ_PLANS = 16;      // plans per wavefront
-constexpr int KQ_ENTRIES = 32;    // ready entries per plan, spread over its lanes
-constexpr uint32_t KQ_TIE_BITS = 20, KQ_TIE_MASK = (1u << KQ_TIE_BITS) - 1u;
+constexpr uint32_t KQ_MAX_NODES = 512, KQ_MAX_SLOTS = 256;   // what the fields of an entry hold
+constexpr uint32_t KQ_TIE_BITS = 20, KQ_TIE_MASK = (1u << KQ_TIE_BITS) - 1u;   // (a round takes at most 1 + 24 + 24 ties and four per new entry: 2^15 for 512 nodes)
 constexpr uint32_t KQ_EMPTY = 0xFFFFFFFFu;
 
-// LDS of one wavefront of `np` plans: class tables (node records, successor lists), the class's reverse order and its
-// nodes grouped by tie-break class (uint16 each, first-node table of 17 words), plan fields, memory terms, then the
-// per-plan state [row][plan]: time and rank (a double per node each; ONE array for both unless the critical-chain
-// masses are asked for: a rank is not read again once the positions are known, a ready time not written before),
-// duration (double per slot), position (uint16 per node), in-degree (byte per node).
-__host__ __device__ inline size_t kq_tab_bytes(uint32_t nodes) { return ((size_t)nodes * 4 + 17 * 2 + 15) & ~size_t(15); }
-__host__ __device__ inline size_t kq_dyn_bytes(uint32_t nv, uint32_t np) {
-  (void)nv; (void)np;   // (plan fields and memory terms used to sit here: the prologue launch computes from them now)
-  return 0;
-}
-__host__ __device__ inline size_t kq_lds_bytes(uint32_t cls_bytes, uint32_t nodes, uint32_t slots, uint32_t nv, uint32_t np, bool mass) {
-  return cls_bytes + kq_tab_bytes(nodes) + kq_dyn_bytes(nv, np) +
-         (size_t)np * (((mass ? 16ull : 8ull) * nodes + 8ull * slots + 3ull * nodes + 15) & ~15ull);
+// LDS of one wavefront.  Class tables: node records, groups, level place -> id, group members and the first place of
+// every level; per plan [row][plan]: ready time and a neutral element (with the critical-chain masses start
+// times too), durations, availability by vertex, a zero and a row nobody reads, node words, in-degrees.
+__host__ __device__ inline size_t kq_tab_bytes(uint32_t nodes) { return (16ull * nodes + 4ull * nodes + 3 * 2ull * (nodes + 2) + 15) & ~size_t(15); }
+__host__ __device__ inline size_t kq_lds_bytes(uint32_t plans, uint32_t nodes, uint32_t slots, bool mass) {
+  return kq_tab_bytes(nodes) +
+         (size_t)plans * (((mass ? 2ull : 1ull) * 8ull * (nodes + 1) + 8ull * slots + 8ull * (RPEG_MAX_V + 2) + 5ull * nodes + 15) & ~15ull);
 }
 
 #if defined(__HIPCC__)
@@ -59,81 +70,87 @@ __device__ inline double kq_dpp(double v) {
 }
 constexpr int KQ_XOR1 = 0xB1, KQ_XOR2 = 0x4E;   // quad_perm [1,0,3,2], [2,3,0,1]
 
-// reductions over the four lanes of a plan (a quad)
+// min of two non-NaN doubles in one instruction
+__device__ inline double kq_vmin(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ inline double kq_vmin(double a, double b, double c, double d) {
+  double r, t;
+  asm("v_min_f64 %0, %2, %3\n\tv_min_f64 %1, %4, %5\n\tv_min_f64 %0, %0, %1" : "=&v"(r), "=&v"(t) : "v"(a), "v"(b), "v"(c), "v"(d));
+  return r;
+}
+// reductions over the lanes of a plan (two or four)
+template <int QL>
 __device__ inline uint32_t kq_or(uint32_t v) {
   v |= kq_dpp<KQ_XOR1>(v);
-  v |= kq_dpp<KQ_XOR2>(v);
+  if (QL == 4) v |= kq_dpp<KQ_XOR2>(v);
   return v;
 }
+template <int QL>
 __device__ inline uint32_t kq_min(uint32_t v) {
   uint32_t o = kq_dpp<KQ_XOR1>(v);
   v = o < v ? o : v;
-  o = kq_dpp<KQ_XOR2>(v);
-  v = o < v ? o : v;
+  if (QL == 4) {
+    o = kq_dpp<KQ_XOR2>(v);
+    v = o < v ? o : v;
+  }
   return v;
 }
+template <int QL>
 __device__ inline double kq_min(double v) {
-  v = __builtin_fmin(v, kq_dpp<KQ_XOR1>(v));
-  v = __builtin_fmin(v, kq_dpp<KQ_XOR2>(v));
+  v = kq_vmin(v, kq_dpp<KQ_XOR1>(v));
+  if (QL == 4) v = kq_vmin(v, kq_dpp<KQ_XOR2>(v));
   return v;
 }
 
+template <int QL, int SL>
 __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* lds) {
-  constexpr int QL = KQ_LANES, NP = KQ_PLANS;
-  constexpr int SL = KQ_ENTRIES / QL;       // ready entries per lane
-  constexpr int RW = NP;
+  constexpr int RW = KE_WAVE / QL;
   const int lane = threadIdx.x, p = lane / QL, q = lane % QL;
-  int first_lane = 0;
+  constexpr int first_lane = 0;
   const rpeg_problem_t& P = *L.P;
   const ClassView cv = class_view(L.pool + (L.wave_cls[w] & ~KE_CLS_LDS));   // uniform
-  const int n = (int)cv.h->n_nodes, n_slots = (int)cv.h->n_slots, n_succ_all = (int)cv.h->n_succ;
+  const int n = (int)cv.h->n_nodes, n_slots = (int)cv.h->n_slots, n_levels = (int)cv.h->n_levels, n_groups = (int)cv.h->n_groups;
 
   // ---- LDS carve-up
-  uint64_t* l_node = (uint64_t*)lds;                                  // NodeRec[n]
-  uint16_t* l_succ = (uint16_t*)(lds + (size_t)n * 8);                // uint16[n_succ]
-  uint16_t* l_topo = (uint16_t*)(lds + L.cls_bytes);                  // uint16[n]: the class's topological order
-  uint16_t* l_bykey = l_topo + L.ws_nodes;                            // uint16[n]: nodes grouped by tie-break class
-  uint16_t* l_kbeg = l_bykey + L.ws_nodes;                            // uint16[17]: first place of every tie-break class
-  uint8_t* dyn = lds + L.cls_bytes + kq_tab_bytes(L.ws_nodes);
-  uint8_t* sbase = dyn + kq_dyn_bytes(L.max_v, NP);
-  const size_t tr_rows = (L.mass ? 2 : 1) * (size_t)L.ws_nodes;   // rows of the time and rank arrays together
-  double* g_time = (double*)sbase + p;
-  double* g_rank = L.mass ? g_time + (size_t)L.ws_nodes * RW : g_time;
-  double* g_dur = (double*)sbase + tr_rows * RW + p;
-  uint16_t* g_pos = (uint16_t*)((double*)sbase + (tr_rows + L.ws_slots) * RW) + p;
-  uint8_t* g_deg = (uint8_t*)((uint16_t*)((double*)sbase + (tr_rows + L.ws_slots) * RW) + (size_t)L.ws_nodes * RW) + p;
+  LevelRec* l_rec = (LevelRec*)lds;
+  uint32_t* l_group = (uint32_t*)(l_rec + L.ws_nodes);
+  uint16_t* l_id = (uint16_t*)(l_group + L.ws_nodes);
+  uint16_t* l_gm = l_id + (L.ws_nodes + 2);
+  uint16_t* l_lbeg = l_gm + (L.ws_nodes + 2);
+  double* rows = (double*)(lds + kq_tab_bytes(L.ws_nodes));
+  double* g_time = rows + p;
+  rows += (size_t)(L.ws_nodes + 1) * RW;
+  double* g_start = rows + p;
+  if (L.mass) rows += (size_t)(L.ws_nodes + 1) * RW;
+  double* g_dur = rows + p;
+  rows += (size_t)L.ws_slots * RW;
+  double* g_lf = rows + p;
+  rows += (size_t)(RPEG_MAX_V + 2) * RW;
+  uint32_t* g_info = (uint32_t*)rows + p;
+  uint8_t* g_deg = (uint8_t*)((uint32_t*)rows + (size_t)L.ws_nodes * RW) + p;
 
-  const uint64_t pi = (uint64_t)L.perm[w * KE_WAVE + p];
+  // a place without a plan repeats the first one of the wavefront, without outputs: every lane is active throughout
+  const uint32_t entry = L.perm[w * KE_WAVE + p];
+  const bool idle = entry == KE_IDLE;
+  const uint64_t pi = (uint64_t)(idle ? L.perm[w * KE_WAVE] : entry);
   __syncthreads();  // the previous task of this wavefront is done with LDS
+  for (int i = lane; i < n; i += KE_WAVE) l_id[cv.orec[i].at] = (uint16_t)i;
+  if (lane == 0) l_id[n] = (uint16_t)n;
+  for (int i = lane; i < n_groups; i += KE_WAVE) l_group[i] = ((const uint32_t*)cv.group)[i];
+  for (int i = lane; i <= n_levels; i += KE_WAVE) l_lbeg[i] = cv.lbeg[i];
+  __syncthreads();
   for (int i = lane; i < n; i += KE_WAVE) {
-    l_node[i] = ((const uint64_t*)cv.node)[i];
-    l_topo[i] = cv.topo[i];
+    LevelRec r = cv.lrec[i];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) r.succ[k] = l_id[r.succ[k]];
+    l_rec[l_id[i]] = r;
   }
-  for (int i = lane; i < n_succ_all; i += KE_WAVE) l_succ[i] = cv.succ[i];
-  __syncthreads();
-  auto node_at = [&](int v) { NodeRec r; const uint64_t b = l_node[v]; __builtin_memcpy(&r, &b, 8); return r; };
-  // nodes grouped by tie-break class (comm_prio*8+topo_idx < 16), ascending: lane k counts and places class k
-  if (lane < 16) {
-    int cnt = 0;
-    for (int v = 0; v < n; ++v) cnt += node_at(v).ptkey == lane ? 1 : 0;
-    int beg = cnt;   // inclusive prefix over the 16 classes, then exclusive
-    for (int d = 1; d < 16; d <<= 1) {
-      const int o = __shfl_up(beg, d, 16);
-      if (lane >= d) beg += o;
-    }
-    beg -= cnt;
-    l_kbeg[lane] = (uint16_t)beg;
-    if (lane == 15) l_kbeg[16] = (uint16_t)(beg + cnt);
-    for (int v = 0; v < n; ++v)
-      if (node_at(v).ptkey == lane) l_bykey[beg++] = (uint16_t)v;
-  }
-  __syncthreads();
-  if (pi == KE_IDLE) return;   // all lanes of a plan leave together: the lane exchanges below stay within a plan
-  first_lane = __builtin_ctzll(__ballot(1));
+  for (int i = lane; i < (int)cv.h->n_gmembers; i += KE_WAVE) l_gm[i] = l_id[cv.glvl[i]];
   KE_STAMP(0);
 
-  const rpeg_struct_t& st = P.st[cv.h->structure];   // uniform (the class fixes the structure)
-  (void)st;
   // pair relations, penalty factor and gate bits of this plan and the durations of its class's slots (out of the table
   // of the slot universe) come from the prologue launches, by plan index
   const uint64_t ovl = L.aux_ovl[pi], dpne = L.aux_dpne[pi];
@@ -143,238 +160,340 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
   bool err = cv.h->error != 0;
   {   // a slot whose duration the reference could not compute (division by zero) is NaN; a share by each lane
     bool bad = false;
-    for (int s = q; s < n_slots; s += QL) {
-      const double d = L.dur[(size_t)cv.umap[s] * L.dur_stride + pi];
-      g_dur[s * RW] = d;
-      bad = bad || d != d;
+    for (int s0 = q; s0 < n_slots; s0 += 4 * QL) {   // four rows in flight
+      double d[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int s = s0 + k * QL;
+        d[k] = L.dur[(size_t)cv.umap[s < n_slots ? s : s0] * L.dur_stride + pi];
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int s = s0 + k * QL;
+        bad = bad || d[k] != d[k];
+        if (s < n_slots) g_dur[s * RW] = d[k];
+      }
     }
-    err = err || kq_or(bad ? 1u : 0u) != 0u;
+    err = err || kq_or<QL>(bad ? 1u : 0u) != 0u;
+    if (err)   // (no NaN in the loops below)
+      for (int s = q; s < n_slots; s += QL) g_dur[s * RW] = 0.0;
+  }
+  if (q == 0) {
+    g_time[n * RW] = 0.0;
+    for (int x = 0; x <= RPEG_MAX_V; ++x) g_lf[x * RW] = 0.0;
   }
   __syncthreads();
   KE_STAMP(2);
   const bool stale_ok = (gates & RPEG_MASK_STALE_OK) != 0, mem_ok = (gates & RPEG_MASK_MEM_OK) != 0;
 
   KE_STAMP(3);
-  // ---- ranks: reverse topological pass, then chain inheritance (scheduler.py:71-100, 367-378); all lanes alike
-  for (int i = n - 1; i >= 0; --i) {
-    const int v = l_topo[i];
-    const NodeRec nr = node_at(v);
-    double best = 0.0;
-    const double dv = g_dur[nr.slot * RW];
-    int j = 0;
-    for (; j + 2 <= nr.n_succ; j += 2) {   // two independent pairs of LDS reads in flight
-      const int u0 = l_succ[nr.succ_begin + j], u1 = l_succ[nr.succ_begin + j + 1];
-      const double r0 = g_rank[u0 * RW], r1 = g_rank[u1 * RW];
-      best = r0 > best ? r0 : best;
-      best = r1 > best ? r1 : best;
+  // ---- ranks: level by level from the nodes without successors, then chain inheritance (scheduler.py:71-100, 367-378);
+  // the record of the next level's node is read while this level's ranks are computed
+  {
+    int i = q, id = l_id[i < n ? i : 0];
+    LevelRec rec = l_rec[id];
+    for (int l = 0; l < n_levels; ++l) {
+      const int end = l_lbeg[l + 1], nx = end + q, id2 = l_id[nx < n ? nx : 0];
+      const LevelRec rec2 = l_rec[id2];
+      for (;;) {
+        const double d = g_dur[rec.slot * RW];
+        const double r0 = g_time[rec.succ[0] * RW], r1 = g_time[rec.succ[1] * RW], r2 = g_time[rec.succ[2] * RW], r3 = g_time[rec.succ[3] * RW];
+        double best = kp_vmax(kp_vmax(r0, r1), kp_vmax(r2, r3));
+        if (__builtin_expect(__ballot(i < end && rec.n_succ > 4) != 0ull, 0))
+          for (int j = 4; i < end && j < rec.n_succ; ++j) best = kp_vmax(best, g_time[l_id[cv.place[cv.succ[cv.node[rec.node].succ_begin + j]]] * RW]);
+        if (i < end) g_time[id * RW] = d + best;
+        i += QL;
+        if (__builtin_expect(__ballot(i < end) == 0ull, 1)) break;
+        id = l_id[i < n ? i : 0];
+        rec = l_rec[id];
+      }
+      i = nx;
+      id = id2;
+      rec = rec2;
     }
-    if (j < nr.n_succ) {
-      const double r = g_rank[(int)l_succ[nr.succ_begin + j] * RW];
-      best = r > best ? r : best;
-    }
-    g_rank[v * RW] = dv + best;
   }
-  for (unsigned g = 0; g < cv.h->n_groups; ++g) {
-    const GroupRec gr = cv.group[g];
-    double top = g_rank[(int)cv.gmember[gr.begin] * RW];
-    for (int j = 1; j < gr.count; ++j) {
-      const double r = g_rank[(int)cv.gmember[gr.begin + j] * RW];
+  for (int g = q; g < n_groups; g += QL) {
+    const int begin = (int)(l_group[g] & 0xFFFFu), count = (int)(l_group[g] >> 16);
+    double top = g_time[l_gm[begin] * RW];
+    for (int j = 1; j < count; ++j) {
+      const double r = g_time[l_gm[begin + j] * RW];
       top = r > top ? r : top;
     }
-    for (int j = 0; j < gr.count; ++j) g_rank[(int)cv.gmember[gr.begin + j] * RW] = top;
+    for (int j = 0; j < count; ++j) g_time[l_gm[begin + j] * RW] = top;
   }
   __syncthreads();
 #ifdef KE_FINE_PROF
   KE_STAMP(4);
 #endif
-  // ---- positions: nodes before v in (comm_prio*8+topo_idx ascending, rank descending) = the nodes of lower
-  // tie-break classes and the nodes of its own class with a larger rank
-  for (int i = q; i < n; i += QL) {
-    const int v = l_bykey[i];
-    const unsigned k = node_at(v).ptkey;
-    const int b0 = l_kbeg[k], b1 = l_kbeg[k + 1];
-    const double rv = g_rank[v * RW];
-    int cnt = b0;
-    int j = b0;
-    for (; j + 4 <= b1; j += 4) {   // four independent pairs of LDS reads in flight
-      const int u0 = l_bykey[j], u1 = l_bykey[j + 1], u2 = l_bykey[j + 2], u3 = l_bykey[j + 3];
-      const double r0 = g_rank[u0 * RW], r1 = g_rank[u1 * RW], r2 = g_rank[u2 * RW], r3 = g_rank[u3 * RW];
-      cnt += (r0 > rv ? 1 : 0) + (r1 > rv ? 1 : 0) + (r2 > rv ? 1 : 0) + (r3 > rv ? 1 : 0);
+  // ---- positions: nodes before v in (comm_prio*8+topo_idx ascending, rank descending) = the nodes of lower tie-break
+  // classes and the nodes of its own class with a larger rank; shared where more nodes than its own chain agree.
+  // Node word: position | shared << 9 | slot << 10 | reserved vertices << 18 | vertices that overlap them << 24
+  {
+    OrderRec next = cv.orec[q < n ? q : 0];
+    for (int i = q; i < n; i += QL) {
+      const OrderRec o = next;
+      next = cv.orec[i + QL < n ? i + QL : 0];
+      const double rv = g_time[i * RW];
+      const int b1 = o.b1;
+      int before = o.b0, same = 0, j = o.b0;
+      for (; j + 4 <= b1; j += 4) {   // four independent LDS reads in flight
+        const double r0 = g_time[j * RW], r1 = g_time[(j + 1) * RW], r2 = g_time[(j + 2) * RW], r3 = g_time[(j + 3) * RW];
+        before += (r0 > rv ? 1 : 0) + (r1 > rv ? 1 : 0) + (r2 > rv ? 1 : 0) + (r3 > rv ? 1 : 0);
+        same += (r0 == rv ? 1 : 0) + (r1 == rv ? 1 : 0) + (r2 == rv ? 1 : 0) + (r3 == rv ? 1 : 0);
+      }
+      for (; j < b1; ++j) {
+        const double r = g_time[j * RW];
+        before += r > rv ? 1 : 0;
+        same += r == rv ? 1 : 0;
+      }
+      const LevelRec rec = l_rec[i];
+      const uint32_t bt = kp_reserved(rec.blocked, rec.cond, ovl, dpne);
+      g_info[i * RW] = (uint32_t)before | (same > (int)o.chain_n ? 0x200u : 0u) | ((uint32_t)rec.slot << 10) | ((bt & 0x3Fu) << 18) | (((bt >> 8) & 0x3Fu) << 24);
+      g_deg[i * RW] = rec.indeg;
     }
-    for (; j < b1; ++j) cnt += g_rank[(int)l_bykey[j] * RW] > rv ? 1 : 0;
-    g_pos[v * RW] = (uint16_t)cnt;
   }
   __syncthreads();   // (the ranks are dead from here on: their array becomes the ready times)
-  for (int v = q; v < n; v += QL) {
-    g_deg[v * RW] = node_at(v).indeg;
-    g_time[v * RW] = 0.0;
-  }
+  for (int v = q; v < n; v += QL) g_time[v * RW] = 0.0;
   __syncthreads();
 
 #ifndef KE_FINE_PROF
   KE_STAMP(4);
 #endif
   // ---- list scheduling (scheduler.py:399-546)
-  double lf[RPEG_MAX_V];
-#pragma unroll
-  for (int x = 0; x < RPEG_MAX_V; ++x) lf[x] = 0.0;
   const double inf = __builtin_inf();
-  double ek[SL];
+  double ek[SL], sk[SL];
   uint32_t eo[SL], em[SL];
 #pragma unroll
-  for (int u = 0; u < SL; ++u) { ek[u] = inf; eo[u] = KQ_EMPTY; em[u] = 0u; }
-  uint32_t tie = 0;
+  for (int u = 0; u < SL; ++u) { ek[u] = inf; sk[u] = inf; eo[u] = KQ_EMPTY; em[u] = 0u; }
+  uint32_t tie = 0, free_slots = (1u << SL) - 1u;
+  int live = 0, longest = 0;   // entries now and at most
   bool ovf = false;
   const unsigned group_shift = (unsigned)(lane & ~(QL - 1));
   const uint32_t below = (1u << q) - 1u;   // the lanes of this plan before this one
-  // Entry `j` of a round of new entries goes to the j-th lane of the plan that has a free slot.  free_rank: the
-  // place of this lane among those lanes (QL if it has none); returns its first free slot in u_free.
-  auto free_rank = [&](int& u_free) {
-    uint32_t fm = 0;
+  // this lane keeps the availability of vertices q, q + QL, ... (where there are fewer: of the row behind the zeros)
+  constexpr int NLF = (RPEG_MAX_V + QL - 1) / QL;
+  double lf[NLF];
+  uint32_t lf_bit[NLF];
+  double* lf_row[NLF];
 #pragma unroll
-    for (int u = 0; u < SL; ++u) fm |= eo[u] == KQ_EMPTY ? 1u << u : 0u;
-    u_free = fm ? __builtin_ctz(fm) : SL;
-    const uint32_t g = (uint32_t)(__ballot(fm != 0u) >> group_shift) & ((1u << QL) - 1u);
-    return fm ? (int)__builtin_popcount(g & below) : QL;
-  };
-  auto file = [&](int u_free, double key, uint32_t ord, uint32_t node_blk) {
+  for (int k = 0; k < NLF; ++k) {
+    const int x = q + k * QL;
+    lf[k] = 0.0;
+    lf_bit[k] = x < RPEG_MAX_V ? 1u << (24 + x) : 0u;
+    lf_row[k] = g_lf + (x < RPEG_MAX_V ? x : RPEG_MAX_V + 1) * RW;
+  }
+  const mask64 quads0 = QL == 4 ? 0x1111111111111111ull : 0x5555555555555555ull;   // the first lane of every plan
+  // an entry into the first free slot of this lane, in the lanes of `take` (conditions are kept as masks of the lanes in
+  // scalar registers: as booleans the compiler moves them through vector registers)
+  auto file = [&](mask64 take, double key, uint32_t info, uint32_t place, uint32_t t) {
+    const uint32_t first = kp_sel(take, free_slots & (0u - free_slots), 0u), u_free = 31u - (uint32_t)__builtin_clz(first | 1u);
+    const uint32_t word = ((info & 0x1FFu) << KQ_TIE_BITS) | t, meta = (info & 0x3FFFFC00u) | place | (u_free << 30) | ((u_free >> 2) << 9);
+    const double heap_key = kp_sel(__ballot((info & 0x200u) != 0u), key, inf);
 #pragma unroll
-    for (int u = 0; u < SL; ++u)
-      if (u_free == u) { ek[u] = key; eo[u] = ord; em[u] = node_blk; }
+    for (int u = 0; u < SL; ++u) {
+      const mask64 m = __ballot(first == (1u << u));
+      ek[u] = kp_sel(m, key, ek[u]);
+      sk[u] = kp_sel(m, heap_key, sk[u]);
+      eo[u] = kp_sel(m, word, eo[u]);
+      em[u] = kp_sel(m, meta, em[u]);
+    }
+    free_slots ^= first;
   };
   {
     const int n_init = (int)cv.h->n_init;
-    if (n_init > KQ_ENTRIES) ovf = true;
-    for (int i0 = 0; i0 < n_init && !ovf; i0 += QL) {   // (at most 32 entries: every lane has room in every round)
-      int u_free;
-      const int r = free_rank(u_free);
-      const bool mine = r < QL && i0 + r < n_init;
-      if (mine) {
-        const int v = cv.init[i0 + r];
-        file(u_free, 0.0, ((uint32_t)g_pos[v * RW] << KQ_TIE_BITS) | (uint32_t)(i0 + r), (uint32_t)v | (blocked_mask(node_at(v), dpne) << 12));
-      }
+    ovf = n_init > QL * SL;
+    for (int i0 = 0; i0 < n_init && i0 < QL * SL; i0 += QL) {
+      const bool mine = i0 + q < n_init;
+      const uint32_t v = l_id[cv.place[cv.init[mine ? i0 + q : 0]]];
+      file(__ballot(mine), 0.0, g_info[v * RW], v, (uint32_t)(i0 + q));
     }
     tie = (uint32_t)n_init;
+    live = longest = n_init;
   }
-  if (kq_or(ovf ? 1u : 0u)) { ovf = true; err = true; }
   double makespan = 0.0;
-  int done = 0;
-  uint32_t guard_total = 0;
+  uint32_t n_back = 0;
+  mask64 lost = 0ull;                             // plans (all four lanes) with an entry that found no room
   auto min_u32 = [](uint32_t x, uint32_t y) { return x < y ? x : y; };
-  while (!err && done < n) {
-    // The heap's pops up to the next dispatch.  A pop: the smallest key of the 32 slots (minima in each lane, then
-    // across the lanes), the smallest order word among the slots of that key, the meta word of the slot that holds
-    // it (order words are unique).  A stale entry is re-keyed in place with a fresh tie (scheduler.py:437-443): every
-    // stale pop makes one entry current, so at most 32 follow one another.  An empty set pops an empty slot, never stale.
-    double bk, est;
-    uint32_t bo, bm;
-    for (;;) {
-      ++guard_total;
-      bk = ek[0];
+  auto key_min = [&](const double (&x)[SL]) {
+    double k;
+    if constexpr (SL == 2) k = kq_vmin(x[0], x[1]);
+    else if constexpr (SL == 4) k = kq_vmin(x[0], x[1], x[2], x[3]);
+    else k = kq_vmin(kq_vmin(x[0], x[1], x[2], x[3]), kq_vmin(x[SL - 2], x[SL - 1]));
+    return kq_min<QL>(k);
+  };
+  // the entry of word o (of every plan: its own) is pushed back
+  auto push_back = [&](uint32_t o) {
+    const uint32_t fresh = (o & ~KQ_TIE_MASK) | tie;
 #pragma unroll
-      for (int u = 1; u < SL; ++u) bk = __builtin_fmin(bk, ek[u]);
-      bk = kq_min(bk);
-      bo = KQ_EMPTY;
+    for (int u = 0; u < SL; ++u) {
+      const mask64 hit = __ballot(eo[u] == o);
+      sk[u] = kp_sel(hit, ek[u], sk[u]);
+      eo[u] = kp_sel(hit, fresh, eo[u]);
+    }
+    ++tie;   // (also in a plan that pushed nothing back: only the order of ties is looked at)
+  };
+  for (int done = 0; done < n; ++done) {
+    const double gk = key_min(ek);
+    // push-backs of entries of shared position below the smallest true start time
+    mask64 back[SL], more = 0ull;
 #pragma unroll
-      for (int u = 0; u < SL; ++u) bo = min_u32(bo, ek[u] == bk ? eo[u] : KQ_EMPTY);
-      bo = kq_min(bo);
-      bm = 0;
+    for (int u = 0; u < SL; ++u) {
+      back[u] = __ballot(sk[u] < gk);
+      more |= back[u];
+    }
+    if (more) {
+      // positions (by their low five bits) that occur twice among them
+      uint32_t bit[SL], seen = 0u, twice = 0u;
 #pragma unroll
-      for (int u = 0; u < SL; ++u) bm |= eo[u] == bo ? em[u] : 0u;
-      bm = kq_or(bm);
-      const double dv = ke_dev_max((bm >> 12) & 0xFFu, lf);
-      est = dv > bk ? dv : bk;
-      if (!(est > bk)) break;
-      const uint32_t no = (bo & ~KQ_TIE_MASK) | tie;
+      for (int u = 0; u < SL; ++u) {
+        bit[u] = kp_sel(back[u], 1u << ((eo[u] >> KQ_TIE_BITS) & 31u), 0u);
+        twice |= seen & bit[u];
+        seen |= bit[u];
+      }
+      uint32_t other = kq_dpp<KQ_XOR1>(seen);
+      twice |= (seen & other) | kq_dpp<KQ_XOR1>(twice);
+      if (QL == 4) {
+        seen |= other;
+        other = kq_dpp<KQ_XOR2>(seen);
+        twice |= (seen & other) | kq_dpp<KQ_XOR2>(twice);
+      }
+      more = 0ull;
+#pragma unroll
+      for (int u = 0; u < SL; ++u) {
+        const mask64 mates = back[u] & __ballot((bit[u] & twice) != 0u), alone = back[u] & ~mates;
+        more |= mates;
+        sk[u] = kp_sel(alone, ek[u], sk[u]);
+        eo[u] = kp_sel(alone, (eo[u] & ~KQ_TIE_MASK) | tie, eo[u]);
+      }
       ++tie;
+      while (more) {
+        ++n_back;
+        const double k = key_min(sk);
+        more = __ballot(k < gk);
+        uint32_t o = KQ_EMPTY;
 #pragma unroll
-      for (int u = 0; u < SL; ++u)
-        if (eo[u] == bo) { ek[u] = est; eo[u] = no; }
-    }
-    if (bo == KQ_EMPTY) { err = true; break; }
+        for (int u = 0; u < SL; ++u) o = min_u32(o, kp_sel(__ballot(sk[u] == k), eo[u], KQ_EMPTY));
+        push_back(kp_sel(more, kq_min<QL>(o), KQ_EMPTY - 1u));   // (no entry has that word)
+        more = 0ull;
 #pragma unroll
-    for (int u = 0; u < SL; ++u)   // the dispatched entry leaves its slot
-      if (eo[u] == bo) { ek[u] = inf; eo[u] = KQ_EMPTY; }
-    const int bv = (int)(bm & 0xFFFu);
-    const unsigned blocked = (bm >> 12) & 0xFFu;
-    const NodeRec nr = node_at(bv);
-    const double fin = est + g_dur[nr.slot * RW];
-    makespan = fin > makespan ? fin : makespan;
-    ++done;
-    if (L.mass && q == 0) {  // keep the trace: a dispatched node needs neither its ready time nor its rank again
-      g_time[bv * RW] = fin;
-      g_rank[bv * RW] = est;
-    }
-    unsigned touched = 0;
-#pragma unroll
-    for (int x = 0; x < RPEG_MAX_V; ++x)
-      if ((blocked >> x) & 1u) touched |= mask_row(ovl, x);
-#pragma unroll
-    for (int x = 0; x < RPEG_MAX_V; ++x)
-      if (((touched >> x) & 1u) && fin > lf[x]) lf[x] = fin;
-    // successors, QL at a time: lane q looks at successor j0 + q; those that became ready are filed in successor
-    // order (scheduler.py:540-546), the j-th of them by the j-th lane with a free slot
-    const int ns = nr.n_succ;
-    for (int j0 = 0; j0 < ns; j0 += QL) {
-      const bool mine = j0 + q < ns;
-      const int wn = mine ? (int)l_succ[nr.succ_begin + j0 + q] : 0;
-      bool ready = false;
-      double t = 0.0;
-      if (mine) {
-        const double t0 = g_time[wn * RW];
-        const uint8_t left = (uint8_t)(g_deg[wn * RW] - 1);
-        t = fin > t0 ? fin : t0;
-        ready = left == 0;
-        if (!ready) {
-          g_time[wn * RW] = t;
-          g_deg[wn * RW] = left;
-        }
+        for (int u = 0; u < SL; ++u) more |= __ballot(sk[u] < gk);
       }
-      uint32_t ord = 0, node_blk = 0;
+    }
+    uint32_t own = KQ_EMPTY;
+    mask64 level = 0ull;
+#pragma unroll
+    for (int u = 0; u < SL; ++u) {
+      const mask64 at_gk = __ballot(ek[u] == gk);
+      own = min_u32(own, kp_sel(at_gk, eo[u], KQ_EMPTY));
+      level |= __ballot(sk[u] == gk) & ~at_gk;
+    }
+    const uint32_t bo = kq_min<QL>(own);
+    // push-backs of entries with that key that come before the one to dispatch
+    if (__builtin_expect(level != 0ull, 0)) {
+      for (;;) {
+        uint32_t o = KQ_EMPTY;
+#pragma unroll
+        for (int u = 0; u < SL; ++u) o = min_u32(o, kp_sel(__ballot(sk[u] == gk) & __ballot(ek[u] > gk), eo[u], KQ_EMPTY));
+        o = kq_min<QL>(o);
+        const mask64 act = __ballot(o < bo);
+        if (!act) break;
+        push_back(kp_sel(act, o, KQ_EMPTY - 1u));
+      }
+    }
+    const mask64 alive = __ballot(gk < inf);   // (nothing waits: an entry was lost, or a start time is infinite: flagged)
+    lost |= ~alive;
+    uint32_t bm = 0;
+#pragma unroll
+    for (int u = 0; u < SL; ++u) {   // the dispatched entry leaves its slot
+      const mask64 hit = __ballot(eo[u] == bo);
+      bm = kp_sel(hit, em[u], bm);
+      ek[u] = kp_sel(hit, inf, ek[u]);
+      sk[u] = kp_sel(hit, inf, sk[u]);
+    }
+    const mask64 winner = __ballot(own == bo) & alive;
+    bm = kp_sel(winner, bm, 0u);
+    free_slots |= kp_sel(winner, 1u << ((bm >> 30) | ((bm >> 7) & 4u)), 0u);
+    bm = kq_or<QL>(bm);
+    mask64 room = __ballot(free_slots != 0u);
+    uint32_t in_plan = (uint32_t)(room >> group_shift) & ((1u << QL) - 1u);
+    uint32_t r = (uint32_t)__builtin_popcount(in_plan & below), n_room = (uint32_t)__builtin_popcount(in_plan);
+    const uint32_t place = bm & 0x1FFu;
+    const uint32_t first_succ = l_rec[place].succ[r], n_succ = l_rec[place].n_succ;
+    const double fin = gk + g_dur[(int)((bm >> 10) & 0xFFu) * RW];
+    if (L.mass) {   // the trace: a dispatched node does not need its ready time again
+      if (kp_in(alive & quads0)) {
+        g_time[place * RW] = fin;
+        g_start[place * RW] = gk;
+      }
+    }
+    makespan = kp_vmax(makespan, fin);
+#pragma unroll
+    for (int k = 0; k < NLF; ++k) {
+      lf[k] = kp_sel(__ballot((bm & lf_bit[k]) != 0u), kp_vmax(lf[k], fin), lf[k]);
+      lf_row[k][0] = lf[k];
+    }
+    --live;
+    const uint32_t touched = (bm >> 6) & (0x3Fu << 18);
+#pragma unroll
+    for (int u = 0; u < SL; ++u) ek[u] = kp_sel(__ballot((em[u] & touched) != 0u), kp_vmax(ek[u], fin), ek[u]);
+    // successors: the lanes with room look at one each; those that became ready are filed where they were looked at
+    // (scheduler.py:540-546: ties in successor order)
+    mask64 mine = room & alive & __ballot(r < n_succ);
+    uint32_t j0 = 0, sp = first_succ;
+    while (mine) {
+      const uint32_t at = kp_sel(mine, sp, 0u);
+      const double t0 = g_time[at * RW];
+      const uint32_t deg = g_deg[at * RW], info = g_info[at * RW];
+      const uint32_t left = deg - 1u;
+      double t = kp_vmax(t0, fin);
+      if (kp_in(mine)) {
+        g_time[at * RW] = t;
+        g_deg[at * RW] = (uint8_t)left;
+      }
+      const mask64 ready = mine & __ballot(left == 0u);
       if (ready) {
-        const unsigned blk = blocked_mask(node_at(wn), dpne);
-        const double d2 = ke_dev_max(blk, lf);
-        t = d2 > t ? d2 : t;
-        ord = (uint32_t)g_pos[wn * RW] << KQ_TIE_BITS;
-        node_blk = (uint32_t)wn | (blk << 12);
+        const uint32_t b6 = (info >> 18) & 0x3Fu;   // one vertex or two (none: the row of zeros)
+        const uint32_t v1 = (uint32_t)__builtin_ctz(b6 | (1u << RPEG_MAX_V)), v2 = b6 ? 31u - (uint32_t)__builtin_clz(b6) : (uint32_t)RPEG_MAX_V;
+        t = kp_vmax(t, kp_vmax(g_lf[v1 * RW], g_lf[v2 * RW]));
+        const uint32_t rdy = (uint32_t)(ready >> group_shift) & ((1u << QL) - 1u);
+        file(ready, t, info, at, tie + (uint32_t)__builtin_popcount(rdy & below));
+        tie += (uint32_t)QL;
+        live += (int)__builtin_popcount(rdy);
+        longest = live > longest ? live : longest;
       }
-      // hand the ready ones over: the j-th ready successor (lane order = successor order) to the j-th lane with room
-      const uint32_t rdy = (uint32_t)(__ballot(ready) >> group_shift) & ((1u << QL) - 1u);
-      const int n_rdy = __builtin_popcount(rdy);
-      if (n_rdy) {   // uniform within the plan
-        // A round hands one entry to every lane that has room; the rounds repeat until every entry is filed, so that a
-        // plan overflows only when fewer free slots than entries are left in all four lanes together.
-        uint32_t rem = rdy;
-        int filed = 0;
-        while (rem) {
-          int u_free;
-          const int r = free_rank(u_free);
-          const uint32_t room = (uint32_t)(__ballot(r < QL) >> group_shift) & ((1u << QL) - 1u);
-          const int n_room = __builtin_popcount(room), n_rem = __builtin_popcount(rem);
-          if (n_room == 0) { ovf = true; break; }
-          // source lane of the r-th ready successor still to file
-          uint32_t src_mask = rem;
-          for (int k = 0; k < r && k < QL; ++k) src_mask &= src_mask - 1u;
-          const bool take = r < n_rem;
-          const int src = (int)group_shift + (take ? __builtin_ctz(src_mask) : 0);
-          const double tk = __hiloint2double(__builtin_amdgcn_ds_bpermute(src << 2, __double2hiint(t)),
-                                             __builtin_amdgcn_ds_bpermute(src << 2, __double2loint(t)));
-          const uint32_t to = (uint32_t)__builtin_amdgcn_ds_bpermute(src << 2, (int)ord);
-          const uint32_t tm = (uint32_t)__builtin_amdgcn_ds_bpermute(src << 2, (int)node_blk);
-          file(take ? u_free : SL, tk, to | (tie + (uint32_t)(filed + r)), tm);
-          const int k_done = n_room < n_rem ? n_room : n_rem;
-          for (int k = 0; k < k_done; ++k) rem &= rem - 1u;
-          filed += k_done;
-        }
-        tie += (uint32_t)n_rdy;
+      j0 += n_room;
+      const mask64 again = alive & __ballot(j0 < n_succ);
+      if (__builtin_expect(again == 0ull, 1)) break;
+      room = __ballot(free_slots != 0u);
+      in_plan = (uint32_t)(room >> group_shift) & ((1u << QL) - 1u);
+      r = (uint32_t)__builtin_popcount(in_plan & below);
+      n_room = (uint32_t)__builtin_popcount(in_plan);
+      const mask64 full = again & __ballot(n_room == 0u);
+      lost |= full;
+      j0 = kp_sel(full, n_succ, j0);
+      mine = again & room & __ballot(j0 + r < n_succ);
+      sp = 0;
+      if (kp_in(mine)) {
+        const uint32_t j = j0 + r;
+        sp = j < 4u ? l_rec[place].succ[j] : l_id[cv.place[cv.succ[cv.node[l_rec[place].node].succ_begin + j]]];
       }
     }
-    if (kq_or(ovf ? 1u : 0u) || tie >= KQ_TIE_MASK - 64u) { ovf = true; err = true; }
   }
-  if (done != n) err = true;
-  if (ovf && q == 0) ke_flag_limit(L, pi, L.wave_cls[w] & ~KE_CLS_LDS);
+  ovf = ovf || kp_in(lost);
+  err = err || ovf;
+  if (ovf && q == 0 && !idle) ke_flag_limit(L, pi, L.wave_cls[w] & ~KE_CLS_LDS);
+  if (L.need) {   // the longest ready set of the wavefront, folded into one of the running maxima
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const int o = __shfl_xor(longest, off);
+      longest = o > longest ? o : longest;
+    }
+    uint32_t* slot = L.need + (blockIdx.x & (KE_NEED_SHARDS - 1));
+    if (lane == 0 && (uint32_t)longest > *slot) atomicMax(slot, (uint32_t)longest);
+    if (lane == 0 && L.cneed && (uint32_t)longest > L.cneed[cv.h->id]) atomicMax(&L.cneed[cv.h->id], (uint32_t)longest);
+  }
   KE_STAMP(5);
-  if (L.prof && q == 0) atomicMax(&L.prof[w * 8 + 7], ((unsigned long long)n << 32) | (unsigned long long)guard_total);
+  if (L.prof && lane == 0) L.prof[w * 8 + 7] = ((unsigned long long)n << 32) | (unsigned long long)(n + n_back);
 
   // ---- outputs
   uint8_t mask = RPEG_MASK_VALID;
@@ -392,7 +511,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
     out_makespan = makespan;
     out_score = score;
   }
-  if (q == 0) {
+  if (q == 0 && !idle) {
     if (L.makespan) L.makespan[pi] = out_makespan;   // (the peak is the prologue launch's output)
     if (L.score) L.score[pi] = out_score;
     if (L.mask) L.mask[pi] = mask;
@@ -402,7 +521,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
 #pragma unroll
         for (int x = 0; x < RPEG_MAX_V; ++x) m[x] = __builtin_nan("");
       } else {
-        critical_mass(cv, [&](int i) { return g_time[i * RW]; }, [&](int i) { return g_rank[i * RW]; }, m);
+        critical_mass(cv, [&](int i) { return g_time[l_id[cv.place[i]] * RW]; }, [&](int i) { return g_start[l_id[cv.place[i]] * RW]; }, m);
       }
 #pragma unroll
       for (int x = 0; x < RPEG_MAX_V; ++x) L.mass[pi * RPEG_MAX_V + x] = m[x];

@@ -72,6 +72,7 @@ def main() -> None:
         ok = E > 0
         S, E, N = S[ok], E[ok], N[ok]
         if len(S) == 0:
+            print(f"{name}: no tasks")
             continue
         d = E - S
         print(f"{name}: {len(S)} tasks, first start {S.min():.1f} us, last end {E.max():.1f} us, sum of durations "

@@ -414,6 +414,36 @@ def test_dense_classes_move_to_four_lanes_per_plan_once_measured():
     assert quad[0] == 0 and quad[1] > 0 and quad[2] > 0 and quad[3] == 0, quad
 
 
+@pytest.mark.parametrize("c,n", [(2, 17001), (4, 33333), (5, 20011), (3, 17003)])
+def test_the_forms_of_the_kernel_of_few_lanes_per_plan(c, n):
+    """Two and four lanes per plan, two, four and six entries per lane: wavefronts with places left over, graphs on both
+    sides of every limit, ready sets learned from one batch and outgrown by the plans of the next (those are redone by
+    the launch that ends the call), with and without the critical-chain masses.  Every call equals the host build."""
+    from rpeg_amd.engine.runtime import Engine
+    cfg, a = seeded_batch(c, n)
+    _, b = seeded_batch(c, n, start=n)
+    port = CpuPort(cfg.problem)
+    eng = Engine(cfg.problem)
+    try:
+        quad = []
+        for batch in (a, b):
+            ref = port.eval(batch, flags=abi.GATE_STALE, threads=16, want_mass=True)
+            for call in range(4):
+                mass = call == 2
+                out = eng.eval(batch, gate_stale=True, mass=mass)
+                quad.append(eng.stats()["quad_tasks"])
+                assert np.array_equal(out["mask"], ref["mask"]), call
+                for k in ("makespan", "peak", "score") + (("mass",) if mass else ()):
+                    assert same_bits(out[k], ref[k]), (call, k)
+        assert quad[3] > 0 and quad[7] > 0, quad
+        eng.set_state_lanes(4)      # every class, the smallest ones too, and classes that were never measured
+        small = port.eval(b, flags=abi.GATE_STALE, threads=16)
+        out = eng.eval(b, gate_stale=True)
+        assert same_bits(out["score"], small["score"]) and np.array_equal(out["mask"], small["mask"])
+    finally:
+        eng.close()
+
+
 def test_the_fitted_figures_of_the_split_move_plans_between_kernels_and_no_bit():
     """rpeg_engine_set_split_model: with the single-plan kernel made to look free, or the four-lanes-per-plan kernel,
     or both dear, other classes change kernels (the task counts say so); every call equals the host build."""
