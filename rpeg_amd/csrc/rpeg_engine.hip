@@ -776,7 +776,7 @@ struct rpeg_engine_s {
   int sa_lanes = 3;     // rpeg_sa_run: groups of chains whose evaluations overlap the host's work on the others
   int lanes_busy = 0;   // evaluations submitted on lanes and not yet collected (their kernels read d_pool)
   uint64_t relearn_at = 0;                // the call that last asked for the measurements again
-  uint32_t one_plan_waves_per_cu = 64;    // batches of at most this many plans per compute unit take one wavefront per plan
+  uint32_t one_plan_waves_per_cu = 52;    // batches of at most this many plans per compute unit take one wavefront per plan
   uint32_t host_small_max = 1024;          // rpeg_eval_host: largest batch whose classes the host looks up itself
   int state_lanes = -1;   // -1: chosen per batch; 0: per-plan state in HBM; 8/16/32/64: in LDS, that many plans per wavefront; 1: one plan per wavefront (k_plan)
   bool prof_on = false;
@@ -1597,6 +1597,8 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // wavefronts of fewer plans whose state fits in LDS, which shortens every scheduler step.
   int ls = e->state_lanes;
   bool one = false;   // one plan per wavefront (k_plan)
+  const bool plan_fits = e->max_nodes <= (uint32_t)(WAVE * KP_MAX_NS) && kp_lds_bytes(e->max_nodes, e->max_slots) <= 64 * 1024;
+  const bool quad_free = ls == -1 && e->quad_share_pct && e->split_heavy && plan_fits;   // k_quad may take the batch (plan_quad)
   const bool quad_all = ls == 4;   // every class in the kernel of two or four lanes per plan (k_quad)
   if (quad_all) {
     ls = 0;
@@ -1615,7 +1617,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       ls = 0;
       if (one_fits && waves_for(1) <= (uint64_t)e->n_cu * e->one_plan_waves_per_cu) {
         one = true;   // the batch does not fill the chip with a plan per lane: spread every plan over a wavefront
-      } else if (waves_for(WAVE) < (uint64_t)e->n_cu * 2) {   // under two wavefronts per compute unit
+      } else if (waves_for(WAVE) < (uint64_t)e->n_cu * 2 && !quad_free) {   // under two wavefronts per compute unit
         for (int l : {8, 16, 32, 64}) {              // fewest plans per wavefront that still gives each its own SIMD
           if (!fits(l)) break;
           ls = l;
@@ -1661,7 +1663,6 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     return need == 0 ? 2 : need <= QUAD_KIND[0].entries && e->cls_nodes[cids[c]] <= QUAD_TWO_NODES ? 0 : need <= QUAD_KIND[1].entries ? 1 : 2;
   };
   std::vector<uint8_t> solo(counts.size(), 0), quad(counts.size(), quad_all ? 1 : 0);
-  const bool plan_fits = e->max_nodes <= (uint32_t)(WAVE * KP_MAX_NS) && kp_lds_bytes(e->max_nodes, e->max_slots) <= 64 * 1024;
   constexpr uint32_t QUAD_TINY = 8, QUAD_MEAN_NODES = 128;
   // k_quad takes the batch, with k_plan beside it, where the model below has them done before the main kernel would be.
   // Into k_plan go the classes of fewer than QUAD_TINY plans (a wavefront of k_quad lasts as long with one plan as with
@@ -1677,7 +1678,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // few plans have room in LDS, and the main kernel keeps its state in HBM: a batch of more than sixteen of its wavefronts
   // per compute unit stays there where the plans have more than QUAD_MEAN_NODES nodes on average.
   auto plan_quad = [&]() -> bool {
-    if (e->state_lanes != -1 || !e->quad_share_pct || !e->split_heavy || !plan_fits) return false;
+    if (!quad_free) return false;
     const DeepModel dm = deep_model(e, rcap_main);
     double t_sum = 0.0, nodes_sum = 0.0, pops_sum = 0.0;
     uint64_t takes = 0, measured = 0, known = 0, nodes = 0, main_tasks = 0;
@@ -1689,8 +1690,12 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       if (w) { t_sum += (double)(w >> 12); nodes_sum += (double)e->cls_nodes[cids[c]]; pops_sum += (w & 0xFFFu) / 16.0; ++known; }
     }
     if (nodes > QUAD_MEAN_NODES * n && main_tasks > (uint64_t)e->n_cu * 16) return false;
-    if (!measured || measured * 2 < takes || !known || t_sum <= 0.0) return false;
-    const double per_node = t_sum / nodes_sum, pops = pops_sum / (double)known;
+    // (A batch of under two wavefronts of the main kernel per compute unit is not for that kernel, whatever it has measured:
+    // k_plan with 64 plans per compute unit and the main kernel with 8 to 64 plans per wavefront beyond that / k_quad, us
+    // per step: DPO 16,384 plans 194 / 137, 20,000 212 / 137; PPO 16,384 473 / 393; AC-share 16,384 1,030 / 850.)
+    const bool shallow = main_tasks < (uint64_t)e->n_cu * 2;
+    if (!shallow && (!measured || measured * 2 < takes || !known || t_sum <= 0.0)) return false;
+    const double per_node = known ? t_sum / nodes_sum : 0.0, pops = known ? pops_sum / (double)known : 2.0;
     double w_main = 0.0, max_main = 0.0, w_quad = 0.0, w_plan = 0.0;
     auto t_quad = [&](uint32_t c) {   // one wavefront
       const uint32_t w = e->cls_pops16[cids[c]];
@@ -1720,7 +1725,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       if (best == 0.0 || t < dm.sm.gain_classes * best) { best = t; best_k = k; }
       if (k < order.size()) { w_quad -= cost_quad(order[k]); w_plan += cost_plan(order[k]); }
     }
-    if (!(dm.sm.quad_margin * best < dm.best(w_main, base_plan, max_main, nullptr))) return false;
+    if (!shallow && !(dm.sm.quad_margin * best < dm.best(w_main, base_plan, max_main, nullptr))) return false;
     for (size_t k = 0; k < order.size(); ++k) {
       const uint32_t c = order[k];
       if (to_plan[c] || k < best_k) solo[c] = 1;
