@@ -334,7 +334,7 @@ __global__ __launch_bounds__(WAVE) void k_prologue(const PrologueLaunch L) {
     const bool mine = active && su == s0;
     todo &= ~__ballot(mine);
     if (mine)
-      for (int row = (int)blockIdx.y; row < (int)(L.max_uni + 1 + RPEG_MAX_V); row += (int)gridDim.y) kpro_row(L, i, s0, split, row);
+      for (int row = (int)(L.row_begin + blockIdx.y); row < (int)L.row_end; row += (int)gridDim.y) kpro_row(L, i, s0, split, row);
   }
 }
 
@@ -1486,6 +1486,8 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     G.aux_pen = e->d_aux_pen; G.aux_mask = e->d_aux_mask;
     G.peak = peak;
     const unsigned pblk = (unsigned)((n + WAVE - 1) / WAVE);
+    G.row_begin = 0;
+    G.row_end = e->max_uni + 1 + (defer ? 0 : e->max_v);
     hipLaunchKernelGGL(k_prologue, dim3(pblk, KPRO_PARTS), dim3(WAVE), 0, ahead ? e->s3 : s, G);
     if (!defer) hipLaunchKernelGGL(k_peaks, dim3(pblk), dim3(WAVE), kpeaks_lds_bytes(e->max_v), s, G);
     HIP_TRY(e, hipGetLastError());
@@ -2192,7 +2194,13 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   }
   // (k_quad second: measured against k_quad first, 0.50 against 0.52-0.53 ms on config 2, and against k_quad last,
   // 0.59 ms; its wavefronts need the most LDS after the main kernel's)
-  if (quad_launch[2].waves || quad_launch[3].waves) HIP_TRY(e, hipStreamWaitEvent(e->s4, e->ev_fork, 0));
+  // The memory-model launches of a batch without work for the main kernel: behind k_plan where that has next to nothing to
+  // do (another stream costs an event between streams, 15 us: 16,384 DPO plans 126 against 143 us), else on the fourth
+  // stream where it is free, else behind k_quad's first launch (behind k_plan they ended the call: 65,536 GRPO plans
+  // 365 against 353 us, 20,011 PPO plans 409 against 381).
+  const bool peaks_apart = peaks_deferred && !peaks_aside && !n_waves, peaks_on_s2 = peaks_apart && n_solo && n_solo <= (uint32_t)e->n_cu;
+  const bool quad_on_s4 = quad_launch[2].waves || quad_launch[3].waves, peaks_on_s4 = peaks_apart && !peaks_on_s2 && !quad_on_s4;
+  if (quad_on_s4 || peaks_on_s4) HIP_TRY(e, hipStreamWaitEvent(e->s4, e->ev_fork, 0));
   if (int rc = launch_quad(quad_launch[2], e->s4)) return rc;
   if (int rc = launch_quad(quad_launch[0], sm)) return rc;
   if (int rc = launch_quad(quad_launch[1], sq)) return rc;
@@ -2210,7 +2218,11 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   }
   if (peaks_deferred) {
     const unsigned pblk = (unsigned)((n + WAVE - 1) / WAVE);
-    hipLaunchKernelGGL(k_peaks, dim3(pblk), dim3(WAVE), kpeaks_lds_bytes(e->max_v), peaks_aside ? sq : n_solo && !n_waves ? e->s2 : sm, G);
+    const hipStream_t sp = peaks_aside ? sq : peaks_on_s2 ? e->s2 : peaks_on_s4 ? e->s4 : sm;
+    G.row_begin = e->max_uni + 1;   // (the memory terms, which nothing but this launch needs: not ahead of the scheduling kernels)
+    G.row_end = G.row_begin + e->max_v;
+    hipLaunchKernelGGL(k_prologue, dim3(pblk, e->max_v), dim3(WAVE), 0, sp, G);
+    hipLaunchKernelGGL(k_peaks, dim3(pblk), dim3(WAVE), kpeaks_lds_bytes(e->max_v), sp, G);
     HIP_TRY(e, hipGetLastError());
   }
   if (n_solo) HIP_TRY(e, hipEventRecord(e->ev_join, e->s2));
@@ -2236,7 +2248,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     ahead_join.joined = true;
   }
   if (n_solo) HIP_TRY(e, hipStreamWaitEvent(s, e->ev_join, 0));
-  if (quad_launch[2].waves || quad_launch[3].waves) {
+  if (quad_on_s4 || peaks_on_s4) {
     HIP_TRY(e, hipEventRecord(e->ev_join4, e->s4));
     HIP_TRY(e, hipStreamWaitEvent(s, e->ev_join4, 0));
   }

@@ -42,7 +42,8 @@ struct PrologueLaunch {
   const uint32_t* cid;         // per plan: KPRO_INVALID for a plan the gate rejected
   const SlotDesc* uni;         // [structure][RPEG_MAX_UNIVERSE]
   uint32_t n_uni[RPEG_MAX_STRUCT];
-  uint32_t max_uni;            // rows of the grid: max_uni durations, one row of pair relations, then one per vertex
+  uint32_t max_uni;            // rows: max_uni durations, one row of pair relations, then one per vertex
+  uint32_t row_begin, row_end; // the rows of a launch of the first kind
   uint32_t max_v;              // largest vertex count of the problem's structures (sizes the LDS of the second launch)
   double* dur;
   uint64_t dur_stride;         // plans per row of dur and vm
