@@ -35,9 +35,9 @@ ALG_FLOPS = {1: 3697.0, 2: 2165.3, 3: 6502.9, 4: 1245.8, 5: 4155.6}
 # (FETCH_SIZE / WRITE_SIZE scaled by a 256 MiB copy) and instructions issued per plan (SQ_INSTS_VALU + SALU + LDS +
 # VMEM_RD + VMEM_WR of the evaluation kernels / plans).
 MEASURED = {
-    2: dict(layout=(6330, 17648, 0, 4815, 574), traffic=209.8e6, instructions_per_plan=3157.5),
+    2: dict(layout=(4101, 21536, 0, 1524, 2577), traffic=89.3e6, instructions_per_plan=1414.0),
     3: dict(layout=(24672, 29984, 0, 20364, 0), traffic=4639.9e6, instructions_per_plan=None),
-    4: dict(layout=(16396, 14640, 0, 6, 0), traffic=1547.6e6, instructions_per_plan=None),
+    4: dict(layout=(32781, 14640, 0, 6, 32775), traffic=357.4e6, instructions_per_plan=None),
 }
 
 
@@ -360,8 +360,9 @@ def main():
     if stats["state_lanes"] == 1:
         kernel_name = "k_plan"
     elif stats["single_plan_tasks"] and stats.get("quad_tasks"):
-        kernel_name = (f"k_eval<0> beside k_quad ({stats['quad_tasks']} wavefronts of 16 plans) and k_plan "
-                       f"({stats['single_plan_tasks']} plans), one launch each, timed from fork to join")
+        main = "" if stats["quad_tasks"] + stats["single_plan_tasks"] == stats["wave_tasks"] else "k_eval<0> beside "
+        kernel_name = (f"{main}k_quad ({stats['quad_tasks']} wavefronts of 16 or 32 plans) and k_plan "
+                       f"({stats['single_plan_tasks']} plans), timed from fork to join")
     elif stats["single_plan_tasks"]:
         kernel_name = f"k_eval<0> beside k_plan ({stats['single_plan_tasks']} plans), one launch each, timed from fork to join"
     else:
