@@ -30,7 +30,7 @@ ALG_BYTES = {1: 149, 2: 109, 3: 149, 4: 89, 5: 149}
 ALG_FLOPS = {1: 3697.0, 2: 2165.3, 3: 6502.9, 4: 1245.8, 5: 4155.6}
 # Counter figures of one step.  A run cannot read hardware counters of itself: these come from the rocprofv3 --pmc
 # summaries under profiles/ and are printed only when the run's kernel layout (`layout`: wave tasks, LDS bytes, plans
-# per wavefront with LDS state, single-plan tasks, four-lanes-per-plan tasks of rpeg_engine_stats) is the profiled
+# per wavefront with LDS state, single-plan tasks, few-lanes-per-plan tasks of rpeg_engine_stats) is the profiled
 # one to within 5 % in every task count; any other run prints null.  HBM bytes of the evaluation kernels
 # (FETCH_SIZE / WRITE_SIZE scaled by a 256 MiB copy) and instructions issued per plan (SQ_INSTS_VALU + SALU + LDS +
 # VMEM_RD + VMEM_WR of the evaluation kernels / plans).

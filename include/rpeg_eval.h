@@ -49,8 +49,8 @@ enum {
   RPEG_MASK_LIMIT = 16     /* set with RPEG_MASK_ERROR when the cause is a limit of this engine: the
                               reference would have evaluated the plan.  No evaluation path sets it
                               for a graph within the stated bounds (4,095 lowered nodes per plan):
-                              a plan whose ready set outgrows what a kernel holds -- 31 or 32 entries
-                              in the plan-per-lane and four-lanes-per-plan kernels -- is redone by
+                              a plan whose ready set outgrows what a kernel holds -- 31 entries in
+                              the plan-per-lane kernel, 8 to 24 in the few-lanes-per-plan one -- is redone by
                               the launch that ends the call with a ready list of one entry per
                               node, as the reference's heap has no capacity
                               (RPEG/schedule/scheduler.py:423-546)                                */
@@ -451,7 +451,7 @@ int rpeg_sa_propose(rpeg_engine_t* e, const rpeg_sa_params_t* prm, int32_t what,
    by this call, [2] wave tasks, [3] dynamic LDS bytes of the evaluation kernel, [4] workspace bytes,
    [5] plans per wavefront with LDS-resident state (0: state in the HBM workspace; 1: one plan per
    wavefront), [6] plans of a large batch that ran one per wavefront beside the main kernel (included
-   in [2]), [7] wave tasks of the four-lanes-per-plan kernel (included in [2]). */
+   in [2]), [7] wave tasks of the few-lanes-per-plan kernel (included in [2]). */
 int rpeg_engine_stats(const rpeg_engine_t* e, uint64_t* out, int32_t n);
 
 /* Host time of the last rpeg_eval_batch call that laid its batch out, in microseconds of the steady clock: [0] from
@@ -507,8 +507,9 @@ int rpeg_engine_set_side_layout(rpeg_engine_t* e, int32_t on);
 int rpeg_engine_set_quad_share(rpeg_engine_t* e, int32_t percent);
 
 /* Ready-list entries per plan in the main kernel: 8, 16, 24 or 32 (default).  A plan with that many nodes
-   ready at once is redone, without a bound, by the launch that ends the call (one plan per lane, its state and
-   ready list in HBM: slow, and rare -- the longest list seen on the shipped problems is 24).  Fewer entries take
+   ready at once is redone, without a bound, by the launch that ends the call (one plan per wavefront; above
+   384 nodes one plan per lane with its state and ready list in HBM: slow, and rare -- the longest list seen on the
+   shipped problems is 24).  Fewer entries take
    less LDS per wavefront.  The kernel that runs one plan per wavefront (small batches) keeps its ready set in
    registers and has no such bound.  Results do not depend on the setting.  No reference counterpart: tests use
    it to reach the redo path. */

@@ -5,10 +5,12 @@
 //   host          new signatures are lowered once into class blobs (rpeg_lower.h) and cached in
 //                 the engine; plans are ordered by class so that the lanes of a wavefront walk the
 //                 same graph tables
-//   k_eval        one thread per plan: durations of the class's slots (fp64 cost model), ranks,
-//                 list scheduling, per-device memory peaks, score.  Per-plan state lives in a
-//                 workspace laid out [row][lane] per wavefront (coalesced whenever lanes agree on
-//                 the row); the ready list lives in LDS, [entry][lane].
+//   k_quad        two or four lanes per plan: full batches (rpeg_kernel_quad.h); beside it
+//   k_plan        one wavefront per plan: small batches, small classes and the largest graphs (rpeg_kernel_plan.h)
+//   k_eval        one thread per plan: what the two above have not measured yet or have no room for; durations come from
+//                 k_prologue, then ranks, list scheduling, score.  Per-plan state lives in a workspace laid out
+//                 [row][lane] per wavefront (coalesced whenever lanes agree on the row); the ready list lives in LDS,
+//                 [entry][lane] (rpeg_kernel_eval.h)
 //
 // Build: hipcc --offload-arch=gfx950 -O3 -ffp-contract=off (no fused multiply-add may be formed:
 // the scores must equal the reference's Python floats bit for bit).
@@ -404,7 +406,7 @@ __global__ __launch_bounds__(WAVE) void k_eval(const EvalLaunch L) {
   }
 }
 
-// Four lanes per plan, sixteen plans per wavefront (rpeg_kernel_quad.h); tasks and permutation as for k_eval.
+// Two or four lanes per plan, 32 or 16 plans per wavefront (rpeg_kernel_quad.h); tasks and permutation as for k_eval.
 // QL: lanes per plan; SL: ready entries per lane.
 struct QuadKind { uint32_t plans, entries; };
 constexpr QuadKind QUAD_KIND[3] = {{32, 8}, {16, 16}, {16, 24}};   // k_quad<2, 4>, <4, 4>, <4, 6>
@@ -797,7 +799,7 @@ struct rpeg_engine_s {
   hipEvent_t ev_counts = nullptr;               // the statistic of a call has reached the host (the calls that read it)
   hipStream_t s4 = nullptr;                     // fourth stream and its join: k_quad's second launches
   hipEvent_t ev_join4 = nullptr;
-  hipStream_t s3 = nullptr;                     // third stream: the four-lanes-per-plan wavefronts (k_quad)
+  hipStream_t s3 = nullptr;                     // third stream: the few-lanes-per-plan wavefronts (k_quad)
   hipEvent_t ev_join3 = nullptr;
   hipEvent_t ev_sig = nullptr;                  // the signature kernel of a call is done (its class ids are there)
   bool layout_ahead = true;                     // prologue, layout and main kernel on k_quad's stream (see `ahead` in eval_batch_impl)

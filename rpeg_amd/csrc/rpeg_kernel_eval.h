@@ -652,7 +652,7 @@ __device__ inline void ke_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
   if (L.prof) atomicMax(&L.prof[w * 8 + 7], ((unsigned long long)n << 32) | (unsigned long long)guard_total);
   if (LS == 0 && L.cstat && !(L.flags & KE_FIXUP) && n > 0) {
     // what the wavefront paid per dispatch: the pops of its slowest plan.  The host reads it to decide which
-    // classes are worth four lanes per plan.
+    // batches are worth k_quad.
     uint32_t g = (uint32_t)guard_total;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {

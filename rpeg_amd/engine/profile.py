@@ -4,7 +4,7 @@
 
 Runs the seeded candidate set of the configuration through rpeg_eval_batch with the per-wavefront stamps switched
 on (rpeg_engine_profile) and prints, for the main kernel (k_eval) and for the one-plan-per-wavefront kernel
-(k_plan) and the four-lanes-per-plan kernel (k_quad) beside it: when their tasks start and end, how many run at a time, the longest tasks, and the durations
+(k_plan) and the few-lanes-per-plan kernel (k_quad) beside it: when their tasks start and end, how many run at a time, the longest tasks, and the durations
 by node count.  A kernel ends with its slowest wavefront, so the table of the longest tasks is the critical
 path of the step.
 
@@ -27,7 +27,7 @@ def main() -> None:
     ap.add_argument("--config", type=int, default=2)
     ap.add_argument("--plans", type=int, default=0, help="plans of the seeded set (default: the configuration's own size)")
     ap.add_argument("--sections", action="store_true", help="section clocks of the scheduling loop (measurement build)")
-    ap.add_argument("--quad-share", type=int, default=-1, help="percent of the batch for the four-lanes-per-plan kernel (default: the engine's)")
+    ap.add_argument("--quad-share", type=int, default=-1, help="percent of the batch for the few-lanes-per-plan kernel (default: the engine's)")
     args = ap.parse_args()
     import torch
     from .. import build as B, configs

@@ -215,7 +215,7 @@ class Engine:
 
     def set_state_lanes(self, lanes: int):
         """-1 automatic; 0 scheduler state in HBM (64 plans per wavefront); 8/16/32/64 state in LDS; 1 a plan per
-        wavefront; 4 four lanes per plan."""
+        wavefront; 4 two or four lanes per plan."""
         self._check(self.lib.rpeg_engine_set_state_lanes(self._h, int(lanes)), "rpeg_engine_set_state_lanes")
 
     def host_us(self) -> Dict[str, float]:
@@ -238,7 +238,7 @@ class Engine:
         self._check(self.lib.rpeg_engine_set_side_layout(self._h, 1 if on else 0), "rpeg_engine_set_side_layout")
 
     def set_quad_share(self, percent: int):
-        """Percentage of a full batch that the four-lanes-per-plan kernel takes beside the main kernel (0: none)."""
+        """Whether full batches may run in the few-lanes-per-plan kernel (percent > 0; 0: no)."""
         self._check(self.lib.rpeg_engine_set_quad_share(self._h, int(percent)), "rpeg_engine_set_quad_share")
 
     def set_ready_cap(self, entries: int):
