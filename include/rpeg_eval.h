@@ -451,7 +451,9 @@ int rpeg_sa_propose(rpeg_engine_t* e, const rpeg_sa_params_t* prm, int32_t what,
    by this call, [2] wave tasks, [3] dynamic LDS bytes of the evaluation kernel, [4] workspace bytes,
    [5] plans per wavefront with LDS-resident state (0: state in the HBM workspace; 1: one plan per
    wavefront), [6] plans of a large batch that ran one per wavefront beside the main kernel (included
-   in [2]), [7] wave tasks of the few-lanes-per-plan kernel (included in [2]). */
+   in [2]), [7] wave tasks of the few-lanes-per-plan kernel (included in [2]), [8] plans that the call BEFORE the last
+   one redid because their ready sets outgrew their kernel's (both calls laid out by the host: a batch that needed no
+   layout leaves the figure as it is). */
 int rpeg_engine_stats(const rpeg_engine_t* e, uint64_t* out, int32_t n);
 
 /* Host time of the last rpeg_eval_batch call that laid its batch out, in microseconds of the steady clock: [0] from

@@ -110,11 +110,15 @@ __global__ void k_upload_fill(const uint4* __restrict__ host_src, uint4* __restr
 // counters become their offsets within the class, in place (k_scatter reads them there); the totals go to the host:
 // written into pinned host memory, then a flag the host polls -- there several microseconds before a copy command
 // behind the kernel would have moved its first byte.  host_count: n_classes totals, the count of the plans of classes
-// not lowered yet, then the KE_NEED_SHARDS running maxima of the ready-list length.
+// not lowered yet, the KE_NEED_SHARDS running maxima of the ready-list length, and the plans that the engine's last
+// laid-out call redid without a bound on the ready set (limit[0]); where there were any, host_need: the longest ready
+// set of every class, so that this call already gives those plans' classes a form with room for them.
 constexpr int HAND_BLOCK = 1024;
 __global__ __launch_bounds__(HAND_BLOCK) void k_hand_counts(uint32_t* __restrict__ count, const uint32_t* __restrict__ need, uint32_t n_classes,
-                                                            uint32_t shards, uint32_t* __restrict__ host_count, uint32_t* __restrict__ host_flag,
-                                                            uint32_t tag) {
+                                                            uint32_t shards, const uint32_t* __restrict__ limit,
+                                                            const uint32_t* __restrict__ cneed, uint32_t* __restrict__ host_count,
+                                                            uint32_t* __restrict__ host_need, uint32_t* __restrict__ host_flag, uint32_t tag) {
+  const uint32_t redone = limit[0];
   // the totals first, and on their way to the host before anything else is written
   for (uint32_t c = threadIdx.x; c < n_classes; c += HAND_BLOCK) {
     const uint32_t* row = count + (size_t)c * shards;
@@ -130,6 +134,9 @@ __global__ __launch_bounds__(HAND_BLOCK) void k_hand_counts(uint32_t* __restrict
   }
   if (threadIdx.x == 0) host_count[n_classes] = count[(size_t)n_classes * shards];
   if (threadIdx.x < KE_NEED_SHARDS) host_count[n_classes + 1 + threadIdx.x] = need[threadIdx.x];
+  if (threadIdx.x == 0) host_count[n_classes + 1 + KE_NEED_SHARDS] = redone;
+  if (redone)
+    for (uint32_t c = threadIdx.x; c < n_classes; c += HAND_BLOCK) host_need[c] = cneed[c];
   __threadfence_system();
   __syncthreads();
   if (threadIdx.x == 0) __hip_atomic_store(host_flag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -753,7 +760,8 @@ struct rpeg_engine_s {
   uint64_t count_clean = 0;                     // leading words of d_ccount that the last call left at zero,
   hipStream_t count_clean_on = nullptr;         // on this stream
   uint32_t* h_ccount_dev = nullptr;             // the same pinned buffer as the device addresses it
-  uint32_t *h_tot = nullptr, *h_tot_dev = nullptr;   // pinned: per-class totals of a call, written by k_hand_counts
+  uint32_t *h_tot = nullptr, *h_tot_dev = nullptr;   // pinned: per-class totals of a call (tot_words), then per-class ready-set lengths, written by k_hand_counts
+  size_t tot_words() const { return (size_t)ccap + 2 + KE_NEED_SHARDS; }
   uint32_t *h_sigflag = nullptr, *h_sigflag_dev = nullptr;   // pinned word: the tag of the call whose counters are in h_ccount
   uint32_t sig_tag = 0;
   uint32_t *d_cid = nullptr, *d_kidx = nullptr;   // per plan: class id, arrival index within the class
@@ -831,7 +839,7 @@ struct rpeg_engine_s {
   bool timing = false;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms = -1.0;
-  uint64_t stats[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  uint64_t stats[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
   double host_us[4] = {0, 0, 0, 0};   // host time of the last laid-out rpeg_eval_batch call: rpeg_engine_host_us
   int n_cu = 256;
   uint8_t* static_ptr = nullptr;    // this device's copy of the file-scope scratch array (rpeg_eval_batch_static)
@@ -920,7 +928,7 @@ static int ensure_class_tables(rpeg_engine_t* e, hipStream_t s) {
     HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_ccount_dev, e->h_ccount, 0));
     if (e->h_tot) hipHostFree(e->h_tot);
     e->h_tot = e->h_tot_dev = nullptr;
-    HIP_TRY(e, hipHostMalloc(&e->h_tot, ((size_t)cap + 1 + KE_NEED_SHARDS) * 4, hipHostMallocCoherent));
+    HIP_TRY(e, hipHostMalloc(&e->h_tot, (2 * (size_t)cap + 2 + KE_NEED_SHARDS) * 4, hipHostMallocCoherent));
     HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_tot_dev, e->h_tot, 0));
     if (!e->h_sigflag) {
       HIP_TRY(e, hipHostMalloc(&e->h_sigflag, 64, hipHostMallocCoherent));
@@ -1288,7 +1296,7 @@ int rpeg_engine_reset_classes(rpeg_engine_t* e) {
 
 int rpeg_engine_stats(const rpeg_engine_t* e, uint64_t* out, int32_t n) {
   if (!e || !out) return -1;
-  for (int i = 0; i < n && i < 8; ++i) out[i] = e->stats[i];
+  for (int i = 0; i < n && i < 9; ++i) out[i] = e->stats[i];
   return 0;
 }
 
@@ -1541,7 +1549,8 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       HIP_TRY(e, hipStreamWaitEvent(e->s3, e->ev_sig, 0));
       if (int rc = launch_prologue(true)) return rc;
     }
-    hipLaunchKernelGGL(k_hand_counts, dim3(1), dim3(HAND_BLOCK), 0, s, e->d_ccount, e->d_need, ncls, shards, e->h_tot_dev, e->h_sigflag_dev, tag);
+    hipLaunchKernelGGL(k_hand_counts, dim3(1), dim3(HAND_BLOCK), 0, s, e->d_ccount, e->d_need, ncls, shards, e->d_limit,
+                       e->d_cstat + e->cstat_cap, e->h_tot_dev, e->h_tot_dev + e->tot_words(), e->h_sigflag_dev, tag);
     HIP_TRY(e, hipGetLastError());
     if (read_stat) {
       HIP_TRY(e, hipMemcpyAsync(e->cls_pops16.data(), e->d_cstat, (size_t)ncls * 4, hipMemcpyDeviceToHost, s));
@@ -1576,6 +1585,11 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     }
     if (read_stat && e->learn_calls > 0) --e->learn_calls;
     for (int q = 0; q < KE_NEED_SHARDS; ++q) e->need = std::max(e->need, e->h_tot[ncls + 1 + q]);
+    if (round == 0) {
+      e->stats[8] = e->h_tot[ncls + 1 + KE_NEED_SHARDS];
+      if (e->stats[8])
+        for (uint32_t c = 0; c < ncls; ++c) e->cls_need[c] = std::max(e->cls_need[c], e->h_tot[e->tot_words() + c]);
+    }
     if (e->h_tot[ncls] == 0) break;
     if (round >= 2) { e->err = "class table did not converge"; return -5; }
     HIP_TRY(e, hipMemcpyAsync(e->h_sig, e->d_sig, n * 8, hipMemcpyDeviceToHost, s));
@@ -1751,9 +1765,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       if (a == 255 && e->split_quad) (counts[c] < QUAD_TINY || e->cls_nodes[cids[c]] > KQ_MAX_NODES ? solo[c] : quad[c]) = 1;
       else if (a == 255) solo[c] = counts[c] < TINY_CLASS ? 1 : 0;
       else if (a == 1) solo[c] = 1;
-      else if (a == 2) {
-        quad[c] = 1;
-      }
+      else if (a == 2) (e->cls_need[cids[c]] > QUAD_KIND[1].entries ? solo[c] : quad[c]) = 1;   // (as plan_quad would, once a ready set has outgrown sixteen entries)
     }
   } else if (!ls && !one && !quad_all && !order.empty() && (by_quad = plan_quad())) {
     // (decided: every class in k_quad or, tiny classes and the largest graphs, in k_plan)

@@ -27,8 +27,11 @@
 // a lane that has room for it; the availability of their vertices.
 //
 // A plan with more entries ready at once than its lanes hold is not evaluated here: it is flagged (EvalLaunch::limit)
-// and redone by the launch that ends the call, a plan per wavefront.  Ranks go level by level with a node per lane of the plan.  A node's id is its place by
-// tie-break class, so that counting the larger ranks of its class walks through consecutive rows.
+// and redone by the launch that ends the call, a plan per wavefront.  Its class then reports one entry more than there was
+// room for (EvalLaunch::cneed), and the next call gives it the form above: without that a class stayed where it was and
+// its plans were redone in every call (20,011 PPO plans, forms learned from other plans: 25 of them, 452 us a step; now
+// 384).  Ranks go level by level with a node per lane of the plan.  A node's id is its place by tie-break class, so that
+// counting the larger ranks of its class walks through consecutive rows.
 //
 // Bound: LDS, which holds the wavefronts in flight to 1-2 per SIMD (13 bytes per node and 8 per slot for a plan), and
 // with them the latency of a round: measured on 65,536 GRPO plans with four lanes of four entries, a round is 394 vector,
@@ -266,7 +269,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
 #pragma unroll
   for (int u = 0; u < SL; ++u) { ek[u] = inf; sk[u] = inf; eo[u] = KQ_EMPTY; em[u] = 0u; }
   uint32_t tie = 0, free_slots = (1u << SL) - 1u;
-  int live = 0, longest = 0;   // entries now and at most
+  int live = 0, longest = 0;   // entries now and at most (one more than there is room for where one was lost)
   bool ovf = false;
   const unsigned group_shift = (unsigned)(lane & ~(QL - 1));
   const uint32_t below = (1u << q) - 1u;   // the lanes of this plan before this one
@@ -470,6 +473,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
       n_room = (uint32_t)__builtin_popcount(in_plan);
       const mask64 full = again & __ballot(n_room == 0u);
       lost |= full;
+      longest = (int)kp_sel(full, (uint32_t)(QL * SL + 1), (uint32_t)longest);   // (an entry without room is not counted in `live`: the class moves up a form)
       j0 = kp_sel(full, n_succ, j0);
       mine = again & room & __ballot(j0 + r < n_succ);
       sp = 0;

@@ -253,10 +253,10 @@ class Engine:
         return float(self.lib.rpeg_engine_last_kernel_ms(self._h))
 
     def stats(self) -> Dict[str, int]:
-        buf = (C.c_uint64 * 8)()
-        self.lib.rpeg_engine_stats(self._h, buf, 8)
+        buf = (C.c_uint64 * 9)()
+        self.lib.rpeg_engine_stats(self._h, buf, 9)
         return dict(classes=buf[0], classes_lowered=buf[1], wave_tasks=buf[2], lds_bytes=buf[3], workspace_bytes=buf[4],
-                    state_lanes=buf[5], single_plan_tasks=buf[6], quad_tasks=buf[7])
+                    state_lanes=buf[5], single_plan_tasks=buf[6], quad_tasks=buf[7], redone_before=buf[8])
 
     def alloc_outputs(self, n: int):
         torch = _torch()
