@@ -111,13 +111,15 @@ __global__ void k_upload_fill(const uint4* __restrict__ host_src, uint4* __restr
 // written into pinned host memory, then a flag the host polls -- there several microseconds before a copy command
 // behind the kernel would have moved its first byte.  host_count: n_classes totals, the count of the plans of classes
 // not lowered yet, the KE_NEED_SHARDS running maxima of the ready-list length, and the plans that the engine's last
-// laid-out call redid without a bound on the ready set (limit[0]); where there were any, host_need: the longest ready
-// set of every class, so that this call already gives those plans' classes a form with room for them.
+// laid-out call redid without a bound on the ready set (limit[0]).  host_need: the longest ready set of every class, where
+// the call wants the statistic or there were such plans (it then already gives their classes a form with room for them);
+// host_pops: the other half of the statistic, where the call wants it.
 constexpr int HAND_BLOCK = 1024;
 __global__ __launch_bounds__(HAND_BLOCK) void k_hand_counts(uint32_t* __restrict__ count, const uint32_t* __restrict__ need, uint32_t n_classes,
                                                             uint32_t shards, const uint32_t* __restrict__ limit,
-                                                            const uint32_t* __restrict__ cneed, uint32_t* __restrict__ host_count,
-                                                            uint32_t* __restrict__ host_need, uint32_t* __restrict__ host_flag, uint32_t tag) {
+                                                            const uint32_t* __restrict__ cpops, const uint32_t* __restrict__ cneed,
+                                                            uint32_t* __restrict__ host_count, uint32_t* __restrict__ host_need,
+                                                            uint32_t* __restrict__ host_pops, uint32_t* __restrict__ host_flag, uint32_t tag) {
   const uint32_t redone = limit[0];
   // the totals first, and on their way to the host before anything else is written
   for (uint32_t c = threadIdx.x; c < n_classes; c += HAND_BLOCK) {
@@ -135,8 +137,10 @@ __global__ __launch_bounds__(HAND_BLOCK) void k_hand_counts(uint32_t* __restrict
   if (threadIdx.x == 0) host_count[n_classes] = count[(size_t)n_classes * shards];
   if (threadIdx.x < KE_NEED_SHARDS) host_count[n_classes + 1 + threadIdx.x] = need[threadIdx.x];
   if (threadIdx.x == 0) host_count[n_classes + 1 + KE_NEED_SHARDS] = redone;
-  if (redone)
+  if (redone || host_pops)
     for (uint32_t c = threadIdx.x; c < n_classes; c += HAND_BLOCK) host_need[c] = cneed[c];
+  if (host_pops)
+    for (uint32_t c = threadIdx.x; c < n_classes; c += HAND_BLOCK) host_pops[c] = cpops[c];
   __threadfence_system();
   __syncthreads();
   if (threadIdx.x == 0) __hip_atomic_store(host_flag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -760,7 +764,7 @@ struct rpeg_engine_s {
   uint64_t count_clean = 0;                     // leading words of d_ccount that the last call left at zero,
   hipStream_t count_clean_on = nullptr;         // on this stream
   uint32_t* h_ccount_dev = nullptr;             // the same pinned buffer as the device addresses it
-  uint32_t *h_tot = nullptr, *h_tot_dev = nullptr;   // pinned: per-class totals of a call (tot_words), then per-class ready-set lengths, written by k_hand_counts
+  uint32_t *h_tot = nullptr, *h_tot_dev = nullptr;   // pinned: per-class totals of a call (tot_words), then the halves of the class statistic (ccap words each), written by k_hand_counts
   size_t tot_words() const { return (size_t)ccap + 2 + KE_NEED_SHARDS; }
   uint32_t *h_sigflag = nullptr, *h_sigflag_dev = nullptr;   // pinned word: the tag of the call whose counters are in h_ccount
   uint32_t sig_tag = 0;
@@ -804,7 +808,6 @@ struct rpeg_engine_s {
   uint32_t max_v = RPEG_MAX_V;   // largest vertex count of the problem's structures
   hipStream_t s2 = nullptr;                     // second stream: single-plan wavefronts of a large batch run beside the others
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  hipEvent_t ev_counts = nullptr;               // the statistic of a call has reached the host (the calls that read it)
   hipStream_t s4 = nullptr;                     // fourth stream and its join: k_quad's second launches
   hipEvent_t ev_join4 = nullptr;
   hipStream_t s3 = nullptr;                     // third stream: the few-lanes-per-plan wavefronts (k_quad)
@@ -928,7 +931,7 @@ static int ensure_class_tables(rpeg_engine_t* e, hipStream_t s) {
     HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_ccount_dev, e->h_ccount, 0));
     if (e->h_tot) hipHostFree(e->h_tot);
     e->h_tot = e->h_tot_dev = nullptr;
-    HIP_TRY(e, hipHostMalloc(&e->h_tot, (2 * (size_t)cap + 2 + KE_NEED_SHARDS) * 4, hipHostMallocCoherent));
+    HIP_TRY(e, hipHostMalloc(&e->h_tot, (3 * (size_t)cap + 2 + KE_NEED_SHARDS) * 4, hipHostMallocCoherent));
     HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_tot_dev, e->h_tot, 0));
     if (!e->h_sigflag) {
       HIP_TRY(e, hipHostMalloc(&e->h_sigflag, 64, hipHostMallocCoherent));
@@ -1184,7 +1187,6 @@ void rpeg_engine_destroy(rpeg_engine_t* e) {
   if (e->s2) { hipStreamSynchronize(e->s2); hipEventDestroy(e->ev_fork); hipEventDestroy(e->ev_join); }
   if (e->s3) { hipStreamSynchronize(e->s3); hipEventDestroy(e->ev_join3); hipStreamSynchronize(e->s4); hipEventDestroy(e->ev_join4); }
   if (e->ev_sig) hipEventDestroy(e->ev_sig);
-  if (e->ev_counts) hipEventDestroy(e->ev_counts);
   e->lane0.release();
   if (e->d_stage) hipFree(e->d_stage);
   if (e->h_stage) hipHostFree(e->h_stage);
@@ -1469,6 +1471,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // memory model to that kernel, which spreads them over the lanes of a plan's wavefront: the prologue launches work a
   // plan per lane, and a few thousand plans are a few dozen wavefronts that take as long as a full grid would.
   const bool own_prologue = e->state_lanes == 1 || (e->state_lanes == -1 && n <= (uint64_t)e->n_cu * e->one_plan_waves_per_cu);
+  auto plan_fits = [&]() { return e->max_nodes <= (uint32_t)(WAVE * KP_MAX_NS) && kp_lds_bytes(e->max_nodes, e->max_slots) <= 64 * 1024; };
   bool prologue_done = false, peaks_deferred = false;
   // ahead: k_quad's stream becomes the main line of the call -- the cost-model launch goes there as soon as the class
   // ids are written (beside the hand-over of the counters to the host), the layout and the scatter follow it there
@@ -1520,12 +1523,13 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     shards = MAX_SHARDS;
     while (shards > 1 && ((uint64_t)ncls * shards > COUNT_SLOTS || (uint64_t)shards * 8 * SIG_BLOCK >= n)) shards >>= 1;
     const uint64_t n_count = (uint64_t)ncls * shards + 1;
-    // what earlier launches of the main kernel learned about the classes (pops per dispatch): read in the calls
-    // that follow new classes, and now and then afterwards
-    const bool read_stat = round == 0 && e->quad_share_pct && ncls && (e->learn_calls > 0 || (e->batch_calls & 63) == 0);
-    // The counters go to the host through k_hand_counts; in the first round the host polls its flag instead of waiting
-    // for the stream, unless a copy of the statistic has to be waited for anyway.
-    const bool handed = round == 0 && !read_stat;
+    // what earlier launches of the main kernel and of k_quad learned about the classes: read in the calls that follow new
+    // classes, and now and then afterwards -- by a batch that may run there; one for k_plan alone neither uses it nor adds
+    // to it
+    const bool read_stat = round == 0 && e->quad_share_pct && ncls && !(own_prologue && plan_fits()) &&
+                           (e->learn_calls > 0 || (e->batch_calls & 63) == 0);
+    // The counters go to the host through k_hand_counts (the statistic with them); in the first round the host polls its
+    // flag instead of waiting for the stream.
     const uint32_t tag = ++e->sig_tag ? e->sig_tag : ++e->sig_tag;
     if (round == 0 && !own_prologue) {
       if (int rc = ensure_side(e)) return rc;
@@ -1550,35 +1554,23 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       if (int rc = launch_prologue(true)) return rc;
     }
     hipLaunchKernelGGL(k_hand_counts, dim3(1), dim3(HAND_BLOCK), 0, s, e->d_ccount, e->d_need, ncls, shards, e->d_limit,
-                       e->d_cstat + e->cstat_cap, e->h_tot_dev, e->h_tot_dev + e->tot_words(), e->h_sigflag_dev, tag);
+                       e->d_cstat, e->d_cstat + e->cstat_cap, e->h_tot_dev, e->h_tot_dev + e->tot_words(),
+                       read_stat ? e->h_tot_dev + e->tot_words() + e->ccap : nullptr, e->h_sigflag_dev, tag);
     HIP_TRY(e, hipGetLastError());
-    if (read_stat) {
-      HIP_TRY(e, hipMemcpyAsync(e->cls_pops16.data(), e->d_cstat, (size_t)ncls * 4, hipMemcpyDeviceToHost, s));
-      HIP_TRY(e, hipMemcpyAsync(e->cls_need.data(), e->d_cstat + e->cstat_cap, (size_t)ncls * 4, hipMemcpyDeviceToHost, s));
-    }
     if (round == 0) {
-      if (!handed) {   // (the copy of the statistic has to be waited for: an event, so that the wait leaves the launch below alone)
-        if (!e->ev_counts) HIP_TRY(e, hipEventCreateWithFlags(&e->ev_counts, hipEventDisableTiming));
-        HIP_TRY(e, hipEventRecord(e->ev_counts, s));
-      }
       if (!own_prologue && !ahead)
         if (int rc = launch_prologue(true)) return rc;
       t_counts = std::chrono::steady_clock::now();
       bool seen = false;
-      if (handed) {
-        for (uint64_t spins = 0;; ++spins) {
-          if (__atomic_load_n(e->h_sigflag, __ATOMIC_ACQUIRE) == tag) { seen = true; break; }
-          // a launch that does not come to an end is the stream's to report
-          if ((spins & 0xFFFFu) == 0xFFFFu && std::chrono::steady_clock::now() - t_counts > std::chrono::seconds(2)) break;
+      for (uint64_t spins = 0;; ++spins) {
+        if (__atomic_load_n(e->h_sigflag, __ATOMIC_ACQUIRE) == tag) { seen = true; break; }
+        // a launch that does not come to an end is the stream's to report
+        if ((spins & 0xFFFFu) == 0xFFFFu && std::chrono::steady_clock::now() - t_counts > std::chrono::seconds(2)) break;
 #if defined(__x86_64__) || defined(__i386__)
-          __builtin_ia32_pause();
+        __builtin_ia32_pause();
 #endif
-        }
       }
-      if (!seen) {
-        if (handed) HIP_TRY(e, hipStreamSynchronize(s));
-        else HIP_TRY(e, hipEventSynchronize(e->ev_counts));
-      }
+      if (!seen) HIP_TRY(e, hipStreamSynchronize(s));
       t_waited = std::chrono::steady_clock::now();
     } else {
       HIP_TRY(e, hipStreamSynchronize(s));
@@ -1587,8 +1579,8 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     for (int q = 0; q < KE_NEED_SHARDS; ++q) e->need = std::max(e->need, e->h_tot[ncls + 1 + q]);
     if (round == 0) {
       e->stats[8] = e->h_tot[ncls + 1 + KE_NEED_SHARDS];
-      if (e->stats[8])
-        for (uint32_t c = 0; c < ncls; ++c) e->cls_need[c] = std::max(e->cls_need[c], e->h_tot[e->tot_words() + c]);
+      if (e->stats[8] || read_stat) std::copy_n(e->h_tot + e->tot_words(), ncls, e->cls_need.begin());
+      if (read_stat) std::copy_n(e->h_tot + e->tot_words() + e->ccap, ncls, e->cls_pops16.begin());
     }
     if (e->h_tot[ncls] == 0) break;
     if (round >= 2) { e->err = "class table did not converge"; return -5; }
@@ -1615,8 +1607,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // wavefronts of fewer plans whose state fits in LDS, which shortens every scheduler step.
   int ls = e->state_lanes;
   bool one = false;   // one plan per wavefront (k_plan)
-  const bool plan_fits = e->max_nodes <= (uint32_t)(WAVE * KP_MAX_NS) && kp_lds_bytes(e->max_nodes, e->max_slots) <= 64 * 1024;
-  const bool quad_free = ls == -1 && e->quad_share_pct && e->split_heavy && plan_fits;   // k_quad may take the batch (plan_quad)
+  const bool quad_free = ls == -1 && e->quad_share_pct && e->split_heavy && plan_fits();   // k_quad may take the batch (plan_quad)
   const bool quad_all = ls == 4;   // every class in the kernel of two or four lanes per plan (k_quad)
   if (quad_all) {
     ls = 0;
@@ -1914,7 +1905,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       }
     }
   }
-  if (!keep_split && !ls && !one && !quad_all && !order.empty() && e->split_heavy && plan_fits && e->quad_share_pct) {   // kept for the next calls
+  if (!keep_split && !ls && !one && !quad_all && !order.empty() && e->split_heavy && plan_fits() && e->quad_share_pct) {   // kept for the next calls
     e->cls_split.assign(ncls, (uint8_t)255);
     for (size_t c = 0; c < counts.size(); ++c) e->cls_split[cids[c]] = solo[c] ? 1 : quad[c] ? 2 : 0;
     e->split_for_n = n; e->split_at = e->batch_calls; e->split_mass = mass != nullptr;
