@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -42,13 +43,16 @@ struct HostMem {
 struct Port {
   rpeg_problem_t P;
   std::unordered_map<uint64_t, LoweredClass> classes;
+  std::unique_ptr<LowerTables> tables;
+  std::unique_ptr<Lowering> low;
   std::mutex mu;
   std::string err;
   const LoweredClass* get(uint64_t sig) {
     std::lock_guard<std::mutex> g(mu);
     auto it = classes.find(sig);
     if (it != classes.end()) return &it->second;
-    return &(classes[sig] = lower_class(P, sig));
+    low->run(sig);
+    return &(classes[sig] = low->out);
   }
 };
 }  // namespace
@@ -58,6 +62,8 @@ extern "C" {
 void* port_create(const rpeg_problem_t* p) {
   Port* e = new Port();
   e->P = *p;
+  e->tables = std::make_unique<LowerTables>(e->P);
+  e->low = std::make_unique<Lowering>(e->P, *e->tables);
   return e;
 }
 void port_destroy(void* h) { delete (Port*)h; }
@@ -147,6 +153,22 @@ int port_lower(void* h, const int16_t* vert, const uint8_t* head, int32_t* kind,
   for (size_t j = 0; j < lc->edges.size(); ++j) { edges[2 * j] = lc->edges[j].first; edges[2 * j + 1] = lc->edges[j].second; }
   *n_edges = (int)lc->edges.size();
   return n;
+}
+
+// the blob of a class and its edges: from the object that lowers one class after the other, or from one of its own
+long port_blob(void* h, uint64_t sig, int own, uint8_t* out, long cap, int32_t* edges, int32_t* n_edges) {
+  Port* e = (Port*)h;
+  LoweredClass mine;
+  const LoweredClass* lc = &mine;
+  try {
+    if (own) mine = lower_class(e->P, sig);
+    else { e->low->run(sig); lc = &e->low->out; }
+  } catch (const std::exception& ex) { e->err = ex.what(); return -2; }
+  if ((long)lc->blob.size() > cap || (long)lc->edges.size() * 8 > cap) return -3;
+  std::memcpy(out, lc->blob.data(), lc->blob.size());
+  for (size_t j = 0; j < lc->edges.size(); ++j) { edges[2 * j] = lc->edges[j].first; edges[2 * j + 1] = lc->edges[j].second; }
+  *n_edges = (int32_t)lc->edges.size();
+  return (long)lc->blob.size();
 }
 
 // isolated operator time / peak of mock nodes (candidate directory)

@@ -21,6 +21,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -739,6 +740,8 @@ struct rpeg_engine_s {
   int device = 0;
   std::string err;
   // lowering classes
+  std::unique_ptr<LowerTables> low_tables;
+  std::unique_ptr<Lowering> low;                     // of this engine's calls; `out` is the class lowered last
   std::unordered_map<uint64_t, uint32_t> class_off;  // signature -> byte offset in the pool
   std::vector<uint64_t> cls_sig;                     // class id -> signature / pool offset / node count
   std::vector<uint32_t> cls_off, cls_nodes, cls_slots;
@@ -998,15 +1001,15 @@ static int ensure_pool(rpeg_engine_t* e, hipStream_t s) {
   return 0;
 }
 
-// appends a lowered class to the engine's tables; returns its pool offset or -1
-static int64_t class_append(rpeg_engine_t* e, uint64_t sig, const LoweredClass& lc) {
-  const ClassHdr* h = (const ClassHdr*)lc.blob.data();
+// appends a lowered class (its blob) to the engine's tables; returns its pool offset or -1
+static int64_t class_append(rpeg_engine_t* e, uint64_t sig, const uint8_t* blob) {
+  const ClassHdr* h = (const ClassHdr*)blob;
   e->max_nodes = std::max(e->max_nodes, h->n_nodes);
   e->max_slots = std::max(e->max_slots, h->n_slots);
   e->max_cls_bytes = std::max(e->max_cls_bytes, h->n_nodes * 8u + h->n_succ * 2u);
-  if (e->pool.size() + lc.blob.size() >= (1ull << 31)) { e->err = "class pool exceeds 2 GiB"; return -1; }   // bit 31 of an offset is a flag
+  if (e->pool.size() + h->bytes >= (1ull << 31)) { e->err = "class pool exceeds 2 GiB"; return -1; }   // bit 31 of an offset is a flag
   uint32_t off = (uint32_t)e->pool.size();
-  e->pool.insert(e->pool.end(), lc.blob.begin(), lc.blob.end());
+  e->pool.insert(e->pool.end(), blob, blob + h->bytes);
   ((ClassHdr*)(e->pool.data() + off))->id = (uint32_t)e->cls_sig.size();
   e->class_off.emplace(sig, off);
   e->cls_sig.push_back(sig);
@@ -1019,19 +1022,18 @@ static int64_t class_append(rpeg_engine_t* e, uint64_t sig, const LoweredClass& 
   return off;
 }
 
-// returns the pool offset of the class of `sig`, lowering it on first sight; -1 on failure
+// returns the pool offset of the class of `sig`, lowering it on first sight (*is_new; e->low->out then holds it); -1 on failure
 static int64_t class_offset(rpeg_engine_t* e, uint64_t sig, bool* is_new) {
   auto it = e->class_off.find(sig);
   if (it != e->class_off.end()) return it->second;
-  LoweredClass lc;
   try {
-    lc = lower_class(e->P, sig);
+    e->low->run(sig);
   } catch (const std::exception& ex) {
     e->err = std::string("lowering failed: ") + ex.what();
     return -1;
   }
   if (is_new) *is_new = true;
-  return class_append(e, sig, lc);
+  return class_append(e, sig, e->low->out.blob.data());
 }
 
 // lowers the classes of `sigs` that the engine does not hold yet, on up to eight host threads (lowering a
@@ -1044,13 +1046,20 @@ static int lower_new_classes(rpeg_engine_t* e, const std::vector<uint64_t>& sigs
       if (!e->class_off.count(sg) && seen.emplace(sg, 1).second) todo.push_back(sg);
   }
   if (todo.empty()) return 0;
-  std::vector<LoweredClass> lowered(todo.size());
+  struct Blob { size_t thread, off; };   // where a class was left: in its thread's bytes
+  std::vector<Blob> lowered(todo.size());
   std::vector<std::string> errors(todo.size());
   const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
   const size_t n_threads = std::min<size_t>({(size_t)8, (size_t)hw, (todo.size() + 15) / 16});
+  std::vector<std::vector<uint8_t>> bytes(std::max<size_t>(n_threads, 1));
   auto work = [&](size_t t) {
+    Lowering low(e->P, *e->low_tables);
     for (size_t i = t; i < todo.size(); i += n_threads) {
-      try { lowered[i] = lower_class(e->P, todo[i]); } catch (const std::exception& ex) { errors[i] = ex.what(); if (errors[i].empty()) errors[i] = "error"; }
+      try {
+        low.run(todo[i]);
+        lowered[i] = {t, bytes[t].size()};
+        bytes[t].insert(bytes[t].end(), low.out.blob.begin(), low.out.blob.end());
+      } catch (const std::exception& ex) { errors[i] = ex.what(); if (errors[i].empty()) errors[i] = "error"; }
     }
   };
   if (n_threads <= 1) {
@@ -1062,7 +1071,7 @@ static int lower_new_classes(rpeg_engine_t* e, const std::vector<uint64_t>& sigs
   }
   for (size_t i = 0; i < todo.size(); ++i) {
     if (!errors[i].empty()) { e->err = "lowering failed: " + errors[i]; return -5; }
-    if (class_append(e, todo[i], lowered[i]) < 0) return -5;
+    if (class_append(e, todo[i], bytes[lowered[i].thread].data() + lowered[i].off) < 0) return -5;
   }
   *n_new += todo.size();
   return 0;
@@ -1119,6 +1128,8 @@ int rpeg_engine_create(const rpeg_problem_t* problem, rpeg_engine_t** out) {
   if (hipGetDeviceCount(&count) != hipSuccess || count < 1) return -4;  // no GPU: there is no CPU path
   rpeg_engine_t* e = new rpeg_engine_s();
   e->P = *problem;
+  e->low_tables = std::make_unique<LowerTables>(e->P);
+  e->low = std::make_unique<Lowering>(e->P, *e->low_tables);
   hipGetDevice(&e->device);
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, e->device) == hipSuccess) e->n_cu = prop.multiProcessorCount;
@@ -2333,7 +2344,7 @@ static void describe_nodes(const rpeg_problem_t& problem, const rpeg_struct_t& s
 static int host_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t* head4, uint32_t flags, double* result,
                       uint8_t* mask, double* start, double* finish, int32_t* dispatched, int32_t* node_kind, int32_t* node_vertex,
                       int32_t* node_step, int32_t* node_sub, int32_t* node_src, int64_t* node_payload, int32_t* node_ref,
-                      uint8_t* node_reserved, int32_t cap, hipStream_t s, LoweredClass& lc);
+                      uint8_t* node_reserved, int32_t cap, hipStream_t s);
 
 extern "C" {
 
@@ -2428,13 +2439,13 @@ int rpeg_eval_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t*
   for (int v = 0; v < e->P.st[h.structure].n_vertex; ++v) load_vertex(vert_fields, 1, 0, v, &a[v]);
   if (!plan_valid(e->P, h, a)) { e->err = "plan violates the integer validity rules"; return -6; }
   const uint64_t sg = plan_signature(e->P, h.structure, h.split, h.tau0, h.tau1, a);
-  LoweredClass lc;
+  const LoweredClass& lc = e->low->out;
   {   // a graph that k_plan takes: one launch, whose times land in pinned memory
     double result[3];
     uint8_t mask = 0;
     std::vector<int32_t> dispatched((size_t)std::max(cap, 1));
     const int m = host_trace(e, vert_fields, head4, 0u, result, &mask, start, finish, dispatched.data(), node_kind, node_vertex,
-                             node_step, node_sub, node_src, nullptr, nullptr, node_reserved, cap, nullptr, lc);
+                             node_step, node_sub, node_src, nullptr, nullptr, node_reserved, cap, nullptr);
     if (m < 0 && m != -8) return m;
     if (m >= 0 && (mask & RPEG_MASK_VALID) && !(mask & RPEG_MASK_ERROR)) {
       if (edges && (int)lc.edges.size() > cap) { e->err = "trace arrays too small"; return -7; }
@@ -2446,11 +2457,12 @@ int rpeg_eval_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t*
       return m;
     }
   }
-  try { lc = lower_class(e->P, sg); } catch (const std::exception& ex) { e->err = ex.what(); return -5; }
+  bool lowered = false;
+  const int64_t off = class_offset(e, sg, &lowered);
+  if (off < 0) return -5;
+  if (!lowered) try { e->low->run(sg); } catch (const std::exception& ex) { e->err = ex.what(); return -5; }
   const int n = (int)lc.nodes.size();
   if (n > cap || (edges && (int)lc.edges.size() > cap)) { e->err = "trace arrays too small"; return -7; }
-  int64_t off = class_offset(e, sg, nullptr);
-  if (off < 0) return -5;
   hipStream_t s = nullptr;
   // This call works on the null stream and reuses the engine's task, lane and state buffers.  A batched call
   // returns without waiting for its stream, and a stream created as non-blocking does not order itself against
@@ -2534,12 +2546,13 @@ int rpeg_plan_detail(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t
   for (int v = 0; v < st.n_vertex; ++v) load_vertex(vert_fields, 1, 0, v, &a[v]);
   if (!plan_valid(e->P, h, a)) { e->err = "plan violates the integer validity rules"; return -6; }
   const uint64_t sg = plan_signature(e->P, h.structure, h.split, h.tau0, h.tau1, a);
-  LoweredClass lc;
-  try { lc = lower_class(e->P, sg); } catch (const std::exception& ex) { e->err = ex.what(); return -5; }
+  bool lowered = false;
+  const int64_t off = class_offset(e, sg, &lowered);
+  if (off < 0) return -5;
+  if (!lowered) try { e->low->run(sg); } catch (const std::exception& ex) { e->err = ex.what(); return -5; }
+  const LoweredClass& lc = e->low->out;
   const int n = (int)lc.nodes.size();
   if ((node_time || node_payload || node_ref) && n > cap) { e->err = "node arrays too small"; return -7; }
-  const int64_t off = class_offset(e, sg, nullptr);
-  if (off < 0) return -5;
   hipStream_t s = nullptr;
   HIP_TRY(e, hipDeviceSynchronize());   // (null stream, shared buffers: as rpeg_eval_trace)
   if (int rc = ensure_pool(e, s)) return rc;
@@ -2844,11 +2857,11 @@ int eval_host_small(rpeg_engine_t* e, uint64_t n, GET get, uint32_t flags, doubl
 
 }  // namespace
 
-// One plan with the times of its nodes from one launch (rpeg_eval_host_trace); lc: its lowered class.
+// One plan with the times of its nodes from one launch (rpeg_eval_host_trace); e->low->out: its lowered class.
 static int host_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t* head4, uint32_t flags, double* result,
                       uint8_t* mask, double* start, double* finish, int32_t* dispatched, int32_t* node_kind, int32_t* node_vertex,
                       int32_t* node_step, int32_t* node_sub, int32_t* node_src, int64_t* node_payload, int32_t* node_ref,
-                      uint8_t* node_reserved, int32_t cap, hipStream_t s, LoweredClass& lc) {
+                      uint8_t* node_reserved, int32_t cap, hipStream_t s) {
   e->err.clear();
   if (e->state_lanes != -1 && e->state_lanes != 1) return -8;   // (a layout was asked for: the caller goes the long way)
   PlanHead h = load_head(head4, 1, 0);
@@ -2860,8 +2873,10 @@ static int host_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_
   for (int v = 0; v < st.n_vertex; ++v) load_vertex(vert_fields, 1, 0, v, &a[v]);
   if (!plan_valid(e->P, h, a)) return 0;
   const uint64_t sg = plan_signature(e->P, h.structure, h.split, h.tau0, h.tau1, a);
-  const int64_t off = class_offset(e, sg, nullptr);
+  bool lowered = false;   // (now, as a class not met before: e->low holds it already)
+  const int64_t off = class_offset(e, sg, &lowered);
   if (off < 0) return -5;
+  const uint64_t n_new = lowered ? 1 : 0;
   const size_t rows = e->max_nodes;
   if (rows > (size_t)(WAVE * KP_MAX_NS)) return -8;
   if (rows > e->h_times_nodes) {   // (no launch that writes the old block is under way: the call that made one has waited for it)
@@ -2875,10 +2890,11 @@ static int host_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_
   auto get = [&](uint64_t, PlanHead& ph, VPlan (&pa)[RPEG_MAX_V]) { ph = h; std::memcpy(pa, a, sizeof pa); };
   e->last_ms = -1.0;
   const int rc = host_small_submit(e, e->lane0, 1, get, flags, false, false, s, (double*)e->h_times_dev);
+  e->stats[1] = n_new;
   if (rc) return rc == 1 ? -8 : rc;
   // while the launch runs: what the records of the nodes hold
-  bool lowered = true;
-  try { lc = lower_class(e->P, sg); } catch (const std::exception& ex) { lowered = false; e->err = ex.what(); }
+  const LoweredClass& lc = e->low->out;
+  if (!lowered) try { e->low->run(sg); lowered = true; } catch (const std::exception& ex) { e->err = ex.what(); }
   const int n = (int)lc.nodes.size();
   if (lowered && n <= cap) {
     describe_nodes(e->P, st, h, a, lc, node_kind, node_vertex, node_step, node_sub, node_src, node_payload, node_ref);
@@ -3213,9 +3229,8 @@ int rpeg_eval_host_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uin
                          int32_t* node_step, int32_t* node_sub, int32_t* node_src, int64_t* node_payload, int32_t* node_ref,
                          uint8_t* node_reserved, int32_t cap, void* stream) {
   if (!e || !vert_fields || !head4 || !result || !mask || !start || !finish || !dispatched) return -1;
-  LoweredClass lc;
   return host_trace(e, vert_fields, head4, flags, result, mask, start, finish, dispatched, node_kind, node_vertex, node_step, node_sub,
-                    node_src, node_payload, node_ref, node_reserved, cap, (hipStream_t)stream, lc);
+                    node_src, node_payload, node_ref, node_reserved, cap, (hipStream_t)stream);
 }
 
 int rpeg_sa_run(rpeg_engine_t* e, const rpeg_sa_params_t* prm, const int16_t* base_plan, rpeg_sa_result_t* res,
