@@ -772,7 +772,12 @@ struct rpeg_engine_s {
   uint32_t *h_sigflag = nullptr, *h_sigflag_dev = nullptr;   // pinned word: the tag of the call whose counters are in h_ccount
   uint32_t sig_tag = 0;
   uint32_t *d_cid = nullptr, *d_kidx = nullptr;   // per plan: class id, arrival index within the class
-  std::vector<uint8_t> pool;
+  // the class blobs live on the device; on the host only those that are still to go there, in stretches of the pool
+  // whose buffers are used again (a copy of the whole pool on the host grew by reallocation: 4 ms of a call that took it
+  // from 8 to 16 MB, and a page fault for every 4 KB)
+  struct Fresh { size_t off = 0; std::vector<uint8_t> bytes; };
+  std::vector<Fresh> fresh;
+  size_t n_fresh = 0, pool_size = 0;
   uint8_t* d_pool = nullptr;
   size_t d_pool_cap = 0, d_pool_used = 0;
   uint32_t max_nodes = 1, max_slots = 1, max_cls_bytes = 16;
@@ -980,46 +985,63 @@ static int ensure_perm(rpeg_engine_t* e, size_t lanes, size_t tasks) {
 }
 
 static int ensure_pool(rpeg_engine_t* e, hipStream_t s) {
-  if (e->pool.size() > e->d_pool_cap) {
-    size_t cap = std::max<size_t>(e->pool.size() * 2, 1 << 20);
+  if (e->pool_size > e->d_pool_cap) {
+    size_t cap = std::max<size_t>(e->pool_size * 2, 1 << 20);
     uint8_t* np = nullptr;
     HIP_TRY(e, hipMalloc(&np, cap));
+    if (e->d_pool_used) {
+      const hipError_t st = hipMemcpyAsync(np, e->d_pool, e->d_pool_used, hipMemcpyDeviceToDevice, s);
+      if (st != hipSuccess) hipFree(np);
+      HIP_TRY(e, st);
+    }
     HIP_TRY(e, hipStreamSynchronize(s));
     if (e->lanes_busy > 0) HIP_TRY(e, hipDeviceSynchronize());   // kernels of other lanes still read the old pool
     if (e->d_pool) hipFree(e->d_pool);
     e->d_pool = np;
     e->d_pool_cap = cap;
-    e->d_pool_used = 0;
   }
-  if (e->pool.size() > e->d_pool_used) {
-    HIP_TRY(e, hipMemcpyAsync(e->d_pool + e->d_pool_used, e->pool.data() + e->d_pool_used,
-                              e->pool.size() - e->d_pool_used, hipMemcpyHostToDevice, s));
-    // the host vector may reallocate on the next insertion: finish the copy first
+  if (e->n_fresh) {
+    for (size_t k = 0; k < e->n_fresh; ++k)
+      HIP_TRY(e, hipMemcpyAsync(e->d_pool + e->fresh[k].off, e->fresh[k].bytes.data(), e->fresh[k].bytes.size(), hipMemcpyHostToDevice, s));
+    // the host buffers are filled again by the next classes: finish the copies first
     HIP_TRY(e, hipStreamSynchronize(s));
-    e->d_pool_used = e->pool.size();
+    e->n_fresh = 0;
   }
+  e->d_pool_used = e->pool_size;
   return 0;
 }
 
-// appends a lowered class (its blob) to the engine's tables; returns its pool offset or -1
-static int64_t class_append(rpeg_engine_t* e, uint64_t sig, const uint8_t* blob) {
-  const ClassHdr* h = (const ClassHdr*)blob;
+// an empty stretch at the end of the pool (valid until the next one is asked for)
+static rpeg_engine_s::Fresh& pool_stretch(rpeg_engine_t* e) {
+  if (e->n_fresh == e->fresh.size()) e->fresh.emplace_back();
+  rpeg_engine_s::Fresh& f = e->fresh[e->n_fresh++];
+  f.off = e->pool_size;
+  f.bytes.clear();
+  return f;
+}
+
+// whether the pool has room for as many bytes more (bit 31 of an offset is a flag)
+static bool pool_room(rpeg_engine_t* e, size_t bytes) {
+  if (e->pool_size + bytes < (1ull << 31)) return true;
+  e->err = "class pool exceeds 2 GiB";
+  return false;
+}
+
+// enters a lowered class, whose blob lies at pool offset `off` (and still in host memory at `blob`), in the engine's tables
+static void class_append(rpeg_engine_t* e, uint64_t sig, uint8_t* blob, size_t off) {
+  ClassHdr* h = (ClassHdr*)blob;
   e->max_nodes = std::max(e->max_nodes, h->n_nodes);
   e->max_slots = std::max(e->max_slots, h->n_slots);
   e->max_cls_bytes = std::max(e->max_cls_bytes, h->n_nodes * 8u + h->n_succ * 2u);
-  if (e->pool.size() + h->bytes >= (1ull << 31)) { e->err = "class pool exceeds 2 GiB"; return -1; }   // bit 31 of an offset is a flag
-  uint32_t off = (uint32_t)e->pool.size();
-  e->pool.insert(e->pool.end(), blob, blob + h->bytes);
-  ((ClassHdr*)(e->pool.data() + off))->id = (uint32_t)e->cls_sig.size();
-  e->class_off.emplace(sig, off);
+  h->id = (uint32_t)e->cls_sig.size();
+  e->class_off.emplace(sig, (uint32_t)off);
   e->cls_sig.push_back(sig);
-  e->cls_off.push_back(off);
+  e->cls_off.push_back((uint32_t)off);
   e->cls_nodes.push_back(h->n_nodes);
   e->cls_slots.push_back(h->n_slots);
   e->cls_pops16.push_back(0);
   e->cls_need.push_back(0);
   e->learn_calls = 3;
-  return off;
 }
 
 // returns the pool offset of the class of `sig`, lowering it on first sight (*is_new; e->low->out then holds it); -1 on failure
@@ -1033,7 +1055,15 @@ static int64_t class_offset(rpeg_engine_t* e, uint64_t sig, bool* is_new) {
     return -1;
   }
   if (is_new) *is_new = true;
-  return class_append(e, sig, e->low->out.blob.data());
+  const std::vector<uint8_t>& blob = e->low->out.blob;
+  const size_t off = e->pool_size;
+  if (!pool_room(e, blob.size())) return -1;
+  // (behind the class before it where that one waits for its upload too)
+  rpeg_engine_s::Fresh& f = e->n_fresh ? e->fresh[e->n_fresh - 1] : pool_stretch(e);
+  f.bytes.insert(f.bytes.end(), blob.begin(), blob.end());
+  e->pool_size += blob.size();
+  class_append(e, sig, f.bytes.data() + (off - f.off), off);
+  return (int64_t)off;
 }
 
 // lowers the classes of `sigs` that the engine does not hold yet, on up to eight host threads (lowering a
@@ -1046,19 +1076,21 @@ static int lower_new_classes(rpeg_engine_t* e, const std::vector<uint64_t>& sigs
       if (!e->class_off.count(sg) && seen.emplace(sg, 1).second) todo.push_back(sg);
   }
   if (todo.empty()) return 0;
-  struct Blob { size_t thread, off; };   // where a class was left: in its thread's bytes
+  struct Blob { size_t thread, off; };   // where a class was left: in its thread's stretch of the pool
   std::vector<Blob> lowered(todo.size());
   std::vector<std::string> errors(todo.size());
   const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
   const size_t n_threads = std::min<size_t>({(size_t)8, (size_t)hw, (todo.size() + 15) / 16});
-  std::vector<std::vector<uint8_t>> bytes(std::max<size_t>(n_threads, 1));
+  const size_t first = e->n_fresh;
+  for (size_t t = 0; t < n_threads; ++t) pool_stretch(e);
   auto work = [&](size_t t) {
     Lowering low(e->P, *e->low_tables);
+    std::vector<uint8_t>& bytes = e->fresh[first + t].bytes;
     for (size_t i = t; i < todo.size(); i += n_threads) {
       try {
         low.run(todo[i]);
-        lowered[i] = {t, bytes[t].size()};
-        bytes[t].insert(bytes[t].end(), low.out.blob.begin(), low.out.blob.end());
+        lowered[i] = {t, bytes.size()};
+        bytes.insert(bytes.end(), low.out.blob.begin(), low.out.blob.end());
       } catch (const std::exception& ex) { errors[i] = ex.what(); if (errors[i].empty()) errors[i] = "error"; }
     }
   };
@@ -1069,10 +1101,24 @@ static int lower_new_classes(rpeg_engine_t* e, const std::vector<uint64_t>& sigs
     for (size_t t = 0; t < n_threads; ++t) pool.emplace_back(work, t);
     for (auto& th : pool) th.join();
   }
-  for (size_t i = 0; i < todo.size(); ++i) {
-    if (!errors[i].empty()) { e->err = "lowering failed: " + errors[i]; return -5; }
-    if (class_append(e, todo[i], bytes[lowered[i].thread].data() + lowered[i].off) < 0) return -5;
+  size_t total = 0;
+  for (size_t t = 0; t < n_threads; ++t) total += e->fresh[first + t].bytes.size();
+  if (!pool_room(e, total)) { e->n_fresh = first; return -5; }
+  for (size_t t = 0; t < n_threads; ++t) {   // the stretches one behind the other
+    e->fresh[first + t].off = e->pool_size;
+    e->pool_size += e->fresh[first + t].bytes.size();
   }
+  int rc = 0;
+  for (size_t i = 0; i < todo.size(); ++i) {
+    if (!errors[i].empty()) {
+      if (!rc) e->err = "lowering failed: " + errors[i];
+      rc = -5;
+      continue;
+    }
+    rpeg_engine_s::Fresh& f = e->fresh[first + lowered[i].thread];
+    class_append(e, todo[i], f.bytes.data() + lowered[i].off, f.off + lowered[i].off);
+  }
+  if (rc) return rc;
   *n_new += todo.size();
   return 0;
 }
@@ -1302,7 +1348,8 @@ int rpeg_engine_reset_classes(rpeg_engine_t* e) {
   if (e->d_cstat) { hipFree(e->d_cstat); e->d_cstat = nullptr; e->cstat_cap = 0; }
   e->cls_sorted.clear();
   e->tables_for = 0xFFFFFFFFu;
-  e->pool.clear();
+  e->n_fresh = 0;
+  e->pool_size = 0;
   e->d_pool_used = 0;
   return 0;
 }
@@ -1442,7 +1489,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // 0.18 ms).
   if ((e->state_lanes == 1 || (e->state_lanes == -1 && n <= (uint64_t)e->n_cu * e->one_plan_waves_per_cu)) && !e->prof_on &&
       !e->cls_sig.empty() && (e->cls_sig.size() <= DIRECT_MAX_CLASSES || n <= (uint64_t)e->n_cu * DIRECT_WAVES_PER_CU) && e->d_hkey && e->tables_for == (uint32_t)e->cls_sig.size() && e->d_pool &&
-      e->d_pool_used == e->pool.size() && e->max_nodes <= (uint32_t)(WAVE * KP_MAX_NS) &&
+      e->d_pool_used == e->pool_size && e->max_nodes <= (uint32_t)(WAVE * KP_MAX_NS) &&
       kp_lds_bytes(e->max_nodes, e->max_slots) <= 64 * 1024) {
     if (int rc = ensure_perm(e, 0, n)) return rc;
     uint32_t* const d_unknown = e->d_queues + (N_QUEUES - 1);
@@ -2368,7 +2415,7 @@ int rpeg_eval_batch_static(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     return -9;
   }
   if (!plans->vert || !plans->head || plans->stride < n) { e->err = "bad plan tensors"; return -1; }
-  if (!e->d_hkey || e->tables_for != (uint32_t)e->cls_sig.size() || e->d_pool_used != e->pool.size() || !e->d_pool) {
+  if (!e->d_hkey || e->tables_for != (uint32_t)e->cls_sig.size() || e->d_pool_used != e->pool_size || !e->d_pool) {
     e->err = "the engine's class tables are not on the device: evaluate a batch with these classes through rpeg_eval_batch first";
     return -10;
   }
@@ -2498,7 +2545,7 @@ int rpeg_eval_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t*
   if (dispatch_index) HIP_TRY(e, hipMemcpy(dispatch_index, d_tr + 2 * (size_t)n, (size_t)n * 4, hipMemcpyDeviceToHost));
   describe_nodes(e->P, e->P.st[h.structure], h, a, lc, node_kind, node_vertex, node_step, node_sub, node_src, nullptr, nullptr);
   if (node_reserved) {   // the vertices whose allocations the scheduler reserves for the node
-    const ClassView cv = class_view(e->pool.data() + off);
+    const ClassView cv = class_view(lc.blob.data());
     const uint64_t dpne = plan_masks(a, e->P.st[h.structure].n_vertex).dpne;
     for (int i = 0; i < n; ++i) node_reserved[i] = (uint8_t)blocked_mask(cv.node[i], dpne);
   }
@@ -2567,7 +2614,7 @@ int rpeg_plan_detail(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t
   HIP_TRY(e, hipGetLastError());
   double out[SLOTS + WAVE];
   HIP_TRY(e, hipMemcpy(out, d_out, sizeof out, hipMemcpyDeviceToHost));
-  const ClassView cv = class_view(e->pool.data() + off);
+  const ClassView cv = class_view(lc.blob.data());
   for (int i = 0; i < n; ++i) {
     const LoweredNode& nd = lc.nodes[i];
     const SlotDesc sd = cv.slot[nd.slot];
