@@ -453,7 +453,7 @@ int rpeg_sa_propose(rpeg_engine_t* e, const rpeg_sa_params_t* prm, int32_t what,
    wavefront), [6] plans of a large batch that ran one per wavefront beside the main kernel (included
    in [2]), [7] wave tasks of the few-lanes-per-plan kernel (included in [2]), [8] plans that the call BEFORE the last
    one redid because their ready sets outgrew their kernel's (both calls laid out by the host: a batch that needed no
-   layout leaves the figure as it is). */
+   layout leaves the figure as it is), [9] plans of the few-lanes-per-plan kernel. */
 int rpeg_engine_stats(const rpeg_engine_t* e, uint64_t* out, int32_t n);
 
 /* Host time of the last rpeg_eval_batch call that laid its batch out, in microseconds of the steady clock: [0] from
@@ -500,12 +500,14 @@ int rpeg_engine_set_sa_groups(rpeg_engine_t* e, int32_t groups);
    it.  No counterpart in the reference. */
 int rpeg_engine_set_side_layout(rpeg_engine_t* e, int32_t on);
 
-/* With lanes = -1: whether full batches may run in the kernel of two or four lanes per plan (percent > 0, default 25;
-   0: no, and nothing that was measured decides where a class runs).  What it takes is learned: the main kernel records, per class,
-   how long its slowest wavefront ran, how many heap pops per dispatch it needed and the longest ready set, and from
-   the second call on a batch that would end earlier there moves, its smallest classes and largest graphs to the
-   one-plan-per-wavefront kernel beside it.  Results do not depend on the setting.  No reference counterpart (a tuning
-   knob). */
+/* With lanes = -1: the largest share of a batch's plans, in percent, that the kernel of two or four lanes per plan may take
+   (default 100; 0: none, and nothing that was measured decides where a class runs).  What it takes is learned: the main
+   kernel records, per class, how long its slowest wavefront ran, how many heap pops per dispatch it needed and the
+   longest ready set, and from the second call on a batch that would end earlier there moves, its smallest classes and
+   largest graphs to the one-plan-per-wavefront kernel beside it.  Below 100 the classes with the largest graphs move, as
+   many as the share holds, and the main kernel keeps the others; a batch of under two of that kernel's wavefronts per
+   compute unit, which moves without being measured, then does not move.  Results do not depend on the setting.  No
+   reference counterpart (a tuning knob). */
 int rpeg_engine_set_quad_share(rpeg_engine_t* e, int32_t percent);
 
 /* Ready-list entries per plan in the main kernel: 8, 16, 24 or 32 (default).  A plan with that many nodes

@@ -823,7 +823,7 @@ struct rpeg_engine_s {
   hipEvent_t ev_sig = nullptr;                  // the signature kernel of a call is done (its class ids are there)
   bool layout_ahead = true;                     // prologue, layout and main kernel on k_quad's stream (see `ahead` in eval_batch_impl)
   int side_dev = 0;                             // device of the side streams
-  uint32_t quad_share_pct = 25;                 // share of a full batch that k_quad takes (rpeg_engine_set_quad_share)
+  uint32_t quad_share_pct = 100;                // largest share of a batch's plans that k_quad takes (rpeg_engine_set_quad_share)
   bool quad_attr_set = false;
   int split_heavy = 1;                          // 0: the classes with the largest graphs stay in the main kernel
   uint64_t* d_sig = nullptr;
@@ -850,7 +850,7 @@ struct rpeg_engine_s {
   bool timing = false;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms = -1.0;
-  uint64_t stats[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  uint64_t stats[10] = {};
   double host_us[4] = {0, 0, 0, 0};   // host time of the last laid-out rpeg_eval_batch call: rpeg_engine_host_us
   int n_cu = 256;
   uint8_t* static_ptr = nullptr;    // this device's copy of the file-scope scratch array (rpeg_eval_batch_static)
@@ -1356,7 +1356,7 @@ int rpeg_engine_reset_classes(rpeg_engine_t* e) {
 
 int rpeg_engine_stats(const rpeg_engine_t* e, uint64_t* out, int32_t n) {
   if (!e || !out) return -1;
-  for (int i = 0; i < n && i < 9; ++i) out[i] = e->stats[i];
+  for (int i = 0; i < n && i < 10; ++i) out[i] = e->stats[i];
   return 0;
 }
 
@@ -1515,7 +1515,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     if (e->h_ccount[0] == 0u) {
       e->stats[0] = e->cls_sig.size();   // (the classes the engine knows: which of them the batch holds was not counted)
       e->stats[1] = 0; e->stats[2] = n; e->stats[3] = lds; e->stats[4] = 0; e->stats[5] = 1; e->stats[6] = 0;
-      e->stats[7] = 0;
+      e->stats[7] = e->stats[9] = 0;
       ++e->batch_calls;
       if (e->timing) {
         float ms = 0.f;
@@ -1684,7 +1684,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       ls = 0;
       if (one_fits && waves_for(1) <= (uint64_t)e->n_cu * e->one_plan_waves_per_cu) {
         one = true;   // the batch does not fill the chip with a plan per lane: spread every plan over a wavefront
-      } else if (waves_for(WAVE) < (uint64_t)e->n_cu * 2 && !quad_free) {   // under two wavefronts per compute unit
+      } else if (waves_for(WAVE) < (uint64_t)e->n_cu * 2 && !(quad_free && e->quad_share_pct == 100)) {   // under two wavefronts per compute unit, and not for k_quad
         for (int l : {8, 16, 32, 64}) {              // fewest plans per wavefront that still gives each its own SIMD
           if (!fits(l)) break;
           ls = l;
@@ -1793,19 +1793,21 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       if (k < order.size()) { w_quad -= cost_quad(order[k]); w_plan += cost_plan(order[k]); }
     }
     if (!shallow && !(dm.sm.quad_margin * best < dm.best(w_main, base_plan, max_main, nullptr))) return false;
+    // (with a bound on its share the largest graphs first, which would end last in the main kernel; that one keeps the rest)
+    uint64_t taken = 0;
     for (size_t k = 0; k < order.size(); ++k) {
       const uint32_t c = order[k];
       if (to_plan[c] || k < best_k) solo[c] = 1;
-      else quad[c] = 1;
+      else if ((taken + counts[c]) * 100 <= n * e->quad_share_pct) { quad[c] = 1; taken += counts[c]; }
     }
     return true;
   };
   // Where every class runs is decided from the class counts and what has been measured (below): on a batch of
   // thousands of classes that is 0.2 ms of host work.  The decision is kept per class for the next fifteen calls on
   // batches of about the same size (a class not seen then goes by the plain size rule), unless new measurements
-  // are about to be read.
+  // are about to be read or k_quad's share is bounded.
   bool by_quad = false;
-  const bool keep_split = !ls && !one && !quad_all && e->quad_share_pct && e->split_for_n && e->learn_calls == 0 &&
+  const bool keep_split = !ls && !one && !quad_all && e->quad_share_pct == 100 && e->split_for_n && e->learn_calls == 0 &&
                           n * 4 >= e->split_for_n * 3 && n * 3 <= e->split_for_n * 4 && e->batch_calls - e->split_at < 16 &&
                           e->split_mass == (mass != nullptr);
   if (keep_split) {
@@ -1817,7 +1819,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       else if (a == 2) (e->cls_need[cids[c]] > QUAD_KIND[1].entries ? solo[c] : quad[c]) = 1;   // (as plan_quad would, once a ready set has outgrown sixteen entries)
     }
   } else if (!ls && !one && !quad_all && !order.empty() && (by_quad = plan_quad())) {
-    // (decided: every class in k_quad or, tiny classes and the largest graphs, in k_plan)
+    // (decided: every class in k_quad, as far as its share goes, or, tiny classes and the largest graphs, in k_plan)
   } else if (!ls && !one && !quad_all && !order.empty()) {
     // The kernel ends with its slowest wavefront, and a wavefront is as slow as its slowest plan.  The
     // classes with the largest graphs (up to 15 % of the batch: beyond that the single-plan kernel would be
@@ -1975,6 +1977,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     if (unmeasured && e->learn_calls == 0 && e->batch_calls - e->relearn_at >= 8) { e->learn_calls = 1; e->relearn_at = e->batch_calls; }
   }
   uint32_t n_eval_waves = 0, n_quad_waves = 0, n_solo = 0;
+  uint64_t n_quad_plans = 0;
   for (size_t k = 0; k < order.size(); ++k) {
     const uint32_t c = order[k];
     if (solo[c] || quad[c]) continue;
@@ -2011,6 +2014,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
         const uint32_t c = qc[k];
         QuadLaunch& q = quad_launch[k < cut ? kind : 3];
         clpw[c] = QUAD_KIND[kind].plans;
+        n_quad_plans += counts[c];
         first[c] = n_eval_waves + n_quad_waves;
         const uint32_t nw = waves_of(c, kind);
         if (!q.waves) { q.first = n_quad_waves; q.kind = kind; }
@@ -2185,6 +2189,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   }
   e->stats[2] = n_waves + n_quad_waves + n_solo;
   e->stats[7] = n_quad_waves;
+  e->stats[9] = n_quad_plans;
   e->stats[3] = lds;
   e->stats[4] = wsb * grid;
   e->stats[5] = one ? 1u : (uint64_t)ls;
@@ -2265,7 +2270,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   const bool quad_on_s4 = quad_launch[2].waves || quad_launch[3].waves, peaks_on_s4 = peaks_apart && !peaks_on_s2 && !quad_on_s4;
   if (quad_on_s4 || peaks_on_s4) HIP_TRY(e, hipStreamWaitEvent(e->s4, e->ev_fork, 0));
   if (int rc = launch_quad(quad_launch[2], e->s4)) return rc;
-  if (int rc = launch_quad(quad_launch[0], sm)) return rc;
+  if (int rc = launch_quad(quad_launch[0], n_waves ? sq : sm)) return rc;   // (beside the main kernel, where that has tasks)
   if (int rc = launch_quad(quad_launch[1], sq)) return rc;
   if (int rc = launch_quad(quad_launch[3], e->s4)) return rc;
   if (n_solo) {   // the single-plan wavefronts, beside the main kernel
@@ -2444,7 +2449,7 @@ int rpeg_eval_batch_static(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   launch_plan(lds, s, L, e->n_cu);
   HIP_TRY(e, hipGetLastError());
   e->stats[0] = 0; e->stats[1] = 0; e->stats[2] = n; e->stats[3] = lds; e->stats[4] = 0; e->stats[5] = 1; e->stats[6] = 0;
-  e->stats[7] = 0;
+  e->stats[7] = e->stats[9] = 0;
   // With RPEG_NO_WAIT the call ends here: three launches on the caller's stream, no copy and no wait (what a
   // capturing stream accepts).  Plans of classes the engine has not met are then told by their mask alone.
   if (flags & RPEG_NO_WAIT) return 0;
@@ -2783,6 +2788,7 @@ int host_small_submit(rpeg_engine_t* e, HostLane& ln, uint64_t n, GET get, uint3
   }
   const size_t m = ln.idx.size();
   e->stats[0] = 0; e->stats[1] = n_new; e->stats[2] = m; e->stats[3] = 0; e->stats[4] = 0; e->stats[5] = 1; e->stats[6] = 0;
+  e->stats[7] = e->stats[9] = 0;
   if (m == 0) return 0;
   if (e->max_nodes > (uint32_t)(WAVE * KP_MAX_NS) || kp_lds_bytes(e->max_nodes, e->max_slots) > 64 * 1024) return 1;
   if (int rc = ensure_pool(e, s)) return rc;

@@ -238,7 +238,7 @@ class Engine:
         self._check(self.lib.rpeg_engine_set_side_layout(self._h, 1 if on else 0), "rpeg_engine_set_side_layout")
 
     def set_quad_share(self, percent: int):
-        """Whether full batches may run in the few-lanes-per-plan kernel (percent > 0; 0: no)."""
+        """The largest share of a batch's plans that the few-lanes-per-plan kernel may take (0: none; 100, the default: all)."""
         self._check(self.lib.rpeg_engine_set_quad_share(self._h, int(percent)), "rpeg_engine_set_quad_share")
 
     def set_ready_cap(self, entries: int):
@@ -253,10 +253,10 @@ class Engine:
         return float(self.lib.rpeg_engine_last_kernel_ms(self._h))
 
     def stats(self) -> Dict[str, int]:
-        buf = (C.c_uint64 * 9)()
-        self.lib.rpeg_engine_stats(self._h, buf, 9)
+        buf = (C.c_uint64 * 10)()
+        self.lib.rpeg_engine_stats(self._h, buf, 10)
         return dict(classes=buf[0], classes_lowered=buf[1], wave_tasks=buf[2], lds_bytes=buf[3], workspace_bytes=buf[4],
-                    state_lanes=buf[5], single_plan_tasks=buf[6], quad_tasks=buf[7], redone_before=buf[8])
+                    state_lanes=buf[5], single_plan_tasks=buf[6], quad_tasks=buf[7], redone_before=buf[8], quad_plans=buf[9])
 
     def alloc_outputs(self, n: int):
         torch = _torch()
