@@ -712,7 +712,7 @@ struct SplitModel {
   double quad_margin = 1.15;
   double gain_threshold = 0.97, gain_classes = 0.98;
 };
-constexpr int SPLIT_MODEL_FIELDS = 9;
+constexpr int SPLIT_MODEL_FIELDS = 10;   // (plan_list last, and optional, in the setter's order)
 
 // Staging of one small host-pointer evaluation: plan records in (EvalLaunch::rec), results out, both pinned, and which
 // of the caller's plans went to the device.  The kernel reads the records where they lie (no copy ahead of the launch)
@@ -1291,12 +1291,13 @@ int rpeg_engine_set_state_lanes(rpeg_engine_t* e, int32_t lanes) {
 }
 
 int rpeg_engine_set_split_model(rpeg_engine_t* e, const double* values, int32_t n) {
-  if (!e || !values || n != SPLIT_MODEL_FIELDS) { if (e) e->err = "nine figures"; return -1; }
+  if (!e || !values || (n != SPLIT_MODEL_FIELDS && n != SPLIT_MODEL_FIELDS - 1)) { if (e) e->err = "nine figures or ten"; return -1; }
   for (int i = 0; i < n; ++i)
     if (!(values[i] >= 0.0)) { e->err = "the figures are non-negative"; return -1; }
   SplitModel& m = e->split_model;
   m.plan_a = values[0]; m.plan_b = values[1]; m.quad_a = values[2]; m.quad_b = values[3]; m.quad_c = values[4];
   m.eff_beside_quad = values[5]; m.quad_margin = values[6]; m.gain_threshold = values[7]; m.gain_classes = values[8];
+  if (n == SPLIT_MODEL_FIELDS) m.plan_list = values[9];
   e->split_for_n = 0;
   return 0;
 }

@@ -225,7 +225,7 @@ class Engine:
         return dict(launch_gate=float(v[0]), wait_counts=float(v[1]), layout_and_split=float(v[2]), launch_schedulers=float(v[3]))
 
     def set_split_model(self, values):
-        """The nine fitted figures of the split between the scheduling kernels (rpeg_engine_set_split_model)."""
+        """The fitted figures of the split between the scheduling kernels, nine or all ten (rpeg_engine_set_split_model)."""
         v = np.ascontiguousarray(values, dtype=np.float64)
         self._check(self.lib.rpeg_engine_set_split_model(self._h, v.ctypes.data, len(v)), "rpeg_engine_set_split_model")
 

@@ -451,7 +451,7 @@ def test_the_fitted_figures_of_the_split_move_plans_between_kernels_and_no_bit()
     cfg, batch = seeded_batch(2, 65536)
     ref = CpuPort(cfg.problem).eval(batch, flags=abi.GATE_STALE, threads=16)
     layouts = []
-    for model in ([40.0, 2.2, 40.0, 1.6, 0.45, 0.65, 1.15, 0.97, 0.98],    # the defaults
+    for model in ([12.0, 0.9, 10.0, 1.3, 0.2, 0.65, 1.15, 0.97, 0.98],     # the defaults
                   [1.0, 0.1, 40.0, 1.6, 0.45, 1.0, 1.15, 0.97, 0.98],      # a plan costs k_plan next to nothing
                   [40.0, 2.2, 1.0, 0.1, 0.0, 0.65, 1.0, 0.97, 0.98],       # a wavefront of k_quad costs next to nothing
                   [400.0, 20.0, 4000.0, 20.0, 5.0, 0.1, 2.0, 0.5, 0.5]):   # both dear
