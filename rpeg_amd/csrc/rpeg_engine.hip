@@ -747,7 +747,7 @@ struct rpeg_engine_s {
   std::vector<uint32_t> cls_off, cls_nodes, cls_slots;
   std::vector<uint32_t> cls_pops16;                  // learned, of the slowest full wavefront of the class in the main kernel:
                                                      // microseconds << 12 | heap pops per dispatch in sixteenths
-  std::vector<uint32_t> cls_need;                    // learned: the longest ready set of the class's plans in k_quad (0: none yet)
+  std::vector<uint32_t> cls_need;                    // learned: the longest ready set of the class's plans in k_quad or the main kernel (0: none yet)
   uint32_t* d_cstat = nullptr;                       // the device's copies, one behind the other (cstat_cap words each)
   uint32_t cstat_cap = 0;
   std::vector<uint8_t> cls_split;                    // where every class ran when that was last decided: 0 main kernel, 1 k_plan,
@@ -1741,7 +1741,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // would take are in classes whose ready sets the main kernel has measured; the others' unknown ready sets take the form with
   // the most entries.
   // Measured, us per step, main kernel / k_quad: GRPO (51 nodes on average) 17,000 plans 402 / 270, 65,536 460 / 365,
-  // 131,072 716 / 580; PPO (98) 20,011 548 / 410, 131,072 1,616 / 1,505; DPO (28) 65,536 277 / 140, 1,048,576 1,686 /
+  // 131,072 716 / 580; PPO (98) 20,011 548 / 384, 131,072 1,616 / 1,505; DPO (28) 65,536 277 / 140, 1,048,576 1,686 /
   // 1,225.  AC-share (152): 20,011 1,216 / 930, but 65,536 2,353 / 2,300-2,500 and 262,144 5,549 / 8,426: of large graphs
   // few plans have room in LDS, and the main kernel keeps its state in HBM: a batch of more than sixteen of its wavefronts
   // per compute unit stays there where the plans have more than QUAD_MEAN_NODES nodes on average.
@@ -1866,10 +1866,11 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
         }
     // A class with a handful of plans would occupy a wavefront of the main kernel with nearly all lanes idle
     // (on the seeded set of config 3, 46 % of the wavefronts carried 4 % of the plans): its plans get a
-    // wavefront each as well.  Six wavefronts of the main kernel and sixteen of k_plan fit on a compute unit,
-    // and a plan takes k_plan about half as long as a wavefront takes the main kernel: below six plans k_plan
-    // is the cheaper place; the two kernels also run side by side (one waits on latencies, the other issues
-    // vector instructions), and on config 3 any threshold between 8 and 32 plans gives the same step time.
+    // wavefront each as well.  Four or five wavefronts of the main kernel and sixteen of k_plan fit on a compute unit,
+    // and a plan takes k_plan about a seventh as long as a wavefront takes the main kernel (100-150 nodes, side by side
+    // on 262,144 AC-share plans: 95 against 700 us): below some twenty plans k_plan is the cheaper place.  The two
+    // kernels also run side by side (one waits on latencies, the other issues vector instructions): with a k_plan that
+    // took two to three times as long any threshold between 8 and 32 plans gave those plans the same step time.
     if (split)
       for (size_t c = 0; c < counts.size(); ++c)
         if (counts[c] < TINY_CLASS) solo[c] = 1;
@@ -2076,7 +2077,8 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     if (solo[c] || one) {
       continue;
     } else {
-      // (never for a task of k_quad, whose eight plans of eight lanes each are not that layout)
+      // (a task of k_quad: the class's ready sets fit two entries per lane; of the main kernel: its few plans keep their
+      // state in LDS)
       const uint32_t flag = (quad[c] ? quad_kind(c) == 1 && e->cls_need[cids[c]] <= QUAD_KIND[0].entries : few_in_lds && clpw[c] == (uint32_t)KE_FEW) ? KE_CLS_LDS : 0u;
       const uint32_t nw = (counts[c] + clpw[c] - 1) / clpw[c];
       for (uint32_t t = 0; t < nw; ++t) h_tasks[first[c] + t] = offs[c] | flag;

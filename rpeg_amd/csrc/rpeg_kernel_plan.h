@@ -1,25 +1,20 @@
-// rpeg_kernel_plan.h - the evaluation kernel for batches too small to fill the chip with one plan per
-// lane (device only): ONE PLAN PER WAVEFRONT.
+// rpeg_kernel_plan.h - the evaluation kernel of small batches, of the smallest classes and of the largest graphs (device
+// only): ONE PLAN PER WAVEFRONT, or per block of four.
 //
 // The lanes share the plan's work instead of each carrying a plan of its own:
 //   cost model      lane = duration slot of the class (NodeCostModel.time of one node variant each)
 //   memory model    lane = template vertex, then lane = vertex subset (candidate device class)
-//   ranks           lane = lowered node; Jacobi rounds of rank = duration + max(rank of successors) until
-//                   nothing changes (the fixed point is the reverse topological pass of scheduler.py:71-100)
-//   list scheduler  lane = lowered node (NS nodes per lane).  Every node keeps its heap key, its tie-break
-//                   word, the latest finish of its predecessors and the availability of the devices it
-//                   reserves in registers.  The heap's pop is a minimum over the wavefront (row shifts and
-//                   broadcasts, no memory); all control flow is uniform, so the loop runs on the scalar unit
-//                   and the successors of the dispatched node are read from the winner lane's registers.
+//   ranks           level by level from the nodes without successors, lane = node of the level (scheduler.py:71-100)
+//   positions       lane = node, which counts the nodes of its tie-break class with a larger rank
+//   list scheduler  rpeg_kernel_sched.h: up to 128 nodes a lane (or two) for every node, dealt by position; beyond that a
+//                   lane for every waiting node, the others in LDS.  All control flow is uniform
+//   outputs         lane = node for the predecessors of the critical chain, lane = set of allocations for the utilisation
 //
-// The heap key of the reference is (est, comm_prio, topo_idx, -rank, tie).  (comm_prio, topo_idx, -rank) is
-// fixed once the ranks are known, so it is replaced by the node's position in that order (equal triples get
-// equal positions), packed above the tie counter in one 32-bit word: a pop is the minimum of a double and,
-// among equals, of that word.
+// Device availability: a node waits for max(avail[d]) over the devices it reserves, i.e. for the largest finish time of
+// any dispatched node whose reserved vertices intersect its own.  Every lane keeps that maximum for its nodes and raises
+// it at each dispatch (max is exact, so the order does not matter).
 //
-// Device availability: a node waits for max(avail[d]) over the devices it reserves, i.e. for the largest
-// finish time of any dispatched node whose reserved vertices intersect its own.  Every lane keeps that
-// maximum for its nodes and raises it at each dispatch (max is exact, so the order does not matter).
+// As a task of a laid-out batch durations, pair relations, penalty factor and gate bits come from the prologue launches.
 #ifndef RPEG_KERNEL_PLAN_H
 #define RPEG_KERNEL_PLAN_H
 

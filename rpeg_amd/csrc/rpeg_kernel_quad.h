@@ -39,7 +39,7 @@
 // and are bound by issue.
 // Scheduling a wavefront: 42-node GRPO class 60 us, 92 nodes 130-190, 28-node DPO class 35.  The step, main kernel and
 // the earlier form of this one (every push-back carried out) against now: 65,536 GRPO plans 460 -> 365 us, 1,048,576 DPO
-// plans 1,686 -> 1,225, 20,011 PPO plans 548 -> 410.
+// plans 1,686 -> 1,190, 20,011 PPO plans 548 -> 384.
 #ifndef RPEG_KERNEL_QUAD_H
 #define RPEG_KERNEL_QUAD_H
 

@@ -24,9 +24,10 @@
 // Bound: instruction issue of one wavefront.  On gfx950 an instruction costs it ~4.4 clocks however simple, a branch
 // that falls through 12, a taken one 25, a value crossing from the vector to the scalar side and back 15 more, an LDS
 // read 50-64.  With every waiting node's push-backs carried out in the reference's order a decision took 1,700 clocks;
-// now it takes 830 (28 nodes, one to a lane), 1,020 (96 nodes, two to a lane) and 1,370 (150 nodes and more, kp_list).
+// now it takes 790-890 (28-45 nodes, one to a lane), 860-1,140 (75-107 nodes, two to a lane) and 1,290-1,470 (130 nodes
+// and more, kp_list), 330-610 ns at 2.4 GHz, by how many positions are shared.
 // Measured, a plan's scheduling alone on its SIMD, 150 plans in one launch, before and after: PPO (K = 4) mean 72 ->
-// 41 us, slowest 133 -> 82; 300-node AC-share graphs 440 -> 228 us.  20,011 PPO plans, a wavefront each: 577 us.
+// 41 us, slowest 133 -> 76; 161-node AC-share graphs 90 us, of 300 nodes 440 -> 228 us.
 #ifndef RPEG_KERNEL_SCHED_H
 #define RPEG_KERNEL_SCHED_H
 

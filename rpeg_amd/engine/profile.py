@@ -67,7 +67,8 @@ def main() -> None:
     nodes = (buf[:, 7] >> np.uint64(32)).astype(np.int64)
     t0 = b[:, 0][b[:, 0] > 0].min()
     start, end = (b[:, 0] - t0) / 100.0, (b[:, 6] - t0) / 100.0          # the stamps tick at 100 MHz: microseconds
-    for name, sl in (("k_eval", slice(0, n_eval)), ("k_quad", slice(n_eval, n_lane)), ("k_plan", slice(n_lane, got))):
+    first = "k_plan" if s["state_lanes"] == 1 else "k_eval"      # (a batch of one plan per wavefront throughout)
+    for name, sl in ((first, slice(0, n_eval)), ("k_quad", slice(n_eval, n_lane)), ("k_plan", slice(n_lane, got))):
         S, E, N = start[sl], end[sl], nodes[sl]
         ok = E > 0
         S, E, N = S[ok], E[ok], N[ok]
