@@ -1002,7 +1002,7 @@ static int ensure_pool(rpeg_engine_t* e, hipStream_t s) {
   }
   if (e->n_fresh) {
     for (size_t k = 0; k < e->n_fresh; ++k)
-      HIP_TRY(e, hipMemcpyAsync(e->d_pool + e->fresh[k].off, e->fresh[k].bytes.data(), e->fresh[k].bytes.size(), hipMemcpyHostToDevice, s));
+      if (!e->fresh[k].bytes.empty()) HIP_TRY(e, hipMemcpyAsync(e->d_pool + e->fresh[k].off, e->fresh[k].bytes.data(), e->fresh[k].bytes.size(), hipMemcpyHostToDevice, s));
     // the host buffers are filled again by the next classes: finish the copies first
     HIP_TRY(e, hipStreamSynchronize(s));
     e->n_fresh = 0;

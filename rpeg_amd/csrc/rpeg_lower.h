@@ -42,10 +42,13 @@ struct LowerTables {
       std::memset(t.rel, NONE, sizeof t.rel);
       if (s >= P.n_struct || (only >= 0 && s != only)) continue;
       t.n_uni = slot_universe(P, P.st[s], t.uni);
-      for (int u = 0; u < t.n_uni && u < RPEG_MAX_UNIVERSE; ++u) t.at[key(t.uni[u].type, t.uni[u].a, t.uni[u].b, t.uni[u].q)] = (uint8_t)u;
-      for (int r = P.st[s].n_rel - 1; r >= 0; --r) {   // (of several entries for a pair the first)
+      for (int u = 0; u < t.n_uni && u < RPEG_MAX_UNIVERSE; ++u) {
+        const unsigned k = key(t.uni[u].type, t.uni[u].a, t.uni[u].b, t.uni[u].q);
+        if (k < sizeof t.at) t.at[k] = (uint8_t)u;
+      }
+      for (int r = std::min<int>(P.st[s].n_rel, RPEG_MAX_REL) - 1; r >= 0; --r) {   // (of several entries for a pair the first)
         const rpeg_rel_t& x = P.st[s].rel[r];
-        t.rel[x.u][x.v] = t.rel[x.v][x.u] = (uint8_t)r;
+        if ((unsigned)x.u < RPEG_MAX_V && (unsigned)x.v < RPEG_MAX_V) t.rel[x.u][x.v] = t.rel[x.v][x.u] = (uint8_t)r;
       }
     }
   }
