@@ -697,7 +697,7 @@ static uint8_t* static_scratch_ptr(int dev, hipError_t* st) {
 // rpeg_engine_set_split_model replaces them (a measurement aid).  A wrong figure
 // costs time, never a result: every kernel computes the same bits.
 //   plan_a + plan_b x nodes                    what a plan costs k_plan (one plan per wavefront), beside the main kernel;
-//                                              plan_list times as much beyond KP_LANE_NODES nodes, where its scheduler
+//                                              plan_list times as much beyond 128 nodes, where its scheduler
 //                                              keeps the nodes in LDS and fewer of its wavefronts fit on a compute unit
 //   quad_a + nodes x (quad_b + quad_c x pops)  a wavefront of k_quad; pops = heap pops per dispatch, as the main kernel
 //                                              measured them for the class
@@ -1391,7 +1391,7 @@ struct DeepModel {
   uint64_t r_max;
   SplitModel sm;
   double plan_cost(uint32_t plans, uint32_t nodes) const {
-    return (double)plans * (sm.plan_a + sm.plan_b * (double)nodes) * (nodes > (uint32_t)KP_LANE_NODES ? sm.plan_list : 1.0);
+    return (double)plans * (sm.plan_a + sm.plan_b * (double)nodes) * (nodes > 128u ? sm.plan_list : 1.0);
   }
   double total(double w_main, double w_plan, double max_t, uint64_t r) const {
     const double t_main = std::max(max_t, w_main / (n_cu * (double)r));

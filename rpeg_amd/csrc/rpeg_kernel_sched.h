@@ -4,7 +4,7 @@
 // have to find room for them among the launch record and the cost model, and spill in their loops):
 //   kp_ranks        ranks of the lowered nodes
 //   kp_positions    from them every node's position in the order that breaks ties
-//   kp_lanes        the scheduler for graphs of at most 128 nodes: every node has a lane of its own
+//   kp_lanes        the scheduler for graphs of at most 192 nodes: every node has a lane of its own, or a third of one
 //   kp_list         the scheduler for larger graphs: every waiting node has a lane, the others live in LDS
 //   kp_plain        the textbook form, for a graph whose waiting nodes outgrow a wavefront in kp_list
 //
@@ -21,13 +21,16 @@
 // true time as key and fresh ties in the order of their old (key, tie), and where several entries share the smallest
 // (e, position), current ones come first, by tie, then stale ones, by old (key, tie).
 //
-// Bound: instruction issue of one wavefront.  On gfx950 an instruction costs it ~4.4 clocks however simple, a branch
-// that falls through 12, a taken one 25, a value crossing from the vector to the scalar side and back 15 more, an LDS
-// read 50-64.  With every waiting node's push-backs carried out in the reference's order a decision took 1,700 clocks;
-// now it takes 790-890 (28-45 nodes, one to a lane), 860-1,140 (75-107 nodes, two to a lane) and 1,290-1,470 (130 nodes
-// and more, kp_list), 330-610 ns at 2.4 GHz, by how many positions are shared.
-// Measured, a plan's scheduling alone on its SIMD, 150 plans in one launch, before and after: PPO (K = 4) mean 72 ->
-// 41 us, slowest 133 -> 76; 161-node AC-share graphs 90 us, of 300 nodes 440 -> 228 us.
+// Bound: one wavefront's instructions, one after the other.  Measured on gfx950, clocks: a vector or scalar instruction 4.6
+// where it does not need the one before it, 8.2 where it does; a step of a reduction over the lanes 16; a branch that
+// falls through 12, a taken one 24; v_readlane of a lane number in a register 8.6, v_readfirstlane 4.9; a comparison to
+// the scalar side and back 32; an LDS read 52.  A decision without live entries of shared position takes 310-330 clocks
+// (one node to a lane), 400 (two), 600 (three) and 1,060-1,110 (kp_list); where such entries wait 100-500 more, and each
+// one pushed back among others of its position 120-260.
+// Before that form (a node's key and the availability of its devices kept apart, the candidates' registers selected and
+// read behind the reduction, four branches): 470, 750, and kp_list beyond 128 nodes.  150 plans in one launch, a plan's
+// scheduling before -> now, mean: DPO 9.4 -> 7.0 us, PPO (K = 4) of 65-128 nodes 37 -> 22, of 129-192 73 -> 48, AC-share of
+// those sizes 51 -> 34 and 82 -> 65.
 #ifndef RPEG_KERNEL_SCHED_H
 #define RPEG_KERNEL_SCHED_H
 
@@ -35,7 +38,7 @@
 
 namespace rpeg {
 
-constexpr int KP_LANE_NODES = 128;   // largest graph of kp_lanes: beyond two nodes to a lane its decisions are the slower ones
+constexpr int KP_LANE_NODES = 192;   // largest graph of kp_lanes: five nodes to a lane were tried, 300-node graphs 150 -> 205 us
 
 #if defined(__HIPCC__)
 
@@ -86,23 +89,46 @@ __device__ inline double kp_vmax(double a, double b) {
   asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
   return r;
 }
-__device__ inline double kp_vmax_s(double a, double uniform) {   // the second operand from the scalar registers
+__device__ inline double kp_vmin(double a, double b) {   // (of a quiet NaN and a number the number)
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+// the second operand from scalar registers, which no vector instruction has written in the two wait states before
+__device__ inline double kp_vmax_s(double a, double uniform) {
   double r;
   asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "s"(uniform));
   return r;
 }
-// mask bit of this lane ? a : b.  (Written out: of a choice between two elements of a register array the compiler makes
-// an indexed load from scratch memory.)
-__device__ inline uint32_t kp_sel(unsigned long long mask, uint32_t a, uint32_t b) {
-  uint32_t r;
-  asm("v_cndmask_b32 %0, %1, %2, %3" : "=v"(r) : "v"(b), "v"(a), "s"(mask));
-  return r;
-}
+__device__ inline bool kp_in(unsigned long long mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }   // this lane's bit of a uniform mask
+// mask bit of this lane ? a : b.  (In the compiler's hands: a vector instruction that reads a mask another one has just
+// written needs two wait states between them, which inline assembly does not get.)
+__device__ inline uint32_t kp_sel(unsigned long long mask, uint32_t a, uint32_t b) { return kp_in(mask) ? a : b; }
 __device__ inline double kp_sel(unsigned long long mask, double a, double b) {
   return __hiloint2double((int)kp_sel(mask, (uint32_t)__double2hiint(a), (uint32_t)__double2hiint(b)),
                           (int)kp_sel(mask, (uint32_t)__double2loint(a), (uint32_t)__double2loint(b)));
 }
-__device__ inline bool kp_in(unsigned long long mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }   // this lane's bit of a uniform mask
+// Masks of 64 lanes by vector instructions, as two words.  (No 64-bit vector shift here: where its amount lies in the last
+// register of a wavefront's allocation, v_lshlrev_b64 has shifted every lane by the same wrong number.)
+struct KpMask { uint32_t lo, hi; };
+__device__ inline KpMask kp_bit(uint32_t l) {   // (none for 64 and more)
+  const uint32_t b = 1u << (l & 31u);
+  return {l < 32u ? b : 0u, l - 32u < 32u ? b : 0u};
+}
+__device__ inline KpMask kp_lanes_from_to(uint32_t a, uint32_t b) {   // a <= b < 64
+  auto word = [](int a, int b) { return b < 0 || a > 31 ? 0u : (0xFFFFFFFFu << (a < 0 ? 0 : a)) & (0xFFFFFFFFu >> (b > 31 ? 0 : 31 - b)); };
+  return {word((int)a, (int)b), word((int)a - 32, (int)b - 32)};
+}
+__device__ inline double kp_settled(double uniform) {   // (for kp_vmax_s)
+  asm("s_nop 1" : "+s"(uniform));
+  return uniform;
+}
+// v minus the mask's bit of this lane (the mask as the operand of kp_vmax_s)
+__device__ inline uint32_t kp_dec(unsigned long long mask, uint32_t v) {
+  uint32_t r;
+  asm("v_subb_co_u32 %0, vcc, %1, 0, %2" : "=v"(r) : "v"(v), "s"(mask) : "vcc");
+  return r;
+}
 
 enum KpTrace { KP_NO_TRACE = 0, KP_TIMES = 1, KP_TIMES_ORDER = 2 };   // what of the schedule is kept: nothing, start and
                                                                        // finish of every node, the dispatch order too
@@ -164,17 +190,13 @@ __device__ inline void kp_barrier() {
   else __syncthreads();
 }
 
-// Places of the fifth successor on of the node at level place `at`.
+// Places of a node's successors, from the first-th on.
 template <class VISIT>
-__device__ inline void kp_more_places(const KpClass& T, uint32_t node, uint32_t n_succ, VISIT&& visit) {
+__device__ inline void kp_more_places(const KpClass& T, uint32_t node, uint32_t first, VISIT&& visit) {
   const KP_CONST ClassHdr* h = T.hdr();
-  const uint32_t sb = T.at<uint16_t>(h->off_node + node * 8u)[0];   // (NodeRec::succ_begin)
-  for (uint32_t j = 4; j < n_succ; ++j) visit(kp_scalar(T.at<uint16_t>(h->off_place)[T.at<uint16_t>(h->off_succ)[sb + j]]));
-}
-template <class VISIT>
-__device__ inline void kp_more(const KpClass& T, const KpLds& M, uint32_t at, VISIT&& visit) {   // their positions
-  const uint32_t node = kp_scalar(M.rec[at].node), ns = kp_scalar(M.rec[at].n_succ);
-  kp_more_places(T, node, ns, [&](uint32_t p) { visit(kp_scalar(M.q[p])); });
+  const uint64_t rec = T.at<uint64_t>(h->off_node)[node];   // (NodeRec: succ_begin, n_succ)
+  const uint32_t sb = (uint32_t)rec & 0xFFFFu, n_succ = (uint32_t)(rec >> 16) & 0xFFu;
+  for (uint32_t j = first; j < n_succ; ++j) visit(kp_scalar(T.at<uint16_t>(h->off_place)[T.at<uint16_t>(h->off_succ)[sb + j]]));
 }
 // Reserved vertices of a node, and (second byte) the vertices whose allocations overlap one of them: its devices are busy
 // until the largest finish time of the dispatched nodes whose reserved vertices meet those (the relation is symmetric).
@@ -318,145 +340,443 @@ __device__ __attribute__((noinline)) void kp_positions(uint64_t blob, int wave, 
   kp_barrier<NW>();
 }
 
-// A graph of at most 64 * NS nodes: the nodes are dealt to the lanes by position (q: register slot q >> 6, lane q & 63),
-// so that among the waiting nodes of smallest true start time the one to dispatch is the lowest set bit of a ballot.  All
-// control flow is uniform.  Returns the makespan, or -1 where nothing was ready (a cycle) or a start time was infinite.
+// The head of a round of kp_lanes, written out because the order of its instructions is what it costs: the smallest high word h
+// over the 64 lanes (ghi), the lanes that have it (m), and the words of the lowest of them, read with the others switched
+// off (v_readlane of a lane number takes twice as long); differ: lanes of m with another first word.  A step of the
+// reduction needs what the step before it wrote two instructions later, a value that goes to the scalar side and back two
+// as well: other work stands in between where there is some, the slots of a lane being merged (in the lanes of `pick` the
+// first's words).  The lanes are all on before and after.
+#define KP_DPP_QUAD1 " quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+#define KP_DPP_QUAD2 " quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+#define KP_DPP_ROR4 " row_ror:4 row_mask:0xf bank_mask:0xf\n\t"
+#define KP_DPP_ROR8 " row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+#define KP_DPP_ROW15 " row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+#define KP_DPP_ROW31 " row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+struct KpHead {
+  uint32_t ghi;
+  mask64 m, differ;
+};
+__device__ inline KpHead kp_head(uint32_t h, double e, double dur, const uint32_t (&a)[7], double* f, uint32_t (&w)[7]) {   // *f = e + dur; a[1], a[2] are not read: f's words
+  KpHead o;
+  uint32_t t;
+  double fm;
+  asm("v_add_f64 %[f], %[e], %[d]\n\t"
+      "s_nop 0\n\t"
+      "v_min_u32_dpp %[t], %[h], %[h]" KP_DPP_QUAD1
+      "s_nop 1\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_QUAD2
+      "s_nop 1\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_ROR4
+      "s_nop 1\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_ROR8
+      "s_nop 1\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_ROW15
+      "s_nop 1\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_ROW31
+      "s_nop 1\n\t"
+      "v_readlane_b32 %[ghi], %[t], 63\n\t"
+      "s_nop 1\n\t"
+      "v_cmp_eq_u32 %[m], %[ghi], %[h]"
+      : [t] "=&v"(t), [f] "=&v"(fm), [ghi] "=&s"(o.ghi), [m] "=&s"(o.m)
+      : [h] "v"(h), [e] "v"(e), [d] "v"(dur));
+  const uint32_t f0 = (uint32_t)__double2loint(fm), f1 = (uint32_t)__double2hiint(fm);
+  asm("s_mov_b64 exec, %[m]\n\t"
+      "v_readfirstlane_b32 %[w0], %[a0]\n\t"
+      "v_readfirstlane_b32 %[w3], %[a3]\n\t"
+      "v_readfirstlane_b32 %[w4], %[a4]\n\t"
+      "v_cmp_ne_u32 %[differ], %[w0], %[a0]\n\t"
+      "v_readfirstlane_b32 %[w1], %[a1]\n\t"
+      "v_readfirstlane_b32 %[w2], %[a2]\n\t"
+      "v_readfirstlane_b32 %[w5], %[a5]\n\t"
+      "v_readfirstlane_b32 %[w6], %[a6]\n\t"
+      "s_mov_b64 exec, -1\n\t"
+      "s_nop 0"
+      : [differ] "=&s"(o.differ), [w0] "=&s"(w[0]), [w1] "=&s"(w[1]), [w2] "=&s"(w[2]), [w3] "=&s"(w[3]), [w4] "=&s"(w[4]), [w5] "=&s"(w[5]), [w6] "=&s"(w[6])
+      : [m] "s"(o.m), [a0] "v"(a[0]), [a1] "v"(f0), [a2] "v"(f1), [a3] "v"(a[3]), [a4] "v"(a[4]), [a5] "v"(a[5]), [a6] "v"(a[6]));
+  *f = fm;
+  return o;
+}
+__device__ inline KpHead kp_head(uint32_t h, const uint32_t (&v)[4], uint32_t (&w)[4]) {
+  KpHead o;
+  uint32_t t;
+  asm("s_nop 1\n\t"
+      "v_min_u32_dpp %[t], %[h], %[h]" KP_DPP_QUAD1
+      "s_nop 1\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_QUAD2
+      "s_nop 1\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_ROR4
+      "s_nop 1\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_ROR8
+      "s_nop 1\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_ROW15
+      "s_nop 1\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_ROW31
+      "s_nop 1\n\t"
+      "v_readlane_b32 %[ghi], %[t], 63\n\t"
+      "s_nop 1\n\t"
+      "v_cmp_eq_u32 %[m], %[ghi], %[h]\n\t"
+      "s_mov_b64 exec, %[m]\n\t"
+      "v_readfirstlane_b32 %[w3], %[v3]\n\t"
+      "v_readfirstlane_b32 %[w0], %[v0]\n\t"
+      "v_readfirstlane_b32 %[w1], %[v1]\n\t"
+      "v_readfirstlane_b32 %[w2], %[v2]\n\t"
+      "v_cmp_ne_u32 %[differ], %[w0], %[v0]\n\t"
+      "s_mov_b64 exec, -1\n\t"
+      "s_nop 0"
+      : [t] "=&v"(t), [ghi] "=&s"(o.ghi), [m] "=&s"(o.m), [differ] "=&s"(o.differ), [w0] "=&s"(w[0]), [w1] "=&s"(w[1]), [w2] "=&s"(w[2]), [w3] "=&s"(w[3])
+      : [h] "v"(h), [v0] "v"(v[0]), [v1] "v"(v[1]), [v2] "v"(v[2]), [v3] "v"(v[3]));
+  return o;
+}
+__device__ inline KpHead kp_head(uint32_t h, mask64 pick, const uint32_t (&a)[11], const uint32_t (&b)[11], uint32_t (&v)[11], uint32_t (&w)[11]) {
+  KpHead o;
+  uint32_t t;
+  asm("s_nop 1\n\t"
+      "v_min_u32_dpp %[t], %[h], %[h]" KP_DPP_QUAD1
+      "s_nop 0\n\t"
+      "v_cndmask_b32 %[v0], %[b0], %[a0], %[p]\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_QUAD2
+      "v_cndmask_b32 %[v1], %[b1], %[a1], %[p]\n\t"
+      "v_cndmask_b32 %[v2], %[b2], %[a2], %[p]\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_ROR4
+      "v_cndmask_b32 %[v3], %[b3], %[a3], %[p]\n\t"
+      "v_cndmask_b32 %[v4], %[b4], %[a4], %[p]\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_ROR8
+      "v_cndmask_b32 %[v5], %[b5], %[a5], %[p]\n\t"
+      "v_cndmask_b32 %[v6], %[b6], %[a6], %[p]\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_ROW15
+      "v_cndmask_b32 %[v7], %[b7], %[a7], %[p]\n\t"
+      "v_cndmask_b32 %[v8], %[b8], %[a8], %[p]\n\t"
+      "v_min_u32_dpp %[t], %[t], %[t]" KP_DPP_ROW31
+      "v_cndmask_b32 %[v9], %[b9], %[a9], %[p]\n\t"
+      "v_cndmask_b32 %[v10], %[b10], %[a10], %[p]\n\t"
+      "v_readlane_b32 %[ghi], %[t], 63\n\t"
+      "s_nop 1\n\t"
+      "v_cmp_eq_u32 %[m], %[ghi], %[h]"
+      : [t] "=&v"(t), [ghi] "=&s"(o.ghi), [m] "=&s"(o.m), [v0] "=&v"(v[0]), [v1] "=&v"(v[1]), [v2] "=&v"(v[2]), [v3] "=&v"(v[3]), [v4] "=&v"(v[4]),
+        [v5] "=&v"(v[5]), [v6] "=&v"(v[6]), [v7] "=&v"(v[7]), [v8] "=&v"(v[8]), [v9] "=&v"(v[9]), [v10] "=&v"(v[10])
+      : [h] "v"(h), [p] "s"(pick), [a0] "v"(a[0]), [a1] "v"(a[1]), [a2] "v"(a[2]), [a3] "v"(a[3]), [a4] "v"(a[4]), [a5] "v"(a[5]), [a6] "v"(a[6]),
+        [a7] "v"(a[7]), [a8] "v"(a[8]), [a9] "v"(a[9]), [a10] "v"(a[10]), [b0] "v"(b[0]), [b1] "v"(b[1]), [b2] "v"(b[2]), [b3] "v"(b[3]),
+        [b4] "v"(b[4]), [b5] "v"(b[5]), [b6] "v"(b[6]), [b7] "v"(b[7]), [b8] "v"(b[8]), [b9] "v"(b[9]), [b10] "v"(b[10]));
+  asm("s_mov_b64 exec, %[m]\n\t"
+      "v_readfirstlane_b32 %[w0], %[v0]\n\t"
+      "v_readfirstlane_b32 %[w3], %[v3]\n\t"
+      "v_readfirstlane_b32 %[w4], %[v4]\n\t"
+      "v_cmp_ne_u32 %[differ], %[w0], %[v0]\n\t"
+      "v_readfirstlane_b32 %[w1], %[v1]\n\t"
+      "v_readfirstlane_b32 %[w2], %[v2]\n\t"
+      "v_readfirstlane_b32 %[w5], %[v5]\n\t"
+      "v_readfirstlane_b32 %[w6], %[v6]\n\t"
+      "v_readfirstlane_b32 %[w7], %[v7]\n\t"
+      "v_readfirstlane_b32 %[w8], %[v8]\n\t"
+      "v_readfirstlane_b32 %[w9], %[v9]\n\t"
+      "v_readfirstlane_b32 %[w10], %[v10]\n\t"
+      "s_mov_b64 exec, -1\n\t"
+      "s_nop 0"
+      : [differ] "=&s"(o.differ), [w0] "=&s"(w[0]), [w1] "=&s"(w[1]), [w2] "=&s"(w[2]), [w3] "=&s"(w[3]), [w4] "=&s"(w[4]), [w5] "=&s"(w[5]),
+        [w6] "=&s"(w[6]), [w7] "=&s"(w[7]), [w8] "=&s"(w[8]), [w9] "=&s"(w[9]), [w10] "=&s"(w[10])
+      : [m] "s"(o.m), [v0] "v"(v[0]), [v1] "v"(v[1]), [v2] "v"(v[2]), [v3] "v"(v[3]), [v4] "v"(v[4]), [v5] "v"(v[5]), [v6] "v"(v[6]), [v7] "v"(v[7]),
+        [v8] "v"(v[8]), [v9] "v"(v[9]), [v10] "v"(v[10]));
+  return o;
+}
+
+// A graph of at most 64 * NS nodes: the nodes are dealt to the lanes by position (q: lane q / NS, slot q % NS), so that
+// among the waiting nodes of smallest true start time the one to dispatch is in the lowest lane of a ballot, and there in
+// the lowest slot.  All control flow is uniform.  Returns the makespan, or -1 where a node was never ready (a cycle) or a
+// start time was infinite.
+//
+// What bounds it is the number of instructions of a round.  So a node has ONE time, the largest finish time of its
+// predecessors and of the nodes dispatched on its devices: once the node is ready that is its true start time, and the heap's
+// key is kept beside it for the nodes of shared position alone.  A dispatched node brings the lanes whose time it raises and
+// the lanes of its successors as masks (three nodes to a lane: the latter from LDS, the former by their reservations), and
+// the slots of a lane are merged in the waits of the reduction.  Everything that is about ties stands behind one branch.
 template <int NS, int TR>
 __device__ __attribute__((noinline)) double kp_lanes(uint64_t blob, uint64_t ovl_, uint64_t dpne_, const KpLds M, unsigned long long* stamp) {
   const int lane = (int)__lane_id();
   const KpClass T{kp_scalar64(blob)};
   const uint64_t ovl = kp_scalar64(ovl_), dpne = kp_scalar64(dpne_);
   const int n = (int)kp_scalar(T.hdr()->n_nodes);
-
+  constexpr bool WIDE = NS > 2;   // the lanes of a node's successors are kept in LDS
   // ---- the nodes in their lanes
-  double key[NS], dvc[NS], dur[NS];
-  uint32_t deg[NS], res[NS], sx01[NS], sx23[NS], tie[NS], pos[NS], mate_lo[NS], mate_hi[NS];   // res: kp_reserved | place << 16 | more than four successors << 31
-  mask64 rm[NS], shm[NS];                                            // waiting nodes; nodes of shared position
+  double e[NS], dur[NS], key[NS], start[NS];
+  uint32_t deg[NS], node[NS], tie[NS], pos[NS], seq[NS], res[NS];   // res: kp_reserved | q << 16
+  uint32_t mate_lo[NS], mate_hi[NS];                     // the other lanes that hold nodes of equal position
+  KpMask raise_lane[NS][NS], succ_lane[NS][NS];          // by slot: the lanes of the nodes whose time this one raises, and of its successors and itself
+  mask64 shm[NS];                                        // nodes of shared position
   mask64 any_shared = 0ull;
+  bool order_pushes = false;                             // nodes of equal position may be successors of one node
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    const int x = s * 64 + lane;
+    const int x = lane * NS + s;
     const bool ok = x < n;
     const uint32_t at = M.at[ok ? x : 0];
     const LevelRec r = M.rec[kp_at_place(at)];
-    sx01[s] = (uint32_t)M.q[r.succ[0]] | ((uint32_t)M.q[r.succ[1]] << 16);
-    sx23[s] = (uint32_t)M.q[r.succ[2]] | ((uint32_t)M.q[r.succ[3]] << 16);
-    res[s] = ok ? (kp_reserved(r.blocked, r.cond, ovl, dpne) | (kp_at_place(at) << 16) | (r.n_succ > 4 ? 0x80000000u : 0u)) : 0u;
-    deg[s] = ok ? (uint32_t)r.indeg : 0xFFFFu;
+    uint32_t before[4];
+    auto succeeds = [&](uint32_t q) {   // (no successor: all ones)
+      const KpMask b = kp_bit(ok ? q / NS : 64u);
+#pragma unroll
+      for (int t = 0; t < NS; ++t) {
+        succ_lane[s][t].lo |= q % NS == (uint32_t)t ? b.lo : 0u;
+        succ_lane[s][t].hi |= q % NS == (uint32_t)t ? b.hi : 0u;
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < NS; ++t) succ_lane[s][t] = KpMask{0u, 0u};
+    succeeds((uint32_t)x);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t q = M.q[r.succ[j]];
+      succeeds(q);
+      before[j] = j < r.n_succ ? kp_at_pos(M.at[q]) : 0xFFFFFFFFu - (uint32_t)j;
+#pragma unroll
+      for (int i = 0; i < j; ++i) order_pushes = order_pushes || __ballot(ok && before[i] == before[j]) != 0ull;
+    }
+    if (__builtin_expect(__ballot(ok && r.n_succ > 4) != 0ull, 0)) {
+      order_pushes = true;
+      const KP_CONST ClassHdr* h = T.hdr();
+      const uint32_t sb = T.at<uint16_t>(h->off_node + r.node * 8u)[0];
+      for (uint32_t j = 4; ok && j < r.n_succ; ++j) succeeds(M.q[T.at<uint16_t>(h->off_place)[T.at<uint16_t>(h->off_succ)[sb + j]]]);
+    }
+    res[s] = ok ? kp_reserved(r.blocked, r.cond, ovl, dpne) | ((uint32_t)x << 16) : 0u;
+    node[s] = r.node;
+    deg[s] = ok ? (uint32_t)r.indeg : 0xFFFFFFFFu;
     dur[s] = M.dur[r.slot];
-    key[s] = 0.0;
-    dvc[s] = 0.0;
-    tie[s] = 0u;
+    e[s] = start[s] = 0.0;
+    key[s] = ok && r.indeg == 0 ? 0.0 : __builtin_inf();
+    tie[s] = seq[s] = 0u;
     pos[s] = kp_at_pos(at);
-    rm[s] = __ballot(ok && r.indeg == 0);
     shm[s] = __ballot(ok && (at & KP_AT_SHARED));
-    {   // the lanes of the other nodes of equal position (all lanes, its own too, where they lie in two slots)
-      const int lo = (int)kp_at_pos(at) - s * 64, hi = lo + (int)kp_at_size(at);
-      mask64 g = ~0ull;
-      if (lo >= 0 && hi <= 64) g = ((hi - lo > 63 ? ~0ull : (1ull << (hi - lo)) - 1ull) << lo) & ~(1ull << lane);
-      mate_lo[s] = (uint32_t)g;
-      mate_hi[s] = (uint32_t)(g >> 32);
+    {
+      const uint32_t p0 = kp_at_pos(at), p1 = p0 + kp_at_size(at);
+      const KpMask g = kp_lanes_from_to(p0 / NS, (p1 > p0 ? p1 - 1u : p0) / NS), own = kp_bit((uint32_t)lane);
+      mate_lo[s] = g.lo & ~own.lo;
+      mate_hi[s] = g.hi & ~own.hi;
     }
     any_shared |= shm[s];
   }
+  KP_LDS mask64* const row = (KP_LDS mask64*)M.rec;   // (WIDE; over the records and the ranks) by position: the lanes of the successors and the node's own
+  if constexpr (WIDE) {
+    kp_sync();
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      if (lane * NS + s < n) {
+#pragma unroll
+        for (int t = 0; t < NS; ++t) row[(lane * NS + s) * NS + t] = (mask64)succ_lane[s][t].lo | ((mask64)succ_lane[s][t].hi << 32);
+      }
+    kp_sync();
+  } else {
+#pragma unroll
+    for (int t = 0; t < NS; ++t) {   // nodes that conflict: this one's reserved vertices among those that overlap the other's
+#pragma unroll
+      for (int s = 0; s < NS; ++s) raise_lane[s][t] = succ_lane[s][t];   // (the node itself among them: it has devices of its own)
+#pragma unroll
+      for (int v = 0; v < RPEG_MAX_V; ++v) {
+        const mask64 overlaps = __ballot((res[t] >> (8 + v)) & 1u);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          raise_lane[s][t].lo |= (res[s] >> v) & 1u ? (uint32_t)overlaps : 0u;
+          raise_lane[s][t].hi |= (res[s] >> v) & 1u ? (uint32_t)(overlaps >> 32) : 0u;
+        }
+      }
+    }
+  }
+  mask64 twins = 0ull;   // lanes two of whose slots hold nodes of equal position (neighbours, then)
+#pragma unroll
+  for (int s = 0; s + 1 < NS; ++s) twins |= __ballot(pos[s] == pos[s + 1]);
   // ties of the nodes without predecessors, in the reference's node order
-  uint32_t ctr = 0;
+  uint32_t ctr = 0;   // (ties: a push's number << 8 | order among those of one push-back)
   if (any_shared) {
     const KP_CONST ClassHdr* h = T.hdr();
     for (uint32_t i = 0; i < h->n_init; ++i) {
-      const int x = (int)kp_scalar(M.q[T.at<uint16_t>(h->off_place)[T.at<uint16_t>(h->off_init)[i]]]);
+      const uint32_t x = kp_scalar(M.q[T.at<uint16_t>(h->off_place)[T.at<uint16_t>(h->off_init)[i]]]);
 #pragma unroll
-      for (int s = 0; s < NS; ++s) tie[s] = s == (x >> 6) && lane == (x & 63) ? ctr : tie[s];
-      ++ctr;
+      for (int s = 0; s < NS; ++s) tie[s] = (uint32_t)s == x % NS && (uint32_t)lane == x / NS ? ctr : tie[s];
+      ctr += 256u;
     }
   }
   if (stamp) stamp[4] = wall_clock64();
 
-  // ---- list scheduling (scheduler.py:399-546): one node per round.  The rare cases are kept out of line: a branch that
-  // falls through costs three instructions, a taken one six.
-  double makespan = 0.0;
+  // ---- list scheduling (scheduler.py:399-546): one node per round.  A node waits while it has no predecessors left
+  // (deg 0); dispatched, it is its own successor (deg -1)
   uint32_t ghi = 0u;
-  for (int done = 0; done < n; ++done) {
-    double e[NS];
+  mask64 last_m = 0ull, last_pick[NS];   // m and pick of the round before
+#pragma unroll
+  for (int s = 0; s < NS; ++s) last_pick[s] = 0ull;
+  for (int round = 0; round < n; ++round) {
+    // a lane's candidate: its waiting node of smallest start time, of several the one in the lowest slot.  Non-negative
+    // doubles order like their bit patterns: the smallest high word first, then -- where the candidates that have it
+    // differ in the low word, which is rare: they were released by one finish, or wait for one device -- that
+    constexpr int NM = WIDE ? 4 : 3 + 4 * NS;
+    uint32_t mine[NM], w[NM];   // of the lane's candidate: low word of its start time, finish time, lanes of its successors, lanes it raises (WIDE: its reservations and position); of the one to dispatch
+    auto words = [&](int s, uint32_t (&x)[NM]) {
+      const double f = e[s] + dur[s];
+      x[0] = (uint32_t)__double2loint(e[s]);
+      x[1] = (uint32_t)__double2loint(f);
+      x[2] = (uint32_t)__double2hiint(f);
+      if constexpr (WIDE) x[3] = res[s];
+      else
+#pragma unroll
+      for (int t = 0; t < NS; ++t) {
+        x[3 + 2 * t] = succ_lane[s][t].lo;
+        x[4 + 2 * t] = succ_lane[s][t].hi;
+        x[3 + 2 * NS + 2 * t] = raise_lane[s][t].lo;
+        x[4 + 2 * NS + 2 * t] = raise_lane[s][t].hi;
+      }
+    };
+    mask64 rm[NS], ls[NS], pick[NS];
     uint32_t eh[NS], h = 0xFFFFFFFFu;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      e[s] = kp_vmax(key[s], dvc[s]);
+      rm[s] = __ballot(deg[s] == 0u);
       eh[s] = kp_sel(rm[s], (uint32_t)__double2hiint(e[s]), 0xFFFFFFFFu);
       h = eh[s] < h ? eh[s] : h;
     }
-    // non-negative doubles order like their bit patterns: the smallest high word, then -- where the waiting nodes that
-    // have it differ in the low word, which is rare: they were released by one finish, or wait for one device -- that
-    ghi = kp_wave_umin(h);
-    mask64 m[NS];
+    KpHead head;
+    if constexpr (NS == 1) {
+      double f;
+      pick[0] = ~0ull;
+      words(0, mine);
+      head = kp_head(h, e[0], dur[0], mine, &f, w);
+      mine[1] = (uint32_t)__double2loint(f);
+      mine[2] = (uint32_t)__double2hiint(f);
+    } else if constexpr (NS == 2) {
+      pick[0] = rm[0] & (__ballot(e[0] <= e[1]) | ~rm[1]);
+      pick[1] = ~pick[0];
+      uint32_t a[NM], b[NM];
+      words(0, a);
+      words(1, b);
+      head = kp_head(h, pick[0], a, b, mine, w);
+    } else {
+      double em = e[NS - 1];
+      mask64 some = rm[NS - 1];
+      words(NS - 1, mine);
+      pick[NS - 1] = ~0ull;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) m[s] = __ballot(eh[s] == ghi);
-    // (a register of the winner's slot: in a lane of m[0] slot 0's, else in a lane of m[1] slot 1's, ...)
-    auto of_slot = [&](auto&& get) {
-      uint32_t v = get(NS - 1);
+      for (int s = NS - 2; s >= 0; --s) {
+        const mask64 p = rm[s] & (__ballot(e[s] <= em) | ~some);
+        some |= rm[s];
+        if (s > 0) em = kp_sel(p, e[s], em);
+        uint32_t a[NM];
+        words(s, a);
 #pragma unroll
-      for (int s = NS - 2; s >= 0; --s) v = kp_sel(m[s], get(s), v);
-      return v;
-    };
-    mask64 mw = m[NS - 1];
+        for (int k = 0; k < NM; ++k) mine[k] = kp_sel(p, a[k], mine[k]);
 #pragma unroll
-    for (int s = NS - 2; s >= 0; --s) mw = m[s] ? m[s] : mw;
-    int wl = __builtin_ctzll(mw);
-    uint32_t glo;
-    {
-      const uint32_t lo0 = (uint32_t)__builtin_amdgcn_readlane((int)of_slot([&](int s) { return (uint32_t)__double2loint(e[s]); }), wl);
-      mask64 differ = 0ull;
-      glo = lo0;
-#pragma unroll
-      for (int s = 0; s < NS; ++s) differ |= m[s] & __ballot((uint32_t)__double2loint(e[s]) != lo0);
-      if (__builtin_expect(differ != 0ull, 0)) {
-        uint32_t l = 0xFFFFFFFFu;
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-          const uint32_t x = kp_sel(m[s], (uint32_t)__double2loint(e[s]), 0xFFFFFFFFu);
-          l = x < l ? x : l;
-        }
-        glo = kp_wave_umin(l);
-#pragma unroll
-        for (int s = 0; s < NS; ++s) m[s] &= __ballot((uint32_t)__double2loint(e[s]) == glo);
-        mw = m[NS - 1];
-#pragma unroll
-        for (int s = NS - 2; s >= 0; --s) mw = m[s] ? m[s] : mw;
-        wl = __builtin_ctzll(mw);
+        for (int t = s + 1; t < NS; ++t) pick[t] &= ~p;
+        pick[s] = p;
       }
+      head = kp_head(h, mine, w);
     }
-
-    // ---- ties among waiting nodes of equal position, and the push-backs they depend on
-    mask64 ls[NS], live_shared = 0ull;
+    ghi = head.ghi;
+    mask64 rare = head.differ;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       ls[s] = rm[s] & shm[s];
-      live_shared |= ls[s];
+      rare |= ls[s];
     }
-    if (__builtin_expect(live_shared != 0ull, 0)) {
-      const double gk = __hiloint2double((int)ghi, (int)glo);
-      // back: stale entries the heap may have met on the way (a stale entry of key gk only if its position and tie are
-      // below the dispatched one's); rivals: entries of shared position that could be dispatched now
-      mask64 back[NS], any_back = 0ull;
-      int n_rivals = 0;
+    mask64 m = head.m;
+    if (__builtin_expect(rare != 0ull, 0)) {
+      // Nodes of shared position wait, or the candidates differ.  A node the last round made ready is pushed: its key is its
+      // time now (the key of those that have not been ready yet is infinite), its tie the number of the push
+      mask64 fresh[NS];
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
-        back[s] = ls[s] & __ballot(dvc[s] > key[s]) & __ballot(key[s] <= gk);
-        any_back |= back[s];
-        n_rivals += __builtin_popcountll(m[s] & ls[s]);
+        const double ew = __hiloint2double((int)eh[s], __double2loint(e[s]));   // (no number where the node does not wait)
+        fresh[s] = __ballot(key[s] > ew);
+        tie[s] = kp_sel(fresh[s], ctr, tie[s]);
+        key[s] = kp_vmin(key[s], ew);
       }
-      if (any_back != 0ull || n_rivals > 1) {
-        int ws = 0;
+      ctr += 256u;
+      // (x[s]: met[s] the lanes of those that meet another one, of equal position, among all of them, and perhaps of others)
+      auto meet = [&](const mask64 (&x)[NS], mask64 (&met)[NS]) {
+        mask64 all = 0ull;
 #pragma unroll
-        for (int s = NS - 1; s >= 0; --s)
-          if (m[s]) ws = s;
-        uint32_t pd = (uint32_t)__builtin_amdgcn_readlane((int)of_slot([&](int s) { return pos[s]; }), wl);
-        if (n_rivals > 1) {
+        for (int s = 0; s < NS; ++s) all |= x[s];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) met[s] = x[s] & __ballot((((uint32_t)all & mate_lo[s]) | ((uint32_t)(all >> 32) & mate_hi[s])) != 0u);
+        if (NS > 1) {   // (within a lane)
+          mask64 one = 0ull, two = 0ull;
+#pragma unroll
+          for (int s = 0; s < NS; ++s) {
+            two |= one & x[s];
+            one |= x[s];
+          }
+#pragma unroll
+          for (int s = 0; s < NS; ++s) met[s] |= x[s] & two & twins;
+        }
+      };
+      if (__builtin_expect(order_pushes, 0)) {   // nodes of equal position among one node's successors: in their order
+        mask64 x[NS], met[NS], any = 0ull;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) x[s] = fresh[s] & shm[s];
+        meet(x, met);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) any |= met[s];
+        if (any != 0ull) {
+          const int ll = __builtin_ctzll(last_m);
+          uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)node[0], ll);
+#pragma unroll
+          for (int s = 1; s < NS; ++s) {
+            const uint32_t y = (uint32_t)__builtin_amdgcn_readlane((int)node[s], ll);
+            v = (last_pick[s] >> ll) & 1ull ? y : v;
+          }
+          kp_more_places(T, v, 0u, [&](uint32_t p) {
+            const uint32_t q = kp_scalar(M.q[p]);
+#pragma unroll
+            for (int s = 0; s < NS; ++s) tie[s] = kp_sel(q % NS == (uint32_t)s ? x[s] & (1ull << (q / NS & 63u)) : 0ull, ctr, tie[s]);
+            ctr += 256u;
+          });
+        }
+      }
+      // back: stale entries -- their devices are busy beyond their key -- the heap may meet on the way; rivals: the lanes of
+      // entries of the dispatched one's position that could be dispatched as well
+      double gk = __hiloint2double((int)ghi, (int)w[0]);
+      int wl = __builtin_ctzll(m);
+      const mask64 bit = 1ull << wl;
+      uint32_t w_lo = mate_lo[NS - 1], w_hi = mate_hi[NS - 1];
+#pragma unroll
+      for (int s = NS - 2; s >= 0; --s) {
+        w_lo = kp_sel(pick[s], mate_lo[s], w_lo);
+        w_hi = kp_sel(pick[s], mate_hi[s], w_hi);
+      }
+      mask64 rivals = m & ((mask64)(uint32_t)__builtin_amdgcn_readlane((int)w_lo, wl) | ((mask64)(uint32_t)__builtin_amdgcn_readlane((int)w_hi, wl) << 32));
+      if constexpr (NS == 2) rivals |= bit & twins & ls[0] & ls[1] & __ballot(e[0] == e[1]);
+      else if constexpr (NS > 2) {   // (two nodes of its lane wait, and nodes of its lane share a position)
+        mask64 one = 0ull;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          rivals |= bit & twins & one & ls[s];
+          one |= ls[s];
+        }
+      }
+      mask64 stale[NS], back[NS], any_back = 0ull;
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        stale[s] = ls[s] & __ballot(e[s] > key[s]);
+        back[s] = stale[s] & __ballot(key[s] <= gk) & ~(pick[s] & bit);
+        any_back |= back[s];
+      }
+      if ((head.differ | rivals | any_back) != 0ull) {
+        mask64 d_stale = 0ull;
+        if ((head.differ | rivals) != 0ull) {
+          if (head.differ) {
+            const uint32_t glo = kp_wave_umin(kp_sel(m, mine[0], 0xFFFFFFFFu));
+            wl = __builtin_ctzll(m & __ballot(mine[0] == glo));
+            gk = __hiloint2double((int)ghi, (int)glo);
+          }
+          int ws = 0;
+#pragma unroll
+          for (int s = NS - 1; s > 0; --s) ws = (pick[s] >> wl) & 1ull ? s : ws;
+          uint32_t pd = (uint32_t)__builtin_amdgcn_readlane((int)pos[0], wl);
+#pragma unroll
+          for (int s = 1; s < NS; ++s) {
+            const uint32_t x = (uint32_t)__builtin_amdgcn_readlane((int)pos[s], wl);
+            pd = s == ws ? x : pd;
+          }
           mask64 c[NS], current[NS], any_current = 0ull;
           int members = 0;
 #pragma unroll
           for (int s = 0; s < NS; ++s) {
-            c[s] = m[s] & __ballot(pos[s] == pd);
+            back[s] = stale[s] & __ballot(key[s] <= gk);
+            c[s] = rm[s] & __ballot(e[s] == gk) & __ballot(pos[s] == pd);
             members += __builtin_popcountll(c[s]);
             current[s] = c[s] & ~back[s];   // (of the entries of true start time gk the stale ones are those of a smaller key)
             any_current |= current[s];
@@ -476,184 +796,162 @@ __device__ __attribute__((noinline)) double kp_lanes(uint64_t blob, uint64_t ovl
                 if (first || kj < bk || (kj == bk && tj < bt)) { first = false; bk = kj; bt = tj; ws = s; wl = j; }
               }
             }
-#pragma unroll
-            for (int s = 0; s < NS; ++s) m[s] = s == ws ? 1ull << wl : 0ull;
+            ws = (int)kp_scalar((uint32_t)ws);
+            wl = (int)kp_scalar((uint32_t)wl);
           }
+          m = 1ull << wl;
+          any_back = 0ull;
+#pragma unroll
+          for (int s = 0; s < NS; ++s) {   // (its lane may have had another candidate)
+            const mask64 here = s == ws ? m : 0ull;
+            d_stale |= back[s] & here;
+            back[s] &= ~here;
+            any_back |= back[s];
+            if (NS > 1) {
+              uint32_t a[NM];
+              words(s, a);
+              pick[s] = (pick[s] & ~m) | here;
+#pragma unroll
+              for (int k = 1; k < NM; ++k) mine[k] = kp_sel(here, a[k], mine[k]);
+            }
+          }
+#pragma unroll
+          for (int k = 1; k < NM; ++k) w[k] = (uint32_t)__builtin_amdgcn_readlane((int)mine[k], wl);
+        } else {
+#pragma unroll
+          for (int s = 0; s < NS; ++s) d_stale |= stale[s] & pick[s] & bit;
         }
         mask64 level = 0ull;
-        int members = 0;
-        mask64 d_stale = 0ull;
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {
-          if (s == ws) {
-            d_stale = (back[s] >> wl) & 1ull;
-            back[s] &= ~(1ull << wl);
-          }
-          level |= back[s] & __ballot(key[s] == gk);
-        }
+        for (int s = 0; s < NS; ++s) level |= back[s] & __ballot(key[s] == gk);
         if (__builtin_expect(level != 0ull, 0)) {
-          // (a stale entry that is dispatched was pushed back with a fresh tie)
-          const uint32_t td = d_stale ? 0xFFFFFFFFu : (uint32_t)__builtin_amdgcn_readlane((int)of_slot([&](int s) { return tie[s]; }), wl);
+          // a stale entry of key gk is met only if its position and tie are below the dispatched one's (of which, if that was
+          // stale, the tie is a fresh one)
+          uint32_t pd = (uint32_t)__builtin_amdgcn_readlane((int)pos[0], wl), td = (uint32_t)__builtin_amdgcn_readlane((int)tie[0], wl);
 #pragma unroll
-          for (int s = 0; s < NS; ++s)
-            back[s] &= __ballot(key[s] < gk) | __ballot(pos[s] < pd) | (__ballot(pos[s] == pd) & __ballot(tie[s] < td));
-        }
-#pragma unroll
-        for (int s = 0; s < NS; ++s) members += __builtin_popcountll(back[s]);
-        if (members) {
-          // fresh ties; only among entries of equal position is their order ever looked at
-          uint32_t fresh[NS];
-          mask64 mated[NS], any_mated = 0ull;
+          for (int s = 1; s < NS; ++s) {
+            const uint32_t p = (uint32_t)__builtin_amdgcn_readlane((int)pos[s], wl), t = (uint32_t)__builtin_amdgcn_readlane((int)tie[s], wl);
+            const bool here = (pick[s] >> wl) & 1ull;
+            pd = here ? p : pd;
+            td = here ? t : td;
+          }
+          td = d_stale ? 0xFFFFFFFFu : td;
+          any_back = 0ull;
 #pragma unroll
           for (int s = 0; s < NS; ++s) {
-            fresh[s] = ctr;
-            mated[s] = back[s] & __ballot((((uint32_t)back[s] & mate_lo[s]) | ((uint32_t)(back[s] >> 32) & mate_hi[s])) != 0u);
-            any_mated |= mated[s];
+            back[s] &= __ballot(key[s] < gk) | __ballot(pos[s] < pd) | (__ballot(pos[s] == pd) & __ballot(tie[s] < td));
+            any_back |= back[s];
           }
-          if (any_mated) {
+        }
+        if (any_back != 0ull) {
+          // fresh ties; only among entries of equal position is their order ever looked at.  They are pushed back in the
+          // order of their old keys and ties: entries that were pushed back together the last time, and have equal keys
+          // since, keep theirs (the low byte of the ties of one push-back tells it)
+          uint32_t t2[NS];
+          mask64 met[NS], any_met = 0ull, apart = 0ull;
+          meet(back, met);
 #pragma unroll
-            for (int s = 0; s < NS; ++s) {
-              mask64 todo = mated[s];
-              while (todo) {
-                const int j = __builtin_ctzll(todo);
-                todo &= todo - 1ull;
-                const double kj = kp_readlane(key[s], j);
-                const uint32_t tj = (uint32_t)__builtin_amdgcn_readlane((int)tie[s], j);
+          for (int s = 0; s < NS; ++s) {
+            any_met |= met[s];
+            t2[s] = ctr | (tie[s] & 0xFFu);
+          }
+          if (any_met != 0ull) {
+            double k1 = 0.0;
+            uint32_t t1 = 0u;
 #pragma unroll
-                for (int t = 0; t < NS; ++t) fresh[t] += ((kj < key[t]) | ((kj == key[t]) & (tj < tie[t]))) ? 1u : 0u;
+            for (int s = NS - 1; s >= 0; --s)
+              if (met[s] != 0ull) {
+                const int j = __builtin_ctzll(met[s]);
+                k1 = kp_readlane(key[s], j);
+                t1 = (uint32_t)__builtin_amdgcn_readlane((int)tie[s], j);
+              }
+#pragma unroll
+            for (int s = 0; s < NS; ++s) apart |= met[s] & (__ballot(key[s] != k1) | __ballot(((tie[s] ^ t1) >> 8) != 0u));
+            if (apart != 0ull) {
+#pragma unroll
+              for (int s = 0; s < NS; ++s) t2[s] = ctr;
+#pragma unroll
+              for (int s = 0; s < NS; ++s) {
+                mask64 todo = met[s];
+                while (todo) {
+                  const int j = __builtin_ctzll(todo);
+                  todo &= todo - 1ull;
+                  const double kj = kp_readlane(key[s], j);
+                  const uint32_t tj = (uint32_t)__builtin_amdgcn_readlane((int)tie[s], j);
+#pragma unroll
+                  for (int t = 0; t < NS; ++t) t2[t] += ((kj < key[t]) | ((kj == key[t]) & (tj < tie[t]))) ? 1u : 0u;
+                }
               }
             }
           }
 #pragma unroll
           for (int s = 0; s < NS; ++s) {
-            key[s] = kp_sel(back[s], dvc[s], key[s]);
-            tie[s] = kp_sel(back[s], fresh[s], tie[s]);
+            key[s] = kp_sel(kp_scalar64(back[s]), e[s], key[s]);
+            tie[s] = kp_sel(kp_scalar64(back[s]), t2[s], tie[s]);
           }
-          ctr += (uint32_t)members;
+          ctr += 256u;
         }
       }
     }
 
     // ---- dispatch
-    double f[NS];
 #pragma unroll
-    for (int s = 0; s < NS; ++s) f[s] = e[s] + dur[s];
-    const uint32_t flo = of_slot([&](int s) { return (uint32_t)__double2loint(f[s]); }), fhi = of_slot([&](int s) { return (uint32_t)__double2hiint(f[s]); });
-    const uint32_t info = (uint32_t)__builtin_amdgcn_readlane((int)of_slot([&](int s) { return res[s]; }), wl);
-    const uint32_t s01 = (uint32_t)__builtin_amdgcn_readlane((int)of_slot([&](int s) { return sx01[s]; }), wl);
-    const uint32_t s23 = (uint32_t)__builtin_amdgcn_readlane((int)of_slot([&](int s) { return sx23[s]; }), wl);
-    const double fin = __hiloint2double(__builtin_amdgcn_readlane((int)fhi, wl), __builtin_amdgcn_readlane((int)flo, wl));
-    {
-      const mask64 bit = 1ull << wl;
-      mask64 left = bit;   // (of the slots that hold candidates, the first is the winner's)
+    for (int k = 1; k < NM; ++k) asm("" : "+s"(w[k]));   // (they are in scalar registers, whichever way they came)
+    const double fin = __hiloint2double((int)w[2], (int)w[1]);
+    last_m = m;
+    mask64 sm[NS], raised[NS];
+    if constexpr (WIDE) {
+      const KP_LDS mask64* const r = row + (w[3] >> 16) * NS;
+      mask64 x[NS];
+#pragma unroll
+      for (int s = 0; s < NS; ++s) x[s] = r[s];
+      const uint32_t reserved = (w[3] & 0x3Fu) << 8;
+#pragma unroll
+      for (int s = 0; s < NS; ++s) raised[s] = __ballot((res[s] & reserved) != 0u);
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
-        rm[s] &= ~(s + 1 < NS && !m[s] ? 0ull : left);
-        left = m[s] ? 0ull : left;
+        sm[s] = kp_scalar64(x[s]);
+        raised[s] |= sm[s];
       }
-      if (TR) {   // start and finish by position
-        if (kp_in(bit)) {
-          uint32_t q = (uint32_t)((NS - 1) * 64 + lane);
+    } else {
 #pragma unroll
-          for (int s = NS - 2; s >= 0; --s) q = kp_sel(m[s], (uint32_t)(s * 64 + lane), q);
-          M.rank[q] = __hiloint2double((int)fhi, (int)flo);
-          M.rk[q] = __hiloint2double((int)ghi, (int)glo);
-          if (TR == KP_TIMES_ORDER) M.order[done] = (uint16_t)((info >> 16) & 0x7FFFu);
-        }
+      for (int s = 0; s < NS; ++s) {
+        sm[s] = (mask64)w[3 + 2 * s] | ((mask64)w[4 + 2 * s] << 32);
+        raised[s] = (mask64)w[3 + 2 * NS + 2 * s] | ((mask64)w[4 + 2 * NS + 2 * s] << 32);
       }
     }
-    makespan = kp_vmax_s(makespan, fin);
-    const uint32_t reserved = (info & 0xFFu) << 8;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      const double r = kp_vmax_s(dvc[s], fin);
-      dvc[s] = (res[s] & reserved) ? r : dvc[s];
-    }
-    // successors; a node whose last predecessor this was becomes ready.  (What waits for the devices of a ready node is
-    // in its availability: only a node of shared position needs it in its key, and its place in the order of pushes.)
-    if (__builtin_expect((s01 & 0xFFFFu) != 0xFFFFu, 1)) {
-      mask64 sm[NS];
-#pragma unroll
-      for (int s = 0; s < NS; ++s) sm[s] = 0ull;
-      auto mark = [&](const uint32_t x) {
-        const mask64 bit = 1ull << (x & 63u);
-#pragma unroll
-        for (int s = 0; s < NS; ++s) sm[s] |= NS == 1 || s == (int)(x >> 6) ? bit : 0ull;
-      };
-      mark(s01 & 0xFFFFu);
-      if (__builtin_expect((s01 >> 16) != 0xFFFFu, 0)) {
-        mark(s01 >> 16);
-        if ((s23 & 0xFFFFu) != 0xFFFFu) {
-          mark(s23 & 0xFFFFu);
-          if ((s23 >> 16) != 0xFFFFu) mark(s23 >> 16);
-        }
-        if (__builtin_expect((info & 0x80000000u) != 0u, 0)) {   // more than four successors
-          kp_more(T, M, (info >> 16) & 0x7FFFu, mark);
-        }
+      last_pick[s] = pick[s];
+      if (TR) {   // (its finish time is the sum, again)
+        const mask64 won = pick[s] & m & (0ull - m);
+        start[s] = kp_sel(won, e[s], start[s]);
+        if (TR == KP_TIMES_ORDER) seq[s] = kp_sel(won, (uint32_t)round, seq[s]);
       }
-      mask64 now[NS], now_shared = 0ull;
-#pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        const double k = kp_vmax_s(key[s], fin);
-        key[s] = kp_sel(sm[s], k, key[s]);
-        deg[s] -= kp_in(sm[s]) ? 1u : 0u;
-        now[s] = sm[s] & __ballot(deg[s] == 0u);
-        rm[s] |= now[s];
-        now_shared |= now[s] & shm[s];
-      }
-      if (__builtin_expect(now_shared != 0ull, 0)) {
-        uint32_t j = 0u;
-        auto push = [&](const uint32_t x) {
-          const mask64 bit = 1ull << (x & 63u);
-#pragma unroll
-          for (int s = 0; s < NS; ++s)
-            if (NS == 1 || s == (int)(x >> 6)) {
-              const mask64 b = bit & now[s];
-              key[s] = kp_sel(b, kp_vmax(key[s], dvc[s]), key[s]);
-              tie[s] = kp_sel(b, ctr + j, tie[s]);
-            }
-          ++j;
-        };
-        push(s01 & 0xFFFFu);
-        if ((s01 >> 16) != 0xFFFFu) {
-          push(s01 >> 16);
-          if ((s23 & 0xFFFFu) != 0xFFFFu) {
-            push(s23 & 0xFFFFu);
-            if ((s23 >> 16) != 0xFFFFu) push(s23 >> 16);
-          }
-        }
-        if (info & 0x80000000u) {
-          kp_more(T, M, (info >> 16) & 0x7FFFu, push);
-        }
-        ctr += j;
-      }
+      deg[s] = WIDE ? deg[s] - (kp_in(sm[s]) ? 1u : 0u) : kp_dec(sm[s], deg[s]);
+      e[s] = kp_sel(raised[s], kp_vmax_s(e[s], fin), e[s]);
     }
   }
-  // (nothing was ready -- a cycle, which the class lowering flags -- or a start time was infinite: it stays so to the end)
-  if (n > 0 && ghi >= 0x7FF00000u) return -1.0;
-  if (TR) {   // from position to node; the dispatch order so far names places
-    double tf[NS], ts[NS];
-    uint32_t node[NS];
-    kp_sync();
+  mask64 never = 0ull;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const int x = s * 64 + lane < n ? s * 64 + lane : 0;
-      tf[s] = M.rank[x];
-      ts[s] = M.rk[x];
-      node[s] = (uint32_t)M.rec[(res[s] >> 16) & 0x7FFFu].node;
-    }
+  for (int s = 0; s < NS; ++s) never |= __ballot(deg[s] != 0xFFFFFFFFu);
+  if (never != 0ull || ghi >= 0x7FF00000u) return -1.0;   // (the smallest start time only grows)
+  // every node raised its own time to its finish time, with the others on its devices: the makespan is the largest
+  double last = e[0];
+#pragma unroll
+  for (int s = 1; s < NS; ++s) last = kp_vmax(last, e[s]);
+  if (TR) {   // from position to node
     kp_sync();
 #pragma unroll
     for (int s = 0; s < NS; ++s)
-      if (s * 64 + lane < n) {
-        M.rank[node[s]] = tf[s];
-        M.rk[node[s]] = ts[s];
+      if (lane * NS + s < n) {
+        M.rank[node[s]] = start[s] + dur[s];
+        M.rk[node[s]] = start[s];
+        if (TR == KP_TIMES_ORDER) M.order[seq[s]] = (uint16_t)node[s];
       }
-    if (TR == KP_TIMES_ORDER)
-      for (int k = lane; k < n; k += KE_WAVE) M.order[k] = M.rec[M.order[k]].node;
     kp_sync();
   }
-  return makespan;
+  return kp_wave_reduce(last, KpMax());
 }
 
 
@@ -706,7 +1004,7 @@ __device__ __attribute__((noinline)) double kp_list(uint64_t blob, uint64_t ovl_
     }
   }
   kp_sync();
-  double key = inf, dvc = 0.0, dur = 0.0, dvm = 0.0;
+  double e = inf, key = inf, dur = 0.0, dvm = 0.0;   // e: the node's true start time (infinite: none); key: the heap's, where its position is shared
   uint32_t word = NONE, res = 0u, tie = 0u, ctr = 0u, mate_lo = 0u, mate_hi = 0u;
   // the lanes whose node shares the position of one that has just come to lane b: each other's mates from now on (of a
   // lane that has been given to another node since, a bit may be left standing: it costs time, no more)
@@ -724,7 +1022,7 @@ __device__ __attribute__((noinline)) double kp_list(uint64_t blob, uint64_t ovl_
     const uint32_t p = T.at<uint16_t>(h->off_place)[T.at<uint16_t>(h->off_init)[ok ? lane : 0]];
     const KpState st = state[p];
     if (ok) {
-      key = 0.0;
+      e = key = 0.0;
       dur = M.dur[(st.left >> 14) & 0xFFu];
       word = st.word;
       res = st.left;
@@ -737,10 +1035,8 @@ __device__ __attribute__((noinline)) double kp_list(uint64_t blob, uint64_t ovl_
   }
   if (stamp) stamp[4] = wall_clock64();
 
-  double makespan = 0.0;
   uint32_t ghi = 0u;
   for (int done = 0; done < n; ++done) {
-    const double e = kp_vmax(key, dvc);
     const uint32_t eh = (uint32_t)__double2hiint(e), el = (uint32_t)__double2loint(e);
     ghi = kp_wave_umin(eh);
     mask64 m = __ballot(eh == ghi);
@@ -759,7 +1055,7 @@ __device__ __attribute__((noinline)) double kp_list(uint64_t blob, uint64_t ovl_
     const mask64 ls = shl & ~free_lanes;
     if (__builtin_expect(ls != 0ull, 0)) {
       const double gk = __hiloint2double((int)ghi, (int)glo);
-      mask64 back = ls & __ballot(dvc > key) & __ballot(key <= gk);
+      mask64 back = ls & __ballot(e > key) & __ballot(key <= gk);
       const mask64 rivals = m & ls;
       if (back != 0ull || (rivals & (rivals - 1ull)) != 0ull) {
         const uint32_t pd = (uint32_t)__builtin_amdgcn_readlane((int)(word >> 16), wl), pos = word >> 16;
@@ -795,7 +1091,7 @@ __device__ __attribute__((noinline)) double kp_list(uint64_t blob, uint64_t ovl_
             const uint32_t tj = (uint32_t)__builtin_amdgcn_readlane((int)tie, j);
             fresh += ((kj < key) | ((kj == key) & (tj < tie))) ? 1u : 0u;
           }
-          key = kp_sel(back, dvc, key);
+          key = kp_sel(back, e, key);
           tie = kp_sel(back, fresh, tie);
           ctr += (uint32_t)__builtin_popcountll(back);
         }
@@ -811,15 +1107,14 @@ __device__ __attribute__((noinline)) double kp_list(uint64_t blob, uint64_t ovl_
     const bool mine = kp_in(free_lanes) && k < 4u;    // this lane takes the k-th successor
     const uint32_t sw = words[place * 4u + (k & 3u)];
     const double f = e + dur;
-    const double fin = kp_readlane(f, wl);
+    const double fin = kp_settled(kp_readlane(f, wl));
     const uint32_t rd = (uint32_t)__builtin_amdgcn_readlane((int)res, wl);
-    key = kp_sel(bit, inf, key);
+    e = kp_sel(bit, inf, e);
     word = kp_sel(bit, NONE, word);
     shl &= ~bit;
-    makespan = kp_vmax_s(makespan, fin);
     {
-      const double r = kp_vmax_s(dvc, fin), rm = kp_vmax_s(dvm, fin);
-      dvc = (res & ((rd & 0x3F00u) << 14)) ? r : dvc;
+      const double r = kp_vmax_s(e, fin), rm = kp_vmax_s(dvm, fin);
+      e = (res & ((rd & 0x3F00u) << 14)) ? r : e;
       dvm = ((uint32_t)lane & ((rd >> 22) & 0x3Fu)) ? rm : dvm;
     }
     if (TR) {
@@ -844,8 +1139,7 @@ __device__ __attribute__((noinline)) double kp_list(uint64_t blob, uint64_t ovl_
         state[sp].ready = ready;
         state[sp].left = left;
       }
-      key = kp_sel(now, kp_vmax(ready, dv), key);
-      dvc = kp_sel(now, dv, dvc);
+      e = kp_sel(now, kp_vmax(ready, dv), e);
       dur = kp_sel(now, du, dur);
       word = kp_sel(now, st.word, word);
       res = kp_sel(now, left, res);
@@ -853,6 +1147,7 @@ __device__ __attribute__((noinline)) double kp_list(uint64_t blob, uint64_t ovl_
       const mask64 now_shared = now & __ballot((res & 0x80000000u) != 0u);
       if (__builtin_expect(now_shared != 0ull, 0)) {
         shl |= now_shared;
+        key = kp_sel(now, e, key);
         tie = kp_sel(now, ctr + k, tie);
         ctr += 4u;
         for (mask64 todo = now_shared; todo; todo &= todo - 1ull) meet(shl, __builtin_ctzll(todo));
@@ -865,7 +1160,7 @@ __device__ __attribute__((noinline)) double kp_list(uint64_t blob, uint64_t ovl_
         const uint32_t ns = kp_scalar(M.n_succ[place]);
         if (ns > 4u) {
           bool full = false;
-          kp_more_places(T, kp_scalar(M.node[place]), ns, [&](uint32_t p) {
+          kp_more_places(T, kp_scalar(M.node[place]), 4u, [&](uint32_t p) {
             const KpState s2 = state[p];
             const double ready2 = kp_vmax_s(s2.ready, fin);
             const uint32_t left2 = s2.left - 1u;
@@ -877,8 +1172,8 @@ __device__ __attribute__((noinline)) double kp_list(uint64_t blob, uint64_t ovl_
             if ((kp_scalar(left2) & 0xFFu) == 0u) {
               if (!free_lanes) { full = true; return; }
               const mask64 b = free_lanes & (0ull - free_lanes);
-              key = kp_sel(b, kp_vmax(ready2, dv2), key);
-              dvc = kp_sel(b, dv2, dvc);
+              e = kp_sel(b, kp_vmax(ready2, dv2), e);
+              key = kp_sel(b, e, key);
               dur = kp_sel(b, M.dur[(s2.left >> 14) & 0xFFu], dur);
               word = kp_sel(b, s2.word, word);
               res = kp_sel(b, left2, res);
@@ -897,6 +1192,7 @@ __device__ __attribute__((noinline)) double kp_list(uint64_t blob, uint64_t ovl_
     }
   }
   if (n > 0 && ghi >= 0x7FF00000u) return -1.0;
+  const double makespan = kp_readlane(dvm, 63);   // (the set of all vertices: every node reserves one)
   if (TR) {   // from place to node; the states are not needed any more
     kp_sync();
     for (int p = lane; p < n; p += KE_WAVE) {
@@ -959,7 +1255,8 @@ template <int TR>
 __device__ inline double kp_schedule(const uint8_t* blob, int n, uint64_t ovl, uint64_t dpne, const KpLds& M, unsigned long long* stamp) {
   const uint64_t b = (uint64_t)blob;
   if (n <= 64) return kp_lanes<1, TR>(b, ovl, dpne, M, stamp);
-  if (n <= KP_LANE_NODES) return kp_lanes<2, TR>(b, ovl, dpne, M, stamp);
+  if (n <= 128) return kp_lanes<2, TR>(b, ovl, dpne, M, stamp);
+  if (n <= KP_LANE_NODES) return kp_lanes<3, TR>(b, ovl, dpne, M, stamp);
   const double ms = kp_list<TR>(b, ovl, dpne, M, stamp);
   return ms == -2.0 ? kp_plain<TR>(b, ovl, dpne, M) : ms;
 }
