@@ -423,11 +423,11 @@ __global__ __launch_bounds__(WAVE) void k_eval(const EvalLaunch L) {
 struct QuadKind { uint32_t plans, entries; };
 constexpr QuadKind QUAD_KIND[3] = {{32, 8}, {16, 16}, {16, 24}};   // k_quad<2, 4>, <4, 4>, <4, 6>
 template <int QL, int SL>
-__global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_quad(const EvalLaunch L) {
+__global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_quad(const EvalLaunch L, const QuadSize Z) {
   extern __shared__ uint8_t kq_lds[];
   const uint64_t w = blockIdx.x;
-  if (SL == 4 && QL == 4 && (L.wave_cls[w] & KE_CLS_LDS)) kq_eval_wave<QL, 2>(L, w, kq_lds);   // uniform branch
-  else kq_eval_wave<QL, SL>(L, w, kq_lds);
+  if (SL == 4 && QL == 4 && (L.wave_cls[w] & KE_CLS_LDS)) kq_eval_wave<QL, 2>(L, Z, w, kq_lds);   // uniform branch
+  else kq_eval_wave<QL, SL>(L, Z, w, kq_lds);
 }
 
 // One plan per wavefront (rpeg_kernel_plan.h); perm[w] is the plan of wavefront task w.  TR: KpTrace.
@@ -744,7 +744,9 @@ struct rpeg_engine_s {
   std::unique_ptr<Lowering> low;                     // of this engine's calls; `out` is the class lowered last
   std::unordered_map<uint64_t, uint32_t> class_off;  // signature -> byte offset in the pool
   std::vector<uint64_t> cls_sig;                     // class id -> signature / pool offset / node count
-  std::vector<uint32_t> cls_off, cls_nodes, cls_slots;
+  std::vector<uint32_t> cls_off, cls_nodes;
+  std::vector<QuadSize> cls_quad;                    // what k_quad's LDS needs for the class; no rows: it is not for that kernel
+  QuadSize max_quad;                                 // the largest of them
   std::vector<uint32_t> cls_pops16;                  // learned, of the slowest full wavefront of the class in the main kernel:
                                                      // microseconds << 12 | heap pops per dispatch in sixteenths
   std::vector<uint32_t> cls_need;                    // learned: the longest ready set of the class's plans in k_quad or the main kernel (0: none yet)
@@ -1038,7 +1040,9 @@ static void class_append(rpeg_engine_t* e, uint64_t sig, uint8_t* blob, size_t o
   e->cls_sig.push_back(sig);
   e->cls_off.push_back((uint32_t)off);
   e->cls_nodes.push_back(h->n_nodes);
-  e->cls_slots.push_back(h->n_slots);
+  const QuadSize quad_size{h->n_nodes, h->n_slots, h->n_rows, h->n_types};
+  e->cls_quad.push_back(quad_size);
+  e->max_quad.fit(quad_size);
   e->cls_pops16.push_back(0);
   e->cls_need.push_back(0);
   e->learn_calls = 3;
@@ -1341,7 +1345,8 @@ int rpeg_engine_reset_classes(rpeg_engine_t* e) {
   e->cls_sig.clear();
   e->cls_off.clear();
   e->cls_nodes.clear();
-  e->cls_slots.clear();
+  e->cls_quad.clear();
+  e->max_quad = QuadSize();
   e->cls_pops16.clear();
   e->cls_need.clear();
   e->cls_split.clear();
@@ -1667,10 +1672,10 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   int ls = e->state_lanes;
   bool one = false;   // one plan per wavefront (k_plan)
   const bool quad_free = ls == -1 && e->quad_share_pct && e->split_heavy && plan_fits();   // k_quad may take the batch (plan_quad)
-  const bool quad_all = ls == 4;   // every class in the kernel of two or four lanes per plan (k_quad)
+  const bool quad_all = ls == 4;   // every class in the kernel of two or four lanes per plan (k_quad), but one that its fields do not hold (QuadRec)
   if (quad_all) {
     ls = 0;
-    if (kq_lds_bytes(16, e->max_nodes, e->max_slots, mass != nullptr) > 160 * 1024 || e->max_nodes > KQ_MAX_NODES) {
+    if (kq_lds_bytes(16, e->max_quad, mass != nullptr) > 160 * 1024 || e->max_nodes > QUAD_NODES + 1) {
       e->err = "per-plan state of this problem does not fit in LDS with sixteen plans per wavefront";
       return -8;
     }
@@ -1723,15 +1728,17 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // ready-list capacity of the main kernel: the full list until the longest list of earlier launches is known
   const uint32_t rcap_main = e->need > 0 ? std::min(e->ready_cap, std::max(8u, (e->need + 2 + 7) & ~7u)) : e->ready_cap;
   // k_quad: the form with the fewest entries that the longest ready set of the class's earlier plans fits.  Two lanes per
-  // plan only up to QUAD_TWO_NODES nodes: thirty-two plans of larger graphs leave too few wavefronts room in LDS.  (No
-  // class / 35 / 60 nodes / all of them, us per step: GRPO 65,536 381 / 386 / 366 / 382; PPO 60,000 787 / 796 / 786 / 1,022.)
+  // plan only up to QUAD_TWO_NODES nodes: thirty-two plans of larger graphs leave too few wavefronts room in LDS.  (35 / 60 /
+  // 100 nodes / all, us per step: GRPO 131,072 494 / 487 / - / -, 65,536 331 / 330 / 354 / 355; PPO 60,000 575 / 578 / 671 /
+  // 652, 20,011 - / 320 / 376 / 450.)
   constexpr uint32_t QUAD_TWO_NODES = 60;
   auto quad_kind = [&](size_t c) {
     const uint32_t need = e->cls_need[cids[c]];
     return need == 0 ? 2 : need <= QUAD_KIND[0].entries && e->cls_nodes[cids[c]] <= QUAD_TWO_NODES ? 0 : need <= QUAD_KIND[1].entries ? 1 : 2;
   };
-  std::vector<uint8_t> solo(counts.size(), 0), quad(counts.size(), quad_all ? 1 : 0);
-  constexpr uint32_t QUAD_TINY = 8, QUAD_MEAN_NODES = 128;
+  std::vector<uint8_t> solo(counts.size(), 0), quad(counts.size(), 0);
+  for (size_t c = 0; quad_all && c < counts.size(); ++c) quad[c] = e->cls_quad[cids[c]].rows ? 1 : 0;
+  constexpr uint32_t QUAD_TINY = 8, QUAD_MEAN_NODES = 128, QUAD_DEEP_PLANS = 896;
   // k_quad takes the batch, with k_plan beside it, where the model below has them done before the main kernel would be.
   // Into k_plan go the classes of fewer than QUAD_TINY plans (a wavefront of k_quad lasts as long with one plan as with
   // all; 4, 8 and 16 measured: 8 is best or within 2 % on five batches), those whose ready sets outgrow sixteen entries,
@@ -1740,11 +1747,12 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // classes' and k_plan's together, and no less than its longest wavefront.  Only once half of the plans it
   // would take are in classes whose ready sets the main kernel has measured; the others' unknown ready sets take the form with
   // the most entries.
-  // Measured, us per step, main kernel / k_quad: GRPO (51 nodes on average) 17,000 plans 402 / 270, 65,536 460 / 365,
-  // 131,072 716 / 580; PPO (98) 20,011 548 / 384, 131,072 1,616 / 1,505; DPO (28) 65,536 277 / 140, 1,048,576 1,686 /
-  // 1,225.  AC-share (152): 20,011 1,216 / 930, but 65,536 2,353 / 2,300-2,500 and 262,144 5,549 / 8,426: of large graphs
-  // few plans have room in LDS, and the main kernel keeps its state in HBM: a batch of more than sixteen of its wavefronts
-  // per compute unit stays there where the plans have more than QUAD_MEAN_NODES nodes on average.
+  // Measured, us per step, main kernel / k_quad: GRPO (51 nodes on average) 17,000 plans 402 / 260, 65,536 460 / 330,
+  // 131,072 716 / 486; PPO (98) 20,011 548 / 320, 131,072 1,616 / 1,075; DPO (28) 65,536 277 / 158, 1,048,576 1,686 /
+  // 1,015.  AC-share (152): 20,011 1,216 / 770, 65,536 2,350 / 1,610, 131,072 3,270 / 2,990, 196,608 4,340 / 4,296, but 262,144
+  // 5,430-5,580 / 5,610-5,650: the time per plan of either falls as classes fill their wavefronts, that of the main kernel
+  // longer.  A batch of more than QUAD_DEEP_PLANS plans per compute unit stays there where the plans have more than
+  // QUAD_MEAN_NODES nodes on average.
   auto plan_quad = [&]() -> bool {
     if (!quad_free) return false;
     const DeepModel dm = deep_model(e, rcap_main);
@@ -1757,7 +1765,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       if (counts[c] >= QUAD_TINY) { takes += counts[c]; measured += e->cls_need[cids[c]] ? counts[c] : 0; }
       if (w) { t_sum += (double)(w >> 12); nodes_sum += (double)e->cls_nodes[cids[c]]; pops_sum += (w & 0xFFFu) / 16.0; ++known; }
     }
-    if (nodes > QUAD_MEAN_NODES * n && main_tasks > (uint64_t)e->n_cu * 16) return false;
+    if (nodes > QUAD_MEAN_NODES * n && n > (uint64_t)e->n_cu * QUAD_DEEP_PLANS) return false;
     // (A batch of under two wavefronts of the main kernel per compute unit is not for that kernel, whatever it has measured:
     // k_plan with 64 plans per compute unit and the main kernel with 8 to 64 plans per wavefront beyond that / k_quad, us
     // per step: DPO 16,384 plans 194 / 137, 20,000 212 / 137; PPO 16,384 473 / 393; AC-share 16,384 1,030 / 850.)
@@ -1771,7 +1779,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     };
     auto cost_quad = [&](uint32_t c) {   // all of the class's, in time of a compute unit
       const QuadKind& k = QUAD_KIND[quad_kind(c)];
-      const double held = std::min(16.0, std::floor(160.0 * 1024 / (double)kq_lds_bytes(k.plans, e->cls_nodes[cids[c]], e->cls_slots[cids[c]], mass != nullptr)));
+      const double held = std::min(16.0, std::floor(160.0 * 1024 / (double)kq_lds_bytes(k.plans, e->cls_quad[cids[c]], mass != nullptr)));
       return (double)((counts[c] + k.plans - 1) / k.plans) * t_quad(c) / std::max(1.0, held);
     };
     auto cost_plan = [&](uint32_t c) { return dm.plan_cost(counts[c], e->cls_nodes[cids[c]]) / (16.0 * dm.sm.eff_beside_quad); };
@@ -1781,7 +1789,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       const double t0 = (double)(e->cls_pops16[cids[c]] >> 12), t = t0 > 0.0 ? t0 : per_node * (double)e->cls_nodes[cids[c]];
       if (counts[c] >= TINY_CLASS) { w_main += (double)((counts[c] + WAVE - 1) / WAVE) * t; max_main = std::max(max_main, t); }
       else base_plan += dm.plan_cost(counts[c], e->cls_nodes[cids[c]]);
-      to_plan[c] = counts[c] < QUAD_TINY || e->cls_need[cids[c]] > QUAD_KIND[1].entries || e->cls_nodes[cids[c]] > KQ_MAX_NODES;
+      to_plan[c] = counts[c] < QUAD_TINY || e->cls_need[cids[c]] > QUAD_KIND[1].entries || !e->cls_quad[cids[c]].rows;
       if (to_plan[c]) w_plan += cost_plan(c);
       else w_quad += cost_quad(c);
     }
@@ -1814,7 +1822,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   if (keep_split) {
     for (size_t c = 0; c < counts.size(); ++c) {
       const uint8_t a = cids[c] < e->cls_split.size() ? e->cls_split[cids[c]] : (uint8_t)255;
-      if (a == 255 && e->split_quad) (counts[c] < QUAD_TINY || e->cls_nodes[cids[c]] > KQ_MAX_NODES ? solo[c] : quad[c]) = 1;
+      if (a == 255 && e->split_quad) (counts[c] < QUAD_TINY || !e->cls_quad[cids[c]].rows ? solo[c] : quad[c]) = 1;
       else if (a == 255) solo[c] = counts[c] < TINY_CLASS ? 1 : 0;
       else if (a == 1) solo[c] = 1;
       else if (a == 2) (e->cls_need[cids[c]] > QUAD_KIND[1].entries ? solo[c] : quad[c]) = 1;   // (as plan_quad would, once a ready set has outgrown sixteen entries)
@@ -1990,7 +1998,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // own, and where a stream is left, one for the larger and one for the smaller graphs of a form -- the LDS of a launch is
   // that of its largest graph, and LDS bounds the wavefronts in flight.  The line lies where the sum over the tasks of
   // time (nodes) times LDS is smallest.
-  struct QuadLaunch { uint32_t first = 0, waves = 0, nodes = 0, slots = 0; int kind = 0; } quad_launch[4];
+  struct QuadLaunch { uint32_t first = 0, waves = 0; QuadSize size; int kind = 0; } quad_launch[4];
   {
     auto waves_of = [&](uint32_t c, int kind) { return (counts[c] + QUAD_KIND[kind].plans - 1) / QUAD_KIND[kind].plans; };
     for (int kind : {2, 0, 1}) {
@@ -2003,7 +2011,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
         }
       size_t cut = qc.size();
       if (kind != 2 && !quad_launch[2].waves && !quad_launch[3].waves && !qc.empty()) {
-        auto lds_of = [&](uint32_t c) { return (double)kq_lds_bytes(QUAD_KIND[kind].plans, e->cls_nodes[cids[c]], e->max_slots, mass != nullptr); };
+        auto lds_of = [&](uint32_t c) { return (double)kq_lds_bytes(QUAD_KIND[kind].plans, e->cls_quad[cids[c]], mass != nullptr); };
         double upto = 0.0, best = all * lds_of(qc[0]);
         for (size_t k = 0; k + 1 < qc.size(); ++k) {
           upto += (double)waves_of(qc[k], kind) * (double)e->cls_nodes[cids[qc[k]]];
@@ -2021,11 +2029,19 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
         const uint32_t nw = waves_of(c, kind);
         if (!q.waves) { q.first = n_quad_waves; q.kind = kind; }
         q.waves += nw;
-        q.nodes = std::max(q.nodes, e->cls_nodes[cids[c]]);
-        q.slots = std::max(q.slots, e->cls_slots[cids[c]]);
+        q.size.fit(e->cls_quad[cids[c]]);
         n_quad_waves += nw;
       }
     }
+  }
+  {   // the ranks of a wavefront all at once, where the launches' wavefronts find room together all the same
+    double cu = 0.0;
+    for (QuadLaunch& q : quad_launch) {
+      q.size.parts = 1;
+      if (q.waves) cu += (double)q.waves / std::floor(160.0 * 1024 / (double)kq_lds_bytes(QUAD_KIND[q.kind].plans, q.size, mass != nullptr));
+    }
+    if (!(cu <= (double)e->n_cu))
+      for (QuadLaunch& q : quad_launch) q.size.parts = KQ_PARTS;
   }
   const uint32_t n_lane_waves = n_eval_waves + n_quad_waves;
   const uint32_t pstride = one ? 1u : (uint32_t)WAVE;
@@ -2224,19 +2240,18 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     Q.perm = e->d_perm + ((uint64_t)n_eval_waves + q.first) * WAVE;
     Q.wave_cls = L.wave_cls + n_eval_waves + q.first;
     Q.n_waves = q.waves;
-    Q.ws_nodes = q.nodes; Q.ws_slots = q.slots;
     Q.ovf = nullptr; Q.cstat = nullptr; Q.queue = nullptr;   // (a plan that outgrows the entries is flagged in Q.limit)
     if (L.prof) Q.prof = L.prof + (n_waves + q.first) * 8;
-    const size_t qlds = kq_lds_bytes(QUAD_KIND[q.kind].plans, q.nodes, q.slots, mass != nullptr);
+    const size_t qlds = kq_lds_bytes(QUAD_KIND[q.kind].plans, q.size, mass != nullptr);
     if (qlds > 64 * 1024 && !e->quad_attr_set) {
       HIP_TRY(e, hipFuncSetAttribute((const void*)k_quad<2, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
       HIP_TRY(e, hipFuncSetAttribute((const void*)k_quad<4, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
       HIP_TRY(e, hipFuncSetAttribute((const void*)k_quad<4, 6>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
       e->quad_attr_set = true;
     }
-    if (q.kind == 0) hipLaunchKernelGGL((k_quad<2, 4>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q);
-    else if (q.kind == 1) hipLaunchKernelGGL((k_quad<4, 4>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q);
-    else hipLaunchKernelGGL((k_quad<4, 6>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q);
+    if (q.kind == 0) hipLaunchKernelGGL((k_quad<2, 4>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q, q.size);
+    else if (q.kind == 1) hipLaunchKernelGGL((k_quad<4, 4>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q, q.size);
+    else hipLaunchKernelGGL((k_quad<4, 6>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q, q.size);
     HIP_TRY(e, hipGetLastError());
     return 0;
   };

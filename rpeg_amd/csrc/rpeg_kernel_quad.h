@@ -21,10 +21,11 @@
 // So every plan of a wavefront dispatches one node per round, and all of them end together: a class has one node count.
 // (With every push-back carried out a round lasted as long as that of the plan with the most of them.)
 //
-// Per-plan state in LDS, interleaved by plan: ready time (the rank before that), in-degree and a word of everything
-// else a new entry needs, per node; durations by slot; availability by vertex.  A round is three LDS trips:
-// the successors' places and the duration of the dispatched node; the state of up to four successors, each looked at by
-// a lane that has room for it; the availability of their vertices.
+// Per-plan state in LDS, interleaved by plan: a word of position, sharing and predecessors to go per node; the ready times
+// of nodes with several predecessors, in rows that later nodes take over (QuadRec); durations by slot; reservations by
+// type; availability by vertex.  What is the same for all plans comes with the successor's place (QuadRec).  A round is
+// three LDS trips: the successors' places and the duration of the dispatched node; the state of up to four successors, each
+// looked at by a lane that has room for it; the availability of their vertices.
 //
 // A plan with more entries ready at once than its lanes hold is not evaluated here: it is flagged (EvalLaunch::limit)
 // and redone by the launch that ends the call, a plan per wavefront.  Its class then reports one entry more than there was
@@ -33,13 +34,13 @@
 // 384).  Ranks go level by level with a node per lane of the plan.  A node's id is its place by tie-break class, so that
 // counting the larger ranks of its class walks through consecutive rows.
 //
-// Bound: LDS, which holds the wavefronts in flight to 1-2 per SIMD (13 bytes per node and 8 per slot for a plan), and
-// with them the latency of a round: measured on 65,536 GRPO plans with four lanes of four entries, a round is 394 vector,
-// 75 scalar and 24 LDS instructions, 40 % of its time vector issue and 38 % waiting.  DPO graphs (28 nodes) fill the SIMDs
-// and are bound by issue.
-// Scheduling a wavefront: 42-node GRPO class 60 us, 92 nodes 130-190, 28-node DPO class 35.  The step, main kernel and
-// the earlier form of this one (every push-back carried out) against now: 65,536 GRPO plans 460 -> 365 us, 1,048,576 DPO
-// plans 1,686 -> 1,190, 20,011 PPO plans 548 -> 384.
+// Bound: vector issue and, with few wavefronts in flight, the latency of a round (four lanes of four entries: some 360 vector
+// instructions a round).  LDS bounds the wavefronts in flight: sixteen plans of 85 nodes and 40 slots take 13 KiB, 3 per
+// SIMD (with a ready time, a word and an in-degree per node and plan, and all plans' ranks at once, 26 KiB and 1.5; 300
+// nodes 28 against 70 KiB).
+// Scheduling a wavefront: 42-node GRPO class 60 us, 92 nodes 130-190, 28-node DPO class 35.  The step, with the larger state
+// against now: 131,072 GRPO plans 568 -> 486 us, 20,011 PPO plans 366 -> 320, 60,000 761 -> 578, 131,072 1,442 -> 1,075,
+// 1,048,576 DPO plans 1,187 -> 1,015; GRPO 17,000 and 65,536 and DPO 65,536 within 8 %.
 #ifndef RPEG_KERNEL_QUAD_H
 #define RPEG_KERNEL_QUAD_H
 
@@ -48,17 +49,31 @@
 
 namespace rpeg {
 
-constexpr uint32_t KQ_MAX_NODES = 512, KQ_MAX_SLOTS = 256;   // what the fields of an entry hold
 constexpr uint32_t KQ_TIE_BITS = 20, KQ_TIE_MASK = (1u << KQ_TIE_BITS) - 1u;   // (a round takes at most 1 + 24 + 24 ties and four per new entry: 2^15 for 512 nodes)
 constexpr uint32_t KQ_EMPTY = 0xFFFFFFFFu;
 
-// LDS of one wavefront.  Class tables: node records, groups, level place -> id, group members and the first place of
-// every level; per plan [row][plan]: ready time and a neutral element (with the critical-chain masses start
-// times too), durations, availability by vertex, a zero and a row nobody reads, node words, in-degrees.
-__host__ __device__ inline size_t kq_tab_bytes(uint32_t nodes) { return (16ull * nodes + 4ull * nodes + 3 * 2ull * (nodes + 2) + 15) & ~size_t(15); }
-__host__ __device__ inline size_t kq_lds_bytes(uint32_t plans, uint32_t nodes, uint32_t slots, bool mass) {
-  return kq_tab_bytes(nodes) +
-         (size_t)plans * (((mass ? 2ull : 1ull) * 8ull * (nodes + 1) + 8ull * slots + 8ull * (RPEG_MAX_V + 2) + 5ull * nodes + 15) & ~15ull);
+constexpr uint32_t KQ_PARTS = 4;
+// What a launch's LDS is sized for: the largest of its classes in each respect.
+struct QuadSize {
+  uint32_t nodes = 0, slots = 0, rows = 0, types = 0;
+  uint32_t parts = KQ_PARTS;   // the ranks of this fraction of the plans at a time: 1 or KQ_PARTS
+  __host__ __device__ void fit(const QuadSize& o) {
+    nodes = o.nodes > nodes ? o.nodes : nodes; slots = o.slots > slots ? o.slots : slots;
+    rows = o.rows > rows ? o.rows : rows; types = o.types > types ? o.types : types;
+  }
+};
+// LDS of one wavefront.  Class tables: per node four successor words, its own, and its level place's id; the first place of
+// every level.  Per plan [row][plan]: durations, availability by vertex with a row of zeros and one nobody reads, ready-time
+// rows -- over them, before they are needed, the ranks of all or a quarter of the plans --, with the critical-chain masses finish
+// and start times, a state word and a reservation each.
+__host__ __device__ inline size_t kq_tab_bytes(uint32_t nodes) { return (20ull * nodes + 2 * 2ull * (nodes + 2) + 15) & ~size_t(15); }
+__host__ __device__ inline size_t kq_union_bytes(uint32_t plans, const QuadSize& z) {
+  const size_t rows = 8ull * plans * z.rows, ranks = 8ull * (plans / z.parts) * (z.nodes + 1);
+  return rows > ranks ? rows : ranks;
+}
+__host__ __device__ inline size_t kq_lds_bytes(uint32_t plans, const QuadSize& z, bool mass) {
+  return (kq_tab_bytes(z.nodes) + (size_t)plans * (8ull * z.slots + 8ull * (RPEG_MAX_V + 2) + (mass ? 16ull * z.nodes : 0ull) + 2ull * z.nodes + 2ull * z.types) +
+          kq_union_bytes(plans, z) + 15) & ~size_t(15);
 }
 
 #if defined(__HIPCC__)
@@ -108,32 +123,120 @@ __device__ inline double kq_min(double v) {
   return v;
 }
 
+// Ranks and, from them, the state words of all plans of a wavefront.  Ranks take eight bytes a node, more than all a plan keeps
+// of it later: where a launch has more wavefronts than find room at once, they are computed for a quarter of the plans at a
+// time, with four times the lanes for each.  (All at once / a quarter at a time, us a step: 16,384 DPO plans 134 / 138, 17,000
+// GRPO 254 / 259, 20,011 PPO 317 / 332; 65,536 GRPO 343 / 325, 65,536 chains 692 / 606, 1,048,576 DPO 1,116 / 1,014.)
+template <int QL, uint32_t PARTS>
+__device__ inline void kq_positions(const ClassView& cv, double* ranks, const double* dur_rows, const uint32_t* l_succ, const uint32_t* l_own,
+                                    const uint16_t* l_id, const uint16_t* l_lbeg, uint16_t* states) {
+  constexpr int RW = KE_WAVE / QL, QR = (int)PARTS * QL, RG = KE_WAVE / QR;   // lanes of a plan, plans at a time
+  const int lane = threadIdx.x, r_q = lane % QR, n = (int)cv.h->n_nodes, n_levels = (int)cv.h->n_levels, n_groups = (int)cv.h->n_groups;
+  for (int part = 0; part < (int)PARTS; ++part) {
+    const int r_p = part * RG + lane / QR;
+    double* const g_rank = ranks + lane / QR;
+    const double* const r_dur = dur_rows + r_p;
+    // ---- ranks: level by level from the nodes without successors, then chain inheritance (scheduler.py:71-100, 367-378);
+    // the words of the next level's node are read while this level's ranks are computed
+    if (r_q == 0) g_rank[n * RG] = 0.0;
+    __syncthreads();
+    {
+      int i = r_q, id = l_id[i < n ? i : 0];
+      uint4 sw = ((const uint4*)l_succ)[id];
+      uint32_t own = l_own[id];
+      for (int l = 0; l < n_levels; ++l) {
+        const int end = l_lbeg[l + 1], nx = end + r_q, id2 = l_id[nx < n ? nx : 0];
+        const uint4 sw2 = ((const uint4*)l_succ)[id2];
+        const uint32_t own2 = l_own[id2];
+        for (;;) {
+          const double d = r_dur[((own >> 10) & 0xFFu) * RW];
+          const double r0 = g_rank[(sw.x & 0x1FFu) * RG], r1 = g_rank[(sw.y & 0x1FFu) * RG], r2 = g_rank[(sw.z & 0x1FFu) * RG], r3 = g_rank[(sw.w & 0x1FFu) * RG];
+          double best = kp_vmax(kp_vmax(r0, r1), kp_vmax(r2, r3));
+          if (__builtin_expect(__ballot(i < end && (own & 7u) > 4u) != 0ull, 0))
+            if (i < end && (own & 7u) > 4u) {
+              const NodeRec nr = cv.node[cv.lrec[i].node];
+              for (int j = 4; j < nr.n_succ; ++j) best = kp_vmax(best, g_rank[l_id[cv.place[cv.succ[nr.succ_begin + j]]] * RG]);
+            }
+          if (i < end) g_rank[id * RG] = d + best;
+          i += QR;
+          if (__builtin_expect(__ballot(i < end) == 0ull, 1)) break;
+          id = l_id[i < n ? i : 0];
+          sw = ((const uint4*)l_succ)[id];
+          own = l_own[id];
+        }
+        i = nx;
+        id = id2;
+        sw = sw2;
+        own = own2;
+      }
+    }
+    for (int g = r_q; g < n_groups; g += QR) {
+      const int begin = (int)cv.group[g].begin, count = (int)cv.group[g].count;
+      double top = g_rank[l_id[cv.glvl[begin]] * RG];
+      for (int j = 1; j < count; ++j) {
+        const double r = g_rank[l_id[cv.glvl[begin + j]] * RG];
+        top = r > top ? r : top;
+      }
+      for (int j = 0; j < count; ++j) g_rank[l_id[cv.glvl[begin + j]] * RG] = top;
+    }
+    __syncthreads();
+    // ---- positions: nodes before v in (comm_prio*8+topo_idx ascending, rank descending) = the nodes of lower tie-break
+    // classes and the nodes of its own class with a larger rank; shared where more nodes than its own chain agree
+    {
+      OrderRec next = cv.orec[r_q < n ? r_q : 0];
+      for (int i = r_q; i < n; i += QR) {
+        const OrderRec o = next;
+        next = cv.orec[i + QR < n ? i + QR : 0];
+        const double rv = g_rank[i * RG];
+        const int b1 = o.b1;
+        int before = o.b0, same = 0, j = o.b0;
+        for (; j + 4 <= b1; j += 4) {   // four independent LDS reads in flight
+          const double r0 = g_rank[j * RG], r1 = g_rank[(j + 1) * RG], r2 = g_rank[(j + 2) * RG], r3 = g_rank[(j + 3) * RG];
+          before += (r0 > rv ? 1 : 0) + (r1 > rv ? 1 : 0) + (r2 > rv ? 1 : 0) + (r3 > rv ? 1 : 0);
+          same += (r0 == rv ? 1 : 0) + (r1 == rv ? 1 : 0) + (r2 == rv ? 1 : 0) + (r3 == rv ? 1 : 0);
+        }
+        for (; j < b1; ++j) {
+          const double r = g_rank[j * RG];
+          before += r > rv ? 1 : 0;
+          same += r == rv ? 1 : 0;
+        }
+        states[i * RW + r_p] = (uint16_t)((uint32_t)before | (same > (int)o.chain_n ? 0x200u : 0u) | (((l_own[i] >> 3) & 0x3Fu) << 10));
+      }
+    }
+    __syncthreads();   // (these ranks are done with)
+  }
+}
+
 template <int QL, int SL>
-__device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* lds) {
+__device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint64_t w, uint8_t* lds) {
   constexpr int RW = KE_WAVE / QL;
   const int lane = threadIdx.x, p = lane / QL, q = lane % QL;
   constexpr int first_lane = 0;
   const rpeg_problem_t& P = *L.P;
   const ClassView cv = class_view(L.pool + (L.wave_cls[w] & ~KE_CLS_LDS));   // uniform
-  const int n = (int)cv.h->n_nodes, n_slots = (int)cv.h->n_slots, n_levels = (int)cv.h->n_levels, n_groups = (int)cv.h->n_groups;
+  const int n = (int)cv.h->n_nodes, n_slots = (int)cv.h->n_slots, n_levels = (int)cv.h->n_levels;
+  const int n_rows = (int)cv.h->n_rows, n_types = (int)cv.h->n_types;
 
   // ---- LDS carve-up
-  LevelRec* l_rec = (LevelRec*)lds;
-  uint32_t* l_group = (uint32_t*)(l_rec + L.ws_nodes);
-  uint16_t* l_id = (uint16_t*)(l_group + L.ws_nodes);
-  uint16_t* l_gm = l_id + (L.ws_nodes + 2);
-  uint16_t* l_lbeg = l_gm + (L.ws_nodes + 2);
-  double* rows = (double*)(lds + kq_tab_bytes(L.ws_nodes));
-  double* g_time = rows + p;
-  rows += (size_t)(L.ws_nodes + 1) * RW;
-  double* g_start = rows + p;
-  if (L.mass) rows += (size_t)(L.ws_nodes + 1) * RW;
+  uint32_t* l_succ = (uint32_t*)lds;               // [node id][4]: id | the successor's QuadRec from bit 10 on; bit 31: none (its id is the neutral element's)
+  uint32_t* l_own = l_succ + 4 * Z.nodes;          // [node id]: QuadRec
+  uint16_t* l_id = (uint16_t*)(l_own + Z.nodes);   // level place -> id
+  uint16_t* l_lbeg = l_id + (Z.nodes + 2);
+  double* rows = (double*)(lds + kq_tab_bytes(Z.nodes));
   double* g_dur = rows + p;
-  rows += (size_t)L.ws_slots * RW;
+  double* const dur_rows = rows;
+  rows += (size_t)Z.slots * RW;
   double* g_lf = rows + p;
   rows += (size_t)(RPEG_MAX_V + 2) * RW;
-  uint32_t* g_info = (uint32_t*)rows + p;
-  uint8_t* g_deg = (uint8_t*)((uint32_t*)rows + (size_t)L.ws_nodes * RW) + p;
+  double* const ranks = rows;                      // [node id][plans of a quarter]
+  double* g_time = rows + p;                       // [row]
+  rows = (double*)((uint8_t*)rows + kq_union_bytes(RW, Z));
+  double* g_fin = rows + p;                        // [node id], with L.mass
+  double* g_start = g_fin + (size_t)Z.nodes * RW;
+  if (L.mass) rows += 2 * (size_t)Z.nodes * RW;
+  uint16_t* const states = (uint16_t*)rows;
+  uint16_t* g_state = states + p;                  // [node id]: position | shared << 9 | predecessors to go << 10
+  uint16_t* g_type = states + (size_t)Z.nodes * RW + p;   // [reservation]: reserved vertices | vertices that overlap them << 6
 
   // a place without a plan repeats the first one of the wavefront, without outputs: every lane is active throughout
   const uint32_t entry = L.perm[w * KE_WAVE + p];
@@ -142,16 +245,18 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
   __syncthreads();  // the previous task of this wavefront is done with LDS
   for (int i = lane; i < n; i += KE_WAVE) l_id[cv.orec[i].at] = (uint16_t)i;
   if (lane == 0) l_id[n] = (uint16_t)n;
-  for (int i = lane; i < n_groups; i += KE_WAVE) l_group[i] = ((const uint32_t*)cv.group)[i];
   for (int i = lane; i <= n_levels; i += KE_WAVE) l_lbeg[i] = cv.lbeg[i];
   __syncthreads();
   for (int i = lane; i < n; i += KE_WAVE) {
-    LevelRec r = cv.lrec[i];
+    const LevelRec r = cv.lrec[i];
+    const uint32_t id = l_id[i];
+    l_own[id] = cv.qrec[i];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) r.succ[k] = l_id[r.succ[k]];
-    l_rec[l_id[i]] = r;
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t at = r.succ[k];
+      l_succ[4 * id + k] = (uint32_t)l_id[at] | (at < (uint32_t)n ? cv.qrec[at] & ~0x3FFu : 0x80000000u);
+    }
   }
-  for (int i = lane; i < (int)cv.h->n_gmembers; i += KE_WAVE) l_gm[i] = l_id[cv.glvl[i]];
   KE_STAMP(0);
 
   // pair relations, penalty factor and gate bits of this plan and the durations of its class's slots (out of the table
@@ -160,9 +265,9 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
   const double pen = L.aux_pen ? L.aux_pen[pi] : 1.0;
   const uint8_t gates = L.aux_mask ? L.aux_mask[pi] : (uint8_t)(RPEG_MASK_VALID | RPEG_MASK_STALE_OK | RPEG_MASK_MEM_OK);
   KE_STAMP(1);
-  bool err = cv.h->error != 0;
+  bool err = cv.h->error != 0, ovf = false;
   {   // a slot whose duration the reference could not compute (division by zero) is NaN; a share by each lane
-    bool bad = false;
+    bool bad = false, shrinks = false;
     for (int s0 = q; s0 < n_slots; s0 += 4 * QL) {   // four rows in flight
       double d[4];
 #pragma unroll
@@ -174,94 +279,33 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
       for (int k = 0; k < 4; ++k) {
         const int s = s0 + k * QL;
         bad = bad || d[k] != d[k];
+        shrinks = shrinks || d[k] < 0.0;   // (nodes could share no rows: QuadRec)
         if (s < n_slots) g_dur[s * RW] = d[k];
       }
     }
-    err = err || kq_or<QL>(bad ? 1u : 0u) != 0u;
+    const uint32_t odd = kq_or<QL>((bad ? 1u : 0u) | (shrinks ? 2u : 0u));
+    err = err || (odd & 1u);
+    ovf = (odd & 2u) != 0u;
     if (err)   // (no NaN in the loops below)
       for (int s = q; s < n_slots; s += QL) g_dur[s * RW] = 0.0;
   }
-  if (q == 0) {
-    g_time[n * RW] = 0.0;
+  if (q == 0)
     for (int x = 0; x <= RPEG_MAX_V; ++x) g_lf[x * RW] = 0.0;
+  for (int t = q; t < n_types; t += QL) {
+    const uint32_t bc = cv.type[t], bt = kp_reserved(bc & 0xFFu, bc >> 8, ovl, dpne);
+    g_type[t * RW] = (uint16_t)((bt & 0x3Fu) | (((bt >> 8) & 0x3Fu) << 6));
   }
   __syncthreads();
   KE_STAMP(2);
   const bool stale_ok = (gates & RPEG_MASK_STALE_OK) != 0, mem_ok = (gates & RPEG_MASK_MEM_OK) != 0;
 
   KE_STAMP(3);
-  // ---- ranks: level by level from the nodes without successors, then chain inheritance (scheduler.py:71-100, 367-378);
-  // the record of the next level's node is read while this level's ranks are computed
-  {
-    int i = q, id = l_id[i < n ? i : 0];
-    LevelRec rec = l_rec[id];
-    for (int l = 0; l < n_levels; ++l) {
-      const int end = l_lbeg[l + 1], nx = end + q, id2 = l_id[nx < n ? nx : 0];
-      const LevelRec rec2 = l_rec[id2];
-      for (;;) {
-        const double d = g_dur[rec.slot * RW];
-        const double r0 = g_time[rec.succ[0] * RW], r1 = g_time[rec.succ[1] * RW], r2 = g_time[rec.succ[2] * RW], r3 = g_time[rec.succ[3] * RW];
-        double best = kp_vmax(kp_vmax(r0, r1), kp_vmax(r2, r3));
-        if (__builtin_expect(__ballot(i < end && rec.n_succ > 4) != 0ull, 0))
-          for (int j = 4; i < end && j < rec.n_succ; ++j) best = kp_vmax(best, g_time[l_id[cv.place[cv.succ[cv.node[rec.node].succ_begin + j]]] * RW]);
-        if (i < end) g_time[id * RW] = d + best;
-        i += QL;
-        if (__builtin_expect(__ballot(i < end) == 0ull, 1)) break;
-        id = l_id[i < n ? i : 0];
-        rec = l_rec[id];
-      }
-      i = nx;
-      id = id2;
-      rec = rec2;
-    }
-  }
-  for (int g = q; g < n_groups; g += QL) {
-    const int begin = (int)(l_group[g] & 0xFFFFu), count = (int)(l_group[g] >> 16);
-    double top = g_time[l_gm[begin] * RW];
-    for (int j = 1; j < count; ++j) {
-      const double r = g_time[l_gm[begin + j] * RW];
-      top = r > top ? r : top;
-    }
-    for (int j = 0; j < count; ++j) g_time[l_gm[begin + j] * RW] = top;
-  }
-  __syncthreads();
-#ifdef KE_FINE_PROF
-  KE_STAMP(4);
-#endif
-  // ---- positions: nodes before v in (comm_prio*8+topo_idx ascending, rank descending) = the nodes of lower tie-break
-  // classes and the nodes of its own class with a larger rank; shared where more nodes than its own chain agree.
-  // Node word: position | shared << 9 | slot << 10 | reserved vertices << 18 | vertices that overlap them << 24
-  {
-    OrderRec next = cv.orec[q < n ? q : 0];
-    for (int i = q; i < n; i += QL) {
-      const OrderRec o = next;
-      next = cv.orec[i + QL < n ? i + QL : 0];
-      const double rv = g_time[i * RW];
-      const int b1 = o.b1;
-      int before = o.b0, same = 0, j = o.b0;
-      for (; j + 4 <= b1; j += 4) {   // four independent LDS reads in flight
-        const double r0 = g_time[j * RW], r1 = g_time[(j + 1) * RW], r2 = g_time[(j + 2) * RW], r3 = g_time[(j + 3) * RW];
-        before += (r0 > rv ? 1 : 0) + (r1 > rv ? 1 : 0) + (r2 > rv ? 1 : 0) + (r3 > rv ? 1 : 0);
-        same += (r0 == rv ? 1 : 0) + (r1 == rv ? 1 : 0) + (r2 == rv ? 1 : 0) + (r3 == rv ? 1 : 0);
-      }
-      for (; j < b1; ++j) {
-        const double r = g_time[j * RW];
-        before += r > rv ? 1 : 0;
-        same += r == rv ? 1 : 0;
-      }
-      const LevelRec rec = l_rec[i];
-      const uint32_t bt = kp_reserved(rec.blocked, rec.cond, ovl, dpne);
-      g_info[i * RW] = (uint32_t)before | (same > (int)o.chain_n ? 0x200u : 0u) | ((uint32_t)rec.slot << 10) | ((bt & 0x3Fu) << 18) | (((bt >> 8) & 0x3Fu) << 24);
-      g_deg[i * RW] = rec.indeg;
-    }
-  }
-  __syncthreads();   // (the ranks are dead from here on: their array becomes the ready times)
-  for (int v = q; v < n; v += QL) g_time[v * RW] = 0.0;
+  if (Z.parts == 1) kq_positions<QL, 1>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_lbeg, states);
+  else kq_positions<QL, KQ_PARTS>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_lbeg, states);
+  for (int r = q; r < n_rows; r += QL) g_time[r * RW] = 0.0;
   __syncthreads();
 
-#ifndef KE_FINE_PROF
   KE_STAMP(4);
-#endif
   // ---- list scheduling (scheduler.py:399-546)
   const double inf = __builtin_inf();
   double ek[SL], sk[SL];
@@ -270,7 +314,6 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
   for (int u = 0; u < SL; ++u) { ek[u] = inf; sk[u] = inf; eo[u] = KQ_EMPTY; em[u] = 0u; }
   uint32_t tie = 0, free_slots = (1u << SL) - 1u;
   int live = 0, longest = 0;   // entries now and at most (one more than there is room for where one was lost)
-  bool ovf = false;
   const unsigned group_shift = (unsigned)(lane & ~(QL - 1));
   const uint32_t below = (1u << q) - 1u;   // the lanes of this plan before this one
   // this lane keeps the availability of vertices q, q + QL, ... (where there are fewer: of the row behind the zeros)
@@ -287,11 +330,11 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
   }
   const mask64 quads0 = QL == 4 ? 0x1111111111111111ull : 0x5555555555555555ull;   // the first lane of every plan
   // an entry into the first free slot of this lane, in the lanes of `take` (conditions are kept as masks of the lanes in
-  // scalar registers: as booleans the compiler moves them through vector registers)
-  auto file = [&](mask64 take, double key, uint32_t info, uint32_t place, uint32_t t) {
+  // scalar registers: as booleans the compiler moves them through vector registers).  node: id | its QuadRec from bit 10 on
+  auto file = [&](mask64 take, double key, uint32_t state, uint32_t node, uint32_t type, uint32_t t) {
     const uint32_t first = kp_sel(take, free_slots & (0u - free_slots), 0u), u_free = 31u - (uint32_t)__builtin_clz(first | 1u);
-    const uint32_t word = ((info & 0x1FFu) << KQ_TIE_BITS) | t, meta = (info & 0x3FFFFC00u) | place | (u_free << 30) | ((u_free >> 2) << 9);
-    const double heap_key = kp_sel(__ballot((info & 0x200u) != 0u), key, inf);
+    const uint32_t word = ((state & 0x1FFu) << KQ_TIE_BITS) | t, meta = (node & 0x3FDFFu) | (type << 18) | (u_free << 30) | ((u_free >> 2) << 9);
+    const double heap_key = kp_sel(__ballot((state & 0x200u) != 0u), key, inf);
 #pragma unroll
     for (int u = 0; u < SL; ++u) {
       const mask64 m = __ballot(first == (1u << u));
@@ -304,11 +347,11 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
   };
   {
     const int n_init = (int)cv.h->n_init;
-    ovf = n_init > QL * SL;
+    ovf = ovf || n_init > QL * SL;
     for (int i0 = 0; i0 < n_init && i0 < QL * SL; i0 += QL) {
       const bool mine = i0 + q < n_init;
-      const uint32_t v = l_id[cv.place[cv.init[mine ? i0 + q : 0]]];
-      file(__ballot(mine), 0.0, g_info[v * RW], v, (uint32_t)(i0 + q));
+      const uint32_t v = l_id[cv.place[cv.init[mine ? i0 + q : 0]]], own = l_own[v];
+      file(__ballot(mine), 0.0, g_state[v * RW], v | (own & ~0x3FFu), g_type[((own >> 18) & 0x3Fu) * RW], (uint32_t)(i0 + q));
     }
     tie = (uint32_t)n_init;
     live = longest = n_init;
@@ -421,11 +464,12 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
     uint32_t in_plan = (uint32_t)(room >> group_shift) & ((1u << QL) - 1u);
     uint32_t r = (uint32_t)__builtin_popcount(in_plan & below), n_room = (uint32_t)__builtin_popcount(in_plan);
     const uint32_t place = bm & 0x1FFu;
-    const uint32_t first_succ = l_rec[place].succ[r], n_succ = l_rec[place].n_succ;
+    const uint32_t first_succ = l_succ[4 * place + r];   // (r < QL)
+    uint32_t n_succ = l_own[place] & 7u;
     const double fin = gk + g_dur[(int)((bm >> 10) & 0xFFu) * RW];
-    if (L.mass) {   // the trace: a dispatched node does not need its ready time again
+    if (L.mass) {
       if (kp_in(alive & quads0)) {
-        g_time[place * RW] = fin;
+        g_fin[place * RW] = fin;
         g_start[place * RW] = gk;
       }
     }
@@ -441,25 +485,24 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
     for (int u = 0; u < SL; ++u) ek[u] = kp_sel(__ballot((em[u] & touched) != 0u), kp_vmax(ek[u], fin), ek[u]);
     // successors: the lanes with room look at one each; those that became ready are filed where they were looked at
     // (scheduler.py:540-546: ties in successor order)
+    if (__builtin_expect(__ballot(n_succ == 7u) != 0ull, 0)) n_succ = n_succ == 7u ? (uint32_t)cv.node[cv.lrec[cv.orec[place].at].node].n_succ : n_succ;
     mask64 mine = room & alive & __ballot(r < n_succ);
     uint32_t j0 = 0, sp = first_succ;
     while (mine) {
-      const uint32_t at = kp_sel(mine, sp, 0u);
-      const double t0 = g_time[at * RW];
-      const uint32_t deg = g_deg[at * RW], info = g_info[at * RW];
-      const uint32_t left = deg - 1u;
-      double t = kp_vmax(t0, fin);
-      if (kp_in(mine)) {
-        g_time[at * RW] = t;
-        g_deg[at * RW] = (uint8_t)left;
+      const uint32_t node = kp_sel(mine, sp, 0u), at = node & 0x1FFu, row = node >> 24;   // (a node of one predecessor: the row of zeros, never written)
+      const uint32_t state = g_state[at * RW], left = state - 0x400u, type = g_type[((node >> 18) & 0x3Fu) * RW];
+      double t = kp_vmax(g_time[row * RW], fin);
+      const mask64 ready = mine & __ballot(left < 0x400u);
+      if (kp_in(mine & ~ready)) {
+        g_time[row * RW] = t;
+        g_state[at * RW] = (uint16_t)left;
       }
-      const mask64 ready = mine & __ballot(left == 0u);
       if (ready) {
-        const uint32_t b6 = (info >> 18) & 0x3Fu;   // one vertex or two (none: the row of zeros)
+        const uint32_t b6 = type & 0x3Fu;   // one vertex or two (none: the row of zeros)
         const uint32_t v1 = (uint32_t)__builtin_ctz(b6 | (1u << RPEG_MAX_V)), v2 = b6 ? 31u - (uint32_t)__builtin_clz(b6) : (uint32_t)RPEG_MAX_V;
         t = kp_vmax(t, kp_vmax(g_lf[v1 * RW], g_lf[v2 * RW]));
         const uint32_t rdy = (uint32_t)(ready >> group_shift) & ((1u << QL) - 1u);
-        file(ready, t, info, at, tie + (uint32_t)__builtin_popcount(rdy & below));
+        file(ready, t, state, node, type, tie + (uint32_t)__builtin_popcount(rdy & below));
         tie += (uint32_t)QL;
         live += (int)__builtin_popcount(rdy);
         longest = live > longest ? live : longest;
@@ -479,7 +522,12 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
       sp = 0;
       if (kp_in(mine)) {
         const uint32_t j = j0 + r;
-        sp = j < 4u ? l_rec[place].succ[j] : l_id[cv.place[cv.succ[cv.node[l_rec[place].node].succ_begin + j]]];
+        if (j < 4u) {
+          sp = l_succ[4 * place + j];
+        } else {
+          const uint32_t to = cv.place[cv.succ[cv.node[cv.lrec[cv.orec[place].at].node].succ_begin + j]];
+          sp = (uint32_t)l_id[to] | (cv.qrec[to] & ~0x3FFu);
+        }
       }
     }
   }
@@ -525,7 +573,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, uint64_t w, uint8_t* ld
 #pragma unroll
         for (int x = 0; x < RPEG_MAX_V; ++x) m[x] = __builtin_nan("");
       } else {
-        critical_mass(cv, [&](int i) { return g_time[l_id[cv.place[i]] * RW]; }, [&](int i) { return g_start[l_id[cv.place[i]] * RW]; }, m);
+        critical_mass(cv, [&](int i) { return g_fin[l_id[cv.place[i]] * RW]; }, [&](int i) { return g_start[l_id[cv.place[i]] * RW]; }, m);
       }
 #pragma unroll
       for (int x = 0; x < RPEG_MAX_V; ++x) L.mass[pi * RPEG_MAX_V + x] = m[x];

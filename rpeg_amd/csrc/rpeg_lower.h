@@ -134,6 +134,51 @@ class Lowering {
   std::vector<Tr> to_train, to_serving;
   // and what the blob needs of it
   std::vector<int> adj_beg, adj_to, indeg, deg, cur, topo, chain_beg, chain_of, level, place, chain_n, chain_i, lbeg;
+  std::vector<uint64_t> anc, row_pred;        // a bit each: per node its ancestors; per row the predecessors of the last node that has it
+  std::vector<int> row_of;                    // per node: its ready-time row
+  std::vector<uint16_t> types, type_of;
+  int n_rows = 0;
+  bool quad_rows(const NodeRec* recs, const uint16_t* pbeg, const uint16_t* pred, int n) {
+    if (n > (int)QUAD_NODES || (int)topo.size() != n) return false;
+    const int W = (n + 63) / 64;
+    anc.assign((size_t)n * W, 0);
+    row_pred.assign(W, 0);
+    row_of.assign(n, 0); types.clear(); type_of.resize(n);
+    n_rows = 1;
+    for (int v : topo) {
+      uint64_t* const a = &anc[(size_t)v * W];
+      const int b = pbeg[v], d = pbeg[v + 1] - b;
+      const uint16_t t = (uint16_t)(recs[v].blocked | recs[v].cond << 8);
+      size_t k = 0;
+      while (k < types.size() && types[k] != t) ++k;
+      if (k == types.size()) types.push_back(t);
+      type_of[v] = (uint16_t)k;
+      if (recs[v].indeg > QUAD_INDEG || types.size() > QUAD_TYPES) return false;
+      uint64_t common[(QUAD_NODES + 64) / 64];   // the ancestors that all predecessors have
+      if (d) std::memcpy(common, &anc[(size_t)pred[b] * W], (size_t)W * 8);
+      if (d) std::memcpy(a, common, (size_t)W * 8);
+      for (int j = 1; j < d; ++j) {
+        const uint64_t* const p = &anc[(size_t)pred[b + j] * W];
+        for (int w = 0; w < W; ++w) { a[w] |= p[w]; common[w] &= p[w]; }
+      }
+      for (int j = 0; j < d; ++j) a[pred[b + j] >> 6] |= 1ull << (pred[b + j] & 63);
+      if (d < 2) continue;
+      int r = 1;
+      for (; r < n_rows; ++r) {
+        const uint64_t* const x = &row_pred[(size_t)r * W];
+        int w = 0;
+        while (w < W && !(x[w] & ~common[w])) ++w;
+        if (w == W) break;
+      }
+      if (r > (int)QUAD_ROWS) return false;
+      if (r == n_rows) row_pred.resize((size_t)++n_rows * W);
+      uint64_t* const x = &row_pred[(size_t)r * W];
+      std::fill(x, x + W, 0);
+      for (int j = 0; j < d; ++j) x[pred[b + j] >> 6] |= 1ull << (pred[b + j] & 63);
+      row_of[v] = r;
+    }
+    return true;
+  }
 
   int slot(const SigView& sg, SlotType t, int a, int b, int q) {
     const uint8_t u = sg.tab->at[LowerTables::key(t, (unsigned)a, (unsigned)b, (unsigned)q)];
@@ -457,11 +502,11 @@ class Lowering {
     h.off_orec = (uint32_t)off; off = align8(off + (size_t)n * sizeof(OrderRec));
     h.off_lbeg = (uint32_t)off; off = align8(off + lbeg.size() * 2);
     h.off_place = (uint32_t)off; off = align8(off + (size_t)n * 2);
-    h.off_glvl = (uint32_t)off; off = (off + (size_t)n_gm * 2 + 15) & ~size_t(15);   // (blobs start on sixteen-byte boundaries of the pool)
-    h.bytes = (uint32_t)off;
-    out.blob.assign(off, 0);
+    h.off_glvl = (uint32_t)off; off = align8(off + (size_t)n_gm * 2);
+    h.off_qrec = (uint32_t)off; off = align8(off + (size_t)n * 4);
+    h.off_type = (uint32_t)off;   // (the last one: its length is known when the nodes are)
+    out.blob.assign(off + 2 * QUAD_TYPES + 16, 0);
     uint8_t* const B = out.blob.data();
-    std::memcpy(B, &h, sizeof h);
     NodeRec* const recs = (NodeRec*)(B + h.off_node);
     uint16_t* const succ = (uint16_t*)(B + h.off_succ);
     for (int i = 0; i < n; ++i) {
@@ -504,10 +549,25 @@ class Lowering {
     uint16_t *const gmember = (uint16_t*)(B + h.off_gmember), *const glvl = (uint16_t*)(B + h.off_glvl);
     for (int k = 0; k < n_gm; ++k) { gmember[k] = (uint16_t)chain_of[k]; glvl[k] = (uint16_t)place[chain_of[k]]; }
     // predecessors in edge order
-    uint16_t *const pbeg = (uint16_t*)(B + h.off_pbeg), *const pred = (uint16_t*)(B + h.off_pred);
-    cur.resize(n);
-    for (int i = 0; i < n; ++i) { cur[i] = pbeg[i]; pbeg[i + 1] = (uint16_t)(pbeg[i] + indeg[i]); }
-    for (auto& ed : edges) pred[cur[ed.second]++] = (uint16_t)ed.first;
+    {
+      uint16_t *const pbeg = (uint16_t*)(B + h.off_pbeg), *const pred = (uint16_t*)(B + h.off_pred);
+      cur.resize(n);
+      for (int i = 0; i < n; ++i) { cur[i] = pbeg[i]; pbeg[i + 1] = (uint16_t)(pbeg[i] + indeg[i]); }
+      for (auto& ed : edges) pred[cur[ed.second]++] = (uint16_t)ed.first;
+      const bool quad = quad_rows(recs, pbeg, pred, n);
+      h.n_rows = quad ? (uint32_t)n_rows : 0u;
+      h.n_types = quad ? (uint32_t)types.size() : 0u;
+    }
+    off = (off + (size_t)h.n_types * 2 + 15) & ~size_t(15);   // (blobs start on sixteen-byte boundaries of the pool)
+    h.bytes = (uint32_t)off;
+    out.blob.resize(off);
+    std::memcpy(B, &h, sizeof h);
+    if (h.n_types) std::memcpy(B + h.off_type, types.data(), types.size() * 2);
+    if (h.n_rows) {
+      uint32_t* const qrec = (uint32_t*)(B + h.off_qrec);
+      for (int v = 0; v < n; ++v)
+        qrec[place[v]] = std::min<uint32_t>(recs[v].n_succ, 7u) | (uint32_t)recs[v].indeg << 3 | (uint32_t)recs[v].slot << 10 | (uint32_t)type_of[v] << 18 | (uint32_t)row_of[v] << 24;
+    }
     // the orders of the one-plan-per-wavefront kernel: by level, and by tie-break class
     LevelRec* const lrec = (LevelRec*)(B + h.off_lrec);
     uint16_t *const lbeg16 = (uint16_t*)(B + h.off_lbeg), *const place16 = (uint16_t*)(B + h.off_place);
