@@ -203,65 +203,63 @@ __device__ inline double kp_class_peak(const rpeg_problem_t& P, const rpeg_struc
 // the sorted order, because a node starts no earlier than the nodes dispatched before it on its devices ended.
 // Then the vertices are taken in the order of their first reservation, and the devices of each allocation that
 // no earlier one holds are added 64 at a time: the lanes find set and value of their device, one running sum
-// takes the values in lane order.  l_start / l_fin: per node; l_order: node dispatched k-th; l_tab: 64 doubles.
+// takes the values in lane order.  l_start / l_fin: per node; l_order: node dispatched k-th; l_tab: 64 doubles;
+// l_span / l_set: two doubles and a byte per node in dispatch order.
+//
+// Bound: one chain of compares and adds per node, whose operands are therefore brought into dispatch order first, a node
+// per lane, and read four nodes at a time; values are added from constant lanes, zeros where there is no device.  (Class
+// records fetched within the chain, and a loop over the devices found: outputs of an AC-share plan 50-70 us, now 21-25; a
+// launch of 41 such plans of 92-300 nodes 298 -> 248 us, one evaluation of a PPO plan 264 -> 248.)
 __device__ inline double kp_utilization(const ClassView& cv, const int n, const int lane, const int nv, const int16_t* l_plan,
                                         const uint64_t dpne, const double* l_start, const double* l_fin,
-                                        const uint16_t* l_order, double* l_tab, const double ms) {
+                                        const uint16_t* l_order, double* l_tab, double2* l_span, uint8_t* l_set, const double ms) {
   if (!(ms > 0.0) || n == 0) return 0.0;
+  // vertices by first reservation, four bits each: of node number k, a transfer's source before its destination
+  uint32_t first = 0xFFFFFFFFu;   // lane v: when vertex v is first reserved
+  unsigned seen = 0u;
+  for (int base = 0; base < n; base += KE_WAVE) {
+    const int k = base + lane, i = (int)l_order[k < n ? k : base];
+    NodeRec nr;
+    const uint64_t bits = ((const uint64_t*)cv.node)[i];
+    __builtin_memcpy(&nr, &bits, 8);
+    const unsigned b = k < n ? blocked_mask(nr, dpne) : 0u;
+    if (k < n) l_span[k] = make_double2(l_start[i], l_fin[i]);
+    if (k < ((n + 3) & ~3)) l_set[k] = (uint8_t)b;
+    for (int v = 0; v < nv; ++v) {
+      const mask64 has = __ballot((b >> v) & 1u);
+      if (!has || ((seen >> v) & 1u)) continue;
+      const int at = __builtin_ctzll(has);
+      const unsigned cond = (unsigned)__builtin_amdgcn_readlane((int)nr.cond, at);
+      if (lane == v) first = (uint32_t)(base + at) << 4 | (cond && (cond - 1u) >> 3 == (unsigned)v ? 0u : (uint32_t)v + 1u);
+      seen |= 1u << v;
+    }
+  }
+  kp_sync();
   {
     const unsigned mine = (unsigned)lane;
-    double merged = 0.0, cs = 0.0, ce = 0.0;
-    bool open = false;
-    for (int k = 0; k < n; ++k) {
-      const int i = (int)l_order[k];
-      const uint64_t bits = ((const uint64_t*)cv.node)[i];
-      NodeRec nr;
-      __builtin_memcpy(&nr, &bits, 8);
-      const unsigned b = blocked_mask(nr, dpne);
-      const double s = l_start[i], f = l_fin[i];
-      if (b & mine) {
-        if (!open || s > ce) {
-          if (open) merged += ce - cs;
-          cs = s;
-          ce = f;
-          open = true;
-        } else {
-          ce = f > ce ? f : ce;
-        }
+    double merged = 0.0, cs = -1.0, ce = -1.0;   // (no span yet: one of no length)
+    for (int k = 0; k < n; k += 4) {
+      const uint32_t sets = *(const uint32_t*)(l_set + k);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {   // (behind the last node: sets without a vertex)
+        const double2 t = l_span[k + j];
+        const bool in = ((sets >> (8 * j)) & mine) != 0u;
+        const double s = in ? t.x : -__builtin_inf(), f = in ? t.y : -__builtin_inf(), span = ce - cs;
+        const bool apart = s > ce;
+        merged = apart ? merged + span : merged;
+        cs = apart ? s : cs;
+        ce = apart || f > ce ? f : ce;
       }
     }
-    if (open) merged += ce - cs;
+    merged += ce - cs;
     l_tab[lane] = merged / ms;
   }
   kp_sync();
-  // vertices by first reservation, four bits each
   uint32_t order = 0u;
-  int n_ev = 0;
-  {
-    unsigned seen = 0u;
-    for (int k = 0; k < n && n_ev < nv; ++k) {
-      const int i = __builtin_amdgcn_readfirstlane((int)l_order[k]);
-      const uint64_t bits = ((const uint64_t*)cv.node)[i];
-      NodeRec nr;
-      __builtin_memcpy(&nr, &bits, 8);
-      unsigned b = blocked_mask(nr, dpne) & ~seen;
-      if (nr.cond) {   // a transfer: source before destination
-        const unsigned src = (nr.cond - 1u) >> 3;
-        if ((b >> src) & 1u) {
-          order |= src << (4 * n_ev);
-          ++n_ev;
-          seen |= 1u << src;
-          b &= ~(1u << src);
-        }
-      }
-      while (b) {
-        const unsigned v = (unsigned)__builtin_ctz(b);
-        b &= b - 1u;
-        order |= v << (4 * n_ev);
-        ++n_ev;
-        seen |= 1u << v;
-      }
-    }
+  const int n_ev = __builtin_popcount(seen);
+  for (int v = 0; v < nv; ++v) {
+    const uint32_t f = (uint32_t)__builtin_amdgcn_readlane((int)first, v);
+    if ((seen >> v) & 1u) order |= (uint32_t)v << (4 * __builtin_popcountll(__ballot(first < f)));
   }
   double total = 0.0;
   int count = 0;
@@ -286,12 +284,15 @@ __device__ inline double kp_utilization(const ClassView& cv, const int n, const 
         M |= in ? 1u << x : 0u;
       }
       const double val = l_tab[M & 63u];
-      unsigned long long fresh = __ballot(idx < cnt && (M & earlier) == 0u);
-      count += (int)__builtin_popcountll(fresh);
-      while (fresh) {
-        const int j = __builtin_ctzll(fresh);
-        fresh &= fresh - 1ull;
-        total += kp_readlane(val, j);
+      const bool fresh = idx < cnt && (M & earlier) == 0u;
+      const mask64 all = __ballot(fresh);
+      const double add = fresh ? val : 0.0;   // (the sum is not negative: zero leaves it as it is)
+      count += (int)__builtin_popcountll(all);
+#pragma unroll
+      for (int j0 = 0; j0 < 64; j0 += 16) {
+        if (!((all >> j0) & 0xFFFFull)) continue;
+#pragma unroll
+        for (int j = j0; j < j0 + 16; ++j) total += kp_readlane(add, j);
       }
     }
     earlier |= 1u << v;
@@ -548,7 +549,7 @@ __device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const
   }
   double util = 0.0;
   if (TR == KP_TIMES_ORDER && L.util)
-    util = err ? __builtin_nan("") : kp_utilization(cv, n, lane, nv, l_plan, pm.dpne, l_start, l_rank, l_ord, l_tab, makespan);
+    util = err ? __builtin_nan("") : kp_utilization(cv, n, lane, nv, l_plan, pm.dpne, l_start, l_rank, l_ord, l_tab, (double2*)l_rec, l_pt, makespan);
   double m = __builtin_nan("");   // lane x < RPEG_MAX_V: mass of vertex x
   if (chain) {
     if (NW > 1) {
