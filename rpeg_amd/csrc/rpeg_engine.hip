@@ -1738,6 +1738,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   };
   std::vector<uint8_t> solo(counts.size(), 0), quad(counts.size(), 0);
   for (size_t c = 0; quad_all && c < counts.size(); ++c) quad[c] = e->cls_quad[cids[c]].rows ? 1 : 0;
+  constexpr double QUAD_HALF_LDS = 1.05;
   constexpr uint32_t QUAD_TINY = 8, QUAD_MEAN_NODES = 128, QUAD_DEEP_PLANS = 896;
   // k_quad takes the batch, with k_plan beside it, where the model below has them done before the main kernel would be.
   // Into k_plan go the classes of fewer than QUAD_TINY plans (a wavefront of k_quad lasts as long with one plan as with
@@ -2034,14 +2035,21 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       }
     }
   }
-  {   // the ranks of a wavefront all at once, where the launches' wavefronts find room together all the same
+  {   // the ranks of a wavefront all at once, where the launches' wavefronts find room together all the same; else of half
+      // its plans, where that needs (next to) no more LDS than those of a quarter, which the rows behind them need anyway
     double cu = 0.0;
     for (QuadLaunch& q : quad_launch) {
       q.size.parts = 1;
       if (q.waves) cu += (double)q.waves / std::floor(160.0 * 1024 / (double)kq_lds_bytes(QUAD_KIND[q.kind].plans, q.size, mass != nullptr));
     }
     if (!(cu <= (double)e->n_cu))
-      for (QuadLaunch& q : quad_launch) q.size.parts = KQ_PARTS;
+      for (QuadLaunch& q : quad_launch) {
+        const uint32_t plans = QUAD_KIND[q.kind].plans;
+        q.size.parts = KQ_PARTS;
+        const double quarter = (double)kq_lds_bytes(plans, q.size, mass != nullptr);
+        q.size.parts = 2;
+        if ((double)kq_lds_bytes(plans, q.size, mass != nullptr) > QUAD_HALF_LDS * quarter) q.size.parts = KQ_PARTS;
+      }
   }
   const uint32_t n_lane_waves = n_eval_waves + n_quad_waves;
   const uint32_t pstride = one ? 1u : (uint32_t)WAVE;

@@ -53,10 +53,15 @@ constexpr uint32_t KQ_TIE_BITS = 20, KQ_TIE_MASK = (1u << KQ_TIE_BITS) - 1u;   /
 constexpr uint32_t KQ_EMPTY = 0xFFFFFFFFu;
 
 constexpr uint32_t KQ_PARTS = 4;
+// Graphs of up to this many nodes have their equal ranks counted along with the larger ones, larger graphs afterwards, by
+// position: along, every pair of a class costs two instructions more, afterwards every node 25 and three LDS trips, and
+// classes grow with the graph.  (Afterwards / along, us a step: 65,536 GRPO plans of 51 nodes 322 / 315, 65,536 DPO plans of 28
+// 163 / 156; 65,536 AC-share plans of 152 1,520 / 1,625, 131,072 PPO plans of 98 1,010 / 1,045.)
+constexpr int KQ_EQ_NODES = 60;
 // What a launch's LDS is sized for: the largest of its classes in each respect.
 struct QuadSize {
   uint32_t nodes = 0, slots = 0, rows = 0, types = 0;
-  uint32_t parts = KQ_PARTS;   // the ranks of this fraction of the plans at a time: 1 or KQ_PARTS
+  uint32_t parts = KQ_PARTS;   // the ranks of this fraction of the plans at a time: 1, 2 or KQ_PARTS
   __host__ __device__ void fit(const QuadSize& o) {
     nodes = o.nodes > nodes ? o.nodes : nodes; slots = o.slots > slots ? o.slots : slots;
     rows = o.rows > rows ? o.rows : rows; types = o.types > types ? o.types : types;
@@ -64,15 +69,15 @@ struct QuadSize {
 };
 // LDS of one wavefront.  Class tables: per node four successor words, its own, and its level place's id; the first place of
 // every level.  Per plan [row][plan]: durations, availability by vertex with a row of zeros and one nobody reads, ready-time
-// rows -- over them, before they are needed, the ranks of all or a quarter of the plans --, with the critical-chain masses finish
+// rows -- over these two, before they are needed, the ranks of all, half or a quarter of the plans --, with the critical-chain masses finish
 // and start times, a state word and a reservation each.
 __host__ __device__ inline size_t kq_tab_bytes(uint32_t nodes) { return (20ull * nodes + 2 * 2ull * (nodes + 2) + 15) & ~size_t(15); }
 __host__ __device__ inline size_t kq_union_bytes(uint32_t plans, const QuadSize& z) {
-  const size_t rows = 8ull * plans * z.rows, ranks = 8ull * (plans / z.parts) * (z.nodes + 1);
+  const size_t rows = 8ull * plans * (z.rows + RPEG_MAX_V + 2), ranks = 8ull * (plans / z.parts) * (z.nodes + 1);
   return rows > ranks ? rows : ranks;
 }
 __host__ __device__ inline size_t kq_lds_bytes(uint32_t plans, const QuadSize& z, bool mass) {
-  return (kq_tab_bytes(z.nodes) + (size_t)plans * (8ull * z.slots + 8ull * (RPEG_MAX_V + 2) + (mass ? 16ull * z.nodes : 0ull) + 2ull * z.nodes + 2ull * z.types) +
+  return (kq_tab_bytes(z.nodes) + (size_t)plans * (8ull * z.slots + (mass ? 16ull * z.nodes : 0ull) + 2ull * z.nodes + 2ull * z.types) +
           kq_union_bytes(plans, z) + 15) & ~size_t(15);
 }
 
@@ -123,85 +128,151 @@ __device__ inline double kq_min(double v) {
   return v;
 }
 
+// Positions of nodes i, i + QR, ... of the tie-break class that takes ids b to e - 1, into their state words; with EQ also
+// whether they are shared.
+template <int QL, int QR, int NB, bool EQ>
+__device__ inline void kq_count(const double* g_rank, const uint32_t* l_own, const uint16_t* l_chain, uint16_t* g_state, int i, int b, int e) {
+  constexpr int RW = KE_WAVE / QL, RG = KE_WAVE / QR, AHEAD = NB == 1 ? 8 : 4;
+  double rv[NB];
+  uint32_t before[NB], same[NB];
+#pragma unroll
+  for (int t = 0; t < NB; ++t) {
+    rv[t] = g_rank[(i + t * QR < e ? i + t * QR : b) * RG];
+    before[t] = (uint32_t)b;
+    same[t] = 0u;
+  }
+  int j = b;
+  for (; j + AHEAD <= e; j += AHEAD) {
+    double r[AHEAD];
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) r[k] = g_rank[(j + k) * RG];
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k)
+#pragma unroll
+      for (int t = 0; t < NB; ++t) {
+        before[t] += r[k] > rv[t] ? 1u : 0u;
+        if (EQ) same[t] += r[k] == rv[t] ? 1u : 0u;
+      }
+  }
+  for (; j < e; ++j) {
+    const double r = g_rank[j * RG];
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      before[t] += r > rv[t] ? 1u : 0u;
+      if (EQ) same[t] += r == rv[t] ? 1u : 0u;
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < NB; ++t) {
+    const int it = i + t * QR;
+    if (it < e) g_state[it * RW] = (uint16_t)(before[t] | (EQ && same[t] > (uint32_t)(l_chain[it] >> 8) ? 0x200u : 0u) | (((l_own[it] >> 3) & 0x3Fu) << 10));
+  }
+}
+// Positions of all nodes: one class after the other, up to four of its nodes to a lane, so that a rank read counts for all of them.
+template <int QL, int QR, bool EQ>
+__device__ inline void kq_count_all(const double* g_rank, const uint32_t* l_own, const uint16_t* l_chain, uint16_t* g_state, uint32_t class_ends, int r_q, int n) {
+  for (int b = 0, k = 0; b < n; ++k) {
+    const int e = __builtin_amdgcn_readlane((int)class_ends, k);
+    int i0 = b;
+    for (; e - i0 > 2 * QR; i0 += 4 * QR) kq_count<QL, QR, 4, EQ>(g_rank, l_own, l_chain, g_state, i0 + r_q, b, e);
+    if (e - i0 > QR) kq_count<QL, QR, 2, EQ>(g_rank, l_own, l_chain, g_state, i0 + r_q, b, e);
+    else if (e - i0 > 0) kq_count<QL, QR, 1, EQ>(g_rank, l_own, l_chain, g_state, i0 + r_q, b, e);
+    b = e;
+  }
+}
+
+// The largest rank among the successors from the fifth on of the node at level place i, or `best`.
+__device__ inline double kq_more_successors(const ClassView& cv, const double* g_rank, const uint16_t* l_id, int RG, int i, double best) {
+  const NodeRec nr = cv.node[cv.lrec[i].node];
+  for (int j = 4; j < nr.n_succ; ++j) best = kp_vmax(best, g_rank[l_id[cv.place[cv.succ[nr.succ_begin + j]]] * RG]);
+  return best;
+}
+
 // Ranks and, from them, the state words of all plans of a wavefront.  Ranks take eight bytes a node, more than all a plan keeps
-// of it later: where a launch has more wavefronts than find room at once, they are computed for a quarter of the plans at a
-// time, with four times the lanes for each.  (All at once / a quarter at a time, us a step: 16,384 DPO plans 134 / 138, 17,000
-// GRPO 254 / 259, 20,011 PPO 317 / 332; 65,536 GRPO 343 / 325, 65,536 chains 692 / 606, 1,048,576 DPO 1,116 / 1,014.)
+// of it later: where a launch has more wavefronts than find room at once, they are computed for half or a quarter of the
+// plans at a time, with two or four times the lanes for each.  (All at once / a quarter at a time, us a step: 16,384 DPO plans
+// 134 / 138, 17,000 GRPO 254 / 259, 20,011 PPO 317 / 332; 65,536 GRPO 343 / 325, 65,536 chains 692 / 606, 1,048,576 DPO 1,116 /
+// 1,014.  Half at a time where that takes the LDS of a quarter: 1,048,576 DPO 1,025 -> 970.)
+// Bound: instruction issue, some 60 instructions a level and part, two for the comparison of up to 64 pairs of ranks.
 template <int QL, uint32_t PARTS>
 __device__ inline void kq_positions(const ClassView& cv, double* ranks, const double* dur_rows, const uint32_t* l_succ, const uint32_t* l_own,
-                                    const uint16_t* l_id, const uint16_t* l_lbeg, uint16_t* states) {
+                                    const uint16_t* l_id, const uint16_t* l_chain, uint32_t class_ends, bool many, uint16_t* states) {
   constexpr int RW = KE_WAVE / QL, QR = (int)PARTS * QL, RG = KE_WAVE / QR;   // lanes of a plan, plans at a time
-  const int lane = threadIdx.x, r_q = lane % QR, n = (int)cv.h->n_nodes, n_levels = (int)cv.h->n_levels, n_groups = (int)cv.h->n_groups;
+  const int lane = threadIdx.x, r_q = lane % QR, n = (int)cv.h->n_nodes, n_levels = (int)cv.h->n_levels;
   for (int part = 0; part < (int)PARTS; ++part) {
     const int r_p = part * RG + lane / QR;
     double* const g_rank = ranks + lane / QR;
     const double* const r_dur = dur_rows + r_p;
-    // ---- ranks: level by level from the nodes without successors, then chain inheritance (scheduler.py:71-100, 367-378);
-    // the words of the next level's node are read while this level's ranks are computed
+    // ---- ranks: level by level from the nodes without successors, then chain inheritance (scheduler.py:71-100, 367-378).
+    // A level waits for one LDS trip, that of its successors' ranks: words and durations of its nodes were read a level ahead,
+    // their ids two levels.
     if (r_q == 0) g_rank[n * RG] = 0.0;
     __syncthreads();
     {
-      int i = r_q, id = l_id[i < n ? i : 0];
+      uint32_t ends = 0;
+      auto end_of = [&](int l) { return l < n_levels ? __builtin_amdgcn_readlane((int)ends, l & 63) : n; };
+      auto id_at = [&](int i) { return (int)l_id[i < n ? i : n - 1]; };
+      int begin = 0;
+      ends = cv.lbeg[lane + 1 <= n_levels ? lane + 1 : n_levels];
+      int end = end_of(0), id = id_at(r_q), id1 = id_at(end + r_q);
       uint4 sw = ((const uint4*)l_succ)[id];
       uint32_t own = l_own[id];
+      double d = r_dur[((own >> 10) & 0xFFu) * RW];
       for (int l = 0; l < n_levels; ++l) {
-        const int end = l_lbeg[l + 1], nx = end + r_q, id2 = l_id[nx < n ? nx : 0];
-        const uint4 sw2 = ((const uint4*)l_succ)[id2];
-        const uint32_t own2 = l_own[id2];
-        for (;;) {
-          const double d = r_dur[((own >> 10) & 0xFFu) * RW];
-          const double r0 = g_rank[(sw.x & 0x1FFu) * RG], r1 = g_rank[(sw.y & 0x1FFu) * RG], r2 = g_rank[(sw.z & 0x1FFu) * RG], r3 = g_rank[(sw.w & 0x1FFu) * RG];
-          double best = kp_vmax(kp_vmax(r0, r1), kp_vmax(r2, r3));
-          if (__builtin_expect(__ballot(i < end && (own & 7u) > 4u) != 0ull, 0))
-            if (i < end && (own & 7u) > 4u) {
-              const NodeRec nr = cv.node[cv.lrec[i].node];
-              for (int j = 4; j < nr.n_succ; ++j) best = kp_vmax(best, g_rank[l_id[cv.place[cv.succ[nr.succ_begin + j]]] * RG]);
-            }
-          if (i < end) g_rank[id * RG] = d + best;
-          i += QR;
-          if (__builtin_expect(__ballot(i < end) == 0ull, 1)) break;
-          id = l_id[i < n ? i : 0];
-          sw = ((const uint4*)l_succ)[id];
-          own = l_own[id];
+        const double r0 = g_rank[(sw.x & 0x1FFu) * RG], r1 = g_rank[(sw.y & 0x1FFu) * RG], r2 = g_rank[(sw.z & 0x1FFu) * RG], r3 = g_rank[(sw.w & 0x1FFu) * RG];
+        const uint4 sw1 = ((const uint4*)l_succ)[id1];
+        const uint32_t own1 = l_own[id1];
+        if (__builtin_expect((l & 63) == 63, 0)) ends = cv.lbeg[l + 1 + lane + 1 <= n_levels ? l + 1 + lane + 1 : n_levels];
+        const int end1 = end_of(l + 1), id2 = id_at(end1 + r_q);
+        double best = kp_vmax(kp_vmax(r0, r1), kp_vmax(r2, r3));
+        int i = begin + r_q;
+        if (__builtin_expect(many, 0))
+          if (i < end && (own & 7u) > 4u) best = kq_more_successors(cv, g_rank, l_id, RG, i, best);
+        if (i < end) g_rank[id * RG] = d + best;
+        for (i += QR; __builtin_expect(__ballot(i < end) != 0ull, 0); i += QR) {   // (more nodes than lanes)
+          const int id_i = id_at(i);
+          const uint4 w = ((const uint4*)l_succ)[id_i];
+          const uint32_t o = l_own[id_i];
+          best = kp_vmax(kp_vmax(g_rank[(w.x & 0x1FFu) * RG], g_rank[(w.y & 0x1FFu) * RG]), kp_vmax(g_rank[(w.z & 0x1FFu) * RG], g_rank[(w.w & 0x1FFu) * RG]));
+          if (many && i < end && (o & 7u) > 4u) best = kq_more_successors(cv, g_rank, l_id, RG, i, best);
+          if (i < end) g_rank[id_i * RG] = r_dur[((o >> 10) & 0xFFu) * RW] + best;
         }
-        i = nx;
-        id = id2;
-        sw = sw2;
-        own = own2;
+        d = r_dur[((own1 >> 10) & 0xFFu) * RW];
+        begin = end;
+        end = end1;
+        id = id1;
+        id1 = id2;
+        sw = sw1;
+        own = own1;
       }
     }
-    for (int g = r_q; g < n_groups; g += QR) {
-      const int begin = (int)cv.group[g].begin, count = (int)cv.group[g].count;
-      double top = g_rank[l_id[cv.glvl[begin]] * RG];
-      for (int j = 1; j < count; ++j) {
-        const double r = g_rank[l_id[cv.glvl[begin + j]] * RG];
-        top = r > top ? r : top;
-      }
-      for (int j = 0; j < count; ++j) g_rank[l_id[cv.glvl[begin + j]] * RG] = top;
-    }
+    // (the nodes of a chain have the chain's largest rank, which is the first one's where no duration is negative)
     __syncthreads();
-    // ---- positions: nodes before v in (comm_prio*8+topo_idx ascending, rank descending) = the nodes of lower tie-break
-    // classes and the nodes of its own class with a larger rank; shared where more nodes than its own chain agree
-    {
-      OrderRec next = cv.orec[r_q < n ? r_q : 0];
+    if (cv.h->n_groups) {
       for (int i = r_q; i < n; i += QR) {
-        const OrderRec o = next;
-        next = cv.orec[i + QR < n ? i + QR : 0];
-        const double rv = g_rank[i * RG];
-        const int b1 = o.b1;
-        int before = o.b0, same = 0, j = o.b0;
-        for (; j + 4 <= b1; j += 4) {   // four independent LDS reads in flight
-          const double r0 = g_rank[j * RG], r1 = g_rank[(j + 1) * RG], r2 = g_rank[(j + 2) * RG], r3 = g_rank[(j + 3) * RG];
-          before += (r0 > rv ? 1 : 0) + (r1 > rv ? 1 : 0) + (r2 > rv ? 1 : 0) + (r3 > rv ? 1 : 0);
-          same += (r0 == rv ? 1 : 0) + (r1 == rv ? 1 : 0) + (r2 == rv ? 1 : 0) + (r3 == rv ? 1 : 0);
-        }
-        for (; j < b1; ++j) {
-          const double r = g_rank[j * RG];
-          before += r > rv ? 1 : 0;
-          same += r == rv ? 1 : 0;
-        }
-        states[i * RW + r_p] = (uint16_t)((uint32_t)before | (same > (int)o.chain_n ? 0x200u : 0u) | (((l_own[i] >> 3) & 0x3Fu) << 10));
+        const int in_chain = (int)(l_chain[i] & 0xFFu);
+        if (in_chain) g_rank[i * RG] = g_rank[(i - in_chain) * RG];
       }
+      __syncthreads();
+    }
+    // ---- positions: nodes before v in (comm_prio*8+topo_idx ascending, rank descending) = the nodes of lower tie-break
+    // classes and the nodes of its own class with a larger rank; shared where more nodes than its own chain agree.  Equal ranks
+    // are found by counting them along, in small graphs, or afterwards, by counting the nodes of a position.
+    if (n <= KQ_EQ_NODES) {
+      kq_count_all<QL, QR, true>(g_rank, l_own, l_chain, states + r_p, class_ends, r_q, n);
+      __syncthreads();   // (these ranks are done with)
+      continue;
+    }
+    kq_count_all<QL, QR, false>(g_rank, l_own, l_chain, states + r_p, class_ends, r_q, n);
+    __syncthreads();   // (these ranks are done with: over them counters, by position)
+    uint32_t* const g_count = (uint32_t*)(ranks + lane / QR);
+    for (int i = r_q; i < n; i += QR) g_count[2 * i * RG] = 0u;
+    __syncthreads();
+    for (int i = r_q; i < n; i += QR) atomicAdd(&g_count[2 * (states[i * RW + r_p] & 0x1FFu) * RG], 1u);
+    __syncthreads();
+    for (int i = r_q; i < n; i += QR) {
+      const uint32_t state = states[i * RW + r_p];
+      if (g_count[2 * (state & 0x1FFu) * RG] > (uint32_t)(l_chain[i] >> 8)) states[i * RW + r_p] = (uint16_t)(state | 0x200u);
     }
     __syncthreads();   // (these ranks are done with)
   }
@@ -214,22 +285,21 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint
   constexpr int first_lane = 0;
   const rpeg_problem_t& P = *L.P;
   const ClassView cv = class_view(L.pool + (L.wave_cls[w] & ~KE_CLS_LDS));   // uniform
-  const int n = (int)cv.h->n_nodes, n_slots = (int)cv.h->n_slots, n_levels = (int)cv.h->n_levels;
+  const int n = (int)cv.h->n_nodes, n_slots = (int)cv.h->n_slots;
   const int n_rows = (int)cv.h->n_rows, n_types = (int)cv.h->n_types;
 
   // ---- LDS carve-up
   uint32_t* l_succ = (uint32_t*)lds;               // [node id][4]: id | the successor's QuadRec from bit 10 on; bit 31: none (its id is the neutral element's)
   uint32_t* l_own = l_succ + 4 * Z.nodes;          // [node id]: QuadRec
   uint16_t* l_id = (uint16_t*)(l_own + Z.nodes);   // level place -> id
-  uint16_t* l_lbeg = l_id + (Z.nodes + 2);
+  uint16_t* l_chain = l_id + (Z.nodes + 2);        // [node id]: place in its chain (whose nodes' ids follow each other) | nodes of the chain << 8
   double* rows = (double*)(lds + kq_tab_bytes(Z.nodes));
   double* g_dur = rows + p;
   double* const dur_rows = rows;
   rows += (size_t)Z.slots * RW;
+  double* const ranks = rows;                      // [node id][plans at a time], before the two below are needed
   double* g_lf = rows + p;
-  rows += (size_t)(RPEG_MAX_V + 2) * RW;
-  double* const ranks = rows;                      // [node id][plans of a quarter]
-  double* g_time = rows + p;                       // [row]
+  double* g_time = g_lf + (size_t)(RPEG_MAX_V + 2) * RW;   // [row]
   rows = (double*)((uint8_t*)rows + kq_union_bytes(RW, Z));
   double* g_fin = rows + p;                        // [node id], with L.mass
   double* g_start = g_fin + (size_t)Z.nodes * RW;
@@ -243,14 +313,23 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint
   const bool idle = entry == KE_IDLE;
   const uint64_t pi = (uint64_t)(idle ? L.perm[w * KE_WAVE] : entry);
   __syncthreads();  // the previous task of this wavefront is done with LDS
-  for (int i = lane; i < n; i += KE_WAVE) l_id[cv.orec[i].at] = (uint16_t)i;
+  uint32_t class_ends = 0;   // lane k: where the ids of tie-break class k end
+  for (int i = lane, k = 0; i - lane < n; i += KE_WAVE) {
+    const OrderRec r = cv.orec[i < n ? i : 0];
+    if (i < n) {
+      l_id[r.at] = (uint16_t)i;
+      l_chain[i] = (uint16_t)(r.chain_i | r.chain_n << 8);
+    }
+    for (mask64 last = __ballot(i < n && (int)r.b1 == i + 1); last; last &= last - 1ull, ++k) class_ends = lane == k ? (uint32_t)(i - lane + __builtin_ctzll(last) + 1) : class_ends;
+  }
   if (lane == 0) l_id[n] = (uint16_t)n;
-  for (int i = lane; i <= n_levels; i += KE_WAVE) l_lbeg[i] = cv.lbeg[i];
   __syncthreads();
+  mask64 many = 0ull;   // some node has more than four successors
   for (int i = lane; i < n; i += KE_WAVE) {
     const LevelRec r = cv.lrec[i];
     const uint32_t id = l_id[i];
     l_own[id] = cv.qrec[i];
+    many |= __ballot((cv.qrec[i] & 7u) > 4u);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const uint32_t at = r.succ[k];
@@ -289,8 +368,6 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint
     if (err)   // (no NaN in the loops below)
       for (int s = q; s < n_slots; s += QL) g_dur[s * RW] = 0.0;
   }
-  if (q == 0)
-    for (int x = 0; x <= RPEG_MAX_V; ++x) g_lf[x * RW] = 0.0;
   for (int t = q; t < n_types; t += QL) {
     const uint32_t bc = cv.type[t], bt = kp_reserved(bc & 0xFFu, bc >> 8, ovl, dpne);
     g_type[t * RW] = (uint16_t)((bt & 0x3Fu) | (((bt >> 8) & 0x3Fu) << 6));
@@ -300,8 +377,11 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint
   const bool stale_ok = (gates & RPEG_MASK_STALE_OK) != 0, mem_ok = (gates & RPEG_MASK_MEM_OK) != 0;
 
   KE_STAMP(3);
-  if (Z.parts == 1) kq_positions<QL, 1>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_lbeg, states);
-  else kq_positions<QL, KQ_PARTS>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_lbeg, states);
+  const bool any_many = __ballot(many != 0ull) != 0ull;   // (lanes that left the loop early)
+  if (Z.parts == 1) kq_positions<QL, 1>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_chain, class_ends, any_many, states);
+  else if (Z.parts == 2) kq_positions<QL, 2>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_chain, class_ends, any_many, states);
+  else kq_positions<QL, KQ_PARTS>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_chain, class_ends, any_many, states);
+  for (int x = q; x <= RPEG_MAX_V; x += QL) g_lf[x * RW] = 0.0;
   for (int r = q; r < n_rows; r += QL) g_time[r * RW] = 0.0;
   __syncthreads();
 

@@ -281,9 +281,13 @@ __device__ __attribute__((noinline)) void kp_ranks(uint64_t blob, const KpLds M)
   kp_sync();
 }
 
-// Positions: within its tie-break class a node comes behind those of larger rank.  Nodes that agree are told apart by
-// their place in the order; `shared` where they are more than the node's own chain.  NW wavefronts share the nodes (the
-// counting is a pass over the class for each: 34 us of one wavefront's time on a graph of 300 nodes).
+// Positions: within its tie-break class a node comes behind those of larger rank.  Nodes that agree have the same position
+// and are told apart by the order in which they counted themselves there (of one chain: by their place in it); `shared`
+// where they are more than the node's own chain.  NW wavefronts share the nodes.
+// Bound: instruction issue.  A wavefront goes through the classes of its 64 nodes rank by rank, all lanes the same one: two
+// instructions for 64 comparisons.  With the equal ranks counted along, the nodes of shared position going through their class
+// once more, and every lane at its own node's class, it took twice that and more (sixteen wavefronts on a compute unit, 300
+// nodes: 44 us, now 18; 92 nodes 10, now 6.  4,096 PPO plans 170 -> 165 us a step).
 template <int NW>
 __device__ __attribute__((noinline)) void kp_positions(uint64_t blob, int wave, const KpLds M) {
   const int first = wave * KE_WAVE + (int)__lane_id();
@@ -293,11 +297,14 @@ __device__ __attribute__((noinline)) void kp_positions(uint64_t blob, int wave, 
   const int n = (int)h->n_nodes;
   const KP_CONST uint64_t* orec = T.at<uint64_t>(h->off_orec);
   const uint64_t w0 = orec[first < n ? first : 0];   // the records by tie-break class
+  KP_LDS uint32_t* const count = M.at;                    // by position: the nodes that have it
+  KP_LDS uint32_t* const found = (KP_LDS uint32_t*)M.rank;   // by node of this order: its position | its turn there << 10 | nodes that have it << 20 (over the ranks by level place)
   {
     uint64_t w = w0;
     for (int p = first; p < n; p += STEP) {
       const uint64_t next = orec[p + STEP < n ? p + STEP : 0];
       M.rk[p] = M.rank[w & 0xFFFFu];
+      count[p] = 0u;
       w = next;
     }
   }
@@ -307,33 +314,41 @@ __device__ __attribute__((noinline)) void kp_positions(uint64_t blob, int wave, 
     const uint64_t next = orec[p + STEP < n ? p + STEP : 0];
     const bool ok = p < n;
     const double rk = M.rk[ok ? p : 0];
-    const int b0 = (int)((oword >> 16) & 0xFFFFu), b1 = ok ? (int)((oword >> 32) & 0xFFFFu) : b0;
-    const uint32_t chain_n = (uint32_t)(oword >> 48) & 0xFFu, chain_i = (uint32_t)(oword >> 56);
-    uint32_t before = 0u, same = 0u;
-    int j = b0;
-    for (; j + 4 <= b1; j += 4) {   // four independent LDS reads in flight
-      const double r0 = M.rk[j], r1 = M.rk[j + 1], r2 = M.rk[j + 2], r3 = M.rk[j + 3];
-      before += (r0 > rk ? 1u : 0u) + (r1 > rk ? 1u : 0u) + (r2 > rk ? 1u : 0u) + (r3 > rk ? 1u : 0u);
-      same += (r0 == rk ? 1u : 0u) + (r1 == rk ? 1u : 0u) + (r2 == rk ? 1u : 0u) + (r3 == rk ? 1u : 0u);
-    }
-    for (; j < b1; ++j) {
-      const double r = M.rk[j];
-      before += r > rk ? 1u : 0u;
-      same += r == rk ? 1u : 0u;
-    }
-    const bool sh = ok && same > chain_n;
-    uint32_t among = chain_i;
-    if (__ballot(sh)) {
-      if (sh) {
-        among = 0u;
-        for (int u = b0; u < p; ++u) among += M.rk[u] == rk ? 1u : 0u;
+    const int b0 = ok ? (int)((oword >> 16) & 0xFFFFu) : n, b1 = ok ? (int)((oword >> 32) & 0xFFFFu) : n;
+    const int c0 = p - (int)__lane_id(), last = c0 + KE_WAVE < n ? c0 + KE_WAVE : n;
+    uint32_t pos = 0u;
+    for (int b = __builtin_amdgcn_readfirstlane(b0); b < last;) {   // the classes of these lanes' nodes
+      const int e = __builtin_amdgcn_readlane(b1, b < c0 ? 0 : b - c0);
+      uint32_t before[2] = {(uint32_t)b, 0u};
+      int j = b;
+      for (; j + 8 <= e; j += 8) {
+        double r[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) r[k] = M.rk[j + k];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) before[k & 1] += r[k] > rk ? 1u : 0u;
       }
+      for (; j < e; ++j) before[0] += M.rk[j] > rk ? 1u : 0u;
+      pos = kp_sel(__ballot(b0 == b), before[0] + before[1], pos);
+      b = e;
     }
-    const uint32_t pos = (uint32_t)b0 + before, q = pos + among;
-    if (ok) {
-      M.at[q] = (uint32_t)(oword & 0x3FFu) | (sh ? KP_AT_SHARED : 0u) | (same << 11) | (pos << 20);
-      M.q[oword & 0xFFFFu] = (uint16_t)q;
-    }
+    if (ok) found[p] = pos | (__hip_atomic_fetch_add(&count[pos], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) << 10);
+    oword = next;
+  }
+  kp_barrier<NW>();
+  for (int p = first; p < n; p += STEP) {   // (the counters make room for the map)
+    const uint32_t f = found[p];
+    found[p] = f | (count[f & 0x3FFu] << 20);
+  }
+  kp_barrier<NW>();
+  oword = w0;
+  for (int p = first; p < n; p += STEP) {
+    const uint64_t next = orec[p + STEP < n ? p + STEP : 0];
+    const uint32_t f = found[p], pos = f & 0x3FFu, same = f >> 20, chain_n = (uint32_t)(oword >> 48) & 0xFFu, chain_i = (uint32_t)(oword >> 56);
+    const bool sh = same > chain_n;
+    const uint32_t q = pos + (sh ? (f >> 10) & 0x3FFu : chain_i);
+    M.at[q] = (uint32_t)(oword & 0x3FFu) | (sh ? KP_AT_SHARED : 0u) | (same << 11) | (pos << 20);
+    M.q[oword & 0xFFFFu] = (uint16_t)q;
     oword = next;
   }
   if (first == 0) M.q[n] = 0xFFFFu;
