@@ -755,7 +755,7 @@ struct rpeg_engine_s {
   std::vector<uint8_t> cls_split;                    // where every class ran when that was last decided: 0 main kernel, 1 k_plan,
   uint64_t split_for_n = 0, split_at = 0;            // 2 k_quad, 255 not in that batch; the batch size and the call of that decision
   bool split_mass = false;
-  bool split_quad = false;                           // k_quad took the batch
+  bool split_quad = false, split_deep = false;       // k_quad took the batch; a deep one (plan_quad)
   uint32_t learn_calls = 0;                          // calls left after which the statistic is read back
   uint64_t batch_calls = 0;
   uint64_t* d_hkey = nullptr;                        // device table signature -> class id
@@ -1739,10 +1739,11 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   std::vector<uint8_t> solo(counts.size(), 0), quad(counts.size(), 0);
   for (size_t c = 0; quad_all && c < counts.size(); ++c) quad[c] = e->cls_quad[cids[c]].rows ? 1 : 0;
   constexpr double QUAD_HALF_LDS = 1.05;
-  constexpr uint32_t QUAD_TINY = 8, QUAD_MEAN_NODES = 128, QUAD_DEEP_PLANS = 896;
+  constexpr size_t QUAD_BINS = 3;
+  constexpr uint32_t QUAD_TINY = 8, QUAD_MEAN_NODES = 128, QUAD_DEEP_PLANS = 512;
   // k_quad takes the batch, with k_plan beside it, where the model below has them done before the main kernel would be.
   // Into k_plan go the classes of fewer than QUAD_TINY plans (a wavefront of k_quad lasts as long with one plan as with
-  // all; 4, 8 and 16 measured: 8 is best or within 2 % on five batches), those whose ready sets outgrow sixteen entries,
+  // all; 4, 8 and 16 measured: 8 is best or within 2 % on five batches), those whose ready sets outgrow sixteen entries (below: 24),
   // and as many of the largest graphs as make the end earliest: a wavefront of k_quad lasts two to three times as long
   // as a plan in k_plan.  The time of k_quad: its wavefronts' (SplitModel) over those a compute unit holds by LDS, all
   // classes' and k_plan's together, and no less than its longest wavefront.  Only once half of the plans it
@@ -1750,10 +1751,15 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // the most entries.
   // Measured, us per step, main kernel / k_quad: GRPO (51 nodes on average) 17,000 plans 402 / 260, 65,536 460 / 330,
   // 131,072 716 / 486; PPO (98) 20,011 548 / 320, 131,072 1,616 / 1,075; DPO (28) 65,536 277 / 158, 1,048,576 1,686 /
-  // 1,015.  AC-share (152): 20,011 1,216 / 770, 65,536 2,350 / 1,610, 131,072 3,270 / 2,990, 196,608 4,340 / 4,296, but 262,144
-  // 5,430-5,580 / 5,610-5,650: the time per plan of either falls as classes fill their wavefronts, that of the main kernel
-  // longer.  A batch of more than QUAD_DEEP_PLANS plans per compute unit stays there where the plans have more than
-  // QUAD_MEAN_NODES nodes on average.
+  // 1,015.  AC-share (152): 20,011 1,216 / 770, 65,536 2,350 / 1,610, 131,072 3,270 / 2,750, 196,608 4,340 / 3,330, 262,144
+  // 5,430 / 4,090.
+  // A deep batch has more than QUAD_DEEP_PLANS plans per compute unit, of more than QUAD_MEAN_NODES nodes on average.  There
+  // ready sets of up to 24 entries stay in k_quad: a wavefront of its largest form takes up to 1.5 ms, three times as long as any other
+  // kernel's task, which shows where the step is not several times that, but a plan in k_plan costs eight times what one of
+  // a full wavefront does.  And the launches go by LDS in up to QUAD_BINS bins a form.  (Neither / bins / both, us per step: AC-share
+  // 262,144 5,133 / 5,197 / 4,090, 131,072 2,767 / 2,727 / 2,650, 98,304 2,180 / - / 2,258, 65,536 1,486 / 1,464 / 2,012; GRPO 131,072, bins
+  // 472 / 609.)
+  bool deep = false;
   auto plan_quad = [&]() -> bool {
     if (!quad_free) return false;
     const DeepModel dm = deep_model(e, rcap_main);
@@ -1766,7 +1772,8 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       if (counts[c] >= QUAD_TINY) { takes += counts[c]; measured += e->cls_need[cids[c]] ? counts[c] : 0; }
       if (w) { t_sum += (double)(w >> 12); nodes_sum += (double)e->cls_nodes[cids[c]]; pops_sum += (w & 0xFFFu) / 16.0; ++known; }
     }
-    if (nodes > QUAD_MEAN_NODES * n && n > (uint64_t)e->n_cu * QUAD_DEEP_PLANS) return false;
+    deep = nodes > QUAD_MEAN_NODES * n && n > (uint64_t)e->n_cu * QUAD_DEEP_PLANS;
+    const uint32_t most_ready = QUAD_KIND[deep ? 2 : 1].entries;
     // (A batch of under two wavefronts of the main kernel per compute unit is not for that kernel, whatever it has measured:
     // k_plan with 64 plans per compute unit and the main kernel with 8 to 64 plans per wavefront beyond that / k_quad, us
     // per step: DPO 16,384 plans 194 / 137, 20,000 212 / 137; PPO 16,384 473 / 393; AC-share 16,384 1,030 / 850.)
@@ -1790,7 +1797,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       const double t0 = (double)(e->cls_pops16[cids[c]] >> 12), t = t0 > 0.0 ? t0 : per_node * (double)e->cls_nodes[cids[c]];
       if (counts[c] >= TINY_CLASS) { w_main += (double)((counts[c] + WAVE - 1) / WAVE) * t; max_main = std::max(max_main, t); }
       else base_plan += dm.plan_cost(counts[c], e->cls_nodes[cids[c]]);
-      to_plan[c] = counts[c] < QUAD_TINY || e->cls_need[cids[c]] > QUAD_KIND[1].entries || !e->cls_quad[cids[c]].rows;
+      to_plan[c] = counts[c] < QUAD_TINY || e->cls_need[cids[c]] > most_ready || !e->cls_quad[cids[c]].rows;
       if (to_plan[c]) w_plan += cost_plan(c);
       else w_quad += cost_quad(c);
     }
@@ -1821,16 +1828,18 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
                           n * 4 >= e->split_for_n * 3 && n * 3 <= e->split_for_n * 4 && e->batch_calls - e->split_at < 16 &&
                           e->split_mass == (mass != nullptr);
   if (keep_split) {
+    deep = e->split_deep;
     for (size_t c = 0; c < counts.size(); ++c) {
       const uint8_t a = cids[c] < e->cls_split.size() ? e->cls_split[cids[c]] : (uint8_t)255;
       if (a == 255 && e->split_quad) (counts[c] < QUAD_TINY || !e->cls_quad[cids[c]].rows ? solo[c] : quad[c]) = 1;
       else if (a == 255) solo[c] = counts[c] < TINY_CLASS ? 1 : 0;
       else if (a == 1) solo[c] = 1;
-      else if (a == 2) (e->cls_need[cids[c]] > QUAD_KIND[1].entries ? solo[c] : quad[c]) = 1;   // (as plan_quad would, once a ready set has outgrown sixteen entries)
+      else if (a == 2) (e->cls_need[cids[c]] > QUAD_KIND[deep ? 2 : 1].entries ? solo[c] : quad[c]) = 1;   // (as plan_quad would, once a ready set has outgrown its lanes)
     }
   } else if (!ls && !one && !quad_all && !order.empty() && (by_quad = plan_quad())) {
     // (decided: every class in k_quad, as far as its share goes, or, tiny classes and the largest graphs, in k_plan)
   } else if (!ls && !one && !quad_all && !order.empty()) {
+    deep = false;
     // The kernel ends with its slowest wavefront, and a wavefront is as slow as its slowest plan.  The
     // classes with the largest graphs (up to 15 % of the batch: beyond that the single-plan kernel would be
     // the one that ends last) are taken out of it, unless the batch is
@@ -1981,6 +1990,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     for (size_t c = 0; c < counts.size(); ++c) e->cls_split[cids[c]] = solo[c] ? 1 : quad[c] ? 2 : 0;
     e->split_for_n = n; e->split_at = e->batch_calls; e->split_mass = mass != nullptr;
     e->split_quad = by_quad;
+    e->split_deep = deep && by_quad;
     // a class that runs in the main kernel or in k_quad for the first time is measured by this launch: read it in the next call
     // (at most once in eight calls, so that a class whose measurement never arrives cannot keep the read-back on)
     bool unmeasured = false;
@@ -1998,41 +2008,69 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // The tasks of k_quad follow those of the main kernel: a launch for every form, each on a stream of its
   // own, and where a stream is left, one for the larger and one for the smaller graphs of a form -- the LDS of a launch is
   // that of its largest graph, and LDS bounds the wavefronts in flight.  The line lies where the sum over the tasks of
-  // time (nodes) times LDS is smallest.
-  struct QuadLaunch { uint32_t first = 0, waves = 0; QuadSize size; int kind = 0; } quad_launch[4];
+  // time (nodes) times LDS is smallest.  In a deep batch (plan_quad) up to QUAD_BINS launches a form, cut the same way one
+  // after the other, the one of the largest LDS on a stream of its own and the others by turns on two: a launch behind another
+  // waits for its slowest task.  (AC-share, us per step, 262,144 / 140,001 plans: 1 launch a form 5,560 / 3,127, 2 4,325 / 2,632, 3
+  // 4,090 / 2,754, 4 4,105 / 2,752; 3 with the last one alone on a stream 4,320 / 2,800, all of them on one 6,190 / 4,290.)
+  struct QuadLaunch { uint32_t first = 0, waves = 0; QuadSize size; int kind = 0; bool aside = false, first_stream = false; };   // on the fourth stream; on the main kernel's, where that has no tasks
+  std::vector<QuadLaunch> quad_launch;
+  bool aside = false;   // some launch is
   {
     auto waves_of = [&](uint32_t c, int kind) { return (counts[c] + QUAD_KIND[kind].plans - 1) / QUAD_KIND[kind].plans; };
+    std::vector<uint32_t> qc[3];
+    for (uint32_t c : order)   // (largest graphs first)
+      if (quad[c]) qc[quad_kind(c)].push_back(c);
     for (int kind : {2, 0, 1}) {
-      std::vector<uint32_t> qc;
-      double all = 0.0;
-      for (uint32_t c : order)   // (largest graphs first)
-        if (quad[c] && quad_kind(c) == kind) {
-          qc.push_back(c);
-          all += (double)waves_of(c, kind) * (double)e->cls_nodes[cids[c]];
-        }
-      size_t cut = qc.size();
-      if (kind != 2 && !quad_launch[2].waves && !quad_launch[3].waves && !qc.empty()) {
-        auto lds_of = [&](uint32_t c) { return (double)kq_lds_bytes(QUAD_KIND[kind].plans, e->cls_quad[cids[c]], mass != nullptr); };
-        double upto = 0.0, best = all * lds_of(qc[0]);
-        for (size_t k = 0; k + 1 < qc.size(); ++k) {
-          upto += (double)waves_of(qc[k], kind) * (double)e->cls_nodes[cids[qc[k]]];
-          if (e->cls_nodes[cids[qc[k]]] == e->cls_nodes[cids[qc[k + 1]]]) continue;
-          const double cost = upto * lds_of(qc[0]) + (all - upto) * lds_of(qc[k + 1]);
-          if (cost < 0.95 * best) { best = cost; cut = k + 1; }
-        }
+      std::vector<uint32_t>& q = qc[kind];
+      if (q.empty()) continue;
+      auto lds_of = [&](uint32_t c) { return (double)kq_lds_bytes(QUAD_KIND[kind].plans, e->cls_quad[cids[c]], mass != nullptr); };
+      std::vector<double> lds(q.size()), upto(q.size() + 1, 0.0);
+      if (deep) std::stable_sort(q.begin(), q.end(), [&](uint32_t x, uint32_t y) { return lds_of(x) > lds_of(y); });
+      for (size_t k = 0; k < q.size(); ++k) {
+        lds[k] = lds_of(q[k]);
+        upto[k + 1] = upto[k] + (double)waves_of(q[k], kind) * (double)e->cls_nodes[cids[q[k]]];
       }
-      for (size_t k = 0; k < qc.size(); ++k) {
-        const uint32_t c = qc[k];
-        QuadLaunch& q = quad_launch[k < cut ? kind : 3];
-        clpw[c] = QUAD_KIND[kind].plans;
-        n_quad_plans += counts[c];
-        first[c] = n_eval_waves + n_quad_waves;
-        const uint32_t nw = waves_of(c, kind);
-        if (!q.waves) { q.first = n_quad_waves; q.kind = kind; }
-        q.waves += nw;
-        q.size.fit(e->cls_quad[cids[c]]);
-        n_quad_waves += nw;
+      std::vector<size_t> cuts = {0, q.size()};
+      const size_t most = deep ? QUAD_BINS : kind != 2 && !aside ? 2 : 1;
+      while (cuts.size() <= most) {
+        double best = 0.05 * upto.back() * lds[0];
+        size_t at = 0;
+        for (size_t i = 0; i + 1 < cuts.size(); ++i)
+          for (size_t k = cuts[i] + 1; k < cuts[i + 1]; ++k) {
+            if (deep ? lds[k] == lds[k - 1] : e->cls_nodes[cids[q[k]]] == e->cls_nodes[cids[q[k - 1]]]) continue;
+            const double gain = (upto[cuts[i + 1]] - upto[k]) * (lds[cuts[i]] - lds[k]);
+            if (gain > best) { best = gain; at = k; }
+          }
+        if (!at) break;
+        cuts.insert(std::upper_bound(cuts.begin(), cuts.end(), at), at);
       }
+      for (size_t i = 0; i + 1 < cuts.size(); ++i) {
+        QuadLaunch l;
+        l.first = n_quad_waves;
+        l.kind = kind;
+        l.aside = kind == 2 || i > 0;
+        l.first_stream = kind == 0;
+        for (size_t k = cuts[i]; k < cuts[i + 1]; ++k) {
+          const uint32_t c = q[k];
+          clpw[c] = QUAD_KIND[kind].plans;
+          n_quad_plans += counts[c];
+          first[c] = n_eval_waves + n_quad_waves;
+          const uint32_t nw = waves_of(c, kind);
+          l.waves += nw;
+          l.size.fit(e->cls_quad[cids[c]]);
+          n_quad_waves += nw;
+        }
+        aside = aside || l.aside;
+        quad_launch.push_back(l);
+      }
+    }
+    if (deep) {   // the largest on a stream of its own, the others by turns on two
+      std::stable_sort(quad_launch.begin(), quad_launch.end(), [&](const QuadLaunch& x, const QuadLaunch& y) {
+        return kq_lds_bytes(QUAD_KIND[x.kind].plans, x.size, mass != nullptr) > kq_lds_bytes(QUAD_KIND[y.kind].plans, y.size, mass != nullptr); });
+      for (size_t k = 0; k < quad_launch.size(); ++k) { quad_launch[k].first_stream = k == 0; quad_launch[k].aside = k % 2 == 1; }
+      aside = quad_launch.size() > 1;
+    } else {   // the smaller graphs of a form last
+      std::stable_partition(quad_launch.begin(), quad_launch.end(), [](const QuadLaunch& x) { return x.kind == 2 || !x.aside; });
     }
   }
   {   // the ranks of a wavefront all at once, where the launches' wavefronts find room together all the same; else of half
@@ -2293,12 +2331,10 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // stream where it is free, else behind k_quad's first launch (behind k_plan they ended the call: 65,536 GRPO plans
   // 365 against 353 us, 20,011 PPO plans 409 against 381).
   const bool peaks_apart = peaks_deferred && !peaks_aside && !n_waves, peaks_on_s2 = peaks_apart && n_solo && n_solo <= (uint32_t)e->n_cu;
-  const bool quad_on_s4 = quad_launch[2].waves || quad_launch[3].waves, peaks_on_s4 = peaks_apart && !peaks_on_s2 && !quad_on_s4;
-  if (quad_on_s4 || peaks_on_s4) HIP_TRY(e, hipStreamWaitEvent(e->s4, e->ev_fork, 0));
-  if (int rc = launch_quad(quad_launch[2], e->s4)) return rc;
-  if (int rc = launch_quad(quad_launch[0], n_waves ? sq : sm)) return rc;   // (beside the main kernel, where that has tasks)
-  if (int rc = launch_quad(quad_launch[1], sq)) return rc;
-  if (int rc = launch_quad(quad_launch[3], e->s4)) return rc;
+  const bool peaks_on_s4 = peaks_apart && !peaks_on_s2 && !aside;
+  if (aside || peaks_on_s4) HIP_TRY(e, hipStreamWaitEvent(e->s4, e->ev_fork, 0));
+  for (const QuadLaunch& q : quad_launch)
+    if (int rc = launch_quad(q, q.aside ? e->s4 : q.first_stream && !n_waves ? sm : sq)) return rc;   // (beside the main kernel, where that has tasks)
   if (n_solo) {   // the single-plan wavefronts, beside the main kernel
     HIP_TRY(e, hipStreamWaitEvent(e->s2, e->ev_fork, 0));
     EvalLaunch S = L;
@@ -2342,7 +2378,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     ahead_join.joined = true;
   }
   if (n_solo) HIP_TRY(e, hipStreamWaitEvent(s, e->ev_join, 0));
-  if (quad_on_s4 || peaks_on_s4) {
+  if (aside || peaks_on_s4) {
     HIP_TRY(e, hipEventRecord(e->ev_join4, e->s4));
     HIP_TRY(e, hipStreamWaitEvent(s, e->ev_join4, 0));
   }
