@@ -477,12 +477,12 @@ int rpeg_engine_host_us(const rpeg_engine_t* e, double* out, int32_t n);
 int rpeg_engine_set_state_lanes(rpeg_engine_t* e, int32_t lanes);
 
 /* The ten fitted figures by which a full batch is split between the three scheduling kernels (microseconds of a
-   wavefront on an MI355X): cost of a plan in the one-plan-per-wavefront kernel a + b x nodes (12, 0.9); of a wavefront
+   wavefront on an MI355X): cost of a plan in the one-plan-per-wavefront kernel a + b x nodes (9, 0.8); of a wavefront
    of the kernel of two or four lanes per plan a + nodes x (b + c x heap pops per dispatch) (10, 1.3, 0.2); the share of
    a compute unit that the former really gets beside the latter (0.65); how much later the main kernel must end for a
    batch to move to the kernel of two or four lanes per plan (1.15); the modelled gain that a split by class size (0.97) and by
    measured time (0.98) must reach; and, where ten values are given (with nine it stays as it is), how many times as much
-   a plan of more than 128 nodes costs the one-plan-per-wavefront kernel (1.2).  A measurement aid: the figures decide
+   a plan of more than 128 nodes costs the one-plan-per-wavefront kernel (1.25).  A measurement aid: the figures decide
    where a plan is evaluated, never what the result is.  No counterpart in the reference. */
 int rpeg_engine_set_split_model(rpeg_engine_t* e, const double* values, int32_t n);
 

@@ -693,7 +693,9 @@ static uint8_t* static_scratch_ptr(int dev, hipError_t* st) {
 
 // The fitted figures behind the split of a full batch between the three scheduling kernels, in one place.  They are
 // microseconds of one wavefront on an MI355X, fitted to the per-wavefront clocks of configurations 2, 3 and 5
-// (python -m rpeg_amd.engine.profile) and then to the step time of configuration 2 over a sweep of each figure;
+// (python -m rpeg_amd.engine.profile) and then to the step time of configuration 2 over a sweep of each figure (what a plan costs
+// k_plan: of eight batches; 12, 0.9, 1.2 / 9, 0.8, 1.25, us per step: 17,000 GRPO plans 263 / 251, 20,011 AC-share 735 / 692, six others
+// within 1 %);
 // rpeg_engine_set_split_model replaces them (a measurement aid).  A wrong figure
 // costs time, never a result: every kernel computes the same bits.
 //   plan_a + plan_b x nodes                    what a plan costs k_plan (one plan per wavefront), beside the main kernel;
@@ -706,7 +708,7 @@ static uint8_t* static_scratch_ptr(int dev, hipError_t* st) {
 //   quad_margin                                a batch moves to k_quad only if the main kernel would end this much later
 //   gain_threshold, gain_classes               a split by class size / by measured time must model this much earlier
 struct SplitModel {
-  double plan_a = 12.0, plan_b = 0.9, plan_list = 1.2;
+  double plan_a = 9.0, plan_b = 0.8, plan_list = 1.25;
   double quad_a = 10.0, quad_b = 1.3, quad_c = 0.2;
   double eff_beside_quad = 0.65;
   double quad_margin = 1.15;

@@ -67,8 +67,8 @@ struct QuadSize {
     rows = o.rows > rows ? o.rows : rows; types = o.types > types ? o.types : types;
   }
 };
-// LDS of one wavefront.  Class tables: per node four successor words, its own, and its level place's id; the first place of
-// every level.  Per plan [row][plan]: durations, availability by vertex with a row of zeros and one nobody reads, ready-time
+// LDS of one wavefront.  Class tables: per node four successor words, its own, its level place's id and its place in its chain.
+// Per plan [row][plan]: durations, availability by vertex with a row of zeros and one nobody reads, ready-time
 // rows -- over these two, before they are needed, the ranks of all, half or a quarter of the plans --, with the critical-chain masses finish
 // and start times, a state word and a reservation each.
 __host__ __device__ inline size_t kq_tab_bytes(uint32_t nodes) { return (20ull * nodes + 2 * 2ull * (nodes + 2) + 15) & ~size_t(15); }
