@@ -35,10 +35,10 @@ ALG_FLOPS = {1: 3697.0, 2: 2165.3, 3: 6502.9, 4: 1245.8, 5: 4155.6}
 # (FETCH_SIZE / WRITE_SIZE scaled by a 256 MiB copy) and instructions issued per plan (SQ_INSTS_VALU + SALU + LDS +
 # VMEM_RD + VMEM_WR of the evaluation kernels / plans).
 MEASURED = {
-    1: dict(layout=(4096, 7168, 1, 0, 0), traffic=17.0e6, instructions_per_plan=16321.0),
-    2: dict(layout=(4101, 21536, 0, 1524, 2577), traffic=89.3e6, instructions_per_plan=1414.0),
-    3: dict(layout=(26010, 29984, 0, 21725, 0), traffic=4483.7e6, instructions_per_plan=7309.0),
-    4: dict(layout=(32781, 14640, 0, 6, 32775), traffic=357.4e6, instructions_per_plan=None),
+    1: dict(layout=(4096, 7168, 1, 0, 0), traffic=18.4e6, instructions_per_plan=13257.0),
+    2: dict(layout=(4129, 21536, 0, 1554, 2575), traffic=90.2e6, instructions_per_plan=1506.0),
+    3: dict(layout=(29518, 29984, 0, 13209, 16309), traffic=845.0e6, instructions_per_plan=6189.0),
+    4: dict(layout=(32781, 14640, 0, 6, 32775), traffic=358.0e6, instructions_per_plan=464.0),
 }
 
 
