@@ -155,14 +155,15 @@ int port_lower(void* h, const int16_t* vert, const uint8_t* head, int32_t* kind,
   return n;
 }
 
-// the blob of a class and its edges: from the object that lowers one class after the other, or from one of its own
-long port_blob(void* h, uint64_t sig, int own, uint8_t* out, long cap, int32_t* edges, int32_t* n_edges) {
+// the blob of a class and its edges: from the object that lowers one class after the other, or from one of its own; with what
+// k_quad keeps of it or without
+long port_blob(void* h, uint64_t sig, int own, int few_lanes, uint8_t* out, long cap, int32_t* edges, int32_t* n_edges) {
   Port* e = (Port*)h;
   LoweredClass mine;
   const LoweredClass* lc = &mine;
   try {
-    if (own) mine = lower_class(e->P, sig);
-    else { e->low->run(sig); lc = &e->low->out; }
+    if (own) mine = lower_class(e->P, sig, few_lanes != 0);
+    else { e->low->run(sig, few_lanes != 0); lc = &e->low->out; }
   } catch (const std::exception& ex) { e->err = ex.what(); return -2; }
   if ((long)lc->blob.size() > cap || (long)lc->edges.size() * 8 > cap) return -3;
   std::memcpy(out, lc->blob.data(), lc->blob.size());

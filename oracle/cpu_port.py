@@ -47,7 +47,7 @@ def lib():
         _lib.port_lower.restype = C.c_int
         _lib.port_lower.argtypes = [C.c_void_p] * 9 + [C.c_int32, C.c_void_p]
         _lib.port_blob.restype = C.c_long
-        _lib.port_blob.argtypes = [C.c_void_p, C.c_uint64, C.c_int, C.c_void_p, C.c_long, C.c_void_p, C.c_void_p]
+        _lib.port_blob.argtypes = [C.c_void_p, C.c_uint64, C.c_int, C.c_int, C.c_void_p, C.c_long, C.c_void_p, C.c_void_p]
         _lib.port_op_time.restype = C.c_int
         _lib.port_op_time.argtypes = [C.c_void_p, C.c_uint64, C.c_int, C.c_int, C.c_void_p, C.c_uint64,
                                       C.c_void_p, C.c_void_p]
@@ -101,10 +101,11 @@ class CpuPort:
         return dict(kind=kind[:n], vertex=vertex[:n], step=step[:n], sub=sub[:n], dur=dur[:n],
                     edges=edges[:2 * ne.value].reshape(-1, 2))
 
-    def blob(self, sig, own=False, cap=1 << 20):
-        """(blob bytes, edges) of the class of a signature; own: from a lowering object that has lowered nothing else."""
+    def blob(self, sig, own=False, cap=1 << 20, few_lanes=True):
+        """(blob bytes, edges) of the class of a signature; own: from a lowering object that has lowered nothing else;
+        few_lanes: with what k_quad keeps of it."""
         out, edges, ne = np.zeros(cap, np.uint8), np.zeros(cap // 4, np.int32), C.c_int32(0)
-        n = lib().port_blob(self.h, int(sig), int(own), out.ctypes.data, cap, edges.ctypes.data, C.addressof(ne))
+        n = lib().port_blob(self.h, int(sig), int(own), int(few_lanes), out.ctypes.data, cap, edges.ctypes.data, C.addressof(ne))
         if n < 0:
             raise RuntimeError(f"port_blob failed ({n}): {lib().port_error(self.h).decode()}")
         return out[:n].copy(), edges[:2 * ne.value].reshape(-1, 2).copy()

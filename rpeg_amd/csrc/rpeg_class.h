@@ -112,7 +112,7 @@ struct ClassHdr {
   uint32_t bytes;
   uint32_t structure, split, error;  // error != 0: the reference would raise for this class
   uint32_t id;                       // index of the class in the tables of the engine that holds it (0 elsewhere)
-  uint32_t n_rows, n_types, off_qrec, off_type;   // what k_quad keeps per plan: ready-time rows and reservations (QuadRec); n_rows 0: not for that kernel
+  uint32_t n_rows, n_types, off_qrec, off_type;   // what k_quad keeps per plan: ready-time rows and reservations (QuadRec); n_rows 0: not for that kernel, or lowered without (Lowering::run)
   uint8_t vorder[8];                 // vertices by first appearance among the lowered operator nodes
 };
 

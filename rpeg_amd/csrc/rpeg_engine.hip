@@ -747,7 +747,8 @@ struct rpeg_engine_s {
   std::unordered_map<uint64_t, uint32_t> class_off;  // signature -> byte offset in the pool
   std::vector<uint64_t> cls_sig;                     // class id -> signature / pool offset / node count
   std::vector<uint32_t> cls_off, cls_nodes;
-  std::vector<QuadSize> cls_quad;                    // what k_quad's LDS needs for the class; no rows: it is not for that kernel
+  std::vector<QuadSize> cls_quad;                    // what k_quad's LDS needs for the class; no rows: it is not for that kernel,
+  std::vector<uint8_t> cls_few;                      // or (0) lowered without what that kernel keeps (Lowering::run)
   QuadSize max_quad;                                 // the largest of them
   std::vector<uint32_t> cls_pops16;                  // learned, of the slowest full wavefront of the class in the main kernel:
                                                      // microseconds << 12 | heap pops per dispatch in sixteenths
@@ -1031,8 +1032,15 @@ static bool pool_room(rpeg_engine_t* e, size_t bytes) {
   return false;
 }
 
+// what k_quad keeps of class c, lowered with it (`few`) or not
+static void class_few(rpeg_engine_t* e, uint32_t c, const ClassHdr* h, bool few) {
+  e->cls_quad[c] = QuadSize{h->n_nodes, h->n_slots, h->n_rows, h->n_types};
+  e->cls_few[c] = few ? 1 : 0;
+  e->max_quad.fit(e->cls_quad[c]);
+}
+
 // enters a lowered class, whose blob lies at pool offset `off` (and still in host memory at `blob`), in the engine's tables
-static void class_append(rpeg_engine_t* e, uint64_t sig, uint8_t* blob, size_t off) {
+static void class_append(rpeg_engine_t* e, uint64_t sig, uint8_t* blob, size_t off, bool few) {
   ClassHdr* h = (ClassHdr*)blob;
   e->max_nodes = std::max(e->max_nodes, h->n_nodes);
   e->max_slots = std::max(e->max_slots, h->n_slots);
@@ -1042,20 +1050,20 @@ static void class_append(rpeg_engine_t* e, uint64_t sig, uint8_t* blob, size_t o
   e->cls_sig.push_back(sig);
   e->cls_off.push_back((uint32_t)off);
   e->cls_nodes.push_back(h->n_nodes);
-  const QuadSize quad_size{h->n_nodes, h->n_slots, h->n_rows, h->n_types};
-  e->cls_quad.push_back(quad_size);
-  e->max_quad.fit(quad_size);
+  e->cls_quad.emplace_back();
+  e->cls_few.push_back(0);
+  class_few(e, h->id, h, few);
   e->cls_pops16.push_back(0);
   e->cls_need.push_back(0);
   e->learn_calls = 3;
 }
 
-// returns the pool offset of the class of `sig`, lowering it on first sight (*is_new; e->low->out then holds it); -1 on failure
+// returns the pool offset of the class of `sig`, lowering it on first sight (*is_new; e->low->out then holds it), for k_plan; -1 on failure
 static int64_t class_offset(rpeg_engine_t* e, uint64_t sig, bool* is_new) {
   auto it = e->class_off.find(sig);
   if (it != e->class_off.end()) return it->second;
   try {
-    e->low->run(sig);
+    e->low->run(sig, false);
   } catch (const std::exception& ex) {
     e->err = std::string("lowering failed: ") + ex.what();
     return -1;
@@ -1068,20 +1076,14 @@ static int64_t class_offset(rpeg_engine_t* e, uint64_t sig, bool* is_new) {
   rpeg_engine_s::Fresh& f = e->n_fresh ? e->fresh[e->n_fresh - 1] : pool_stretch(e);
   f.bytes.insert(f.bytes.end(), blob.begin(), blob.end());
   e->pool_size += blob.size();
-  class_append(e, sig, f.bytes.data() + (off - f.off), off);
+  class_append(e, sig, f.bytes.data() + (off - f.off), off, false);
   return (int64_t)off;
 }
 
-// lowers the classes of `sigs` that the engine does not hold yet, on up to eight host threads (lowering a
-// class reads only the problem tables), and appends them in the order of `sigs`
-static int lower_new_classes(rpeg_engine_t* e, const std::vector<uint64_t>& sigs, uint64_t* n_new) {
-  std::vector<uint64_t> todo;
-  {
-    std::unordered_map<uint64_t, char> seen;
-    for (uint64_t sg : sigs)
-      if (!e->class_off.count(sg) && seen.emplace(sg, 1).second) todo.push_back(sg);
-  }
-  if (todo.empty()) return 0;
+// Lowers the classes of `todo` on up to eight host threads (lowering a class reads only the problem tables) into the pool;
+// done(i, blob, offset) for each, in their order.  0, -5 with e->err.
+template <class DONE>
+static int lower_classes(rpeg_engine_t* e, const std::vector<uint64_t>& todo, bool few, DONE done) {
   struct Blob { size_t thread, off; };   // where a class was left: in its thread's stretch of the pool
   std::vector<Blob> lowered(todo.size());
   std::vector<std::string> errors(todo.size());
@@ -1094,7 +1096,7 @@ static int lower_new_classes(rpeg_engine_t* e, const std::vector<uint64_t>& sigs
     std::vector<uint8_t>& bytes = e->fresh[first + t].bytes;
     for (size_t i = t; i < todo.size(); i += n_threads) {
       try {
-        low.run(todo[i]);
+        low.run(todo[i], few);
         lowered[i] = {t, bytes.size()};
         bytes.insert(bytes.end(), low.out.blob.begin(), low.out.blob.end());
       } catch (const std::exception& ex) { errors[i] = ex.what(); if (errors[i].empty()) errors[i] = "error"; }
@@ -1122,11 +1124,43 @@ static int lower_new_classes(rpeg_engine_t* e, const std::vector<uint64_t>& sigs
       continue;
     }
     rpeg_engine_s::Fresh& f = e->fresh[first + lowered[i].thread];
-    class_append(e, todo[i], f.bytes.data() + lowered[i].off, f.off + lowered[i].off);
+    done(i, f.bytes.data() + lowered[i].off, f.off + lowered[i].off);
   }
-  if (rc) return rc;
+  return rc;
+}
+
+// lowers the classes of `sigs` that the engine does not hold yet and appends them in the order of `sigs`
+static int lower_new_classes(rpeg_engine_t* e, const std::vector<uint64_t>& sigs, bool few, uint64_t* n_new) {
+  std::vector<uint64_t> todo;
+  {
+    std::unordered_map<uint64_t, char> seen;
+    for (uint64_t sg : sigs)
+      if (!e->class_off.count(sg) && seen.emplace(sg, 1).second) todo.push_back(sg);
+  }
+  if (todo.empty()) return 0;
+  if (int rc = lower_classes(e, todo, few, [&](size_t i, uint8_t* blob, size_t off) { class_append(e, todo[i], blob, off, few); })) return rc;
   *n_new += todo.size();
   return 0;
+}
+
+// Lowers once more, with what k_quad keeps, those of the classes `cids` that calls for k_plan have met first.  The longer
+// blob takes the class's place; the one before it stays in the pool, where launches under way and the device's table of
+// offsets may still name it (k_plan reads the same of either).  A class for which the pool has no room is not for k_quad.
+static void lower_for_quad(rpeg_engine_t* e, const std::vector<uint32_t>& cids) {
+  std::vector<uint32_t> which;
+  std::vector<uint64_t> todo;
+  for (uint32_t c : cids)
+    if (!e->cls_few[c]) { which.push_back(c); todo.push_back(e->cls_sig[c]); }
+  if (todo.empty()) return;
+  if (lower_classes(e, todo, true, [&](size_t i, uint8_t* blob, size_t off) {
+        ClassHdr* h = (ClassHdr*)blob;
+        const uint32_t c = which[i];
+        h->id = c;
+        e->class_off[todo[i]] = e->cls_off[c] = (uint32_t)off;
+        class_few(e, c, h, true);
+      }))
+    e->err.clear();
+  for (uint32_t c : which) e->cls_few[c] = 1;
 }
 
 static int ensure_ws(rpeg_engine_t* e, size_t bytes, hipStream_t s) {
@@ -1348,6 +1382,7 @@ int rpeg_engine_reset_classes(rpeg_engine_t* e) {
   e->cls_off.clear();
   e->cls_nodes.clear();
   e->cls_quad.clear();
+  e->cls_few.clear();
   e->max_quad = QuadSize();
   e->cls_pops16.clear();
   e->cls_need.clear();
@@ -1579,6 +1614,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // classes of the batch: every plan looks its class id up on the device and counts itself; only the
   // per-class counts come back.  Plans of classes not lowered yet make the call take the slow round:
   // their signatures are read back, the classes are lowered on the host, the tables are rebuilt.
+  const bool for_quad = !own_prologue && (e->state_lanes == 4 || (e->state_lanes == -1 && e->quad_share_pct && e->split_heavy));
   uint64_t n_new = 0;
   uint32_t ncls = 0, shards = 1;
   for (int round = 0;; ++round) {
@@ -1660,13 +1696,14 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       last_sig = sg;
       sigs.push_back(sg);
     }
-    if (int rc = lower_new_classes(e, sigs, &n_new)) return rc;
+    if (int rc = lower_new_classes(e, sigs, for_quad, &n_new)) return rc;
   }
   ++e->batch_calls;
   std::vector<uint32_t> offs, counts, cids;   // the classes present in this batch
+  uint64_t n_valid = 0;
   for (uint32_t c = 0; c < ncls; ++c) {
     const uint32_t total = e->h_tot[c];
-    if (total) { cids.push_back(c); offs.push_back(e->cls_off[c]); counts.push_back(total); }
+    if (total) { cids.push_back(c); counts.push_back(total); n_valid += total; }
   }
   // Plans per wavefront and where their scheduler state lives.  A full batch keeps 64 plans per wavefront
   // with the state in the HBM workspace; a batch too small to fill the chip that way is spread over more
@@ -1675,6 +1712,8 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   bool one = false;   // one plan per wavefront (k_plan)
   const bool quad_free = ls == -1 && e->quad_share_pct && e->split_heavy && plan_fits();   // k_quad may take the batch (plan_quad)
   const bool quad_all = ls == 4;   // every class in the kernel of two or four lanes per plan (k_quad), but one that its fields do not hold (QuadRec)
+  if (quad_all || (quad_free && n_valid > (uint64_t)e->n_cu * e->one_plan_waves_per_cu)) lower_for_quad(e, cids);
+  for (uint32_t c : cids) offs.push_back(e->cls_off[c]);
   if (quad_all) {
     ls = 0;
     if (kq_lds_bytes(16, e->max_quad, mass != nullptr) > 160 * 1024 || e->max_nodes > QUAD_NODES + 1) {
@@ -2576,7 +2615,7 @@ int rpeg_eval_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t*
   bool lowered = false;
   const int64_t off = class_offset(e, sg, &lowered);
   if (off < 0) return -5;
-  if (!lowered) try { e->low->run(sg); } catch (const std::exception& ex) { e->err = ex.what(); return -5; }
+  if (!lowered) try { e->low->run(sg, false); } catch (const std::exception& ex) { e->err = ex.what(); return -5; }
   const int n = (int)lc.nodes.size();
   if (n > cap || (edges && (int)lc.edges.size() > cap)) { e->err = "trace arrays too small"; return -7; }
   hipStream_t s = nullptr;
@@ -2640,7 +2679,7 @@ int rpeg_lower_plan(const rpeg_problem_t* problem, const int16_t* vert_fields, c
   for (int v = 0; v < st.n_vertex; ++v) load_vertex(vert_fields, 1, 0, v, &a[v]);
   const uint64_t sg = plan_signature(*problem, h.structure, h.split, h.tau0, h.tau1, a);
   LoweredClass lc;
-  try { lc = lower_class(*problem, sg); } catch (const std::exception&) { return -5; }
+  try { lc = lower_class(*problem, sg, false); } catch (const std::exception&) { return -5; }
   const int n = (int)lc.nodes.size();
   if (n > cap || (edges && (int)lc.edges.size() > cap)) return -7;
   describe_nodes(*problem, st, h, a, lc, node_kind, node_vertex, node_step, node_sub, node_src, node_payload, node_ref);
@@ -2665,7 +2704,7 @@ int rpeg_plan_detail(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_t
   bool lowered = false;
   const int64_t off = class_offset(e, sg, &lowered);
   if (off < 0) return -5;
-  if (!lowered) try { e->low->run(sg); } catch (const std::exception& ex) { e->err = ex.what(); return -5; }
+  if (!lowered) try { e->low->run(sg, false); } catch (const std::exception& ex) { e->err = ex.what(); return -5; }
   const LoweredClass& lc = e->low->out;
   const int n = (int)lc.nodes.size();
   if ((node_time || node_payload || node_ref) && n > cap) { e->err = "node arrays too small"; return -7; }
@@ -3011,7 +3050,7 @@ static int host_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_
   if (rc) return rc == 1 ? -8 : rc;
   // while the launch runs: what the records of the nodes hold
   const LoweredClass& lc = e->low->out;
-  if (!lowered) try { e->low->run(sg); lowered = true; } catch (const std::exception& ex) { e->err = ex.what(); }
+  if (!lowered) try { e->low->run(sg, false); lowered = true; } catch (const std::exception& ex) { e->err = ex.what(); }
   const int n = (int)lc.nodes.size();
   if (lowered && n <= cap) {
     describe_nodes(e->P, st, h, a, lc, node_kind, node_vertex, node_step, node_sub, node_src, node_payload, node_ref);

@@ -104,19 +104,23 @@ struct LoweredClass {
 // the problem's tables, an edge is looked for among its source's few successors, and the blob's records are written where
 // they belong.  us per class (one core of a 2.7 GHz host; with arrays of its own for every class, slots and universe searched
 // linearly and an open-addressing table of edges -> now): PPO, 84 nodes 11.4 -> 6.0; GRPO, 47 nodes 6.2 -> 3.2; AC-share,
-// 150 nodes 16.0 -> 9.1; PPO of 4 steps, 91 nodes 11.2 -> 5.7.
+// 150 nodes 16.0 -> 9.1; PPO of 4 steps, 91 nodes 11.2 -> 5.7.  With what k_quad keeps (few_lanes): 6.7, 3.4, 11.0 and 6.7.
 class Lowering {
  public:
   LoweredClass out;
 
   Lowering(const rpeg_problem_t& problem, const LowerTables& tables) : P(problem), T(tables) {}
 
-  void run(uint64_t sig_bits) {
+  // few_lanes: with what only k_quad reads of a class (QuadRec), a sixth to a fifth of the rest in time, a tenth in bytes.
+  // The calls that give every plan a wavefront lower without it, on the calling thread (the first pass on 100 new PPO plans
+  // 378 -> 340 us, on 41 AC-share plans 634 -> 561); a class that they have met first is lowered once more when it comes up in a
+  // batch for k_quad.
+  void run(uint64_t sig_bits, bool few_lanes = true) {
     const int s = (int)(sig_bits & 3);
     const SigView sg{&P.st[s], &T.st[s], sig_bits};
     if (T.st[s].n_uni > RPEG_MAX_UNIVERSE) throw std::runtime_error("slot universe too large");
     graph(sg);
-    blob(sg);
+    blob(sg, few_lanes);
   }
 
  private:
@@ -134,50 +138,71 @@ class Lowering {
   std::vector<Tr> to_train, to_serving;
   // and what the blob needs of it
   std::vector<int> adj_beg, adj_to, indeg, deg, cur, topo, chain_beg, chain_of, level, place, chain_n, chain_i, lbeg;
+  // and what k_quad keeps of it (few_lanes)
   std::vector<uint64_t> anc, row_pred;        // a bit each: per node its ancestors; per row the predecessors of the last node that has it
   std::vector<int> row_of;                    // per node: its ready-time row
-  std::vector<uint16_t> types, type_of;
+  std::vector<uint16_t> types;
+  std::vector<uint8_t> type_of;               // per node
+  uint8_t type_at[RPEG_MAX_V * 8 + 1][1 << RPEG_MAX_V] = {};   // (cond, blocked) -> type + 1; all zero between classes
   int n_rows = 0;
+  // Reservation types and ready-time rows (QuadRec); false where they outgrow its fields.  W: words of a set of nodes.
+  template <int W>
   bool quad_rows(const NodeRec* recs, const uint16_t* pbeg, const uint16_t* pred, int n) {
-    if (n > (int)QUAD_NODES || (int)topo.size() != n) return false;
-    const int W = (n + 63) / 64;
-    anc.assign((size_t)n * W, 0);
-    row_pred.assign(W, 0);
-    row_of.assign(n, 0); types.clear(); type_of.resize(n);
+    anc.resize((size_t)n * W);   // (in topological order a node's set is written before it is read)
+    row_pred.resize((size_t)(QUAD_ROWS + 1) * W);
+    row_of.assign(n, 0); type_of.resize(n);
     n_rows = 1;
     for (int v : topo) {
-      uint64_t* const a = &anc[(size_t)v * W];
-      const int b = pbeg[v], d = pbeg[v + 1] - b;
-      const uint16_t t = (uint16_t)(recs[v].blocked | recs[v].cond << 8);
-      size_t k = 0;
-      while (k < types.size() && types[k] != t) ++k;
-      if (k == types.size()) types.push_back(t);
-      type_of[v] = (uint16_t)k;
-      if (recs[v].indeg > QUAD_INDEG || types.size() > QUAD_TYPES) return false;
-      uint64_t common[(QUAD_NODES + 64) / 64];   // the ancestors that all predecessors have
-      if (d) std::memcpy(common, &anc[(size_t)pred[b] * W], (size_t)W * 8);
-      if (d) std::memcpy(a, common, (size_t)W * 8);
-      for (int j = 1; j < d; ++j) {
-        const uint64_t* const p = &anc[(size_t)pred[b + j] * W];
-        for (int w = 0; w < W; ++w) { a[w] |= p[w]; common[w] &= p[w]; }
+      uint8_t& type = type_at[recs[v].cond][recs[v].blocked];
+      if (!type) {
+        types.push_back((uint16_t)(recs[v].blocked | recs[v].cond << 8));
+        type = (uint8_t)types.size();
       }
-      for (int j = 0; j < d; ++j) a[pred[b + j] >> 6] |= 1ull << (pred[b + j] & 63);
+      type_of[v] = (uint8_t)(type - 1);
+      if (recs[v].indeg > QUAD_INDEG || types.size() > QUAD_TYPES) return false;
+      uint64_t* const a = &anc[(size_t)v * W];
+      const uint16_t* const p = pred + pbeg[v];
+      const int d = recs[v].indeg;
+      if (d == 0) { for (int w = 0; w < W; ++w) a[w] = 0; continue; }
+      uint64_t all[W], common[W], own[W] = {};   // ancestors that some predecessor has, and that all have; the predecessors
+      for (int w = 0; w < W; ++w) all[w] = common[w] = anc[(size_t)p[0] * W + w];
+      own[p[0] >> 6] |= 1ull << (p[0] & 63);
+      for (int j = 1; j < d; ++j) {
+        const uint64_t* const x = &anc[(size_t)p[j] * W];
+        for (int w = 0; w < W; ++w) { all[w] |= x[w]; common[w] &= x[w]; }
+        own[p[j] >> 6] |= 1ull << (p[j] & 63);
+      }
+      for (int w = 0; w < W; ++w) a[w] = all[w] | own[w];
       if (d < 2) continue;
       int r = 1;
       for (; r < n_rows; ++r) {
-        const uint64_t* const x = &row_pred[(size_t)r * W];
-        int w = 0;
-        while (w < W && !(x[w] & ~common[w])) ++w;
-        if (w == W) break;
+        uint64_t missing = 0;
+        for (int w = 0; w < W; ++w) missing |= row_pred[(size_t)r * W + w] & ~common[w];
+        if (!missing) break;
       }
       if (r > (int)QUAD_ROWS) return false;
-      if (r == n_rows) row_pred.resize((size_t)++n_rows * W);
-      uint64_t* const x = &row_pred[(size_t)r * W];
-      std::fill(x, x + W, 0);
-      for (int j = 0; j < d; ++j) x[pred[b + j] >> 6] |= 1ull << (pred[b + j] & 63);
+      n_rows = std::max(n_rows, r + 1);
+      for (int w = 0; w < W; ++w) row_pred[(size_t)r * W + w] = own[w];
       row_of[v] = r;
     }
     return true;
+  }
+  bool quad_rows(const NodeRec* recs, const uint16_t* pbeg, const uint16_t* pred, int n) {
+    static_assert(QUAD_NODES < 8 * 64, "sets of up to eight words");
+    types.clear();
+    if (n > (int)QUAD_NODES || (int)topo.size() != n) return false;
+    const auto f = [&] {
+      switch ((n + 63) / 64) {
+        case 0: case 1: return quad_rows<1>(recs, pbeg, pred, n);
+        case 2: return quad_rows<2>(recs, pbeg, pred, n);
+        case 3: return quad_rows<3>(recs, pbeg, pred, n);
+        case 4: return quad_rows<4>(recs, pbeg, pred, n);
+        default: return quad_rows<8>(recs, pbeg, pred, n);
+      }
+    };
+    const bool fits = f();
+    for (uint16_t t : types) type_at[t >> 8][t & 0xFFu] = 0;
+    return fits;
   }
 
   int slot(const SigView& sg, SlotType t, int a, int b, int q) {
@@ -391,7 +416,7 @@ class Lowering {
       }
     }
   }
-  void blob(const SigView& sg) {
+  void blob(const SigView& sg, bool few_lanes) {
     const rpeg_struct_t& st = *sg.st;
     const int nv = st.n_vertex, K = P.K_eval, split = sg.split();
     const int nph = split > 0 ? P.n_phase[split] : 0;
@@ -503,9 +528,11 @@ class Lowering {
     h.off_lbeg = (uint32_t)off; off = align8(off + lbeg.size() * 2);
     h.off_place = (uint32_t)off; off = align8(off + (size_t)n * 2);
     h.off_glvl = (uint32_t)off; off = align8(off + (size_t)n_gm * 2);
-    h.off_qrec = (uint32_t)off; off = align8(off + (size_t)n * 4);
+    h.off_qrec = (uint32_t)off;
+    if (few_lanes) off = align8(off + (size_t)n * 4);
     h.off_type = (uint32_t)off;   // (the last one: its length is known when the nodes are)
-    out.blob.assign(off + 2 * QUAD_TYPES + 16, 0);
+    off = (off + 15) & ~size_t(15);   // (blobs start on sixteen-byte boundaries of the pool)
+    out.blob.assign(off + (few_lanes ? 2 * QUAD_TYPES : 0), 0);
     uint8_t* const B = out.blob.data();
     NodeRec* const recs = (NodeRec*)(B + h.off_node);
     uint16_t* const succ = (uint16_t*)(B + h.off_succ);
@@ -549,25 +576,24 @@ class Lowering {
     uint16_t *const gmember = (uint16_t*)(B + h.off_gmember), *const glvl = (uint16_t*)(B + h.off_glvl);
     for (int k = 0; k < n_gm; ++k) { gmember[k] = (uint16_t)chain_of[k]; glvl[k] = (uint16_t)place[chain_of[k]]; }
     // predecessors in edge order
-    {
-      uint16_t *const pbeg = (uint16_t*)(B + h.off_pbeg), *const pred = (uint16_t*)(B + h.off_pred);
-      cur.resize(n);
-      for (int i = 0; i < n; ++i) { cur[i] = pbeg[i]; pbeg[i + 1] = (uint16_t)(pbeg[i] + indeg[i]); }
-      for (auto& ed : edges) pred[cur[ed.second]++] = (uint16_t)ed.first;
-      const bool quad = quad_rows(recs, pbeg, pred, n);
-      h.n_rows = quad ? (uint32_t)n_rows : 0u;
-      h.n_types = quad ? (uint32_t)types.size() : 0u;
+    uint16_t *const pbeg = (uint16_t*)(B + h.off_pbeg), *const pred = (uint16_t*)(B + h.off_pred);
+    cur.resize(n);
+    for (int i = 0; i < n; ++i) { cur[i] = pbeg[i]; pbeg[i + 1] = (uint16_t)(pbeg[i] + indeg[i]); }
+    for (auto& ed : edges) pred[cur[ed.second]++] = (uint16_t)ed.first;
+    if (few_lanes) {
+      if (quad_rows(recs, pbeg, pred, n)) {
+        h.n_rows = (uint32_t)n_rows;
+        h.n_types = (uint32_t)types.size();
+        std::memcpy(B + h.off_type, types.data(), types.size() * 2);
+        uint32_t* const qrec = (uint32_t*)(B + h.off_qrec);
+        for (int v = 0; v < n; ++v)
+          qrec[place[v]] = std::min<uint32_t>(recs[v].n_succ, 7u) | (uint32_t)recs[v].indeg << 3 | (uint32_t)recs[v].slot << 10 | (uint32_t)type_of[v] << 18 | (uint32_t)row_of[v] << 24;
+      }
+      off = (h.off_type + (size_t)h.n_types * 2 + 15) & ~size_t(15);
+      out.blob.resize(off);   // (never more: B stays)
     }
-    off = (off + (size_t)h.n_types * 2 + 15) & ~size_t(15);   // (blobs start on sixteen-byte boundaries of the pool)
     h.bytes = (uint32_t)off;
-    out.blob.resize(off);
     std::memcpy(B, &h, sizeof h);
-    if (h.n_types) std::memcpy(B + h.off_type, types.data(), types.size() * 2);
-    if (h.n_rows) {
-      uint32_t* const qrec = (uint32_t*)(B + h.off_qrec);
-      for (int v = 0; v < n; ++v)
-        qrec[place[v]] = std::min<uint32_t>(recs[v].n_succ, 7u) | (uint32_t)recs[v].indeg << 3 | (uint32_t)recs[v].slot << 10 | (uint32_t)type_of[v] << 18 | (uint32_t)row_of[v] << 24;
-    }
     // the orders of the one-plan-per-wavefront kernel: by level, and by tie-break class
     LevelRec* const lrec = (LevelRec*)(B + h.off_lrec);
     uint16_t *const lbeg16 = (uint16_t*)(B + h.off_lbeg), *const place16 = (uint16_t*)(B + h.off_place);
@@ -600,10 +626,10 @@ class Lowering {
 };
 
 // one class of a problem (a caller with many keeps the tables and a Lowering)
-inline LoweredClass lower_class(const rpeg_problem_t& P, uint64_t sig_bits) {
+inline LoweredClass lower_class(const rpeg_problem_t& P, uint64_t sig_bits, bool few_lanes = true) {
   const LowerTables tables(P, (int)(sig_bits & 3));
   Lowering l(P, tables);
-  l.run(sig_bits);
+  l.run(sig_bits, few_lanes);
   return std::move(l.out);
 }
 
