@@ -68,8 +68,8 @@ RPEG_HD unsigned blocked_mask(const NodeRec& r, uint64_t dpne) {
   unsigned b = r.blocked;
   if (r.cond) {
     const unsigned c = r.cond - 1u;
-    // (by words: where the amount of a 64-bit vector shift lies in the last register of a wavefront's allocation, it has
-    // shifted every lane by the same wrong number)
+    // (by words: a 64-bit vector shift whose amount lies in the last register of a wavefront's allocation now and then takes
+    // v0 for it.  The build looks every kernel over for one: shifts_by_last_register in build.py)
     const uint32_t w = c < 32u ? (uint32_t)dpne : (uint32_t)(dpne >> 32);
     b |= (unsigned)((w >> (c & 31u)) & 1u) << (c >> 3);
   }

@@ -108,8 +108,8 @@ __device__ inline double kp_sel(unsigned long long mask, double a, double b) {
   return __hiloint2double((int)kp_sel(mask, (uint32_t)__double2hiint(a), (uint32_t)__double2hiint(b)),
                           (int)kp_sel(mask, (uint32_t)__double2loint(a), (uint32_t)__double2loint(b)));
 }
-// Masks of 64 lanes by vector instructions, as two words.  (No 64-bit vector shift here: where its amount lies in the last
-// register of a wavefront's allocation, v_lshlrev_b64 has shifted every lane by the same wrong number.)
+// Masks of 64 lanes by vector instructions, as two words (two 32-bit shifts: no 64-bit one whose amount could lie in the last
+// register of the allocation, blocked_mask).
 struct KpMask { uint32_t lo, hi; };
 __device__ inline KpMask kp_bit(uint32_t l) {   // (none for 64 and more)
   const uint32_t b = 1u << (l & 31u);
