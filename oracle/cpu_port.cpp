@@ -172,6 +172,14 @@ long port_blob(void* h, uint64_t sig, int own, int few_lanes, uint8_t* out, long
   return (long)lc->blob.size();
 }
 
+// chains_in_sequence of a graph given by its successors and the tie-break class of every node
+int port_chains_in_sequence(int32_t n, const uint8_t* ptkey, const int32_t* adj_beg, const int32_t* adj_to, int32_t n_chains,
+                            const int32_t* beg, const int32_t* of) {
+  std::vector<NodeRec> recs(n);
+  for (int32_t v = 0; v < n; ++v) recs[v].ptkey = ptkey[v];
+  return chains_in_sequence(beg, (size_t)n_chains, of, adj_beg, adj_to, recs.data()) ? 1 : 0;
+}
+
 // isolated operator time / peak of mock nodes (candidate directory)
 int port_op_time(void* h, uint64_t n, int structure, int vertex, const int16_t* strat, uint64_t stride, double* time,
                  double* peak) {

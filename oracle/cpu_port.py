@@ -48,6 +48,8 @@ def lib():
         _lib.port_lower.argtypes = [C.c_void_p] * 9 + [C.c_int32, C.c_void_p]
         _lib.port_blob.restype = C.c_long
         _lib.port_blob.argtypes = [C.c_void_p, C.c_uint64, C.c_int, C.c_int, C.c_void_p, C.c_long, C.c_void_p, C.c_void_p]
+        _lib.port_chains_in_sequence.restype = C.c_int
+        _lib.port_chains_in_sequence.argtypes = [C.c_int32] + [C.c_void_p] * 3 + [C.c_int32] + [C.c_void_p] * 2
         _lib.port_op_time.restype = C.c_int
         _lib.port_op_time.argtypes = [C.c_void_p, C.c_uint64, C.c_int, C.c_int, C.c_void_p, C.c_uint64,
                                       C.c_void_p, C.c_void_p]

@@ -246,7 +246,8 @@ __device__ inline void kq_positions(const ClassView& cv, double* ranks, const do
         own = own1;
       }
     }
-    // (the nodes of a chain have the chain's largest rank, which is the first one's where no duration is negative)
+    // (the nodes of a chain have the chain's largest rank, which is the first one's where no duration is negative: a class
+    // whose chains are not runs of ids, each node a successor of the one before, has no rows -- chains_in_sequence)
     __syncthreads();
     if (cv.h->n_groups) {
       for (int i = r_q; i < n; i += QR) {

@@ -99,6 +99,21 @@ struct LoweredClass {
   std::vector<uint8_t> blob;
 };
 
+// Whether the nodes of[beg[k]], ... of every chain k follow each other within their tie-break class, in that order and with no
+// other node of the class between them, and each is a successor of the one before it.  k_quad gives all of them the rank of the
+// first, which it finds by the place in the chain.
+inline bool chains_in_sequence(const int* beg, size_t n_chains, const int* of, const int* adj_beg, const int* adj_to, const NodeRec* recs) {
+  for (size_t k = 0; k < n_chains; ++k)
+    for (int j = beg[k] + 1; j < beg[k + 1]; ++j) {
+      const int u = of[j - 1], v = of[j];
+      if (u > v || recs[u].ptkey != recs[v].ptkey) return false;
+      for (int w = u + 1; w < v; ++w)
+        if (recs[w].ptkey == recs[u].ptkey) return false;
+      if (std::find(adj_to + adj_beg[u], adj_to + adj_beg[u + 1], v) == adj_to + adj_beg[u + 1]) return false;
+    }
+  return true;
+}
+
 // Lowers one class after the other; run() leaves the last one in `out`.  A class is lowered on the critical path of the
 // first call that meets it, so the arrays live as long as the object and keep their memory, the slots are found through
 // the problem's tables, an edge is looked for among its source's few successors, and the blob's records are written where
@@ -581,7 +596,7 @@ class Lowering {
     for (int i = 0; i < n; ++i) { cur[i] = pbeg[i]; pbeg[i + 1] = (uint16_t)(pbeg[i] + indeg[i]); }
     for (auto& ed : edges) pred[cur[ed.second]++] = (uint16_t)ed.first;
     if (few_lanes) {
-      if (quad_rows(recs, pbeg, pred, n)) {
+      if (chains_in_sequence(chain_beg.data(), (size_t)nv * K, chain_of.data(), adj_beg.data(), adj_to.data(), recs) && quad_rows(recs, pbeg, pred, n)) {
         h.n_rows = (uint32_t)n_rows;
         h.n_types = (uint32_t)types.size();
         std::memcpy(B + h.off_type, types.data(), types.size() * 2);
