@@ -453,7 +453,8 @@ int rpeg_sa_propose(rpeg_engine_t* e, const rpeg_sa_params_t* prm, int32_t what,
    wavefront), [6] plans of a large batch that ran one per wavefront beside the main kernel (included
    in [2]), [7] wave tasks of the few-lanes-per-plan kernel (included in [2]), [8] plans that the call BEFORE the last
    one redid because their ready sets outgrew their kernel's (both calls laid out by the host: a batch that needed no
-   layout leaves the figure as it is), [9] plans of the few-lanes-per-plan kernel. */
+   layout leaves the figure as it is), [9] plans of the few-lanes-per-plan kernel, [10], [11], [12] launches of its forms for
+   ready sets of up to 8, 16 and 24 entries. */
 int rpeg_engine_stats(const rpeg_engine_t* e, uint64_t* out, int32_t n);
 
 /* Host time of the last rpeg_eval_batch call that laid its batch out, in microseconds of the steady clock: [0] from
