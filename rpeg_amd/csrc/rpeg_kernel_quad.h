@@ -196,7 +196,7 @@ __device__ inline double kq_more_successors(const ClassView& cv, const double* g
 // Bound: instruction issue, some 60 instructions a level and part, two for the comparison of up to 64 pairs of ranks.
 template <int QL, uint32_t PARTS>
 __device__ inline void kq_positions(const ClassView& cv, double* ranks, const double* dur_rows, const uint32_t* l_succ, const uint32_t* l_own,
-                                    const uint16_t* l_id, const uint16_t* l_chain, uint32_t class_ends, bool many, uint16_t* states) {
+                                    const uint16_t* l_id, const uint16_t* l_chain, uint32_t class_ends, bool many, bool shrink, uint16_t* states) {
   constexpr int RW = KE_WAVE / QL, QR = (int)PARTS * QL, RG = KE_WAVE / QR;   // lanes of a plan, plans at a time
   const int lane = threadIdx.x, r_q = lane % QR, n = (int)cv.h->n_nodes, n_levels = (int)cv.h->n_levels;
   for (int part = 0; part < (int)PARTS; ++part) {
@@ -250,6 +250,15 @@ __device__ inline void kq_positions(const ClassView& cv, double* ranks, const do
     // whose chains are not runs of ids, each node a successor of the one before, has no rows -- chains_in_sequence)
     __syncthreads();
     if (cv.h->n_groups) {
+      if (__builtin_expect(shrink, 0)) {
+        for (int i = r_q; i < n; i += QR) {
+          const int size = (l_chain[i] & 0xFFu) ? 1 : (int)(l_chain[i] >> 8);
+          double top = g_rank[i * RG];
+          for (int j = 1; j < size; ++j) top = kp_vmax(top, g_rank[(i + j) * RG]);
+          if (size > 1) g_rank[i * RG] = top;
+        }
+        __syncthreads();
+      }
       for (int i = r_q; i < n; i += QR) {
         const int in_chain = (int)(l_chain[i] & 0xFFu);
         if (in_chain) g_rank[i * RG] = g_rank[(i - in_chain) * RG];
@@ -345,7 +354,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint
   const double pen = L.aux_pen ? L.aux_pen[pi] : 1.0;
   const uint8_t gates = L.aux_mask ? L.aux_mask[pi] : (uint8_t)(RPEG_MASK_VALID | RPEG_MASK_STALE_OK | RPEG_MASK_MEM_OK);
   KE_STAMP(1);
-  bool err = cv.h->error != 0, ovf = false;
+  bool err = cv.h->error != 0, shrink = false;   // shrink: some plan has a node that ends before it starts
   {   // a slot whose duration the reference could not compute (division by zero) is NaN; a share by each lane
     bool bad = false, shrinks = false;
     for (int s0 = q; s0 < n_slots; s0 += 4 * QL) {   // four rows in flight
@@ -359,13 +368,12 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint
       for (int k = 0; k < 4; ++k) {
         const int s = s0 + k * QL;
         bad = bad || d[k] != d[k];
-        shrinks = shrinks || d[k] < 0.0;   // (nodes could share no rows: QuadRec)
+        shrinks = shrinks || d[k] < 0.0;
         if (s < n_slots) g_dur[s * RW] = d[k];
       }
     }
-    const uint32_t odd = kq_or<QL>((bad ? 1u : 0u) | (shrinks ? 2u : 0u));
-    err = err || (odd & 1u);
-    ovf = (odd & 2u) != 0u;
+    err = err || kq_or<QL>(bad ? 1u : 0u) != 0u;
+    shrink = __ballot(shrinks) != 0ull;
     if (err)   // (no NaN in the loops below)
       for (int s = q; s < n_slots; s += QL) g_dur[s * RW] = 0.0;
   }
@@ -379,9 +387,9 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint
 
   KE_STAMP(3);
   const bool any_many = __ballot(many != 0ull) != 0ull;   // (lanes that left the loop early)
-  if (Z.parts == 1) kq_positions<QL, 1>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_chain, class_ends, any_many, states);
-  else if (Z.parts == 2) kq_positions<QL, 2>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_chain, class_ends, any_many, states);
-  else kq_positions<QL, KQ_PARTS>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_chain, class_ends, any_many, states);
+  if (Z.parts == 1) kq_positions<QL, 1>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_chain, class_ends, any_many, shrink, states);
+  else if (Z.parts == 2) kq_positions<QL, 2>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_chain, class_ends, any_many, shrink, states);
+  else kq_positions<QL, KQ_PARTS>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_chain, class_ends, any_many, shrink, states);
   for (int x = q; x <= RPEG_MAX_V; x += QL) g_lf[x * RW] = 0.0;
   for (int r = q; r < n_rows; r += QL) g_time[r * RW] = 0.0;
   __syncthreads();
@@ -394,6 +402,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint
 #pragma unroll
   for (int u = 0; u < SL; ++u) { ek[u] = inf; sk[u] = inf; eo[u] = KQ_EMPTY; em[u] = 0u; }
   uint32_t tie = 0, free_slots = (1u << SL) - 1u;
+  bool ovf = false;
   int live = 0, longest = 0;   // entries now and at most (one more than there is room for where one was lost)
   const unsigned group_shift = (unsigned)(lane & ~(QL - 1));
   const uint32_t below = (1u << q) - 1u;   // the lanes of this plan before this one
@@ -428,7 +437,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint
   };
   {
     const int n_init = (int)cv.h->n_init;
-    ovf = ovf || n_init > QL * SL;
+    ovf = n_init > QL * SL;
     for (int i0 = 0; i0 < n_init && i0 < QL * SL; i0 += QL) {
       const bool mine = i0 + q < n_init;
       const uint32_t v = l_id[cv.place[cv.init[mine ? i0 + q : 0]]], own = l_own[v];
@@ -570,12 +579,12 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint
     mask64 mine = room & alive & __ballot(r < n_succ);
     uint32_t j0 = 0, sp = first_succ;
     while (mine) {
-      const uint32_t node = kp_sel(mine, sp, 0u), at = node & 0x1FFu, row = node >> 24;   // (a node of one predecessor: the row of zeros, never written)
+      const uint32_t node = kp_sel(mine, sp, 0u), at = node & 0x1FFu, row = node >> 24;   // (a node of one predecessor: the row that stays zero)
       const uint32_t state = g_state[at * RW], left = state - 0x400u, type = g_type[((node >> 18) & 0x3Fu) * RW];
       double t = kp_vmax(g_time[row * RW], fin);
       const mask64 ready = mine & __ballot(left < 0x400u);
-      if (kp_in(mine & ~ready)) {
-        g_time[row * RW] = t;
+      if (kp_in(mine)) {
+        g_time[row * RW] = kp_sel(ready, 0.0, t);   // (for the next node of the row)
         g_state[at * RW] = (uint16_t)left;
       }
       if (ready) {
