@@ -100,7 +100,8 @@ struct OrderRec {
 // The ready time of a node is the largest finish time of its predecessors: with one predecessor that is known when it is
 // asked for, and the node has row 0, which holds zeros.  The others share rows: X's row serves Y after it where every
 // predecessor of X is an ancestor of every predecessor of Y.  Then all of X's are dispatched, and X's ready time has been
-// used and the row set back to zero, before the first of Y's is.  (PPO, 85 nodes on average: 17 with several predecessors, 6.5 rows; AC-share of 300 nodes: 94 and 20.)
+// used, before the first of Y's is; and what X left there is no later than any of Y's predecessors ends, so that it need not
+// be cleared -- but where some node ends before it starts: then the row is set back when X is ready.  (PPO, 85 nodes on average: 17 with several predecessors, 6.5 rows; AC-share of 300 nodes: 94 and 20.)
 constexpr uint32_t QUAD_NODES = 511, QUAD_ROWS = 127, QUAD_TYPES = 64, QUAD_INDEG = 63;   // what the fields hold
 struct ClassHdr {
   uint32_t n_nodes, n_slots, n_succ, n_init, n_groups, n_gmembers;

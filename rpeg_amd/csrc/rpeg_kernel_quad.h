@@ -583,11 +583,14 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint
       const uint32_t state = g_state[at * RW], left = state - 0x400u, type = g_type[((node >> 18) & 0x3Fu) * RW];
       double t = kp_vmax(g_time[row * RW], fin);
       const mask64 ready = mine & __ballot(left < 0x400u);
-      if (kp_in(mine)) {
-        g_time[row * RW] = kp_sel(ready, 0.0, t);   // (for the next node of the row)
+      if (kp_in(mine & ~ready)) {
+        g_time[row * RW] = t;
         g_state[at * RW] = (uint16_t)left;
       }
       if (ready) {
+        if (__builtin_expect(shrink, 0)) {   // (a later node of the row may be ready before what this one leaves there)
+          if (kp_in(ready)) g_time[row * RW] = 0.0;
+        }
         const uint32_t b6 = type & 0x3Fu;   // one vertex or two (none: the row of zeros)
         const uint32_t v1 = (uint32_t)__builtin_ctz(b6 | (1u << RPEG_MAX_V)), v2 = b6 ? 31u - (uint32_t)__builtin_clz(b6) : (uint32_t)RPEG_MAX_V;
         t = kp_vmax(t, kp_vmax(g_lf[v1 * RW], g_lf[v2 * RW]));

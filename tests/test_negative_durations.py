@@ -1,6 +1,6 @@
 """Latencies below zero (Hardware.alpha_*: an intercept fitted to measurements may be) make transfers of small payloads end before
-they start, and operators too.  The kernel of a few lanes per plan shares ready-time rows, which it sets back when they have
-been read, and gives a chain's nodes the first one's rank, or the largest where some node ends before it starts.  Held to the
+they start, and operators too.  The kernel of a few lanes per plan shares ready-time rows, which it then sets back when they
+have been read, and gives a chain's nodes the largest rank instead of the first one's.  Held to the
 host build, without a plan redone for it.  (Not to the reference, whose devices become available again when the last node on them
 ends, earlier than another where that node ends before it starts: here availability only grows, on every path.)"""
 
