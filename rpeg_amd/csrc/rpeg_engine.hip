@@ -699,8 +699,9 @@ static uint8_t* static_scratch_ptr(int dev, hipError_t* st) {
 // rpeg_engine_set_split_model replaces them (a measurement aid).  A wrong figure
 // costs time, never a result: every kernel computes the same bits.
 //   plan_a + plan_b x nodes                    what a plan costs k_plan (one plan per wavefront), beside the main kernel;
-//                                              plan_list times as much beyond 128 nodes, where its scheduler
-//                                              keeps the nodes in LDS and fewer of its wavefronts fit on a compute unit
+//                                              plan_list times as much beyond KP_PAIR_NODES nodes: one figure for both slower
+//                                              forms of its scheduler (three nodes to a lane 600 clocks a decision, the nodes
+//                                              in LDS 1,060-1,110; two to a lane 400), with fewer wavefronts on a compute unit
 //   quad_a + nodes x (quad_b + quad_c x pops)  a wavefront of k_quad; pops = heap pops per dispatch, as the main kernel
 //                                              measured them for the class
 //   eff_beside_quad                            the part of a compute unit's sixteen wavefronts of k_plan that get
@@ -1433,7 +1434,7 @@ struct DeepModel {
   uint64_t r_max;
   SplitModel sm;
   double plan_cost(uint32_t plans, uint32_t nodes) const {
-    return (double)plans * (sm.plan_a + sm.plan_b * (double)nodes) * (nodes > 128u ? sm.plan_list : 1.0);
+    return (double)plans * (sm.plan_a + sm.plan_b * (double)nodes) * (nodes > (uint32_t)KP_PAIR_NODES ? sm.plan_list : 1.0);
   }
   double total(double w_main, double w_plan, double max_t, uint64_t r) const {
     const double t_main = std::max(max_t, w_main / (n_cu * (double)r));
@@ -1799,7 +1800,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // kernel's task, which shows where the step is not several times that, but a plan in k_plan costs eight times what one of
   // a full wavefront does.  And the launches go by LDS in up to QUAD_BINS bins a form.  (Neither / bins / both, us per step: AC-share
   // 262,144 5,133 / 5,197 / 4,090, 131,072 2,767 / 2,727 / 2,650, 98,304 2,180 / - / 2,258, 65,536 1,486 / 1,464 / 2,012; GRPO 131,072, bins
-  // 472 / 609.)
+  // 472 / 609.  Between the 51 nodes of those GRPO plans and the 152 of AC-share no workload was measured.)
   bool deep = false;
   auto plan_quad = [&]() -> bool {
     if (!quad_free) return false;

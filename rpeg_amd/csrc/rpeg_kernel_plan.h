@@ -6,8 +6,8 @@
 //   memory model    lane = template vertex, then lane = vertex subset (candidate device class)
 //   ranks           level by level from the nodes without successors, lane = node of the level (scheduler.py:71-100)
 //   positions       lane = node, which counts the nodes of its tie-break class with a larger rank
-//   list scheduler  rpeg_kernel_sched.h: up to 128 nodes a lane (or two) for every node, dealt by position; beyond that a
-//                   lane for every waiting node, the others in LDS.  All control flow is uniform
+//   list scheduler  rpeg_kernel_sched.h: up to 192 nodes every node in a lane, one to three to each, dealt by position; beyond
+//                   that a lane for every waiting node, the others in LDS.  All control flow is uniform
 //   outputs         lane = node for the predecessors of the critical chain, lane = set of allocations for the utilisation
 //
 // Device availability: a node waits for max(avail[d]) over the devices it reserves, i.e. for the largest finish time of

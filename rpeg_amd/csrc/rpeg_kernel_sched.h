@@ -38,6 +38,7 @@
 
 namespace rpeg {
 
+constexpr int KP_PAIR_NODES = 128;   // up to here kp_lanes has at most two nodes to a lane
 constexpr int KP_LANE_NODES = 192;   // largest graph of kp_lanes: five nodes to a lane were tried, 300-node graphs 150 -> 205 us
 
 #if defined(__HIPCC__)
@@ -1270,7 +1271,7 @@ template <int TR>
 __device__ inline double kp_schedule(const uint8_t* blob, int n, uint64_t ovl, uint64_t dpne, const KpLds& M, unsigned long long* stamp) {
   const uint64_t b = (uint64_t)blob;
   if (n <= 64) return kp_lanes<1, TR>(b, ovl, dpne, M, stamp);
-  if (n <= 128) return kp_lanes<2, TR>(b, ovl, dpne, M, stamp);
+  if (n <= KP_PAIR_NODES) return kp_lanes<2, TR>(b, ovl, dpne, M, stamp);
   if (n <= KP_LANE_NODES) return kp_lanes<3, TR>(b, ovl, dpne, M, stamp);
   const double ms = kp_list<TR>(b, ovl, dpne, M, stamp);
   return ms == -2.0 ? kp_plain<TR>(b, ovl, dpne, M) : ms;
