@@ -103,6 +103,15 @@ struct OrderRec {
 // used, before the first of Y's is; and what X left there is no later than any of Y's predecessors ends, so that it need not
 // be cleared -- but where some node ends before it starts: then the row is set back when X is ready.  (PPO, 85 nodes on average: 17 with several predecessors, 6.5 rows; AC-share of 300 nodes: 94 and 20.)
 constexpr uint32_t QUAD_NODES = 511, QUAD_ROWS = 127, QUAD_TYPES = 64, QUAD_INDEG = 63;   // what the fields hold
+// And what its rank pass reads of a node, by level place.  A rank is needed in LDS from the level that computes it to the last one
+// with a predecessor of its node: such stretches share rows.  Row 0 holds zeros (a successor there is not), row 1 is written and
+// never read (nodes without predecessors, lanes without a node).  The record behind the last one is that of a lane without a
+// node (its id is the number of nodes); one more has the number of rows in the place of an id.  (AC-share, 141 nodes on average: 14 rows; GRPO, 51 nodes: 8.)
+struct RankRec {
+  uint8_t succ[4], row, slot;   // rows of the first four successors, its own; duration slot
+  uint16_t id;                  // place in the order by tie-break class; RANK_MORE: more than four successors
+};
+constexpr uint32_t RANK_ROWS = 256, RANK_MORE = 0x8000;
 struct ClassHdr {
   uint32_t n_nodes, n_slots, n_succ, n_init, n_groups, n_gmembers;
   uint32_t off_node, off_succ, off_init, off_topo, off_slot, off_group, off_gmember;  // byte offsets in the blob
@@ -134,8 +143,12 @@ struct ClassView {
   const uint16_t* glvl;
   const uint16_t* place;
   const uint32_t* qrec;
+  const RankRec* rrec;
   const uint16_t* type;   // blocked | cond << 8
 };
+
+// (behind the QuadRecs)
+RPEG_HD uint32_t rank_rec_offset(const ClassHdr& h) { return h.off_qrec + ((4u * h.n_nodes + 7u) & ~7u); }
 
 RPEG_HD ClassView class_view(const uint8_t* blob) {
   ClassView v;
@@ -156,6 +169,7 @@ RPEG_HD ClassView class_view(const uint8_t* blob) {
   v.glvl = (const uint16_t*)(blob + v.h->off_glvl);
   v.place = (const uint16_t*)(blob + v.h->off_place);
   v.qrec = (const uint32_t*)(blob + v.h->off_qrec);
+  v.rrec = (const RankRec*)(blob + rank_rec_offset(*v.h));
   v.type = (const uint16_t*)(blob + v.h->off_type);
   return v;
 }

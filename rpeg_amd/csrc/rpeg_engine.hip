@@ -423,11 +423,12 @@ __global__ __launch_bounds__(WAVE) void k_eval(const EvalLaunch L) {
 struct QuadKind { uint32_t plans, entries; };
 constexpr QuadKind QUAD_KIND[3] = {{32, 8}, {16, 16}, {16, 24}};   // k_quad<2, 4>, <4, 4>, <4, 6>
 template <int QL, int SL>
-__global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_quad(const EvalLaunch L, const QuadSize Z) {
+__global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_quad(const EvalLaunch L, const QuadSize Z, double* const ranks) {
   extern __shared__ uint8_t kq_lds[];
   const uint64_t w = blockIdx.x;
-  if (SL == 4 && QL == 4 && (L.wave_cls[w] & KE_CLS_LDS)) kq_eval_wave<QL, 2>(L, Z, w, kq_lds);   // uniform branch
-  else kq_eval_wave<QL, SL>(L, Z, w, kq_lds);
+  double* const keep = ranks + w * kq_rank_doubles(WAVE / QL, Z);
+  if (SL == 4 && QL == 4 && (L.wave_cls[w] & KE_CLS_LDS)) kq_eval_wave<QL, 2>(L, Z, keep, w, kq_lds);   // uniform branch
+  else kq_eval_wave<QL, SL>(L, Z, keep, w, kq_lds);
 }
 
 // One plan per wavefront (rpeg_kernel_plan.h); perm[w] is the plan of wavefront task w.  TR: KpTrace.
@@ -836,6 +837,8 @@ struct rpeg_engine_s {
   uint64_t* h_sig = nullptr;
   uint32_t *d_perm = nullptr, *d_cls = nullptr, *h_cls = nullptr;   // lane -> plan; wavefront -> class blob
   uint8_t* d_ws = nullptr;
+  double* d_ranks = nullptr;                    // ranks of k_quad's tasks on their way to the comparison of positions
+  size_t ranks_cap = 0;
   // outputs of the prologue launches (rpeg_kernel_prologue.h), cap_n plans each: pair relations, penalty factor, gate
   // bits; the durations of the slot universe ([slot][plan]); and the universe itself
   uint64_t *d_aux_ovl = nullptr, *d_aux_dpne = nullptr, *d_aux_eq = nullptr;
@@ -1035,7 +1038,7 @@ static bool pool_room(rpeg_engine_t* e, size_t bytes) {
 
 // what k_quad keeps of class c, lowered with it (`few`) or not
 static void class_few(rpeg_engine_t* e, uint32_t c, const ClassHdr* h, bool few) {
-  e->cls_quad[c] = QuadSize{h->n_nodes, h->n_slots, h->n_rows, h->n_types};
+  e->cls_quad[c] = QuadSize{h->n_nodes, h->n_slots, h->n_rows, h->n_types, h->n_rows ? class_view((const uint8_t*)h).rrec[h->n_nodes + 1].id : 0u};
   e->cls_few[c] = few ? 1 : 0;
   e->max_quad.fit(e->cls_quad[c]);
 }
@@ -1175,6 +1178,18 @@ static int ensure_ws(rpeg_engine_t* e, size_t bytes, hipStream_t s) {
   return 0;
 }
 
+// ranks of the tasks of k_quad
+static int ensure_ranks(rpeg_engine_t* e, size_t doubles, hipStream_t s) {
+  if (doubles <= e->ranks_cap) return 0;
+  HIP_TRY(e, hipStreamSynchronize(s));
+  if (e->d_ranks) hipFree(e->d_ranks);
+  e->d_ranks = nullptr;
+  e->ranks_cap = 0;
+  HIP_TRY(e, hipMalloc(&e->d_ranks, doubles * 8));
+  e->ranks_cap = doubles;
+  return 0;
+}
+
 // state of the launch that redoes flagged plans: as many wavefronts as 128 MiB hold, at most one per compute unit
 static int ensure_limit_ws(rpeg_engine_t* e, hipStream_t s) {
   const size_t per_wave = limit_ws_bytes(e->max_nodes, e->max_slots);
@@ -1291,6 +1306,7 @@ void rpeg_engine_destroy(rpeg_engine_t* e) {
   if (e->h_times) hipHostFree(e->h_times);
   if (e->d_trace) hipFree(e->d_trace);
   if (e->d_detail) hipFree(e->d_detail);
+  if (e->d_ranks) hipFree(e->d_ranks);
   if (e->d_ws) hipFree(e->d_ws);
   if (e->ev0) hipEventDestroy(e->ev0);
   if (e->ev1) hipEventDestroy(e->ev1);
@@ -1780,7 +1796,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   };
   std::vector<uint8_t> solo(counts.size(), 0), quad(counts.size(), 0);
   for (size_t c = 0; quad_all && c < counts.size(); ++c) quad[c] = e->cls_quad[cids[c]].rows ? 1 : 0;
-  constexpr double QUAD_HALF_LDS = 1.05;
+  constexpr double QUAD_PART_LDS = 1.05;
   constexpr size_t QUAD_BINS = 3;
   constexpr uint32_t QUAD_TINY = 8, QUAD_MEAN_NODES = 128, QUAD_DEEP_PLANS = 512;
   // k_quad takes the batch, with k_plan beside it, where the model below has them done before the main kernel would be.
@@ -2054,7 +2070,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // after the other, the one of the largest LDS on a stream of its own and the others by turns on two: a launch behind another
   // waits for its slowest task.  (AC-share, us per step, 262,144 / 140,001 plans: 1 launch a form 5,560 / 3,127, 2 4,325 / 2,632, 3
   // 4,090 / 2,754, 4 4,105 / 2,752; 3 with the last one alone on a stream 4,320 / 2,800, all of them on one 6,190 / 4,290.)
-  struct QuadLaunch { uint32_t first = 0, waves = 0; QuadSize size; int kind = 0; bool aside = false, first_stream = false; };   // on the fourth stream; on the main kernel's, where that has no tasks
+  struct QuadLaunch { uint32_t first = 0, waves = 0; QuadSize size; size_t ranks = 0; int kind = 0; bool aside = false, first_stream = false; };   // on the fourth stream; on the main kernel's, where that has no tasks
   std::vector<QuadLaunch> quad_launch;
   bool aside = false;   // some launch is
   {
@@ -2115,8 +2131,8 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       std::stable_partition(quad_launch.begin(), quad_launch.end(), [](const QuadLaunch& x) { return x.kind == 2 || !x.aside; });
     }
   }
-  {   // the ranks of a wavefront all at once, where the launches' wavefronts find room together all the same; else of half
-      // its plans, where that needs (next to) no more LDS than those of a quarter, which the rows behind them need anyway
+  {   // the positions of a wavefront's plans all at once, its ranks in LDS, where the launches' wavefronts find room together all the
+      // same; else by the larger parts where they need (next to) no more LDS than the smaller, the rows behind them needing as much anyway
     double cu = 0.0;
     for (QuadLaunch& q : quad_launch) {
       q.size.parts = 1;
@@ -2125,11 +2141,17 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     if (!(cu <= (double)e->n_cu))
       for (QuadLaunch& q : quad_launch) {
         const uint32_t plans = QUAD_KIND[q.kind].plans;
-        q.size.parts = KQ_PARTS;
-        const double quarter = (double)kq_lds_bytes(plans, q.size, mass != nullptr);
-        q.size.parts = 2;
-        if ((double)kq_lds_bytes(plans, q.size, mass != nullptr) > QUAD_HALF_LDS * quarter) q.size.parts = KQ_PARTS;
+        const uint32_t parts = kq_parts_least(WAVE / plans);
+        auto lds_by = [&](uint32_t x) { q.size.parts = x; return (double)kq_lds_bytes(plans, q.size, mass != nullptr); };
+        q.size.parts = lds_by(parts) > QUAD_PART_LDS * lds_by(2 * parts) ? 2 * parts : parts;
       }
+    size_t doubles = 0;
+    for (QuadLaunch& q : quad_launch) {
+      if (q.size.parts == 1) continue;   // (in LDS)
+      q.ranks = doubles;
+      doubles += (size_t)q.waves * kq_rank_doubles(QUAD_KIND[q.kind].plans, q.size);
+    }
+    if (int rc = ensure_ranks(e, doubles, s)) return rc;
   }
   const uint32_t n_lane_waves = n_eval_waves + n_quad_waves;
   const uint32_t pstride = one ? 1u : (uint32_t)WAVE;
@@ -2339,9 +2361,9 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       HIP_TRY(e, hipFuncSetAttribute((const void*)k_quad<4, 6>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
       e->quad_attr_set = true;
     }
-    if (q.kind == 0) hipLaunchKernelGGL((k_quad<2, 4>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q, q.size);
-    else if (q.kind == 1) hipLaunchKernelGGL((k_quad<4, 4>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q, q.size);
-    else hipLaunchKernelGGL((k_quad<4, 6>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q, q.size);
+    if (q.kind == 0) hipLaunchKernelGGL((k_quad<2, 4>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q, q.size, e->d_ranks + q.ranks);
+    else if (q.kind == 1) hipLaunchKernelGGL((k_quad<4, 4>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q, q.size, e->d_ranks + q.ranks);
+    else hipLaunchKernelGGL((k_quad<4, 6>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q, q.size, e->d_ranks + q.ranks);
     HIP_TRY(e, hipGetLastError());
     return 0;
   };

@@ -31,7 +31,7 @@
 // and redone by the launch that ends the call, a plan per wavefront.  Its class then reports one entry more than there was
 // room for (EvalLaunch::cneed), and the next call gives it the form above: without that a class stayed where it was and
 // its plans were redone in every call (20,011 PPO plans, forms learned from other plans: 25 of them, 452 us a step; now
-// 384).  Ranks go level by level with a node per lane of the plan.  A node's id is its place by tie-break class, so that
+// 384).  Ranks go level by level with a node per lane of the plan, all plans together (kq_ranks).  A node's id is its place by tie-break class, so that
 // counting the larger ranks of its class walks through consecutive rows.
 //
 // Bound: vector issue and, with few wavefronts in flight, the latency of a round (four lanes of four entries: some 360 vector
@@ -52,7 +52,9 @@ namespace rpeg {
 constexpr uint32_t KQ_TIE_BITS = 20, KQ_TIE_MASK = (1u << KQ_TIE_BITS) - 1u;   // (a round takes at most 1 + 24 + 24 ties and four per new entry: 2^15 for 512 nodes)
 constexpr uint32_t KQ_EMPTY = 0xFFFFFFFFu;
 
-constexpr uint32_t KQ_PARTS = 4;
+// Positions are found for 1 / parts of a wavefront's plans at a time: all at once, or half or a quarter with two lanes a plan, a
+// quarter or an eighth with four.
+__host__ __device__ constexpr uint32_t kq_parts_least(uint32_t lanes) { return lanes == 2 ? 2u : 4u; }
 // Graphs of up to this many nodes have their equal ranks counted along with the larger ones, larger graphs afterwards, by
 // position: along, every pair of a class costs two instructions more, afterwards every node 25 and three LDS trips, and
 // classes grow with the graph.  (Afterwards / along, us a step: 65,536 GRPO plans of 51 nodes 322 / 315, 65,536 DPO plans of 28
@@ -60,22 +62,28 @@ constexpr uint32_t KQ_PARTS = 4;
 constexpr int KQ_EQ_NODES = 60;
 // What a launch's LDS is sized for: the largest of its classes in each respect.
 struct QuadSize {
-  uint32_t nodes = 0, slots = 0, rows = 0, types = 0;
-  uint32_t parts = KQ_PARTS;   // the ranks of this fraction of the plans at a time: 1, 2 or KQ_PARTS
+  uint32_t nodes = 0, slots = 0, rows = 0, types = 0, ranks = 0;   // (ranks: rows of the rank pass)
+  uint32_t parts = 4;
   __host__ __device__ void fit(const QuadSize& o) {
     nodes = o.nodes > nodes ? o.nodes : nodes; slots = o.slots > slots ? o.slots : slots;
     rows = o.rows > rows ? o.rows : rows; types = o.types > types ? o.types : types;
+    ranks = o.ranks > ranks ? o.ranks : ranks;
   }
 };
 // LDS of one wavefront.  Class tables: per node four successor words, its own, its level place's id and its place in its chain.
 // Per plan [row][plan]: durations, availability by vertex with a row of zeros and one nobody reads, ready-time
-// rows -- over these two, before they are needed, the ranks of all, half or a quarter of the plans --, with the critical-chain masses finish
+// rows -- over these two, before they are needed, the rows and records of the rank pass, then the ranks of the plans whose
+// positions are being found, or, where that is all of them, both --, with the critical-chain masses finish
 // and start times, a state word and a reservation each.
 __host__ __device__ inline size_t kq_tab_bytes(uint32_t nodes) { return (20ull * nodes + 2 * 2ull * (nodes + 2) + 15) & ~size_t(15); }
 __host__ __device__ inline size_t kq_union_bytes(uint32_t plans, const QuadSize& z) {
-  const size_t rows = 8ull * plans * (z.rows + RPEG_MAX_V + 2), ranks = 8ull * (plans / z.parts) * (z.nodes + 1);
-  return rows > ranks ? rows : ranks;
+  const size_t rows = 8ull * plans * (z.rows + RPEG_MAX_V + 2), part = 8ull * (plans / z.parts) * z.nodes,
+               ranks = 8ull * plans * z.ranks + sizeof(RankRec) * (z.nodes + 2ull) + (z.parts == 1 ? part + 8ull * plans : 0ull);
+  const size_t most = rows > part ? rows : part;
+  return ((most > ranks ? most : ranks) + 15) & ~size_t(15);
 }
+// Ranks of one wavefront in memory, by part of the plans: [part][node id][plan of the part].
+__host__ __device__ inline size_t kq_rank_doubles(uint32_t plans, const QuadSize& z) { return (size_t)plans * z.nodes; }
 __host__ __device__ inline size_t kq_lds_bytes(uint32_t plans, const QuadSize& z, bool mass) {
   return (kq_tab_bytes(z.nodes) + (size_t)plans * (8ull * z.slots + (mass ? 16ull * z.nodes : 0ull) + 2ull * z.nodes + 2ull * z.types) +
           kq_union_bytes(plans, z) + 15) & ~size_t(15);
@@ -182,73 +190,111 @@ __device__ inline void kq_count_all(const double* g_rank, const uint32_t* l_own,
 }
 
 // The largest rank among the successors from the fifth on of the node at level place i, or `best`.
-__device__ inline double kq_more_successors(const ClassView& cv, const double* g_rank, const uint16_t* l_id, int RG, int i, double best) {
+__device__ inline double kq_more_successors(const ClassView& cv, const double* g_rank, int RW, int i, double best) {
   const NodeRec nr = cv.node[cv.lrec[i].node];
-  for (int j = 4; j < nr.n_succ; ++j) best = kp_vmax(best, g_rank[l_id[cv.place[cv.succ[nr.succ_begin + j]]] * RG]);
+  for (int j = 4; j < nr.n_succ; ++j) best = kp_vmax(best, g_rank[cv.rrec[cv.place[cv.succ[nr.succ_begin + j]]].row * RW]);
   return best;
 }
 
-// Ranks and, from them, the state words of all plans of a wavefront.  Ranks take eight bytes a node, more than all a plan keeps
-// of it later: where a launch has more wavefronts than find room at once, they are computed for half or a quarter of the
-// plans at a time, with two or four times the lanes for each.  (All at once / a quarter at a time, us a step: 16,384 DPO plans
-// 134 / 138, 17,000 GRPO 254 / 259, 20,011 PPO 317 / 332; 65,536 GRPO 343 / 325, 65,536 chains 692 / 606, 1,048,576 DPO 1,116 /
-// 1,014.  Half at a time where that takes the LDS of a quarter: 1,048,576 DPO 1,025 -> 970.)
-// Bound: instruction issue, some 60 instructions a level and part, two for the comparison of up to 64 pairs of ranks.
+// Ranks of all plans of a wavefront (scheduler.py:71-100), level by level from the nodes without successors, a node per lane of
+// the plan, out to `keep`.
+// Bound: a trip (up to two or four nodes a plan) is some 35 vector instructions and one LDS round trip; records are read two trips
+// ahead, durations one.  A rank takes eight bytes a node, more than all a plan keeps of it later, but is read back only by the
+// few levels below: in LDS lie rows that nodes share (RankRec), and the ranks go through memory (240 MB for 1,048,576 DPO plans, most of
+// it never out of the L2) to the comparison of positions, which takes them a part of the plans at a time; where the launches'
+// wavefronts find room together with all of their ranks (AT_ONCE) those stay in LDS.  Before, the pass ran once for every part,
+// with two to four times the lanes for levels of two or three nodes, and a part's ranks all lay in LDS.  us a step, before / now:
+// 262,144 AC-share plans 4,196 / 3,953, 131,072 2,720 / 2,572, 65,536 1,550 / 1,430; 131,072 PPO 989 / 935, GRPO 490 / 442; 65,536
+// GRPO 320 / 307; 1,048,576 DPO 971 / 971; 20,011 PPO (all at once in either) 310 / 308.
+template <int QL, bool AT_ONCE>
+__device__ inline void kq_ranks(const ClassView& cv, double* rows, uint32_t n_rows, uint32_t ends, const double* g_dur, double* keep, uint32_t parts, bool many) {
+  constexpr int RW = KE_WAVE / QL;
+  const int lane = threadIdx.x, p = lane / QL, q = lane % QL, n = (int)cv.h->n_nodes, n_levels = (int)cv.h->n_levels;
+  double* const g_rank = rows + p;
+  const uint2* const l_rec = (const uint2*)(rows + (size_t)n_rows * RW);
+  // (bytes, of the nodes' ranks of a plan)
+  const uint32_t rg = (uint32_t)__builtin_ctz(RW / parts) + 3u, out = AT_ONCE ? 0u : (((uint32_t)p >> (rg - 3u)) * (uint32_t)n << rg) + (((uint32_t)p & (RW / parts - 1u)) << 3);
+  int level = 0;
+  auto end_of = [&](int l) {   // (asked for level by level)
+    if (__builtin_expect(l && (l & 63) == 0, 0)) ends = cv.lbeg[l + lane + 1 <= n_levels ? l + lane + 1 : n_levels];
+    return l < n_levels ? __builtin_amdgcn_readlane((int)ends, l & 63) : n;
+  };
+  // a trip: places at to end - 1, QL at most.  This one, the next, the one after that
+  int at = 0, end = end_of(0), at1, end1, at2, end2;
+  auto next = [&](int a, int e, int& a1, int& e1) {
+    a1 = a + QL;
+    e1 = e;
+    if (a1 >= e) {
+      a1 = e;
+      e1 = end_of(++level);
+    }
+  };
+  auto record = [&](int a, int e) { return l_rec[a + q < e ? a + q : n]; };
+  next(at, end, at1, end1);
+  uint2 rec = record(at, end), rec1 = record(at1, end1);
+  double d = g_dur[((rec.y >> 8) & 0xFFu) * RW];
+  while (at < n) {
+    const double r0 = g_rank[(rec.x & 0xFFu) * RW], r1 = g_rank[((rec.x >> 8) & 0xFFu) * RW];
+    double best;
+    next(at1, end1, at2, end2);
+    const uint2 rec2 = record(at2, end2);
+    const double d1 = g_dur[((rec1.y >> 8) & 0xFFu) * RW];
+    if (AT_ONCE || __ballot(rec.x > 0xFFFFu)) {   // (a branch is a quarter of a trip's latency)
+      const double r2 = g_rank[((rec.x >> 16) & 0xFFu) * RW], r3 = g_rank[(rec.x >> 24) * RW];
+      best = kp_vmax(kp_vmax(r0, r1), kp_vmax(r2, r3));
+      if (__builtin_expect(many, 0))
+        if (at + q < end && (rec.y >> 31)) best = kq_more_successors(cv, g_rank, RW, at + q, best);
+    } else {
+      best = kp_vmax(r0, r1);
+    }
+    const double rank = d + best;
+    g_rank[(rec.y & 0xFFu) * RW] = rank;
+    const uint32_t id = (rec.y >> 16) & 0x1FFu;
+    if (AT_ONCE) keep[id * RW + p] = rank;
+    else if (at + q < end) *(double*)((uint8_t*)keep + (out + (id << rg))) = rank;
+    rec = rec1;
+    rec1 = rec2;
+    d = d1;
+    at = at1;
+    end = end1;
+    at1 = at2;
+    end1 = end2;
+  }
+  __syncthreads();   // (the ranks are in memory: a wavefront reads its own)
+}
+
+// From the ranks the state words of all plans of a wavefront, a part of them at a time with as many times the lanes for each.  The
+// next part's ranks are fetched while one's are compared with four lanes a plan; with two the sixteen registers this takes kept the
+// memory model's launch off the compute units (1,048,576 DPO plans 982 us a step, without 971).
+// Bound: instruction issue, two instructions for the comparison of up to 64 pairs of ranks.
 template <int QL, uint32_t PARTS>
-__device__ inline void kq_positions(const ClassView& cv, double* ranks, const double* dur_rows, const uint32_t* l_succ, const uint32_t* l_own,
-                                    const uint16_t* l_id, const uint16_t* l_chain, uint32_t class_ends, bool many, bool shrink, uint16_t* states) {
+__device__ inline void kq_positions(const ClassView& cv, double* ranks, const double* keep, const uint32_t* l_own, const uint16_t* l_chain,
+                                    uint32_t class_ends, bool shrink, uint16_t* states) {
   constexpr int RW = KE_WAVE / QL, QR = (int)PARTS * QL, RG = KE_WAVE / QR;   // lanes of a plan, plans at a time
-  const int lane = threadIdx.x, r_q = lane % QR, n = (int)cv.h->n_nodes, n_levels = (int)cv.h->n_levels;
+  const int lane = threadIdx.x, r_q = lane % QR, n = (int)cv.h->n_nodes;
+  const uint4* const from = (const uint4*)keep;
+  uint4* const to = (uint4*)ranks;
+  const int n4 = n * RG / 2;
+  uint4 ahead0, ahead1, ahead2, ahead3;   // (an array would lie in scratch memory)
+  auto fetch = [&](int part) {
+    const uint4* const f = from + part * n4;
+    auto at = [&](int k) { return f[lane + k * KE_WAVE < n4 ? lane + k * KE_WAVE : 0]; };
+    ahead0 = at(0); ahead1 = at(1); ahead2 = at(2); ahead3 = at(3);
+  };
+  if (PARTS > 1 && QL == 4) fetch(0);
   for (int part = 0; part < (int)PARTS; ++part) {
     const int r_p = part * RG + lane / QR;
     double* const g_rank = ranks + lane / QR;
-    const double* const r_dur = dur_rows + r_p;
-    // ---- ranks: level by level from the nodes without successors, then chain inheritance (scheduler.py:71-100, 367-378).
-    // A level waits for one LDS trip, that of its successors' ranks: words and durations of its nodes were read a level ahead,
-    // their ids two levels.
-    if (r_q == 0) g_rank[n * RG] = 0.0;
-    __syncthreads();
-    {
-      uint32_t ends = 0;
-      auto end_of = [&](int l) { return l < n_levels ? __builtin_amdgcn_readlane((int)ends, l & 63) : n; };
-      auto id_at = [&](int i) { return (int)l_id[i < n ? i : n - 1]; };
-      int begin = 0;
-      ends = cv.lbeg[lane + 1 <= n_levels ? lane + 1 : n_levels];
-      int end = end_of(0), id = id_at(r_q), id1 = id_at(end + r_q);
-      uint4 sw = ((const uint4*)l_succ)[id];
-      uint32_t own = l_own[id];
-      double d = r_dur[((own >> 10) & 0xFFu) * RW];
-      for (int l = 0; l < n_levels; ++l) {
-        const double r0 = g_rank[(sw.x & 0x1FFu) * RG], r1 = g_rank[(sw.y & 0x1FFu) * RG], r2 = g_rank[(sw.z & 0x1FFu) * RG], r3 = g_rank[(sw.w & 0x1FFu) * RG];
-        const uint4 sw1 = ((const uint4*)l_succ)[id1];
-        const uint32_t own1 = l_own[id1];
-        if (__builtin_expect((l & 63) == 63, 0)) ends = cv.lbeg[l + 1 + lane + 1 <= n_levels ? l + 1 + lane + 1 : n_levels];
-        const int end1 = end_of(l + 1), id2 = id_at(end1 + r_q);
-        double best = kp_vmax(kp_vmax(r0, r1), kp_vmax(r2, r3));
-        int i = begin + r_q;
-        if (__builtin_expect(many, 0))
-          if (i < end && (own & 7u) > 4u) best = kq_more_successors(cv, g_rank, l_id, RG, i, best);
-        if (i < end) g_rank[id * RG] = d + best;
-        for (i += QR; __builtin_expect(__ballot(i < end) != 0ull, 0); i += QR) {   // (more nodes than lanes)
-          const int id_i = id_at(i);
-          const uint4 w = ((const uint4*)l_succ)[id_i];
-          const uint32_t o = l_own[id_i];
-          best = kp_vmax(kp_vmax(g_rank[(w.x & 0x1FFu) * RG], g_rank[(w.y & 0x1FFu) * RG]), kp_vmax(g_rank[(w.z & 0x1FFu) * RG], g_rank[(w.w & 0x1FFu) * RG]));
-          if (many && i < end && (o & 7u) > 4u) best = kq_more_successors(cv, g_rank, l_id, RG, i, best);
-          if (i < end) g_rank[id_i * RG] = r_dur[((o >> 10) & 0xFFu) * RW] + best;
-        }
-        d = r_dur[((own1 >> 10) & 0xFFu) * RW];
-        begin = end;
-        end = end1;
-        id = id1;
-        id1 = id2;
-        sw = sw1;
-        own = own1;
-      }
+    if (PARTS > 1) {
+      auto put = [&](int k, const uint4 w) { if (lane + k * KE_WAVE < n4) to[lane + k * KE_WAVE] = w; };
+      if (QL == 2) fetch(part);
+      put(0, ahead0); put(1, ahead1); put(2, ahead2); put(3, ahead3);
+      for (int i = lane + 4 * KE_WAVE; i < n4; i += KE_WAVE) to[i] = from[part * n4 + i];
+      __syncthreads();
+      if (QL == 4 && part + 1 < (int)PARTS) fetch(part + 1);
     }
     // (the nodes of a chain have the chain's largest rank, which is the first one's where no duration is negative: a class
     // whose chains are not runs of ids, each node a successor of the one before, has no rows -- chains_in_sequence)
-    __syncthreads();
     if (cv.h->n_groups) {
       if (__builtin_expect(shrink, 0)) {
         for (int i = r_q; i < n; i += QR) {
@@ -289,7 +335,7 @@ __device__ inline void kq_positions(const ClassView& cv, double* ranks, const do
 }
 
 template <int QL, int SL>
-__device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint64_t w, uint8_t* lds) {
+__device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, double* keep, uint64_t w, uint8_t* lds) {   // keep: ranks (kq_rank_doubles)
   constexpr int RW = KE_WAVE / QL;
   const int lane = threadIdx.x, p = lane / QL, q = lane % QL;
   constexpr int first_lane = 0;
@@ -305,7 +351,6 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint
   uint16_t* l_chain = l_id + (Z.nodes + 2);        // [node id]: place in its chain (whose nodes' ids follow each other) | nodes of the chain << 8
   double* rows = (double*)(lds + kq_tab_bytes(Z.nodes));
   double* g_dur = rows + p;
-  double* const dur_rows = rows;
   rows += (size_t)Z.slots * RW;
   double* const ranks = rows;                      // [node id][plans at a time], before the two below are needed
   double* g_lf = rows + p;
@@ -334,6 +379,12 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint
   }
   if (lane == 0) l_id[n] = (uint16_t)n;
   __syncthreads();
+  const uint32_t level_ends = cv.lbeg[lane + 1 <= (int)cv.h->n_levels ? lane + 1 : (int)cv.h->n_levels];
+  {   // what the rank pass reads, behind its rows
+    uint2* const l_rec = (uint2*)(ranks + (size_t)Z.ranks * RW);
+    for (int i = lane; i <= n; i += KE_WAVE) l_rec[i] = ((const uint2*)cv.rrec)[i];
+    if (q == 0) ranks[p] = 0.0;
+  }
   mask64 many = 0ull;   // some node has more than four successors
   for (int i = lane; i < n; i += KE_WAVE) {
     const LevelRec r = cv.lrec[i];
@@ -385,11 +436,18 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, uint
   KE_STAMP(2);
   const bool stale_ok = (gates & RPEG_MASK_STALE_OK) != 0, mem_ok = (gates & RPEG_MASK_MEM_OK) != 0;
 
-  KE_STAMP(3);
   const bool any_many = __ballot(many != 0ull) != 0ull;   // (lanes that left the loop early)
-  if (Z.parts == 1) kq_positions<QL, 1>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_chain, class_ends, any_many, shrink, states);
-  else if (Z.parts == 2) kq_positions<QL, 2>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_chain, class_ends, any_many, shrink, states);
-  else kq_positions<QL, KQ_PARTS>(cv, ranks, dur_rows, l_succ, l_own, l_id, l_chain, class_ends, any_many, shrink, states);
+  if (Z.parts == 1) {
+    double* const all = ranks + (size_t)Z.ranks * RW + Z.nodes + 2;
+    kq_ranks<QL, true>(cv, ranks, Z.ranks, level_ends, g_dur, all, 1, any_many);
+    KE_STAMP(3);
+    kq_positions<QL, 1>(cv, all, keep, l_own, l_chain, class_ends, shrink, states);
+  } else {
+    kq_ranks<QL, false>(cv, ranks, Z.ranks, level_ends, g_dur, keep, Z.parts, any_many);
+    KE_STAMP(3);
+    if (Z.parts == kq_parts_least(QL)) kq_positions<QL, kq_parts_least(QL)>(cv, ranks, keep, l_own, l_chain, class_ends, shrink, states);
+    else kq_positions<QL, 2 * kq_parts_least(QL)>(cv, ranks, keep, l_own, l_chain, class_ends, shrink, states);
+  }
   for (int x = q; x <= RPEG_MAX_V; x += QL) g_lf[x * RW] = 0.0;
   for (int r = q; r < n_rows; r += QL) g_time[r * RW] = 0.0;
   __syncthreads();

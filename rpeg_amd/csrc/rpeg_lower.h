@@ -159,7 +159,8 @@ class Lowering {
   std::vector<uint16_t> types;
   std::vector<uint8_t> type_of;               // per node
   uint8_t type_at[RPEG_MAX_V * 8 + 1][1 << RPEG_MAX_V] = {};   // (cond, blocked) -> type + 1; all zero between classes
-  int n_rows = 0;
+  int n_rows = 0, n_rank_rows = 0;
+  std::vector<int> rank_row, by_place, freed_first, freed_next, free_rows;   // per node, by place, per level, per node, rows
   // Reservation types and ready-time rows (QuadRec); false where they outgrow its fields.  W: words of a set of nodes.
   template <int W>
   bool quad_rows(const NodeRec* recs, const uint16_t* pbeg, const uint16_t* pred, int n) {
@@ -218,6 +219,36 @@ class Lowering {
     const bool fits = f();
     for (uint16_t t : types) type_at[t >> 8][t & 0xFFu] = 0;
     return fits;
+  }
+
+  // Rows of the rank pass (RankRec), level by level: a row is given on in the level behind the last one that reads it.  False
+  // where there are too many.
+  bool rank_rows(const uint16_t* pbeg, const uint16_t* pred, int n, int n_levels) {
+    rank_row.resize(n); by_place.resize(n); freed_next.resize(n);
+    freed_first.assign(n_levels, -1);   // per level: the nodes whose rows it reads last
+    for (int v = 0; v < n; ++v) by_place[place[v]] = v;
+    free_rows.clear();
+    n_rank_rows = 2;
+    for (int l = 0; l < n_levels; ++l) {
+      if (l > 0)
+        for (int v = freed_first[l - 1]; v >= 0; v = freed_next[v]) free_rows.push_back(rank_row[v]);
+      for (int i = lbeg[l]; i < lbeg[l + 1]; ++i) {
+        const int v = by_place[i];
+        int last = -1;
+        for (int j = pbeg[v]; j < pbeg[v + 1]; ++j) last = std::max(last, level[pred[j]]);
+        rank_row[v] = 1;
+        if (last < 0) continue;
+        if (free_rows.empty()) {
+          rank_row[v] = n_rank_rows++;
+        } else {
+          rank_row[v] = free_rows.back();
+          free_rows.pop_back();
+        }
+        freed_next[v] = freed_first[last];
+        freed_first[last] = v;
+      }
+    }
+    return n_rank_rows <= (int)RANK_ROWS;
   }
 
   int slot(const SigView& sg, SlotType t, int a, int b, int q) {
@@ -544,7 +575,7 @@ class Lowering {
     h.off_place = (uint32_t)off; off = align8(off + (size_t)n * 2);
     h.off_glvl = (uint32_t)off; off = align8(off + (size_t)n_gm * 2);
     h.off_qrec = (uint32_t)off;
-    if (few_lanes) off = align8(off + (size_t)n * 4);
+    if (few_lanes) off = align8(rank_rec_offset(h) + ((size_t)n + 2) * sizeof(RankRec));
     h.off_type = (uint32_t)off;   // (the last one: its length is known when the nodes are)
     off = (off + 15) & ~size_t(15);   // (blobs start on sixteen-byte boundaries of the pool)
     out.blob.assign(off + (few_lanes ? 2 * QUAD_TYPES : 0), 0);
@@ -596,7 +627,7 @@ class Lowering {
     for (int i = 0; i < n; ++i) { cur[i] = pbeg[i]; pbeg[i + 1] = (uint16_t)(pbeg[i] + indeg[i]); }
     for (auto& ed : edges) pred[cur[ed.second]++] = (uint16_t)ed.first;
     if (few_lanes) {
-      if (chains_in_sequence(chain_beg.data(), (size_t)nv * K, chain_of.data(), adj_beg.data(), adj_to.data(), recs) && quad_rows(recs, pbeg, pred, n)) {
+      if (chains_in_sequence(chain_beg.data(), (size_t)nv * K, chain_of.data(), adj_beg.data(), adj_to.data(), recs) && quad_rows(recs, pbeg, pred, n) && rank_rows(pbeg, pred, n, n_levels)) {
         h.n_rows = (uint32_t)n_rows;
         h.n_types = (uint32_t)types.size();
         std::memcpy(B + h.off_type, types.data(), types.size() * 2);
@@ -624,6 +655,7 @@ class Lowering {
       place16[v] = (uint16_t)place[v];
     }
     OrderRec* const orec = (OrderRec*)(B + h.off_orec);
+    RankRec* const rrec = (RankRec*)(B + rank_rec_offset(h));   // (with rows)
     int first[257] = {}, next[256];
     for (int v = 0; v < n; ++v) ++first[recs[v].ptkey + 1];
     for (int k = 0; k < 256; ++k) { next[k] = first[k]; first[k + 1] += first[k]; }
@@ -635,7 +667,19 @@ class Lowering {
     }
     for (int v = 0; v < n; ++v) {
       const int k = recs[v].ptkey;
+      if (h.n_rows) {
+        RankRec r{};
+        for (int j = 0; j < 4 && j < recs[v].n_succ; ++j) r.succ[j] = (uint8_t)rank_row[adj_to[adj_beg[v] + j]];
+        r.row = (uint8_t)rank_row[v];
+        r.slot = recs[v].slot;
+        r.id = (uint16_t)((uint32_t)next[k] | (recs[v].n_succ > 4 ? RANK_MORE : 0u));
+        rrec[place[v]] = r;
+      }
       orec[next[k]++] = OrderRec{(uint16_t)place[v], (uint16_t)first[k], (uint16_t)first[k + 1], (uint8_t)chain_n[v], (uint8_t)chain_i[v]};
+    }
+    if (h.n_rows) {
+      rrec[n] = RankRec{{0, 0, 0, 0}, 1, 0, (uint16_t)n};
+      rrec[n + 1] = RankRec{{0, 0, 0, 0}, 1, 0, (uint16_t)n_rank_rows};
     }
   }
 };
