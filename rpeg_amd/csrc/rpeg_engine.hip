@@ -443,7 +443,7 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) vo
     const ClassView cv = class_view(L.pool + off);
     kp_sync();   // the previous plan of this wavefront is done with LDS
     uint32_t head = 0u;
-    if (!L.dur) {
+    if (!L.aux_ovl) {
       head = kp_load_plan(L, pi, 0u, L.P->st[cv.h->structure].n_vertex, threadIdx.x, (int16_t*)kp_lds);
       kp_sync();
     }
@@ -1205,6 +1205,34 @@ static int ensure_limit_ws(rpeg_engine_t* e, hipStream_t s) {
   return 0;
 }
 
+// What every launch of k_prologue is handed; the rows are the caller's to choose.
+static PrologueLaunch prologue_launch(const rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, const uint32_t* cid) {
+  PrologueLaunch G;
+  G.P = e->dP; G.vert = plans->vert; G.head = plans->head; G.stride = plans->stride; G.n = n; G.cid = cid;
+  G.uni = e->d_uni;
+  for (int q = 0; q < RPEG_MAX_STRUCT; ++q) G.n_uni[q] = e->n_uni[q];
+  G.max_uni = e->max_uni;
+  G.max_v = e->max_v;
+  G.dur = e->d_dur; G.dur_stride = e->cap_n;
+  G.aux_ovl = e->d_aux_ovl; G.aux_eq = e->d_aux_eq; G.aux_dpne = e->d_aux_dpne; G.vm = e->d_vm;
+  G.aux_pen = e->d_aux_pen; G.aux_mask = e->d_aux_mask;
+  G.peak = nullptr;
+  G.row_begin = G.row_end = 0;
+  return G;
+}
+// Wavefronts that share the rows of 64 plans: as many as fill the chip once.  A row is a chain of a few loads, so the launch takes
+// as long as a wavefront has rows (20,011 PPO plans, six / thirteen wavefronts: the step 308 / 300 us).
+static uint32_t prologue_parts(const rpeg_engine_t* e, const PrologueLaunch& G, uint64_t n) {
+  const uint64_t blocks = (n + WAVE - 1) / WAVE;
+  return std::min(G.row_end - G.row_begin, std::max<uint32_t>(KPRO_PARTS, (uint32_t)((uint64_t)e->n_cu * 16u / blocks)));
+}
+// The durations alone, for k_plan.  cid: KPRO_INVALID where a plan is not to be evaluated.
+static void launch_durations(const rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, const uint32_t* cid, hipStream_t s) {
+  PrologueLaunch G = prologue_launch(e, n, plans, cid);
+  G.row_end = e->max_uni;
+  hipLaunchKernelGGL(k_prologue, dim3((unsigned)((n + WAVE - 1) / WAVE), prologue_parts(e, G, n)), dim3(WAVE), 0, s, G);
+}
+
 static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, uint32_t flags, double* makespan,
                            double* peak, double* score, uint8_t* mask, double* mass, void* stream);
 static int eval_host_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, uint32_t flags, double* makespan,
@@ -1567,6 +1595,11 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     L.mass = mass; L.prof = nullptr;
     const size_t lds = kp_lds_bytes(e->max_nodes, e->max_slots);
     if (e->timing) HIP_TRY(e, hipEventRecord(e->ev0, s));
+    if (n > (uint64_t)e->n_cu * 16u) {   // more than one round of wavefronts
+      launch_durations(e, n, plans, e->d_cls, s);
+      L.dur = e->d_dur;
+      L.dur_stride = e->cap_n;
+    }
     launch_plan(lds, s, L, e->n_cu);
     HIP_TRY(e, hipGetLastError());
     if (e->timing) HIP_TRY(e, hipEventRecord(e->ev1, s));
@@ -1585,10 +1618,15 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       return 0;
     }
   }
-  // A batch small enough to get a wavefront per plan whatever its classes are (k_plan) leaves the cost model and the
-  // memory model to that kernel, which spreads them over the lanes of a plan's wavefront: the prologue launches work a
-  // plan per lane, and a few thousand plans are a few dozen wavefronts that take as long as a full grid would.
+  // A batch small enough to get a wavefront per plan whatever its classes are (k_plan) leaves the memory model to that kernel, which
+  // spreads it over the lanes of a plan's wavefront: the launches work a plan per lane, and a few thousand plans are a few dozen
+  // wavefronts that take as long as a full grid would.  The durations of its slots are a launch of their own from a quarter of that on
+  // (plan_rows): a row to a wavefront that launch takes 7-12 us while the host lays the batch out, and in k_plan, where every kind of
+  // slot is a branch of divergent code, they are 13 us of a plan's wavefront.  us a step, in k_plan / ahead of it: GRPO 9,001 plans 174 /
+  // 152; PPO 2,500 145 / 139, 4,096 154 / 149, 13,000 315 / 286; AC-share 6,000 400 / 394.  (With the memory model too, which then
+  // is another 25-50 us ahead of k_plan: 4,096 PPO plans 177, 6,000 AC-share 480.)
   const bool own_prologue = e->state_lanes == 1 || (e->state_lanes == -1 && n <= (uint64_t)e->n_cu * e->one_plan_waves_per_cu);
+  const bool plan_rows = own_prologue && e->state_lanes == -1 && n > (uint64_t)e->n_cu * DIRECT_WAVES_PER_CU;
   auto plan_fits = [&]() { return e->max_nodes <= (uint32_t)(WAVE * KP_MAX_NS) && kp_lds_bytes(e->max_nodes, e->max_slots) <= 64 * 1024; };
   bool prologue_done = false, peaks_deferred = false;
   // ahead: k_quad's stream becomes the main line of the call -- the cost-model launch goes there as soon as the class
@@ -1607,19 +1645,11 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // defer: only the cost-model launch now; the memory-model launch (k_peaks) goes out beside the scheduling kernels,
   // which need nothing of it, and k_finish applies its verdicts when all of them are done
   auto launch_prologue = [&](bool defer) -> int {
-    G.P = e->dP; G.vert = plans->vert; G.head = plans->head; G.stride = plans->stride; G.n = n; G.cid = e->d_cid;
-    G.uni = e->d_uni;
-    for (int q = 0; q < RPEG_MAX_STRUCT; ++q) G.n_uni[q] = e->n_uni[q];
-    G.max_uni = e->max_uni;
-    G.max_v = e->max_v;
-    G.dur = e->d_dur; G.dur_stride = e->cap_n;
-    G.aux_ovl = e->d_aux_ovl; G.aux_eq = e->d_aux_eq; G.aux_dpne = e->d_aux_dpne; G.vm = e->d_vm;
-    G.aux_pen = e->d_aux_pen; G.aux_mask = e->d_aux_mask;
+    G = prologue_launch(e, n, plans, e->d_cid);
     G.peak = peak;
-    const unsigned pblk = (unsigned)((n + WAVE - 1) / WAVE);
-    G.row_begin = 0;
     G.row_end = e->max_uni + 1 + (defer ? 0 : e->max_v);
-    hipLaunchKernelGGL(k_prologue, dim3(pblk, KPRO_PARTS), dim3(WAVE), 0, ahead ? e->s3 : s, G);
+    const unsigned pblk = (unsigned)((n + WAVE - 1) / WAVE);
+    hipLaunchKernelGGL(k_prologue, dim3(pblk, prologue_parts(e, G, n)), dim3(WAVE), 0, ahead ? e->s3 : s, G);
     if (!defer) hipLaunchKernelGGL(k_peaks, dim3(pblk), dim3(WAVE), kpeaks_lds_bytes(e->max_v), s, G);
     HIP_TRY(e, hipGetLastError());
     prologue_done = true;
@@ -1679,6 +1709,10 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     if (round == 0) {
       if (!own_prologue && !ahead)
         if (int rc = launch_prologue(true)) return rc;
+      if (plan_rows) {
+        launch_durations(e, n, plans, e->d_cid, s);
+        HIP_TRY(e, hipGetLastError());
+      }
       t_counts = std::chrono::steady_clock::now();
       bool seen = false;
       for (uint64_t spins = 0;; ++spins) {
@@ -2292,6 +2326,9 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   if (prologue_done) {
     L.dur = e->d_dur; L.aux_ovl = e->d_aux_ovl; L.aux_dpne = e->d_aux_dpne;
     if (!peaks_deferred) { L.aux_pen = e->d_aux_pen; L.aux_mask = e->d_aux_mask; }
+    L.dur_stride = e->cap_n;
+  } else if (plan_rows && one) {
+    L.dur = e->d_dur;
     L.dur_stride = e->cap_n;
   }
   const bool bounded = !one;   // some kernel of this call holds a bounded ready set

@@ -63,8 +63,8 @@ struct EvalLaunch {              // uniform launch parameters
   uint32_t* cstat = nullptr;     // per class (ClassHdr::id), of its slowest 64-plan wavefront so far: microseconds
                                  // << 12 | heap pops per dispatch in sixteenths; or null
   uint32_t* cneed = nullptr;     // per class: the longest ready set of its plans so far; or null
-  // What the prologue launches (rpeg_kernel_prologue.h) computed for every plan of the call, indexed by plan.  All null
-  // where a kernel computes these itself (the single-plan kernel without a layout).
+  // What the prologue launches (rpeg_kernel_prologue.h) computed for every plan of the call, indexed by plan.  Null where k_plan
+  // computes these itself: all of them, or all but the durations.
   const double* dur = nullptr;         // [universe slot][plan], rows dur_stride apart; NaN where the reference would raise
   const uint64_t* aux_ovl = nullptr;   // PlanMasks::ovl
   const uint64_t* aux_dpne = nullptr;  // PlanMasks::dpne

@@ -14,7 +14,8 @@
 // any dispatched node whose reserved vertices intersect its own.  Every lane keeps that maximum for its nodes and raises
 // it at each dispatch (max is exact, so the order does not matter).
 //
-// As a task of a laid-out batch durations, pair relations, penalty factor and gate bits come from the prologue launches.
+// As a task of a full batch durations, pair relations, penalty factor and gate bits come from the prologue launches; in a batch that
+// gets a wavefront per plan throughout the durations do (EvalLaunch::dur without ::aux_ovl).
 #ifndef RPEG_KERNEL_PLAN_H
 #define RPEG_KERNEL_PLAN_H
 
@@ -418,7 +419,7 @@ __device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const
   pm.ovl = pm.eq = pm.dpne = 0;
   bool err = cv.h->error != 0, stale_ok = false, mem_ok = false;
   double peak = -1.0, pen = 1.0;
-  if (NW == 1 && L.dur) {
+  if (NW == 1 && L.aux_ovl) {
     // a task of a laid-out batch: the prologue launches have left the durations of the slot universe, the pair
     // relations, the penalty factor and the gate bits by plan index (and written the peak themselves)
     const uint64_t sp = pi;
@@ -455,7 +456,15 @@ __device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const
     }
 
     // ---- durations of the class's slots, one slot per lane
-    if (NW == 1 || wave < 3) {
+    if (NW == 1 && L.dur) {   // (the prologue launch has left those of the slot universe)
+      bool bad = false;
+      for (int s = lane; s < n_slots; s += KE_WAVE) {
+        const double d = L.dur[(size_t)cv.umap[s] * L.dur_stride + pi];
+        l_dur[s] = d;
+        bad = bad || d != d;
+      }
+      err = err || __ballot(bad) != 0ull;
+    } else if (NW == 1 || wave < 3) {
       bool zero_div = false;
       const int split = (int)cv.h->split;
       for (int s = lane; s < n_slots; s += KE_WAVE) {
@@ -565,7 +574,7 @@ __device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const
   if (lane == 0) {
     if (TR == KP_TIMES_ORDER && L.util) L.util[pi] = util;
     if (L.makespan) L.makespan[pi] = out_makespan;
-    if (L.peak && !L.dur) L.peak[pi] = peak;   // (with a prologue launch the peak is that launch's output)
+    if (L.peak && !L.aux_ovl) L.peak[pi] = peak;   // (where the memory model is a launch of its own the peak is its output)
     if (L.score) L.score[pi] = out_score;
     if (L.mask) L.mask[pi] = mask;
   }

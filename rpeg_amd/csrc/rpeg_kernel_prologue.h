@@ -31,7 +31,7 @@
 
 namespace rpeg {
 
-constexpr int KPRO_PARTS = 6;                    // wavefronts that share the rows of a block of 64 plans
+constexpr int KPRO_PARTS = 6;                    // wavefronts that share the rows of a block of 64 plans, at least
 constexpr uint32_t KPRO_INVALID = 0xFFFFFFFFu;   // class id of a plan that breaks an integer rule: not evaluated
 
 struct PrologueLaunch {
