@@ -164,8 +164,11 @@ __global__ __launch_bounds__(HAND_BLOCK) void k_hand_counts(uint32_t* __restrict
 // and the per-class plan counts.  Blocks of SIG_BLOCK plans; shard = block mod shards.
 constexpr int SIG_BLOCK = 256, SIG_TABLE = 512;
 constexpr size_t DIRECT_MAX_CLASSES = 32;   // engines of at most this many classes evaluate small batches without a layout,
-constexpr uint64_t DIRECT_WAVES_PER_CU = 8; // and so does every batch of at most this many plans per compute unit
-constexpr uint32_t N_QUEUES = 4;   // task counters of a call's evaluation launches (main kernel, k_quad, k_plan, spare)
+constexpr uint64_t KP_RESIDENT_PER_CU = 16; // wavefronts of k_plan that a compute unit holds, by registers
+constexpr uint64_t DIRECT_PER_CU = 8;       // and so does every batch of at most this many plans per compute unit
+// Task counters of a call's evaluation launches (the main kernel's), what k_deal says of classes not lowered, and the two of
+// k_class_direct: plans of such classes, and the blocks that are done (both are zero between launches).
+constexpr uint32_t N_QUEUES = 4, Q_DEAL = 1, Q_DIRECT = 2;
 struct SigPlans {   // the plan fields of one thread's plan, a column of an LDS array [field][thread]
   const int16_t* col;
   __device__ VPlan operator[](int v) const { return ke_vplan<SIG_BLOCK>(col, v); }
@@ -276,12 +279,13 @@ __global__ __launch_bounds__(SIG_BLOCK) void k_signature(
 // table of the classes lowered so far, the pool offset of the plan's class blob, written to cls[i] for the
 // single-plan kernel (KP_SKIP for a plan that is not evaluated).  Plans that break a rule get the outputs
 // k_signature gives them; plans of a class that is not on the device yet get NaN outputs, RPEG_MASK_ERROR and
-// are counted in counters[0].
+// are counted in counters[0].  With a host flag the block that is done last (counters[1]) hands the count to the host, as
+// k_hand_counts does, and leaves both counters at zero.
 __global__ __launch_bounds__(SIG_BLOCK) void k_class_direct(
     const rpeg_problem_t* __restrict__ P, uint64_t n, const int16_t* __restrict__ vert,
     const uint8_t* __restrict__ head, uint64_t stride, double* makespan, double* peak, double* score, uint8_t* mask,
     double* mass, const uint64_t* __restrict__ hkey, const uint32_t* __restrict__ hoff, uint32_t hmask,
-    uint32_t* __restrict__ cls, uint32_t* __restrict__ counters) {
+    uint32_t* __restrict__ cls, uint32_t* __restrict__ counters, uint32_t* __restrict__ host_count, uint32_t* __restrict__ host_flag, uint32_t tag) {
   __shared__ int16_t s_plan[RPEG_MAX_V * RPEG_FIELDS * SIG_BLOCK];
   const uint64_t i = (uint64_t)blockIdx.x * SIG_BLOCK + threadIdx.x;
   const bool active = i < n;
@@ -313,6 +317,14 @@ __global__ __launch_bounds__(SIG_BLOCK) void k_class_direct(
   }
   const unsigned long long u = __ballot(unknown);
   if (u && (threadIdx.x & (WAVE - 1)) == 0) atomicAdd(&counters[0], (uint32_t)__builtin_popcountll(u));
+  if (!host_flag) return;
+  __threadfence();
+  __syncthreads();
+  if (threadIdx.x == 0 && atomicAdd(&counters[1], 1u) == gridDim.x - 1u) {
+    host_count[0] = atomicExch(&counters[0], 0u);
+    atomicExch(&counters[1], 0u);
+    __hip_atomic_store(host_flag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 // cbase[class * shards + shard]: plans of the class in lower shards; shard as in k_signature.
@@ -322,7 +334,7 @@ __global__ void k_scatter(uint64_t n, const uint32_t* __restrict__ cid, const ui
                           uint32_t pstride, const uint32_t* __restrict__ coff, uint32_t* __restrict__ task_cls,
                           uint32_t first_entry, uint32_t* __restrict__ queues, uint32_t* __restrict__ limit) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < N_QUEUES) queues[i] = 0u;   // the task counters of the evaluation kernels that follow on this stream
+  if (i < Q_DEAL) queues[i] = 0u;     // the task counters of the evaluation kernels that follow on this stream
   if (i == 0) limit[0] = 0u;          // and the count of plans for the launch that ends the call
   if (i >= n) return;
   const uint32_t c = cid[i];
@@ -332,6 +344,116 @@ __global__ void k_scatter(uint64_t n, const uint32_t* __restrict__ cid, const ui
     perm[(uint64_t)cfirst[c] + k] = (uint32_t)i;
     task_cls[cfirst[c] + k - first_entry] = coff[c];
   } else perm[(uint64_t)(cfirst[c] + k / l) * pstride + k % l] = (uint32_t)i;
+}
+
+// The layout of a batch that gets a wavefront per plan, by a block of its own: the classes one after the other in `order` (largest
+// graphs first: their wavefronts run longest), and within a class the shards in turn.  The counters are left clear for the engine's
+// next call; start[class * shards + shard]: the first task of the class's plans of that shard.  Tasks without a plan are KP_SKIP, and
+// all of them where the batch has plans of classes not lowered yet (k_deal_plans then deals nothing).  host_count, behind the
+// place of the totals: as from k_hand_counts, and the classes of the batch and their plans.
+// Bound: latency, and the accesses of one compute unit, a line for a class: its shards' counters are one load and one store
+// (4,096 PPO plans, 2,005 classes: 11 us; 13,000, 3,400 classes of four shards: a word at a time 38, now 15).
+constexpr uint32_t DEAL_SHARDS = 4;   // (of a batch of at most 16,384 plans)
+template <uint32_t N> struct alignas(4 * N) DealRow { uint32_t of[N]; };
+template <uint32_t SHARDS>
+__global__ __launch_bounds__(HAND_BLOCK) void k_deal(uint32_t* __restrict__ count, uint32_t n_classes, const uint32_t* __restrict__ order,
+                                                     uint32_t* __restrict__ start, uint32_t n, uint32_t* __restrict__ task_cls, uint32_t* __restrict__ unknown,
+                                                     const uint32_t* __restrict__ need, const uint32_t* __restrict__ limit,
+                                                     uint32_t* __restrict__ host_count, uint32_t* __restrict__ host_flag, uint32_t tag) {
+  using Row = DealRow<SHARDS>;
+  __shared__ uint32_t wave_total[HAND_BLOCK / WAVE], present;
+  const uint32_t lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  Row* const rows = (Row*)count;
+  const uint32_t not_lowered = count[(size_t)n_classes * SHARDS], redone = limit[0];
+  if (threadIdx.x == 0) present = 0u;
+  // a stretch of the order for every thread, four classes at a time
+  constexpr uint32_t AT_ONCE = 4;
+  const uint32_t each = (n_classes + HAND_BLOCK - 1) / HAND_BLOCK, k_begin = threadIdx.x * each, k_end = k_begin + each < n_classes ? k_begin + each : n_classes;
+  uint32_t c[AT_ONCE];
+  Row v[AT_ONCE];
+  auto fetch = [&](uint32_t k) {
+#pragma unroll
+    for (uint32_t j = 0; j < AT_ONCE; ++j) c[j] = k + j < k_end ? order[k + j] : n_classes;
+#pragma unroll
+    for (uint32_t j = 0; j < AT_ONCE; ++j) {
+      if (c[j] < n_classes) v[j] = rows[c[j]];
+      else
+#pragma unroll
+        for (uint32_t q = 0; q < SHARDS; ++q) v[j].of[q] = 0u;
+    }
+  };
+  uint32_t total = 0, met = 0;
+  for (uint32_t k = k_begin; k < k_end; k += AT_ONCE) {
+    fetch(k);
+#pragma unroll
+    for (uint32_t j = 0; j < AT_ONCE; ++j) {
+      uint32_t plans = 0;
+#pragma unroll
+      for (uint32_t q = 0; q < SHARDS; ++q) plans += v[j].of[q];
+      total += plans;
+      met += plans ? 1u : 0u;
+    }
+  }
+  uint32_t upto = total;
+#pragma unroll
+  for (uint32_t off = 1; off < WAVE; off <<= 1) {
+    const uint32_t o = (uint32_t)__shfl_up((int)upto, off);
+    upto += lane >= off ? o : 0u;
+  }
+  if (lane == WAVE - 1) wave_total[wave] = upto;
+  __syncthreads();
+  if (met) atomicAdd(&present, met);
+  uint32_t before = 0, base = 0;   // tasks of the wavefronts before, of all classes
+#pragma unroll
+  for (uint32_t w = 0; w < HAND_BLOCK / WAVE; ++w) {
+    const uint32_t t = wave_total[w];
+    before += w < wave ? t : 0u;
+    base += t;
+  }
+  uint32_t at = before + upto - total;
+  for (uint32_t k = k_begin; k < k_end; k += AT_ONCE) {
+    if (each > AT_ONCE) fetch(k);
+#pragma unroll
+    for (uint32_t j = 0; j < AT_ONCE; ++j) {
+      if (c[j] >= n_classes) continue;
+      Row first, zero;
+#pragma unroll
+      for (uint32_t q = 0; q < SHARDS; ++q) {
+        first.of[q] = at;
+        zero.of[q] = 0u;
+        at += v[j].of[q];
+      }
+      ((Row*)start)[c[j]] = first;
+      rows[c[j]] = zero;
+    }
+  }
+  for (uint32_t i = (not_lowered ? 0u : base) + threadIdx.x; i < n; i += HAND_BLOCK) task_cls[i] = KP_SKIP;
+  __syncthreads();
+  if (threadIdx.x < KE_NEED_SHARDS) host_count[n_classes + 1 + threadIdx.x] = need[threadIdx.x];
+  if (threadIdx.x == 0) {
+    host_count[n_classes] = *unknown = not_lowered;
+    host_count[n_classes + 1 + KE_NEED_SHARDS] = redone;
+    host_count[n_classes + 2 + KE_NEED_SHARDS] = present;
+    host_count[n_classes + 3 + KE_NEED_SHARDS] = base;
+  }
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    count[(size_t)n_classes * SHARDS] = 0u;
+    __hip_atomic_store(host_flag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+__global__ void k_deal_plans(uint32_t n, const uint32_t* __restrict__ cid, const uint32_t* __restrict__ kidx, const uint32_t* __restrict__ start,
+                             uint32_t shards, const uint32_t* __restrict__ coff, uint32_t* __restrict__ perm, uint32_t* __restrict__ task_cls,
+                             const uint32_t* __restrict__ unknown, uint32_t* __restrict__ limit) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) limit[0] = 0u;   // (as k_scatter)
+  if (i >= n || *unknown) return;
+  const uint32_t c = cid[i];
+  if (c >= CID_UNKNOWN) return;
+  const uint32_t task = start[c * shards + ((i / SIG_BLOCK) & (shards - 1u))] + kidx[i];
+  perm[task] = i;
+  task_cls[task] = coff[c];
 }
 
 // The prologue launches (rpeg_kernel_prologue.h), a thread per plan in the caller's order.  The structure decides
@@ -849,6 +971,7 @@ struct rpeg_engine_s {
   size_t dur_cap = 0;
   SlotDesc* d_uni = nullptr;
   uint32_t n_uni[RPEG_MAX_STRUCT] = {0, 0, 0}, max_uni = 0;
+  uint32_t* d_order = nullptr;                  // class ids, largest graphs first, then the pool offset of every class (ensure_class_tables)
   uint32_t* d_queues = nullptr;                 // N_QUEUES task counters, cleared by k_scatter
   uint32_t* d_limit = nullptr;                  // count, then (plan, class offset) pairs: plans to redo without a bound on the ready set
   uint8_t* d_limit_ws = nullptr;                // state of the launch that redoes them
@@ -914,11 +1037,12 @@ static int ensure_class_tables(rpeg_engine_t* e, hipStream_t s) {
   uint32_t hcap = 1024;
   while (hcap < 4 * ncls) hcap *= 2;
   if (hcap != e->hcap) {
-    if (e->d_hkey) { hipFree(e->d_hkey); hipFree(e->d_hval); hipFree(e->d_hoff); }
+    if (e->d_hkey) { hipFree(e->d_hkey); hipFree(e->d_hval); hipFree(e->d_hoff); hipFree(e->d_order); }
     e->d_hkey = nullptr; e->hcap = 0;
     HIP_TRY(e, hipMalloc(&e->d_hkey, (size_t)hcap * 8));
     HIP_TRY(e, hipMalloc(&e->d_hval, (size_t)hcap * 4));
     HIP_TRY(e, hipMalloc(&e->d_hoff, (size_t)hcap * 4));
+    HIP_TRY(e, hipMalloc(&e->d_order, (size_t)hcap * 4));   // (four times the classes: twice as many as it needs)
     e->hcap = hcap;
   }
   std::vector<uint64_t> hk(hcap, SIG_INVALID);
@@ -933,6 +1057,13 @@ static int ensure_class_tables(rpeg_engine_t* e, hipStream_t s) {
   HIP_TRY(e, hipMemcpy(e->d_hkey, hk.data(), (size_t)hcap * 8, hipMemcpyHostToDevice));
   HIP_TRY(e, hipMemcpy(e->d_hval, hv.data(), (size_t)hcap * 4, hipMemcpyHostToDevice));
   HIP_TRY(e, hipMemcpy(e->d_hoff, ho.data(), (size_t)hcap * 4, hipMemcpyHostToDevice));
+  // classes with the largest graphs first (kept from call to call: sorting the ten thousand of config 3 in every call took 0.4 ms)
+  e->cls_sorted.resize(ncls);
+  for (uint32_t c = 0; c < ncls; ++c) e->cls_sorted[c] = c;
+  std::stable_sort(e->cls_sorted.begin(), e->cls_sorted.end(), [&](uint32_t a, uint32_t b) { return e->cls_nodes[a] > e->cls_nodes[b]; });
+  std::copy_n(e->cls_sorted.begin(), ncls, ho.begin());
+  std::copy_n(e->cls_off.begin(), ncls, ho.begin() + ncls);
+  HIP_TRY(e, hipMemcpy(e->d_order, ho.data(), 2 * (size_t)ncls * 4, hipMemcpyHostToDevice));
   if (ncls + 1 > e->ccap) {
     const uint32_t cap = std::max<uint32_t>(2 * (ncls + 1), 4096);
     if (e->d_ccount) {
@@ -1233,6 +1364,46 @@ static void launch_durations(const rpeg_engine_t* e, uint64_t n, const rpeg_plan
   hipLaunchKernelGGL(k_prologue, dim3((unsigned)((n + WAVE - 1) / WAVE), prologue_parts(e, G, n)), dim3(WAVE), 0, s, G);
 }
 
+static uint32_t next_tag(rpeg_engine_t* e) { return ++e->sig_tag ? e->sig_tag : ++e->sig_tag; }
+// Until a kernel on s has handed over what it was to hand over with this tag; a launch that does not come to an end is the stream's
+// to report.
+static int wait_tag(rpeg_engine_t* e, hipStream_t s, uint32_t tag) {
+  const auto begin = std::chrono::steady_clock::now();
+  for (uint64_t spins = 0; __atomic_load_n(e->h_sigflag, __ATOMIC_ACQUIRE) != tag; ++spins) {
+    if ((spins & 0xFFFFu) == 0xFFFFu && std::chrono::steady_clock::now() - begin > std::chrono::seconds(2)) {
+      HIP_TRY(e, hipStreamSynchronize(s));
+      if (__atomic_load_n(e->h_sigflag, __ATOMIC_ACQUIRE) == tag) break;
+      e->err = "a launch ended without its hand-over";
+      return -5;
+    }
+#if defined(__x86_64__) || defined(__i386__)
+    __builtin_ia32_pause();
+#endif
+  }
+  return 0;
+}
+static int read_timing(rpeg_engine_t* e) {
+  if (!e->timing) return 0;
+  HIP_TRY(e, hipEventSynchronize(e->ev1));
+  float ms = 0.f;
+  HIP_TRY(e, hipEventElapsedTime(&ms, e->ev0, e->ev1));
+  e->last_ms = ms;
+  return 0;
+}
+
+// A launch of k_plan over n plans; tasks and durations are the caller's to say.
+static EvalLaunch plan_launch(const rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, uint32_t flags, double* makespan, double* peak,
+                              double* score, uint8_t* mask, double* mass) {
+  EvalLaunch L;
+  L.P = e->dP; L.vert = plans->vert; L.head = plans->head; L.stride = plans->stride;
+  L.perm = nullptr; L.wave_cls = nullptr; L.pool = e->d_pool; L.ws = nullptr;
+  L.n_waves = n; L.ws_nodes = e->max_nodes; L.ws_slots = e->max_slots;
+  L.cls_bytes = 0; L.rcap = 0; L.max_v = e->max_v; L.ovf = nullptr; L.need = nullptr;
+  L.flags = flags; L.makespan = makespan; L.peak = peak; L.score = score; L.mask = mask;
+  L.mass = mass; L.prof = nullptr;
+  return L;
+}
+
 static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, uint32_t flags, double* makespan,
                            double* peak, double* score, uint8_t* mask, double* mass, void* stream);
 static int eval_host_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, uint32_t flags, double* makespan,
@@ -1312,7 +1483,7 @@ void rpeg_engine_destroy(rpeg_engine_t* e) {
   if (e->d_need) hipFree(e->d_need);
   if (e->d_queues) hipFree(e->d_queues);
   if (e->d_cstat) hipFree(e->d_cstat);
-  if (e->d_hkey) { hipFree(e->d_hkey); hipFree(e->d_hval); hipFree(e->d_hoff); }
+  if (e->d_hkey) { hipFree(e->d_hkey); hipFree(e->d_hval); hipFree(e->d_hoff); hipFree(e->d_order); }
   if (e->h_static) hipHostFree(e->h_static);
   if (e->h_sigflag) hipHostFree(e->h_sigflag);
   if (e->h_tot) hipHostFree(e->h_tot);
@@ -1566,36 +1737,31 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   if (int rc = ensure_batch(e, n)) return rc;
   const unsigned blk = 256;
   const unsigned nblk = (unsigned)((n + blk - 1) / blk);
-  // A batch that gets one wavefront per plan whatever its classes are needs no layout: every plan finds the pool
+  // A batch that gets one wavefront (or four) per plan whatever its classes are needs no layout: every plan finds the pool
   // offset of its class through the table of the classes lowered so far, k_plan takes the plans in their own order,
-  // and the host only learns afterwards whether a plan belonged to a class not lowered yet (then the call goes the
-  // long way below and evaluates the batch again).  Two launches and one wait instead of a round trip between them.
+  // and the host learns meanwhile whether a plan belonged to a class not lowered yet (then the call goes the
+  // long way below and evaluates the batch again).  Two launches; with a fill for the count ahead of them, a copy behind and the
+  // wait for it, us a call / now: 600 DPO plans 55 / 36, 3,000 68 / 50; 900 PPO plans 124 / 105, 2,000 140 / 122; 1,500 GRPO 123 / 105;
+  // 2,000 AC-share 342 / 326.
   // Only for an engine of few classes or a batch that is resident at once with room to spare: with hundreds of
-  // classes the plans in their own order make neighbouring wavefronts work on different classes, and k_plan ran
-  // half as long again as on the sorted batch (config 2 with 8,192 plans: 0.28 against 0.19 ms; with 2,048 plans
-  // 0.17 against 0.16 ms and the step 0.21 against 0.23 ms; config 4, 16 classes, 8,192 plans: the step 0.15 against
-  // 0.18 ms).
+  // classes the plans in their own order make neighbouring wavefronts work on different classes, and k_plan runs
+  // half as long again as on the sorted batch, which k_deal makes: 8 us (2,000 PPO plans 122 / 130 us a call, 1,100 DPO plans 45 / 54).
+  // In more than one round of wavefronts the durations are worth a launch of their own (13,000 DPO plans 147 / 138 us a call).
   if ((e->state_lanes == 1 || (e->state_lanes == -1 && n <= (uint64_t)e->n_cu * e->one_plan_waves_per_cu)) && !e->prof_on &&
-      !e->cls_sig.empty() && (e->cls_sig.size() <= DIRECT_MAX_CLASSES || n <= (uint64_t)e->n_cu * DIRECT_WAVES_PER_CU) && e->d_hkey && e->tables_for == (uint32_t)e->cls_sig.size() && e->d_pool &&
-      e->d_pool_used == e->pool_size && e->max_nodes <= (uint32_t)(WAVE * KP_MAX_NS) &&
-      kp_lds_bytes(e->max_nodes, e->max_slots) <= 64 * 1024) {
+      !e->cls_sig.empty() && (e->cls_sig.size() <= DIRECT_MAX_CLASSES || n <= (uint64_t)e->n_cu * DIRECT_PER_CU) && e->d_hkey &&
+      e->tables_for == (uint32_t)e->cls_sig.size() && e->d_pool && e->d_pool_used == e->pool_size &&
+      e->max_nodes <= (uint32_t)(WAVE * KP_MAX_NS) && kp_lds_bytes(e->max_nodes, e->max_slots) <= 64 * 1024) {
     if (int rc = ensure_perm(e, 0, n)) return rc;
-    uint32_t* const d_unknown = e->d_queues + (N_QUEUES - 1);
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, d_unknown, (uint64_t)1, 0u);
+    const uint32_t tag = next_tag(e);
     hipLaunchKernelGGL(k_class_direct, dim3((unsigned)((n + SIG_BLOCK - 1) / SIG_BLOCK)), dim3(SIG_BLOCK), 0, s, e->dP, n,
                        plans->vert, plans->head, plans->stride, makespan, peak, score, mask, mass, e->d_hkey, e->d_hoff,
-                       e->hcap - 1, e->d_cls, d_unknown);
+                       e->hcap - 1, e->d_cls, e->d_queues + Q_DIRECT, e->h_tot_dev, e->h_sigflag_dev, tag);
     HIP_TRY(e, hipGetLastError());
-    EvalLaunch L;
-    L.P = e->dP; L.vert = plans->vert; L.head = plans->head; L.stride = plans->stride;
-    L.perm = nullptr; L.wave_cls = e->d_cls; L.pool = e->d_pool; L.ws = nullptr;
-    L.n_waves = n; L.ws_nodes = e->max_nodes; L.ws_slots = e->max_slots;
-    L.cls_bytes = 0; L.rcap = 0; L.max_v = e->max_v; L.ovf = nullptr; L.need = nullptr;
-    L.flags = flags; L.makespan = makespan; L.peak = peak; L.score = score; L.mask = mask;
-    L.mass = mass; L.prof = nullptr;
+    EvalLaunch L = plan_launch(e, n, plans, flags, makespan, peak, score, mask, mass);
+    L.wave_cls = e->d_cls;
     const size_t lds = kp_lds_bytes(e->max_nodes, e->max_slots);
     if (e->timing) HIP_TRY(e, hipEventRecord(e->ev0, s));
-    if (n > (uint64_t)e->n_cu * 16u) {   // more than one round of wavefronts
+    if (n > (uint64_t)e->n_cu * KP_RESIDENT_PER_CU) {
       launch_durations(e, n, plans, e->d_cls, s);
       L.dur = e->d_dur;
       L.dur_stride = e->cap_n;
@@ -1603,30 +1769,24 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     launch_plan(lds, s, L, e->n_cu);
     HIP_TRY(e, hipGetLastError());
     if (e->timing) HIP_TRY(e, hipEventRecord(e->ev1, s));
-    HIP_TRY(e, hipMemcpyAsync(e->h_ccount, d_unknown, 4, hipMemcpyDeviceToHost, s));
-    HIP_TRY(e, hipStreamSynchronize(s));
-    if (e->h_ccount[0] == 0u) {
+    if (int rc = wait_tag(e, s, tag)) return rc;
+    if (e->h_tot[0] == 0u) {
       e->stats[0] = e->cls_sig.size();   // (the classes the engine knows: which of them the batch holds was not counted)
       e->stats[1] = 0; e->stats[2] = n; e->stats[3] = lds; e->stats[4] = 0; e->stats[5] = 1; e->stats[6] = 0;
       e->stats[7] = e->stats[9] = e->stats[10] = e->stats[11] = e->stats[12] = 0;
       ++e->batch_calls;
-      if (e->timing) {
-        float ms = 0.f;
-        HIP_TRY(e, hipEventElapsedTime(&ms, e->ev0, e->ev1));
-        e->last_ms = ms;
-      }
-      return 0;
+      return read_timing(e);
     }
   }
   // A batch small enough to get a wavefront per plan whatever its classes are (k_plan) leaves the memory model to that kernel, which
   // spreads it over the lanes of a plan's wavefront: the launches work a plan per lane, and a few thousand plans are a few dozen
-  // wavefronts that take as long as a full grid would.  The durations of its slots are a launch of their own from a quarter of that on
-  // (plan_rows): a row to a wavefront that launch takes 7-12 us while the host lays the batch out, and in k_plan, where every kind of
+  // wavefronts that take as long as a full grid would.  The durations of its slots are a launch of their own (plan_rows): with a row
+  // to a wavefront that launch takes 7-12 us beside the layout, and in k_plan, where every kind of
   // slot is a branch of divergent code, they are 13 us of a plan's wavefront.  us a step, in k_plan / ahead of it: GRPO 9,001 plans 174 /
   // 152; PPO 2,500 145 / 139, 4,096 154 / 149, 13,000 315 / 286; AC-share 6,000 400 / 394.  (With the memory model too, which then
   // is another 25-50 us ahead of k_plan: 4,096 PPO plans 177, 6,000 AC-share 480.)
   const bool own_prologue = e->state_lanes == 1 || (e->state_lanes == -1 && n <= (uint64_t)e->n_cu * e->one_plan_waves_per_cu);
-  const bool plan_rows = own_prologue && e->state_lanes == -1 && n > (uint64_t)e->n_cu * DIRECT_WAVES_PER_CU;
+  const bool plan_rows = own_prologue && e->state_lanes == -1 && n > (uint64_t)e->n_cu * DIRECT_PER_CU;
   auto plan_fits = [&]() { return e->max_nodes <= (uint32_t)(WAVE * KP_MAX_NS) && kp_lds_bytes(e->max_nodes, e->max_slots) <= 64 * 1024; };
   bool prologue_done = false, peaks_deferred = false;
   // ahead: k_quad's stream becomes the main line of the call -- the cost-model launch goes there as soon as the class
@@ -1679,11 +1839,18 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
                            (e->learn_calls > 0 || (e->batch_calls & 63) == 0);
     // The counters go to the host through k_hand_counts (the statistic with them); in the first round the host polls its
     // flag instead of waiting for the stream.
-    const uint32_t tag = ++e->sig_tag ? e->sig_tag : ++e->sig_tag;
+    const uint32_t tag = next_tag(e);
     if (round == 0 && !own_prologue) {
       if (int rc = ensure_side(e)) return rc;
       ahead = !e->prof_on && e->layout_ahead && side_claim(e);
     }
+    // A batch for k_plan whose classes may all be lowered is laid out on the device, and everything goes out at once; the host only
+    // learns afterwards whether a plan belonged to a class not lowered yet (then the launches found nothing to do, and the call goes
+    // on the long way).  us a step, laid out by the host / on the device: PPO 2,500 139 / 132, 4,096 149 / 136, 13,000 286 / 270; GRPO
+    // 9,001 152 / 147; AC-share 6,000 394 / 388.
+    const bool deal = round == 0 && shards <= DEAL_SHARDS && plan_rows && plan_fits() && !e->prof_on && ncls && e->d_pool && e->d_pool_used == e->pool_size;
+    if (deal)
+      if (int rc = ensure_perm(e, n, n)) return rc;
     if (round > 0 && ahead) HIP_TRY(e, hipStreamSynchronize(e->s3));   // (the cost-model launch reads the class ids)
     // (clear already where the launch that ended the engine's last call did it)
     if (e->count_clean < n_count || e->count_clean_on != s)
@@ -1702,6 +1869,21 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       HIP_TRY(e, hipStreamWaitEvent(e->s3, e->ev_sig, 0));
       if (int rc = launch_prologue(true)) return rc;
     }
+    if (deal) {
+      uint32_t* const start = e->d_ccount + ((n_count + 3) & ~(uint64_t)3);
+      uint32_t* const unknown = e->d_queues + Q_DEAL;
+      hipLaunchKernelGGL(shards == 1 ? k_deal<1> : shards == 2 ? k_deal<2> : k_deal<DEAL_SHARDS>, dim3(1), dim3(HAND_BLOCK), 0, s, e->d_ccount, ncls, e->d_order, start, (uint32_t)n, e->d_cls, unknown,
+                         e->d_need, e->d_limit, e->h_tot_dev, e->h_sigflag_dev, tag);
+      launch_durations(e, n, plans, e->d_cid, s);
+      hipLaunchKernelGGL(k_deal_plans, dim3(nblk), dim3(blk), 0, s, (uint32_t)n, e->d_cid, e->d_kidx, start, shards, e->d_order + ncls, e->d_perm,
+                         e->d_cls, unknown, e->d_limit);
+      EvalLaunch L = plan_launch(e, n, plans, flags, makespan, peak, score, mask, mass);
+      L.perm = e->d_perm; L.wave_cls = e->d_cls;
+      L.dur = e->d_dur; L.dur_stride = e->cap_n;
+      if (e->timing) HIP_TRY(e, hipEventRecord(e->ev0, s));
+      launch_plan(kp_lds_bytes(e->max_nodes, e->max_slots), s, L, e->n_cu);
+      if (e->timing) HIP_TRY(e, hipEventRecord(e->ev1, s));
+    } else
     hipLaunchKernelGGL(k_hand_counts, dim3(1), dim3(HAND_BLOCK), 0, s, e->d_ccount, e->d_need, ncls, shards, e->d_limit,
                        e->d_cstat, e->d_cstat + e->cstat_cap, e->h_tot_dev, e->h_tot_dev + e->tot_words(),
                        read_stat ? e->h_tot_dev + e->tot_words() + e->ccap : nullptr, e->h_sigflag_dev, tag);
@@ -1709,21 +1891,12 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     if (round == 0) {
       if (!own_prologue && !ahead)
         if (int rc = launch_prologue(true)) return rc;
-      if (plan_rows) {
+      if (plan_rows && !deal) {
         launch_durations(e, n, plans, e->d_cid, s);
         HIP_TRY(e, hipGetLastError());
       }
       t_counts = std::chrono::steady_clock::now();
-      bool seen = false;
-      for (uint64_t spins = 0;; ++spins) {
-        if (__atomic_load_n(e->h_sigflag, __ATOMIC_ACQUIRE) == tag) { seen = true; break; }
-        // a launch that does not come to an end is the stream's to report
-        if ((spins & 0xFFFFu) == 0xFFFFu && std::chrono::steady_clock::now() - t_counts > std::chrono::seconds(2)) break;
-#if defined(__x86_64__) || defined(__i386__)
-        __builtin_ia32_pause();
-#endif
-      }
-      if (!seen) HIP_TRY(e, hipStreamSynchronize(s));
+      if (int rc = wait_tag(e, s, tag)) return rc;
       t_waited = std::chrono::steady_clock::now();
     } else {
       HIP_TRY(e, hipStreamSynchronize(s));
@@ -1734,6 +1907,20 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       e->stats[8] = e->h_tot[ncls + 1 + KE_NEED_SHARDS];
       if (e->stats[8] || read_stat) std::copy_n(e->h_tot + e->tot_words(), ncls, e->cls_need.begin());
       if (read_stat) std::copy_n(e->h_tot + e->tot_words() + e->ccap, ncls, e->cls_pops16.begin());
+    }
+    if (deal && e->h_tot[ncls] == 0) {
+      e->count_clean = n_count;
+      e->count_clean_on = s;
+      ++e->batch_calls;
+      for (uint64_t& x : e->stats) x = &x == &e->stats[8] ? x : 0;
+      e->stats[0] = e->h_tot[ncls + 2 + KE_NEED_SHARDS];
+      e->stats[2] = e->h_tot[ncls + 3 + KE_NEED_SHARDS];
+      e->stats[3] = kp_lds_bytes(e->max_nodes, e->max_slots);
+      e->stats[5] = 1;
+      e->host_us[0] = std::chrono::duration<double, std::micro>(t_counts - t_call).count();
+      e->host_us[1] = std::chrono::duration<double, std::micro>(t_waited - t_counts).count();
+      e->host_us[2] = e->host_us[3] = 0.0;
+      return read_timing(e);
     }
     if (e->h_tot[ncls] == 0) break;
     if (round >= 2) { e->err = "class table did not converge"; return -5; }
@@ -1801,13 +1988,6 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   const uint32_t lpw = one ? 1u : ls ? (uint32_t)ls : (uint32_t)WAVE;   // plans per wavefront
   // every class starts on a wavefront boundary; the lanes left over are idle
   // classes with the largest graphs first: their wavefronts run longest and should not start last
-  // (the order of all known classes is kept from call to call and only filtered here: a batch of config 3 meets
-  // over ten thousand classes, and sorting them in every call took 0.4 ms)
-  if (e->cls_sorted.size() != ncls) {
-    e->cls_sorted.resize(ncls);
-    for (uint32_t c = 0; c < ncls; ++c) e->cls_sorted[c] = c;
-    std::stable_sort(e->cls_sorted.begin(), e->cls_sorted.end(), [&](uint32_t a, uint32_t b) { return e->cls_nodes[a] > e->cls_nodes[b]; });
-  }
   e->cls_pos.assign(ncls, 0xFFFFFFFFu);
   for (size_t c = 0; c < counts.size(); ++c) e->cls_pos[cids[c]] = (uint32_t)c;
   std::vector<uint32_t> order;
@@ -2517,14 +2697,8 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     e->host_us[2] = us(t_waited, t_laid);    // layout of the batch and the split between the kernels, tables up
     e->host_us[3] = us(t_laid, t_end);       // scatter, fork, the scheduling launches, join, the launches that end the call
   }
-  if (e->timing) {
-    HIP_TRY(e, hipEventRecord(e->ev1, s));
-    HIP_TRY(e, hipEventSynchronize(e->ev1));
-    float ms = 0.f;
-    HIP_TRY(e, hipEventElapsedTime(&ms, e->ev0, e->ev1));
-    e->last_ms = ms;
-  }
-  return 0;
+  if (e->timing) HIP_TRY(e, hipEventRecord(e->ev1, s));
+  return read_timing(e);
 }
 
 // What the records of lower() hold of every node of a plan's class (arrays may be null).
@@ -2601,7 +2775,7 @@ int rpeg_eval_batch_static(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, d_counters, (uint64_t)(STATIC_COUNTER_BYTES / 4), 0u);
   hipLaunchKernelGGL(k_class_direct, dim3((unsigned)((n + SIG_BLOCK - 1) / SIG_BLOCK)), dim3(SIG_BLOCK), 0, s, e->dP, n,
                      plans->vert, plans->head, plans->stride, makespan, peak, score, mask, (double*)nullptr, e->d_hkey, e->d_hoff,
-                     e->hcap - 1, d_cls, d_counters);
+                     e->hcap - 1, d_cls, d_counters, (uint32_t*)nullptr, (uint32_t*)nullptr, 0u);
   HIP_TRY(e, hipGetLastError());
   EvalLaunch L;
   L.P = e->dP; L.vert = plans->vert; L.head = plans->head; L.stride = plans->stride;
@@ -3197,6 +3371,7 @@ static int eval_host_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* p
                          mass ? (double*)(d + o_ms) : nullptr, stream);
   }
   const double last_ms = e->last_ms;
+  if (!rc && (st = hipStreamSynchronize(s)) != hipSuccess) fail(st, "hipStreamSynchronize");   // (a copy command behind running kernels starts late)
   if (!rc && (st = hipMemcpyAsync(e->h_stage, d + o_mk, b_out, hipMemcpyDeviceToHost, s)) != hipSuccess) fail(st, "hipMemcpyAsync");
   const hipError_t sy = hipStreamSynchronize(s);
   if (!rc && sy != hipSuccess) fail(sy, "hipStreamSynchronize");
