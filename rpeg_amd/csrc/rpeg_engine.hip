@@ -167,8 +167,8 @@ constexpr size_t DIRECT_MAX_CLASSES = 32;   // engines of at most this many clas
 constexpr uint64_t KP_RESIDENT_PER_CU = 16; // wavefronts of k_plan that a compute unit holds, by registers
 constexpr uint64_t DIRECT_PER_CU = 8;       // and so does every batch of at most this many plans per compute unit
 // Task counters of a call's evaluation launches (the main kernel's), what k_deal says of classes not lowered, and the two of
-// k_class_direct: plans of such classes, and the blocks that are done (both are zero between launches).
-constexpr uint32_t N_QUEUES = 4, Q_DEAL = 1, Q_DIRECT = 2;
+// k_class_direct: plans of such classes, and the blocks that are done; the blocks of k_copy that are (zero between launches).
+constexpr uint32_t N_QUEUES = 5, Q_DEAL = 1, Q_DIRECT = 2, Q_COPY = 4;
 struct SigPlans {   // the plan fields of one thread's plan, a column of an LDS array [field][thread]
   const int16_t* col;
   __device__ VPlan operator[](int v) const { return ke_vplan<SIG_BLOCK>(col, v); }
@@ -344,6 +344,22 @@ __global__ void k_scatter(uint64_t n, const uint32_t* __restrict__ cid, const ui
     perm[(uint64_t)cfirst[c] + k] = (uint32_t)i;
     task_cls[cfirst[c] + k - first_entry] = coff[c];
   } else perm[(uint64_t)(cfirst[c] + k / l) * pstride + k % l] = (uint32_t)i;
+}
+
+// Between pinned host memory and the device, sixteen bytes a thread, in order on the call's stream: no other engine's signal to
+// wait for, no command queue of its own.  With a flag the block that is done last hands over the tag (done: a counter, zero between
+// launches).
+constexpr uint32_t COPY_BLOCK = 256;
+__global__ __launch_bounds__(COPY_BLOCK) void k_copy(uint4* __restrict__ to, const uint4* __restrict__ from, uint64_t n, uint32_t* __restrict__ done,
+                                                     uint32_t* __restrict__ host_flag, uint32_t tag) {
+  for (uint64_t i = (uint64_t)blockIdx.x * COPY_BLOCK + threadIdx.x; i < n; i += (uint64_t)gridDim.x * COPY_BLOCK) to[i] = from[i];
+  if (!host_flag) return;
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0 && atomicAdd(done, 1u) == gridDim.x - 1u) {
+    atomicExch(done, 0u);
+    __hip_atomic_store(host_flag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 // The layout of a batch that gets a wavefront per plan, by a block of its own: the classes one after the other in `order` (largest
@@ -914,10 +930,9 @@ struct rpeg_engine_s {
   // staging of the host-pointer path: plans and class offsets in (pinned, then device), results out (pinned,
   // written by the kernel itself)
   HostLane lane0;
-  uint8_t* d_stage = nullptr;   // device copy of host tensors and results for larger host-pointer batches
-  size_t d_stage_cap = 0;
-  uint8_t* h_stage = nullptr;   // pinned mirror of the result region of d_stage
-  size_t h_stage_cap = 0;
+  uint8_t* d_stage = nullptr;   // host tensors and results of larger host-pointer batches on the device
+  uint8_t *h_stage = nullptr, *h_stage_dev = nullptr;   // and its pinned mirror
+  size_t stage_cap = 0;
   uint8_t *h_times = nullptr, *h_times_dev = nullptr;   // pinned: EvalLaunch::trace
   size_t h_times_nodes = 0;
   uint8_t* d_trace = nullptr;   // rpeg_eval_trace: one plan's fields and header, then start / finish / dispatch index
@@ -1367,12 +1382,12 @@ static void launch_durations(const rpeg_engine_t* e, uint64_t n, const rpeg_plan
 static uint32_t next_tag(rpeg_engine_t* e) { return ++e->sig_tag ? e->sig_tag : ++e->sig_tag; }
 // Until a kernel on s has handed over what it was to hand over with this tag; a launch that does not come to an end is the stream's
 // to report.
-static int wait_tag(rpeg_engine_t* e, hipStream_t s, uint32_t tag) {
+static int wait_tag(rpeg_engine_t* e, hipStream_t s, uint32_t tag, uint32_t flag = 0) {
   const auto begin = std::chrono::steady_clock::now();
-  for (uint64_t spins = 0; __atomic_load_n(e->h_sigflag, __ATOMIC_ACQUIRE) != tag; ++spins) {
+  for (uint64_t spins = 0; __atomic_load_n(e->h_sigflag + flag, __ATOMIC_ACQUIRE) != tag; ++spins) {
     if ((spins & 0xFFFFu) == 0xFFFFu && std::chrono::steady_clock::now() - begin > std::chrono::seconds(2)) {
       HIP_TRY(e, hipStreamSynchronize(s));
-      if (__atomic_load_n(e->h_sigflag, __ATOMIC_ACQUIRE) == tag) break;
+      if (__atomic_load_n(e->h_sigflag + flag, __ATOMIC_ACQUIRE) == tag) break;
       e->err = "a launch ended without its hand-over";
       return -5;
     }
@@ -3308,6 +3323,9 @@ static int host_trace(rpeg_engine_t* e, const int16_t* vert_fields, const uint8_
   return n;
 }
 
+// Plans and results go to and from the device in pieces of this many bytes.
+constexpr size_t HOST_CHUNK = 512 * 1024;
+
 // rpeg_eval_host: plans and results in host memory.  Small batches go through eval_host_small; larger ones
 // (or problems whose classes are too large for it) are copied to the device and take the batch path.
 static int eval_host_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, uint32_t flags, double* makespan,
@@ -3331,60 +3349,82 @@ static int eval_host_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* p
     const int rc = eval_host_small(e, n, get, flags, makespan, peak, score, mask, mass, s);
     if (rc <= 0) return rc;
   }
-  // device path: stage the tensors and the results in device memory for this call
-  const size_t V = (size_t)RPEG_MAX_V * RPEG_FIELDS;
-  const size_t b_vert = V * 2 * n, b_head = 4 * n, b_f64 = 8 * n;
-  const size_t o_head = (b_vert + 255) & ~size_t(255), o_mk = (o_head + b_head + 255) & ~size_t(255), o_pk = o_mk + b_f64,
-               o_sc = o_pk + b_f64, o_ms = o_sc + b_f64, o_mask = o_ms + (mass ? b_f64 * RPEG_MAX_V : 0), total = o_mask + n;
-  if (total > e->d_stage_cap) {   // grow-only staging block, kept by the engine
+  // Device path: plans and results staged in device memory for this call, with a pinned mirror of the block in host memory.  The
+  // plans go up in chunks: while the device fetches one, the host copies the next into the mirror.
+  // Bound: the bus (some 50 GB/s) and, beside it, the host's copies (70 GB/s).  Copies of the caller's pageable memory by the runtime,
+  // and of the results by a command behind the kernels, which waits for them on a queue of its own, against these, us a call: 9,001
+  // GRPO plans 258 / 213, 131,072 1,140 / 948; 2,500 PPO 207 / 172, 30,001 609 / 577; 1,500 DPO 92 / 83, 131,072 848 / 616.
+  const size_t V = (size_t)e->max_v * RPEG_FIELDS;   // (fields of vertices that no structure has are not read)
+  const size_t b_row = 2 * n, b_vert = V * b_row, b_head = 4 * n, b_f64 = 8 * n;
+  auto align = [](size_t x) { return (x + 255) & ~size_t(255); };
+  const size_t o_head = align(b_vert), o_mk = align(o_head + b_head), o_pk = align(o_mk + b_f64), o_sc = align(o_pk + b_f64),
+               o_ms = align(o_sc + b_f64), o_mask = align(o_ms + (mass ? b_f64 * RPEG_MAX_V : 0)), total = align(o_mask + n);
+  if (total > e->stage_cap) {   // grow-only, kept by the engine
     HIP_TRY(e, hipStreamSynchronize(s));
     if (e->d_stage) hipFree(e->d_stage);
-    e->d_stage = nullptr;
-    e->d_stage_cap = 0;
-    HIP_TRY(e, hipMalloc(&e->d_stage, total + total / 4));
-    e->d_stage_cap = total + total / 4;
-  }
-  uint8_t* d = e->d_stage;
-  int rc = 0;
-  auto fail = [&](hipError_t st, const char* what) { e->err = std::string(what) + ": " + hipGetErrorString(st); rc = -2; };
-  // results come back in one copy into a pinned mirror of the output region
-  const size_t b_out = total - o_mk;
-  if (b_out > e->h_stage_cap) {
-    HIP_TRY(e, hipStreamSynchronize(s));
     if (e->h_stage) hipHostFree(e->h_stage);
-    e->h_stage = nullptr;
-    e->h_stage_cap = 0;
-    HIP_TRY(e, hipHostMalloc(&e->h_stage, b_out + b_out / 4));
-    e->h_stage_cap = b_out + b_out / 4;
+    e->d_stage = e->h_stage = e->h_stage_dev = nullptr;
+    e->stage_cap = 0;
+    const size_t cap = total + total / 4;
+    HIP_TRY(e, hipMalloc(&e->d_stage, cap));
+    HIP_TRY(e, hipHostMalloc(&e->h_stage, cap, hipHostMallocCoherent));
+    HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_stage_dev, e->h_stage, 0));
+    e->stage_cap = cap;
   }
-  hipError_t st = stride == n ? hipMemcpyAsync(d, vert, b_vert, hipMemcpyHostToDevice, s)
-                              : hipMemcpy2DAsync(d, n * 2, vert, stride * 2, n * 2, V, hipMemcpyHostToDevice, s);
-  if (st != hipSuccess) fail(st, "hipMemcpyAsync");
-  if (!rc) {
-    st = stride == n ? hipMemcpyAsync(d + o_head, head, b_head, hipMemcpyHostToDevice, s)
-                     : hipMemcpy2DAsync(d + o_head, n, head, stride, n, 4, hipMemcpyHostToDevice, s);
-    if (st != hipSuccess) fail(st, "hipMemcpyAsync");
+  uint8_t *const d = e->d_stage, *const h = e->h_stage, *const hd = e->h_stage_dev;
+  if (int rc = ensure_batch(e, n)) return rc;
+  auto copy = [&](uint8_t* to, const uint8_t* from, size_t bytes, uint32_t flag, uint32_t tag) {
+    const uint64_t n16 = (bytes + 15) / 16;
+    hipLaunchKernelGGL(k_copy, dim3((unsigned)std::min<uint64_t>((n16 + COPY_BLOCK - 1) / COPY_BLOCK, 4ull * e->n_cu)), dim3(COPY_BLOCK), 0, s, (uint4*)to,
+                       (const uint4*)from, n16, e->d_queues + Q_COPY, tag ? e->h_sigflag_dev + flag : nullptr, tag);
+  };
+  {
+    size_t sent = 0;   // bytes on their way, a multiple of sixteen
+    auto send = [&](size_t upto) {
+      if (upto > sent) copy(d + sent, hd + sent, upto - sent, 0, 0);
+      sent = upto;
+    };
+    size_t put = 0;    // rows of the mirror that are filled
+    for (const size_t chunk = std::max<size_t>(1, HOST_CHUNK / b_row); put < V;) {
+      const size_t rows = std::min(chunk, V - put);
+      if (stride == n) std::memcpy(h + put * b_row, vert + put * n, rows * b_row);
+      else
+        for (size_t r = put; r < put + rows; ++r) std::memcpy(h + r * b_row, vert + r * stride, b_row);
+      put += rows;
+      if (put < V) send((put * b_row) & ~size_t(15));
+    }
+    for (size_t r = 0; r < 4; ++r) std::memcpy(h + o_head + r * n, head + r * stride, n);
+    send(o_mk);
+    HIP_TRY(e, hipGetLastError());
   }
-  if (!rc) {
-    rpeg_plan_soa_t soa{(const int16_t*)d, d + o_head, n};
-    rc = eval_batch_impl(e, n, &soa, flags, (double*)(d + o_mk), (double*)(d + o_pk), (double*)(d + o_sc), d + o_mask,
-                         mass ? (double*)(d + o_ms) : nullptr, stream);
+  rpeg_plan_soa_t soa{(const int16_t*)d, d + o_head, n};
+  if (int rc = eval_batch_impl(e, n, &soa, flags, (double*)(d + o_mk), (double*)(d + o_pk), (double*)(d + o_sc), d + o_mask,
+                               mass ? (double*)(d + o_ms) : nullptr, stream)) {
+    const std::string what = e->err;
+    hipStreamSynchronize(s);   // (nothing of this call goes on reading the mirror)
+    e->err = what;
+    return rc;
   }
-  const double last_ms = e->last_ms;
-  if (!rc && (st = hipStreamSynchronize(s)) != hipSuccess) fail(st, "hipStreamSynchronize");   // (a copy command behind running kernels starts late)
-  if (!rc && (st = hipMemcpyAsync(e->h_stage, d + o_mk, b_out, hipMemcpyDeviceToHost, s)) != hipSuccess) fail(st, "hipMemcpyAsync");
-  const hipError_t sy = hipStreamSynchronize(s);
-  if (!rc && sy != hipSuccess) fail(sy, "hipStreamSynchronize");
-  if (!rc) {
-    const uint8_t* h = e->h_stage - o_mk;   // same offsets as in the device block
-    if (makespan) std::memcpy(makespan, h + o_mk, b_f64);
-    if (peak) std::memcpy(peak, h + o_pk, b_f64);
-    if (score) std::memcpy(score, h + o_sc, b_f64);
-    if (mass) std::memcpy(mass, h + o_ms, b_f64 * RPEG_MAX_V);
-    if (mask) std::memcpy(mask, h + o_mask, n);
+  // the results in one piece, or, where that is worth a launch each, one after the other: the host copies one to the caller while
+  // the next crosses the bus
+  struct Part { size_t at, bytes; void* to; };
+  const Part part[5] = {{o_mk, b_f64, makespan}, {o_pk, b_f64, peak}, {o_sc, b_f64, score}, {o_ms, mass ? b_f64 * RPEG_MAX_V : 0, mass}, {o_mask, n, mask}};
+  uint32_t tag[5] = {};
+  if (total - o_mk <= HOST_CHUNK) {
+    const uint32_t t = next_tag(e);
+    copy(hd + o_mk, d + o_mk, total - o_mk, 1, t);
+    for (uint32_t& x : tag) x = t;
+  } else {
+    for (int k = 0; k < 5; ++k)
+      if (part[k].to && part[k].bytes) copy(hd + part[k].at, d + part[k].at, part[k].bytes, 1 + k, tag[k] = next_tag(e));
   }
-  e->last_ms = last_ms;
-  return rc;
+  HIP_TRY(e, hipGetLastError());
+  for (int k = 0; k < 5; ++k) {
+    if (!part[k].to || !part[k].bytes) continue;
+    if (int rc = wait_tag(e, s, tag[k], total - o_mk <= HOST_CHUNK ? 1u : 1u + (uint32_t)k)) return rc;
+    std::memcpy(part[k].to, h + part[k].at, part[k].bytes);
+  }
+  return 0;
 }
 
 namespace {
