@@ -73,12 +73,12 @@ struct QuadSize {
 // LDS of one wavefront.  Class tables: per node four successor words, its own, its level place's id and its place in its chain.
 // Per plan [row][plan]: durations, availability by vertex with a row of zeros and one nobody reads, ready-time
 // rows -- over these two, before they are needed, the rows and records of the rank pass, then the ranks of the plans whose
-// positions are being found, or, where that is all of them, both --, with the critical-chain masses finish
+// positions are being found --, with the critical-chain masses finish
 // and start times, a state word and a reservation each.
 __host__ __device__ inline size_t kq_tab_bytes(uint32_t nodes) { return (20ull * nodes + 2 * 2ull * (nodes + 2) + 15) & ~size_t(15); }
 __host__ __device__ inline size_t kq_union_bytes(uint32_t plans, const QuadSize& z) {
-  const size_t rows = 8ull * plans * (z.rows + RPEG_MAX_V + 2), part = 8ull * (plans / z.parts) * z.nodes,
-               ranks = 8ull * plans * z.ranks + sizeof(RankRec) * (z.nodes + 2ull) + (z.parts == 1 ? part + 8ull * plans : 0ull);
+  const size_t rows = 8ull * plans * (z.rows + RPEG_MAX_V + 2), part = 8ull * (plans / z.parts) * (z.nodes + 1ull),
+               ranks = z.parts == 1 ? 0 : 8ull * plans * z.ranks + sizeof(RankRec) * (z.nodes + 1ull);
   const size_t most = rows > part ? rows : part;
   return ((most > ranks ? most : ranks) + 15) & ~size_t(15);
 }
@@ -189,10 +189,11 @@ __device__ inline void kq_count_all(const double* g_rank, const uint32_t* l_own,
   }
 }
 
-// The largest rank among the successors from the fifth on of the node at level place i, or `best`.
-__device__ inline double kq_more_successors(const ClassView& cv, const double* g_rank, int RW, int i, double best) {
+// The largest rank among the successors from the fifth on of the node at level place i, or `best`; rank_at: by level place.
+template <class AT>
+__device__ inline double kq_more_successors(const ClassView& cv, int i, double best, AT&& rank_at) {
   const NodeRec nr = cv.node[cv.lrec[i].node];
-  for (int j = 4; j < nr.n_succ; ++j) best = kp_vmax(best, g_rank[cv.rrec[cv.place[cv.succ[nr.succ_begin + j]]].row * RW]);
+  for (int j = 4; j < nr.n_succ; ++j) best = kp_vmax(best, rank_at(cv.place[cv.succ[nr.succ_begin + j]]));
   return best;
 }
 
@@ -202,18 +203,18 @@ __device__ inline double kq_more_successors(const ClassView& cv, const double* g
 // ahead, durations one.  A rank takes eight bytes a node, more than all a plan keeps of it later, but is read back only by the
 // few levels below: in LDS lie rows that nodes share (RankRec), and the ranks go through memory (240 MB for 1,048,576 DPO plans, most of
 // it never out of the L2) to the comparison of positions, which takes them a part of the plans at a time; where the launches'
-// wavefronts find room together with all of their ranks (AT_ONCE) those stay in LDS.  Before, the pass ran once for every part,
+// wavefronts find room together with all of their ranks those stay in LDS (kq_ranks_in_lds).  Before, the pass ran once for every part,
 // with two to four times the lanes for levels of two or three nodes, and a part's ranks all lay in LDS.  us a step, before / now:
 // 262,144 AC-share plans 4,196 / 3,953, 131,072 2,720 / 2,572, 65,536 1,550 / 1,430; 131,072 PPO 989 / 935, GRPO 490 / 442; 65,536
-// GRPO 320 / 307; 1,048,576 DPO 971 / 971; 20,011 PPO (all at once in either) 310 / 308.
-template <int QL, bool AT_ONCE>
+// GRPO 320 / 307; 1,048,576 DPO 971 / 971.
+template <int QL>
 __device__ inline void kq_ranks(const ClassView& cv, double* rows, uint32_t n_rows, uint32_t ends, const double* g_dur, double* keep, uint32_t parts, bool many) {
   constexpr int RW = KE_WAVE / QL;
   const int lane = threadIdx.x, p = lane / QL, q = lane % QL, n = (int)cv.h->n_nodes, n_levels = (int)cv.h->n_levels;
   double* const g_rank = rows + p;
   const uint2* const l_rec = (const uint2*)(rows + (size_t)n_rows * RW);
   // (bytes, of the nodes' ranks of a plan)
-  const uint32_t rg = (uint32_t)__builtin_ctz(RW / parts) + 3u, out = AT_ONCE ? 0u : (((uint32_t)p >> (rg - 3u)) * (uint32_t)n << rg) + (((uint32_t)p & (RW / parts - 1u)) << 3);
+  const uint32_t rg = (uint32_t)__builtin_ctz(RW / parts) + 3u, out = (((uint32_t)p >> (rg - 3u)) * (uint32_t)n << rg) + (((uint32_t)p & (RW / parts - 1u)) << 3);
   int level = 0;
   auto end_of = [&](int l) {   // (asked for level by level)
     if (__builtin_expect(l && (l & 63) == 0, 0)) ends = cv.lbeg[l + lane + 1 <= n_levels ? l + lane + 1 : n_levels];
@@ -239,19 +240,17 @@ __device__ inline void kq_ranks(const ClassView& cv, double* rows, uint32_t n_ro
     next(at1, end1, at2, end2);
     const uint2 rec2 = record(at2, end2);
     const double d1 = g_dur[((rec1.y >> 8) & 0xFFu) * RW];
-    if (AT_ONCE || __ballot(rec.x > 0xFFFFu)) {   // (a branch is a quarter of a trip's latency)
+    if (__ballot(rec.x > 0xFFFFu)) {
       const double r2 = g_rank[((rec.x >> 16) & 0xFFu) * RW], r3 = g_rank[(rec.x >> 24) * RW];
       best = kp_vmax(kp_vmax(r0, r1), kp_vmax(r2, r3));
       if (__builtin_expect(many, 0))
-        if (at + q < end && (rec.y >> 31)) best = kq_more_successors(cv, g_rank, RW, at + q, best);
+        if (at + q < end && (rec.y >> 31)) best = kq_more_successors(cv, at + q, best, [&](uint32_t to) { return g_rank[cv.rrec[to].row * RW]; });
     } else {
       best = kp_vmax(r0, r1);
     }
     const double rank = d + best;
     g_rank[(rec.y & 0xFFu) * RW] = rank;
-    const uint32_t id = (rec.y >> 16) & 0x1FFu;
-    if (AT_ONCE) keep[id * RW + p] = rank;
-    else if (at + q < end) *(double*)((uint8_t*)keep + (out + (id << rg))) = rank;
+    if (at + q < end) *(double*)((uint8_t*)keep + (out + (((rec.y >> 16) & 0x1FFu) << rg))) = rank;
     rec = rec1;
     rec1 = rec2;
     d = d1;
@@ -261,6 +260,58 @@ __device__ inline void kq_ranks(const ClassView& cv, double* rows, uint32_t n_ro
     end1 = end2;
   }
   __syncthreads();   // (the ranks are in memory: a wavefront reads its own)
+}
+
+// The same where the ranks of all plans stay in LDS, by node id: no rows, nor their records.  (With them, which take 3 KB more beside
+// 33 of graphs of 152 nodes: 20,011 PPO plans 308 / 314 us a step.)
+template <int QL>
+__device__ inline void kq_ranks_in_lds(const ClassView& cv, double* ranks, const double* g_dur, const uint32_t* l_succ, const uint32_t* l_own,
+                                       const uint16_t* l_id, uint32_t ends, bool many) {
+  constexpr int RW = KE_WAVE / QL;
+  const int lane = threadIdx.x, q = lane % QL, n = (int)cv.h->n_nodes, n_levels = (int)cv.h->n_levels;
+  double* const g_rank = ranks + lane / QL;
+  // A level waits for one LDS trip, that of its successors' ranks: words and durations of its nodes were read a level ahead,
+  // their ids two levels.
+  auto rank_at = [&](uint32_t to) { return g_rank[l_id[to] * RW]; };
+  if (q == 0) g_rank[n * RW] = 0.0;
+  __syncthreads();
+  {
+    auto end_of = [&](int l) { return l < n_levels ? __builtin_amdgcn_readlane((int)ends, l & 63) : n; };
+    auto id_at = [&](int i) { return (int)l_id[i < n ? i : n - 1]; };
+    int begin = 0;
+    int end = end_of(0), id = id_at(q), id1 = id_at(end + q);
+    uint4 sw = ((const uint4*)l_succ)[id];
+    uint32_t own = l_own[id];
+    double d = g_dur[((own >> 10) & 0xFFu) * RW];
+    for (int l = 0; l < n_levels; ++l) {
+      const double r0 = g_rank[(sw.x & 0x1FFu) * RW], r1 = g_rank[(sw.y & 0x1FFu) * RW], r2 = g_rank[(sw.z & 0x1FFu) * RW], r3 = g_rank[(sw.w & 0x1FFu) * RW];
+      const uint4 sw1 = ((const uint4*)l_succ)[id1];
+      const uint32_t own1 = l_own[id1];
+      if (__builtin_expect((l & 63) == 63, 0)) ends = cv.lbeg[l + 1 + lane + 1 <= n_levels ? l + 1 + lane + 1 : n_levels];
+      const int end1 = end_of(l + 1), id2 = id_at(end1 + q);
+      double best = kp_vmax(kp_vmax(r0, r1), kp_vmax(r2, r3));
+      int i = begin + q;
+      if (__builtin_expect(many, 0))
+        if (i < end && (own & 7u) > 4u) best = kq_more_successors(cv, i, best, rank_at);
+      if (i < end) g_rank[id * RW] = d + best;
+      for (i += QL; __builtin_expect(__ballot(i < end) != 0ull, 0); i += QL) {   // (more nodes than lanes)
+        const int id_i = id_at(i);
+        const uint4 w = ((const uint4*)l_succ)[id_i];
+        const uint32_t o = l_own[id_i];
+        best = kp_vmax(kp_vmax(g_rank[(w.x & 0x1FFu) * RW], g_rank[(w.y & 0x1FFu) * RW]), kp_vmax(g_rank[(w.z & 0x1FFu) * RW], g_rank[(w.w & 0x1FFu) * RW]));
+        if (many && i < end && (o & 7u) > 4u) best = kq_more_successors(cv, i, best, rank_at);
+        if (i < end) g_rank[id_i * RW] = g_dur[((o >> 10) & 0xFFu) * RW] + best;
+      }
+      d = g_dur[((own1 >> 10) & 0xFFu) * RW];
+      begin = end;
+      end = end1;
+      id = id1;
+      id1 = id2;
+      sw = sw1;
+      own = own1;
+    }
+  }
+  __syncthreads();
 }
 
 // From the ranks the state words of all plans of a wavefront, a part of them at a time with as many times the lanes for each.  The
@@ -380,7 +431,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
   if (lane == 0) l_id[n] = (uint16_t)n;
   __syncthreads();
   const uint32_t level_ends = cv.lbeg[lane + 1 <= (int)cv.h->n_levels ? lane + 1 : (int)cv.h->n_levels];
-  {   // what the rank pass reads, behind its rows
+  if (Z.parts > 1) {   // what the rank pass reads, behind its rows
     uint2* const l_rec = (uint2*)(ranks + (size_t)Z.ranks * RW);
     for (int i = lane; i <= n; i += KE_WAVE) l_rec[i] = ((const uint2*)cv.rrec)[i];
     if (q == 0) ranks[p] = 0.0;
@@ -438,12 +489,11 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
 
   const bool any_many = __ballot(many != 0ull) != 0ull;   // (lanes that left the loop early)
   if (Z.parts == 1) {
-    double* const all = ranks + (size_t)Z.ranks * RW + Z.nodes + 2;
-    kq_ranks<QL, true>(cv, ranks, Z.ranks, level_ends, g_dur, all, 1, any_many);
+    kq_ranks_in_lds<QL>(cv, ranks, g_dur, l_succ, l_own, l_id, level_ends, any_many);
     KE_STAMP(3);
-    kq_positions<QL, 1>(cv, all, keep, l_own, l_chain, class_ends, shrink, states);
+    kq_positions<QL, 1>(cv, ranks, keep, l_own, l_chain, class_ends, shrink, states);
   } else {
-    kq_ranks<QL, false>(cv, ranks, Z.ranks, level_ends, g_dur, keep, Z.parts, any_many);
+    kq_ranks<QL>(cv, ranks, Z.ranks, level_ends, g_dur, keep, Z.parts, any_many);
     KE_STAMP(3);
     if (Z.parts == kq_parts_least(QL)) kq_positions<QL, kq_parts_least(QL)>(cv, ranks, keep, l_own, l_chain, class_ends, shrink, states);
     else kq_positions<QL, 2 * kq_parts_least(QL)>(cv, ranks, keep, l_own, l_chain, class_ends, shrink, states);
