@@ -67,9 +67,12 @@ __device__ inline void kp_hop(const ClassView& cv, int v, const KpHop& p, const 
   l_next[v] = (uint16_t)nx;
   l_vx[v] = (uint8_t)p.vx;
 }
-// Lane x < RPEG_MAX_V returns the mass of vertex x, summed in the order of the walk.
+// Lane x < RPEG_MAX_V returns the mass of vertex x, summed in the order of the walk.  scratch: sixteen bytes a node.
+// Bound: the walk, a dependent LDS trip a hop.  So it is done in steps of eight hops -- where those lead is found for all nodes at
+// once by doubling --, every lane then walks one of these stretches, and the sums read the chain from consecutive places.  (Hop by
+// hop: @M@)
 __device__ inline double kp_critical_mass(const int n, const int lane, const double* l_fin, const double* l_start,
-                                          const uint16_t* l_next, const uint8_t* l_vx) {
+                                          const uint16_t* l_next, const uint8_t* l_vx, uint8_t* scratch) {
   double bf = -1.0;
   uint32_t bi = 0xFFFFFFFFu;
   for (int v = lane; v < n; v += KE_WAVE) {
@@ -79,13 +82,62 @@ __device__ inline double kp_critical_mass(const int n, const int lane, const dou
   const double top = kp_wave_reduce(bf, KpMax());
   int cur = (int)kp_wave_umin(bf == top ? bi : 0xFFFFFFFFu);
   double m = 0.0;
-  for (int hops = 0; hops <= n; ++hops) {   // a chain visits a node at most once
-    const int vx = l_vx[cur];
-    const double d = l_fin[cur] - l_start[cur];
-    const int nx = __builtin_amdgcn_readfirstlane((int)l_next[cur]);
-    if (lane == vx) m += d;
-    if (nx == 0xFFFF) break;
+  constexpr int STEP = 8, FEW = 32;   // (a graph of at most FEW nodes has no room for the stretches, nor use for them)
+  static_assert(STEP * KE_WAVE >= KE_WAVE * KP_MAX_NS, "a stretch for every lane");
+  if (n <= FEW) {
+    for (int hops = 0; hops <= n; ++hops) {   // a chain visits a node at most once
+      const int vx = l_vx[cur];
+      const double d = l_fin[cur] - l_start[cur];
+      const int nx = __builtin_amdgcn_readfirstlane((int)l_next[cur]);
+      if (lane == vx) m += d;
+      if (nx == 0xFFFF) break;
+      cur = nx;
+    }
+    return m;
+  }
+  const int places = (n + STEP - 1) & ~(STEP - 1);
+  double* const time = (double*)scratch;                       // of the chain, by place
+  uint8_t* const vertex = scratch + 8 * (size_t)places;
+  uint16_t *const twice = (uint16_t*)(vertex + places), *const four = twice + n;   // where two, four and, over the first, eight hops lead
+  auto after = [&](const uint16_t* from, const uint16_t* by, uint16_t* to) {
+    for (int v = lane; v < n; v += KE_WAVE) {
+      const uint32_t x = from[v];
+      const uint16_t y = by[x < (uint32_t)n ? x : 0u];
+      to[v] = x < (uint32_t)n ? y : (uint16_t)0xFFFFu;
+    }
+    kp_sync();
+  };
+  after(l_next, l_next, twice);
+  after(twice, twice, four);
+  after(four, four, twice);
+  int n_stretch = 0;
+  uint32_t at = 0xFFFFu;   // lane k: where stretch k begins
+  for (;;) {
+    const int nx = __builtin_amdgcn_readfirstlane((int)twice[cur]);
+    at = lane == n_stretch ? (uint32_t)cur : at;
+    ++n_stretch;
+    if (nx == 0xFFFF || n_stretch * STEP >= places) break;
     cur = nx;
+  }
+  for (int j = 0; j < STEP; ++j) {
+    const uint32_t v = at < (uint32_t)n ? at : 0u;
+    const double d = l_fin[v] - l_start[v];
+    const uint8_t vx = l_vx[v];
+    const uint32_t nx = l_next[v];
+    if (lane < n_stretch) {
+      time[lane * STEP + j] = at < (uint32_t)n ? d : 0.0;
+      vertex[lane * STEP + j] = at < (uint32_t)n ? vx : (uint8_t)0xFFu;
+    }
+    at = at < (uint32_t)n ? nx : 0xFFFFu;
+  }
+  kp_sync();
+  for (int k = 0; k < n_stretch; ++k) {
+    const uint64_t vx = *(const uint64_t*)(vertex + k * STEP);
+    double d[STEP];
+#pragma unroll
+    for (int j = 0; j < STEP; ++j) d[j] = time[k * STEP + j];
+#pragma unroll
+    for (int j = 0; j < STEP; ++j) m += (int)((vx >> (8 * j)) & 0xFFu) == lane ? d[j] : 0.0;   // (no sum is a negative zero: zero leaves it as it is)
   }
   return m;
 }
@@ -502,10 +554,11 @@ __device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const
 
   // ---- ranks, positions and list scheduling
   double makespan = 0.0;
+  const uint64_t order_rec = kp_order_rec(cv, wave * KE_WAVE + lane);
   if (!err && (NW == 1 || wave == 0)) kp_ranks((uint64_t)cv.h, M);
   kp_barrier<NW>();
   if (stamp) stamp[3] = wall_clock64();
-  if (!err) kp_positions<NW>((uint64_t)cv.h, wave, M);
+  if (!err) kp_positions<NW>((uint64_t)cv.h, wave, order_rec, M);
   if (NW > 1 && wave == 0) {
     peak = shared.peak;
     pen = shared.pen;
@@ -569,7 +622,7 @@ __device__ inline void kp_eval_plan(const EvalLaunch& L, const uint64_t w, const
       for (int v = lane; v < n; v += KE_WAVE) kp_hop(cv, v, kp_hop_of(cv, v), l_rank, l_next, l_pt);
       kp_sync();
     }
-    if (!err) m = kp_critical_mass(n, lane, l_rank, l_start, l_next, l_pt);
+    if (!err) m = kp_critical_mass(n, lane, l_rank, l_start, l_next, l_pt, (uint8_t*)l_rec);
   }
   if (lane == 0) {
     if (TR == KP_TIMES_ORDER && L.util) L.util[pi] = util;

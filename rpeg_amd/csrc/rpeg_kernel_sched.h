@@ -212,30 +212,100 @@ __device__ inline uint32_t kp_reserved(uint32_t blocked, uint32_t cond, uint64_t
   return b | (touch << 8);
 }
 
-// The class's level records go to LDS.
+// What the rank pass reads of the class beside the level records, in LDS over the ranks by order place: where the levels end, the
+// chains and, by level place, their members.
+struct KpRankTables {
+  KP_LDS uint16_t* ends;     // lbeg
+  KP_LDS uint32_t* group;    // GroupRec: begin | count << 16
+  KP_LDS uint16_t* member;
+};
+__device__ inline KpRankTables kp_rank_tables(const KpLds& M, uint32_t n_levels, uint32_t n_groups) {   // (2 n + 2, 4 n and 2 n bytes at most)
+  KpRankTables t;
+  t.ends = (KP_LDS uint16_t*)M.rk;
+  t.group = (KP_LDS uint32_t*)(t.ends + ((n_levels + 2u) & ~1u));
+  t.member = (KP_LDS uint16_t*)(t.group + n_groups);
+  return t;
+}
+// These and the level records go to LDS.
 __device__ inline void kp_stage(const uint8_t* blob, const KpLds& M) {
   const int lane = (int)__lane_id();
   const KpClass T{kp_scalar64((uint64_t)blob)};
   const KP_CONST ClassHdr* h = T.hdr();
-  const int n = (int)h->n_nodes;
+  const int n = (int)h->n_nodes, n_levels = (int)h->n_levels, n_groups = (int)h->n_groups, n_members = (int)h->n_gmembers;
   const KP_CONST uint4* src = T.at<uint4>(h->off_lrec);
-  for (int v = lane; v < n; v += KE_WAVE) ((KP_LDS uint4*)M.rec)[v] = src[v];
+  const KP_CONST uint16_t* lbeg = T.at<uint16_t>(h->off_lbeg);
+  const KP_CONST uint32_t* group = T.at<uint32_t>(h->off_group);
+  const KP_CONST uint16_t* gm = T.at<uint16_t>(h->off_glvl);
+  const KpRankTables t = kp_rank_tables(M, (uint32_t)n_levels, (uint32_t)n_groups);
+  for (int v = lane; v - lane < n; v += KE_WAVE) {   // (one round trip for all of a stretch)
+    uint4 rec;
+    uint32_t g = 0u;
+    uint16_t e = 0, m = 0;
+    if (v < n) rec = src[v];
+    if (v <= n_levels) e = lbeg[v];
+    if (v < n_groups) g = group[v];
+    if (v < n_members) m = gm[v];
+    if (v < n) ((KP_LDS uint4*)M.rec)[v] = rec;
+    if (v <= n_levels) t.ends[v] = e;
+    if (v < n_groups) t.group[v] = g;
+    if (v < n_members) t.member[v] = m;
+  }
+  if (n_levels == n && n % KE_WAVE == 0 && lane == 0) t.ends[n] = lbeg[n];   // (a chain of a whole number of wavefronts: one more end)
 }
 
-// Ranks.
+// Ranks (scheduler.py:71-100), level by level from the nodes without successors; then chain inheritance (scheduler.py:367-378):
+// the sub-nodes of one split vertex share the chain's top rank.
+// Bound: the latency of a level, one LDS trip for its successors' ranks.  So nothing else stands in it: records are read two levels
+// ahead, durations and addresses one, lanes without a node write where nobody reads, and what only few graphs have (more than 62
+// levels, a level of more than 64 nodes, a node of more than four successors) is a loop of its own.  What it reads of the class is in
+// LDS before (kp_stage).  (With ballots, a duration and branches in every level, and ends, chains and their members from memory:
+// PPO graphs of 82-117 nodes 6.2 us, now @K2@; AC-share of 92-300 9.0, now @K4@.)
 __device__ __attribute__((noinline)) void kp_ranks(uint64_t blob, const KpLds M) {
   const int lane = (int)__lane_id();
   const KpClass T{kp_scalar64(blob)};
   const KP_CONST ClassHdr* h = T.hdr();
   const int n = (int)h->n_nodes, n_levels = (int)h->n_levels;
+  const uint32_t n_groups = h->n_groups;
+  const KpRankTables t = kp_rank_tables(M, (uint32_t)n_levels, n_groups);
+  const KP_LDS uint16_t* const lbeg = t.ends;
+  const KP_LDS uint32_t* const group = t.group;
+  const KP_LDS uint16_t* const gm = t.member;
+  KP_LDS double* const nowhere = (KP_LDS double*)M.at;   // written by lanes without a node
+  constexpr int MEMBERS = 8;
+  uint32_t ends = lbeg[lane + 1 <= n_levels ? lane + 1 : n_levels];   // lane l: where level l ends
+  const uint32_t g0 = (uint32_t)lane < n_groups ? group[lane] : 1u << 16;
+  uint32_t member[MEMBERS];
+#pragma unroll
+  for (int j = 0; j < MEMBERS; ++j) {   // (behind a chain's last member that one again)
+    const uint32_t count = g0 >> 16;
+    member[j] = n_groups ? gm[(g0 & 0xFFFFu) + ((uint32_t)j < count ? (uint32_t)j : count - 1u)] : 0u;
+  }
   if (lane == 0) M.rank[n] = 0.0;
   kp_sync();
-
-  // ---- ranks (scheduler.py:71-100), level by level from the nodes without successors; the record and the duration of
-  // the next level are read while this one's ranks are computed (the levels follow each other in this order)
-  {
-    const KP_CONST uint16_t* lbeg = T.at<uint16_t>(h->off_lbeg);
-    uint32_t ends = 0;
+  const KP_LDS uint4* const recs = (const KP_LDS uint4*)M.rec;   // succ[0..3]; node | slot << 16 | ..; .. | n_succ << 16 | ..
+  const int before = __shfl_up((int)ends, 1);
+  mask64 odd = __ballot(lane < n_levels && (int)ends - (lane ? before : 0) > KE_WAVE);
+  for (int i = lane; i < n; i += KE_WAVE) odd |= __ballot(((recs[i].w >> 16) & 0xFFu) > 4u);
+  if (__builtin_expect(n_levels <= KE_WAVE - 2 && __ballot(odd != 0ull) == 0ull, 1)) {
+    auto end_of = [&](int l) { return __builtin_amdgcn_readlane((int)ends, l); };   // (n behind the last level)
+    auto at = [&](int i) { return recs[i < n ? i : n - 1]; };
+    int begin = 0, end = end_of(0), end1 = end_of(1);
+    uint4 rec = at(lane), rec1 = at(end + lane);
+    double d = M.dur[(rec.z >> 16) & 0xFFu];
+    for (int l = 0; l < n_levels; ++l) {
+      const double r0 = M.rank[rec.x & 0xFFFFu], r1 = M.rank[rec.x >> 16], r2 = M.rank[rec.y & 0xFFFFu], r3 = M.rank[rec.y >> 16];
+      const double d1 = M.dur[(rec1.z >> 16) & 0xFFu];
+      const uint4 rec2 = at(end1 + lane);
+      const int i = begin + lane, end2 = end_of(l + 2);
+      *(i < end ? M.rank + i : nowhere) = d + kp_vmax(kp_vmax(r0, r1), kp_vmax(r2, r3));
+      begin = end;
+      end = end1;
+      end1 = end2;
+      rec = rec1;
+      rec1 = rec2;
+      d = d1;
+    }
+  } else {   // the record and the duration of the next level are read while this one's ranks are computed
     int i = lane;
     LevelRec rec = M.rec[i < n ? i : 0];
     double d = M.dur[rec.slot];
@@ -247,11 +317,9 @@ __device__ __attribute__((noinline)) void kp_ranks(uint64_t blob, const KpLds M)
       for (;;) {   // (a level of more than 64 nodes goes round more than once)
         const double r0 = M.rank[rec.succ[0]], r1 = M.rank[rec.succ[1]], r2 = M.rank[rec.succ[2]], r3 = M.rank[rec.succ[3]];
         double best = kp_vmax(kp_vmax(r0, r1), kp_vmax(r2, r3));
-        if (__builtin_expect(__ballot(i < end && rec.n_succ > 4) != 0ull, 0)) {
-          if (i < end && rec.n_succ > 4) {
-            const uint32_t sb = T.at<uint16_t>(h->off_node + rec.node * 8u)[0];
-            for (uint32_t j = 4; j < rec.n_succ; ++j) best = kp_vmax(best, M.rank[T.at<uint16_t>(h->off_place)[T.at<uint16_t>(h->off_succ)[sb + j]]]);
-          }
+        if (i < end && rec.n_succ > 4) {
+          const uint32_t sb = T.at<uint16_t>(h->off_node + rec.node * 8u)[0];
+          for (uint32_t j = 4; j < rec.n_succ; ++j) best = kp_vmax(best, M.rank[T.at<uint16_t>(h->off_place)[T.at<uint16_t>(h->off_succ)[sb + j]]]);
         }
         if (i < end) M.rank[i] = d + best;
         i += 64;
@@ -265,11 +333,24 @@ __device__ __attribute__((noinline)) void kp_ranks(uint64_t blob, const KpLds M)
     }
   }
   kp_sync();
-  // chain inheritance (scheduler.py:367-378): the sub-nodes of one split vertex share the chain's top rank
-  {
-    const KP_CONST uint32_t* group = T.at<uint32_t>(h->off_group);   // GroupRec: begin | count << 16
-    const KP_CONST uint16_t* gm = T.at<uint16_t>(h->off_glvl);
-    for (uint32_t g = lane; g < h->n_groups; g += KE_WAVE) {
+  if (n_groups) {
+    if ((uint32_t)lane < n_groups) {
+      double r[MEMBERS], top;
+#pragma unroll
+      for (int j = 0; j < MEMBERS; ++j) r[j] = M.rank[member[j]];
+      top = r[0];
+#pragma unroll
+      for (int j = 1; j < MEMBERS; ++j) top = r[j] > top ? r[j] : top;
+      const uint32_t begin = g0 & 0xFFFFu, count = g0 >> 16;
+      for (uint32_t j = MEMBERS; j < count; ++j) {   // (a chain of more)
+        const double x = M.rank[gm[begin + j]];
+        top = x > top ? x : top;
+      }
+#pragma unroll
+      for (int j = 0; j < MEMBERS; ++j) M.rank[member[j]] = top;
+      for (uint32_t j = MEMBERS; j < count; ++j) M.rank[gm[begin + j]] = top;
+    }
+    for (uint32_t g = (uint32_t)lane + KE_WAVE; g < n_groups; g += KE_WAVE) {   // (more chains than lanes)
       const uint32_t begin = group[g] & 0xFFFFu, count = group[g] >> 16;
       double top = M.rank[gm[begin]];
       for (uint32_t j = 1; j < count; ++j) {
@@ -278,10 +359,13 @@ __device__ __attribute__((noinline)) void kp_ranks(uint64_t blob, const KpLds M)
       }
       for (uint32_t j = 0; j < count; ++j) M.rank[gm[begin + j]] = top;
     }
+    kp_sync();
   }
-  kp_sync();
 }
 
+__device__ inline uint64_t kp_order_rec(const ClassView& cv, int place) {   // (OrderRec)
+  return ((const uint64_t*)cv.orec)[place < (int)cv.h->n_nodes ? place : 0];
+}
 // Positions: within its tie-break class a node comes behind those of larger rank.  Nodes that agree have the same position
 // and are told apart by the order in which they counted themselves there (of one chain: by their place in it); `shared`
 // where they are more than the node's own chain.  NW wavefronts share the nodes.
@@ -289,15 +373,15 @@ __device__ __attribute__((noinline)) void kp_ranks(uint64_t blob, const KpLds M)
 // instructions for 64 comparisons.  With the equal ranks counted along, the nodes of shared position going through their class
 // once more, and every lane at its own node's class, it took twice that and more (sixteen wavefronts on a compute unit, 300
 // nodes: 44 us, now 18; 92 nodes 10, now 6.  4,096 PPO plans 170 -> 165 us a step).
+// w0: this lane's first record, kp_order_rec, which is fetched ahead of the ranks.
 template <int NW>
-__device__ __attribute__((noinline)) void kp_positions(uint64_t blob, int wave, const KpLds M) {
+__device__ __attribute__((noinline)) void kp_positions(uint64_t blob, int wave, const uint64_t w0, const KpLds M) {
   const int first = wave * KE_WAVE + (int)__lane_id();
   constexpr int STEP = NW * KE_WAVE;
   const KpClass T{kp_scalar64(blob)};
   const KP_CONST ClassHdr* h = T.hdr();
   const int n = (int)h->n_nodes;
   const KP_CONST uint64_t* orec = T.at<uint64_t>(h->off_orec);
-  const uint64_t w0 = orec[first < n ? first : 0];   // the records by tie-break class
   KP_LDS uint32_t* const count = M.at;                    // by position: the nodes that have it
   KP_LDS uint32_t* const found = (KP_LDS uint32_t*)M.rank;   // by node of this order: its position | its turn there << 10 | nodes that have it << 20 (over the ranks by level place)
   {
