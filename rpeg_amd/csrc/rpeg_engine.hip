@@ -238,8 +238,9 @@ __device__ inline uint64_t sig_of_thread(const rpeg_problem_t* __restrict__ P, c
     todo &= ~__ballot(mine);
     if (mine) {
       PlanHead hu = h;
-      hu.structure = su;
-      if (plan_valid(*P, hu, a)) sg = plan_signature(*P, su, h.split, h.tau0, h.tau1, a);
+      hu.structure = __builtin_amdgcn_readfirstlane(su);
+      const rpeg_problem_t& table = ke_common(*P);
+      if (plan_valid(table, hu, a)) sg = plan_signature(table, hu.structure, h.split, h.tau0, h.tau1, a);
     }
   }
   return sg;
@@ -518,8 +519,9 @@ __global__ __launch_bounds__(WAVE) void k_prologue(const PrologueLaunch L) {
     const int s0 = __builtin_amdgcn_readlane(su, __builtin_ctzll(todo));
     const bool mine = active && su == s0;
     todo &= ~__ballot(mine);
-    if (mine)
-      for (int row = (int)(L.row_begin + blockIdx.y); row < (int)L.row_end; row += (int)gridDim.y) kpro_row(L, i, s0, split, row);
+    if (!mine) continue;
+    const int common = __builtin_amdgcn_readfirstlane(s0);
+    for (int row = (int)(L.row_begin + blockIdx.y); row < (int)L.row_end; row += (int)gridDim.y) kpro_row(L, i, common, split, row);
   }
 }
 
@@ -540,7 +542,7 @@ __global__ __launch_bounds__(WAVE) void k_peaks(const PrologueLaunch L) {
     const int su = __builtin_amdgcn_readlane(h.structure, __builtin_ctzll(todo));
     const bool mine = active && h.structure == su;
     todo &= ~__ballot(mine);
-    if (mine) kpro_peaks(L, i, su, h, l_vm + threadIdx.x, l_ord + threadIdx.x);
+    if (mine) kpro_peaks(L, i, __builtin_amdgcn_readfirstlane(su), h, l_vm + threadIdx.x, l_ord + threadIdx.x);
   }
 }
 

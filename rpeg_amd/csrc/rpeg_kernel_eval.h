@@ -161,6 +161,22 @@ __device__ inline double ke_slot_duration(const rpeg_problem_t& P, const rpeg_st
   }
 }
 
+#if defined(__HIP_DEVICE_COMPILE__)
+#define KP_CONST __attribute__((address_space(4)))
+#else
+#define KP_CONST
+#endif
+// x, the same for all lanes at work and written by no kernel, for reads through the scalar cache.  (Without it a table of the problem
+// is read by a load a lane wherever the compiler does not see that: behind a store of the kernel, in a function that is
+// not inlined, and where a lane takes part because a field of its own equals the common one, which may then be read for it.
+// k_prologue's durations / k_peaks, us, with a load a lane and without: 1,048,576 DPO plans 129 / 93 -> 103 / 64, 262,144
+// AC-share plans 310 / 664 -> 239 / 563, the latter beside k_quad; the step 945 -> 875 and 3,968 -> 3,894.)
+template <class T>
+__device__ inline const T& ke_common(const T& x) {
+  const uint64_t at = (uint64_t)&x;
+  const uint64_t uniform = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32)) << 32;
+  return *(const T*)(const KP_CONST T*)uniform;
+}
 template <int RW>
 struct KeVMem {  // per-vertex memory quantities in LDS, [vertex*4 + field][lane]
   const double* p;

@@ -73,7 +73,7 @@ __device__ inline VPlan kpro_vplan(const int16_t* p, uint64_t stride, int v) {
 __device__ __attribute__((noinline)) double kpro_op_time(const rpeg_problem_t& P, const rpeg_vertex_t& vx, const rpeg_opconst_t& oc,
                                                          const int16_t* pl, uint64_t stride, int v) {
   bool zero_div = false;
-  const double t = op_time(P, vx, oc, kpro_vplan(pl, stride, v), &zero_div);
+  const double t = op_time(ke_common(P), ke_common(vx), oc, kpro_vplan(pl, stride, v), &zero_div);   // (the constants: those of the lane's own split)
   return zero_div ? __builtin_nan("") : t;
 }
 
@@ -115,7 +115,9 @@ __device__ __attribute__((noinline)) void kpro_masks(const int16_t* pl, const ui
 
 __device__ __attribute__((noinline)) void kpro_vmem(const rpeg_problem_t& P, const int16_t* pl, const uint64_t stride,
                                                     const rpeg_struct_t& st, const int v, double* out, const uint64_t out_stride) {
-  const VMem m = vertex_memory(P, st.vertex[v], kpro_vplan(pl, stride, v), struct_coresident(st));
+  const rpeg_struct_t& su = ke_common(st);
+  const int x = __builtin_amdgcn_readfirstlane(v);
+  const VMem m = vertex_memory(ke_common(P), su.vertex[x], kpro_vplan(pl, stride, x), struct_coresident(su));
   out[0 * out_stride] = (double)m.w_shard;
   out[1 * out_stride] = m.mem_w;
   out[2 * out_stride] = m.opt;
@@ -125,12 +127,12 @@ __device__ __attribute__((noinline)) void kpro_vmem(const rpeg_problem_t& P, con
 // Plan i of this lane, structure su (uniform), one row of the first launch's grid (uniform): the duration of one slot
 // of the universe; or the pair relations of the plan; or the memory terms of one vertex.
 __device__ inline void kpro_row(const PrologueLaunch& L, const uint64_t i, const int su, const int split, const int row) {
-  const rpeg_problem_t& P = *L.P;
+  const rpeg_problem_t& P = ke_common(*L.P);
   const rpeg_struct_t& st = P.st[su];
   const int16_t* pl = L.vert + i;
   if (row < (int)L.max_uni) {
     if (row >= (int)L.n_uni[su]) return;
-    const SlotDesc sd = L.uni[(size_t)su * RPEG_MAX_UNIVERSE + row];   // uniform
+    const SlotDesc sd = ke_common(L.uni[(size_t)su * RPEG_MAX_UNIVERSE + row]);   // uniform
     if (!slot_in_split(P, split, sd)) return;                          // this lane's split variant has no such phase
     L.dur[(uint64_t)row * L.dur_stride + i] = kpro_slot_duration(P, st, split, sd, pl, L.stride);
   } else if (row == (int)L.max_uni) {
@@ -180,7 +182,7 @@ __device__ inline void kpro_vorder(const rpeg_problem_t& P, const rpeg_struct_t&
 // per-thread arrays into scratch memory).
 __device__ inline void kpro_peaks(const PrologueLaunch& L, const uint64_t i, const int su, const PlanHead h, double* l_vm,
                                   uint8_t* l_ord) {
-  const rpeg_problem_t& P = *L.P;
+  const rpeg_problem_t& P = ke_common(*L.P);
   const rpeg_struct_t& st = P.st[su];
   const int nv = st.n_vertex;
   PlanMasks pm;

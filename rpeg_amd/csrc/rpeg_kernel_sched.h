@@ -139,10 +139,8 @@ typedef unsigned long long mask64;
 // would make every access of theirs a flat one.)
 #if defined(__HIP_DEVICE_COMPILE__)
 #define KP_LDS __attribute__((address_space(3)))
-#define KP_CONST __attribute__((address_space(4)))
 #else
 #define KP_LDS
-#define KP_CONST
 #endif
 
 constexpr uint32_t KP_AT_SHARED = 1u << 10;
