@@ -525,13 +525,8 @@ __global__ __launch_bounds__(WAVE) void k_prologue(const PrologueLaunch L) {
   }
 }
 
-// (LDS by the problem's largest vertex count, kpeaks_lds_bytes: beside a resident main kernel the blocks of this launch
-// get what LDS that kernel leaves, and with the 12.8 KB of six vertices a DPO batch of three had half as many of them)
-static size_t kpeaks_lds_bytes(uint32_t max_v) { return (size_t)max_v * 4 * WAVE * 8 + 8 * WAVE; }
-__global__ __launch_bounds__(WAVE) void k_peaks(const PrologueLaunch L) {
-  extern __shared__ double kpk_lds[];
-  double* l_vm = kpk_lds;                                        // [vertex * 4 + field][lane]
-  uint8_t* l_ord = (uint8_t*)(kpk_lds + (size_t)L.max_v * 4 * WAVE);   // [position][lane]
+template <int NV>
+__global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_peaks(const PrologueLaunch L) {
   const uint64_t i = (uint64_t)blockIdx.x * WAVE + threadIdx.x;
   const bool active = i < L.n && L.cid[i] != KPRO_INVALID;
   PlanHead h;
@@ -542,9 +537,11 @@ __global__ __launch_bounds__(WAVE) void k_peaks(const PrologueLaunch L) {
     const int su = __builtin_amdgcn_readlane(h.structure, __builtin_ctzll(todo));
     const bool mine = active && h.structure == su;
     todo &= ~__ballot(mine);
-    if (mine) kpro_peaks(L, i, __builtin_amdgcn_readfirstlane(su), h, l_vm + threadIdx.x, l_ord + threadIdx.x);
+    if (mine) kpro_peaks<NV>(L, i, __builtin_amdgcn_readfirstlane(su), h);
   }
 }
+// By the problem's largest vertex count: the registers of six vertices are twice those of three.
+static void (*peaks_kernel(uint32_t max_v))(const PrologueLaunch) { return max_v <= 3 ? k_peaks<3> : max_v == 4 ? k_peaks<4> : k_peaks<RPEG_MAX_V>; }
 
 // The verdicts of the memory-model launch put into the outputs of the scheduling kernels, where that launch ran beside
 // them instead of ahead of them: the gate bits of the mask, the soft OOM penalty and the stale-layout gate of the
@@ -1393,7 +1390,6 @@ static PrologueLaunch prologue_launch(const rpeg_engine_t* e, uint64_t n, const 
   G.uni = e->d_uni;
   for (int q = 0; q < RPEG_MAX_STRUCT; ++q) G.n_uni[q] = e->n_uni[q];
   G.max_uni = e->max_uni;
-  G.max_v = e->max_v;
   G.dur = e->d_dur; G.dur_stride = e->cap_n;
   G.aux_ovl = e->d_aux_ovl; G.aux_eq = e->d_aux_eq; G.aux_dpne = e->d_aux_dpne; G.vm = e->d_vm;
   G.aux_pen = e->d_aux_pen; G.aux_mask = e->d_aux_mask;
@@ -1860,7 +1856,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     G.row_end = e->max_uni + 1 + (defer ? 0 : e->max_v);
     const unsigned pblk = (unsigned)((n + WAVE - 1) / WAVE);
     hipLaunchKernelGGL(k_prologue, dim3(pblk, prologue_parts(e, G, n)), dim3(WAVE), 0, ahead ? e->s3 : s, G);
-    if (!defer) hipLaunchKernelGGL(k_peaks, dim3(pblk), dim3(WAVE), kpeaks_lds_bytes(e->max_v), s, G);
+    if (!defer) hipLaunchKernelGGL(peaks_kernel(e->max_v), dim3(pblk), dim3(WAVE), 0, s, G);
     HIP_TRY(e, hipGetLastError());
     prologue_done = true;
     peaks_deferred = defer;
@@ -2685,7 +2681,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     G.row_begin = e->max_uni + 1;   // (the memory terms, which nothing but this launch needs: not ahead of the scheduling kernels)
     G.row_end = G.row_begin + e->max_v;
     hipLaunchKernelGGL(k_prologue, dim3(pblk, e->max_v), dim3(WAVE), 0, sp, G);
-    hipLaunchKernelGGL(k_peaks, dim3(pblk), dim3(WAVE), kpeaks_lds_bytes(e->max_v), sp, G);
+    hipLaunchKernelGGL(peaks_kernel(e->max_v), dim3(pblk), dim3(WAVE), 0, sp, G);
     HIP_TRY(e, hipGetLastError());
   }
   if (n_solo) HIP_TRY(e, hipEventRecord(e->ev_join, e->s2));
