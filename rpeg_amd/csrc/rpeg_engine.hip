@@ -99,11 +99,14 @@ __global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
 
 // The layout of a call from the pinned buffer the host wrote it to (read in place, sixteen bytes per thread: a copy
 // command ahead of the kernels costs a dozen microseconds before its first byte moves), and the idle marks of the
-// permutation, in one launch.  n_quads: sixteen-byte words of the layout.
-__global__ void k_upload_fill(const uint4* __restrict__ host_src, uint4* __restrict__ dst, uint64_t n_quads, uint32_t* __restrict__ p,
-                              uint64_t n, uint32_t v) {
+// permutation, in one launch.  n_quads: sixteen-byte words of the layout; n_tasks: of the tasks' classes, where they are in a buffer
+// of their own (1,048,576 DPO plans, 32,800 tasks: two copy commands and a fill of the marks took 30 us between the durations and
+// k_scatter, this launch takes 7).
+__global__ void k_upload_fill(const uint4* __restrict__ host_src, uint4* __restrict__ dst, uint64_t n_quads, const uint4* __restrict__ host_tasks,
+                              uint4* __restrict__ tasks, uint64_t n_tasks, uint32_t* __restrict__ p, uint64_t n, uint32_t v) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n_quads) dst[i] = host_src[i];
+  if (i < n_tasks) tasks[i] = host_tasks[i];
   if (i < n) p[i] = v;
 }
 
@@ -1004,7 +1007,7 @@ struct rpeg_engine_s {
   int split_heavy = 1;                          // 0: the classes with the largest graphs stay in the main kernel
   uint64_t* d_sig = nullptr;
   uint64_t* h_sig = nullptr;
-  uint32_t *d_perm = nullptr, *d_cls = nullptr, *h_cls = nullptr;   // lane -> plan; wavefront -> class blob
+  uint32_t *d_perm = nullptr, *d_cls = nullptr, *h_cls = nullptr, *h_cls_dev = nullptr;   // lane -> plan; wavefront -> class blob (and the pinned buffer it comes from)
   uint8_t* d_ws = nullptr;
   double* d_ranks = nullptr;                    // ranks of k_quad's tasks on their way to the comparison of positions
   size_t ranks_cap = 0;
@@ -1160,12 +1163,13 @@ static int ensure_perm(rpeg_engine_t* e, size_t lanes, size_t tasks) {
     e->cap_perm = cap;
   }
   if (tasks > e->cap_cls) {
-    size_t cap = std::max<size_t>(tasks + tasks / 4, 1024);
+    size_t cap = (std::max<size_t>(tasks + tasks / 4, 1024) + 3) & ~size_t(3);   // (k_upload_fill: sixteen bytes at a time)
     if (e->d_cls) { hipFree(e->d_cls); hipHostFree(e->h_cls); }
-    e->d_cls = e->h_cls = nullptr;
+    e->d_cls = e->h_cls = e->h_cls_dev = nullptr;
     e->cap_cls = 0;
     HIP_TRY(e, hipMalloc(&e->d_cls, cap * 4));
-    HIP_TRY(e, hipHostMalloc(&e->h_cls, cap * 4));
+    HIP_TRY(e, hipHostMalloc(&e->h_cls, cap * 4, hipHostMallocCoherent));
+    HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_cls_dev, e->h_cls, 0));
     e->cap_cls = cap;
   }
   return 0;
@@ -2480,17 +2484,10 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   }
   const hipStream_t sl = ahead ? e->s3 : s;
   const uint64_t n_idle = !one ? n_sorted : 0;   // with one plan per wavefront every entry is written by the scatter
-  if (e->h_ccount_dev && (tasks_in_block || !n_host_tasks)) {
-    const uint64_t n_quads = (block_words - tab0 + (tasks_in_block ? n_host_tasks : 0u) + 3) / 4;
-    const uint64_t threads = std::max<uint64_t>(n_quads, n_idle);
-    hipLaunchKernelGGL(k_upload_fill, dim3((unsigned)((threads + blk - 1) / blk)), dim3(blk), 0, sl, (const uint4*)(e->h_ccount_dev + tab0),
-                       (uint4*)(e->d_ccount + tab0), n_quads, e->d_perm, n_idle, IDLE_LANE);
-  } else {
-    HIP_TRY(e, hipMemcpyAsync(e->d_ccount + tab0, e->h_ccount + tab0, (block_words - tab0 + (tasks_in_block ? n_host_tasks : 0u)) * 4, hipMemcpyHostToDevice, sl));
-    if (n_host_tasks && !tasks_in_block) HIP_TRY(e, hipMemcpyAsync(e->d_cls, e->h_cls, (size_t)n_host_tasks * 4, hipMemcpyHostToDevice, sl));
-    if (n_idle)
-      hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((n_idle + blk - 1) / blk)), dim3(blk), 0, sl, e->d_perm, n_idle, IDLE_LANE);
-  }
+  const uint64_t n_quads = (block_words - tab0 + (tasks_in_block ? n_host_tasks : 0u) + 3) / 4, n_task_quads = tasks_in_block ? 0 : ((uint64_t)n_host_tasks + 3) / 4;
+  const uint64_t threads = std::max(std::max<uint64_t>(n_quads, n_task_quads), n_idle);
+  hipLaunchKernelGGL(k_upload_fill, dim3((unsigned)((threads + blk - 1) / blk)), dim3(blk), 0, sl, (const uint4*)(e->h_ccount_dev + tab0), (uint4*)(e->d_ccount + tab0),
+                     n_quads, (const uint4*)e->h_cls_dev, (uint4*)e->d_cls, n_task_quads, e->d_perm, n_idle, IDLE_LANE);
   const auto t_laid = std::chrono::steady_clock::now();
   hipLaunchKernelGGL(k_scatter, dim3(nblk), dim3(blk), 0, sl, n, e->d_cid, e->d_kidx, d_cfirst, d_clpw, e->d_ccount, shards, e->d_perm, pstride,
                      d_coff, e->d_cls + n_host_tasks, one ? 0u : (uint32_t)n_sorted, e->d_queues, e->d_limit);
