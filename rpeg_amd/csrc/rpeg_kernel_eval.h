@@ -177,14 +177,6 @@ __device__ inline const T& ke_common(const T& x) {
   const uint64_t uniform = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32)) << 32;
   return *(const T*)(const KP_CONST T*)uniform;
 }
-template <int RW>
-struct KeVMem {  // per-vertex memory quantities in LDS, [vertex*4 + field][lane]
-  const double* p;
-  __device__ double w_shard(int v) const { return p[(v * 4 + 0) * RW]; }
-  __device__ double mem_w(int v) const { return p[(v * 4 + 1) * RW]; }
-  __device__ double opt(int v) const { return p[(v * 4 + 2) * RW]; }
-  __device__ double extra(int v) const { return p[(v * 4 + 3) * RW]; }
-};
 
 // max of last_fin over the vertices of a bit set
 __device__ inline double ke_dev_max(unsigned m, const double (&lf)[RPEG_MAX_V]) {
