@@ -3401,6 +3401,11 @@ static int eval_host_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* p
   }
   uint8_t *const d = e->d_stage, *const h = e->h_stage, *const hd = e->h_stage_dev;
   if (int rc = ensure_batch(e, n)) return rc;
+  // No kernel of this call goes on reading or writing the mirror, whatever way it ends: the next call's plans go there without a wait.
+  struct AtRest {
+    hipStream_t s; bool waited = false;
+    ~AtRest() { if (!waited) hipStreamSynchronize(s); }
+  } at_rest{s};
   auto copy = [&](uint8_t* to, const uint8_t* from, size_t bytes, uint32_t flag, uint32_t tag) {
     const uint64_t n16 = (bytes + 15) / 16;
     hipLaunchKernelGGL(k_copy, dim3((unsigned)std::min<uint64_t>((n16 + COPY_BLOCK - 1) / COPY_BLOCK, 4ull * e->n_cu)), dim3(COPY_BLOCK), 0, s, (uint4*)to,
@@ -3427,29 +3432,34 @@ static int eval_host_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* p
   }
   rpeg_plan_soa_t soa{(const int16_t*)d, d + o_head, n};
   if (int rc = eval_batch_impl(e, n, &soa, flags, (double*)(d + o_mk), (double*)(d + o_pk), (double*)(d + o_sc), d + o_mask,
-                               mass ? (double*)(d + o_ms) : nullptr, stream)) {
-    const std::string what = e->err;
-    hipStreamSynchronize(s);   // (nothing of this call goes on reading the mirror)
-    e->err = what;
+                               mass ? (double*)(d + o_ms) : nullptr, stream))
     return rc;
-  }
   // the results in one piece, or, where that is worth a launch each, one after the other: the host copies one to the caller while
-  // the next crosses the bus
+  // the next crosses the bus.  A piece that nobody waits for is not sent.
   struct Part { size_t at, bytes; void* to; };
   const Part part[5] = {{o_mk, b_f64, makespan}, {o_pk, b_f64, peak}, {o_sc, b_f64, score}, {o_ms, mass ? b_f64 * RPEG_MAX_V : 0, mass}, {o_mask, n, mask}};
+  auto wanted = [&](int k) { return part[k].to && part[k].bytes; };
+  int last = 4;
+  while (last >= 0 && !wanted(last)) --last;
+  if (last < 0) {
+    at_rest.waited = true;
+    HIP_TRY(e, hipStreamSynchronize(s));
+    return 0;
+  }
+  const bool at_once = total - o_mk <= HOST_CHUNK;
   uint32_t tag[5] = {};
-  if (total - o_mk <= HOST_CHUNK) {
-    const uint32_t t = next_tag(e);
-    copy(hd + o_mk, d + o_mk, total - o_mk, 1, t);
-    for (uint32_t& x : tag) x = t;
+  if (at_once) {
+    copy(hd + o_mk, d + o_mk, total - o_mk, 1, tag[0] = next_tag(e));
   } else {
     for (int k = 0; k < 5; ++k)
-      if (part[k].to && part[k].bytes) copy(hd + part[k].at, d + part[k].at, part[k].bytes, 1 + k, tag[k] = next_tag(e));
+      if (wanted(k)) copy(hd + part[k].at, d + part[k].at, part[k].bytes, 1 + k, tag[k] = next_tag(e));
   }
   HIP_TRY(e, hipGetLastError());
   for (int k = 0; k < 5; ++k) {
-    if (!part[k].to || !part[k].bytes) continue;
-    if (int rc = wait_tag(e, s, tag[k], total - o_mk <= HOST_CHUNK ? 1u : 1u + (uint32_t)k)) return rc;
+    if (!wanted(k)) continue;
+    const uint32_t from = at_once ? 0u : (uint32_t)k;
+    if (int rc = wait_tag(e, s, tag[from], 1u + from)) return rc;
+    at_rest.waited = at_once || k == last;   // (a call's pieces follow each other)
     std::memcpy(part[k].to, h + part[k].at, part[k].bytes);
   }
   return 0;
