@@ -403,7 +403,8 @@ __global__ __launch_bounds__(COPY_BLOCK) void k_copy(uint4* __restrict__ to, con
 // graphs first: their wavefronts run longest), and within a class the shards in turn.  The counters are left clear for the engine's
 // next call; start[class * shards + shard]: the first task of the class's plans of that shard.  Tasks without a plan are KP_SKIP, and
 // all of them where the batch has plans of classes not lowered yet (k_deal_plans then deals nothing).  host_count, behind the
-// place of the totals: as from k_hand_counts, and the classes of the batch and their plans.
+// place of the totals: as from k_hand_counts, and the classes of the batch and their plans; host_need: likewise, where plans were
+// redone since the last hand-over (whose count k_deal_plans clears).
 // Bound: latency, and the accesses of one compute unit, a line for a class: its shards' counters are one load and one store
 // (4,096 PPO plans, 2,005 classes: 11 us; 13,000, 3,400 classes of four shards: a word at a time 38, now 15).
 constexpr uint32_t DEAL_SHARDS = 4;   // (of a batch of at most 16,384 plans)
@@ -411,8 +412,8 @@ template <uint32_t N> struct alignas(4 * N) DealRow { uint32_t of[N]; };
 template <uint32_t SHARDS>
 __global__ __launch_bounds__(HAND_BLOCK) void k_deal(uint32_t* __restrict__ count, uint32_t n_classes, const uint32_t* __restrict__ order,
                                                      uint32_t* __restrict__ start, uint32_t n, uint32_t* __restrict__ task_cls, uint32_t* __restrict__ unknown,
-                                                     const uint32_t* __restrict__ need, const uint32_t* __restrict__ limit,
-                                                     uint32_t* __restrict__ host_count, uint32_t* __restrict__ host_flag, uint32_t tag) {
+                                                     const uint32_t* __restrict__ need, const uint32_t* __restrict__ limit, const uint32_t* __restrict__ cneed,
+                                                     uint32_t* __restrict__ host_count, uint32_t* __restrict__ host_need, uint32_t* __restrict__ host_flag, uint32_t tag) {
   using Row = DealRow<SHARDS>;
   __shared__ uint32_t wave_total[HAND_BLOCK / WAVE], present;
   const uint32_t lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
@@ -489,6 +490,8 @@ __global__ __launch_bounds__(HAND_BLOCK) void k_deal(uint32_t* __restrict__ coun
     host_count[n_classes + 2 + KE_NEED_SHARDS] = present;
     host_count[n_classes + 3 + KE_NEED_SHARDS] = base;
   }
+  if (redone)
+    for (uint32_t c = threadIdx.x; c < n_classes; c += HAND_BLOCK) host_need[c] = cneed[c];
   __threadfence_system();
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -947,8 +950,11 @@ struct rpeg_engine_s {
   uint64_t count_clean = 0;                     // leading words of d_ccount that the last call left at zero,
   hipStream_t count_clean_on = nullptr;         // on this stream
   uint32_t* h_ccount_dev = nullptr;             // the same pinned buffer as the device addresses it
-  uint32_t *h_tot = nullptr, *h_tot_dev = nullptr;   // pinned: per-class totals of a call (tot_words), then the halves of the class statistic (ccap words each), written by k_hand_counts
-  size_t tot_words() const { return (size_t)ccap + 2 + KE_NEED_SHARDS; }
+  // pinned, written by k_hand_counts or k_deal: what a call's counters came to (tot_words), then the halves of the class statistic
+  // (ccap words each)
+  uint32_t *h_tot = nullptr, *h_tot_dev = nullptr;
+  static size_t tot_words(uint32_t ccap) { return (size_t)ccap + 3 + KE_NEED_SHARDS; }   // (fewer classes than ccap; behind their totals four words and those of `need`)
+  size_t tot_words() const { return tot_words(ccap); }
   uint32_t *h_sigflag = nullptr, *h_sigflag_dev = nullptr;   // pinned word: the tag of the call whose counters are in h_ccount
   uint32_t sig_tag = 0;
   uint32_t *d_cid = nullptr, *d_kidx = nullptr;   // per plan: class id, arrival index within the class
@@ -1129,7 +1135,7 @@ static int ensure_class_tables(rpeg_engine_t* e, hipStream_t s) {
     HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_ccount_dev, e->h_ccount, 0));
     if (e->h_tot) hipHostFree(e->h_tot);
     e->h_tot = e->h_tot_dev = nullptr;
-    HIP_TRY(e, hipHostMalloc(&e->h_tot, (3 * (size_t)cap + 2 + KE_NEED_SHARDS) * 4, hipHostMallocCoherent));
+    HIP_TRY(e, hipHostMalloc(&e->h_tot, (e->tot_words(cap) + 2 * (size_t)cap) * 4, hipHostMallocCoherent));
     HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_tot_dev, e->h_tot, 0));
     if (!e->h_sigflag) {
       HIP_TRY(e, hipHostMalloc(&e->h_sigflag, 64, hipHostMallocCoherent));
@@ -1923,7 +1929,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       uint32_t* const start = e->d_ccount + ((n_count + 3) & ~(uint64_t)3);
       uint32_t* const unknown = e->d_queues + Q_DEAL;
       hipLaunchKernelGGL(shards == 1 ? k_deal<1> : shards == 2 ? k_deal<2> : k_deal<DEAL_SHARDS>, dim3(1), dim3(HAND_BLOCK), 0, s, e->d_ccount, ncls, e->d_order, start, (uint32_t)n, e->d_cls, unknown,
-                         e->d_need, e->d_limit, e->h_tot_dev, e->h_sigflag_dev, tag);
+                         e->d_need, e->d_limit, e->d_cstat + e->cstat_cap, e->h_tot_dev, e->h_tot_dev + e->tot_words(), e->h_sigflag_dev, tag);
       launch_durations(e, n, plans, e->d_cid, s);
       hipLaunchKernelGGL(k_deal_plans, dim3(nblk), dim3(blk), 0, s, (uint32_t)n, e->d_cid, e->d_kidx, start, shards, e->d_order + ncls, e->d_perm,
                          e->d_cls, unknown, e->d_limit);

@@ -42,3 +42,34 @@ def test_plans_that_outgrow_their_form_have_room_in_the_next_calls(c, n, lanes):
         assert redone[4:] == [0, 0, 0], redone    # the calls from the fourth on
     finally:
         eng.close()
+
+
+def test_a_small_batch_between_takes_over_what_the_plans_needed():
+    """The same with batches of a wavefront per plan between the large ones: they are the calls that hear of the redone plans
+    (and that leave nothing of it for the next), so they hand over the classes' ready sets too."""
+    from rpeg_amd.engine.runtime import Engine
+    cfg, a = seeded_batch(5, 20011)
+    _, b = seeded_batch(5, 20011, start=20011)
+    ref = CpuPort(cfg.problem).eval(b, flags=abi.GATE_STALE, threads=16)
+    eng = Engine(cfg.problem)
+    try:
+        eng.set_state_lanes(1)      # (every class is lowered, no ready set measured)
+        eng.eval(b, gate_stale=True)
+        eng.eval(a, gate_stale=True)
+        eng.set_state_lanes(-1)
+        for _ in range(6):
+            eng.eval(a, gate_stale=True)
+        redone = []
+        for call in range(6):
+            out = eng.eval(b, gate_stale=True)
+            assert eng.stats()["quad_tasks"] > 0
+            assert np.array_equal(out["mask"], ref["mask"]), call
+            for k in ("makespan", "peak", "score"):
+                assert same_bits(out[k], ref[k]), (call, k)
+            eng.eval(a.slice(0, 6000), gate_stale=True)
+            assert eng.stats()["state_lanes"] == 1 and eng.stats()["classes_lowered"] == 0
+            redone.append(eng.stats()["redone_before"])
+        assert redone[0] > 0, redone              # (the batches do what the test is about)
+        assert redone[3:] == [0, 0, 0], redone
+    finally:
+        eng.close()
