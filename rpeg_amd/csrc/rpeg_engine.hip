@@ -204,9 +204,11 @@ constexpr int SIG_BLOCK = 256, SIG_TABLE = 512;
 constexpr size_t DIRECT_MAX_CLASSES = 32;   // engines of at most this many classes evaluate small batches without a layout,
 constexpr uint64_t KP_RESIDENT_PER_CU = 16; // wavefronts of k_plan that a compute unit holds, by registers
 constexpr uint64_t DIRECT_PER_CU = 8;       // and so does every batch of at most this many plans per compute unit
-// Task counters of a call's evaluation launches (the main kernel's), what k_deal says of classes not lowered, and the two of
-// k_class_direct: plans of such classes, and the blocks that are done; the blocks of k_copy that are (zero between launches).
-constexpr uint32_t N_QUEUES = 5, Q_DEAL = 1, Q_DIRECT = 2, Q_COPY = 4;
+// Task counters of a call's evaluation launches (the main kernel's), and the two of k_class_direct: plans of classes not lowered,
+// and the blocks that are done; the blocks of k_copy that are (zero between launches).
+constexpr uint32_t N_QUEUES = 4, Q_DIRECT = 1, Q_COPY = 3;
+// Words of h_sigflag: of the counters of a call, of the pieces of the results that k_copy brings, and of the tasks that k_deal dealt.
+constexpr uint32_t FLAG_COUNTS = 0, FLAG_COPY = 1, FLAG_DEALT = 6, N_FLAGS = 16;
 struct SigPlans {   // the plan fields of one thread's plan, a column of an LDS array [field][thread]
   const int16_t* col;
   __device__ VPlan operator[](int v) const { return ke_vplan<SIG_BLOCK>(col, v); }
@@ -371,7 +373,7 @@ __global__ void k_scatter(uint64_t n, const uint32_t* __restrict__ cid, const ui
                           uint32_t pstride, const uint32_t* __restrict__ coff, uint32_t* __restrict__ task_cls,
                           uint32_t first_entry, uint32_t* __restrict__ queues, uint32_t* __restrict__ limit) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < Q_DEAL) queues[i] = 0u;     // the task counters of the evaluation kernels that follow on this stream
+  if (i < Q_DIRECT) queues[i] = 0u;   // the task counters of the evaluation kernels that follow on this stream
   if (i == 0) limit[0] = 0u;          // and the count of plans for the launch that ends the call
   if (i >= n) return;
   const uint32_t c = cid[i];
@@ -401,24 +403,42 @@ __global__ __launch_bounds__(COPY_BLOCK) void k_copy(uint4* __restrict__ to, con
 
 // The layout of a batch that gets a wavefront per plan, by a block of its own: the classes one after the other in `order` (largest
 // graphs first: their wavefronts run longest), and within a class the shards in turn.  The counters are left clear for the engine's
-// next call; start[class * shards + shard]: the first task of the class's plans of that shard.  Tasks without a plan are KP_SKIP, and
-// all of them where the batch has plans of classes not lowered yet (k_deal_plans then deals nothing).  host_count, behind the
-// place of the totals: as from k_hand_counts, and the classes of the batch and their plans; host_need: likewise, where plans were
-// redone since the last hand-over (whose count k_deal_plans clears).
+// next call; start[class * shards + shard]: the first task of the class's plans of that shard.  Tasks without a plan are KP_SKIP.
+// Before that the last wavefront hands over what the host goes on with, under host_flag[FLAG_COUNTS]: host_count, behind the place of
+// the totals, the plans of classes not lowered yet, and from there on as k_hand_counts; host_need: likewise, where plans were redone
+// since the last hand-over (whose count k_deal_plans clears).  With plans of such classes nothing is dealt; the launches that deal and
+// evaluate follow when the host has heard that there are none, which is before this one ends.  (Sent out ahead, to find nothing to do
+// where there are, they kept a first pass over new classes waiting: 4,096 PPO plans, 61 classes to lower, 915 us, now 876; 6,000
+// AC-share, 78 classes, 1,180 / 1,144; laid out by the host 899 and 1,137.)  Behind all these words, under host_flag[FLAG_DEALT]: the
+// classes of the batch and their plans.
 // Bound: latency, and the accesses of one compute unit, a line for a class: its shards' counters are one load and one store
 // (4,096 PPO plans, 2,005 classes: 11 us; 13,000, 3,400 classes of four shards: a word at a time 38, now 15).
 constexpr uint32_t DEAL_SHARDS = 4;   // (of a batch of at most 16,384 plans)
 template <uint32_t N> struct alignas(4 * N) DealRow { uint32_t of[N]; };
 template <uint32_t SHARDS>
 __global__ __launch_bounds__(HAND_BLOCK) void k_deal(uint32_t* __restrict__ count, uint32_t n_classes, const uint32_t* __restrict__ order,
-                                                     uint32_t* __restrict__ start, uint32_t n, uint32_t* __restrict__ task_cls, uint32_t* __restrict__ unknown,
+                                                     uint32_t* __restrict__ start, uint32_t n, uint32_t* __restrict__ task_cls,
                                                      const uint32_t* __restrict__ need, const uint32_t* __restrict__ limit, const uint32_t* __restrict__ cneed,
                                                      uint32_t* __restrict__ host_count, uint32_t* __restrict__ host_need, uint32_t* __restrict__ host_flag, uint32_t tag) {
   using Row = DealRow<SHARDS>;
   __shared__ uint32_t wave_total[HAND_BLOCK / WAVE], present;
   const uint32_t lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
   Row* const rows = (Row*)count;
-  const uint32_t not_lowered = count[(size_t)n_classes * SHARDS], redone = limit[0];
+  const uint32_t not_lowered = count[(size_t)n_classes * SHARDS];
+  if (wave == HAND_BLOCK / WAVE - 1) {
+    const uint32_t redone = limit[0];
+    if (lane < KE_NEED_SHARDS) host_count[n_classes + 1 + lane] = need[lane];
+    if (lane == 0) {
+      host_count[n_classes] = not_lowered;
+      host_count[n_classes + 1 + KE_NEED_SHARDS] = redone;
+    }
+    if (redone)
+      for (uint32_t c = lane; c < n_classes; c += WAVE) host_need[c] = cneed[c];
+    __threadfence_system();
+    __builtin_amdgcn_wave_barrier();
+    if (lane == 0) __hip_atomic_store(host_flag + FLAG_COUNTS, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  if (not_lowered) return;
   if (threadIdx.x == 0) present = 0u;
   // a stretch of the order for every thread, four classes at a time
   constexpr uint32_t AT_ONCE = 4;
@@ -481,30 +501,20 @@ __global__ __launch_bounds__(HAND_BLOCK) void k_deal(uint32_t* __restrict__ coun
       rows[c[j]] = zero;
     }
   }
-  for (uint32_t i = (not_lowered ? 0u : base) + threadIdx.x; i < n; i += HAND_BLOCK) task_cls[i] = KP_SKIP;
+  for (uint32_t i = base + threadIdx.x; i < n; i += HAND_BLOCK) task_cls[i] = KP_SKIP;
   __syncthreads();
-  if (threadIdx.x < KE_NEED_SHARDS) host_count[n_classes + 1 + threadIdx.x] = need[threadIdx.x];
   if (threadIdx.x == 0) {
-    host_count[n_classes] = *unknown = not_lowered;
-    host_count[n_classes + 1 + KE_NEED_SHARDS] = redone;
     host_count[n_classes + 2 + KE_NEED_SHARDS] = present;
     host_count[n_classes + 3 + KE_NEED_SHARDS] = base;
-  }
-  if (redone)
-    for (uint32_t c = threadIdx.x; c < n_classes; c += HAND_BLOCK) host_need[c] = cneed[c];
-  __threadfence_system();
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    count[(size_t)n_classes * SHARDS] = 0u;
-    __hip_atomic_store(host_flag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(host_flag + FLAG_DEALT, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 __global__ void k_deal_plans(uint32_t n, const uint32_t* __restrict__ cid, const uint32_t* __restrict__ kidx, const uint32_t* __restrict__ start,
                              uint32_t shards, const uint32_t* __restrict__ coff, uint32_t* __restrict__ perm, uint32_t* __restrict__ task_cls,
-                             const uint32_t* __restrict__ unknown, uint32_t* __restrict__ limit) {
+                             uint32_t* __restrict__ limit) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) limit[0] = 0u;   // (as k_scatter)
-  if (i >= n || *unknown) return;
+  if (i >= n) return;
   const uint32_t c = cid[i];
   if (c >= CID_UNKNOWN) return;
   const uint32_t task = start[c * shards + ((i / SIG_BLOCK) & (shards - 1u))] + kidx[i];
@@ -955,7 +965,7 @@ struct rpeg_engine_s {
   uint32_t *h_tot = nullptr, *h_tot_dev = nullptr;
   static size_t tot_words(uint32_t ccap) { return (size_t)ccap + 3 + KE_NEED_SHARDS; }   // (fewer classes than ccap; behind their totals four words and those of `need`)
   size_t tot_words() const { return tot_words(ccap); }
-  uint32_t *h_sigflag = nullptr, *h_sigflag_dev = nullptr;   // pinned word: the tag of the call whose counters are in h_ccount
+  uint32_t *h_sigflag = nullptr, *h_sigflag_dev = nullptr;   // pinned words by FLAG_*: the tag of what was handed over last
   uint32_t sig_tag = 0;
   uint32_t *d_cid = nullptr, *d_kidx = nullptr;   // per plan: class id, arrival index within the class
   // the class blobs live on the device; on the host only those that are still to go there, in stretches of the pool
@@ -1138,8 +1148,8 @@ static int ensure_class_tables(rpeg_engine_t* e, hipStream_t s) {
     HIP_TRY(e, hipHostMalloc(&e->h_tot, (e->tot_words(cap) + 2 * (size_t)cap) * 4, hipHostMallocCoherent));
     HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_tot_dev, e->h_tot, 0));
     if (!e->h_sigflag) {
-      HIP_TRY(e, hipHostMalloc(&e->h_sigflag, 64, hipHostMallocCoherent));
-      std::memset(e->h_sigflag, 0, 64);
+      HIP_TRY(e, hipHostMalloc(&e->h_sigflag, N_FLAGS * 4, hipHostMallocCoherent));
+      std::memset(e->h_sigflag, 0, N_FLAGS * 4);
       HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_sigflag_dev, e->h_sigflag, 0));
     }
     e->ccap = cap;
@@ -1423,7 +1433,7 @@ static void launch_durations(const rpeg_engine_t* e, uint64_t n, const rpeg_plan
 static uint32_t next_tag(rpeg_engine_t* e) { return ++e->sig_tag ? e->sig_tag : ++e->sig_tag; }
 // Until a kernel on s has handed over what it was to hand over with this tag; a launch that does not come to an end is the stream's
 // to report.
-static int wait_tag(rpeg_engine_t* e, hipStream_t s, uint32_t tag, uint32_t flag = 0) {
+static int wait_tag(rpeg_engine_t* e, hipStream_t s, uint32_t tag, uint32_t flag = FLAG_COUNTS) {
   const auto begin = std::chrono::steady_clock::now();
   for (uint64_t spins = 0; __atomic_load_n(e->h_sigflag + flag, __ATOMIC_ACQUIRE) != tag; ++spins) {
     if ((spins & 0xFFFFu) == 0xFFFFu && std::chrono::steady_clock::now() - begin > std::chrono::seconds(2)) {
@@ -1811,7 +1821,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     const uint32_t tag = next_tag(e);
     hipLaunchKernelGGL(k_class_direct, dim3((unsigned)((n + SIG_BLOCK - 1) / SIG_BLOCK)), dim3(SIG_BLOCK), 0, s, e->dP, n,
                        plans->vert, plans->head, plans->stride, makespan, peak, score, mask, mass, e->d_hkey, e->d_hoff,
-                       e->hcap - 1, e->d_cls, e->d_queues + Q_DIRECT, e->h_tot_dev, e->h_sigflag_dev, tag);
+                       e->hcap - 1, e->d_cls, e->d_queues + Q_DIRECT, e->h_tot_dev, e->h_sigflag_dev + FLAG_COUNTS, tag);
     HIP_TRY(e, hipGetLastError());
     EvalLaunch L = plan_launch(e, n, plans, flags, makespan, peak, score, mask, mass);
     L.wave_cls = e->d_cls;
@@ -1900,10 +1910,9 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       if (int rc = ensure_side(e)) return rc;
       ahead = !e->prof_on && e->layout_ahead && side_claim(e);
     }
-    // A batch for k_plan whose classes may all be lowered is laid out on the device, and everything goes out at once; the host only
-    // learns afterwards whether a plan belonged to a class not lowered yet (then the launches found nothing to do, and the call goes
-    // on the long way).  us a step, laid out by the host / on the device: PPO 2,500 139 / 132, 4,096 149 / 136, 13,000 286 / 270; GRPO
-    // 9,001 152 / 147; AC-share 6,000 394 / 388.
+    // A batch for k_plan whose classes may all be lowered is laid out on the device; the host only waits to hear that they are
+    // (else the call goes on the long way).  us a step, laid out by the host / on the device: PPO 2,500 139 / 132, 4,096 149 / 136,
+    // 13,000 286 / 270; GRPO 9,001 152 / 147; AC-share 6,000 394 / 388.
     const bool deal = round == 0 && shards <= DEAL_SHARDS && plan_rows && plan_fits() && !e->prof_on && ncls && e->d_pool && e->d_pool_used == e->pool_size;
     if (deal)
       if (int rc = ensure_perm(e, n, n)) return rc;
@@ -1925,29 +1934,20 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       HIP_TRY(e, hipStreamWaitEvent(e->s3, e->ev_sig, 0));
       if (int rc = launch_prologue(true)) return rc;
     }
+    uint32_t* const start = e->d_ccount + ((n_count + 3) & ~(uint64_t)3);   // (k_deal)
     if (deal) {
-      uint32_t* const start = e->d_ccount + ((n_count + 3) & ~(uint64_t)3);
-      uint32_t* const unknown = e->d_queues + Q_DEAL;
-      hipLaunchKernelGGL(shards == 1 ? k_deal<1> : shards == 2 ? k_deal<2> : k_deal<DEAL_SHARDS>, dim3(1), dim3(HAND_BLOCK), 0, s, e->d_ccount, ncls, e->d_order, start, (uint32_t)n, e->d_cls, unknown,
+      hipLaunchKernelGGL(shards == 1 ? k_deal<1> : shards == 2 ? k_deal<2> : k_deal<DEAL_SHARDS>, dim3(1), dim3(HAND_BLOCK), 0, s, e->d_ccount, ncls, e->d_order, start, (uint32_t)n, e->d_cls,
                          e->d_need, e->d_limit, e->d_cstat + e->cstat_cap, e->h_tot_dev, e->h_tot_dev + e->tot_words(), e->h_sigflag_dev, tag);
-      launch_durations(e, n, plans, e->d_cid, s);
-      hipLaunchKernelGGL(k_deal_plans, dim3(nblk), dim3(blk), 0, s, (uint32_t)n, e->d_cid, e->d_kidx, start, shards, e->d_order + ncls, e->d_perm,
-                         e->d_cls, unknown, e->d_limit);
-      EvalLaunch L = plan_launch(e, n, plans, flags, makespan, peak, score, mask, mass);
-      L.perm = e->d_perm; L.wave_cls = e->d_cls;
-      L.dur = e->d_dur; L.dur_stride = e->cap_n;
-      if (e->timing) HIP_TRY(e, hipEventRecord(e->ev0, s));
-      launch_plan(kp_lds_bytes(e->max_nodes, e->max_slots), s, L, e->n_cu);
-      if (e->timing) HIP_TRY(e, hipEventRecord(e->ev1, s));
-    } else
-    hipLaunchKernelGGL(k_hand_counts, dim3(1), dim3(HAND_BLOCK), 0, s, e->d_ccount, e->d_need, ncls, shards, e->d_limit,
-                       e->d_cstat, e->d_cstat + e->cstat_cap, e->h_tot_dev, e->h_tot_dev + e->tot_words(),
-                       read_stat ? e->h_tot_dev + e->tot_words() + e->ccap : nullptr, e->h_sigflag_dev, tag);
+    } else {
+      hipLaunchKernelGGL(k_hand_counts, dim3(1), dim3(HAND_BLOCK), 0, s, e->d_ccount, e->d_need, ncls, shards, e->d_limit,
+                         e->d_cstat, e->d_cstat + e->cstat_cap, e->h_tot_dev, e->h_tot_dev + e->tot_words(),
+                         read_stat ? e->h_tot_dev + e->tot_words() + e->ccap : nullptr, e->h_sigflag_dev + FLAG_COUNTS, tag);
+    }
     HIP_TRY(e, hipGetLastError());
     if (round == 0) {
       if (!own_prologue && !ahead)
         if (int rc = launch_prologue(true)) return rc;
-      if (plan_rows && !deal) {
+      if (plan_rows) {
         launch_durations(e, n, plans, e->d_cid, s);
         HIP_TRY(e, hipGetLastError());
       }
@@ -1965,7 +1965,17 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       if (read_stat) std::copy_n(e->h_tot + e->tot_words() + e->ccap, ncls, e->cls_pops16.begin());
     }
     if (deal && e->h_tot[ncls] == 0) {
-      e->count_clean = n_count;
+      hipLaunchKernelGGL(k_deal_plans, dim3(nblk), dim3(blk), 0, s, (uint32_t)n, e->d_cid, e->d_kidx, start, shards, e->d_order + ncls, e->d_perm,
+                         e->d_cls, e->d_limit);
+      EvalLaunch L = plan_launch(e, n, plans, flags, makespan, peak, score, mask, mass);
+      L.perm = e->d_perm; L.wave_cls = e->d_cls;
+      L.dur = e->d_dur; L.dur_stride = e->cap_n;
+      if (e->timing) HIP_TRY(e, hipEventRecord(e->ev0, s));
+      launch_plan(kp_lds_bytes(e->max_nodes, e->max_slots), s, L, e->n_cu);
+      HIP_TRY(e, hipGetLastError());
+      if (e->timing) HIP_TRY(e, hipEventRecord(e->ev1, s));
+      if (int rc = wait_tag(e, s, tag, FLAG_DEALT)) return rc;
+      e->count_clean = n_count;   // (the last one was zero)
       e->count_clean_on = s;
       ++e->batch_calls;
       for (uint64_t& x : e->stats) x = &x == &e->stats[8] ? x : 0;
@@ -1975,7 +1985,8 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       e->stats[5] = 1;
       e->host_us[0] = std::chrono::duration<double, std::micro>(t_counts - t_call).count();
       e->host_us[1] = std::chrono::duration<double, std::micro>(t_waited - t_counts).count();
-      e->host_us[2] = e->host_us[3] = 0.0;
+      e->host_us[2] = 0.0;
+      e->host_us[3] = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t_waited).count();
       return read_timing(e);
     }
     if (e->h_tot[ncls] == 0) break;
@@ -3455,16 +3466,16 @@ static int eval_host_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* p
   const bool at_once = total - o_mk <= HOST_CHUNK;
   uint32_t tag[5] = {};
   if (at_once) {
-    copy(hd + o_mk, d + o_mk, total - o_mk, 1, tag[0] = next_tag(e));
+    copy(hd + o_mk, d + o_mk, total - o_mk, FLAG_COPY, tag[0] = next_tag(e));
   } else {
     for (int k = 0; k < 5; ++k)
-      if (wanted(k)) copy(hd + part[k].at, d + part[k].at, part[k].bytes, 1 + k, tag[k] = next_tag(e));
+      if (wanted(k)) copy(hd + part[k].at, d + part[k].at, part[k].bytes, FLAG_COPY + k, tag[k] = next_tag(e));
   }
   HIP_TRY(e, hipGetLastError());
   for (int k = 0; k < 5; ++k) {
     if (!wanted(k)) continue;
     const uint32_t from = at_once ? 0u : (uint32_t)k;
-    if (int rc = wait_tag(e, s, tag[from], 1u + from)) return rc;
+    if (int rc = wait_tag(e, s, tag[from], FLAG_COPY + from)) return rc;
     at_rest.waited = at_once || k == last;   // (a call's pieces follow each other)
     std::memcpy(part[k].to, h + part[k].at, part[k].bytes);
   }
