@@ -521,6 +521,12 @@ int rpeg_engine_set_quad_share(rpeg_engine_t* e, int32_t percent);
    it to reach the redo path. */
 int rpeg_engine_set_ready_cap(rpeg_engine_t* e, int32_t entries);
 
+/* Device memory, in bytes, that the kernel of two or four lanes per plan may hold for the node ranks of a batch, eight bytes for
+   each plan and node of the largest graphs among them (0, the default: 4 GiB; what it holds is kept for the engine's later
+   calls).  A batch that needs more, or more than the device has left, takes its plans in turns.  Results do not depend on the
+   setting.  No reference counterpart. */
+int rpeg_engine_set_rank_memory(rpeg_engine_t* e, uint64_t bytes);
+
 /* Forgets every lowered class, so that the next rpeg_eval_batch lowers all the classes of its batch
    again (used to measure a cold call). */
 int rpeg_engine_reset_classes(rpeg_engine_t* e);

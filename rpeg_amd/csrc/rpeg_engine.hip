@@ -895,6 +895,9 @@ static uint8_t* static_scratch_ptr(int dev, hipError_t* st) {
 //                                              through where k_quad runs beside them
 //   quad_margin                                a batch moves to k_quad only if the main kernel would end this much later
 //   gain_threshold, gain_classes               a split by class size / by measured time must model this much earlier
+// Ranks that an engine holds room for, unless told otherwise: 4 GiB (two million plans of graphs of 250 nodes; 1,048,576 DPO plans
+// take 0.23 GiB, 262,144 AC-share plans 0.35).
+constexpr size_t RANKS_MOST = ((size_t)4 << 30) / 8;
 struct SplitModel {
   double plan_a = 9.0, plan_b = 0.8, plan_list = 1.25;
   double quad_a = 10.0, quad_b = 1.3, quad_c = 0.2;
@@ -1026,7 +1029,7 @@ struct rpeg_engine_s {
   uint32_t *d_perm = nullptr, *d_cls = nullptr, *h_cls = nullptr, *h_cls_dev = nullptr;   // lane -> plan; wavefront -> class blob (and the pinned buffer it comes from)
   uint8_t* d_ws = nullptr;
   double* d_ranks = nullptr;                    // ranks of k_quad's tasks on their way to the comparison of positions
-  size_t ranks_cap = 0;
+  size_t ranks_cap = 0, ranks_most = RANKS_MOST;   // doubles: it holds, it may hold (rpeg_engine_set_rank_memory)
   // outputs of the prologue launches (rpeg_kernel_prologue.h), cap_n plans each: pair relations, penalty factor, gate
   // bits; the durations of the slot universe ([slot][plan]); and the universe itself
   uint64_t *d_aux_ovl = nullptr, *d_aux_dpne = nullptr, *d_aux_eq = nullptr;
@@ -1376,16 +1379,24 @@ static int ensure_ws(rpeg_engine_t* e, size_t bytes, hipStream_t s) {
   return 0;
 }
 
-// ranks of the tasks of k_quad
-static int ensure_ranks(rpeg_engine_t* e, size_t doubles, hipStream_t s) {
-  if (doubles <= e->ranks_cap) return 0;
+// Room for the ranks of the tasks of k_quad, a quarter more than asked for (what a batch needs goes with its largest graphs, from call
+// to call at the same number of plans).  Where that is more than the engine may hold, or than there is, half of it, and so on down to
+// `least`: the launches then take their tasks in turns (QuadLaunch::at_once).
+static int ensure_ranks(rpeg_engine_t* e, size_t doubles, size_t least, hipStream_t s) {
+  const size_t most = std::max(e->ranks_most, least);
+  if (doubles <= e->ranks_cap || (least <= e->ranks_cap && 2 * e->ranks_cap > most)) return 0;
   HIP_TRY(e, hipStreamSynchronize(s));
   if (e->d_ranks) hipFree(e->d_ranks);
   e->d_ranks = nullptr;
   e->ranks_cap = 0;
-  HIP_TRY(e, hipMalloc(&e->d_ranks, doubles * 8));
-  e->ranks_cap = doubles;
-  return 0;
+  for (size_t ask = doubles + doubles / 4;; ask = ask > doubles ? doubles : std::max(ask / 2, least)) {
+    if (ask > most) continue;
+    const hipError_t got = hipMalloc(&e->d_ranks, ask * 8);
+    if (got == hipSuccess) { e->ranks_cap = ask; return 0; }
+    hipGetLastError();   // (not the next launch's)
+    e->d_ranks = nullptr;
+    if (got != hipErrorOutOfMemory || ask == least) HIP_TRY(e, got);
+  }
 }
 
 // state of the launch that redoes flagged plans: as many wavefronts as 128 MiB hold, at most one per compute unit
@@ -1653,6 +1664,18 @@ int rpeg_engine_set_ready_cap(rpeg_engine_t* e, int32_t entries) {
   }
   e->ready_cap = (uint32_t)entries;
   e->split_for_n = 0;
+  return 0;
+}
+
+int rpeg_engine_set_rank_memory(rpeg_engine_t* e, uint64_t bytes) {
+  if (!e) return -1;
+  e->ranks_most = bytes ? bytes / 8 : RANKS_MOST;
+  if (e->ranks_cap > e->ranks_most) {
+    hipDeviceSynchronize();
+    hipFree(e->d_ranks);
+    e->d_ranks = nullptr;
+    e->ranks_cap = 0;
+  }
   return 0;
 }
 
@@ -2351,7 +2374,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // after the other, the one of the largest LDS on a stream of its own and the others by turns on two: a launch behind another
   // waits for its slowest task.  (AC-share, us per step, 262,144 / 140,001 plans: 1 launch a form 5,560 / 3,127, 2 4,325 / 2,632, 3
   // 4,090 / 2,754, 4 4,105 / 2,752; 3 with the last one alone on a stream 4,320 / 2,800, all of them on one 6,190 / 4,290.)
-  struct QuadLaunch { uint32_t first = 0, waves = 0; QuadSize size; size_t ranks = 0; int kind = 0; bool aside = false, first_stream = false; };   // on the fourth stream; on the main kernel's, where that has no tasks
+  struct QuadLaunch { uint32_t first = 0, waves = 0; QuadSize size; size_t ranks = 0; uint32_t at_once = 0; int kind = 0; bool aside = false, first_stream = false; };   // on the fourth stream; on the main kernel's, where that has no tasks
   std::vector<QuadLaunch> quad_launch;
   bool aside = false;   // some launch is
   {
@@ -2426,13 +2449,20 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
         auto lds_by = [&](uint32_t x) { q.size.parts = x; return (double)kq_lds_bytes(plans, q.size, mass != nullptr); };
         q.size.parts = lds_by(parts) > QUAD_PART_LDS * lds_by(2 * parts) ? 2 * parts : parts;
       }
-    size_t doubles = 0;
-    for (QuadLaunch& q : quad_launch) {
-      if (q.size.parts == 1) continue;   // (in LDS)
-      q.ranks = doubles;
-      doubles += (size_t)q.waves * kq_rank_doubles(QUAD_KIND[q.kind].plans, q.size);
+    size_t doubles = 0, least = 0;   // of all tasks; of one of each launch
+    auto rank_doubles = [](const QuadLaunch& q) { return q.size.parts == 1 ? 0 : kq_rank_doubles(QUAD_KIND[q.kind].plans, q.size); };   // (0: in LDS)
+    for (const QuadLaunch& q : quad_launch) {
+      doubles += q.waves * rank_doubles(q);
+      least += rank_doubles(q);
     }
-    if (int rc = ensure_ranks(e, doubles, s)) return rc;
+    if (int rc = ensure_ranks(e, doubles, least, s)) return rc;
+    size_t at = 0;
+    for (QuadLaunch& q : quad_launch) {
+      q.at_once = q.waves;
+      if (doubles > e->ranks_cap && rank_doubles(q)) q.at_once = std::min<uint32_t>(q.waves, 1u + (uint32_t)(q.waves * (e->ranks_cap - least) / doubles));
+      q.ranks = at;
+      at += q.at_once * rank_doubles(q);
+    }
   }
   const uint32_t n_lane_waves = n_eval_waves + n_quad_waves;
   const uint32_t pstride = one ? 1u : (uint32_t)WAVE;
@@ -2624,13 +2654,6 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     HIP_TRY(e, hipEventRecord(e->ev0, s));
   }
   auto launch_quad = [&](const QuadLaunch& q, hipStream_t on) -> int {
-    if (!q.waves) return 0;
-    EvalLaunch Q = L;
-    Q.perm = e->d_perm + ((uint64_t)n_eval_waves + q.first) * WAVE;
-    Q.wave_cls = L.wave_cls + n_eval_waves + q.first;
-    Q.n_waves = q.waves;
-    Q.ovf = nullptr; Q.cstat = nullptr; Q.queue = nullptr;   // (a plan that outgrows the entries is flagged in Q.limit)
-    if (L.prof) Q.prof = L.prof + (n_waves + q.first) * 8;
     const size_t qlds = kq_lds_bytes(QUAD_KIND[q.kind].plans, q.size, mass != nullptr);
     if (qlds > 64 * 1024 && !e->quad_attr_set) {
       HIP_TRY(e, hipFuncSetAttribute((const void*)k_quad<2, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
@@ -2638,10 +2661,19 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       HIP_TRY(e, hipFuncSetAttribute((const void*)k_quad<4, 6>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
       e->quad_attr_set = true;
     }
-    if (q.kind == 0) hipLaunchKernelGGL((k_quad<2, 4>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q, q.size, e->d_ranks + q.ranks);
-    else if (q.kind == 1) hipLaunchKernelGGL((k_quad<4, 4>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q, q.size, e->d_ranks + q.ranks);
-    else hipLaunchKernelGGL((k_quad<4, 6>), dim3((unsigned)q.waves), dim3(WAVE), qlds, on, Q, q.size, e->d_ranks + q.ranks);
-    HIP_TRY(e, hipGetLastError());
+    for (uint32_t w = q.first; w < q.first + q.waves; w += q.at_once) {
+      EvalLaunch Q = L;
+      Q.perm = e->d_perm + ((uint64_t)n_eval_waves + w) * WAVE;
+      Q.wave_cls = L.wave_cls + n_eval_waves + w;
+      Q.n_waves = std::min(q.at_once, q.first + q.waves - w);
+      Q.ovf = nullptr; Q.cstat = nullptr; Q.queue = nullptr;   // (a plan that outgrows the entries is flagged in Q.limit)
+      if (L.prof) Q.prof = L.prof + (n_waves + w) * 8;
+      const dim3 grid_q((unsigned)Q.n_waves);
+      if (q.kind == 0) hipLaunchKernelGGL((k_quad<2, 4>), grid_q, dim3(WAVE), qlds, on, Q, q.size, e->d_ranks + q.ranks);
+      else if (q.kind == 1) hipLaunchKernelGGL((k_quad<4, 4>), grid_q, dim3(WAVE), qlds, on, Q, q.size, e->d_ranks + q.ranks);
+      else hipLaunchKernelGGL((k_quad<4, 6>), grid_q, dim3(WAVE), qlds, on, Q, q.size, e->d_ranks + q.ranks);
+      HIP_TRY(e, hipGetLastError());
+    }
     return 0;
   };
   auto launch_main = [&]() {

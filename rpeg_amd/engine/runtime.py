@@ -23,7 +23,7 @@ _lib = None
 EXPORTS = ("rpeg_engine_create", "rpeg_engine_destroy", "rpeg_last_error", "rpeg_eval_batch",
            "rpeg_op_time_batch", "rpeg_eval_trace", "rpeg_engine_stats", "rpeg_engine_set_timing",
            "rpeg_engine_last_kernel_ms", "rpeg_device_exp", "rpeg_engine_reset_classes", "rpeg_eval_batch_mass",
-           "rpeg_sa_run", "rpeg_sa_propose", "rpeg_eval_host_util", "rpeg_engine_set_state_lanes", "rpeg_engine_set_sa_groups", "rpeg_engine_set_side_layout", "rpeg_engine_host_us", "rpeg_engine_set_split_model", "rpeg_engine_set_quad_share", "rpeg_engine_set_ready_cap", "rpeg_engine_profile", "rpeg_sa_optimize", "rpeg_eval_host",
+           "rpeg_sa_run", "rpeg_sa_propose", "rpeg_eval_host_util", "rpeg_engine_set_state_lanes", "rpeg_engine_set_sa_groups", "rpeg_engine_set_side_layout", "rpeg_engine_host_us", "rpeg_engine_set_split_model", "rpeg_engine_set_quad_share", "rpeg_engine_set_ready_cap", "rpeg_engine_set_rank_memory", "rpeg_engine_profile", "rpeg_sa_optimize", "rpeg_eval_host",
            "rpeg_sa_optimize_families", "rpeg_eval_trace_metrics", "rpeg_eval_batch_static", "rpeg_plan_detail",
            "rpeg_lower_plan", "rpeg_eval_host_trace")
 
@@ -97,6 +97,8 @@ def load_library(path: Optional[str] = None):
     lib.rpeg_engine_set_quad_share.argtypes = [vp, i32]
     lib.rpeg_engine_set_ready_cap.restype = C.c_int
     lib.rpeg_engine_set_ready_cap.argtypes = [vp, i32]
+    lib.rpeg_engine_set_rank_memory.restype = C.c_int
+    lib.rpeg_engine_set_rank_memory.argtypes = [vp, u64]
     lib.rpeg_engine_reset_classes.restype = C.c_int
     lib.rpeg_engine_reset_classes.argtypes = [vp]
     lib.rpeg_engine_profile.restype = C.c_int
@@ -245,6 +247,11 @@ class Engine:
         """Ready-list entries per plan in the main kernel (8, 16, 24 or 32); plans that need more are redone by the
         launch that ends the call, without a bound."""
         self._check(self.lib.rpeg_engine_set_ready_cap(self._h, int(entries)), "rpeg_engine_set_ready_cap")
+
+    def set_rank_memory(self, nbytes: int):
+        """Device memory that the few-lanes-per-plan kernel may hold for the ranks of a batch (0: the default); a batch that
+        needs more takes its plans in turns."""
+        self._check(self.lib.rpeg_engine_set_rank_memory(self._h, int(nbytes)), "rpeg_engine_set_rank_memory")
 
     def reset_classes(self):
         self.lib.rpeg_engine_reset_classes(self._h)

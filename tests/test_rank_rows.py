@@ -86,3 +86,57 @@ def test_ranks_at_once_and_by_parts(c, K, n):
                 assert same_bits(out[k], want[k]), (call, k)
     finally:
         eng.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c,n,nbytes", [(4, 140001, 1), (2, 70001, 1 << 20), (5, 60011, 3 << 20)])
+def test_ranks_by_turns(c, n, nbytes):
+    """Less memory for ranks than the launches' tasks take at once (1 byte: one task of each launch at a time)."""
+    from rpeg_amd.engine.runtime import Engine
+    cfg, batch = seeded_batch(c, n)
+    want = CpuPort(cfg.problem).eval(batch, flags=abi.GATE_STALE, threads=16)
+    eng = Engine(cfg.problem)
+    try:
+        eng.set_state_lanes(4)
+        for most in (0, nbytes, 0):
+            eng.set_rank_memory(most)
+            out = eng.eval(batch, gate_stale=True)
+            assert eng.stats()["quad_tasks"] > 0 and np.array_equal(out["mask"], want["mask"])
+            for k in ("makespan", "peak", "score"):
+                assert same_bits(out[k], want[k]), (most, k)
+    finally:
+        eng.close()
+
+
+@pytest.mark.gpu
+def test_a_batch_with_slightly_larger_graphs_needs_no_new_memory():
+    import torch
+    from rpeg_amd.engine.runtime import DeviceBatch, Engine
+    cfg, batch = seeded_batch(5, 60011)
+    port = CpuPort(cfg.problem)
+    sig = port.eval(batch, threads=16)["sig"]
+    known, of = np.unique(sig[sig != np.uint64(2 ** 64 - 1)], return_inverse=True)
+    nodes = np.array([port.blob(x)[0][:4].view("<u4")[0] for x in known])[of]
+    by_size = np.flatnonzero(sig != np.uint64(2 ** 64 - 1))[np.argsort(nodes, kind="stable")]
+    n = 40000
+    # mostly plans of the smallest graphs, with some of the next larger (up to 132 nodes), and with fewer of the largest (158)
+    first, second = (np.concatenate([by_size[:n - n // k], by_size[at:at + n // k]]) for at, k in ((44000, 3), (56000, 10)))
+    eng = Engine(cfg.problem)
+    try:
+        eng.set_state_lanes(4)
+        out = eng.alloc_outputs(n)
+        for _ in range(3):                          # every class is lowered and has its form
+            for k in range(6):
+                eng.eval_device(DeviceBatch(batch.take(by_size[k::6]), "cuda:0"), out)
+        batches = [DeviceBatch(batch.take(idx), "cuda:0") for idx in (first, second)]
+        free = []
+        for b in batches:
+            for _ in range(2):
+                eng.eval_device(b, out)
+            torch.cuda.synchronize()
+            free.append(torch.cuda.mem_get_info()[0])
+        assert free[0] == free[1]
+        eng.set_rank_memory(8)                      # (gives back what it holds: there was some)
+        assert torch.cuda.mem_get_info()[0] > free[1]
+    finally:
+        eng.close()
