@@ -207,8 +207,10 @@ constexpr uint64_t DIRECT_PER_CU = 8;       // and so does every batch of at mos
 // Task counters of a call's evaluation launches (the main kernel's), and the two of k_class_direct: plans of classes not lowered,
 // and the blocks that are done; the blocks of k_copy that are (zero between launches).
 constexpr uint32_t N_QUEUES = 4, Q_DIRECT = 1, Q_COPY = 3;
-// Words of h_sigflag: of the counters of a call, of the pieces of the results that k_copy brings, and of the tasks that k_deal dealt.
-constexpr uint32_t FLAG_COUNTS = 0, FLAG_COPY = 1, FLAG_DEALT = 6, N_FLAGS = 16;
+// Words of h_sigflag: of the counters of a call, of the pieces of the results that k_copy brings (5), of the tasks that k_deal
+// dealt, and of the pieces of plans that k_copy fetched.
+constexpr uint32_t STAGE_SLOTS = 4;
+constexpr uint32_t FLAG_COUNTS = 0, FLAG_COPY = 1, FLAG_DEALT = 6, FLAG_SLOT = 7, N_FLAGS = FLAG_SLOT + STAGE_SLOTS;
 struct SigPlans {   // the plan fields of one thread's plan, a column of an LDS array [field][thread]
   const int16_t* col;
   __device__ VPlan operator[](int v) const { return ke_vplan<SIG_BLOCK>(col, v); }
@@ -387,17 +389,20 @@ __global__ void k_scatter(uint64_t n, const uint32_t* __restrict__ cid, const ui
 
 // Between pinned host memory and the device, sixteen bytes a thread, in order on the call's stream: no other engine's signal to
 // wait for, no command queue of its own.  With a flag the block that is done last hands over the tag (done: a counter, zero between
-// launches).
+// launches).  On the way to the host what was written must be there before the flag; on the way from it what was read has been read,
+// as it was stored, and nothing is to be made visible (a fence of the whole system a block takes the device's cache back to memory:
+// 131,072 GRPO plans 1,110 us a call, without it 935).
 constexpr uint32_t COPY_BLOCK = 256;
+template <bool TO_HOST>
 __global__ __launch_bounds__(COPY_BLOCK) void k_copy(uint4* __restrict__ to, const uint4* __restrict__ from, uint64_t n, uint32_t* __restrict__ done,
                                                      uint32_t* __restrict__ host_flag, uint32_t tag) {
   for (uint64_t i = (uint64_t)blockIdx.x * COPY_BLOCK + threadIdx.x; i < n; i += (uint64_t)gridDim.x * COPY_BLOCK) to[i] = from[i];
   if (!host_flag) return;
-  __threadfence_system();
+  if (TO_HOST) __threadfence_system();
   __syncthreads();
   if (threadIdx.x == 0 && atomicAdd(done, 1u) == gridDim.x - 1u) {
     atomicExch(done, 0u);
-    __hip_atomic_store(host_flag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(host_flag, tag, TO_HOST ? __ATOMIC_RELEASE : __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -985,8 +990,9 @@ struct rpeg_engine_s {
   // written by the kernel itself)
   HostLane lane0;
   uint8_t* d_stage = nullptr;   // host tensors and results of larger host-pointer batches on the device
-  uint8_t *h_stage = nullptr, *h_stage_dev = nullptr;   // and its pinned mirror
   size_t stage_cap = 0;
+  uint8_t *h_stage = nullptr, *h_stage_dev = nullptr;   // pinned: STAGE_SLOTS pieces of plans on their way there, then the results on their way back
+  size_t pinned_cap = 0;
   uint8_t *h_times = nullptr, *h_times_dev = nullptr;   // pinned: EvalLaunch::trace
   size_t h_times_nodes = 0;
   uint8_t* d_trace = nullptr;   // rpeg_eval_trace: one plan's fields and header, then start / finish / dispatch index
@@ -1075,6 +1081,11 @@ static int ensure_batch(rpeg_engine_t* e, size_t n) {
     HIP_TRY(e, hipMalloc(&e->d_queues, N_QUEUES * 4));
     HIP_TRY(e, hipMemset(e->d_queues, 0, N_QUEUES * 4));
   }
+  if (!e->h_sigflag) {
+    HIP_TRY(e, hipHostMalloc(&e->h_sigflag, N_FLAGS * 4, hipHostMallocCoherent));
+    std::memset(e->h_sigflag, 0, N_FLAGS * 4);
+    HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_sigflag_dev, e->h_sigflag, 0));
+  }
   if (!e->d_need) {
     HIP_TRY(e, hipMalloc(&e->d_need, (KE_NEED_SHARDS + 1) * 4));
     HIP_TRY(e, hipMemset(e->d_need, 0, (KE_NEED_SHARDS + 1) * 4));
@@ -1150,11 +1161,6 @@ static int ensure_class_tables(rpeg_engine_t* e, hipStream_t s) {
     e->h_tot = e->h_tot_dev = nullptr;
     HIP_TRY(e, hipHostMalloc(&e->h_tot, (e->tot_words(cap) + 2 * (size_t)cap) * 4, hipHostMallocCoherent));
     HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_tot_dev, e->h_tot, 0));
-    if (!e->h_sigflag) {
-      HIP_TRY(e, hipHostMalloc(&e->h_sigflag, N_FLAGS * 4, hipHostMallocCoherent));
-      std::memset(e->h_sigflag, 0, N_FLAGS * 4);
-      HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_sigflag_dev, e->h_sigflag, 0));
-    }
     e->ccap = cap;
   }
   if (ncls > e->cstat_cap) {   // the per-class statistic keeps what it has learned
@@ -3426,57 +3432,64 @@ static int eval_host_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* p
     const int rc = eval_host_small(e, n, get, flags, makespan, peak, score, mask, mass, s);
     if (rc <= 0) return rc;
   }
-  // Device path: plans and results staged in device memory for this call, with a pinned mirror of the block in host memory.  The
-  // plans go up in chunks: while the device fetches one, the host copies the next into the mirror.
-  // Bound: the bus (some 50 GB/s) and, beside it, the host's copies (70 GB/s).  Copies of the caller's pageable memory by the runtime,
-  // and of the results by a command behind the kernels, which waits for them on a queue of its own, against these, us a call: 9,001
-  // GRPO plans 258 / 213, 131,072 1,140 / 948; 2,500 PPO 207 / 172, 30,001 609 / 577; 1,500 DPO 92 / 83, 131,072 848 / 616.
+  // Device path: plans and results staged in device memory for this call.  The plans go up in pieces through STAGE_SLOTS pinned
+  // ones: while the device fetches one, the host copies the next.
+  // Bound: the bus (some 50 GB/s) and, beside it, the host's copies (70 GB/s).  Plans from the caller's pageable memory by the runtime
+  // and results by a command behind the kernels, which waits for them on a queue of its own / all of it through a pinned copy of the
+  // whole call / now, us a call: 9,001 GRPO plans 304 / 215 / 211, 131,072 1,212 / 927 / 935; 2,500 PPO 215 / 166 / 162, 30,001 748 / 584 /
+  // 591; 1,500 DPO 96 / 77 / 78, 131,072 837 / 598 / 606, 1,048,576 6,417 / 4,755 / 4,027.  The first host call of an engine, which
+  // pins the memory: 65,536 GRPO 1.7 / 3.5 / 2.4 ms, 1,048,576 DPO 16.5 / 36.8 / 14.5.
   const size_t V = (size_t)e->max_v * RPEG_FIELDS;   // (fields of vertices that no structure has are not read)
   const size_t b_row = 2 * n, b_vert = V * b_row, b_head = 4 * n, b_f64 = 8 * n;
   auto align = [](size_t x) { return (x + 255) & ~size_t(255); };
   const size_t o_head = align(b_vert), o_mk = align(o_head + b_head), o_pk = align(o_mk + b_f64), o_sc = align(o_pk + b_f64),
                o_ms = align(o_sc + b_f64), o_mask = align(o_ms + (mass ? b_f64 * RPEG_MAX_V : 0)), total = align(o_mask + n);
+  const size_t b_slots = std::min<size_t>(o_mk, STAGE_SLOTS * HOST_CHUNK), pinned = b_slots + (total - o_mk);
+  if (total > e->stage_cap || pinned > e->pinned_cap) HIP_TRY(e, hipStreamSynchronize(s));
   if (total > e->stage_cap) {   // grow-only, kept by the engine
-    HIP_TRY(e, hipStreamSynchronize(s));
     if (e->d_stage) hipFree(e->d_stage);
-    if (e->h_stage) hipHostFree(e->h_stage);
-    e->d_stage = e->h_stage = e->h_stage_dev = nullptr;
+    e->d_stage = nullptr;
     e->stage_cap = 0;
-    const size_t cap = total + total / 4;
-    HIP_TRY(e, hipMalloc(&e->d_stage, cap));
-    HIP_TRY(e, hipHostMalloc(&e->h_stage, cap, hipHostMallocCoherent));
+    HIP_TRY(e, hipMalloc(&e->d_stage, total + total / 4));
+    e->stage_cap = total + total / 4;
+  }
+  if (pinned > e->pinned_cap) {
+    if (e->h_stage) hipHostFree(e->h_stage);
+    e->h_stage = e->h_stage_dev = nullptr;
+    e->pinned_cap = 0;
+    HIP_TRY(e, hipHostMalloc(&e->h_stage, pinned + pinned / 4, hipHostMallocCoherent));
     HIP_TRY(e, hipHostGetDevicePointer((void**)&e->h_stage_dev, e->h_stage, 0));
-    e->stage_cap = cap;
+    e->pinned_cap = pinned + pinned / 4;
   }
   uint8_t *const d = e->d_stage, *const h = e->h_stage, *const hd = e->h_stage_dev;
   if (int rc = ensure_batch(e, n)) return rc;
-  // No kernel of this call goes on reading or writing the mirror, whatever way it ends: the next call's plans go there without a wait.
+  // No kernel of this call goes on reading or writing pinned memory, whatever way it ends: the next call's plans go there without a wait.
   struct AtRest {
     hipStream_t s; bool waited = false;
     ~AtRest() { if (!waited) hipStreamSynchronize(s); }
   } at_rest{s};
-  auto copy = [&](uint8_t* to, const uint8_t* from, size_t bytes, uint32_t flag, uint32_t tag) {
+  auto copy = [&](void (*kernel)(uint4*, const uint4*, uint64_t, uint32_t*, uint32_t*, uint32_t), uint8_t* to, const uint8_t* from, size_t bytes, uint32_t flag, uint32_t tag) {
     const uint64_t n16 = (bytes + 15) / 16;
-    hipLaunchKernelGGL(k_copy, dim3((unsigned)std::min<uint64_t>((n16 + COPY_BLOCK - 1) / COPY_BLOCK, 4ull * e->n_cu)), dim3(COPY_BLOCK), 0, s, (uint4*)to,
+    hipLaunchKernelGGL(kernel, dim3((unsigned)std::min<uint64_t>((n16 + COPY_BLOCK - 1) / COPY_BLOCK, 4ull * e->n_cu)), dim3(COPY_BLOCK), 0, s, (uint4*)to,
                        (const uint4*)from, n16, e->d_queues + Q_COPY, tag ? e->h_sigflag_dev + flag : nullptr, tag);
   };
-  {
-    size_t sent = 0;   // bytes on their way, a multiple of sixteen
-    auto send = [&](size_t upto) {
-      if (upto > sent) copy(d + sent, hd + sent, upto - sent, 0, 0);
-      sent = upto;
+  uint32_t slot_tag[STAGE_SLOTS] = {};
+  for (size_t at = 0, piece = 0; at < o_mk; at += HOST_CHUNK, ++piece) {   // bytes at to end - 1 of the plans
+    const uint32_t slot = piece % STAGE_SLOTS;
+    const size_t end = std::min(at + HOST_CHUNK, o_mk);
+    uint8_t* const to = h + slot * HOST_CHUNK;
+    if (piece >= STAGE_SLOTS)
+      if (int rc = wait_tag(e, s, slot_tag[slot], FLAG_SLOT + slot)) return rc;
+    auto put = [&](size_t begin, const void* from, size_t bytes) {   // what of a stretch falls into this piece
+      const size_t lo = std::max(begin, at), hi = std::min(begin + bytes, end);
+      if (lo < hi) std::memcpy(to + (lo - at), (const uint8_t*)from + (lo - begin), hi - lo);
     };
-    size_t put = 0;    // rows of the mirror that are filled
-    for (const size_t chunk = std::max<size_t>(1, HOST_CHUNK / b_row); put < V;) {
-      const size_t rows = std::min(chunk, V - put);
-      if (stride == n) std::memcpy(h + put * b_row, vert + put * n, rows * b_row);
-      else
-        for (size_t r = put; r < put + rows; ++r) std::memcpy(h + r * b_row, vert + r * stride, b_row);
-      put += rows;
-      if (put < V) send((put * b_row) & ~size_t(15));
-    }
-    for (size_t r = 0; r < 4; ++r) std::memcpy(h + o_head + r * n, head + r * stride, n);
-    send(o_mk);
+    if (stride == n) put(0, vert, b_vert);
+    else
+      for (size_t r = at / b_row; r < V && r * b_row < end; ++r) put(r * b_row, vert + r * stride, b_row);
+    for (size_t r = 0; r < 4; ++r) put(o_head + r * n, head + r * stride, n);
+    slot_tag[slot] = at + STAGE_SLOTS * HOST_CHUNK < o_mk ? next_tag(e) : 0u;   // (the last ones are not waited for)
+    copy(k_copy<false>, d + at, hd + slot * HOST_CHUNK, end - at, FLAG_SLOT + slot, slot_tag[slot]);
     HIP_TRY(e, hipGetLastError());
   }
   rpeg_plan_soa_t soa{(const int16_t*)d, d + o_head, n};
@@ -3486,6 +3499,7 @@ static int eval_host_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* p
   // the results in one piece, or, where that is worth a launch each, one after the other: the host copies one to the caller while
   // the next crosses the bus.  A piece that nobody waits for is not sent.
   struct Part { size_t at, bytes; void* to; };
+  uint8_t *const h_out = h + b_slots, *const hd_out = hd + b_slots;   // (of the results, which begin at o_mk)
   const Part part[5] = {{o_mk, b_f64, makespan}, {o_pk, b_f64, peak}, {o_sc, b_f64, score}, {o_ms, mass ? b_f64 * RPEG_MAX_V : 0, mass}, {o_mask, n, mask}};
   auto wanted = [&](int k) { return part[k].to && part[k].bytes; };
   int last = 4;
@@ -3498,10 +3512,10 @@ static int eval_host_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* p
   const bool at_once = total - o_mk <= HOST_CHUNK;
   uint32_t tag[5] = {};
   if (at_once) {
-    copy(hd + o_mk, d + o_mk, total - o_mk, FLAG_COPY, tag[0] = next_tag(e));
+    copy(k_copy<true>, hd_out, d + o_mk, total - o_mk, FLAG_COPY, tag[0] = next_tag(e));
   } else {
     for (int k = 0; k < 5; ++k)
-      if (wanted(k)) copy(hd + part[k].at, d + part[k].at, part[k].bytes, FLAG_COPY + k, tag[k] = next_tag(e));
+      if (wanted(k)) copy(k_copy<true>, hd_out + (part[k].at - o_mk), d + part[k].at, part[k].bytes, FLAG_COPY + k, tag[k] = next_tag(e));
   }
   HIP_TRY(e, hipGetLastError());
   for (int k = 0; k < 5; ++k) {
@@ -3509,7 +3523,7 @@ static int eval_host_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* p
     const uint32_t from = at_once ? 0u : (uint32_t)k;
     if (int rc = wait_tag(e, s, tag[from], FLAG_COPY + from)) return rc;
     at_rest.waited = at_once || k == last;   // (a call's pieces follow each other)
-    std::memcpy(part[k].to, h + part[k].at, part[k].bytes);
+    std::memcpy(part[k].to, h_out + (part[k].at - o_mk), part[k].bytes);
   }
   return 0;
 }

@@ -1,5 +1,5 @@
 """Host-pointer batches that are staged in chunks through pinned memory: sizes at the edges of a chunk (512 KiB, of fields and of
-results) and of its sixteen-byte copies, odd ones, rows apart from each other by more than the batch, with and without masses,
+results) and of its sixteen-byte copies, several rounds of the four pinned chunks, odd ones, rows apart from each other by more than the batch, with and without masses,
 larger and smaller calls in turn on one engine, calls that want some or none of the results between them; outputs of the host build
 bit for bit."""
 
@@ -15,7 +15,7 @@ from tests.test_class_pool import same_bits
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("c,sizes", [(4, (1025, 26214, 26215, 1031)), (2, (2049, 20971, 20973, 5243)), (1, (8738, 1027))])
+@pytest.mark.parametrize("c,sizes", [(4, (1025, 26214, 26215, 1031)), (2, (2049, 20971, 20973, 5243)), (1, (8738, 1027)), (4, (131071, 34953, 32768)), (3, (60001, 17478))])
 def test_staged_batches(c, sizes):
     from rpeg_amd.engine.runtime import Engine
     cfg, batch = seeded_batch(c, max(sizes))
@@ -45,7 +45,7 @@ def test_staged_batches(c, sizes):
 @pytest.mark.parametrize("n_between", [1500, 30001])      # results in one piece, and one by one
 @pytest.mark.parametrize("wanted", [(), ("makespan",), ("mask",)])
 def test_calls_that_want_few_results_or_none(n_between, wanted):
-    """The pinned mirror is at rest when a call returns: the plans of the next one go there at once."""
+    """The pinned chunks are at rest when a call returns: the plans of the next one go there at once."""
     from rpeg_amd.engine.runtime import Engine
     cfg, batch = seeded_batch(2, 30001)
     want = CpuPort(cfg.problem).eval(batch, flags=abi.GATE_STALE, threads=16)
