@@ -212,9 +212,10 @@ int rpeg_eval_batch_mass(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* pl
    is what one step of the reference's search hands to its evaluation pool: a handful of candidate
    configurations held by the host (RPEG/search/optimizer.py:793-798, the `map` over `_eval_worker`; and
    every single call of evaluate / evaluate_cached, RPEG/search/evaluate.py:235-403).  For a batch of at most
-   32 plans per compute unit the host computes the lowering class of each plan itself and the call is one
+   1,024 plans the host computes the lowering class of each plan itself and the call is one
    launch (one plan per wavefront) that reads the plans from pinned host memory, leaves the results there and
-   flags them; larger batches are staged through device memory and take the path of rpeg_eval_batch.  Returns when
+   flags them; larger batches are staged through device memory (by way of a few pinned pieces that the engine keeps)
+   and take the path of rpeg_eval_batch.  Returns when
    the results are in place. */
 int rpeg_eval_host(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, uint32_t flags, double* makespan,
                    double* peak, double* score, uint8_t* mask, double* mass, void* stream);
@@ -452,8 +453,8 @@ int rpeg_sa_propose(rpeg_engine_t* e, const rpeg_sa_params_t* prm, int32_t what,
    [5] plans per wavefront with LDS-resident state (0: state in the HBM workspace; 1: one plan per
    wavefront), [6] plans of a large batch that ran one per wavefront beside the main kernel (included
    in [2]), [7] wave tasks of the few-lanes-per-plan kernel (included in [2]), [8] plans that the call BEFORE the last
-   one redid because their ready sets outgrew their kernel's (both calls laid out by the host: a batch that needed no
-   layout leaves the figure as it is), [9] plans of the few-lanes-per-plan kernel, [10], [11], [12] launches of its forms for
+   one redid because their ready sets outgrew their kernel's (of the calls that were laid out, by the host or on the device: a
+   batch that needed no layout leaves the figure as it is), [9] plans of the few-lanes-per-plan kernel, [10], [11], [12] launches of its forms for
    ready sets of up to 8, 16 and 24 entries. */
 int rpeg_engine_stats(const rpeg_engine_t* e, uint64_t* out, int32_t n);
 

@@ -202,10 +202,11 @@ __global__ __launch_bounds__(HAND_BLOCK) void k_hand_counts(uint32_t* __restrict
 // and the per-class plan counts.  Blocks of SIG_BLOCK plans; shard = block mod shards.
 constexpr int SIG_BLOCK = 256, SIG_TABLE = 512;
 constexpr size_t DIRECT_MAX_CLASSES = 32;   // engines of at most this many classes evaluate small batches without a layout,
-constexpr uint64_t KP_RESIDENT_PER_CU = 16; // wavefronts of k_plan that a compute unit holds, by registers
 constexpr uint64_t DIRECT_PER_CU = 8;       // and so does every batch of at most this many plans per compute unit
-// Task counters of a call's evaluation launches (the main kernel's), and the two of k_class_direct: plans of classes not lowered,
-// and the blocks that are done; the blocks of k_copy that are (zero between launches).
+constexpr uint64_t KP_RESIDENT_PER_CU = 16; // wavefronts of k_plan that a compute unit holds, by registers
+// Words of d_queues: the task counter of the main kernel, which k_scatter clears for the launch that follows it; the two of
+// k_class_direct, plans of classes not lowered and blocks that are done, and the blocks of k_copy that are: zero between launches,
+// the block that is done last sees to that.
 constexpr uint32_t N_QUEUES = 4, Q_DIRECT = 1, Q_COPY = 3;
 // Words of h_sigflag: of the counters of a call, of the pieces of the results that k_copy brings (5), of the tasks that k_deal
 // dealt, and of the pieces of plans that k_copy fetched.
@@ -1047,7 +1048,7 @@ struct rpeg_engine_s {
   SlotDesc* d_uni = nullptr;
   uint32_t n_uni[RPEG_MAX_STRUCT] = {0, 0, 0}, max_uni = 0;
   uint32_t* d_order = nullptr;                  // class ids, largest graphs first, then the pool offset of every class (ensure_class_tables)
-  uint32_t* d_queues = nullptr;                 // N_QUEUES task counters, cleared by k_scatter
+  uint32_t* d_queues = nullptr;                 // N_QUEUES counters of blocks and tasks
   uint32_t* d_limit = nullptr;                  // count, then (plan, class offset) pairs: plans to redo without a bound on the ready set
   uint8_t* d_limit_ws = nullptr;                // state of the launch that redoes them
   size_t limit_ws_cap = 0;
@@ -1219,7 +1220,8 @@ static int ensure_pool(rpeg_engine_t* e, hipStream_t s) {
   if (e->n_fresh) {
     for (size_t k = 0; k < e->n_fresh; ++k)
       if (!e->fresh[k].bytes.empty()) HIP_TRY(e, hipMemcpyAsync(e->d_pool + e->fresh[k].off, e->fresh[k].bytes.data(), e->fresh[k].bytes.size(), hipMemcpyHostToDevice, s));
-    // the host buffers are filled again by the next classes: finish the copies first
+    // the host buffers are filled again by the next classes: finish the copies first.  (Waiting for each by itself costs 0.2 ms of a
+    // call with eight of them; side by side, one call of a process now and then spends 6 ms in one of them.)
     HIP_TRY(e, hipStreamSynchronize(s));
     e->n_fresh = 0;
   }
@@ -1836,8 +1838,9 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // offset of its class through the table of the classes lowered so far, k_plan takes the plans in their own order,
   // and the host learns meanwhile whether a plan belonged to a class not lowered yet (then the call goes the
   // long way below and evaluates the batch again).  Two launches; with a fill for the count ahead of them, a copy behind and the
-  // wait for it, us a call / now: 600 DPO plans 55 / 36, 3,000 68 / 50; 900 PPO plans 124 / 105, 2,000 140 / 122; 1,500 GRPO 123 / 105;
-  // 2,000 AC-share 342 / 326.
+  // wait for it, us until the results are there / now: 600 DPO plans 57 / 53, 3,000 70 / 65; 900 PPO plans 126 / 119, 2,000 142 / 136;
+  // 1,500 GRPO 130 / 125; 2,000 AC-share 345 / 341.  (Calls in a row, whose kernels then follow each other without a gap: 55 / 38, 67 /
+  // 51; 123 / 104, 140 / 121; 127 / 108; 341 / 325.)
   // Only for an engine of few classes or a batch that is resident at once with room to spare: with hundreds of
   // classes the plans in their own order make neighbouring wavefronts work on different classes, and k_plan runs
   // half as long again as on the sorted batch, which k_deal makes: 8 us (2,000 PPO plans 122 / 130 us a call, 1,100 DPO plans 45 / 54).
@@ -1940,8 +1943,9 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       ahead = !e->prof_on && e->layout_ahead && side_claim(e);
     }
     // A batch for k_plan whose classes may all be lowered is laid out on the device; the host only waits to hear that they are
-    // (else the call goes on the long way).  us a step, laid out by the host / on the device: PPO 2,500 139 / 132, 4,096 149 / 136,
-    // 13,000 286 / 270; GRPO 9,001 152 / 147; AC-share 6,000 394 / 388.
+    // (else the call goes on the long way).  us a step, laid out by the host / on the device, all launches at once / now, those that
+    // follow when the host has heard: PPO 2,500 139 / 132 / 128, 4,096 149 / 139 / 137, 13,000 286 / 266 / 262; GRPO 9,001 152 / 146 / 143;
+    // AC-share 6,000 394 / 379 / 377.
     const bool deal = round == 0 && shards <= DEAL_SHARDS && plan_rows && plan_fits() && !e->prof_on && ncls && e->d_pool && e->d_pool_used == e->pool_size;
     if (deal)
       if (int rc = ensure_perm(e, n, n)) return rc;

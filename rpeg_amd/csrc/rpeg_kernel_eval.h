@@ -170,7 +170,8 @@ __device__ inline double ke_slot_duration(const rpeg_problem_t& P, const rpeg_st
 // is read by a load a lane wherever the compiler does not see that: behind a store of the kernel, in a function that is
 // not inlined, and where a lane takes part because a field of its own equals the common one, which may then be read for it.
 // k_prologue's durations / k_peaks, us, with a load a lane and without: 1,048,576 DPO plans 129 / 93 -> 103 / 64, 262,144
-// AC-share plans 310 / 664 -> 239 / 563, the latter beside k_quad; the step 945 -> 875 and 3,968 -> 3,894.)
+// AC-share plans 310 / 664 -> 239 / 563, the latter beside k_quad; the step 945 -> 875 and 3,968 -> 3,894.  k_peaks has been rewritten
+// since: 35 and 172.)
 template <class T>
 __device__ inline const T& ke_common(const T& x) {
   const uint64_t at = (uint64_t)&x;

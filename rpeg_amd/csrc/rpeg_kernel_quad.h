@@ -201,8 +201,9 @@ __device__ inline double kq_more_successors(const ClassView& cv, int i, double b
 // the plan, out to `keep`.
 // Bound: a trip (up to two or four nodes a plan) is some 35 vector instructions and one LDS round trip; records are read two trips
 // ahead, durations one.  A rank takes eight bytes a node, more than all a plan keeps of it later, but is read back only by the
-// few levels below: in LDS lie rows that nodes share (RankRec), and the ranks go through memory (240 MB for 1,048,576 DPO plans, most of
-// it never out of the L2) to the comparison of positions, which takes them a part of the plans at a time; where the launches'
+// few levels below: in LDS lie rows that nodes share (RankRec), and the ranks go through memory to the comparison of positions, which takes
+// them a part of the plans at a time (1,048,576 DPO plans, 240 MB of ranks: by the counters all of them are written out and most read
+// back from beyond the L2, the launch moves 779 MB, before 358; 262,144 AC-share plans, all schedulers, 1,555, before 845); where the launches'
 // wavefronts find room together with all of their ranks those stay in LDS (kq_ranks_in_lds).  Before, the pass ran once for every part,
 // with two to four times the lanes for levels of two or three nodes, and a part's ranks all lay in LDS.  us a step, before / now:
 // 262,144 AC-share plans 4,196 / 3,953, 131,072 2,720 / 2,572, 65,536 1,550 / 1,430; 131,072 PPO 989 / 935, GRPO 490 / 442; 65,536

@@ -1,5 +1,6 @@
 """Batches of a wavefront per plan (more than four and at most 52 plans per compute unit, with the edges of that range and of the
-blocks of 64 and 256 plans), dealt to their tasks on the device, and of four wavefronts, with durations ahead of the former: outputs and masks of the host build bit for bit, plans that break a rule and
+blocks of 64 and 256 plans), in the plans' own order up to eight per compute unit and for few classes, else dealt to their tasks on the
+device, with durations ahead of those of more than sixteen and of those dealt, and of four wavefronts: outputs and masks of the host build bit for bit, plans that break a rule and
 plans of both structures among them, critical-chain masses too, on an engine that has met none, some and all of the classes."""
 
 import numpy as np
