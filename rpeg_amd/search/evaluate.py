@@ -15,7 +15,8 @@ integer part of `is_valid`) are host code as in the reference.
 from __future__ import annotations
 
 import weakref
-from dataclasses import dataclass
+from array import array
+from dataclasses import dataclass, replace
 from typing import Dict, List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -23,7 +24,7 @@ import numpy as np
 from ..core.types import (Allocation, DeviceSpace, RPEG_TRANSFER_RESOURCE_POLICY, TransferResourcePolicy,
                           packing_geometry, rectangular_node_layouts)
 from ..engine import abi
-from ..engine.problem import STRUCTURES, EvalProblem, PlanBatch
+from ..engine.problem import FIELDS_PER_VERTEX, STRUCTURES, EvalProblem, PlanBatch
 from ..ir.plan import ExecutionPlan
 from ..ir.rpeg import RPEG
 from ..model.hardware import Hardware
@@ -33,7 +34,7 @@ from ..model.workload import Workload
 from ..passes.lower import ExecEdge, ExecNode, ExecNodeType, ExecutableRPEG, graph_nodes, lower   # noqa: F401  (re-exported)
 from ..schedule.scheduler import trace_from
 from ..schedule.trace import Trace   # noqa: F401  (re-exported: the reference's evaluate module names it)
-from .cache import EvalCache, config_hash
+from .cache import EvalCache, by_vertex, config_hash
 
 _OOM_BETA = 40.0
 ABLATION_HARD_OOM = False
@@ -106,8 +107,6 @@ def _engine_for(rpeg: RPEG, suite: ModelSuite, workload: Workload, hw: Hardware,
     trainable models when that is given and differs from the template's), `more_structures` follow.
     `transfer_policy` (a TransferResourcePolicy, None = the default) is part of the problem: it decides
     which allocations the lowered transfers reserve."""
-    from dataclasses import replace
-    from ..engine.runtime import Engine
     st = _structure_of(rpeg)
     if memory_trainable is not None and frozenset(memory_trainable) != frozenset(st.tau_models):
         st = replace(st, memory_trainable=frozenset(memory_trainable))
@@ -116,6 +115,8 @@ def _engine_for(rpeg: RPEG, suite: ModelSuite, workload: Workload, hw: Hardware,
     rest = (tuple(sorted((m.value, s) for m, s in suite.specs.items())), workload, hw, space, K_eval, policy,
             transfer_policy)
     key = (tuple((s.name, s.memory_trainable) for s in structures),) + rest
+    if _engines and key == next(reversed(_engines)):     # (a comparison: a hash goes through every number of the problem)
+        return next(reversed(_engines.values())), st
     alias = ((st.name, st.memory_trainable), "first") + rest
     hit = key if key in _engines else alias if not more_structures and alias in _engines else None
     if hit is not None:
@@ -123,6 +124,7 @@ def _engine_for(rpeg: RPEG, suite: ModelSuite, workload: Workload, hw: Hardware,
         eng = _engines.pop(hit)
         _engines[hit] = eng          # most recently used last
         return eng, st
+    from ..engine.runtime import Engine
     problem = EvalProblem(structures=structures, suite=suite, workload=workload, hw=hw, device_space=space,
                           K_eval=K_eval, memory_policy=policy, transfer_resource_policy=transfer_policy)
     eng = _engines[key] = Engine(problem)
@@ -186,16 +188,38 @@ def _check_supported(config: Configuration):
 
 
 def _pack(configs: Sequence[Configuration], st, workload: Workload) -> PlanBatch:
-    batch = PlanBatch.empty(len(configs))
     split = 1 if workload.gen_quantiles else 0
-    for i, cfg in enumerate(configs):
-        for v in cfg.rpeg.vertices:  # a missing vertex raises KeyError as lower() does (lower.py:447-451)
-            cfg.plan.sigma[v], cfg.plan.pi[v]
-        taus = [int(cfg.rpeg.tau[m]) for m in st.tau_models]
-        plan = cfg.plan
-        if any(v not in plan.mb for v in cfg.rpeg.vertices):
-            raise KeyError("plan.mb misses a template vertex")
-        batch.set_plan(i, 0, split, taus, cfg.rpeg, plan)
+    numbers, head, width = [], [], 0
+    for cfg in configs:
+        plan, verts = cfg.plan, tuple(cfg.rpeg.vertices)
+        parts = by_vertex(verts, plan)
+        if parts is None:
+            for v in verts:  # a missing vertex raises KeyError as lower() does (lower.py:447-451)
+                plan.sigma[v], plan.pi[v]
+            if any(v not in plan.mb for v in verts):
+                raise KeyError("plan.mb misses a template vertex")
+            parts = [(plan.sigma[v], plan.pi[v], plan.mb[v]) for v in verts]
+        at = len(numbers)
+        for a, p, m in parts:
+            numbers += (*p, m, *a.origin, *a.extent)
+            at += FIELDS_PER_VERTEX
+            if len(numbers) != at:
+                raise ValueError("a strategy has three degrees, an allocation three coordinates")
+        tau = cfg.rpeg.tau
+        head.append((0, split, *[int(tau[m]) for m in st.tau_models]))
+        width = max(width, len(verts) * FIELDS_PER_VERTEX)
+    n = len(configs)
+    batch = PlanBatch.empty(n)
+    if len(numbers) == n * width:
+        try:      # (whole numbers, as they come)
+            rows = np.frombuffer(array("h", numbers), np.int16)
+        except TypeError:
+            rows = np.array(numbers).astype(np.int16)
+        batch.vert[:width] = rows.reshape(n, width).T
+    else:         # (templates of several sizes)
+        for i, cfg in enumerate(configs):
+            batch.set_plan(i, 0, split, (), cfg.rpeg, cfg.plan)
+    batch.head[:len(head[0])] = np.array(head, np.uint8).T
     return batch
 
 
@@ -290,10 +314,9 @@ def is_valid(config: Configuration, suite: ModelSuite, workload: Workload, mem_m
     return bool(mask & abi.MASK_VALID) and bool(mask & abi.MASK_STALE_OK) and bool(mask & abi.MASK_MEM_OK)
 
 
-def evaluation_cache_key(config: Configuration, memory_policy: MemoryPolicy = MemoryPolicy()) -> str:
-    """Same key text as evaluate.py:301-326."""
+def _key_ending(config: Configuration, memory_policy: MemoryPolicy) -> str:
     pol = config.transfer_resource_policy or RPEG_TRANSFER_RESOURCE_POLICY
-    return (f"{config_hash(config.rpeg, config.plan)}:mem:"
+    return (f":mem:"
             f"fusion={int(config.intra_stage_fusion)}:"
             f"transfer={','.join(pol.to_dict().values())}:"
             f"{memory_policy.optimizer_stage}:"
@@ -302,6 +325,11 @@ def evaluation_cache_key(config: Configuration, memory_policy: MemoryPolicy = Me
             f"{memory_policy.worker_overhead_bytes:.12g}:"
             f"activation_cache={memory_policy.semantic_activation_cache_bytes:.12g}:"
             f"groups={memory_policy.max_worker_groups_per_gpu}")
+
+
+def evaluation_cache_key(config: Configuration, memory_policy: MemoryPolicy = MemoryPolicy()) -> str:
+    """Same key text as evaluate.py:301-326."""
+    return config_hash(config.rpeg, config.plan) + _key_ending(config, memory_policy)
 
 
 _no_graph = weakref.ref(Trace({}, {}))     # (of an object that is gone)

@@ -25,9 +25,9 @@ from ..model.hardware import Hardware
 from ..model.memory import MemoryPolicy
 from ..model.models import ModelSuite
 from ..model.workload import Workload
-from .cache import EvalCache
+from .cache import EvalCache, key_text
 from .evaluate import (Configuration, _check_supported, _engine_for, _structure_of, evaluate_batch, evaluate_cached,
-                       evaluation_cache_key)
+                       _key_ending, evaluation_cache_key)
 from .inter_model import DEFAULT_T_CAND, _iter_staleness as _staleness_assignments
 from .moves import build_candidate_directory, directory_arrays
 
@@ -319,20 +319,20 @@ def _carry_into(cache: EvalCache, problem, families, res, base_tau, suite, workl
     optimize() would have left there: score and feasibility as stored, and in the trace's place the
     utilisation (the one number of a trace that polish reads) when the utilisation objective is on."""
     templates = {}
-    for row, var, score, feasible, util in zip(res["eval_log"], res["eval_log_variant"], res["eval_log_score"],
-                                               res["eval_log_feasible"], res["eval_log_util"]):
-        var = int(var)
+    for row, var, score, feasible, util in zip(res["eval_log"].tolist(), res["eval_log_variant"].tolist(), res["eval_log_score"].tolist(),
+                                               res["eval_log_feasible"].tolist(), res["eval_log_util"].tolist()):
         if var not in templates:
             f, k = (0, None) if var == 255 else (var // 8, var % 8)
             st = problem.structures[families[f][0].structure]
             taus = list(base_tau) if k is None else [int(families[f][0].tau[k][i]) for i in range(len(st.tau_models))]
-            templates[var] = st.build(suite, workload, tau={m: taus[i] for i, m in enumerate(st.tau_models)})
-        rpeg = templates[var]
-        config = Configuration(rpeg, row_plan(rpeg, row), base_config.device_space, intra_stage_fusion=False,
-                               transfer_resource_policy=base_config.transfer_resource_policy)
-        h = evaluation_cache_key(config, policy)
+            rpeg = st.build(suite, workload, tau={m: taus[i] for i, m in enumerate(st.tau_models)})
+            ending = _key_ending(Configuration(rpeg, None, base_config.device_space, intra_stage_fusion=False,
+                                               transfer_resource_policy=base_config.transfer_resource_policy), policy)
+            templates[var] = key_text(rpeg), ending
+        text, ending = templates[var]
+        h = text.of_row(row) + ending
         if h not in cache:
-            cache.put(h, float(score), _Utilization(float(util)) if with_util else None, bool(feasible))
+            cache.put(h, score, _Utilization(util) if with_util else None, feasible)
 
 
 def configuration_of(problem: EvalProblem, families, res, base_tau, suite, workload, base_config) -> Configuration:

@@ -1,0 +1,74 @@
+"""The text of a plan's cache key put together from its row of numbers, and plans packed many at a time, against the plain forms."""
+
+import dataclasses
+
+import numpy as np
+import pytest
+
+from rpeg_amd import configs
+from rpeg_amd.engine.problem import PlanBatch
+from rpeg_amd.search import candidates
+from rpeg_amd.search.cache import _config_hash_plain, config_hash, key_text
+from rpeg_amd.search.evaluate import Configuration, _pack, _structure_of
+from rpeg_amd.search.optimizer import plan_row
+
+
+def seeded(workload, structure, n):
+    cfg = configs.config(workload)
+    p = dataclasses.replace(cfg.problem, structures=cfg.problem.structures[structure:structure + 1])
+    batch = candidates.generate(p, n, cfg.tau_choices, seed=3, tag=workload)
+    return p, [batch.configuration(p, i)[:2] for i in range(n)]
+
+
+CASES = [(1, 0), (2, 0), (3, 0), (3, 1), (4, 0), (5, 0)]
+
+
+@pytest.mark.parametrize("workload,structure", CASES)
+def test_key_of_a_row_is_the_key_of_its_plan(workload, structure):
+    for rpeg, plan in seeded(workload, structure, 20)[1]:
+        want = _config_hash_plain(rpeg, plan)
+        assert config_hash(rpeg, plan) == want
+        assert key_text(rpeg).of_row(plan_row(rpeg, plan).tolist()) == want
+
+
+def test_plans_that_are_no_row_of_whole_numbers():
+    _, [(rpeg, plan)] = seeded(1, 0, 1)
+    v, w = rpeg.vertices[:2]
+    other = dataclasses.replace(v, id="x%d")
+    forms = [dataclasses.replace(plan, mb={**plan.mb, v: True}), dataclasses.replace(plan, mb={**plan.mb, v: 2.0}),
+             dataclasses.replace(plan, pi={**plan.pi, v: (1, 2)}), dataclasses.replace(plan, pi={**plan.pi, v: [2, 1, 1]}),
+             dataclasses.replace(plan, mb={x: m for x, m in plan.mb.items() if x != w}),
+             dataclasses.replace(plan, sigma={**plan.sigma, other: plan.sigma[v]}),
+             dataclasses.replace(plan, mb={**{x: m for x, m in plan.mb.items() if x != w}, other: 1}),
+             dataclasses.replace(plan, sigma=dict(reversed(plan.sigma.items())))]
+    for p in forms:
+        assert config_hash(rpeg, p) == _config_hash_plain(rpeg, p)
+    with pytest.raises(TypeError):      # (as json refuses it)
+        config_hash(rpeg, dataclasses.replace(plan, mb={**plan.mb, v: np.int64(2)}))
+    odd = dataclasses.replace(rpeg, vertices=(other,) + rpeg.vertices[1:])      # a name with a format character
+    move = lambda d: {other if x == v else x: y for x, y in d.items()}  # noqa: E731
+    p = dataclasses.replace(plan, sigma=move(plan.sigma), pi=move(plan.pi), mb=move(plan.mb))
+    assert config_hash(odd, p) == _config_hash_plain(odd, p)
+
+
+@pytest.mark.parametrize("workload,structure", CASES)
+def test_packed_plans_are_the_plans_one_by_one(workload, structure):
+    problem, plans = seeded(workload, structure, 9)
+    st = _structure_of(plans[0][0])
+    got = _pack([Configuration(r, p, problem.device_space) for r, p in plans], st, problem.workload)
+    want = PlanBatch.empty(len(plans))
+    for i, (r, p) in enumerate(plans):
+        want.set_plan(i, 0, 1 if problem.workload.gen_quantiles else 0, [int(r.tau[m]) for m in st.tau_models], r, p)
+    assert np.array_equal(got.vert, want.vert) and np.array_equal(got.head, want.head)
+    assert got.vert.dtype == want.vert.dtype and got.head.dtype == want.head.dtype and got.vert.flags.c_contiguous
+
+
+def test_plans_that_cannot_be_packed():
+    problem, [(rpeg, plan)] = seeded(5, 0, 1)
+    st, v = _structure_of(rpeg), rpeg.vertices[3]
+    without = lambda d: {x: y for x, y in d.items() if x != v}  # noqa: E731
+    for change, error in (({"sigma": without(plan.sigma)}, KeyError), ({"pi": without(plan.pi)}, KeyError),
+                          ({"mb": without(plan.mb)}, KeyError), ({"pi": {**plan.pi, v: (1, 1)}}, ValueError),
+                          ({"mb": {**plan.mb, v: 1 << 15}}, OverflowError)):
+        with pytest.raises(error):
+            _pack([Configuration(rpeg, dataclasses.replace(plan, **change), problem.device_space)], st, problem.workload)
