@@ -412,7 +412,7 @@ __global__ __launch_bounds__(COPY_BLOCK) void k_copy(uint4* __restrict__ to, con
 // next call; start[class * shards + shard]: the first task of the class's plans of that shard.  Tasks without a plan are KP_SKIP.
 // Before that the last wavefront hands over what the host goes on with, under host_flag[FLAG_COUNTS]: host_count, behind the place of
 // the totals, the plans of classes not lowered yet, and from there on as k_hand_counts; host_need: likewise, where plans were redone
-// since the last hand-over (whose count k_deal_plans clears).  With plans of such classes nothing is dealt; the launches that deal and
+// since the last hand-over (whose count k_prologue clears).  With plans of such classes nothing is dealt; the launches that deal and
 // evaluate follow when the host has heard that there are none, which is before this one ends.  (Sent out ahead, to find nothing to do
 // where there are, they kept a first pass over new classes waiting: 4,096 PPO plans, 61 classes to lower, 915 us, now 876; 6,000
 // AC-share, 78 classes, 1,180 / 1,144; laid out by the host 899 and 1,137.)  Behind all these words, under host_flag[FLAG_DEALT]: the
@@ -515,25 +515,21 @@ __global__ __launch_bounds__(HAND_BLOCK) void k_deal(uint32_t* __restrict__ coun
     __hip_atomic_store(host_flag + FLAG_DEALT, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
-__global__ void k_deal_plans(uint32_t n, const uint32_t* __restrict__ cid, const uint32_t* __restrict__ kidx, const uint32_t* __restrict__ start,
-                             uint32_t shards, const uint32_t* __restrict__ coff, uint32_t* __restrict__ perm, uint32_t* __restrict__ task_cls,
-                             uint32_t* __restrict__ limit) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) limit[0] = 0u;   // (as k_scatter)
-  if (i >= n) return;
-  const uint32_t c = cid[i];
-  if (c >= CID_UNKNOWN) return;
-  const uint32_t task = start[c * shards + ((i / SIG_BLOCK) & (shards - 1u))] + kidx[i];
-  perm[task] = i;
-  task_cls[task] = coff[c];
-}
-
 // The prologue launches (rpeg_kernel_prologue.h), a thread per plan in the caller's order.  The structure decides
 // which tables a plan reads; it is made uniform (one pass per distinct structure among the plans of the wavefront) so
 // that those reads are scalar loads and the walk through the slot universe is one path.
 __global__ __launch_bounds__(WAVE) void k_prologue(const PrologueLaunch L) {
   const uint64_t i = (uint64_t)blockIdx.x * WAVE + threadIdx.x;
-  const bool active = i < L.n && L.cid[i] != KPRO_INVALID;
+  const uint32_t c = i < L.n ? L.cid[i] : KPRO_INVALID;
+  const bool active = c != KPRO_INVALID;
+  if (L.deal.start && blockIdx.y == 0 && *L.deal.not_lowered == 0u) {   // uniform
+    if (i == 0) L.deal.limit[0] = 0u;   // (as k_scatter)
+    if (c < CID_UNKNOWN) {
+      const uint32_t task = L.deal.start[c * L.deal.shards + ((uint32_t)(i / SIG_BLOCK) & (L.deal.shards - 1u))] + L.deal.kidx[i];
+      L.deal.perm[task] = (uint32_t)i;
+      L.deal.task_cls[task] = L.deal.coff[c];
+    }
+  }
   int su = 0, split = 0;
   if (active) { su = L.head[0 * L.stride + i]; split = L.head[1 * L.stride + i]; }
   unsigned long long todo = __ballot(active);
@@ -1434,6 +1430,7 @@ static PrologueLaunch prologue_launch(const rpeg_engine_t* e, uint64_t n, const 
   G.aux_pen = e->d_aux_pen; G.aux_mask = e->d_aux_mask;
   G.peak = nullptr;
   G.row_begin = G.row_end = 0;
+  G.deal = DealtTasks{};
   return G;
 }
 // Wavefronts that share the rows of 64 plans: as many as fill the chip once.  A row is a chain of a few loads, so the launch takes
@@ -1442,9 +1439,12 @@ static uint32_t prologue_parts(const rpeg_engine_t* e, const PrologueLaunch& G, 
   const uint64_t blocks = (n + WAVE - 1) / WAVE;
   return std::min(G.row_end - G.row_begin, std::max<uint32_t>(KPRO_PARTS, (uint32_t)((uint64_t)e->n_cu * 16u / blocks)));
 }
-// The durations alone, for k_plan.  cid: KPRO_INVALID where a plan is not to be evaluated.
-static void launch_durations(const rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, const uint32_t* cid, hipStream_t s) {
+// The durations alone, for k_plan, and where k_deal has laid the batch out its tasks: a launch of
+// their own took 3 us, and k_plan, which goes out when the host has heard from k_deal, was one launch further off (us a step, with it / without:
+// 4,096 PPO plans 139.2 / 136.8, 9,001 GRPO plans in host memory 206.3 / 203.2).  cid: KPRO_INVALID where a plan is not to be evaluated.
+static void launch_durations(const rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* plans, const uint32_t* cid, hipStream_t s, const DealtTasks& deal = {}) {
   PrologueLaunch G = prologue_launch(e, n, plans, cid);
+  G.deal = deal;
   G.row_end = e->max_uni;
   hipLaunchKernelGGL(k_prologue, dim3((unsigned)((n + WAVE - 1) / WAVE), prologue_parts(e, G, n)), dim3(WAVE), 0, s, G);
 }
@@ -1981,7 +1981,8 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       if (!own_prologue && !ahead)
         if (int rc = launch_prologue(true)) return rc;
       if (plan_rows) {
-        launch_durations(e, n, plans, e->d_cid, s);
+        launch_durations(e, n, plans, e->d_cid, s,
+                         deal ? DealtTasks{start, e->d_kidx, e->d_order + ncls, e->d_ccount + (size_t)ncls * shards, shards, e->d_perm, e->d_cls, e->d_limit} : DealtTasks{});
         HIP_TRY(e, hipGetLastError());
       }
       t_counts = std::chrono::steady_clock::now();
@@ -1998,8 +1999,6 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
       if (read_stat) std::copy_n(e->h_tot + e->tot_words() + e->ccap, ncls, e->cls_pops16.begin());
     }
     if (deal && e->h_tot[ncls] == 0) {
-      hipLaunchKernelGGL(k_deal_plans, dim3(nblk), dim3(blk), 0, s, (uint32_t)n, e->d_cid, e->d_kidx, start, shards, e->d_order + ncls, e->d_perm,
-                         e->d_cls, e->d_limit);
       EvalLaunch L = plan_launch(e, n, plans, flags, makespan, peak, score, mask, mass);
       L.perm = e->d_perm; L.wave_cls = e->d_cls;
       L.dur = e->d_dur; L.dur_stride = e->cap_n;

@@ -34,6 +34,14 @@ namespace rpeg {
 constexpr int KPRO_PARTS = 6;                    // wavefronts that share the rows of a block of 64 plans, at least
 constexpr uint32_t KPRO_INVALID = 0xFFFFFFFFu;   // class id of a plan that breaks an integer rule: not evaluated
 
+// The tasks of a batch of a wavefront per plan: start (or null), [class * shards + shard], the first task of the class's plans of that
+// shard; what a plan's own is, its class's blob and the plan go into the task.  Where *not_lowered there are none yet.
+struct DealtTasks {
+  const uint32_t *start, *kidx, *coff, *not_lowered;
+  uint32_t shards;
+  uint32_t *perm, *task_cls, *limit;
+};
+
 struct PrologueLaunch {
   const rpeg_problem_t* P;
   const int16_t* vert;         // the caller's plan tensors
@@ -53,6 +61,7 @@ struct PrologueLaunch {
   double* aux_pen;
   uint8_t* aux_mask;
   double* peak;                // or null
+  DealtTasks deal;             // beside durations for k_plan
 };
 
 #if defined(__HIPCC__)
