@@ -5,7 +5,7 @@
 //
 //   e     true start time: the larger of the node's key and the availability of the devices it reserves, raised at every
 //         dispatch that reserves one of them
-//   key   the key the reference's heap holds for it, where its position is shared (below); infinity elsewhere
+//   key   the key the reference's heap holds for it, where its position is shared (below); KQ_NO_TIME elsewhere
 //   word  position << 20 | tie
 //   meta  node id | duration slot | reserved vertices | vertices whose allocations overlap those | register slot
 //
@@ -51,6 +51,9 @@ namespace rpeg {
 
 constexpr uint32_t KQ_TIE_BITS = 20, KQ_TIE_MASK = (1u << KQ_TIE_BITS) - 1u;   // (a round takes at most 1 + 24 + 24 ties and four per new entry: 2^15 for 512 nodes)
 constexpr uint32_t KQ_EMPTY = 0xFFFFFFFFu;
+// High word of the times of a slot without an entry, whatever the low one is: larger than any start time that is evaluated here
+// (a plan with a larger one is flagged and redone by the launch that ends the call).
+constexpr uint32_t KQ_NO_TIME = 0x7FEFFFFFu;
 
 // Positions are found for 1 / parts of a wavefront's plans at a time: all at once, or half or a quarter with two lanes a plan, a
 // quarter or an eighth with four.
@@ -91,9 +94,11 @@ __host__ __device__ inline size_t kq_lds_bytes(uint32_t plans, const QuadSize& z
 
 #if defined(__HIPCC__)
 
+// (a permutation within quads reads lanes that are on, throughout: without a value for others the move needs no copy before it and
+// folds into the instruction that uses it)
 template <int CTRL>
 __device__ inline uint32_t kq_dpp(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xF, 0xF, false);
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
 }
 template <int CTRL>
 __device__ inline double kq_dpp(double v) {
@@ -505,11 +510,16 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
 
   KE_STAMP(4);
   // ---- list scheduling (scheduler.py:399-546)
-  const double inf = __builtin_inf();
+  const double no_time = __hiloint2double((int)KQ_NO_TIME, 0);
+  auto no_time_in = [&](mask64 m, double x) {   // (in the lanes of m)
+    return __hiloint2double((int)kp_sel(m, KQ_NO_TIME, (uint32_t)__double2hiint(x)), __double2loint(x));
+  };
+  uint32_t tie_mask;   // (in a register: as a constant it takes an instruction of its own with every use)
+  asm("v_mov_b32 %0, %1" : "=v"(tie_mask) : "s"(KQ_TIE_MASK));
   double ek[SL], sk[SL];
   uint32_t eo[SL], em[SL];
 #pragma unroll
-  for (int u = 0; u < SL; ++u) { ek[u] = inf; sk[u] = inf; eo[u] = KQ_EMPTY; em[u] = 0u; }
+  for (int u = 0; u < SL; ++u) { ek[u] = no_time; sk[u] = no_time; eo[u] = KQ_EMPTY; em[u] = 0u; }
   uint32_t tie = 0, free_slots = (1u << SL) - 1u;
   bool ovf = false;
   int live = 0, longest = 0;   // entries now and at most (one more than there is room for where one was lost)
@@ -533,7 +543,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
   auto file = [&](mask64 take, double key, uint32_t state, uint32_t node, uint32_t type, uint32_t t) {
     const uint32_t first = kp_sel(take, free_slots & (0u - free_slots), 0u), u_free = 31u - (uint32_t)__builtin_clz(first | 1u);
     const uint32_t word = ((state & 0x1FFu) << KQ_TIE_BITS) | t, meta = (node & 0x3FDFFu) | (type << 18) | (u_free << 30) | ((u_free >> 2) << 9);
-    const double heap_key = kp_sel(__ballot((state & 0x200u) != 0u), key, inf);
+    const double heap_key = no_time_in(__ballot((state & 0x200u) == 0u), key);
 #pragma unroll
     for (int u = 0; u < SL; ++u) {
       const mask64 m = __ballot(first == (1u << u));
@@ -568,7 +578,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
   };
   // the entry of word o (of every plan: its own) is pushed back
   auto push_back = [&](uint32_t o) {
-    const uint32_t fresh = (o & ~KQ_TIE_MASK) | tie;
+    const uint32_t fresh = (o & ~tie_mask) | tie;
 #pragma unroll
     for (int u = 0; u < SL; ++u) {
       const mask64 hit = __ballot(eo[u] == o);
@@ -608,7 +618,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
         const mask64 mates = back[u] & __ballot((bit[u] & twice) != 0u), alone = back[u] & ~mates;
         more |= mates;
         sk[u] = kp_sel(alone, ek[u], sk[u]);
-        eo[u] = kp_sel(alone, (eo[u] & ~KQ_TIE_MASK) | tie, eo[u]);
+        eo[u] = kp_sel(alone, (eo[u] & ~tie_mask) | tie, eo[u]);
       }
       ++tie;
       while (more) {
@@ -645,15 +655,15 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
         push_back(kp_sel(act, o, KQ_EMPTY - 1u));
       }
     }
-    const mask64 alive = __ballot(gk < inf);   // (nothing waits: an entry was lost, or a start time is infinite: flagged)
+    const mask64 alive = __ballot(gk < no_time);   // (nothing waits: an entry was lost, or a start time is as good as infinite: flagged)
     lost |= ~alive;
     uint32_t bm = 0;
 #pragma unroll
     for (int u = 0; u < SL; ++u) {   // the dispatched entry leaves its slot
       const mask64 hit = __ballot(eo[u] == bo);
       bm = kp_sel(hit, em[u], bm);
-      ek[u] = kp_sel(hit, inf, ek[u]);
-      sk[u] = kp_sel(hit, inf, sk[u]);
+      ek[u] = no_time_in(hit, ek[u]);
+      sk[u] = no_time_in(hit, sk[u]);
     }
     const mask64 winner = __ballot(own == bo) & alive;
     bm = kp_sel(winner, bm, 0u);
