@@ -7,7 +7,7 @@
 //         dispatch that reserves one of them
 //   key   the key the reference's heap holds for it, where its position is shared (below); KQ_NO_TIME elsewhere
 //   word  position << 20 | tie
-//   meta  node id | duration slot | reserved vertices | vertices whose allocations overlap those | register slot
+//   meta  node id | duration slot | reserved vertices | vertices whose allocations overlap those
 //
 // Order.  The heap's key is (est, comm_prio, topo_idx, -rank, tie) (scheduler.py:427); (comm_prio, topo_idx, -rank) is
 // replaced by the node's position, equal for nodes that agree in all three.  The heap pops stale entries (key < e) in key
@@ -541,8 +541,8 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
   // an entry into the first free slot of this lane, in the lanes of `take` (conditions are kept as masks of the lanes in
   // scalar registers: as booleans the compiler moves them through vector registers).  node: id | its QuadRec from bit 10 on
   auto file = [&](mask64 take, double key, uint32_t state, uint32_t node, uint32_t type, uint32_t t) {
-    const uint32_t first = kp_sel(take, free_slots & (0u - free_slots), 0u), u_free = 31u - (uint32_t)__builtin_clz(first | 1u);
-    const uint32_t word = ((state & 0x1FFu) << KQ_TIE_BITS) | t, meta = (node & 0x3FDFFu) | (type << 18) | (u_free << 30) | ((u_free >> 2) << 9);
+    const uint32_t first = kp_sel(take, free_slots & (0u - free_slots), 0u);
+    const uint32_t word = ((state & 0x1FFu) << KQ_TIE_BITS) | t, meta = (node & 0x3FDFFu) | (type << 18);
     const double heap_key = no_time_in(__ballot((state & 0x200u) == 0u), key);
 #pragma unroll
     for (int u = 0; u < SL; ++u) {
@@ -659,15 +659,15 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
     lost |= ~alive;
     uint32_t bm = 0;
 #pragma unroll
-    for (int u = 0; u < SL; ++u) {   // the dispatched entry leaves its slot
+    for (int u = 0; u < SL; ++u) {   // the dispatched entry leaves its slot (what an emptied slot keeps of one is no other's word)
       const mask64 hit = __ballot(eo[u] == bo);
+      free_slots |= kp_sel(hit, 1u << u, 0u);
       bm = kp_sel(hit, em[u], bm);
       ek[u] = no_time_in(hit, ek[u]);
       sk[u] = no_time_in(hit, sk[u]);
     }
     const mask64 winner = __ballot(own == bo) & alive;
     bm = kp_sel(winner, bm, 0u);
-    free_slots |= kp_sel(winner, 1u << ((bm >> 30) | ((bm >> 7) & 4u)), 0u);
     bm = kq_or<QL>(bm);
     mask64 room = __ballot(free_slots != 0u);
     uint32_t in_plan = (uint32_t)(room >> group_shift) & ((1u << QL) - 1u);
