@@ -629,9 +629,31 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
 #pragma unroll
         for (int u = 0; u < SL; ++u) o = min_u32(o, kp_sel(__ballot(sk[u] == k), eo[u], KQ_EMPTY));
         push_back(kp_sel(more, kq_min<QL>(o), KQ_EMPTY - 1u));   // (no entry has that word)
-        more = 0ull;
+        if constexpr (QL == 2) {   // the last one of every plan needs not be looked for (four lanes a plan, AC-share: 3,472 us a step, with this 3,510)
+          mask64 left[SL], several = 0ull;
+          more = 0ull;
 #pragma unroll
-        for (int u = 0; u < SL; ++u) more |= __ballot(sk[u] < gk);
+          for (int u = 0; u < SL; ++u) {
+            left[u] = __ballot(sk[u] < gk);
+            several |= more & left[u];
+            more |= left[u];
+          }
+          if (!more) break;
+          several |= more & (more >> 1) & quads0;
+          if (several == 0ull) {
+#pragma unroll
+            for (int u = 0; u < SL; ++u) {
+              sk[u] = kp_sel(left[u], ek[u], sk[u]);
+              eo[u] = kp_sel(left[u], (eo[u] & ~tie_mask) | tie, eo[u]);
+            }
+            ++tie;
+            break;
+          }
+        } else {
+          more = 0ull;
+#pragma unroll
+          for (int u = 0; u < SL; ++u) more |= __ballot(sk[u] < gk);
+        }
       }
     }
     uint32_t own = KQ_EMPTY;
