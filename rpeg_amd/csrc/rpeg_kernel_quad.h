@@ -6,7 +6,7 @@
 //   e     true start time: the larger of the node's key and the availability of the devices it reserves, raised at every
 //         dispatch that reserves one of them
 //   key   the key the reference's heap holds for it, where its position is shared (below); KQ_NO_TIME elsewhere
-//   word  position << 20 | tie
+//   word  position << 16 | tie
 //   meta  node id | duration slot | reserved vertices | vertices whose allocations overlap those
 //
 // Order.  The heap's key is (est, comm_prio, topo_idx, -rank, tie) (scheduler.py:427); (comm_prio, topo_idx, -rank) is
@@ -49,7 +49,10 @@
 
 namespace rpeg {
 
-constexpr uint32_t KQ_TIE_BITS = 20, KQ_TIE_MASK = (1u << KQ_TIE_BITS) - 1u;   // (a round takes at most 1 + 24 + 24 ties and four per new entry: 2^15 for 512 nodes)
+// Ties are counted for all plans of a wavefront together: a round takes one for its entries alone in their position, one for each of up to
+// 24 others below the smallest start time and as many at it, and a lane each for successors that became ready, once for every node of
+// every plan at most: 512 x 49 + 64 x 512 < 2^16.
+constexpr uint32_t KQ_TIE_BITS = 16, KQ_TIE_MASK = (1u << KQ_TIE_BITS) - 1u;
 constexpr uint32_t KQ_EMPTY = 0xFFFFFFFFu;
 // High word of the times of a slot without an entry, whatever the low one is: larger than any start time that is evaluated here
 // (a plan with a larger one is flagged and redone by the launch that ends the call).
@@ -116,6 +119,65 @@ __device__ inline double kq_vmin(double a, double b, double c, double d) {
   double r, t;
   asm("v_min_f64 %0, %2, %3\n\tv_min_f64 %1, %4, %5\n\tv_min_f64 %0, %0, %1" : "=&v"(r), "=&v"(t) : "v"(a), "v"(b), "v"(c), "v"(d));
   return r;
+}
+// What changes in some lanes only, mostly for two slots at a time: the lanes of m0, those of m1, then all (a wavefront schedules with
+// all of them on).  A move or a maximum each, where a select takes an instruction for every word and one for what it selects; the masks go
+// to EXEC by scalar instructions, which other wavefronts' vector instructions overlap.  (us a step, selects / moves: 1,048,576 DPO plans
+// 787 / 720, 262,144 AC-share 3,455 / 3,370, 131,072 PPO 838 / 810, GRPO 418 / 402, 65,536 GRPO 304 / 291, 20,011 PPO 297 / 284.)
+// -- the larger of two times
+__device__ inline void kq_raise(mask64 m0, mask64 m1, double& a, double& b, double t) {
+  asm("s_mov_b64 exec, %2\n\tv_max_f64 %0, %0, %4\n\ts_mov_b64 exec, %3\n\tv_max_f64 %1, %1, %4\n\ts_mov_b64 exec, -1"
+      : "+v"(a), "+v"(b) : "s"(m0), "s"(m1), "v"(t));
+}
+__device__ inline void kq_raise(mask64 m0, mask64 m1, mask64 m2, double& a, double& b, double& c, double t) {
+  asm("s_mov_b64 exec, %3\n\tv_max_f64 %0, %0, %6\n\ts_mov_b64 exec, %4\n\tv_max_f64 %1, %1, %6\n\ts_mov_b64 exec, %5\n\tv_max_f64 %2, %2, %6\n\t"
+      "s_mov_b64 exec, -1"
+      : "+v"(a), "+v"(b), "+v"(c) : "s"(m0), "s"(m1), "s"(m2), "v"(t));
+}
+// -- the smallest of some words
+__device__ inline void kq_least(mask64 m0, uint32_t& least, uint32_t o0) {
+  asm("s_mov_b64 exec, %1\n\tv_min_u32 %0, %2, %0\n\ts_mov_b64 exec, -1" : "+v"(least) : "s"(m0), "v"(o0));
+}
+__device__ inline void kq_least(mask64 m0, mask64 m1, uint32_t& least, uint32_t o0, uint32_t o1) {
+  asm("s_mov_b64 exec, %1\n\tv_min_u32 %0, %3, %0\n\ts_mov_b64 exec, %2\n\tv_min_u32 %0, %4, %0\n\ts_mov_b64 exec, -1"
+      : "+v"(least) : "s"(m0), "s"(m1), "v"(o0), "v"(o1));
+}
+// -- bits met so far, and those met twice
+__device__ inline void kq_meet(mask64 m0, mask64 m1, uint32_t& seen, uint32_t& twice, uint32_t bit0, uint32_t bit1) {
+  asm("s_mov_b64 exec, %2\n\tv_and_or_b32 %1, %0, %4, %1\n\tv_or_b32 %0, %4, %0\n\t"
+      "s_mov_b64 exec, %3\n\tv_and_or_b32 %1, %0, %5, %1\n\tv_or_b32 %0, %5, %0\n\t"
+      "s_mov_b64 exec, -1"
+      : "+v"(seen), "+v"(twice) : "s"(m0), "s"(m1), "v"(bit0), "v"(bit1));
+}
+// -- an entry into its slot
+__device__ inline void kq_put(mask64 m0, mask64 m1, double& e0, double& e1, double& s0, double& s1, uint32_t& o0, uint32_t& o1, uint32_t& w0, uint32_t& w1,
+                              double e, double s, uint32_t o, uint32_t w) {
+  asm("s_mov_b64 exec, %8\n\tv_mov_b64 %0, %10\n\tv_mov_b64 %2, %11\n\tv_mov_b32 %4, %12\n\tv_mov_b32 %6, %13\n\t"
+      "s_mov_b64 exec, %9\n\tv_mov_b64 %1, %10\n\tv_mov_b64 %3, %11\n\tv_mov_b32 %5, %12\n\tv_mov_b32 %7, %13\n\t"
+      "s_mov_b64 exec, -1"
+      : "+v"(e0), "+v"(e1), "+v"(s0), "+v"(s1), "+v"(o0), "+v"(o1), "+v"(w0), "+v"(w1) : "s"(m0), "s"(m1), "v"(e), "v"(s), "v"(o), "v"(w));
+}
+// -- the dispatched entry out of it: a slot without times, free, its word in `out`
+template <int U>
+__device__ inline void kq_take(mask64 m0, mask64 m1, double& e0, double& e1, double& s0, double& s1, uint32_t& free_slots, uint32_t& out, uint32_t w0, uint32_t w1,
+                               double none) {
+  asm("s_mov_b64 exec, %6\n\tv_mov_b64 %0, %8\n\tv_mov_b64 %2, %8\n\tv_or_b32 %4, %11, %4\n\tv_mov_b32 %5, %9\n\t"
+      "s_mov_b64 exec, %7\n\tv_mov_b64 %1, %8\n\tv_mov_b64 %3, %8\n\tv_or_b32 %4, %12, %4\n\tv_mov_b32 %5, %10\n\t"
+      "s_mov_b64 exec, -1"
+      : "+v"(e0), "+v"(e1), "+v"(s0), "+v"(s1), "+v"(free_slots), "+v"(out) : "s"(m0), "s"(m1), "s"(none), "v"(w0), "v"(w1), "n"(1 << U), "n"(2 << U));
+}
+// -- push-backs with ties from `tie` on (kq_again) or a word of their own
+__device__ inline void kq_again(mask64 m0, mask64 m1, double& s0, double& s1, uint32_t& o0, uint32_t& o1, double e0, double e1, uint32_t tie_mask, uint32_t tie) {
+  asm("s_mov_b64 exec, %4\n\tv_mov_b64 %0, %6\n\tv_bfi_b32 %2, %8, %9, %2\n\t"
+      "s_mov_b64 exec, %5\n\tv_mov_b64 %1, %7\n\tv_bfi_b32 %3, %8, %9, %3\n\t"
+      "s_mov_b64 exec, -1"
+      : "+v"(s0), "+v"(s1), "+v"(o0), "+v"(o1) : "s"(m0), "s"(m1), "v"(e0), "v"(e1), "v"(tie_mask), "s"(tie));
+}
+__device__ inline void kq_again(mask64 m0, mask64 m1, double& s0, double& s1, uint32_t& o0, uint32_t& o1, double e0, double e1, uint32_t word) {
+  asm("s_mov_b64 exec, %4\n\tv_mov_b64 %0, %6\n\tv_mov_b32 %2, %8\n\t"
+      "s_mov_b64 exec, %5\n\tv_mov_b64 %1, %7\n\tv_mov_b32 %3, %8\n\t"
+      "s_mov_b64 exec, -1"
+      : "+v"(s0), "+v"(s1), "+v"(o0), "+v"(o1) : "s"(m0), "s"(m1), "v"(e0), "v"(e1), "v"(word));
 }
 // reductions over the lanes of a plan (two or four)
 template <int QL>
@@ -487,7 +549,8 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
   }
   for (int t = q; t < n_types; t += QL) {
     const uint32_t bc = cv.type[t], bt = kp_reserved(bc & 0xFFu, bc >> 8, ovl, dpne);
-    g_type[t * RW] = (uint16_t)((bt & 0x3Fu) | (((bt >> 8) & 0x3Fu) << 6));
+    const uint32_t b6 = bt & 0x3Fu;
+    g_type[t * RW] = (uint16_t)(b6 | (((bt >> 8) & 0x3Fu) << 6) | ((b6 ? 31u - (uint32_t)__builtin_clz(b6) : (uint32_t)RPEG_MAX_V) << 12));
   }
   __syncthreads();
   KE_STAMP(2);
@@ -543,15 +606,10 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
   auto file = [&](mask64 take, double key, uint32_t state, uint32_t node, uint32_t type, uint32_t t) {
     const uint32_t first = kp_sel(take, free_slots & (0u - free_slots), 0u);
     const uint32_t word = ((state & 0x1FFu) << KQ_TIE_BITS) | t, meta = (node & 0x3FDFFu) | (type << 18);
-    const double heap_key = no_time_in(__ballot((state & 0x200u) == 0u), key);
+    const double heap_key = no_time_in(__ballot(state < 0x200u), key);
 #pragma unroll
-    for (int u = 0; u < SL; ++u) {
-      const mask64 m = __ballot(first == (1u << u));
-      ek[u] = kp_sel(m, key, ek[u]);
-      sk[u] = kp_sel(m, heap_key, sk[u]);
-      eo[u] = kp_sel(m, word, eo[u]);
-      em[u] = kp_sel(m, meta, em[u]);
-    }
+    for (int u = 0; u < SL; u += 2)
+      kq_put(__ballot(first == (1u << u)), __ballot(first == (2u << u)), ek[u], ek[u + 1], sk[u], sk[u + 1], eo[u], eo[u + 1], em[u], em[u + 1], key, heap_key, word, meta);
     free_slots ^= first;
   };
   {
@@ -568,7 +626,13 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
   double makespan = 0.0;
   uint32_t n_back = 0;
   mask64 lost = 0ull;                             // plans (all four lanes) with an entry that found no room
-  auto min_u32 = [](uint32_t x, uint32_t y) { return x < y ? x : y; };
+  auto least = [&](const mask64 (&m)[SL]) {   // the smallest word of this lane's entries in m
+    uint32_t o = kp_sel(m[0], eo[0], KQ_EMPTY);
+    kq_least(m[1], o, eo[1]);
+#pragma unroll
+    for (int u = 2; u < SL; u += 2) kq_least(m[u], m[u + 1], o, eo[u], eo[u + 1]);
+    return o;
+  };
   auto key_min = [&](const double (&x)[SL]) {
     double k;
     if constexpr (SL == 2) k = kq_vmin(x[0], x[1]);
@@ -580,11 +644,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
   auto push_back = [&](uint32_t o) {
     const uint32_t fresh = (o & ~tie_mask) | tie;
 #pragma unroll
-    for (int u = 0; u < SL; ++u) {
-      const mask64 hit = __ballot(eo[u] == o);
-      sk[u] = kp_sel(hit, ek[u], sk[u]);
-      eo[u] = kp_sel(hit, fresh, eo[u]);
-    }
+    for (int u = 0; u < SL; u += 2) kq_again(__ballot(eo[u] == o), __ballot(eo[u + 1] == o), sk[u], sk[u + 1], eo[u], eo[u + 1], ek[u], ek[u + 1], fresh);
     ++tie;   // (also in a plan that pushed nothing back: only the order of ties is looked at)
   };
   for (int done = 0; done < n; ++done) {
@@ -600,10 +660,10 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
       // positions (by their low five bits) that occur twice among them
       uint32_t bit[SL], seen = 0u, twice = 0u;
 #pragma unroll
-      for (int u = 0; u < SL; ++u) {
-        bit[u] = kp_sel(back[u], 1u << ((eo[u] >> KQ_TIE_BITS) & 31u), 0u);
-        twice |= seen & bit[u];
-        seen |= bit[u];
+      for (int u = 0; u < SL; u += 2) {
+        bit[u] = 1u << ((eo[u] >> KQ_TIE_BITS) & 31u);
+        bit[u + 1] = 1u << ((eo[u + 1] >> KQ_TIE_BITS) & 31u);
+        kq_meet(back[u], back[u + 1], seen, twice, bit[u], bit[u + 1]);
       }
       uint32_t other = kq_dpp<KQ_XOR1>(seen);
       twice |= (seen & other) | kq_dpp<KQ_XOR1>(twice);
@@ -613,22 +673,24 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
         twice |= (seen & other) | kq_dpp<KQ_XOR2>(twice);
       }
       more = 0ull;
+      mask64 alone[SL];
 #pragma unroll
       for (int u = 0; u < SL; ++u) {
-        const mask64 mates = back[u] & __ballot((bit[u] & twice) != 0u), alone = back[u] & ~mates;
+        const mask64 mates = back[u] & __ballot((bit[u] & twice) != 0u);
+        alone[u] = back[u] & ~mates;
         more |= mates;
-        sk[u] = kp_sel(alone, ek[u], sk[u]);
-        eo[u] = kp_sel(alone, (eo[u] & ~tie_mask) | tie, eo[u]);
       }
+#pragma unroll
+      for (int u = 0; u < SL; u += 2) kq_again(alone[u], alone[u + 1], sk[u], sk[u + 1], eo[u], eo[u + 1], ek[u], ek[u + 1], tie_mask, tie);
       ++tie;
       while (more) {
         ++n_back;
         const double k = key_min(sk);
         more = __ballot(k < gk);
-        uint32_t o = KQ_EMPTY;
+        mask64 at_k[SL];
 #pragma unroll
-        for (int u = 0; u < SL; ++u) o = min_u32(o, kp_sel(__ballot(sk[u] == k), eo[u], KQ_EMPTY));
-        push_back(kp_sel(more, kq_min<QL>(o), KQ_EMPTY - 1u));   // (no entry has that word)
+        for (int u = 0; u < SL; ++u) at_k[u] = __ballot(sk[u] == k);
+        push_back(kp_sel(more, kq_min<QL>(least(at_k)), KQ_EMPTY - 1u));   // (no entry has that word)
         if constexpr (QL == 2) {   // the last one of every plan needs not be looked for (four lanes a plan, AC-share: 3,472 us a step, with this 3,510)
           mask64 left[SL], several = 0ull;
           more = 0ull;
@@ -642,10 +704,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
           several |= more & (more >> 1) & quads0;
           if (several == 0ull) {
 #pragma unroll
-            for (int u = 0; u < SL; ++u) {
-              sk[u] = kp_sel(left[u], ek[u], sk[u]);
-              eo[u] = kp_sel(left[u], (eo[u] & ~tie_mask) | tie, eo[u]);
-            }
+            for (int u = 0; u < SL; u += 2) kq_again(left[u], left[u + 1], sk[u], sk[u + 1], eo[u], eo[u + 1], ek[u], ek[u + 1], tie_mask, tie);
             ++tie;
             break;
           }
@@ -656,22 +715,20 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
         }
       }
     }
-    uint32_t own = KQ_EMPTY;
-    mask64 level = 0ull;
+    mask64 at_gk[SL], level = 0ull;
 #pragma unroll
     for (int u = 0; u < SL; ++u) {
-      const mask64 at_gk = __ballot(ek[u] == gk);
-      own = min_u32(own, kp_sel(at_gk, eo[u], KQ_EMPTY));
-      level |= __ballot(sk[u] == gk) & ~at_gk;
+      at_gk[u] = __ballot(ek[u] == gk);
+      level |= __ballot(sk[u] == gk) & ~at_gk[u];
     }
-    const uint32_t bo = kq_min<QL>(own);
+    uint32_t bo = kq_min<QL>(least(at_gk));
     // push-backs of entries with that key that come before the one to dispatch
     if (__builtin_expect(level != 0ull, 0)) {
       for (;;) {
-        uint32_t o = KQ_EMPTY;
+        mask64 stale[SL];
 #pragma unroll
-        for (int u = 0; u < SL; ++u) o = min_u32(o, kp_sel(__ballot(sk[u] == gk) & __ballot(ek[u] > gk), eo[u], KQ_EMPTY));
-        o = kq_min<QL>(o);
+        for (int u = 0; u < SL; ++u) stale[u] = __ballot(sk[u] == gk) & __ballot(ek[u] > gk);
+        const uint32_t o = kq_min<QL>(least(stale));
         const mask64 act = __ballot(o < bo);
         if (!act) break;
         push_back(kp_sel(act, o, KQ_EMPTY - 1u));
@@ -679,17 +736,15 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
     }
     const mask64 alive = __ballot(gk < no_time);   // (nothing waits: an entry was lost, or a start time is as good as infinite: flagged)
     lost |= ~alive;
+    bo = kp_sel(alive, bo, KQ_EMPTY - 1u);
     uint32_t bm = 0;
 #pragma unroll
-    for (int u = 0; u < SL; ++u) {   // the dispatched entry leaves its slot (what an emptied slot keeps of one is no other's word)
-      const mask64 hit = __ballot(eo[u] == bo);
-      free_slots |= kp_sel(hit, 1u << u, 0u);
-      bm = kp_sel(hit, em[u], bm);
-      ek[u] = no_time_in(hit, ek[u]);
-      sk[u] = no_time_in(hit, sk[u]);
+    for (int u = 0; u < SL; u += 2) {   // the dispatched entry leaves its slot (what an emptied slot keeps of one is no other's word)
+      const mask64 hit0 = __ballot(eo[u] == bo), hit1 = __ballot(eo[u + 1] == bo);
+      if (u == 0) kq_take<0>(hit0, hit1, ek[0], ek[1], sk[0], sk[1], free_slots, bm, em[0], em[1], no_time);
+      if constexpr (SL > 2) if (u == 2) kq_take<2>(hit0, hit1, ek[2], ek[3], sk[2], sk[3], free_slots, bm, em[2], em[3], no_time);
+      if constexpr (SL > 4) if (u == 4) kq_take<4>(hit0, hit1, ek[4], ek[5], sk[4], sk[5], free_slots, bm, em[4], em[5], no_time);
     }
-    const mask64 winner = __ballot(own == bo) & alive;
-    bm = kp_sel(winner, bm, 0u);
     bm = kq_or<QL>(bm);
     mask64 room = __ballot(free_slots != 0u);
     uint32_t in_plan = (uint32_t)(room >> group_shift) & ((1u << QL) - 1u);
@@ -705,23 +760,27 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
       }
     }
     makespan = kp_vmax(makespan, fin);
+    auto reserved = [&](int k) { return __ballot((bm & lf_bit[k]) != 0u); };
+    static_assert(NLF == 2 || NLF == 3, "");
+    if constexpr (NLF == 2) kq_raise(reserved(0), reserved(1), lf[0], lf[1], fin);
+    else kq_raise(reserved(0), reserved(1), reserved(2), lf[0], lf[1], lf[2], fin);
 #pragma unroll
-    for (int k = 0; k < NLF; ++k) {
-      lf[k] = kp_sel(__ballot((bm & lf_bit[k]) != 0u), kp_vmax(lf[k], fin), lf[k]);
-      lf_row[k][0] = lf[k];
-    }
+    for (int k = 0; k < NLF; ++k) lf_row[k][0] = lf[k];
     --live;
     const uint32_t touched = (bm >> 6) & (0x3Fu << 18);
 #pragma unroll
-    for (int u = 0; u < SL; ++u) ek[u] = kp_sel(__ballot((em[u] & touched) != 0u), kp_vmax(ek[u], fin), ek[u]);
+    for (int u = 0; u < SL; u += 2) kq_raise(__ballot((em[u] & touched) != 0u), __ballot((em[u + 1] & touched) != 0u), ek[u], ek[u + 1], fin);
     // successors: the lanes with room look at one each; those that became ready are filed where they were looked at
     // (scheduler.py:540-546: ties in successor order)
     if (__builtin_expect(__ballot(n_succ == 7u) != 0ull, 0)) n_succ = n_succ == 7u ? (uint32_t)cv.node[cv.lrec[cv.orec[place].at].node].n_succ : n_succ;
     mask64 mine = room & alive & __ballot(r < n_succ);
     uint32_t j0 = 0, sp = first_succ;
     while (mine) {
-      const uint32_t node = kp_sel(mine, sp, 0u), at = node & 0x1FFu, row = node >> 24;   // (a node of one predecessor: the row that stays zero)
-      const uint32_t state = g_state[at * RW], left = state - 0x400u, type = g_type[((node >> 18) & 0x3Fu) * RW];
+      const uint32_t node = kp_sel(mine, sp, 0u), row = node >> 24;   // (a node of one predecessor: the row that stays zero)
+      uint32_t at = node & 0x1FFu, type_at = (node >> 18) & 0x3Fu;
+      asm("" : "+v"(at), "+v"(type_at));   // (a field, then its address: two instructions, where the compiler shifts, masks and adds)
+      const uint32_t state = g_state[at * RW], left = state - 0x400u;
+      uint32_t type = g_type[type_at * RW];
       double t = kp_vmax(g_time[row * RW], fin);
       const mask64 ready = mine & __ballot(left < 0x400u);
       if (kp_in(mine & ~ready)) {
@@ -732,11 +791,12 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
         if (__builtin_expect(shrink, 0)) {   // (a later node of the row may be ready before what this one leaves there)
           if (kp_in(ready)) g_time[row * RW] = 0.0;
         }
-        const uint32_t b6 = type & 0x3Fu;   // one vertex or two (none: the row of zeros)
-        const uint32_t v1 = (uint32_t)__builtin_ctz(b6 | (1u << RPEG_MAX_V)), v2 = b6 ? 31u - (uint32_t)__builtin_clz(b6) : (uint32_t)RPEG_MAX_V;
+        asm("" : "+v"(type));   // (all of the register: not narrowed to 16 bits again)
+        // one vertex or two (none: the row of zeros)
+        const uint32_t v1 = (uint32_t)__builtin_ctz((type & 0x3Fu) | (1u << RPEG_MAX_V)), v2 = type >> 12;
         t = kp_vmax(t, kp_vmax(g_lf[v1 * RW], g_lf[v2 * RW]));
         const uint32_t rdy = (uint32_t)(ready >> group_shift) & ((1u << QL) - 1u);
-        file(ready, t, state, node, type, tie + (uint32_t)__builtin_popcount(rdy & below));
+        file(ready, t, left, node, type, tie + (uint32_t)__builtin_popcount(rdy & below));
         tie += (uint32_t)QL;
         live += (int)__builtin_popcount(rdy);
         longest = live > longest ? live : longest;
