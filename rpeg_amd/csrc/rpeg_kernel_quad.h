@@ -464,7 +464,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
   const int n_rows = (int)cv.h->n_rows, n_types = (int)cv.h->n_types;
 
   // ---- LDS carve-up
-  uint32_t* l_succ = (uint32_t*)lds;               // [node id][4]: id | the successor's QuadRec from bit 10 on; bit 31: none (its id is the neutral element's)
+  uint32_t* l_succ = (uint32_t*)lds;               // [node id][4]: id | the successor's QuadRec from bit 10 on (none: the neutral element's id, alone)
   uint32_t* l_own = l_succ + 4 * Z.nodes;          // [node id]: QuadRec
   uint16_t* l_id = (uint16_t*)(l_own + Z.nodes);   // level place -> id
   uint16_t* l_chain = l_id + (Z.nodes + 2);        // [node id]: place in its chain (whose nodes' ids follow each other) | nodes of the chain << 8
@@ -513,7 +513,7 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const uint32_t at = r.succ[k];
-      l_succ[4 * id + k] = (uint32_t)l_id[at] | (at < (uint32_t)n ? cv.qrec[at] & ~0x3FFu : 0x80000000u);
+      l_succ[4 * id + k] = (uint32_t)l_id[at] | (at < (uint32_t)n ? cv.qrec[at] & ~0x3FFu : 0u);
     }
   }
   KE_STAMP(0);
@@ -626,6 +626,19 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
   double makespan = 0.0;
   uint32_t n_back = 0;
   mask64 lost = 0ull;                             // plans (all four lanes) with an entry that found no room
+  // Lanes of this plan with room: before this one, all.  (Of two from one another; of four by a shift of 64 bits, which with these is
+  // shorter than bits put together: AC-share 3,355 us a step, so 3,375.)
+  auto count_room = [&](mask64 room, uint32_t& r, uint32_t& n_room) {
+    if constexpr (QL == 2) {
+      const uint32_t one = free_slots < 1u ? free_slots : 1u, other = kq_dpp<KQ_XOR1>(one);
+      r = other & below;
+      n_room = one + other;
+    } else {
+      const uint32_t in_plan = (uint32_t)(room >> group_shift) & ((1u << QL) - 1u);
+      r = (uint32_t)__builtin_popcount(in_plan & below);
+      n_room = (uint32_t)__builtin_popcount(in_plan);
+    }
+  };
   auto least = [&](const mask64 (&m)[SL]) {   // the smallest word of this lane's entries in m
     uint32_t o = kp_sel(m[0], eo[0], KQ_EMPTY);
     kq_least(m[1], o, eo[1]);
@@ -747,12 +760,14 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
     }
     bm = kq_or<QL>(bm);
     mask64 room = __ballot(free_slots != 0u);
-    uint32_t in_plan = (uint32_t)(room >> group_shift) & ((1u << QL) - 1u);
-    uint32_t r = (uint32_t)__builtin_popcount(in_plan & below), n_room = (uint32_t)__builtin_popcount(in_plan);
+    uint32_t r, n_room;
+    count_room(room, r, n_room);
     const uint32_t place = bm & 0x1FFu;
     const uint32_t first_succ = l_succ[4 * place + r];   // (r < QL)
     uint32_t n_succ = l_own[place] & 7u;
-    const double fin = gk + g_dur[(int)((bm >> 10) & 0xFFu) * RW];
+    uint32_t slot = (bm >> 10) & 0xFFu;
+    asm("" : "+v"(slot));   // (a field, then its address: two instructions, where the compiler shifts, masks and adds)
+    const double fin = gk + g_dur[slot * RW];
     if (L.mass) {
       if (kp_in(alive & quads0)) {
         g_fin[place * RW] = fin;
@@ -772,13 +787,13 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
     for (int u = 0; u < SL; u += 2) kq_raise(__ballot((em[u] & touched) != 0u), __ballot((em[u + 1] & touched) != 0u), ek[u], ek[u + 1], fin);
     // successors: the lanes with room look at one each; those that became ready are filed where they were looked at
     // (scheduler.py:540-546: ties in successor order)
-    if (__builtin_expect(__ballot(n_succ == 7u) != 0ull, 0)) n_succ = n_succ == 7u ? (uint32_t)cv.node[cv.lrec[cv.orec[place].at].node].n_succ : n_succ;
+    if (__builtin_expect(any_many, 0)) n_succ = n_succ == 7u ? (uint32_t)cv.node[cv.lrec[cv.orec[place].at].node].n_succ : n_succ;
     mask64 mine = room & alive & __ballot(r < n_succ);
-    uint32_t j0 = 0, sp = first_succ;
+    uint32_t j0 = n_room, node = first_succ;   // (in lanes that have none to look at: another's, or the neutral element, which are read alone)
     while (mine) {
-      const uint32_t node = kp_sel(mine, sp, 0u), row = node >> 24;   // (a node of one predecessor: the row that stays zero)
+      const uint32_t row = node >> 24;   // (a node of one predecessor: the row that stays zero)
       uint32_t at = node & 0x1FFu, type_at = (node >> 18) & 0x3Fu;
-      asm("" : "+v"(at), "+v"(type_at));   // (a field, then its address: two instructions, where the compiler shifts, masks and adds)
+      asm("" : "+v"(at), "+v"(type_at));
       const uint32_t state = g_state[at * RW], left = state - 0x400u;
       uint32_t type = g_type[type_at * RW];
       double t = kp_vmax(g_time[row * RW], fin);
@@ -795,34 +810,41 @@ __device__ inline void kq_eval_wave(const EvalLaunch& L, const QuadSize& Z, doub
         // one vertex or two (none: the row of zeros)
         const uint32_t v1 = (uint32_t)__builtin_ctz((type & 0x3Fu) | (1u << RPEG_MAX_V)), v2 = type >> 12;
         t = kp_vmax(t, kp_vmax(g_lf[v1 * RW], g_lf[v2 * RW]));
-        const uint32_t rdy = (uint32_t)(ready >> group_shift) & ((1u << QL) - 1u);
-        file(ready, t, left, node, type, tie + (uint32_t)__builtin_popcount(rdy & below));
+        uint32_t before, filed;
+        if constexpr (QL == 2) {
+          const uint32_t one = kp_sel(ready, 1u, 0u), other = kq_dpp<KQ_XOR1>(one);
+          before = other & below;
+          filed = one + other;
+        } else {
+          const uint32_t rdy = (uint32_t)(ready >> group_shift) & ((1u << QL) - 1u);
+          before = (uint32_t)__builtin_popcount(rdy & below);
+          filed = (uint32_t)__builtin_popcount(rdy);
+        }
+        file(ready, t, left, node, type, tie + before);
         tie += (uint32_t)QL;
-        live += (int)__builtin_popcount(rdy);
+        live += (int)filed;
         longest = live > longest ? live : longest;
       }
-      j0 += n_room;
       const mask64 again = alive & __ballot(j0 < n_succ);
       if (__builtin_expect(again == 0ull, 1)) break;
       room = __ballot(free_slots != 0u);
-      in_plan = (uint32_t)(room >> group_shift) & ((1u << QL) - 1u);
-      r = (uint32_t)__builtin_popcount(in_plan & below);
-      n_room = (uint32_t)__builtin_popcount(in_plan);
+      count_room(room, r, n_room);
       const mask64 full = again & __ballot(n_room == 0u);
       lost |= full;
       longest = (int)kp_sel(full, (uint32_t)(QL * SL + 1), (uint32_t)longest);   // (an entry without room is not counted in `live`: the class moves up a form)
       j0 = kp_sel(full, n_succ, j0);
       mine = again & room & __ballot(j0 + r < n_succ);
-      sp = 0;
+      node = 0;
       if (kp_in(mine)) {
         const uint32_t j = j0 + r;
         if (j < 4u) {
-          sp = l_succ[4 * place + j];
+          node = l_succ[4 * place + j];
         } else {
           const uint32_t to = cv.place[cv.succ[cv.node[cv.lrec[cv.orec[place].at].node].succ_begin + j]];
-          sp = (uint32_t)l_id[to] | (cv.qrec[to] & ~0x3FFu);
+          node = (uint32_t)l_id[to] | (cv.qrec[to] & ~0x3FFu);
         }
       }
+      j0 += n_room;
     }
   }
   ovf = ovf || kp_in(lost);
