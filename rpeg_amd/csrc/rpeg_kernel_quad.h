@@ -243,11 +243,67 @@ __device__ inline void kq_count(const double* g_rank, const uint32_t* l_own, con
     if (it < e) g_state[it * RW] = (uint16_t)(before[t] | (EQ && same[t] > (uint32_t)(l_chain[it] >> 8) ? 0x200u : 0u) | (((l_own[it] >> 3) & 0x3Fu) << 10));
   }
 }
-// Positions of all nodes: one class after the other, up to four of its nodes to a lane, so that a rank read counts for all of them.
+// The same for two nodes a lane of classes of `size` nodes each that follow one another, ids b to e - 1 together; per_size: 1 / size.
+template <int QL, int QR, bool EQ>
+__device__ inline void kq_count_run(const double* g_rank, const uint32_t* l_own, const uint16_t* l_chain, uint16_t* g_state, int i, int b, int e, int size, float per_size) {
+  constexpr int RW = KE_WAVE / QL, RG = KE_WAVE / QR, NB = 2, AHEAD = 4;
+  const double* from[NB];
+  double rv[NB];
+  uint32_t before[NB], same[NB];
+#pragma unroll
+  for (int t = 0; t < NB; ++t) {
+    const int it = i + t * QR < e ? i + t * QR : b;
+    before[t] = (uint32_t)(b + (int)(((float)(it - b) + 0.5f) * per_size) * size);   // (its class's first: exact, a half is far more than what is rounded)
+    from[t] = g_rank + before[t] * RG;
+    rv[t] = g_rank[it * RG];
+    same[t] = 0u;
+  }
+  auto count = [&](int t, double r) {
+    before[t] += r > rv[t] ? 1u : 0u;
+    if (EQ) same[t] += r == rv[t] ? 1u : 0u;
+  };
+  int j = 0;
+  for (; j + AHEAD <= size; j += AHEAD) {
+    double r[NB][AHEAD];
+#pragma unroll
+    for (int t = 0; t < NB; ++t)
+#pragma unroll
+      for (int k = 0; k < AHEAD; ++k) r[t][k] = from[t][(j + k) * RG];
+#pragma unroll
+    for (int t = 0; t < NB; ++t)
+#pragma unroll
+      for (int k = 0; k < AHEAD; ++k) count(t, r[t][k]);
+  }
+  for (; j < size; ++j)
+#pragma unroll
+    for (int t = 0; t < NB; ++t) count(t, from[t][j * RG]);
+#pragma unroll
+  for (int t = 0; t < NB; ++t) {
+    const int it = i + t * QR;
+    if (it < e) g_state[it * RW] = (uint16_t)(before[t] | (EQ && same[t] > (uint32_t)(l_chain[it] >> 8) ? 0x200u : 0u) | (((l_own[it] >> 3) & 0x3Fu) << 10));
+  }
+}
+// Positions of all nodes: one class after the other, up to four of its nodes to a lane, so that a rank read counts for all of them;
+// of small classes (the iterations of an operator: five or eight nodes) as many of one size as follow one another, where one by one a
+// class of five leaves eleven of sixteen lanes idle.  (us a step, one by one / together: 131,072 PPO plans 813 / 798, GRPO 401 / 398;
+// 65,536 GRPO, 1,048,576 DPO and 262,144 AC-share within 0.2 %.)
 template <int QL, int QR, bool EQ>
 __device__ inline void kq_count_all(const double* g_rank, const uint32_t* l_own, const uint16_t* l_chain, uint16_t* g_state, uint32_t class_ends, int r_q, int n) {
-  for (int b = 0, k = 0; b < n; ++k) {
-    const int e = __builtin_amdgcn_readlane((int)class_ends, k);
+  for (int b = 0, k = 0; b < n;) {
+    int e = __builtin_amdgcn_readlane((int)class_ends, k++);
+    const int size = e - b;
+    if (size <= 2 * QR) {
+      while (e < n && __builtin_amdgcn_readlane((int)class_ends, k) == e + size) {
+        e += size;
+        ++k;
+      }
+      if (e > b + size) {
+        const float per_size = __builtin_amdgcn_rcpf((float)size);
+        for (int i0 = b; i0 < e; i0 += 2 * QR) kq_count_run<QL, QR, EQ>(g_rank, l_own, l_chain, g_state, i0 + r_q, b, e, size, per_size);
+        b = e;
+        continue;
+      }
+    }
     int i0 = b;
     for (; e - i0 > 2 * QR; i0 += 4 * QR) kq_count<QL, QR, 4, EQ>(g_rank, l_own, l_chain, g_state, i0 + r_q, b, e);
     if (e - i0 > QR) kq_count<QL, QR, 2, EQ>(g_rank, l_own, l_chain, g_state, i0 + r_q, b, e);
