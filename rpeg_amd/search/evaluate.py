@@ -115,8 +115,10 @@ def _engine_for(rpeg: RPEG, suite: ModelSuite, workload: Workload, hw: Hardware,
     rest = (tuple(sorted((m.value, s) for m, s in suite.specs.items())), workload, hw, space, K_eval, policy,
             transfer_policy)
     key = (tuple((s.name, s.memory_trainable) for s in structures),) + rest
-    if _engines and key == next(reversed(_engines)):     # (a comparison: a hash goes through every number of the problem)
-        return next(reversed(_engines.values())), st
+    # (a comparison: a hash goes through every number of the problem; key and engine of one look: another thread may add one)
+    last = next(reversed(_engines.items()), None)
+    if last is not None and last[0] == key:
+        return last[1], st
     alias = ((st.name, st.memory_trainable), "first") + rest
     hit = key if key in _engines else alias if not more_structures and alias in _engines else None
     if hit is not None:

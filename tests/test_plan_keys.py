@@ -7,7 +7,7 @@ import pytest
 
 from rpeg_amd import configs
 from rpeg_amd.engine.problem import PlanBatch
-from rpeg_amd.search import candidates
+from rpeg_amd.search import candidates, evaluate
 from rpeg_amd.search.cache import _config_hash_plain, config_hash, key_text
 from rpeg_amd.search.evaluate import Configuration, _pack, _structure_of
 from rpeg_amd.search.optimizer import plan_row
@@ -72,3 +72,26 @@ def test_plans_that_cannot_be_packed():
                           ({"mb": {**plan.mb, v: 1 << 15}}, OverflowError)):
         with pytest.raises(error):
             _pack([Configuration(rpeg, dataclasses.replace(plan, **change), problem.device_space)], st, problem.workload)
+
+
+def test_an_engine_used_last_is_that_of_its_key(monkeypatch):
+    """... also where another thread adds one between the comparison and the return."""
+    problem, [(rpeg, plan)] = seeded(5, 0, 1)
+
+    class Engines(dict):
+        pass
+
+    class Key(tuple):
+        def __eq__(self, other):
+            same = tuple.__eq__(self, other)
+            engines["another"] = "engine of another problem"
+            return same
+        __hash__ = tuple.__hash__
+
+    p, engines = problem, Engines()
+    monkeypatch.setattr(evaluate, "_engines", engines)
+    st = _structure_of(rpeg)
+    key = Key((((st.name, st.memory_trainable),), tuple(sorted((m.value, s) for m, s in p.suite.specs.items())), p.workload, p.hw,
+               p.device_space, p.K_eval, p.memory_policy, evaluate.RPEG_TRANSFER_RESOURCE_POLICY))
+    engines[key] = "its engine"
+    assert evaluate._engine_for(rpeg, p.suite, p.workload, p.hw, p.device_space, p.K_eval, p.memory_policy)[0] == "its engine"
