@@ -212,13 +212,15 @@ def _pack(configs: Sequence[Configuration], st, workload: Workload) -> PlanBatch
         width = max(width, len(verts) * FIELDS_PER_VERTEX)
     n = len(configs)
     batch = PlanBatch.empty(n)
+    rows = None
     if len(numbers) == n * width:
-        try:      # (whole numbers, as they come)
+        try:
             rows = np.frombuffer(array("h", numbers), np.int16)
-        except TypeError:
-            rows = np.array(numbers).astype(np.int16)
+        except TypeError:      # (some are no whole numbers)
+            pass
+    if rows is not None:
         batch.vert[:width] = rows.reshape(n, width).T
-    else:         # (templates of several sizes)
+    else:
         for i, cfg in enumerate(configs):
             batch.set_plan(i, 0, split, (), cfg.rpeg, cfg.plan)
     batch.head[:len(head[0])] = np.array(head, np.uint8).T

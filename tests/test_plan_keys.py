@@ -69,7 +69,8 @@ def test_plans_that_cannot_be_packed():
     without = lambda d: {x: y for x, y in d.items() if x != v}  # noqa: E731
     for change, error in (({"sigma": without(plan.sigma)}, KeyError), ({"pi": without(plan.pi)}, KeyError),
                           ({"mb": without(plan.mb)}, KeyError), ({"pi": {**plan.pi, v: (1, 1)}}, ValueError),
-                          ({"mb": {**plan.mb, v: 1 << 15}}, OverflowError)):
+                          ({"mb": {**plan.mb, v: 1 << 15}}, OverflowError),
+                          ({"mb": {**plan.mb, v: 1 << 15, rpeg.vertices[0]: 2.0}}, OverflowError)):
         with pytest.raises(error):
             _pack([Configuration(rpeg, dataclasses.replace(plan, **change), problem.device_space)], st, problem.workload)
 
