@@ -2391,6 +2391,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     std::vector<uint32_t> qc[3];
     for (uint32_t c : order)   // (largest graphs first)
       if (quad[c]) qc[quad_kind(c)].push_back(c);
+    bool shared = !qc[2].empty();   // the streams are, by as many launches as there are
     for (int kind : {2, 0, 1}) {
       std::vector<uint32_t>& q = qc[kind];
       if (q.empty()) continue;
@@ -2402,7 +2403,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
         upto[k + 1] = upto[k] + (double)waves_of(q[k], kind) * (double)e->cls_nodes[cids[q[k]]];
       }
       std::vector<size_t> cuts = {0, q.size()};
-      const size_t most = deep ? QUAD_BINS : kind != 2 && !aside ? 2 : 1;
+      const size_t most = deep ? QUAD_BINS : !shared ? 2 : 1;
       while (cuts.size() <= most) {
         double best = 0.05 * upto.back() * lds[0];
         size_t at = 0;
@@ -2419,8 +2420,6 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
         QuadLaunch l;
         l.first = n_quad_waves;
         l.kind = kind;
-        l.aside = kind == 2 || i > 0;
-        l.first_stream = kind == 0;
         for (size_t k = cuts[i]; k < cuts[i + 1]; ++k) {
           const uint32_t c = q[k];
           clpw[c] = QUAD_KIND[kind].plans;
@@ -2431,18 +2430,23 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
           l.size.fit(e->cls_quad[cids[c]]);
           n_quad_waves += nw;
         }
-        aside = aside || l.aside;
         quad_launch.push_back(l);
       }
+      shared = shared || cuts.size() > 2;
     }
     if (deep) {   // the largest on a stream of its own, the others by turns on two
       std::stable_sort(quad_launch.begin(), quad_launch.end(), [&](const QuadLaunch& x, const QuadLaunch& y) {
         return kq_lds_bytes(QUAD_KIND[x.kind].plans, x.size, mass != nullptr) > kq_lds_bytes(QUAD_KIND[y.kind].plans, y.size, mass != nullptr); });
       for (size_t k = 0; k < quad_launch.size(); ++k) { quad_launch[k].first_stream = k == 0; quad_launch[k].aside = k % 2 == 1; }
-      aside = quad_launch.size() > 1;
-    } else {   // the smaller graphs of a form last
-      std::stable_partition(quad_launch.begin(), quad_launch.end(), [](const QuadLaunch& x) { return x.kind == 2 || !x.aside; });
+    } else {
+      // The form of most entries first, whose wavefronts last longest, then larger graphs before smaller ones: the first follows the
+      // scatter on its own stream, the others start when the host has sent them and their streams have seen the fork, 10 to 50 us later.
+      // (us a step, the 16 entries of GRPO behind the 8, all of PPO's and AC-share's behind the fork / now: 65,536 GRPO 287 / 281, 131,072
+      // 400 / 384, 20,000 241 / 231; 20,011 PPO 282 / 276, 50,000 410 / 399; 20,000 AC-share 659 / 641, 65,536 1,321 / 1,306.)
+      std::stable_sort(quad_launch.begin(), quad_launch.end(), [](const QuadLaunch& x, const QuadLaunch& y) { return x.kind > y.kind; });
+      for (size_t k = 0; k < quad_launch.size(); ++k) { quad_launch[k].first_stream = k == 0; quad_launch[k].aside = k >= (n_eval_waves ? 1u : 2u); }
     }
+    for (const QuadLaunch& q : quad_launch) aside = aside || q.aside;
   }
   {   // the positions of a wavefront's plans all at once, its ranks in LDS, where the launches' wavefronts find room together all the
       // same; else by the larger parts where they need (next to) no more LDS than the smaller, the rows behind them needing as much anyway
@@ -2700,27 +2704,31 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // (The main kernel first also when k_plan has only a handful of tasks, which then wait until wavefronts of the main
   // kernel retire: with those few in front the step was 30 us longer on config 4.)
   HIP_TRY(e, launch_main());
-  // (the three launches back to back: every call between them delays the start of the later kernels)
   const bool side_q = n_quad_waves || peaks_aside;
-  if (ahead) {
-    HIP_TRY(e, hipStreamWaitEvent(s, e->ev_fork, 0));
-    if (e->timing) HIP_TRY(e, hipEventRecord(e->ev0, s));
-  } else if (side_q) {
-    HIP_TRY(e, hipStreamWaitEvent(e->s3, e->ev_fork, 0));
+  // A stream waits for the fork right ahead of what first goes there: every call between launches delays the later ones, and the one
+  // that starts everything on the fork's own stream needs none.  (All waits ahead of the launches / now: 16,384 DPO plans 131 / 125 us
+  // a step, 65,536 150 / 137.)
+  hipStream_t followed[3];
+  int n_followed = 0;
+  auto follow = [&](hipStream_t on) -> hipError_t {
+    if (on == sm || std::find(followed, followed + n_followed, on) != followed + n_followed) return hipSuccess;
+    followed[n_followed++] = on;   // (of s, s2, s3 and s4 one is the fork's own)
+    return hipStreamWaitEvent(on, e->ev_fork, 0);
+  };
+  if (ahead && e->timing) {
+    HIP_TRY(e, follow(s));
+    HIP_TRY(e, hipEventRecord(e->ev0, s));
   }
-  // (k_quad second: measured against k_quad first, 0.50 against 0.52-0.53 ms on config 2, and against k_quad last,
-  // 0.59 ms; its wavefronts need the most LDS after the main kernel's)
-  // The memory-model launches of a batch without work for the main kernel: behind k_plan where that has next to nothing to
-  // do (another stream costs an event between streams, 15 us: 16,384 DPO plans 126 against 143 us), else on the fourth
-  // stream where it is free, else behind k_quad's first launch (behind k_plan they ended the call: 65,536 GRPO plans
-  // 365 against 353 us, 20,011 PPO plans 409 against 381).
-  const bool peaks_apart = peaks_deferred && !peaks_aside && !n_waves, peaks_on_s2 = peaks_apart && n_solo && n_solo <= (uint32_t)e->n_cu;
-  const bool peaks_on_s4 = peaks_apart && !peaks_on_s2 && !aside;
-  if (aside || peaks_on_s4) HIP_TRY(e, hipStreamWaitEvent(e->s4, e->ev_fork, 0));
-  for (const QuadLaunch& q : quad_launch)
-    if (int rc = launch_quad(q, q.aside ? e->s4 : q.first_stream && !n_waves ? sm : sq)) return rc;   // (beside the main kernel, where that has tasks)
+  // (k_quad ahead of k_plan: measured behind a main kernel, 0.50 ms on config 2 against 0.59 with k_plan in between, and without one,
+  // k_plan behind the first of its launches: 65,536 GRPO plans 282 / 300 us, 20,011 PPO 277 / 332; its wavefronts need the most LDS after the
+  // main kernel's)
+  for (const QuadLaunch& q : quad_launch) {
+    const hipStream_t on = q.aside ? e->s4 : q.first_stream && !n_waves ? sm : sq;   // (beside the main kernel, where that has tasks)
+    HIP_TRY(e, follow(on));
+    if (int rc = launch_quad(q, on)) return rc;
+  }
   if (n_solo) {   // the single-plan wavefronts, beside the main kernel
-    HIP_TRY(e, hipStreamWaitEvent(e->s2, e->ev_fork, 0));
+    HIP_TRY(e, follow(e->s2));
     EvalLaunch S = L;
     S.queue = nullptr;
     S.perm = e->d_perm + n_sorted;
@@ -2730,9 +2738,17 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     launch_plan(kp_lds_bytes(e->max_nodes, e->max_slots), e->s2, S, e->n_cu);
     HIP_TRY(e, hipGetLastError());
   }
+  // The memory-model launches of a batch without work for the main kernel: behind k_plan where that has next to nothing to
+  // do (another stream costs an event between streams, 15 us: 16,384 DPO plans 126 against 143 us), else on a stream that is free (the one
+  // of k_quad's second launch, then the fourth), else behind a launch of k_quad that is not the longest, or of a deep batch's the first
+  // (behind k_plan they ended the call: 65,536 GRPO plans 365 against 353 us, 20,011 PPO plans 409 against 381; behind the second of
+  // two launches 131,072 PPO 824 us, on the fourth stream 787, though 20,000 AC-share 640 and 646).
+  const bool peaks_apart = peaks_deferred && !peaks_aside && !n_waves, peaks_on_s2 = peaks_apart && n_solo && n_solo <= (uint32_t)e->n_cu;
+  const bool peaks_on_s4 = peaks_apart && !peaks_on_s2 && !aside && quad_launch.size() > 1;
   if (peaks_deferred) {
     const unsigned pblk = (unsigned)((n + WAVE - 1) / WAVE);
-    const hipStream_t sp = peaks_aside ? sq : peaks_on_s2 ? e->s2 : peaks_on_s4 ? e->s4 : sm;
+    const hipStream_t sp = peaks_aside ? sq : peaks_on_s2 ? e->s2 : peaks_on_s4 ? e->s4 : peaks_apart && !(deep && aside) ? sq : sm;
+    HIP_TRY(e, follow(sp));
     G.row_begin = e->max_uni + 1;   // (the memory terms, which nothing but this launch needs: not ahead of the scheduling kernels)
     G.row_end = G.row_begin + e->max_v;
     hipLaunchKernelGGL(k_prologue, dim3(pblk, e->max_v), dim3(WAVE), 0, sp, G);
