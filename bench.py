@@ -36,9 +36,9 @@ ALG_FLOPS = {1: 3697.0, 2: 2165.3, 3: 6502.9, 4: 1245.8, 5: 4155.6}
 # VMEM_RD + VMEM_WR of the evaluation kernels / plans).
 MEASURED = {
     1: dict(layout=(4096, 7168, 1, 0, 0), traffic=23.1e6, instructions_per_plan=11699.0),
-    2: dict(layout=(4129, 21536, 0, 1554, 2575), traffic=144.8e6, instructions_per_plan=1372.0),
-    3: dict(layout=(29518, 29984, 0, 13209, 16309), traffic=1555.1e6, instructions_per_plan=5841.0),
-    4: dict(layout=(32781, 14640, 0, 6, 32775), traffic=779.4e6, instructions_per_plan=443.0),
+    2: dict(layout=(4129, 21536, 0, 1554, 2575), traffic=144.9e6, instructions_per_plan=1288.0),
+    3: dict(layout=(29518, 29984, 0, 13209, 16309), traffic=1556.4e6, instructions_per_plan=5423.0),
+    4: dict(layout=(32781, 14640, 0, 6, 32775), traffic=768.9e6, instructions_per_plan=409.0),
 }
 
 
