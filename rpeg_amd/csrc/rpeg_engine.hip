@@ -1022,7 +1022,7 @@ struct rpeg_engine_s {
   hipStream_t s3 = nullptr;                     // third stream: the few-lanes-per-plan wavefronts (k_quad)
   hipEvent_t ev_join3 = nullptr;
   hipEvent_t ev_sig = nullptr;                  // the signature kernel of a call is done (its class ids are there)
-  bool layout_ahead = true;                     // prologue, layout and main kernel on k_quad's stream (see `ahead` in eval_batch_impl)
+  bool layout_ahead = false;                    // prologue, layout and main kernel on k_quad's stream (see `ahead` in eval_batch_impl)
   int side_dev = 0;                             // device of the side streams
   uint32_t quad_share_pct = 100;                // largest share of a batch's plans that k_quad takes (rpeg_engine_set_quad_share)
   bool quad_attr_set = false;
@@ -1890,7 +1890,11 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   // ahead: k_quad's stream becomes the main line of the call -- the cost-model launch goes there as soon as the class
   // ids are written (beside the hand-over of the counters to the host), the layout and the scatter follow it there
   // as soon as the host has them, and the main kernel follows those in order; the caller's stream carries k_quad
-  // and joins at the end.  Only when no other engine of the process is using the side streams.
+  // and joins at the end.  Only when no other engine of the process is using the side streams, and only where the caller asks for it
+  // (rpeg_engine_set_side_layout): the events between the streams, ahead of the cost model and of k_quad's other launches, cost more
+  // than the hand-over, 8 us, that the cost model waits for in order.  us a step, ahead / in order: 16,384 DPO plans 127 / 110, 65,536 139 /
+  // 126, 300,000 266 / 257, 1,048,576 712 / 708; GRPO 20,000 234 / 229, 65,536 283 / 279, 131,072 381 / 382; PPO 20,011 275 / 262, 50,000 396 /
+  // 384, 131,072 782 / 785; AC-share 20,000 647 / 623, 65,536 1,303 / 1,299, 262,144 3,323 / 3,319.
   bool ahead = false;
   // (whatever way the call ends, the caller's stream follows what went to k_quad's stream)
   struct AheadJoin {

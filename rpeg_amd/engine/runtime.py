@@ -236,7 +236,7 @@ class Engine:
         self._check(self.lib.rpeg_engine_set_sa_groups(self._h, int(groups)), "rpeg_engine_set_sa_groups")
 
     def set_side_layout(self, on: bool):
-        """Cost-model launch, layout and main kernel of a full batch on a side stream (default) or on the caller's."""
+        """Cost-model launch, layout and main kernel of a full batch on a side stream or on the caller's (default)."""
         self._check(self.lib.rpeg_engine_set_side_layout(self._h, 1 if on else 0), "rpeg_engine_set_side_layout")
 
     def set_quad_share(self, percent: int):

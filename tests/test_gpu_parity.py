@@ -479,8 +479,8 @@ def test_the_fitted_figures_of_the_split_move_plans_between_kernels_and_no_bit()
 
 @pytest.mark.parametrize("c,n", [(2, 65536), (4, 200000), (3, 50000)])
 def test_the_stream_that_carries_the_layout_changes_no_bit(c, n):
-    """rpeg_engine_set_side_layout: cost-model launch, layout and main kernel on the side stream (the default) or on
-    the caller's; cold calls (classes lowered, several rounds) and warm ones; two engines that step in turn on two
+    """rpeg_engine_set_side_layout: cost-model launch, layout and main kernel on the side stream or on the caller's
+    (the default); cold calls (classes lowered, several rounds) and warm ones; two engines that step in turn on two
     threads, of which the one that finds the side streams taken stays on its own; a batch that no plan of is valid.
     Every call equals the host build."""
     import threading
