@@ -14,6 +14,7 @@ integer part of `is_valid`) are host code as in the reference.
 
 from __future__ import annotations
 
+import threading
 import weakref
 from array import array
 from dataclasses import dataclass, replace
@@ -85,6 +86,7 @@ def stale_publication_layout_valid(config: Configuration) -> bool:
 # ----------------------------------------------------------------------------- engine plumbing
 _engines: Dict[tuple, object] = {}   # insertion-ordered: least recently used first
 _MAX_ENGINES = 16
+_engines_lock = threading.RLock()    # held for every look at the table and change of it: a look-up puts its entry last
 
 
 def _structure_of(rpeg: RPEG):
@@ -115,25 +117,35 @@ def _engine_for(rpeg: RPEG, suite: ModelSuite, workload: Workload, hw: Hardware,
     rest = (tuple(sorted((m.value, s) for m, s in suite.specs.items())), workload, hw, space, K_eval, policy,
             transfer_policy)
     key = (tuple((s.name, s.memory_trainable) for s in structures),) + rest
-    # (a comparison: a hash goes through every number of the problem; key and engine of one look: another thread may add one)
-    last = next(reversed(_engines.items()), None)
-    if last is not None and last[0] == key:
-        return last[1], st
-    alias = ((st.name, st.memory_trainable), "first") + rest
-    hit = key if key in _engines else alias if not more_structures and alias in _engines else None
-    if hit is not None:
-        # (an engine that holds this template as structure 0 beside others serves as well, and keeps its classes)
-        eng = _engines.pop(hit)
-        _engines[hit] = eng          # most recently used last
-        return eng, st
+    with _engines_lock:
+        # (a comparison: a hash goes through every number of the problem)
+        last = next(reversed(_engines.items()), None)
+        if last is not None and last[0] == key:
+            return last[1], st
+        alias = ((st.name, st.memory_trainable), "first") + rest
+        hit = key if key in _engines else alias if not more_structures and alias in _engines else None
+        if hit is not None:
+            # (an engine that holds this template as structure 0 beside others serves as well, and keeps its classes)
+            eng = _engines.pop(hit)
+            _engines[hit] = eng          # most recently used last
+            return eng, st
     from ..engine.runtime import Engine
     problem = EvalProblem(structures=structures, suite=suite, workload=workload, hw=hw, device_space=space,
                           K_eval=K_eval, memory_policy=policy, transfer_resource_policy=transfer_policy)
-    eng = _engines[key] = Engine(problem)
-    _engines.setdefault(alias, eng)
-    while len(_engines) > _MAX_ENGINES:      # a long-lived process that sees many problems keeps the recent ones;
-        _engines.pop(next(iter(_engines)))   # an engine frees its device memory when its last holder lets go
+    made = Engine(problem)     # (other threads' look-ups go on meanwhile)
+    with _engines_lock:
+        eng = _engines.setdefault(key, made)    # (of two threads that made one for the same problem: the first one's)
+        _engines.setdefault(alias, eng)
+        gone = []
+        while len(_engines) > _MAX_ENGINES:                  # a long-lived process that sees many problems keeps the recent ones;
+            gone.append(_engines.pop(next(iter(_engines))))  # an engine frees its device memory when its last holder lets go
     return eng, st
+
+
+def _recent_engines() -> list:
+    """The engines, most recently used first."""
+    with _engines_lock:
+        return list(reversed(_engines.values()))
 
 
 def _engine_like(rpeg, space: Optional[DeviceSpace], suite=None, workload=None, vertex=None, hw=None, policy=None):
@@ -144,7 +156,7 @@ def _engine_like(rpeg, space: Optional[DeviceSpace], suite=None, workload=None, 
     whose results depend on neither.  With `vertex` in place of `rpeg`: an engine with a template that holds that
     vertex, the structure and the vertex's slot in it."""
     want = None if rpeg is None else _structure_of(rpeg).name
-    for eng in reversed(list(_engines.values())):
+    for eng in _recent_engines():
         p = eng.problem
         if (space is not None and p.device_space != space) or (suite is not None and p.suite.specs != suite.specs) or \
                 (workload is not None and p.workload != workload) or (hw is not None and p.hw != hw) or \
@@ -170,7 +182,7 @@ def _engine_space_for(rpeg, plan, suite, workload, hw) -> DeviceSpace:
     def fits(space):
         return all(is_compatible(plan.sigma[v], plan.pi[v], space) for v in rpeg.vertices)
     want = _structure_of(rpeg).name
-    for eng in reversed(list(_engines.values())):
+    for eng in _recent_engines():
         p = eng.problem
         if p.suite.specs == suite.specs and p.workload == workload and p.hw == hw and \
                 any(st.name == want for st in p.structures) and fits(p.device_space):

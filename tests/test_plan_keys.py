@@ -1,6 +1,8 @@
 """The text of a plan's cache key put together from its row of numbers, and plans packed many at a time, against the plain forms."""
 
 import dataclasses
+import threading
+import time
 
 import numpy as np
 import pytest
@@ -96,3 +98,90 @@ def test_an_engine_used_last_is_that_of_its_key(monkeypatch):
                p.device_space, p.K_eval, p.memory_policy, evaluate.RPEG_TRANSFER_RESOURCE_POLICY))
     engines[key] = "its engine"
     assert evaluate._engine_for(rpeg, p.suite, p.workload, p.hw, p.device_space, p.K_eval, p.memory_policy)[0] == "its engine"
+
+
+def two_problems(monkeypatch):
+    """Look-ups of the engines of two problems, of a table that calls `meanwhile` (in another thread, and goes on when that is
+    done or waits) the first time `where` is reached."""
+    (problem, [(rpeg, plan)]), (other, [(other_rpeg, _)]) = seeded(5, 0, 1), seeded(2, 0, 1)
+
+    class Engine:
+        def __init__(self, problem):
+            self.problem = problem
+
+    class Reversed:
+        def __init__(self, engines):
+            self.engines = engines
+
+        def __reversed__(self):
+            it = reversed(dict.items(self.engines))
+            self.engines.reach("reversed")
+            return it
+
+    class Engines(dict):
+        where, meanwhile, thread = None, None, None
+
+        def reach(self, where):
+            if where == self.where:
+                self.where, self.taken = None, threading.Event()
+                self.thread = threading.Thread(target=self.meanwhile)
+                self.thread.start()
+                self.taken.wait(0.3) if where == "found" else self.thread.join(0.3)
+
+        def items(self):
+            return Reversed(self)
+
+        def pop(self, key):
+            self.reach("found")
+            got = dict.pop(self, key)
+            if threading.current_thread() is self.thread:    # (the first thread goes on while the entry is out)
+                self.taken.set()
+                time.sleep(0.3)
+            return got
+
+    import rpeg_amd.engine.runtime as runtime
+    engines = Engines()
+    monkeypatch.setattr(runtime, "Engine", Engine)
+    monkeypatch.setattr(evaluate, "_engines", engines)
+
+    def look_up(p, r):
+        return evaluate._engine_for(r, p.suite, p.workload, p.hw, p.device_space, p.K_eval, p.memory_policy)[0]
+    return engines, lambda: look_up(problem, rpeg), lambda: look_up(other, other_rpeg)
+
+
+def test_an_engine_is_looked_up_while_another_thread_changes_the_table(monkeypatch):
+    engines, one, other = two_problems(monkeypatch)
+    got = [one()]
+    engines.where, engines.meanwhile = "reversed", lambda: got.append(other())
+    assert one() is got[0]
+    engines.thread.join()
+    assert got[1] is other() and got[1] is not got[0]
+
+
+def test_an_engine_that_another_thread_looks_up_too_is_the_same(monkeypatch):
+    engines, one, other = two_problems(monkeypatch)
+    want = one()
+    other()
+    got = []
+    engines.where, engines.meanwhile = "found", lambda: got.append(one())
+    assert one() is want
+    engines.thread.join()
+    assert got == [want]
+
+
+def test_two_threads_that_make_an_engine_of_one_problem_get_the_same(monkeypatch):
+    import rpeg_amd.engine.runtime as runtime
+    _, one, _ = two_problems(monkeypatch)
+    both, made = threading.Barrier(2), runtime.Engine
+
+    def slow(problem):
+        both.wait(10)
+        return made(problem)
+    monkeypatch.setattr(runtime, "Engine", slow)
+    got = []
+    threads = [threading.Thread(target=lambda: got.append(one())) for _ in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(got) == 2 and got[0] is got[1]
