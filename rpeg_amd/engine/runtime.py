@@ -8,7 +8,9 @@ missing library or a missing GPU raises.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import os
+import threading
 from typing import Dict, Optional
 
 import numpy as np
@@ -182,10 +184,28 @@ class DeviceBatch:
         self.soa = abi.PlanSoaT(self.vert.data_ptr(), self.head.data_ptr(), self.vert.shape[1])
 
 
+def _one_at_a_time(cls):
+    """A class whose objects' public calls wait for each other (a thread's calls may nest)."""
+    def alone(call):
+        @functools.wraps(call)
+        def f(self, *args, **kwargs):
+            with self._calls:
+                return call(self, *args, **kwargs)
+        return f
+    for name, call in list(vars(cls).items()):
+        if callable(call) and not name.startswith("_"):
+            setattr(cls, name, alone(call))
+    return cls
+
+
+@_one_at_a_time
 class Engine:
-    """One compiled problem on one GPU.  Not thread-safe; use one engine per host thread."""
+    """One compiled problem on one GPU.  Its calls are taken one at a time, since threads that evaluate plans of one problem through
+    rpeg_amd.search share an engine (the library's engines take no calls from several threads at once); for evaluations that overlap,
+    one engine per host thread."""
 
     def __init__(self, problem: EvalProblem, device: str = "cuda:0"):
+        self._calls = threading.RLock()
         torch = _torch()
         self.lib = load_library()
         self.problem = problem
