@@ -65,6 +65,10 @@ class _KeyText:
         self.tau = dumps({m.value: t for m, t in rpeg.tau.items()})
         self.vertices = dumps(sorted((_vertex(v) for v in rpeg.vertices), key=lambda x: x["id"]))
         ids = [v.id for v in rpeg.vertices]
+        # (of other names, or none, json makes the text)
+        self.vertex_of = tuple(rpeg.vertices) if ids and len(set(ids)) == len(ids) and all(type(x) is str for x in ids) else None
+        if self.vertex_of is None:
+            return
         order = sorted(range(len(ids)), key=ids.__getitem__)
         name = [dumps(x).replace("%", "%%") for x in ids]
         three = "[%d,%d,%d]"
@@ -76,7 +80,6 @@ class _KeyText:
         row = 10     # of a vertex: three degrees, micro-batches, origin, extent
         self.places = itemgetter(*([row * x + 3 for x in order] + [row * x + f for x in order for f in (0, 1, 2)] +
                                    [row * x + f for x in order for f in (7, 8, 9, 4, 5, 6)]))
-        self.vertex_of = tuple(rpeg.vertices) if len(set(ids)) == len(ids) else None
 
     def of_row(self, row) -> str:
         return hashlib.sha256((self.format % self.places(row)).encode("utf-8")).hexdigest()

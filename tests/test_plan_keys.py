@@ -53,6 +53,17 @@ def test_plans_that_are_no_row_of_whole_numbers():
     assert config_hash(odd, p) == _config_hash_plain(odd, p)
 
 
+@pytest.mark.parametrize("names", [(), (0, 1, 2, 3, 4, 5), (10, 9, 8, 7, 6, 5), (1.5, 2, True, 4, 5, 6), ("a",)])
+def test_key_of_a_template_without_vertices_or_with_other_names_than_texts(names):
+    _, [(rpeg, plan)] = seeded(1, 0, 1)
+    verts = tuple(dataclasses.replace(v, id=x) for v, x in zip(rpeg.vertices, names))
+    move = lambda d: dict(zip(verts, d.values()))  # noqa: E731
+    for edges in ((), tuple(dataclasses.replace(e, src=verts[0], dst=verts[-1]) for e in rpeg.data_edges[:1] if verts)):
+        r = dataclasses.replace(rpeg, vertices=verts, data_edges=edges, pub_edges=())
+        p = dataclasses.replace(plan, sigma=move(plan.sigma), pi=move(plan.pi), mb=move(plan.mb))
+        assert config_hash(r, p) == config_hash(r, p) == _config_hash_plain(r, p)
+
+
 @pytest.mark.parametrize("workload,structure", CASES)
 def test_packed_plans_are_the_plans_one_by_one(workload, structure):
     problem, plans = seeded(workload, structure, 9)
