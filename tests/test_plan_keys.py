@@ -53,6 +53,16 @@ def test_plans_that_are_no_row_of_whole_numbers():
     assert config_hash(odd, p) == _config_hash_plain(odd, p)
 
 
+def test_a_key_makes_no_encoder(monkeypatch):
+    """... neither a new template's nor that of a plan that is no row (six to ten a key were a tenth of its time)."""
+    import json
+    _, [(rpeg, plan), (other, _)] = seeded(1, 0, 2)
+    half = dataclasses.replace(plan, mb={v: float(m) for v, m in plan.mb.items()})
+    want = [_config_hash_plain(rpeg, plan), _config_hash_plain(other, half)]
+    monkeypatch.setattr(json, "JSONEncoder", None)
+    assert [config_hash(rpeg, plan), config_hash(other, half)] == want
+
+
 @pytest.mark.parametrize("names", [(), (0, 1, 2, 3, 4, 5), (10, 9, 8, 7, 6, 5), (1.5, 2, True, 4, 5, 6), ("a",)])
 def test_key_of_a_template_without_vertices_or_with_other_names_than_texts(names):
     _, [(rpeg, plan)] = seeded(1, 0, 1)
