@@ -124,30 +124,31 @@ __device__ inline double kq_vmin(double a, double b, double c, double d) {
 // all of them on).  A move or a maximum each, where a select takes an instruction for every word and one for what it selects; the masks go
 // to EXEC by scalar instructions, which other wavefronts' vector instructions overlap.  (us a step, selects / moves: 1,048,576 DPO plans
 // 787 / 720, 262,144 AC-share 3,455 / 3,370, 131,072 PPO 838 / 810, GRPO 418 / 402, 65,536 GRPO 304 / 291, 20,011 PPO 297 / 284.)
+// What is written here is written before the last of the other operands is read: early-clobber, also what is read itself.
 // -- the larger of two times
 __device__ inline void kq_raise(mask64 m0, mask64 m1, double& a, double& b, double t) {
   asm("s_mov_b64 exec, %2\n\tv_max_f64 %0, %0, %4\n\ts_mov_b64 exec, %3\n\tv_max_f64 %1, %1, %4\n\ts_mov_b64 exec, -1"
-      : "+v"(a), "+v"(b) : "s"(m0), "s"(m1), "v"(t));
+      : "+&v"(a), "+&v"(b) : "s"(m0), "s"(m1), "v"(t));
 }
 __device__ inline void kq_raise(mask64 m0, mask64 m1, mask64 m2, double& a, double& b, double& c, double t) {
   asm("s_mov_b64 exec, %3\n\tv_max_f64 %0, %0, %6\n\ts_mov_b64 exec, %4\n\tv_max_f64 %1, %1, %6\n\ts_mov_b64 exec, %5\n\tv_max_f64 %2, %2, %6\n\t"
       "s_mov_b64 exec, -1"
-      : "+v"(a), "+v"(b), "+v"(c) : "s"(m0), "s"(m1), "s"(m2), "v"(t));
+      : "+&v"(a), "+&v"(b), "+&v"(c) : "s"(m0), "s"(m1), "s"(m2), "v"(t));
 }
 // -- the smallest of some words
 __device__ inline void kq_least(mask64 m0, uint32_t& least, uint32_t o0) {
-  asm("s_mov_b64 exec, %1\n\tv_min_u32 %0, %2, %0\n\ts_mov_b64 exec, -1" : "+v"(least) : "s"(m0), "v"(o0));
+  asm("s_mov_b64 exec, %1\n\tv_min_u32 %0, %2, %0\n\ts_mov_b64 exec, -1" : "+&v"(least) : "s"(m0), "v"(o0));
 }
 __device__ inline void kq_least(mask64 m0, mask64 m1, uint32_t& least, uint32_t o0, uint32_t o1) {
   asm("s_mov_b64 exec, %1\n\tv_min_u32 %0, %3, %0\n\ts_mov_b64 exec, %2\n\tv_min_u32 %0, %4, %0\n\ts_mov_b64 exec, -1"
-      : "+v"(least) : "s"(m0), "s"(m1), "v"(o0), "v"(o1));
+      : "+&v"(least) : "s"(m0), "s"(m1), "v"(o0), "v"(o1));
 }
 // -- bits met so far, and those met twice
 __device__ inline void kq_meet(mask64 m0, mask64 m1, uint32_t& seen, uint32_t& twice, uint32_t bit0, uint32_t bit1) {
   asm("s_mov_b64 exec, %2\n\tv_and_or_b32 %1, %0, %4, %1\n\tv_or_b32 %0, %4, %0\n\t"
       "s_mov_b64 exec, %3\n\tv_and_or_b32 %1, %0, %5, %1\n\tv_or_b32 %0, %5, %0\n\t"
       "s_mov_b64 exec, -1"
-      : "+v"(seen), "+v"(twice) : "s"(m0), "s"(m1), "v"(bit0), "v"(bit1));
+      : "+&v"(seen), "+&v"(twice) : "s"(m0), "s"(m1), "v"(bit0), "v"(bit1));
 }
 // -- an entry into its slot
 __device__ inline void kq_put(mask64 m0, mask64 m1, double& e0, double& e1, double& s0, double& s1, uint32_t& o0, uint32_t& o1, uint32_t& w0, uint32_t& w1,
@@ -155,7 +156,7 @@ __device__ inline void kq_put(mask64 m0, mask64 m1, double& e0, double& e1, doub
   asm("s_mov_b64 exec, %8\n\tv_mov_b64 %0, %10\n\tv_mov_b64 %2, %11\n\tv_mov_b32 %4, %12\n\tv_mov_b32 %6, %13\n\t"
       "s_mov_b64 exec, %9\n\tv_mov_b64 %1, %10\n\tv_mov_b64 %3, %11\n\tv_mov_b32 %5, %12\n\tv_mov_b32 %7, %13\n\t"
       "s_mov_b64 exec, -1"
-      : "+v"(e0), "+v"(e1), "+v"(s0), "+v"(s1), "+v"(o0), "+v"(o1), "+v"(w0), "+v"(w1) : "s"(m0), "s"(m1), "v"(e), "v"(s), "v"(o), "v"(w));
+      : "+&v"(e0), "+&v"(e1), "+&v"(s0), "+&v"(s1), "+&v"(o0), "+&v"(o1), "+&v"(w0), "+&v"(w1) : "s"(m0), "s"(m1), "v"(e), "v"(s), "v"(o), "v"(w));
 }
 // -- the dispatched entry out of it: a slot without times, free, its word in `out`
 template <int U>
@@ -164,20 +165,20 @@ __device__ inline void kq_take(mask64 m0, mask64 m1, double& e0, double& e1, dou
   asm("s_mov_b64 exec, %6\n\tv_mov_b64 %0, %8\n\tv_mov_b64 %2, %8\n\tv_or_b32 %4, %11, %4\n\tv_mov_b32 %5, %9\n\t"
       "s_mov_b64 exec, %7\n\tv_mov_b64 %1, %8\n\tv_mov_b64 %3, %8\n\tv_or_b32 %4, %12, %4\n\tv_mov_b32 %5, %10\n\t"
       "s_mov_b64 exec, -1"
-      : "+v"(e0), "+v"(e1), "+v"(s0), "+v"(s1), "+v"(free_slots), "+v"(out) : "s"(m0), "s"(m1), "s"(none), "v"(w0), "v"(w1), "n"(1 << U), "n"(2 << U));
+      : "+&v"(e0), "+&v"(e1), "+&v"(s0), "+&v"(s1), "+&v"(free_slots), "+&v"(out) : "s"(m0), "s"(m1), "s"(none), "v"(w0), "v"(w1), "n"(1 << U), "n"(2 << U));
 }
 // -- push-backs with ties from `tie` on (kq_again) or a word of their own
 __device__ inline void kq_again(mask64 m0, mask64 m1, double& s0, double& s1, uint32_t& o0, uint32_t& o1, double e0, double e1, uint32_t tie_mask, uint32_t tie) {
   asm("s_mov_b64 exec, %4\n\tv_mov_b64 %0, %6\n\tv_bfi_b32 %2, %8, %9, %2\n\t"
       "s_mov_b64 exec, %5\n\tv_mov_b64 %1, %7\n\tv_bfi_b32 %3, %8, %9, %3\n\t"
       "s_mov_b64 exec, -1"
-      : "+v"(s0), "+v"(s1), "+v"(o0), "+v"(o1) : "s"(m0), "s"(m1), "v"(e0), "v"(e1), "v"(tie_mask), "s"(tie));
+      : "+&v"(s0), "+&v"(s1), "+&v"(o0), "+&v"(o1) : "s"(m0), "s"(m1), "v"(e0), "v"(e1), "v"(tie_mask), "s"(tie));
 }
 __device__ inline void kq_again(mask64 m0, mask64 m1, double& s0, double& s1, uint32_t& o0, uint32_t& o1, double e0, double e1, uint32_t word) {
   asm("s_mov_b64 exec, %4\n\tv_mov_b64 %0, %6\n\tv_mov_b32 %2, %8\n\t"
       "s_mov_b64 exec, %5\n\tv_mov_b64 %1, %7\n\tv_mov_b32 %3, %8\n\t"
       "s_mov_b64 exec, -1"
-      : "+v"(s0), "+v"(s1), "+v"(o0), "+v"(o1) : "s"(m0), "s"(m1), "v"(e0), "v"(e1), "v"(word));
+      : "+&v"(s0), "+&v"(s1), "+&v"(o0), "+&v"(o1) : "s"(m0), "s"(m1), "v"(e0), "v"(e1), "v"(word));
 }
 // reductions over the lanes of a plan (two or four)
 template <int QL>

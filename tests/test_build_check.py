@@ -1,9 +1,12 @@
 """The look over the assembly of a build (rpeg_amd/build.py): a 64-bit vector shift must not take its amount from the last
-vector register of a kernel's allocation.  CPU only."""
+vector register of a kernel's allocation.  And over the inline assembly of the sources: what several instructions write may not share a
+register with what they read.  CPU only."""
+
+import re
 
 import pytest
 
-from rpeg_amd.build import shifts_by_last_register
+from rpeg_amd.build import HEADERS, SOURCES, shifts_by_last_register
 
 LISTING = """
 helper:                                 ; @helper
@@ -54,3 +57,35 @@ def test_a_shift_by_the_last_register_is_found(in_one, n_one, in_helper, called,
 def test_a_listing_without_kernels_is_refused():
     with pytest.raises(RuntimeError):
         shifts_by_last_register("k_one:\n\ts_endpgm\n")
+
+
+def several_instructions(source):
+    """(instructions, constraints of the outputs) of the inline assembly of a source that is more than one instruction."""
+    for m in re.finditer(r"\basm\s*(?:volatile\s*)?\(", source):
+        parts, depth, quoted, at = [""], 1, False, m.end()
+        while depth:
+            c = source[at]
+            if c == '"' and source[at - 1] != "\\":
+                quoted = not quoted
+            if not quoted:
+                depth += (c == "(") - (c == ")")
+            if c == ":" and depth == 1 and not quoted:
+                parts.append("")
+            else:
+                parts[-1] += c
+            at += 1
+        if "\\n" in parts[0] and len(parts) > 1:
+            yield parts[0], re.findall(r'"([=+][^"]*)"', parts[1])
+
+
+def test_outputs_of_several_instructions_share_no_register_with_inputs():
+    """An operand that is written may be given the register of one that is read and has the same value, unless it is early-clobber:
+    right only where nothing is read behind the first write."""
+    seen = 0
+    for path in SOURCES + HEADERS:
+        with open(path) as f:
+            for instructions, outputs in several_instructions(f.read()):
+                seen += 1
+                assert outputs and all("&" in x for x in outputs), (path, instructions, outputs)
+    assert seen >= 15
+    assert [x for _, x in several_instructions('asm("v_a %0, %1\\n\\tv_b %2" : "+v"(a), "=&v"(b[f(0)]) : "s"(m)); asm("v_c %0" : "=v"(d));')] == [["+v", "=&v"]]
