@@ -10,6 +10,8 @@ import shutil
 import subprocess
 import tempfile
 
+from .exec_check import exec_set_under_a_mask
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB = os.path.join(HERE, "librpeg_eval.so")
 SOURCES = [os.path.join(HERE, "csrc", "rpeg_engine.hip")]
@@ -91,9 +93,11 @@ def _compile(lib: str, extra: list, verbose: bool) -> str:
             raise RuntimeError("hipcc left no gfx950 assembly")
         for path in listings:
             with open(path) as f:
-                bad = shifts_by_last_register(f.read())
-            if bad:
-                raise RuntimeError("64-bit shift by the last register of an allocation: " + "; ".join(" / ".join(x) for x in bad))
+                asm = f.read()
+            for bad, what in ((shifts_by_last_register(asm), "64-bit shift by the last register of an allocation"),
+                              (exec_set_under_a_mask(asm), "inline assembly sets EXEC where some lanes may be off")):
+                if bad:
+                    raise RuntimeError(what + ": " + "; ".join(" / ".join(x) for x in bad))
         os.replace(out, lib)
     finally:
         shutil.rmtree(tmp, ignore_errors=True)

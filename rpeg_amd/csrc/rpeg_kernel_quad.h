@@ -121,9 +121,10 @@ __device__ inline double kq_vmin(double a, double b, double c, double d) {
   return r;
 }
 // What changes in some lanes only, mostly for two slots at a time: the lanes of m0, those of m1, then all (a wavefront schedules with
-// all of them on).  A move or a maximum each, where a select takes an instruction for every word and one for what it selects; the masks go
-// to EXEC by scalar instructions, which other wavefronts' vector instructions overlap.  (us a step, selects / moves: 1,048,576 DPO plans
-// 787 / 720, 262,144 AC-share 3,455 / 3,370, 131,072 PPO 838 / 810, GRPO 418 / 402, 65,536 GRPO 304 / 291, 20,011 PPO 297 / 284.)
+// all of them on; the build refuses a listing in which one of these stands where some may be off: exec_check.py).  A move or a maximum
+// each, where a select takes an instruction for every word and one for what it selects; the masks go to EXEC by scalar instructions,
+// which other wavefronts' vector instructions overlap.  (us a step, selects / moves: 1,048,576 DPO plans 787 / 720, 262,144 AC-share
+// 3,455 / 3,370, 131,072 PPO 838 / 810, GRPO 418 / 402, 65,536 GRPO 304 / 291, 20,011 PPO 297 / 284.)
 // What is written here is written before the last of the other operands is read: early-clobber, also what is read itself.
 // -- the larger of two times
 __device__ inline void kq_raise(mask64 m0, mask64 m1, double& a, double& b, double t) {
