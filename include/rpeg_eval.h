@@ -455,7 +455,7 @@ int rpeg_sa_propose(rpeg_engine_t* e, const rpeg_sa_params_t* prm, int32_t what,
    in [2]), [7] wave tasks of the few-lanes-per-plan kernel (included in [2]), [8] plans that the call BEFORE the last
    one redid because their ready sets outgrew their kernel's (of the calls that were laid out, by the host or on the device: a
    batch that needed no layout leaves the figure as it is), [9] plans of the few-lanes-per-plan kernel, [10], [11], [12] launches of its forms for
-   ready sets of up to 8, 16 and 24 entries. */
+   ready sets of up to 8, 16 and 24 entries, [13] 1 where the call was laid out on the side stream (rpeg_engine_set_side_layout). */
 int rpeg_engine_stats(const rpeg_engine_t* e, uint64_t* out, int32_t n);
 
 /* Host time of the last rpeg_eval_batch call that laid its batch out, in microseconds of the steady clock: [0] from

@@ -1054,7 +1054,7 @@ struct rpeg_engine_s {
   bool timing = false;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms = -1.0;
-  uint64_t stats[13] = {};
+  uint64_t stats[14] = {};
   double host_us[4] = {0, 0, 0, 0};   // host time of the last laid-out rpeg_eval_batch call: rpeg_engine_host_us
   int n_cu = 256;
   uint8_t* static_ptr = nullptr;    // this device's copy of the file-scope scratch array (rpeg_eval_batch_static)
@@ -1712,7 +1712,7 @@ int rpeg_engine_reset_classes(rpeg_engine_t* e) {
 
 int rpeg_engine_stats(const rpeg_engine_t* e, uint64_t* out, int32_t n) {
   if (!e || !out) return -1;
-  for (int i = 0; i < n && i < 13; ++i) out[i] = e->stats[i];
+  for (int i = 0; i < n && i < 14; ++i) out[i] = e->stats[i];
   return 0;
 }
 
@@ -1871,7 +1871,7 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     if (e->h_tot[0] == 0u) {
       e->stats[0] = e->cls_sig.size();   // (the classes the engine knows: which of them the batch holds was not counted)
       e->stats[1] = 0; e->stats[2] = n; e->stats[3] = lds; e->stats[4] = 0; e->stats[5] = 1; e->stats[6] = 0;
-      e->stats[7] = e->stats[9] = e->stats[10] = e->stats[11] = e->stats[12] = 0;
+      e->stats[7] = e->stats[9] = e->stats[10] = e->stats[11] = e->stats[12] = e->stats[13] = 0;
       ++e->batch_calls;
       return read_timing(e);
     }
@@ -2643,8 +2643,9 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   e->stats[2] = n_waves + n_quad_waves + n_solo;
   e->stats[7] = n_quad_waves;
   e->stats[9] = n_quad_plans;
-  e->stats[10] = e->stats[11] = e->stats[12] = 0;
+  e->stats[10] = e->stats[11] = e->stats[12] = e->stats[13] = 0;
   for (const QuadLaunch& q : quad_launch) ++e->stats[10 + q.kind];
+  e->stats[13] = ahead ? 1u : 0u;
   e->stats[3] = lds;
   e->stats[4] = wsb * grid;
   e->stats[5] = one ? 1u : (uint64_t)ls;
@@ -2909,7 +2910,7 @@ int rpeg_eval_batch_static(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   launch_plan(lds, s, L, e->n_cu);
   HIP_TRY(e, hipGetLastError());
   e->stats[0] = 0; e->stats[1] = 0; e->stats[2] = n; e->stats[3] = lds; e->stats[4] = 0; e->stats[5] = 1; e->stats[6] = 0;
-  e->stats[7] = e->stats[9] = e->stats[10] = e->stats[11] = e->stats[12] = 0;
+  e->stats[7] = e->stats[9] = e->stats[10] = e->stats[11] = e->stats[12] = e->stats[13] = 0;
   // With RPEG_NO_WAIT the call ends here: three launches on the caller's stream, no copy and no wait (what a
   // capturing stream accepts).  Plans of classes the engine has not met are then told by their mask alone.
   if (flags & RPEG_NO_WAIT) return 0;
@@ -3248,7 +3249,7 @@ int host_small_submit(rpeg_engine_t* e, HostLane& ln, uint64_t n, GET get, uint3
   }
   const size_t m = ln.idx.size();
   e->stats[0] = 0; e->stats[1] = n_new; e->stats[2] = m; e->stats[3] = 0; e->stats[4] = 0; e->stats[5] = 1; e->stats[6] = 0;
-  e->stats[7] = e->stats[9] = e->stats[10] = e->stats[11] = e->stats[12] = 0;
+  e->stats[7] = e->stats[9] = e->stats[10] = e->stats[11] = e->stats[12] = e->stats[13] = 0;
   if (m == 0) return 0;
   if (e->max_nodes > (uint32_t)(WAVE * KP_MAX_NS) || kp_lds_bytes(e->max_nodes, e->max_slots) > 64 * 1024) return 1;
   if (int rc = ensure_pool(e, s)) return rc;

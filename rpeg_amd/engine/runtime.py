@@ -280,11 +280,11 @@ class Engine:
         return float(self.lib.rpeg_engine_last_kernel_ms(self._h))
 
     def stats(self) -> Dict[str, int]:
-        buf = (C.c_uint64 * 13)()
-        self.lib.rpeg_engine_stats(self._h, buf, 13)
+        buf = (C.c_uint64 * 14)()
+        self.lib.rpeg_engine_stats(self._h, buf, 14)
         return dict(classes=buf[0], classes_lowered=buf[1], wave_tasks=buf[2], lds_bytes=buf[3], workspace_bytes=buf[4],
                     state_lanes=buf[5], single_plan_tasks=buf[6], quad_tasks=buf[7], redone_before=buf[8], quad_plans=buf[9],
-                    quad_launches_8=buf[10], quad_launches_16=buf[11], quad_launches_24=buf[12])
+                    quad_launches_8=buf[10], quad_launches_16=buf[11], quad_launches_24=buf[12], side_layout=buf[13])
 
     def alloc_outputs(self, n: int):
         torch = _torch()

@@ -481,7 +481,7 @@ def test_the_fitted_figures_of_the_split_move_plans_between_kernels_and_no_bit()
 def test_the_stream_that_carries_the_layout_changes_no_bit(c, n):
     """rpeg_engine_set_side_layout: cost-model launch, layout and main kernel on the side stream or on the caller's
     (the default); cold calls (classes lowered, several rounds) and warm ones; two engines that step in turn on two
-    threads, of which the one that finds the side streams taken stays on its own; a batch that no plan of is valid.
+    threads, with it (of which the one that finds the side streams taken stays on its own) and without; a batch that no plan of is valid.
     Every call equals the host build."""
     import threading
     from rpeg_amd.engine.runtime import Engine
@@ -499,6 +499,7 @@ def test_the_stream_that_carries_the_layout_changes_no_bit(c, n):
         try:
             for call in range(3):
                 check(eng.eval(batch, gate_stale=True), (on, call))
+                assert eng.stats()["side_layout"] == on
             bad = batch.slice(0, 30000)
             bad.vert[0, :] = 0   # dp = 0 in every plan: the gate rejects the whole batch
             out = eng.eval(bad, gate_stale=True)
@@ -506,26 +507,30 @@ def test_the_stream_that_carries_the_layout_changes_no_bit(c, n):
             check(eng.eval(batch, gate_stale=True), (on, "after a batch without a valid plan"))
         finally:
             eng.close()
-    engines = [Engine(cfg.problem) for _ in range(2)]
-    errors = []
+    for on in (True, False):
+        engines = [Engine(cfg.problem) for _ in range(2)]
+        errors, aside = [], []
 
-    def work(eng, who):
+        def work(eng, who):
+            try:
+                eng.set_side_layout(on)
+                for call in range(4):
+                    check(eng.eval(batch, gate_stale=True), ("two engines", on, who, call))
+                    aside.append(eng.stats()["side_layout"])
+            except Exception as exc:   # noqa: BLE001 - handed to the main thread
+                errors.append(exc)
+
         try:
-            for call in range(4):
-                check(eng.eval(batch, gate_stale=True), ("two engines", who, call))
-        except Exception as exc:   # noqa: BLE001 - handed to the main thread
-            errors.append(exc)
-
-    try:
-        threads = [threading.Thread(target=work, args=(e, k)) for k, e in enumerate(engines)]
-        for t in threads:
-            t.start()
-        for t in threads:
-            t.join()
-        assert not errors, errors
-    finally:
-        for e in engines:
-            e.close()
+            threads = [threading.Thread(target=work, args=(e, k)) for k, e in enumerate(engines)]
+            for t in threads:
+                t.start()
+            for t in threads:
+                t.join()
+            assert not errors, errors
+            assert len(aside) == 8 and any(aside) == on, aside
+        finally:
+            for e in engines:
+                e.close()
 
 
 @pytest.mark.parametrize("c,n,what", [(3, 65536, "single_plan_tasks"), (5, 40000, "quad_tasks"), (2, 131072, "quad_tasks"),

@@ -1,6 +1,6 @@
 """Batches whose launches of the few-lanes-per-plan kernel are one, two or three, on the streams of a call that lays them out ahead and
 of one that does not, timed and not: every stream waits for the layout before its first launch.  The oracle is the host build,
-bit for bit."""
+bit for bit.  (One launch: on the caller's stream.  Of two, the second on a stream of its own, of three the last two.)"""
 
 import numpy as np
 import pytest
@@ -13,7 +13,7 @@ from tests.test_positions import same_bits
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("c,n,most", [(4, 17000, 2), (5, 20011, 3), (2, 17000, 3), (2, 65536, 3), (1, 30000, 3), (3, 30000, 3)])
+@pytest.mark.parametrize("c,n,most", [(4, 17000, 1), (5, 20011, 2), (2, 17000, 2), (3, 30000, 2), (2, 65536, 3), (1, 30000, 3)])
 def test_launches_of_a_call(c, n, most):
     from rpeg_amd.engine.runtime import DeviceBatch, Engine
     cfg, batch = seeded_batch(c, n)
@@ -29,6 +29,7 @@ def test_launches_of_a_call(c, n, most):
                 eng.eval_device(resident, out, gate_stale=True)
                 got = {k: v.cpu().numpy() for k, v in out.items()}
                 s = eng.stats()
+                assert s["side_layout"] == side
                 if s["quad_tasks"]:
                     launches.add(s["quad_launches_8"] + s["quad_launches_16"] + s["quad_launches_24"])
                 assert np.array_equal(got["mask"], want["mask"]), (side, timing, call)
@@ -39,4 +40,4 @@ def test_launches_of_a_call(c, n, most):
             assert not timing or eng.last_kernel_ms() > 0.0
     finally:
         eng.close()
-    assert launches and max(launches) <= most, launches
+    assert launches and max(launches) == most, launches
