@@ -1964,8 +1964,8 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
     HIP_TRY(e, hipGetLastError());
     // Cost model, memory model and gates of every plan: they need the verdict of the gate (which plans to skip) and
     // nothing of the classes, so they run behind the signature kernel while the host waits for the counts (their
-    // flag, not the stream) and lays the batch out.  On k_quad's stream the launch goes out first: it does not wait for
-    // the hand-over of the counts, and the hand-over has a few microseconds to spare.
+    // flag, not the stream) and lays the batch out.  On the caller's stream they follow the hand-over of the counts, which the
+    // host waits for; with `ahead` they go out first, on k_quad's stream, and do not wait for it.
     if (round == 0 && ahead) {
       HIP_TRY(e, hipEventRecord(e->ev_sig, s));
       HIP_TRY(e, hipStreamWaitEvent(e->s3, e->ev_sig, 0));
@@ -2651,13 +2651,13 @@ static int eval_batch_impl(rpeg_engine_t* e, uint64_t n, const rpeg_plan_soa_t* 
   e->stats[5] = one ? 1u : (uint64_t)ls;
   e->stats[6] = n_solo;
   // The main kernel is submitted first: it needs 26 KB of LDS per wavefront, and once single-plan wavefronts
-  // fill a compute unit its wavefronts only fit in as those retire.
+  // fill a compute unit its wavefronts only fit in as those retire.  It follows the scatter in order, and starts first, as it must: the
+  // kernels of the other streams see the fork event a few microseconds later.
   // The memory-model launch, where it was deferred: on k_quad's stream when that kernel has nothing to do in this call
   // (the launch then runs beside all scheduling kernels), else behind the main kernel, where it runs beside the tails
-  // of the two other kernels.
-  // With the layout ahead on k_quad's stream, that stream and the caller's change places until the join: the main
-  // kernel follows the scatter in order (it starts first, as it must: the kernels of the two other streams see the
-  // fork event a few microseconds later), and k_quad follows the cost-model launch on the caller's stream.
+  // of the two other kernels; without a main kernel, see below.
+  // With `ahead` (rpeg_engine_set_side_layout) k_quad's stream and the caller's change places until the join: layout, scatter and what
+  // follows them in order are on the former, what else goes to k_quad's stream on the latter.
   const bool peaks_aside = peaks_deferred && !n_quad_waves;
   const hipStream_t sm = ahead ? e->s3 : s;    // the main kernel and what follows it
   hipStream_t sq = ahead ? s : e->s3;          // k_quad, or the memory-model launch in its place

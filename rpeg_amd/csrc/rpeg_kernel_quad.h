@@ -1,7 +1,7 @@
 // rpeg_kernel_quad.h - two or four lanes per plan, 32 or 16 plans of one class per wavefront (device only).
 //
 // The kernel of large batches.  The ready set of a plan lives in the REGISTERS of its QL lanes, SL entries each
-// (two, four or six, by what the classes of the launch need), unordered.  An entry:
+// (two, four or six, by what the class needs), unordered.  An entry:
 //
 //   e     true start time: the larger of the node's key and the availability of the devices it reserves, raised at every
 //         dispatch that reserves one of them
@@ -34,8 +34,9 @@
 // 384).  Ranks go level by level with a node per lane of the plan, all plans together (kq_ranks).  A node's id is its place by tie-break class, so that
 // counting the larger ranks of its class walks through consecutive rows.
 //
-// Bound: vector issue and, with few wavefronts in flight, the latency of a round (four lanes of four entries: some 360 vector
-// instructions a round).  LDS bounds the wavefronts in flight: sixteen plans of 85 nodes and 40 slots take 13 KiB, 3 per
+// Bound: vector issue and, with few wavefronts in flight, the latency of a round (four lanes of four entries: 114 vector
+// instructions in a round that looks at its successors once and files some, 47 more where entries are pushed back; some 360
+// and then 270 in earlier builds).  LDS bounds the wavefronts in flight: sixteen plans of 85 nodes and 40 slots take 13 KiB, 3 per
 // SIMD (with a ready time, a word and an in-degree per node and plan, and all plans' ranks at once, 26 KiB and 1.5; 300
 // nodes 28 against 70 KiB).
 // Scheduling a wavefront: 42-node GRPO class 60 us, 92 nodes 130-190, 28-node DPO class 35.  The step, with the larger state
@@ -328,7 +329,7 @@ __device__ inline double kq_more_successors(const ClassView& cv, int i, double b
 // ahead, durations one.  A rank takes eight bytes a node, more than all a plan keeps of it later, but is read back only by the
 // few levels below: in LDS lie rows that nodes share (RankRec), and the ranks go through memory to the comparison of positions, which takes
 // them a part of the plans at a time (1,048,576 DPO plans, 240 MB of ranks: by the counters all of them are written out and most read
-// back from beyond the L2, the launch moves 779 MB, before 358; 262,144 AC-share plans, all schedulers, 1,555, before 845); where the launches'
+// back from beyond the L2, the launch moves 769 MB, before 358; 262,144 AC-share plans, all schedulers, 1,555, before 845); where the launches'
 // wavefronts find room together with all of their ranks those stay in LDS (kq_ranks_in_lds).  Before, the pass ran once for every part,
 // with two to four times the lanes for levels of two or three nodes, and a part's ranks all lay in LDS.  us a step, before / now:
 // 262,144 AC-share plans 4,196 / 3,953, 131,072 2,720 / 2,572, 65,536 1,550 / 1,430; 131,072 PPO 989 / 935, GRPO 490 / 442; 65,536
