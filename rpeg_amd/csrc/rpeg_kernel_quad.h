@@ -35,8 +35,8 @@
 // counting the larger ranks of its class walks through consecutive rows.
 //
 // Bound: vector issue and, with few wavefronts in flight, the latency of a round (four lanes of four entries: 114 vector
-// instructions in a round that looks at its successors once and files some, 47 more where entries are pushed back; some 360
-// and then 270 in earlier builds).  LDS bounds the wavefronts in flight: sixteen plans of 85 nodes and 40 slots take 13 KiB, 3 per
+// instructions in a round that looks at its successors once and files some, 47 more where entries are pushed back; some 360 at
+// first, then 270).  LDS bounds the wavefronts in flight: sixteen plans of 85 nodes and 40 slots take 13 KiB, 3 per
 // SIMD (with a ready time, a word and an in-degree per node and plan, and all plans' ranks at once, 26 KiB and 1.5; 300
 // nodes 28 against 70 KiB).
 // Scheduling a wavefront: 42-node GRPO class 60 us, 92 nodes 130-190, 28-node DPO class 35.  The step, with the larger state
